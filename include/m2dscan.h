@@ -357,6 +357,15 @@ int m2d_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, con
                    int pre_act, const void* pre_scale, const void* pre_bias,
                    int post_act, const void* post_scale, const void* post_bias, void* y, void* stream);
 
+/* m2d_linear_fwd (no pre_act) that also keeps the layer's output before the activation: z (P,N) bf16, y = post(z). */
+int m2d_linear_keep_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias,
+                        int post_act, const void* post_scale, const void* post_bias, void* z, void* y, void* stream);
+
+/* m2d_dwconv3x3_fwd of StarReLU(x) (rounded to bf16; models/utils.py:101-114), bf16 activations; the zero padding lies
+ * outside the StarReLU. */
+int m2d_starrelu_dwconv3x3_fwd(int B, int H, int W, int C, int weight_dtype, const void* x, const void* star_scale,
+                               const void* star_bias, const void* weight, void* y, void* stream);
+
 /* m2d_linear_fwd with a LayerNorm over the K inputs in front of the layer (ln_weight, ln_bias: (K), weight_dtype):
  * y = post(LayerNorm(x) weight^T + bias), for a norm whose only reader is the layer (local_norm before pwconv1,
  * models/mamba2d.py:57,161; norm2 before fc1, :248).  The normalised rows are rounded to bf16 as a LayerNorm
@@ -375,6 +384,49 @@ int m2d_layernorm_linear_fwd(int64_t P, int K, int N, int weight_dtype, const vo
 int m2d_mlp_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x,
                 const void* ln_weight, const void* ln_bias, float eps,
                 const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream);
+
+/* ---- Operators of a residual block in training (models/mamba2d.py:191-254, models/utils.py:58-118), bf16-mixed:
+ * the residual stream x, its gradient and all parameters are fp32, everything between the norms and the residual
+ * updates is bf16.  Parameter gradients are left as per-workgroup sums in `part` (fp32): as many slices as the
+ * function's _parts query says, each of the stated length; m2d_train_reduce adds slices in a fixed order.
+ *
+ * m2d_train_norm_fwd: x_out = x * scale[c] + keep[row / rows_per_sample] * (r + r2) (left out where r is NULL; scale, r2
+ *   and keep may be NULL), y1 = LayerNorm(x_out; w1, b1, eps1), y2 = LayerNorm(y1 before its rounding; w2, b2, eps2); y1
+ *   and y2 may be NULL.  C a multiple of 4 up to 256.
+ * m2d_train_norm_bwd: for the gradients d1, d2 (may be NULL) of y1, y2 and dx_out of an update x_out = x * scale + ...,
+ *   dx = the gradient of x, branch = bf16(dx * keep) (may be NULL).  part: (slices, 5, C) sums for w1, b1, w2, b2, scale.
+ * m2d_train_branch: y = bf16(x * keep[i / per_sample]) over n elements.
+ * m2d_train_dwconv_bwd: p is the input of the StarReLU in front of the depthwise 3x3 (weight (C,1,3,3)), g the gradient
+ *   of the convolution's output; dp the gradient of p.  part: (slices, 9 C + 2) sums for the weight, the StarReLU's
+ *   scale and its bias.
+ * m2d_train_linear_bwd: for y = post(pre(x) weight^T + b) with z the value before post: dx from dy.  post_act nothing or
+ *   GELU, pre_act any; pre StarReLU leaves part: (slices, 2) sums for its scale and bias.  K a multiple of 16, N of 32,
+ *   both up to 512.
+ * m2d_train_wgrad: part: (slices, N K + N) sums for the weight and, with `bias`, the bias of that layer. */
+int m2d_train_norm_fwd(int64_t rows, int C, int rows_per_sample, const float* x, const float* scale, const void* r, const void* r2,
+                       const float* keep, float* x_out, const float* w1, const float* b1, float eps1, void* y1,
+                       const float* w2, const float* b2, float eps2, void* y2, void* stream);
+int m2d_train_norm_parts(int64_t rows, int C);
+int m2d_train_norm_bwd(int64_t rows, int C, int rows_per_sample, const float* x, const void* d1, const void* d2, const float* dx_out,
+                       const float* scale, const float* keep, const float* w1, const float* b1, float eps1, const float* w2,
+                       float eps2, float* dx, void* branch, float* part, void* stream);
+int m2d_train_branch(int64_t n, int64_t per_sample, const float* x, const float* keep, void* y, void* stream);
+int m2d_train_dwconv_parts(int B, int H, int W, int C);
+int m2d_train_dwconv_bwd(int B, int H, int W, int C, const void* p, const void* g, const float* weight, const float* star_scale,
+                         const float* star_bias, void* dp, float* part, void* stream);
+int m2d_train_linear_parts(int64_t P, int K, int N);
+int m2d_train_linear_bwd(int64_t P, int K, int N, const void* dy, const void* z, int post_act, const float* weight, const void* x,
+                         int pre_act, const float* pre_scale, void* dx, float* part, void* stream);
+int m2d_train_wgrad_parts(int64_t P, int N, int K);
+int m2d_train_wgrad(int64_t P, int N, int K, const void* dy, const void* z, int post_act, const void* x, int pre_act,
+                    const float* pre_scale, const float* pre_bias, int bias, float* part, void* stream);
+typedef struct m2d_reduce_seg {
+  const float* part;          /* slice s starts at part + s * stride */
+  float* out;
+  int64_t stride;
+  int32_t n, parts;           /* out[i] = sum over s < parts of part[s * stride + i], i < n */
+} m2d_reduce_seg;
+int m2d_train_reduce(int nsegs, const m2d_reduce_seg* segs, void* stream);
 
 /* Measurement aid; no counterpart in the reference.  While enabled, every m2d_scan_fwd /
  * m2d_scan_bwd call records a pair of HIP events on its stream around the main scan kernel of

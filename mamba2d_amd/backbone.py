@@ -22,10 +22,11 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import wavefront
 from .wavefront import (dwconv3x3_fwd_op, layernorm_fwd_op, layernorm_linear_act_fwd_op, linear_act_fwd_op, mlp_fwd_op,
                         rope_qknorm_fwd_op,
                         rope_attention_fwd_op, scale_residual_fwd_op, scale_residual_layernorm_fwd_op, starrelu_fwd_op,
-                        wavefront_scan_cuda)
+                        train_block_op, wavefront_scan_cuda)
 
 M2D_T = dict(n_blocks=(3, 3, 9, 3), embed_dim=(64, 128, 320, 512),
              token_mixer=("2D_local", "2D_local", "RopeAttention", "RopeAttention"),
@@ -328,6 +329,18 @@ def _drop_path(x, p, training):
     return x * keep.to(x.dtype) / (1.0 - p)
 
 
+def _kept(x, p, training):
+    """The factor of every sample that _drop_path applies, (B,) in fp32; None where it applies none."""
+    if p == 0.0 or not training:
+        return None
+    return (torch.rand(x.shape[0], device=x.device) >= p).float() / (1.0 - p)
+
+
+def _plain(mod, kind):
+    """The module is what its class says: exactly ``kind``, without hooks that a call past its forward would skip."""
+    return type(mod) is kind and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks)
+
+
 class ResBlock(nn.Module):
     """x <- s1*x + mixer(norm1 x);  x <- s2*x + MLP(norm2 x)  (``models/mamba2d.py:191-254``)."""
 
@@ -376,10 +389,63 @@ class ResBlock(nn.Module):
         y = ResBlock._residual(x, scale, *terms)
         return y, (norm(y) if norm is not None else None)
 
+    def _train_parameters(self, x):
+        """The block's parameters in the order of ``m2dscan::train_block``, or None where that operator does not take the
+        call.  It takes a scan block under bf16 autocast with fp32 parameters when gradients are asked for: forward and
+        backward in the library's kernels (the stock depthwise convolution's weight gradient alone takes 27 ms at
+        64x56x56x128, the library's whole block 2 ms)."""
+        mix, mlp = self.token_mixer, self.MLP
+        if not (x.is_cuda and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda") and x.dim() == 4 and x.numel() > 0
+                and torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.dtype in (torch.float32, torch.bfloat16)
+                and type(mix) is M2DBlock and not torch.compiler.is_compiling() and wavefront.FUSED_PROJECTIONS):
+            return None
+        C = x.shape[-1]
+        if C % 32 or C > 128 or x.shape[1] < 2 or x.shape[2] < 2 or mix.recomp not in ("partial", "full"):
+            return None
+        mods = [(self.norm1, LayerNorm), (mix, M2DBlock), (mix.in_proj, nn.Linear), (mix.x_proj, nn.Linear), (mix.dt_projT, nn.Linear),
+                (mix.dt_projL, nn.Linear), (mix.out_proj, nn.Linear), (self.res_scale1, Scale), (self.norm2, LayerNorm), (mlp, MLP),
+                (mlp.fc1, nn.Linear), (mlp.fc2, nn.Linear), (self.res_scale2, Scale)]
+        path = mix.local_path
+        if path is not None:
+            mods += [(mix.local_norm, LayerNorm), (path, SepConv), (path.pwconv1, nn.Linear), (path.act1, StarReLU),
+                     (path.dwconv, nn.Conv2d), (path.act2, StarReLU), (path.pwconv2, nn.Linear)]
+        if not all(_plain(m, kind) for m, kind in mods):
+            return None
+        par = [self.norm1.weight, self.norm1.bias, mix.in_proj.weight, mix.in_proj.bias, mix.AT_log, mix.AL_log, mix.x_proj.weight,
+               mix.dt_projT.weight, mix.dt_projT.bias, mix.dt_projL.weight, mix.dt_projL.bias, mix.D, mix.out_proj.weight, mix.out_proj.bias,
+               self.res_scale1.scale, self.norm2.weight, self.norm2.bias, mlp.fc1.weight, mlp.fc1.bias, mlp.fc2.weight, mlp.fc2.bias,
+               self.res_scale2.scale]
+        want = [(C,), (C,), (C, C), (C,), None, None, None, None, None, None, None, None, (C, C), (C,), (C,), (C,), (C,), (4 * C, C), (4 * C,),
+                (C, 4 * C), (C,), (C,)]
+        if path is not None:
+            conv = path.dwconv
+            if conv.kernel_size != (3, 3) or conv.padding != (1, 1) or conv.stride != (1, 1) or conv.dilation != (1, 1) or conv.bias is not None \
+                    or conv.padding_mode != "zeros" or path.pwconv1.bias is not None or path.pwconv2.bias is not None:
+                return None
+            par += [mix.local_norm.weight, mix.local_norm.bias, path.pwconv1.weight, path.act1.scale, path.act1.bias, conv.weight,
+                    path.act2.scale, path.act2.bias, path.pwconv2.weight]
+            want += [(C,), (C,), (2 * C, C), (1,), (1,), (2 * C, 1, 3, 3), (1,), (1,), (C, 2 * C)]
+        for t, shape in zip(par, want):
+            if t is None or t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() % 16 or (shape is not None and t.shape != shape) \
+                    or t.device != x.device:
+                return None
+        if mix.x_proj.bias is not None or mix.AT_log.shape[1] != wavefront.STATES_PER_CALL or mix.dt_projT.weight.shape[1] > 32:
+            return None
+        return par
+
     def forward_fused(self, x, normed=None, next_norm=None):
         """The block on x, with ``normed`` = norm1(x) where the caller has it already; returns the block's output
         and ``next_norm`` of it (None without ``next_norm``): the LayerNorm that follows the block, computed in
-        the pass of the second residual update."""
+        the pass of the second residual update.  (None too where the training operator runs the block: it computes
+        its norms itself.)"""
+        par = self._train_parameters(x)
+        if par is not None:
+            mix = self.token_mixer
+            keep1, keep2 = _kept(x, self.drop_path, self.training), _kept(x, self.drop_path, self.training)
+            local_eps = mix.local_norm.eps if mix.local_norm is not None else 0.0
+            y = train_block_op(x.float().contiguous(), par, keep1, keep2, self.norm1.eps, self.norm2.eps, local_eps, mix.flip,
+                               mix.recomp == "full", wavefront.SAVE_CHECKPOINTS, wavefront._interval())
+            return y, None
         n1 = self.norm1(x) if normed is None else normed
         if isinstance(self.token_mixer, M2DBlock) and not self.training:
             mixed = self.token_mixer(n1, split=True)       # scan path and local path, summed in the update

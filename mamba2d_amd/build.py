@@ -36,6 +36,7 @@ SOURCES = {
     "m2dscan.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
     "m2dproj.hip": [],
     "m2dblock.hip": [],
+    "m2dtrain.hip": [],
     "m2dcompat.hip": [],
 }
 
@@ -100,16 +101,16 @@ def build_lib(verbose: bool = True) -> str:
 
 
 def build_shim(verbose: bool = True) -> str:
-    """Compile csrc/m2d_torch.cpp (host only) against torch and link it to libm2dscan.so."""
+    """Compile csrc/m2d_torch.cpp and m2d_train.cpp (host only) against torch and link it to libm2dscan.so."""
     import torch
     from torch.utils import cpp_extension as ce
 
-    src = os.path.join(HERE, "csrc", "m2d_torch.cpp")
+    src = [os.path.join(HERE, "csrc", name) for name in ("m2d_torch.cpp", "m2d_train.cpp")]
     inc = [f"-I{p}" for p in ce.include_paths(device_type="cuda")] + [f"-I{os.path.join(ROOT, 'include')}"]
     libdirs = ce.library_paths(device_type="cuda")
     cmd = ["hipcc", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-unused-result",
-           *inc, "-o", SHIM, src,
+           *inc, "-o", SHIM, *src,
            *[f"-L{d}" for d in libdirs], f"-L{HERE}", "-lm2dscan", "-lc10", "-lc10_hip", "-ltorch_cpu",
            "-ltorch_hip", "-ltorch", "-Wl,-rpath,$ORIGIN", *[f"-Wl,-rpath,{d}" for d in libdirs]]
     if verbose:

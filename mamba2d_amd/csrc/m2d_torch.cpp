@@ -17,10 +17,9 @@
 #include <vector>
 
 #include "m2dscan.h"
+#include "m2d_torch.h"
 
-namespace {
-
-using at::Tensor;
+namespace m2dshim {
 
 m2d_desc describe(const Tensor& x, const Tensor& AT, bool flip, bool raw_params = false, bool packed_bc = false,
                   bool dpre = false, int64_t ckpt_interval = 0) {
@@ -82,8 +81,6 @@ void expect_all(const m2d_desc& d, const Tensor& x, const Tensor& dT, const Tens
   }
   expect_param(D, "D", x, {E}, raw);
 }
-
-void check(int status) { TORCH_CHECK(status == M2D_OK, "m2dscan: ", m2d_status_str(status), " (status ", status, ")"); }
 
 Tensor bytes(size_t n, const Tensor& like) {
   return at::empty({static_cast<int64_t>(n > 0 ? n : 1)}, like.options().dtype(at::kByte));
@@ -513,8 +510,9 @@ void wf_bwd(const Tensor& hs, const Tensor& x, const Tensor& dT, const Tensor& d
                    AT.data_ptr(), AL.data_ptr(), grad_output.data_ptr(), dDAT.data_ptr(), dDAL.data_ptr(), omega.data_ptr(), st));
 }
 
+}  // namespace m2dshim
 
-}  // namespace
+using namespace m2dshim;
 
 TORCH_LIBRARY(m2dscan, m) {
   m.def("scan_fwd(Tensor x, Tensor deltaT, Tensor deltaL, Tensor AT, Tensor AL, Tensor BT, Tensor BL, Tensor C, "

@@ -1,0 +1,245 @@
+// m2d_train.cpp -- a residual block of a scan stage in bf16-mixed training as one autograd function.
+//
+// The block of models/mamba2d.py:191-254 with the token mixer of :157-188 and the local path and MLP of
+// models/utils.py:58-118: x1 = s1 x + mixer(norm1 x), x2 = s2 x1 + MLP(norm2 x1).  Forward and backward are a fixed
+// sequence of the library's kernels on one stream (9 + 12 launches beside the scan's own), issued from here: no
+// Python between them, no cast kernels (the fp32 parameters are read as they are), activations rounded to bf16 where
+// autocast rounds them.
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/library.h>
+
+#include <algorithm>
+
+#include "m2d_torch.h"
+
+namespace {
+
+using at::Tensor;
+using m2dshim::check;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+using OptTensor = c10::optional<Tensor>;
+
+// The block's parameters, in the order of the operator's list.
+enum Par { kN1W, kN1B, kInW, kInB, kATLog, kALLog, kXProj, kDtTW, kDtTB, kDtLW, kDtLB, kD, kOutW, kOutB, kRs1, kN2W, kN2B,
+           kFc1W, kFc1B, kFc2W, kFc2B, kRs2, kBase,
+           kLnW = kBase, kLnB, kPw1, kS1S, kS1B, kDw, kS2S, kS2B, kPw2, kAll };
+
+struct Shape { int64_t B, H, W, C, P, R, N; bool local; };
+
+Shape shape_of(const Tensor& x, at::TensorList p) {
+  TORCH_CHECK(x.dim() == 4 && x.is_cuda() && x.is_contiguous() && x.scalar_type() == at::kFloat,
+              "m2dscan: x must be a contiguous float32 (B,H,W,C) tensor on the GPU");
+  TORCH_CHECK(p.size() == kBase || p.size() == kAll, "m2dscan: a block has ", (int)kBase, " parameters, or ", (int)kAll, " with a local path, got ", p.size());
+  Shape s;
+  s.B = x.size(0); s.H = x.size(1); s.W = x.size(2); s.C = x.size(3);
+  s.P = s.B * s.H * s.W;
+  s.local = p.size() == kAll;
+  TORCH_CHECK(s.P > 0 && s.H > 1 && s.W > 1, "m2dscan: grid must be larger than one cell, got ", x.sizes());
+  TORCH_CHECK(p[kDtTW].dim() == 2 && p[kATLog].dim() == 2, "m2dscan: dt_projT must be (C, dt_rank), AT_log (C, d_state)");
+  s.R = p[kDtTW].size(1);
+  s.N = p[kATLog].size(1);
+  const int64_t C = s.C, M = 2 * C;
+  auto want = [&](int i, at::IntArrayRef shape) {
+    TORCH_CHECK(p[i].device() == x.device() && p[i].scalar_type() == at::kFloat && p[i].is_contiguous() && p[i].sizes() == shape,
+                "m2dscan: parameter ", i, " of the block must be a contiguous float32 ", shape, " tensor on x's device, got ", p[i].sizes());
+  };
+  want(kN1W, {C}); want(kN1B, {C}); want(kInW, {C, C}); want(kInB, {C}); want(kOutW, {C, C}); want(kOutB, {C}); want(kRs1, {C});
+  want(kN2W, {C}); want(kN2B, {C}); want(kFc1W, {4 * C, C}); want(kFc1B, {4 * C}); want(kFc2W, {C, 4 * C}); want(kFc2B, {C}); want(kRs2, {C});
+  if (s.local) {
+    want(kLnW, {C}); want(kLnB, {C}); want(kPw1, {M, C}); want(kDw, {M, 1, 3, 3}); want(kPw2, {C, M});
+    for (int i : {(int)kS1S, (int)kS1B, (int)kS2S, (int)kS2B}) want(i, {1});
+  }
+  return s;
+}
+
+const float* f32(const Tensor& t) { return t.data_ptr<float>(); }
+const float* opt(const OptTensor& t) { return t.has_value() && t->defined() ? t->data_ptr<float>() : nullptr; }
+
+Tensor bf16_like(const Tensor& x, int64_t C) {
+  return at::empty({x.size(0), x.size(1), x.size(2), C}, x.options().dtype(at::kBFloat16));
+}
+
+struct Block : public torch::autograd::Function<Block> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, at::TensorList par, const OptTensor& keep1, const OptTensor& keep2,
+                        double eps1, double eps2, double eps_local, bool flip, bool full, bool save_ckpt, int64_t interval) {
+    const std::vector<Tensor> p = par.vec();
+    const Shape s = shape_of(x, p);
+    c10::DeviceGuard guard(x.device());
+    hipStream_t st = m2dshim::current_stream(x);
+    const int C = (int)s.C, M = 2 * C, HD = 4 * C, rps = (int)(s.H * s.W);
+    const Tensor none;
+    Tensor n1 = bf16_like(x, C), nl = s.local ? bf16_like(x, C) : none;
+    check(m2d_train_norm_fwd(s.P, C, rps, f32(x), nullptr, nullptr, nullptr, nullptr, nullptr, f32(p[kN1W]), f32(p[kN1B]), (float)eps1,
+                             n1.data_ptr(), s.local ? f32(p[kLnW]) : nullptr, s.local ? f32(p[kLnB]) : nullptr, (float)eps_local,
+                             s.local ? nl.data_ptr() : nullptr, st));
+    Tensor pre, conv, loc;
+    if (s.local) {
+      pre = bf16_like(x, M); conv = bf16_like(x, M); loc = bf16_like(x, C);
+      check(m2d_linear_fwd(s.P, C, M, M2D_F32, nl.data_ptr(), f32(p[kPw1]), nullptr, M2D_ACT_NONE, nullptr, nullptr, M2D_ACT_NONE, nullptr,
+                           nullptr, pre.data_ptr(), st));
+      check(m2d_starrelu_dwconv3x3_fwd((int)s.B, (int)s.H, (int)s.W, M, M2D_F32, pre.data_ptr(), f32(p[kS1S]), f32(p[kS1B]), f32(p[kDw]),
+                                       conv.data_ptr(), st));
+      check(m2d_linear_fwd(s.P, M, C, M2D_F32, conv.data_ptr(), f32(p[kPw2]), nullptr, M2D_ACT_STARRELU, f32(p[kS2S]), f32(p[kS2B]),
+                           M2D_ACT_NONE, nullptr, nullptr, loc.data_ptr(), st));
+    }
+    Tensor u0 = bf16_like(x, C), u = bf16_like(x, C);
+    check(m2d_linear_keep_fwd(s.P, C, C, M2D_F32, n1.data_ptr(), f32(p[kInW]), f32(p[kInB]), M2D_ACT_GELU, nullptr, nullptr, u0.data_ptr(),
+                              u.data_ptr(), st));
+    auto pr = m2dshim::proj_fwd(u, p[kXProj], p[kDtTW], p[kDtTB], p[kDtLW], p[kDtLB], s.N, true, true);
+    auto [y, ck] = m2dshim::scan_fwd(u, pr[1], pr[2], p[kATLog], p[kALLog], pr[3], pr[4], pr[5], p[kD], save_ckpt && !full, flip, true, true,
+                                     interval);
+    Tensor mix = bf16_like(x, C);
+    check(m2d_linear_fwd(s.P, C, C, M2D_F32, y.data_ptr(), f32(p[kOutW]), f32(p[kOutB]), M2D_ACT_GELU, nullptr, nullptr, M2D_ACT_NONE, nullptr,
+                         nullptr, mix.data_ptr(), st));
+    Tensor x1 = at::empty_like(x), n2 = bf16_like(x, C);
+    check(m2d_train_norm_fwd(s.P, C, rps, f32(x), f32(p[kRs1]), mix.data_ptr(), s.local ? loc.data_ptr() : nullptr, opt(keep1),
+                             x1.data_ptr<float>(), f32(p[kN2W]), f32(p[kN2B]), (float)eps2, n2.data_ptr(), nullptr, nullptr, 0.f, nullptr, st));
+    Tensor h0 = bf16_like(x, HD), m = mix;      // (the mixer's answer has been added: its buffer takes the MLP's)
+    check(m2d_linear_fwd(s.P, C, HD, M2D_F32, n2.data_ptr(), f32(p[kFc1W]), f32(p[kFc1B]), M2D_ACT_NONE, nullptr, nullptr, M2D_ACT_NONE,
+                         nullptr, nullptr, h0.data_ptr(), st));
+    check(m2d_linear_fwd(s.P, HD, C, M2D_F32, h0.data_ptr(), f32(p[kFc2W]), f32(p[kFc2B]), M2D_ACT_GELU, nullptr, nullptr, M2D_ACT_NONE,
+                         nullptr, nullptr, m.data_ptr(), st));
+    Tensor x2 = at::empty_like(x);
+    check(m2d_train_norm_fwd(s.P, C, rps, f32(x1), f32(p[kRs2]), m.data_ptr(), nullptr, opt(keep2), x2.data_ptr<float>(), nullptr, nullptr, 0.f,
+                             nullptr, nullptr, nullptr, 0.f, nullptr, st));
+    variable_list saved = {x, n1, u0, u, y, x1, n2, h0, keep1.value_or(none), keep2.value_or(none), nl, pre, conv,
+                           full ? none : pr[0], full ? none : pr[1], full ? none : pr[2], full ? none : pr[3], full ? none : ck};
+    saved.insert(saved.end(), p.begin(), p.end());
+    ctx->save_for_backward(saved);
+    ctx->saved_data["eps"] = std::vector<double>{eps1, eps2, eps_local};
+    ctx->saved_data["flip"] = flip;
+    ctx->saved_data["full"] = full;
+    ctx->saved_data["interval"] = interval;
+    return x2;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &n1 = saved[1], &u0 = saved[2], &u = saved[3], &y = saved[4], &x1 = saved[5], &n2 = saved[6], &h0 = saved[7],
+                 &keep1 = saved[8], &keep2 = saved[9], &nl = saved[10], &pre = saved[11], &conv = saved[12];
+    const std::vector<Tensor> p(saved.begin() + 18, saved.end());
+    const Shape s = shape_of(x, p);
+    c10::DeviceGuard guard(x.device());
+    hipStream_t st = m2dshim::current_stream(x);
+    const int C = (int)s.C, M = 2 * C, HD = 4 * C, rps = (int)(s.H * s.W);
+    const auto eps = ctx->saved_data["eps"].toDoubleVector();
+    const bool flip = ctx->saved_data["flip"].toBool(), full = ctx->saved_data["full"].toBool();
+    const int64_t interval = ctx->saved_data["interval"].toInt();
+    Tensor dy = grads[0];
+    TORCH_CHECK(dy.scalar_type() == at::kFloat, "m2dscan: the gradient of a block's output must be float32, got ", dy.scalar_type());
+    dy = dy.contiguous();
+    if (reinterpret_cast<uintptr_t>(dy.data_ptr()) % 16) dy = dy.clone();
+
+    // one workspace for the workgroups' sums of all parameter gradients
+    std::vector<m2d_reduce_seg> segs;
+    std::vector<Tensor> out(p.size());
+    int64_t at = 0;
+    auto take = [&](int64_t n) { const int64_t o = at; at += (n + 63) / 64 * 64; return o; };
+    const int np = m2d_train_norm_parts(s.P, C);
+    const int64_t o_n2 = take((int64_t)np * 5 * C), o_n1 = take((int64_t)np * 5 * C);
+    struct W { int w, b, N, K, parts; int64_t off; };
+    std::vector<W> ws = {{kFc2W, kFc2B, C, HD, 0, 0}, {kFc1W, kFc1B, HD, C, 0, 0}, {kOutW, kOutB, C, C, 0, 0}, {kInW, kInB, C, C, 0, 0}};
+    if (s.local) { ws.push_back({kPw2, -1, C, M, 0, 0}); ws.push_back({kPw1, -1, M, C, 0, 0}); }
+    for (auto& w : ws) {
+      w.parts = m2d_train_wgrad_parts(s.P, w.N, w.K);
+      w.off = take((int64_t)w.parts * ((int64_t)w.N * w.K + w.N));
+    }
+    const int lp = s.local ? m2d_train_linear_parts(s.P, M, C) : 0, dp = s.local ? m2d_train_dwconv_parts((int)s.B, (int)s.H, (int)s.W, M) : 0;
+    TORCH_CHECK(!s.local || (lp > 0 && dp > 0), "m2dscan: block shapes outside what the training kernels are built for");
+    const int64_t o_s2 = take((int64_t)lp * 2), o_dw = take((int64_t)dp * (9 * M + 2));
+    Tensor part_t = at::empty({at}, x.options());
+    float* part = part_t.data_ptr<float>();
+    auto seg = [&](int i, int64_t off, int64_t stride, int parts) {
+      out[i] = at::empty_like(p[i]);
+      segs.push_back({part + off, out[i].data_ptr<float>(), stride, (int32_t)p[i].numel(), parts});
+    };
+    auto wgrad = [&](int i, const Tensor& g, const Tensor* z, const Tensor& in, int act, const float* as, const float* ab) {
+      const W& w = ws[i];
+      check(m2d_train_wgrad(s.P, w.N, w.K, g.data_ptr(), z ? z->data_ptr() : nullptr, z ? M2D_ACT_GELU : M2D_ACT_NONE, in.data_ptr(), act, as,
+                            ab, w.b >= 0, part + w.off, st));
+      const int64_t stride = (int64_t)w.N * w.K + w.N;
+      seg(w.w, w.off, stride, w.parts);
+      if (w.b >= 0) seg(w.b, w.off + (int64_t)w.N * w.K, stride, w.parts);
+    };
+    auto dgrad = [&](int K, int N, const Tensor& g, const Tensor* z, const Tensor& w, const Tensor* in, int act, const float* as, Tensor& dx,
+                     float* sums) {
+      check(m2d_train_linear_bwd(s.P, K, N, g.data_ptr(), z ? z->data_ptr() : nullptr, z ? M2D_ACT_GELU : M2D_ACT_NONE, f32(w),
+                                 in ? in->data_ptr() : nullptr, act, as, dx.data_ptr(), sums, st));
+    };
+
+    // MLP
+    Tensor dm = bf16_like(x, C), dh = bf16_like(x, HD), dn = bf16_like(x, C);
+    check(m2d_train_branch(s.P * C, (int64_t)rps * C, f32(dy), keep2.defined() ? f32(keep2) : nullptr, dm.data_ptr(), st));
+    dgrad(HD, C, dm, nullptr, p[kFc2W], &h0, M2D_ACT_GELU, nullptr, dh, nullptr);
+    wgrad(0, dm, nullptr, h0, M2D_ACT_GELU, nullptr, nullptr);
+    dgrad(C, HD, dh, nullptr, p[kFc1W], nullptr, M2D_ACT_NONE, nullptr, dn, nullptr);
+    wgrad(1, dh, nullptr, n2, M2D_ACT_NONE, nullptr, nullptr);
+    // second update and norm2; dm takes the gradient of the mixer's answer
+    Tensor dx1 = at::empty_like(x);
+    check(m2d_train_norm_bwd(s.P, C, rps, f32(x1), dn.data_ptr(), nullptr, f32(dy), f32(p[kRs2]), keep1.defined() ? f32(keep1) : nullptr,
+                             f32(p[kN2W]), f32(p[kN2B]), (float)eps[1], nullptr, 0.f, dx1.data_ptr<float>(), dm.data_ptr(), part + o_n2, st));
+    seg(kN2W, o_n2, 5 * C, np); seg(kN2B, o_n2 + C, 5 * C, np); seg(kRs2, o_n2 + 4 * C, 5 * C, np);
+    // local path
+    Tensor dl;
+    if (s.local) {
+      Tensor dc = bf16_like(x, M), dpre = bf16_like(x, M);
+      dl = bf16_like(x, C);
+      dgrad(M, C, dm, nullptr, p[kPw2], &conv, M2D_ACT_STARRELU, f32(p[kS2S]), dc, part + o_s2);
+      wgrad(4, dm, nullptr, conv, M2D_ACT_STARRELU, f32(p[kS2S]), f32(p[kS2B]));
+      seg(kS2S, o_s2, 2, lp); seg(kS2B, o_s2 + 1, 2, lp);
+      check(m2d_train_dwconv_bwd((int)s.B, (int)s.H, (int)s.W, M, pre.data_ptr(), dc.data_ptr(), f32(p[kDw]), f32(p[kS1S]), f32(p[kS1B]),
+                                 dpre.data_ptr(), part + o_dw, st));
+      seg(kDw, o_dw, 9 * M + 2, dp); seg(kS1S, o_dw + 9 * M, 9 * M + 2, dp); seg(kS1B, o_dw + 9 * M + 1, 9 * M + 2, dp);
+      dgrad(C, M, dpre, nullptr, p[kPw1], nullptr, M2D_ACT_NONE, nullptr, dl, nullptr);
+      wgrad(5, dpre, nullptr, nl, M2D_ACT_NONE, nullptr, nullptr);
+    }
+    // scan path
+    Tensor dyy = dn;
+    dgrad(C, C, dm, nullptr, p[kOutW], &y, M2D_ACT_GELU, nullptr, dyy, nullptr);
+    wgrad(2, dm, nullptr, y, M2D_ACT_GELU, nullptr, nullptr);
+    Tensor low, dT, dL, BC, ck;
+    const Tensor no_bc = at::empty({0}, u.options());
+    if (full) {
+      auto pr = m2dshim::proj_fwd(u, p[kXProj], p[kDtTW], p[kDtTB], p[kDtLW], p[kDtLB], s.N, true, true);
+      low = pr[0]; dT = pr[1]; dL = pr[2]; BC = pr[3];
+      ck = at::empty({1}, u.options().dtype(at::kByte));
+    } else {
+      low = saved[13]; dT = saved[14]; dL = saved[15]; BC = saved[16]; ck = saved[17];
+    }
+    auto g = m2dshim::scan_bwd(u, dT, dL, p[kATLog], p[kALLog], BC, no_bc, no_bc, p[kD], dyy, ck, flip, true, true, true, interval, true);
+    Tensor du = g[0];
+    out[kATLog] = g[3]; out[kALLog] = g[4]; out[kD] = g[8];
+    std::tie(out[kXProj], out[kDtTW], out[kDtTB], out[kDtLW], out[kDtLB]) =
+        m2dshim::proj_bwd(u, low, dT, dL, p[kXProj], p[kDtTW], p[kDtLW], g[1], g[2], g[5], g[6], g[7], du, true, true, g[5].size(0));
+    dgrad(C, C, du, &u0, p[kInW], nullptr, M2D_ACT_NONE, nullptr, dn, nullptr);
+    wgrad(3, du, &u0, n1, M2D_ACT_NONE, nullptr, nullptr);
+    // first update, norm1 and the local path's norm
+    Tensor dx = at::empty_like(x);
+    check(m2d_train_norm_bwd(s.P, C, rps, f32(x), dn.data_ptr(), s.local ? dl.data_ptr() : nullptr, f32(dx1), f32(p[kRs1]), nullptr, f32(p[kN1W]),
+                             f32(p[kN1B]), (float)eps[0], s.local ? f32(p[kLnW]) : nullptr, (float)eps[2], dx.data_ptr<float>(), nullptr,
+                             part + o_n1, st));
+    seg(kN1W, o_n1, 5 * C, np); seg(kN1B, o_n1 + C, 5 * C, np); seg(kRs1, o_n1 + 4 * C, 5 * C, np);
+    if (s.local) { seg(kLnW, o_n1 + 2 * C, 5 * C, np); seg(kLnB, o_n1 + 3 * C, 5 * C, np); }
+    check(m2d_train_reduce((int)segs.size(), segs.data(), st));
+
+    variable_list all = {dx};
+    all.insert(all.end(), out.begin(), out.end());
+    all.resize(all.size() + 9);      // keep1, keep2 and the seven options take none
+    return all;
+  }
+};
+
+Tensor train_block(const Tensor& x, at::TensorList par, const OptTensor& keep1, const OptTensor& keep2, double eps1, double eps2,
+                   double eps_local, bool flip, bool full, bool save_ckpt, int64_t interval) {
+  return Block::apply(x, par, keep1, keep2, eps1, eps2, eps_local, flip, full, save_ckpt, interval);
+}
+
+}  // namespace
+
+TORCH_LIBRARY_FRAGMENT(m2dscan, m) {
+  m.def("train_block(Tensor x, Tensor[] params, Tensor? keep1, Tensor? keep2, float eps1, float eps2, float eps_local, bool flip, "
+        "bool full, bool save_ckpt, int ckpt_interval) -> Tensor");
+}
+TORCH_LIBRARY_IMPL(m2dscan, AutogradCUDA, m) { m.impl("train_block", &train_block); }
+TORCH_LIBRARY_IMPL(m2dscan, CUDA, m) { m.impl("train_block", &train_block); }

@@ -16,82 +16,9 @@
 #include <stdint.h>
 
 #include "../../include/m2dscan.h"
+#include "m2dcommon.h"
 
 namespace {
-
-struct bf16_t { uint16_t v; };
-
-__device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {   // one v_cvt_pk_bf16_f32 (round to nearest even)
-  const f32x2_t v = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
-}
-
-// A chunk is 16 bytes of a row: kV elements.
-template <typename T> struct Chunk;
-template <> struct Chunk<float> {
-  static constexpr int kV = 4;
-  static __device__ __forceinline__ void load(const float* p, float (&v)[4]) {
-    const float4 q = *reinterpret_cast<const float4*>(p);
-    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-  }
-  static __device__ __forceinline__ void store(float* p, const float (&v)[4]) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  }
-  static __device__ __forceinline__ void store_rounded(float* p, float (&v)[4]) { store(p, v); }
-  static __device__ __forceinline__ void unpack(const uint4& q, float (&v)[4]) {
-    v[0] = __uint_as_float(q.x); v[1] = __uint_as_float(q.y); v[2] = __uint_as_float(q.z); v[3] = __uint_as_float(q.w);
-  }
-};
-template <> struct Chunk<bf16_t> {
-  static constexpr int kV = 8;
-  static __device__ __forceinline__ void load(const bf16_t* p, float (&v)[8]) {
-    const uint4 q = *reinterpret_cast<const uint4*>(p);
-    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { v[2 * j] = bf_lo(w[j]); v[2 * j + 1] = bf_hi(w[j]); }
-  }
-  static __device__ __forceinline__ void store(bf16_t* p, const float (&v)[8]) {
-    *reinterpret_cast<uint4*>(p) = make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
-  }
-  static __device__ __forceinline__ void unpack(const uint4& q, float (&v)[8]) {
-    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { v[2 * j] = bf_lo(w[j]); v[2 * j + 1] = bf_hi(w[j]); }
-  }
-  // stores v and leaves in v what a reader of p will find
-  static __device__ __forceinline__ void store_rounded(bf16_t* p, float (&v)[8]) {
-    const uint32_t w[4] = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
-    *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { v[2 * j] = bf_lo(w[j]); v[2 * j + 1] = bf_hi(w[j]); }
-  }
-};
-
-__device__ __forceinline__ float ldw(const void* w, int wbf16, int i) {
-  return wbf16 ? __uint_as_float((uint32_t)static_cast<const uint16_t*>(w)[i] << 16) : static_cast<const float*>(w)[i];
-}
-// V weights from index i0 on (a multiple of V, the array 16-byte aligned), in the fewest loads
-template <int V>
-__device__ __forceinline__ void ldwv(const void* w, int wbf16, int i0, float (&o)[V]) {
-  if (wbf16) {
-    if constexpr (V == 8) {
-      Chunk<bf16_t>::load(static_cast<const bf16_t*>(w) + i0, o);
-    } else {
-      const uint2 q = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(w) + i0);
-      o[0] = bf_lo(q.x); o[1] = bf_hi(q.x); o[2] = bf_lo(q.y); o[3] = bf_hi(q.y);
-    }
-  } else {
-#pragma unroll
-    for (int h = 0; h < V / 4; ++h) {
-      const float4 q = *reinterpret_cast<const float4*>(static_cast<const float*>(w) + i0 + 4 * h);
-      o[4 * h] = q.x; o[4 * h + 1] = q.y; o[4 * h + 2] = q.z; o[4 * h + 3] = q.w;
-    }
-  }
-}
 
 // ------------------------------------------------------------------------------------ LayerNorm
 // G lanes share a row (G a power of two, 4..64), lane g holds the chunks g, g + G, ... of it: at
@@ -229,7 +156,7 @@ int run_ln(const LnArgs& a, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------ depthwise 3x3, channel-last
-// y[b,h,w,c] = sum_{i,j} wt[c][i][j] x[b,h+i-1,w+j-1,c], zero padding.  A thread owns one chunk of
+// y[b,h,w,c] = sum_{i,j} wt[c][i][j] x[b,h+i-1,w+j-1,c], zero padding (STAR: of StarReLU(x)).  A thread owns one chunk of
 // channels and a strip of STRIP cells along W; the 3x3 window slides along the strip, so every
 // output costs three 16-byte loads plus the strip's two extra columns, and the 9 x kV weights of
 // the chunk stay in registers.  The kernel is bound by the number of loads: strips of 14 (which
@@ -243,9 +170,10 @@ struct DwArgs {
   void* y;
   int B, H, W, C, wbf16;
   int strips;       // strips per image row
+  const void *star_s, *star_b;   // STAR: scale and bias (one element each, type of w) of a StarReLU in front of the convolution
 };
 
-template <typename T, int STRIP>
+template <typename T, int STRIP, bool STAR = false>
 __global__ __launch_bounds__(kDwThreads) void m2d_dwconv3x3_kernel(const DwArgs a) {
   constexpr int V = Chunk<T>::kV;
   const int nchunks = a.C / V;
@@ -278,6 +206,25 @@ __global__ __launch_bounds__(kDwThreads) void m2d_dwconv3x3_kernel(const DwArgs 
   // the time).  Unpacked at every use: the conversions are cheap next to the registers a float window costs.
   constexpr int NS = kDwAhead + 2;      // columns held
   uint4 win[3][NS];
+  // STAR: a column passes through StarReLU when it becomes the window's right one, and is rounded as an activation
+  // kernel in front would have stored it; the padding around the image stays zero
+  float star_s = 0.f, star_b = 0.f;
+  if constexpr (STAR) { star_s = ldw(a.star_s, a.wbf16, 0); star_b = ldw(a.star_b, a.wbf16, 0); }
+  auto activate = [&](int col, int slot) {
+    if constexpr (STAR) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int hh = h + i - 1;
+        if (hh >= 0 && hh < a.H && col >= 0 && col < a.W) {
+          float v[V];
+          Chunk<T>::unpack(win[i][slot], v);
+#pragma unroll
+          for (int j = 0; j < V; ++j) { const float t = fmaxf(v[j], 0.f); v[j] = __builtin_fmaf(star_s * t, t, star_b); }
+          Chunk<T>::store(reinterpret_cast<T*>(&win[i][slot]), v);
+        }
+      }
+    }
+  };
   auto load_col = [&](int col, int slot) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -289,12 +236,15 @@ __global__ __launch_bounds__(kDwThreads) void m2d_dwconv3x3_kernel(const DwArgs 
   };
 #pragma unroll
   for (int k = 0; k <= kDwAhead; ++k) load_col(w0 - 1 + k, k);
+  activate(w0 - 1, 0);
+  activate(w0, 1);
 #pragma unroll
   for (int s = 0; s < STRIP; ++s) {
     const int w = w0 + s;
     if (w >= a.W) break;
     const int sl = s % NS, sm = (s + 1) % NS, sr = (s + 2) % NS;      // slots of columns w-1, w, w+1
     if (s + kDwAhead <= STRIP) load_col(w + kDwAhead, (s + kDwAhead + 1) % NS);
+    activate(w + 1, sr);
     float o[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) o[j] = 0.f;
@@ -473,30 +423,12 @@ int run_rope(const RopeArgs& a, int G, hipStream_t st) {
 // of 32), W's rows are the B operands (lane l: output l & 15, the same columns), results leave through a
 // per-wave LDS block so that memory sees 16-byte pieces of rows.  pre and post are nothing, GELU (exact
 // form, through erf) or StarReLU: the activation that the block applies before or after the layer.
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ f32x4_t mfma_bf16(uint4 a, uint4 b, f32x4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
-
 constexpr int kLinThreads = 256;
 constexpr int kLinWaves = 4;
 constexpr int kLinStage = 72;      // floats per row of a wave's result block: 64 + 8
 constexpr int kLinMaxKC = 16;      // steps of 32 along K: K <= 512
 enum { kActNone = 0, kActGelu = 1, kActStarRelu = 2, kActLayerNorm = 3 };   // the last one only before the layer, and only inside this file
 
-// erf by Abramowitz & Stegun 7.1.26 (absolute error below 1.5e-7), one v_exp_f32 and one v_rcp_f32
-__device__ __forceinline__ float gelu_exact(float v) {
-  const float z = fabsf(v) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.3275911f, z, 1.f));
-  float poly = __builtin_fmaf(t, 1.061405429f, -1.453152027f);
-  poly = __builtin_fmaf(t, poly, 1.421413741f);
-  poly = __builtin_fmaf(t, poly, -0.284496736f);
-  poly = __builtin_fmaf(t, poly, 0.254829592f);
-  const float e = 1.f - poly * t * __builtin_amdgcn_exp2f(-z * z * 1.44269504088896341f);   // erf(|v| / sqrt 2)
-  return 0.5f * v + 0.5f * fabsf(v) * e;                                                   // v erf(v/sqrt 2) = |v| erf(|v|/sqrt 2)
-}
 __device__ __forceinline__ float act(int kind, float v, float s, float b) {
   if (kind == kActGelu) return gelu_exact(v);
   if (kind == kActStarRelu) { const float t = fmaxf(v, 0.f); return __builtin_fmaf(s * t, t, b); }
@@ -557,6 +489,7 @@ struct LinArgs {
   const void *pre_s, *pre_b, *post_s, *post_b;   // StarReLU scale and bias (one element each, type of w) where pre / post is StarReLU
   const void *ln_w, *ln_b;                       // LayerNorm over the K inputs in front of the layer (pre == kActLayerNorm): weight and bias, (K), type of w
   float ln_eps;
+  void* z;              // (P, N) bf16 or null: the layer's output before post, for a caller whose backward wants its slope
 };
 
 template <int KCMAX>   // steps of 32 along K that the kernel is built for: 2, 4, 8 or 16
@@ -633,7 +566,7 @@ __global__ __launch_bounds__(kLinThreads) void m2d_linear_kernel(const LinArgs a
             if (kc < KC) acc = mfma_bf16(A[kc], ld16(wrow + 32 * kc), acc);
           const float bn = a.bias ? ldw(a.bias, a.wbf16, nbase + n) : 0.f;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] = act(a.post, acc[i] + bn, post_s, post_b);
+          for (int i = 0; i < 4; ++i) acc[i] = a.z ? acc[i] + bn : act(a.post, acc[i] + bn, post_s, post_b);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) stage[(4 * kb + i) * kLinStage + 16 * nt + mn] = acc[i];   // position 4 kb + i, output 16 nt + mn
@@ -644,8 +577,16 @@ __global__ __launch_bounds__(kLinThreads) void m2d_linear_kernel(const LinArgs a
       for (int k = 0; k < 2; ++k) {   // the block's 16 x 8 pieces of 8 outputs, two per lane
         const int piece = l + 64 * k, c = piece >> 3, c8 = 8 * (piece & 7);
         if (c < rows && n0 + c8 < a.Ns) {
-          const float4 lo = *reinterpret_cast<const float4*>(stage + c * kLinStage + c8);
-          const float4 hi = *reinterpret_cast<const float4*>(stage + c * kLinStage + c8 + 4);
+          float4 lo = *reinterpret_cast<const float4*>(stage + c * kLinStage + c8);
+          float4 hi = *reinterpret_cast<const float4*>(stage + c * kLinStage + c8 + 4);
+          if (a.z) {   // (uniform) both values leave; the activation reads what is stored, as the backward will
+            const uint4 q = make_uint4(pack_bf16(lo.x, lo.y), pack_bf16(lo.z, lo.w), pack_bf16(hi.x, hi.y), pack_bf16(hi.z, hi.w));
+            *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.z) + (p0 + c) * a.N + nbase + n0 + c8) = q;
+            lo = make_float4(act(a.post, bf_lo(q.x), post_s, post_b), act(a.post, bf_hi(q.x), post_s, post_b),
+                             act(a.post, bf_lo(q.y), post_s, post_b), act(a.post, bf_hi(q.y), post_s, post_b));
+            hi = make_float4(act(a.post, bf_lo(q.z), post_s, post_b), act(a.post, bf_hi(q.z), post_s, post_b),
+                             act(a.post, bf_lo(q.w), post_s, post_b), act(a.post, bf_hi(q.w), post_s, post_b));
+          }
           *reinterpret_cast<uint4*>(Y + (p0 + c) * a.N + nbase + n0 + c8) =
               make_uint4(pack_bf16(lo.x, lo.y), pack_bf16(lo.z, lo.w), pack_bf16(hi.x, hi.y), pack_bf16(hi.z, hi.w));
         }
@@ -792,8 +733,6 @@ inline bool allow_big_lds() {
 inline size_t linear_lds_bytes(int K, int N, bool ln = false) {
   return ((size_t)N * (K + 8) / 2 + 3) / 4 * 4 * 4 + (size_t)kLinWaves * 16 * kLinStage * 4 + (ln ? (size_t)2 * K * 4 : 0);
 }
-
-inline bool misaligned(const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) != 0; }
 
 // ------------------------------------------ attention of the rotary stages, one head per workgroup
 // softmax(q k^T / sqrt(hd)) v with q and k rotated by position and LayerNormed per head first
@@ -1014,16 +953,17 @@ int m2d_scale_residual_layernorm_fwd(int64_t rows, int C, int dtype, int weight_
   return dtype == M2D_F32 ? run_ln<float, true>(a, st) : run_ln<bf16_t, true>(a, st);
 }
 
-int m2d_dwconv3x3_fwd(int B, int H, int W, int C, int dtype, int weight_dtype, const void* x, const void* weight,
-                      void* y, void* stream) {
+static int run_dwconv(int B, int H, int W, int C, int dtype, int weight_dtype, const void* x, const void* weight, void* y,
+                      const void* star_scale, const void* star_bias, void* stream) {
   if (!x || !weight || !y) return M2D_ERR_NULL_POINTER;
   if (B < 1 || H < 1 || W < 1 || C < 1) return M2D_ERR_BAD_SHAPE;
   if ((dtype != M2D_F32 && dtype != M2D_BF16) || (weight_dtype != M2D_F32 && weight_dtype != M2D_BF16)) return M2D_ERR_UNSUPPORTED;
   const int V = dtype == M2D_BF16 ? 8 : 4;
   if (C % V != 0) return M2D_ERR_UNSUPPORTED;
   if (misaligned(x, 16) || misaligned(y, 16) || misaligned(weight, 16)) return M2D_ERR_MISALIGNED;
-  DwArgs a;
+  DwArgs a = {};
   a.x = x; a.w = weight; a.y = y; a.B = B; a.H = H; a.W = W; a.C = C; a.wbf16 = weight_dtype == M2D_BF16;
+  a.star_s = star_scale; a.star_b = star_bias;
   const int strip = W % 14 == 0 ? 14 : 8;
   a.strips = (W + strip - 1) / strip;
   const int64_t total = (int64_t)B * H * a.strips * (C / V);
@@ -1031,7 +971,10 @@ int m2d_dwconv3x3_fwd(int B, int H, int W, int C, int dtype, int weight_dtype, c
   if (blocks >= ((int64_t)1 << 31)) return M2D_ERR_UNSUPPORTED;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)blocks), block(kDwThreads);
-  if (dtype == M2D_F32) {
+  if (star_scale) {
+    if (strip == 14) hipLaunchKernelGGL((m2d_dwconv3x3_kernel<bf16_t, 14, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((m2d_dwconv3x3_kernel<bf16_t, 8, true>), grid, block, 0, st, a);
+  } else if (dtype == M2D_F32) {
     if (strip == 14) hipLaunchKernelGGL((m2d_dwconv3x3_kernel<float, 14>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((m2d_dwconv3x3_kernel<float, 8>), grid, block, 0, st, a);
   } else {
@@ -1039,6 +982,17 @@ int m2d_dwconv3x3_fwd(int B, int H, int W, int C, int dtype, int weight_dtype, c
     else hipLaunchKernelGGL((m2d_dwconv3x3_kernel<bf16_t, 8>), grid, block, 0, st, a);
   }
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
+}
+
+int m2d_dwconv3x3_fwd(int B, int H, int W, int C, int dtype, int weight_dtype, const void* x, const void* weight,
+                      void* y, void* stream) {
+  return run_dwconv(B, H, W, C, dtype, weight_dtype, x, weight, y, nullptr, nullptr, stream);
+}
+
+int m2d_starrelu_dwconv3x3_fwd(int B, int H, int W, int C, int weight_dtype, const void* x, const void* star_scale,
+                               const void* star_bias, const void* weight, void* y, void* stream) {
+  if (!star_scale || !star_bias) return M2D_ERR_NULL_POINTER;
+  return run_dwconv(B, H, W, C, M2D_BF16, weight_dtype, x, weight, y, star_scale, star_bias, stream);
 }
 
 int m2d_starrelu_fwd(int64_t n, int dtype, int weight_dtype, const void* x, const void* scale, const void* bias, void* y,
@@ -1158,7 +1112,8 @@ int m2d_rope_attention_fwd(int B, int L, int heads, int head_dim, int weight_dty
 
 static int run_linear(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias,
                       int pre_act, const void* pre_scale, const void* pre_bias, int post_act, const void* post_scale,
-                      const void* post_bias, void* y, void* stream, const void* ln_w, const void* ln_b, float ln_eps) {
+                      const void* post_bias, void* y, void* stream, const void* ln_w, const void* ln_b, float ln_eps,
+                      void* z = nullptr) {
   if (!x || !weight || !y) return M2D_ERR_NULL_POINTER;
   const bool ln = pre_act == kActLayerNorm;
   if (ln && (!ln_w || !ln_b)) return M2D_ERR_NULL_POINTER;
@@ -1183,7 +1138,7 @@ static int run_linear(int64_t P, int K, int N, int weight_dtype, const void* x, 
   a.x = x; a.w = weight; a.bias = bias; a.y = y; a.P = P; a.K = K; a.N = N; a.wbf16 = weight_dtype == M2D_BF16;
   a.pre = pre_act; a.post = post_act; a.pre_s = pre_scale; a.pre_b = pre_bias; a.post_s = post_scale; a.post_b = post_bias;
   a.ntiles = (int)((P + 63) / 64);
-  a.nsplit = nsplit; a.Ns = Ns;
+  a.nsplit = nsplit; a.Ns = Ns; a.z = z;
   const size_t lds = linear_lds_bytes(K, Ns, ln);
   if (lds > 64 * 1024 && !allow_big_lds()) return M2D_ERR_HIP;
   // persistent: the weights are loaded into LDS once per workgroup; as many workgroups as fit the device at once
@@ -1208,6 +1163,14 @@ int m2d_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, con
   if (pre_act == kActLayerNorm) return M2D_ERR_UNSUPPORTED;      // that one has an entry point of its own
   return run_linear(P, K, N, weight_dtype, x, weight, bias, pre_act, pre_scale, pre_bias, post_act, post_scale, post_bias, y, stream,
                     nullptr, nullptr, 0.f);
+}
+
+int m2d_linear_keep_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias,
+                        int post_act, const void* post_scale, const void* post_bias, void* z, void* y, void* stream) {
+  if (!z) return M2D_ERR_NULL_POINTER;
+  if (misaligned(z, 16)) return M2D_ERR_MISALIGNED;
+  return run_linear(P, K, N, weight_dtype, x, weight, bias, kActNone, nullptr, nullptr, post_act, post_scale, post_bias, y, stream,
+                    nullptr, nullptr, 0.f, z);
 }
 
 int m2d_layernorm_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias,

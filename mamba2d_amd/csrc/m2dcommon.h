@@ -1,0 +1,107 @@
+// m2dcommon.h -- device helpers shared by the kernels of a residual block (m2dblock.hip, m2dtrain.hip): bf16 <-> fp32,
+// 16-byte chunks of a row, weights of either type, the bf16 matrix product, GELU.
+#ifndef M2D_COMMON_H
+#define M2D_COMMON_H
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace {
+
+struct bf16_t { uint16_t v; };
+
+__device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {   // one v_cvt_pk_bf16_f32 (round to nearest even)
+  const f32x2_t v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+}
+
+// A chunk is 16 bytes of a row: kV elements.
+template <typename T> struct Chunk;
+template <> struct Chunk<float> {
+  static constexpr int kV = 4;
+  static __device__ __forceinline__ void load(const float* p, float (&v)[4]) {
+    const float4 q = *reinterpret_cast<const float4*>(p);
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+  }
+  static __device__ __forceinline__ void store(float* p, const float (&v)[4]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  static __device__ __forceinline__ void store_rounded(float* p, float (&v)[4]) { store(p, v); }
+  static __device__ __forceinline__ void unpack(const uint4& q, float (&v)[4]) {
+    v[0] = __uint_as_float(q.x); v[1] = __uint_as_float(q.y); v[2] = __uint_as_float(q.z); v[3] = __uint_as_float(q.w);
+  }
+};
+template <> struct Chunk<bf16_t> {
+  static constexpr int kV = 8;
+  static __device__ __forceinline__ void load(const bf16_t* p, float (&v)[8]) {
+    const uint4 q = *reinterpret_cast<const uint4*>(p);
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { v[2 * j] = bf_lo(w[j]); v[2 * j + 1] = bf_hi(w[j]); }
+  }
+  static __device__ __forceinline__ void store(bf16_t* p, const float (&v)[8]) {
+    *reinterpret_cast<uint4*>(p) = make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
+  }
+  static __device__ __forceinline__ void unpack(const uint4& q, float (&v)[8]) {
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { v[2 * j] = bf_lo(w[j]); v[2 * j + 1] = bf_hi(w[j]); }
+  }
+  // stores v and leaves in v what a reader of p will find
+  static __device__ __forceinline__ void store_rounded(bf16_t* p, float (&v)[8]) {
+    const uint32_t w[4] = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+    *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { v[2 * j] = bf_lo(w[j]); v[2 * j + 1] = bf_hi(w[j]); }
+  }
+};
+
+__device__ __forceinline__ float ldw(const void* w, int wbf16, int i) {
+  return wbf16 ? __uint_as_float((uint32_t)static_cast<const uint16_t*>(w)[i] << 16) : static_cast<const float*>(w)[i];
+}
+// V weights from index i0 on (a multiple of V, the array 16-byte aligned), in the fewest loads
+template <int V>
+__device__ __forceinline__ void ldwv(const void* w, int wbf16, int i0, float (&o)[V]) {
+  if (wbf16) {
+    if constexpr (V == 8) {
+      Chunk<bf16_t>::load(static_cast<const bf16_t*>(w) + i0, o);
+    } else {
+      const uint2 q = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(w) + i0);
+      o[0] = bf_lo(q.x); o[1] = bf_hi(q.x); o[2] = bf_lo(q.y); o[3] = bf_hi(q.y);
+    }
+  } else {
+#pragma unroll
+    for (int h = 0; h < V / 4; ++h) {
+      const float4 q = *reinterpret_cast<const float4*>(static_cast<const float*>(w) + i0 + 4 * h);
+      o[4 * h] = q.x; o[4 * h + 1] = q.y; o[4 * h + 2] = q.z; o[4 * h + 3] = q.w;
+    }
+  }
+}
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4_t mfma_bf16(uint4 a, uint4 b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
+
+
+// erf by Abramowitz & Stegun 7.1.26 (absolute error below 1.5e-7), one v_exp_f32 and one v_rcp_f32
+__device__ __forceinline__ float gelu_exact(float v) {
+  const float z = fabsf(v) * 0.70710678118654752f;
+  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.3275911f, z, 1.f));
+  float poly = __builtin_fmaf(t, 1.061405429f, -1.453152027f);
+  poly = __builtin_fmaf(t, poly, 1.421413741f);
+  poly = __builtin_fmaf(t, poly, -0.284496736f);
+  poly = __builtin_fmaf(t, poly, 0.254829592f);
+  const float e = 1.f - poly * t * __builtin_amdgcn_exp2f(-z * z * 1.44269504088896341f);   // erf(|v| / sqrt 2)
+  return 0.5f * v + 0.5f * fabsf(v) * e;                                                   // v erf(v/sqrt 2) = |v| erf(|v|/sqrt 2)
+}
+
+inline bool misaligned(const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) != 0; }
+
+}  // namespace
+#endif

@@ -50,6 +50,7 @@ rope_attention_fwd_op = torch.ops.m2dscan.rope_attention_fwd
 mlp_fwd_op = torch.ops.m2dscan.mlp_fwd
 linear_act_fwd_op = torch.ops.m2dscan.linear_act_fwd
 layernorm_linear_act_fwd_op = torch.ops.m2dscan.layernorm_linear_act_fwd
+train_block_op = torch.ops.m2dscan.train_block
 
 # Keep the forward's anti-diagonal checkpoints for the backward (faster backward, more saved
 # memory) or rebuild them inside the backward (nothing saved beyond the inputs, like the
