@@ -357,6 +357,12 @@ int m2d_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, con
                    int pre_act, const void* pre_scale, const void* pre_bias,
                    int post_act, const void* post_scale, const void* post_bias, void* y, void* stream);
 
+/* y = post(x weight^T + bias) for wide layers and few positions (P (P,K) and (P,N) bf16, post_act nothing or GELU of the
+ * layer's output rounded to bf16): K and N multiples of 32, any size.  Reads its operands straight from memory, made for
+ * the latency of a few hundred positions; beyond about a thousand a tiled product is faster. */
+int m2d_wide_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias, int post_act,
+                        void* y, void* stream);
+
 /* m2d_linear_fwd (no pre_act) that also keeps the layer's output before the activation: z (P,N) bf16, y = post(z). */
 int m2d_linear_keep_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias,
                         int post_act, const void* post_scale, const void* post_bias, void* z, void* y, void* stream);
@@ -384,6 +390,15 @@ int m2d_layernorm_linear_fwd(int64_t P, int K, int N, int weight_dtype, const vo
 int m2d_mlp_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x,
                 const void* ln_weight, const void* ln_bias, float eps,
                 const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream);
+
+/* bf16 -> fp32 for up to 64 arrays of n elements per launch: the parameters of a model held in bf16, for the calls that
+ * take fp32 parameters. */
+typedef struct m2d_widen_seg {
+  const void* in;
+  float* out;
+  int64_t n;
+} m2d_widen_seg;
+int m2d_widen(int nsegs, const m2d_widen_seg* segs, void* stream);
 
 /* ---- Operators of a residual block in training (models/mamba2d.py:191-254, models/utils.py:58-118), bf16-mixed:
  * the residual stream x, its gradient and all parameters are fp32, everything between the norms and the residual

@@ -17,6 +17,8 @@ Differences in how it runs (not in what it computes):
   * the rotary tables of the attention stages are built once per grid size.
 """
 import math
+import operator
+import weakref
 
 import torch
 import torch.nn as nn
@@ -25,8 +27,8 @@ import torch.nn.functional as F
 from . import wavefront
 from .wavefront import (dwconv3x3_fwd_op, layernorm_fwd_op, layernorm_linear_act_fwd_op, linear_act_fwd_op, mlp_fwd_op,
                         rope_qknorm_fwd_op,
-                        rope_attention_fwd_op, scale_residual_fwd_op, scale_residual_layernorm_fwd_op, starrelu_fwd_op,
-                        train_block_op, wavefront_scan_cuda)
+                        infer_stage_op, rope_attention_fwd_op, scale_residual_fwd_op, scale_residual_layernorm_fwd_op,
+                        starrelu_fwd_op, train_block_op, wavefront_scan_cuda)
 
 M2D_T = dict(n_blocks=(3, 3, 9, 3), embed_dim=(64, 128, 320, 512),
              token_mixer=("2D_local", "2D_local", "RopeAttention", "RopeAttention"),
@@ -433,6 +435,40 @@ class ResBlock(nn.Module):
             return None
         return par
 
+    def _infer_parameters(self, x):
+        """(kind, parameters in the order of ``m2dscan::infer_stage``, eps of norm1, norm2 and the mixer's own norm) for a
+        block whose inference is that operator's sequence of kernels; None otherwise."""
+        mix, mlp = self.token_mixer, self.MLP
+        n1, n2, s1, s2, fc1, fc2 = self.norm1, self.norm2, self.res_scale1, self.res_scale2, mlp.fc1, mlp.fc2
+        if not (_plain(mlp, MLP) and type(s1) is Scale and type(s2) is Scale and type(n1) is LayerNorm and type(n2) is LayerNorm
+                and _plain(fc1, nn.Linear) and _plain(fc2, nn.Linear)):
+            return None
+        tail = [s1.scale, n2.weight, n2.bias, fc1.weight, fc1.bias, fc2.weight, fc2.bias, s2.scale]
+        if _plain(mix, RoPEAttention2D):
+            qn, kn = mix.q_norm, mix.k_norm
+            if not (mix.head_dim == 32 and qn.eps == kn.eps and _plain(mix.qkv, nn.Linear)
+                    and _plain(mix.proj, nn.Linear) and mix.qkv.bias is None and mix.proj.bias is None):
+                return None
+            return 4, [n1.weight, n1.bias, mix.qkv.weight, qn.weight, qn.bias, kn.weight, kn.bias, mix.proj.weight, *tail], (n1.eps, n2.eps, qn.eps)
+        if not (_plain(mix, M2DBlock) and _plain(mix.in_proj, nn.Linear) and _plain(mix.out_proj, nn.Linear)
+                and mix.recomp in ("partial", "full") and mix.x_proj.bias is None and mix.AT_log.shape[1] == wavefront.STATES_PER_CALL and mix.dt_projT.weight.shape[1] <= 32):
+            return None
+        par = [n1.weight, n1.bias, mix.in_proj.weight, mix.in_proj.bias, mix.AT_log, mix.AL_log, mix.x_proj.weight, mix.dt_projT.weight,
+               mix.dt_projT.bias, mix.dt_projL.weight, mix.dt_projL.bias, mix.D, mix.out_proj.weight, mix.out_proj.bias, *tail]
+        path = mix.local_path
+        if path is None:
+            return int(mix.flip), par, (n1.eps, n2.eps, 0.0)
+        conv = path.dwconv
+        if not (_plain(path, SepConv) and type(mix.local_norm) is LayerNorm and _plain(path.pwconv1, nn.Linear) and _plain(path.pwconv2, nn.Linear)
+                and type(conv) is nn.Conv2d and conv.kernel_size == (3, 3) and conv.padding == (1, 1) and conv.stride == (1, 1)
+                and conv.dilation == (1, 1) and conv.bias is None and conv.padding_mode == "zeros" and type(path.act1) is StarReLU
+                and type(path.act2) is StarReLU and path.pwconv1.bias is None and path.pwconv2.bias is None
+                and path.pwconv1.weight.shape[0] <= 256):      # (StarReLU joins the kernels of narrow layers only)
+            return None
+        par += [mix.local_norm.weight, mix.local_norm.bias, path.pwconv1.weight, path.act1.scale, path.act1.bias, conv.weight,
+                path.act2.scale, path.act2.bias, path.pwconv2.weight]
+        return 2 + int(mix.flip), par, (n1.eps, n2.eps, mix.local_norm.eps)
+
     def forward_fused(self, x, normed=None, next_norm=None):
         """The block on x, with ``normed`` = norm1(x) where the caller has it already; returns the block's output
         and ``next_norm`` of it (None without ``next_norm``): the LayerNorm that follows the block, computed in
@@ -462,6 +498,100 @@ class ResBlock(nn.Module):
 
     def forward(self, x):
         return self.forward_fused(x)[0]
+
+
+def _module_ops():
+    return (dwconv3x3_fwd_op, layernorm_fwd_op, layernorm_linear_act_fwd_op, linear_act_fwd_op, mlp_fwd_op, rope_attention_fwd_op,
+            scale_residual_fwd_op, scale_residual_layernorm_fwd_op, wavefront_scan_cuda)
+
+
+_OWN_OPS = _module_ops()
+
+
+class _StagePlan:
+    """What a stage's call needs and everything it was read from: the parameters, the modules and options in between, the
+    hooks.  Looking all of that up again is what a call would mostly be on one image (420 us of 1640); comparing it, object
+    by object, with what is there now takes a tenth."""
+
+    OPTIONS = ("training", "eps", "flip", "recomp", "kernel_size", "padding", "stride", "dilation", "padding_mode", "head_dim", "num_heads",
+               "rope_base", "axis_dim", "normalized_shape")
+
+    def __init__(self, stage, kinds, par, eps, att):
+        self.kinds, self.par, self.eps, self.att = kinds, par, eps, att
+        self.own, self.keys, self.was, self.hooks = [], [], [], []
+        for m in stage.modules():
+            d = m.__dict__
+            for own in (m._modules, m._parameters, {k: d[k] for k in self.OPTIONS if k in d}):
+                for k, v in own.items():
+                    self.own.append(own if own is m._modules or own is m._parameters else d)
+                    self.keys.append(k)
+                    self.was.append(v)
+            self.own.append(d)
+            self.keys.append("_modules")
+            self.was.append(m._modules)
+            self.hooks += [m._forward_hooks, m._forward_pre_hooks, m._backward_hooks, m._backward_pre_hooks]
+
+    def holds(self, stage):
+        try:
+            return (all(map(operator.is_, map(operator.getitem, self.own, self.keys), self.was)) and not any(self.hooks)
+                    and len(stage) == len(self.kinds) + 1)
+        except KeyError:
+            return False
+
+
+_STAGE_PLANS = weakref.WeakKeyDictionary()
+
+
+def _stage_plan(stage, x):
+    mods = list(stage)
+    end = mods[-1]
+    if type(end) is not LayerNorm or end.weight is None or end.bias is None or end.training:
+        return None
+    kinds, par, eps, att = [], [], [], None
+    for m in mods[:-1]:
+        got = m._infer_parameters(x) if type(m) is ResBlock and not m.training else None
+        if got is None:
+            return None
+        kinds.append(got[0])
+        par += got[1]
+        eps += got[2]
+        if got[0] == 4:
+            if att is not None and (att.rope_base, att.axis_dim) != (m.token_mixer.rope_base, m.token_mixer.axis_dim):
+                return None
+            att = m.token_mixer
+    par += [end.weight, end.bias]
+    eps.append(end.eps)
+    if any(t is None for t in par):
+        return None
+    return _StagePlan(stage, kinds, par, eps, att)
+
+
+def _infer_stage(stage, x):
+    """A stage (residual blocks and the LayerNorm behind them) at inference on bf16 activations as one call: the kernels
+    that the modules would run, in their order, without Python in between.  None where a module asks for something
+    else (gradients, training mode, hooks, foreign modules, parameters of mixed types), or where somebody has put
+    another operator in the place of one that the call stands for (to count or to time it)."""
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 4 and x.numel() > 0 and x.is_contiguous() and len(stage) > 1
+            and x.shape[3] % 16 == 0 and x.shape[3] <= 512 and not torch.compiler.is_compiling()):
+        return None
+    if _module_ops() != _OWN_OPS or not wavefront.FUSED_PROJECTIONS:
+        return None
+    plan = _STAGE_PLANS.get(stage)
+    if plan is None or not plan.holds(stage):
+        plan = _stage_plan(stage, x)
+        if plan is None:
+            return None
+        _STAGE_PLANS[stage] = plan
+    att, dtype = plan.att, plan.par[0].dtype
+    if not _inference(x, *(plan.par if torch.is_grad_enabled() else ())) or x.shape[1] < 2 or x.shape[2] < 2:
+        return None
+    cos = sin = x
+    if att is not None:
+        if x.shape[1] * x.shape[2] > 256 or (dtype == torch.float32 and not torch.is_autocast_enabled("cuda")):
+            return None      # (larger grids take another attention; fp32 weights meet bf16 activations only under autocast)
+        cos, sin = att._rope_tables(x.shape[1], x.shape[2], x.device, x.dtype)
+    out = infer_stage_op(x, plan.par, plan.kinds, plan.eps, cos, sin, 32 ** -0.5)
+    return out if out.numel() else None      # (empty: parameters of mixed types or devices)
 
 
 class Mamba2DBackbone(nn.Module):
@@ -499,6 +629,9 @@ class Mamba2DBackbone(nn.Module):
     def _run_stage(stage, x):
         """The stage's modules in order; a block is handed the LayerNorm that follows it (the next block's norm1 or
         the norm that ends the stage) so that it can compute it together with its last residual update."""
+        fast = _infer_stage(stage, x)
+        if fast is not None:
+            return fast
         mods = list(stage)
         normed = None
         for i, m in enumerate(mods):

@@ -101,11 +101,11 @@ def build_lib(verbose: bool = True) -> str:
 
 
 def build_shim(verbose: bool = True) -> str:
-    """Compile csrc/m2d_torch.cpp and m2d_train.cpp (host only) against torch and link it to libm2dscan.so."""
+    """Compile the csrc/m2d_*.cpp (host only) against torch and link it to libm2dscan.so."""
     import torch
     from torch.utils import cpp_extension as ce
 
-    src = [os.path.join(HERE, "csrc", name) for name in ("m2d_torch.cpp", "m2d_train.cpp")]
+    src = [os.path.join(HERE, "csrc", name) for name in ("m2d_torch.cpp", "m2d_train.cpp", "m2d_infer.cpp")]
     inc = [f"-I{p}" for p in ce.include_paths(device_type="cuda")] + [f"-I{os.path.join(ROOT, 'include')}"]
     libdirs = ce.library_paths(device_type="cuda")
     cmd = ["hipcc", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",

@@ -30,7 +30,7 @@ EXPORTS = ("m2d_version", "m2d_status_str", "m2d_desc_check", "m2d_scan_workspac
            "m2d_scan_ckpt_bytes", "m2d_scan_fwd", "m2d_scan_fwd_noalloc", "m2d_scan_link_error", "m2d_scan_plan", "m2d_scan_bwd", "m2d_proj_workspace_bytes", "m2d_proj_fwd",
            "m2d_proj_bwd", "m2d_proj_bwd_parts", "m2d_scan_sum_parts", "m2d_layernorm_fwd", "m2d_dwconv3x3_fwd", "m2d_starrelu_fwd",
            "m2d_scale_residual_fwd", "m2d_scale_residual_layernorm_fwd", "m2d_rope_qknorm_fwd", "m2d_rope_attention_fwd", "m2d_mlp_fwd", "m2d_layernorm_linear_fwd", "m2d_linear_fwd", "m2d_profile_enable", "m2d_profile_last_ms", "m2d_valu_rate_probe", "m2d_wf_fwd", "m2d_wf_bwd",
-           "m2d_linear_keep_fwd", "m2d_starrelu_dwconv3x3_fwd", "m2d_train_norm_fwd", "m2d_train_norm_parts", "m2d_train_norm_bwd",
+           "m2d_widen", "m2d_wide_linear_fwd", "m2d_linear_keep_fwd", "m2d_starrelu_dwconv3x3_fwd", "m2d_train_norm_fwd", "m2d_train_norm_parts", "m2d_train_norm_bwd",
            "m2d_train_branch", "m2d_train_dwconv_parts", "m2d_train_dwconv_bwd", "m2d_train_linear_parts", "m2d_train_linear_bwd",
            "m2d_train_wgrad_parts", "m2d_train_wgrad", "m2d_train_reduce")
 
@@ -92,6 +92,8 @@ def _load():
     lib.m2d_layernorm_fwd.argtypes = [ctypes.c_int64, i32, i32, i32, vp, vp, vp, ctypes.c_float, vp, vp]
     lib.m2d_dwconv3x3_fwd.restype = i32
     lib.m2d_dwconv3x3_fwd.argtypes = [i32, i32, i32, i32, i32, i32, vp, vp, vp, vp]
+    lib.m2d_wide_linear_fwd.restype = i32
+    lib.m2d_wide_linear_fwd.argtypes = [ctypes.c_int64, i32, i32, i32, vp, vp, vp, i32, vp, vp]
     lib.m2d_starrelu_fwd.restype = i32
     lib.m2d_starrelu_fwd.argtypes = [ctypes.c_int64, i32, i32, vp, vp, vp, vp, vp]
     lib.m2d_scale_residual_layernorm_fwd.restype = i32
@@ -446,6 +448,23 @@ def scale_residual_layernorm_fwd(x, scale, residual, residual2, weight, bias, ep
                                                _ptr(residual), None if residual2 is None else _ptr(residual2), _ptr(weight),
                                                _ptr(bias), float(eps), _ptr(xo), _ptr(y), _stream(x.device)))
     return xo, y
+
+
+def wide_linear_fwd(x, weight, bias=None, gelu=False):
+    """gelu(x weight^T + bias) or the layer alone on a contiguous bf16 (..., K) tensor, through m2d_wide_linear_fwd."""
+    K = x.shape[-1]
+    if not x.is_cuda or not x.is_contiguous() or x.dtype != torch.bfloat16:
+        raise ValueError("m2dscan: x must be a contiguous bfloat16 tensor on the GPU")
+    if weight.dim() != 2 or weight.shape[1] != K or (bias is not None and tuple(bias.shape) != (weight.shape[0],)):
+        raise ValueError(f"m2dscan: weight must be (N,{K}) and bias (N,)")
+    for t in (weight, bias):
+        if t is not None and (t.device != x.device or not t.is_contiguous() or t.dtype != weight.dtype):
+            raise ValueError(f"m2dscan: weight and bias must be contiguous tensors of one dtype on {x.device}")
+    N = weight.shape[0]
+    y = x.new_empty((*x.shape[:-1], N))
+    check(lib.m2d_wide_linear_fwd(x.numel() // K, K, N, _dtype_code(weight), _ptr(x), _ptr(weight), None if bias is None else _ptr(bias),
+                                  int(gelu), _ptr(y), _stream(x.device)))
+    return y
 
 
 def mlp_fwd(x, w1, b1, w2, b2, ln_weight=None, ln_bias=None, eps=1e-5):

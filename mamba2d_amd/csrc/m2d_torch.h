@@ -30,5 +30,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> proj_bwd(const Tensor& x, con
                                                             const Tensor& ddL, const Tensor& dBT, const Tensor& dBL, const Tensor& dC,
                                                             Tensor dx, bool round_weights, bool dpre, int64_t sum_parts);
 
+std::vector<Tensor> widen(at::TensorList in);      // m2d_infer.cpp
+
 }  // namespace m2dshim
 #endif

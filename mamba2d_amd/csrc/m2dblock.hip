@@ -14,6 +14,7 @@
 
 #include <atomic>
 #include <stdint.h>
+#include <type_traits>
 
 #include "../../include/m2dscan.h"
 #include "m2dcommon.h"
@@ -40,7 +41,9 @@ struct LnArgs {
   void* xo;
 };
 
-template <typename T, int G, int NC, bool RES>
+// WB: the weights are bf16.  A template, not a branch at every load: with the branch the loads of a lane's weights waited
+// for each other, 7 us for the 196 rows of one image where the whole kernel now takes 4.
+template <typename T, int G, int NC, bool RES, bool WB>
 __global__ __launch_bounds__(kLnThreads) void m2d_layernorm_kernel(const LnArgs a) {
   constexpr int V = Chunk<T>::kV;
   const int lane_in_row = threadIdx.x & (G - 1);
@@ -56,8 +59,8 @@ __global__ __launch_bounds__(kLnThreads) void m2d_layernorm_kernel(const LnArgs 
 #pragma unroll
     for (int j = 0; j < V; ++j) { wv[k][j] = 0.f; bv[k][j] = 0.f; }
     if (c < nchunks) {
-      ldwv<V>(a.w, a.wbf16, c * V, wv[k]);
-      ldwv<V>(a.b, a.wbf16, c * V, bv[k]);
+      ldwv<V>(a.w, WB, c * V, wv[k]);
+      ldwv<V>(a.b, WB, c * V, bv[k]);
     }
   }
   float sv[RES ? NC : 1][V];
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(kLnThreads) void m2d_layernorm_kernel(const LnArgs 
       const int c = lane_in_row + k * G;
 #pragma unroll
       for (int j = 0; j < V; ++j) sv[k][j] = 0.f;
-      if (c < nchunks) ldwv<V>(a.s, a.wbf16, c * V, sv[k]);
+      if (c < nchunks) ldwv<V>(a.s, WB, c * V, sv[k]);
     }
   }
   const T* X = static_cast<const T*>(a.x);
@@ -136,7 +139,8 @@ int launch_ln(const LnArgs& a, hipStream_t st) {
   constexpr int kRows = kLnThreads / G;
   int64_t blocks = (a.rows + kRows - 1) / kRows;
   if (blocks > 256 * 8) blocks = 256 * 8;   // grid-stride beyond that: the lane's weights are loaded once and serve several rows
-  hipLaunchKernelGGL((m2d_layernorm_kernel<T, G, NC, RES>), dim3((unsigned)blocks), dim3(kLnThreads), 0, st, a);
+  if (a.wbf16) hipLaunchKernelGGL((m2d_layernorm_kernel<T, G, NC, RES, true>), dim3((unsigned)blocks), dim3(kLnThreads), 0, st, a);
+  else hipLaunchKernelGGL((m2d_layernorm_kernel<T, G, NC, RES, false>), dim3((unsigned)blocks), dim3(kLnThreads), 0, st, a);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
 }
 
@@ -478,6 +482,43 @@ __device__ __forceinline__ void norm_rows(uint4 (&A)[KCMAX], int KC, int K, cons
     }
 }
 
+// Pieces 0 .. pieces-1 of 8 weights from element `first` on, as bf16, to put(piece, value): kStageAhead loads of a thread in
+// flight (one at a time, staging was most of the 8 us that such a layer took on one image's rows).
+constexpr int kStageAhead = 4;
+template <typename PUT>
+__device__ __forceinline__ void stage_rows(const void* w, int wbf16, int64_t first, int pieces, int tid, PUT&& put) {
+  if (wbf16) {
+    const uint16_t* src = static_cast<const uint16_t*>(w) + first;
+    for (int i0 = tid; i0 < pieces; i0 += kStageAhead * kLinThreads) {
+      uint4 q[kStageAhead];
+#pragma unroll
+      for (int k = 0; k < kStageAhead; ++k) {
+        const int i = i0 + k * kLinThreads;
+        q[k] = ld16(src + (int64_t)8 * (i < pieces ? i : i0));
+      }
+#pragma unroll
+      for (int k = 0; k < kStageAhead; ++k)
+        if (i0 + k * kLinThreads < pieces) put(i0 + k * kLinThreads, q[k]);
+    }
+  } else {
+    const float* src = static_cast<const float*>(w) + first;
+    for (int i0 = tid; i0 < pieces; i0 += kStageAhead * kLinThreads) {
+      float4 lo[kStageAhead], hi[kStageAhead];
+#pragma unroll
+      for (int k = 0; k < kStageAhead; ++k) {
+        const int i = i0 + k * kLinThreads;
+        const float* p = src + (int64_t)8 * (i < pieces ? i : i0);
+        lo[k] = *reinterpret_cast<const float4*>(p);
+        hi[k] = *reinterpret_cast<const float4*>(p + 4);
+      }
+#pragma unroll
+      for (int k = 0; k < kStageAhead; ++k)
+        if (i0 + k * kLinThreads < pieces)
+          put(i0 + k * kLinThreads, make_uint4(pack_bf16(lo[k].x, lo[k].y), pack_bf16(lo[k].z, lo[k].w), pack_bf16(hi[k].x, hi[k].y), pack_bf16(hi[k].z, hi[k].w)));
+    }
+  }
+}
+
 struct LinArgs {
   const void* x;        // (P, K) bf16
   const void* w;        // (N, K)
@@ -502,17 +543,11 @@ __global__ __launch_bounds__(kLinThreads) void m2d_linear_kernel(const LinArgs a
   float* stage = smem + (a.Ns * ws / 2 + 3) / 4 * 4 + wave * 16 * kLinStage;
   const int slice = blockIdx.x % a.nsplit, nbase = slice * a.Ns;   // this workgroup's outputs: nbase .. nbase + Ns
   const int first_tile = blockIdx.x / a.nsplit, tile_step = gridDim.x / a.nsplit;
-  for (int i = tid; i < a.Ns * (a.K / 8); i += kLinThreads) {
-    const int n = i / (a.K / 8), k8 = i - n * (a.K / 8);
-    uint4 q;
-    if (a.wbf16) {
-      q = ld16(static_cast<const uint16_t*>(a.w) + (int64_t)(nbase + n) * a.K + 8 * k8);
-    } else {
-      const float* src = static_cast<const float*>(a.w) + (int64_t)(nbase + n) * a.K + 8 * k8;
-      q = make_uint4(pack_bf16(src[0], src[1]), pack_bf16(src[2], src[3]), pack_bf16(src[4], src[5]), pack_bf16(src[6], src[7]));
-    }
-    *reinterpret_cast<uint4*>(wl + n * ws + 8 * k8) = q;
-  }
+  const int kp = a.K / 8, pieces = a.Ns * kp;
+  stage_rows(a.w, a.wbf16, (int64_t)nbase * a.K, pieces, tid, [&](int i, const uint4& q) {
+    const int n = i / kp;
+    *reinterpret_cast<uint4*>(wl + n * ws + 8 * (i - n * kp)) = q;
+  });
   float* lnp = smem + (a.Ns * ws / 2 + 3) / 4 * 4 + kLinWaves * 16 * kLinStage;      // behind the waves' result blocks
   if (a.pre == kActLayerNorm)
     for (int i = tid; i < a.K; i += kLinThreads) { lnp[i] = ldw(a.ln_w, a.wbf16, i); lnp[a.K + i] = ldw(a.ln_b, a.wbf16, i); }
@@ -597,6 +632,98 @@ __global__ __launch_bounds__(kLinThreads) void m2d_linear_kernel(const LinArgs a
   }
 }
 
+// ------------------------------------------------ wide linear layers of a few positions, bf16
+// y = post(x W^T + bias) for the wide layers of the attention stages when a batch has few positions (one image: 196 and
+// 49 rows).  The stock product takes the host 19 us to issue and the device 6 to 9 us; here the weights are the
+// traffic and latency is the cost, so nothing is staged: a workgroup owns 32 positions x 16 NT outputs, its four
+// waves share out the contraction in steps of 32 (neighbouring waves read neighbouring 64-byte pieces of a row), every
+// operand is a 16-byte piece of a row straight from memory with the loads of kWideAhead steps in flight, and the
+// waves' sums meet in LDS.  W's rows are the first operand: a lane ends with four neighbouring outputs of a position.
+constexpr int kWideAhead = 4;
+constexpr int kWideWaves = 4;
+struct WideArgs {
+  const uint16_t* x;      // (P, K)
+  const void* w;          // (N, K)
+  const void* bias;       // (N) or null
+  uint16_t* y;            // (P, N)
+  int P, K, N, post;
+};
+
+template <int NT, bool WBF16>
+__global__ __launch_bounds__(256) void m2d_wide_linear_kernel(const WideArgs a) {
+  __shared__ f32x4_t sums[kWideWaves][2 * NT][64];
+  const int l = threadIdx.x & 63, mn = l & 15, kb = l >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 32;
+  const uint16_t* xr[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int m = m0 + 16 * j + mn;
+    xr[j] = a.x + (int64_t)(m < a.P ? m : a.P - 1) * a.K + 8 * kb;      // rows past the end repeat the last one and are not stored
+  }
+  const int64_t wrow = (int64_t)(n0 + mn) * a.K + 8 * kb;
+  auto load_w = [&](int i, int step) {
+    const int64_t at = wrow + (int64_t)16 * i * a.K + 32 * step;
+    if constexpr (WBF16) {
+      return ld16(static_cast<const uint16_t*>(a.w) + at);
+    } else {
+      const float4 lo = *reinterpret_cast<const float4*>(static_cast<const float*>(a.w) + at), hi = *reinterpret_cast<const float4*>(static_cast<const float*>(a.w) + at + 4);
+      return make_uint4(pack_bf16(lo.x, lo.y), pack_bf16(lo.z, lo.w), pack_bf16(hi.x, hi.y), pack_bf16(hi.z, hi.w));
+    }
+  };
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[NT][2];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) acc[i][0] = acc[i][1] = zero;
+  const int steps = a.K / 32;
+  for (int s0 = wave; s0 < steps; s0 += kWideWaves * kWideAhead) {
+    uint4 wf[kWideAhead][NT], xf[kWideAhead][2];
+#pragma unroll
+    for (int k = 0; k < kWideAhead; ++k) {
+      const int s = s0 + kWideWaves * k < steps ? s0 + kWideWaves * k : s0;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) wf[k][i] = load_w(i, s);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) xf[k][j] = ld16(xr[j] + 32 * s);
+    }
+#pragma unroll
+    for (int k = 0; k < kWideAhead; ++k)
+      if (s0 + kWideWaves * k < steps) {      // (uniform)
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma_bf16(wf[k][i], xf[k][j], acc[i][j]);
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) sums[wave][2 * i + j][l] = acc[i][j];
+  __syncthreads();
+  for (int t = wave; t < 2 * NT; t += kWideWaves) {
+    f32x4_t v = sums[0][t][l];
+#pragma unroll
+    for (int w = 1; w < kWideWaves; ++w) v += sums[w][t][l];
+    const int n = n0 + 16 * (t >> 1) + 4 * kb, m = m0 + 16 * (t & 1) + mn;
+    if (a.bias) {
+      float b[4];
+      ldwv<4>(a.bias, WBF16, n, b);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] += b[r];
+    }
+    if (a.post == kActGelu) {
+      // the stock layer stores its output before the activation reads it: the same rounding here
+#pragma unroll
+      for (int r = 0; r < 4; r += 2) {
+        const uint32_t q = pack_bf16(v[r], v[r + 1]);
+        v[r] = gelu_exact(bf_lo(q));
+        v[r + 1] = gelu_exact(bf_hi(q));
+      }
+    }
+    if (m < a.P) *reinterpret_cast<uint2*>(a.y + (int64_t)m * a.N + n) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+  }
+}
+
 // ------------------------------------------------------------ the MLP of a narrow stage, bf16
 // y = fc2(GELU(fc1 x)) (models/utils.py:58-81) where both weight matrices fit LDS together (C = 32 or 64
 // channels, 4 C hidden units): the hidden activations, four times the size of x and y and the reason why
@@ -629,20 +756,12 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
   const int tid = threadIdx.x, l = tid & 63, mn = l & 15, kb = l >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto stage_weights = [&](const void* w, int rows, int cols, uint16_t* dst, int stride) {   // 8 elements at a time
-    for (int i = tid; i < rows * (cols / 8); i += kLinThreads) {
+    stage_rows(w, a.wbf16, 0, rows * (cols / 8), tid, [&](int i, const uint4& q) {
       const int n = i / (cols / 8), k8 = i - n * (cols / 8);
-      if (a.wbf16) {
-        const uint4 q = ld16(static_cast<const uint16_t*>(w) + (int64_t)n * cols + 8 * k8);
-        uint2* d = reinterpret_cast<uint2*>(dst + n * stride + 8 * k8);      // rows of W2 are 8-byte aligned only
-        d[0] = make_uint2(q.x, q.y);
-        d[1] = make_uint2(q.z, q.w);
-      } else {
-        const float* src = static_cast<const float*>(w) + (int64_t)n * cols + 8 * k8;
-        uint2* d = reinterpret_cast<uint2*>(dst + n * stride + 8 * k8);
-        d[0] = make_uint2(pack_bf16(src[0], src[1]), pack_bf16(src[2], src[3]));
-        d[1] = make_uint2(pack_bf16(src[4], src[5]), pack_bf16(src[6], src[7]));
-      }
-    }
+      uint2* d = reinterpret_cast<uint2*>(dst + n * stride + 8 * k8);      // rows of W2 are 8-byte aligned only
+      d[0] = make_uint2(q.x, q.y);
+      d[1] = make_uint2(q.z, q.w);
+    });
   };
   stage_weights(a.w1, HD, C, w1l, W1S);
   stage_weights(a.w2, C, HD, w2l, W2S);
@@ -912,6 +1031,21 @@ void m2d_rope_attention_kernel(const AttnArgs a) {
   }
 }
 
+// ------------------------------------------------------------------ parameters held in bf16
+// One launch for all the small parameters that the scans of a stage want in fp32 (48 casts of 4.4 us each in a batch of
+// the backbone otherwise).
+constexpr int kWidenSegs = 64;
+struct WidenArgs {
+  struct { const uint16_t* in; float* out; int n, first; } s[kWidenSegs];
+  int nsegs;
+};
+__global__ __launch_bounds__(256) void m2d_widen_kernel(const WidenArgs a) {
+  int k = 0;
+  while (k + 1 < a.nsegs && (int)blockIdx.x >= a.s[k + 1].first) ++k;
+  const int i = ((int)blockIdx.x - a.s[k].first) * 256 + threadIdx.x;
+  if (i < a.s[k].n) a.s[k].out[i] = __uint_as_float((uint32_t)a.s[k].in[i] << 16);
+}
+
 template <int NT>
 void launch_attention(const AttnArgs& a, unsigned blocks, hipStream_t st) {
   hipLaunchKernelGGL(m2d_rope_attention_kernel<NT>, dim3(blocks), dim3(64 * att_waves(NT)), 0, st, a);
@@ -920,6 +1054,25 @@ void launch_attention(const AttnArgs& a, unsigned blocks, hipStream_t st) {
 }  // namespace
 
 extern "C" {
+
+int m2d_widen(int nsegs, const m2d_widen_seg* segs, void* stream) {
+  if (!segs) return M2D_ERR_NULL_POINTER;
+  if (nsegs < 1) return M2D_ERR_BAD_SHAPE;
+  for (int at = 0; at < nsegs;) {
+    WidenArgs a = {};
+    int64_t blocks = 0;
+    for (; at < nsegs && a.nsegs < kWidenSegs; ++at) {
+      if (!segs[at].in || !segs[at].out) return M2D_ERR_NULL_POINTER;
+      if (segs[at].n < 1 || segs[at].n >= ((int64_t)1 << 31)) return M2D_ERR_BAD_SHAPE;
+      auto& s = a.s[a.nsegs++];
+      s.in = static_cast<const uint16_t*>(segs[at].in); s.out = segs[at].out; s.n = (int)segs[at].n; s.first = (int)blocks;
+      blocks += (segs[at].n + 255) / 256;
+      if (blocks >= ((int64_t)1 << 31)) return M2D_ERR_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL(m2d_widen_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  }
+  return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
+}
 
 int m2d_layernorm_fwd(int64_t rows, int C, int dtype, int weight_dtype, const void* x, const void* weight,
                       const void* bias, float eps, void* y, void* stream) {
@@ -1163,6 +1316,28 @@ int m2d_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, con
   if (pre_act == kActLayerNorm) return M2D_ERR_UNSUPPORTED;      // that one has an entry point of its own
   return run_linear(P, K, N, weight_dtype, x, weight, bias, pre_act, pre_scale, pre_bias, post_act, post_scale, post_bias, y, stream,
                     nullptr, nullptr, 0.f);
+}
+
+int m2d_wide_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias, int post_act,
+                        void* y, void* stream) {
+  if (!x || !weight || !y) return M2D_ERR_NULL_POINTER;
+  if (P < 1 || K < 1 || N < 1) return M2D_ERR_BAD_SHAPE;
+  if (weight_dtype != M2D_F32 && weight_dtype != M2D_BF16) return M2D_ERR_UNSUPPORTED;
+  if (K % 32 != 0 || N % 32 != 0 || P > ((int64_t)1 << 20) || (post_act != kActNone && post_act != kActGelu)) return M2D_ERR_UNSUPPORTED;
+  if (misaligned(x, 16) || misaligned(weight, 16) || misaligned(y, 16) || misaligned(bias, 16)) return M2D_ERR_MISALIGNED;
+  WideArgs a = {static_cast<const uint16_t*>(x), weight, bias, static_cast<uint16_t*>(y), (int)P, K, N, post_act};
+  const unsigned mt = (unsigned)((P + 31) / 32);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool narrow = (int64_t)mt * (N / 32) < 128;      // few workgroups: 16 outputs each instead of 32
+  const dim3 g((unsigned)(narrow ? N / 16 : N / 32), mt), t(64 * kWideWaves);
+  auto go = [&](auto wb) {
+    constexpr bool WB = decltype(wb)::value;
+    if (narrow) hipLaunchKernelGGL((m2d_wide_linear_kernel<1, WB>), g, t, 0, st, a);
+    else hipLaunchKernelGGL((m2d_wide_linear_kernel<2, WB>), g, t, 0, st, a);
+  };
+  if (weight_dtype == M2D_BF16) go(std::true_type{});
+  else go(std::false_type{});
+  return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
 }
 
 int m2d_linear_keep_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias,

@@ -51,6 +51,8 @@ mlp_fwd_op = torch.ops.m2dscan.mlp_fwd
 linear_act_fwd_op = torch.ops.m2dscan.linear_act_fwd
 layernorm_linear_act_fwd_op = torch.ops.m2dscan.layernorm_linear_act_fwd
 train_block_op = torch.ops.m2dscan.train_block
+infer_stage_op = torch.ops.m2dscan.infer_stage
+widen_op = torch.ops.m2dscan.widen
 
 # Keep the forward's anti-diagonal checkpoints for the backward (faster backward, more saved
 # memory) or rebuild them inside the backward (nothing saved beyond the inputs, like the
@@ -421,7 +423,10 @@ class wf_cuda_fn_proj(torch.autograd.Function):
     def _params(x, AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D):
         """The parameters as fp32 tensors (no copy if they already are): the library itself forms
         A = -exp(A_log) and rounds everything to x.dtype as the reference's casts do."""
-        return [_as_f32(t) for t in (AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D)]
+        raw = (AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D)
+        if all(t.dtype == torch.bfloat16 and t.is_cuda for t in raw) and not torch.compiler.is_compiling():
+            return widen_op([t.detach().contiguous() for t in raw])      # one launch in place of eight casts
+        return [_as_f32(t) for t in raw]
 
     @staticmethod
     def forward(ctx, x, AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D,
