@@ -105,7 +105,7 @@ def build_shim(verbose: bool = True) -> str:
     import torch
     from torch.utils import cpp_extension as ce
 
-    src = [os.path.join(HERE, "csrc", name) for name in ("m2d_torch.cpp", "m2d_train.cpp", "m2d_infer.cpp")]
+    src = [os.path.join(HERE, "csrc", name) for name in ("m2d_torch.cpp", "m2d_train.cpp", "m2d_infer.cpp", "m2d_entry.cpp")]
     inc = [f"-I{p}" for p in ce.include_paths(device_type="cuda")] + [f"-I{os.path.join(ROOT, 'include')}"]
     libdirs = ce.library_paths(device_type="cuda")
     cmd = ["hipcc", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",

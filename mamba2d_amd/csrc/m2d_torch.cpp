@@ -86,16 +86,17 @@ Tensor bytes(size_t n, const Tensor& like) {
   return at::empty({static_cast<int64_t>(n > 0 ? n : 1)}, like.options().dtype(at::kByte));
 }
 
-std::tuple<Tensor, Tensor> scan_fwd(const Tensor& x, const Tensor& dT, const Tensor& dL, const Tensor& AT,
-                                    const Tensor& AL, const Tensor& BT, const Tensor& BL, const Tensor& C,
-                                    const Tensor& D, bool save_ckpt, bool flip, bool raw_params, bool packed_bc,
-                                    int64_t ckpt_interval) {
+// y and, if asked for, what the backward wants (an undefined tensor otherwise)
+std::tuple<Tensor, Tensor> scan_y(const Tensor& x, const Tensor& dT, const Tensor& dL, const Tensor& AT, const Tensor& AL,
+                                  const Tensor& BT, const Tensor& BL, const Tensor& C, const Tensor& D, bool save_ckpt, bool flip,
+                                  bool raw_params, bool packed_bc, int64_t ckpt_interval) {
   const m2d_desc d = describe(x, AT, flip, raw_params, packed_bc, false, ckpt_interval);
   expect_all(d, x, dT, dL, AT, AL, BT, BL, C, D);
   check(m2d_desc_check(&d));
   c10::DeviceGuard guard(x.device());
   Tensor y = at::empty_like(x);
-  Tensor ck = bytes(save_ckpt ? m2d_scan_ckpt_bytes(&d) : 0, x);
+  Tensor ck;
+  if (save_ckpt) ck = bytes(m2d_scan_ckpt_bytes(&d), x);
   Tensor ws = bytes(m2d_scan_workspace_bytes(&d, M2D_PASS_FWD, save_ckpt), x);
   hipStream_t st = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   check(m2d_scan_fwd(&d, x.data_ptr(), dT.data_ptr(), dL.data_ptr(), AT.data_ptr(), AL.data_ptr(), BT.data_ptr(),
@@ -103,6 +104,15 @@ std::tuple<Tensor, Tensor> scan_fwd(const Tensor& x, const Tensor& dT, const Ten
                      save_ckpt ? static_cast<size_t>(ck.numel()) : 0, ws.data_ptr(), static_cast<size_t>(ws.numel()),
                      st));
   return {y, ck};
+}
+
+std::tuple<Tensor, Tensor> scan_fwd(const Tensor& x, const Tensor& dT, const Tensor& dL, const Tensor& AT,
+                                    const Tensor& AL, const Tensor& BT, const Tensor& BL, const Tensor& C,
+                                    const Tensor& D, bool save_ckpt, bool flip, bool raw_params, bool packed_bc,
+                                    int64_t ckpt_interval) {
+  auto r = scan_y(x, dT, dL, AT, AL, BT, BL, C, D, save_ckpt, flip, raw_params, packed_bc, ckpt_interval);
+  if (!save_ckpt) std::get<1>(r) = bytes(0, x);
+  return r;
 }
 
 std::vector<Tensor> scan_bwd(const Tensor& x, const Tensor& dT, const Tensor& dL, const Tensor& AT, const Tensor& AL,

@@ -19,6 +19,9 @@ inline hipStream_t current_stream(const Tensor& t) { return c10::hip::getCurrent
 std::tuple<Tensor, Tensor> scan_fwd(const Tensor& x, const Tensor& dT, const Tensor& dL, const Tensor& AT, const Tensor& AL,
                                     const Tensor& BT, const Tensor& BL, const Tensor& C, const Tensor& D, bool save_ckpt,
                                     bool flip, bool raw_params, bool packed_bc, int64_t ckpt_interval);
+std::tuple<Tensor, Tensor> scan_y(const Tensor& x, const Tensor& dT, const Tensor& dL, const Tensor& AT, const Tensor& AL,
+                                  const Tensor& BT, const Tensor& BL, const Tensor& C, const Tensor& D, bool save_ckpt,
+                                  bool flip, bool raw_params, bool packed_bc, int64_t ckpt_interval);
 std::vector<Tensor> scan_bwd(const Tensor& x, const Tensor& dT, const Tensor& dL, const Tensor& AT, const Tensor& AL,
                              const Tensor& BT, const Tensor& BL, const Tensor& C, const Tensor& D, const Tensor& dy,
                              const Tensor& ckpt, bool flip, bool raw_params, bool packed_bc, bool dpre, int64_t ckpt_interval,

@@ -228,6 +228,8 @@ struct ScanParams {
   int ck_half;                      // a snapshot every 2 steps (before the steps 0 and 2 of every block, and one behind the last block): snapshot 2m + s is the state before step 4m + 2s
   int ck_pb;                        // kept snapshots per band (linked sweep)
   int ck_nblk;                      // kept snapshots per image
+  const void *AT, *AL, *D;          // the caller's A_T, A_L and D; raw: fp32 A_log and D as a module holds them
+  int raw;
   void* ring;                       // [workgroup][2^ck_shift - 1][channel of the workgroup][4][16] snapshot quads
 };
 
@@ -1346,10 +1348,33 @@ __device__ __forceinline__ float sum_over_groups(float v) {
   v = fold16(v, v);
   return fold32(v, v);
 }
+// the value a tensor of type T would hold
+__device__ __forceinline__ float as_stored(float v, const float*) { return v; }
+__device__ __forceinline__ float as_stored(float v, const bf16_t*) { return bf16_bits_to_f32(f32_to_bf16_bits(v)); }
+
+// A * log2 e and D from the caller's tensors: of type T, or the parameters as the module holds them (fp32 A_log and D:
+// A = -exp(A_log), and both are rounded to T, which is what the reference's casts to x.dtype do, wavefront_cuda.py:72-73,
+// 90-91, 332).
+template <typename T>
+__device__ __forceinline__ float gate_rate(const ScanParams& p, const void* A, int i) {
+  return (p.raw ? as_stored(-expf(static_cast<const float*>(A)[i]), static_cast<const T*>(nullptr)) : IO<T>::ld(static_cast<const T*>(A) + i)) * kLog2e;
+}
+template <typename T>
+__device__ __forceinline__ float skip_gain(const ScanParams& p, int e) {
+  return p.raw ? as_stored(static_cast<const float*>(p.D)[e], static_cast<const T*>(nullptr)) : IO<T>::ld(static_cast<const T*>(p.D) + e);
+}
+// The set-up launch (m2d_prep_kernel) is for kernels whose lanes hold all states of a channel, for a backward that will
+// read the same values, and for progress counts.  A lane here holds 4 states of one channel, so a forward with neither
+// works them out itself and saves the launch and the gap behind it (4 of 15 us on one 14x14x320 image).
+template <bool CKPT, int MODE>
+constexpr bool split_owns_setup() { return !CKPT && MODE != kModeSliced; }
+__device__ float m2d_zero_page[kZeroFloats];     // the page of zeros of such a forward: never written
+
 template <typename T, bool CKPT, bool WRITE_Y, bool STAGE_X, int MODE, int NWS = kSplitWaves>
 __global__ __launch_bounds__((NWS + split_helpers<MODE, NWS, STAGE_X>()) * 64) void m2d_fwd_split_kernel(const ScanParams pin) {
   static_assert(MODE != kModeStacked, "stacked images are many: they never need the split");
   constexpr bool SLICED = MODE == kModeSliced;
+  constexpr bool OWN_SETUP = split_owns_setup<CKPT, MODE>();
   const ScanParams& p = pin;
   __builtin_assume(p.stacked == 0);
   __builtin_assume(p.rb == kRB);
@@ -1399,11 +1424,11 @@ __global__ __launch_bounds__((NWS + split_helpers<MODE, NWS, STAGE_X>()) * 64) v
   for (int w = 0; w < 4; ++w) {
     const int q = w == 1 ? 2 : (w == 2 ? 1 : w);   // sinv<true>(4g + w) = q * 4 + g
     const int n = (!WIDEN && direct) ? 4 * g + w : q * 4 + g;
-    a2t[w] = p.A2T[e0 * kN + n];
-    a2l[w] = p.A2L[e0 * kN + n];
+    a2t[w] = OWN_SETUP ? gate_rate<T>(p, p.AT, e0 * kN + n) : p.A2T[e0 * kN + n];
+    a2l[w] = OWN_SETUP ? gate_rate<T>(p, p.AL, e0 * kN + n) : p.A2L[e0 * kN + n];
   }
   static_assert(sinv<true>(1) == 8 && sinv<true>(6) == 5 && sinv<true>(15) == 15, "fold order");
-  const float dsk = p.Df[e0];
+  const float dsk = OWN_SETUP ? skip_gain<T>(p, e0) : p.Df[e0];
   settle_loads();
   __syncthreads();
 
@@ -3049,35 +3074,17 @@ __global__ __launch_bounds__((NWS + split_helpers<MODE, NWS, STAGE_X>()) * 64) v
 }
 
 // -------------------------------------------------------------------------- small helper kernels
-// the value a tensor of type T would hold
-__device__ __forceinline__ float as_stored(float v, const float*) { return v; }
-__device__ __forceinline__ float as_stored(float v, const bf16_t*) { return bf16_bits_to_f32(f32_to_bf16_bits(v)); }
-
-// RAW: the parameters as the module holds them (fp32 A_log, fp32 D): A = -exp(A_log), and both
-// are rounded to T, which is what the reference's casts to x.dtype do (wavefront_cuda.py:72-73,
-// 90-91, 332).
-template <typename T, bool RAW>
-__global__ void m2d_prep_kernel(const void* ATv, const void* ALv, const void* Dv, float* zeros, float* A2T, float* A2L, float* Df, int E,
-                                uint32_t* link_words, int n_link_words) {
+template <typename T>
+__global__ void m2d_prep_kernel(const ScanParams p, float* zeros, float* A2T, float* A2L, float* Df, uint32_t* link_words, int n_link_words) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx < kZeroFloats) zeros[idx] = 0.f;
   // linked sweep: error word and progress counts start at zero
   for (int i = idx; i < n_link_words; i += gridDim.x * blockDim.x) link_words[i] = 0u;
-  if constexpr (RAW) {
-    const float *AT = static_cast<const float*>(ATv), *AL = static_cast<const float*>(ALv), *D = static_cast<const float*>(Dv);
-    if (idx < E * kN) {
-      A2T[idx] = as_stored(-expf(AT[idx]), static_cast<const T*>(nullptr)) * kLog2e;
-      A2L[idx] = as_stored(-expf(AL[idx]), static_cast<const T*>(nullptr)) * kLog2e;
-    }
-    if (idx < E) Df[idx] = as_stored(D[idx], static_cast<const T*>(nullptr));
-  } else {
-    const T *AT = static_cast<const T*>(ATv), *AL = static_cast<const T*>(ALv), *D = static_cast<const T*>(Dv);
-    if (idx < E * kN) {
-      A2T[idx] = IO<T>::ld(AT + idx) * kLog2e;
-      A2L[idx] = IO<T>::ld(AL + idx) * kLog2e;
-    }
-    if (idx < E) Df[idx] = IO<T>::ld(D + idx);
+  if (idx < p.E * kN) {
+    A2T[idx] = gate_rate<T>(p, p.AT, idx);
+    A2L[idx] = gate_rate<T>(p, p.AL, idx);
   }
+  if (idx < p.E) Df[idx] = skip_gain<T>(p, idx);
 }
 
 // B_T, B_L, C -> one fp32 record of 48 values per cell (three runs of 16, each in fold order,
@@ -3497,6 +3504,7 @@ void fill_common(ScanParams& sp, const m2d_desc* d, const Geometry& g) {
   sp.bot_stride = g.sliced ? (int64_t)g.vB * d->W * d->E * kN : 0;
   sp.flip = (d->flags & M2D_FLAG_FLIP) ? 1 : 0;
   sp.dpre = (d->flags & M2D_FLAG_DPRE) ? 1 : 0;
+  sp.raw = (d->flags & M2D_FLAG_RAW_PARAMS) ? 1 : 0;
   sp.ck_shift = g.ck_shift; sp.ck_pb = g.ck_pb; sp.ck_nblk = g.ck_nblk; sp.ck_half = g.ck_half ? 1 : 0;
   sp.ring = nullptr;
 }
@@ -3515,8 +3523,7 @@ inline bool allow_dynamic_lds(const void* kernel, size_t bytes, std::atomic<uint
 
 // Set-up area: [page of zeros][A_T*log2e][A_L*log2e][D], all fp32.
 template <typename T>
-int launch_prep(ScanParams& sp, const m2d_desc* d, const Geometry& g, const void* AT, const void* AL, const void* D, float* base,
-                uint32_t* link_words, hipStream_t st, bool ready = false) {
+int launch_prep(ScanParams& sp, const m2d_desc* d, const Geometry& g, float* base, uint32_t* link_words, hipStream_t st, bool ready = false) {
   const int n_link = (int)(g.link_bytes / sizeof(uint32_t));
   sp.link_err = link_words;   // (the first 64 words: the error word; then forward counts, then backward counts)
   float* zeros = base;
@@ -3526,11 +3533,24 @@ int launch_prep(ScanParams& sp, const m2d_desc* d, const Geometry& g, const void
   sp.zeros = zeros; sp.A2T = A2T; sp.A2L = A2L; sp.Df = Df;
   if (ready && n_link == 0) return M2D_OK;   // the forward of this problem filled the area, and there is nothing to clear
   const int n = d->E * kN > kZeroFloats ? d->E * kN : kZeroFloats;
-  if (d->flags & M2D_FLAG_RAW_PARAMS)
-    hipLaunchKernelGGL((m2d_prep_kernel<T, true>), dim3((n + 255) / 256), dim3(256), 0, st, AT, AL, D, zeros, A2T, A2L, Df, d->E, link_words, n_link);
-  else
-    hipLaunchKernelGGL((m2d_prep_kernel<T, false>), dim3((n + 255) / 256), dim3(256), 0, st, AT, AL, D, zeros, A2T, A2L, Df, d->E, link_words, n_link);
+  hipLaunchKernelGGL(m2d_prep_kernel<T>, dim3((n + 255) / 256), dim3(256), 0, st, sp, zeros, A2T, A2L, Df, link_words, n_link);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
+}
+
+// The address of m2d_zero_page on the current device (each device has its own; asked for once per device).
+int zero_page(const float** page) {
+  static std::atomic<const float*> known[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return M2D_ERR_HIP;
+  const float* at = dev < 64 ? known[dev].load(std::memory_order_relaxed) : nullptr;
+  if (!at) {
+    void* q = nullptr;
+    if (hipGetSymbolAddress(&q, HIP_SYMBOL(m2d_zero_page)) != hipSuccess) return M2D_ERR_HIP;
+    at = static_cast<const float*>(q);
+    if (dev < 64) known[dev].store(at, std::memory_order_relaxed);
+  }
+  *page = at;
+  return M2D_OK;
 }
 
 // Points sp.bt/bl/cc at the packed fp32 copy of B_T, B_L, C (made here unless `ready`, or brought
@@ -3674,7 +3694,8 @@ int run_fwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
   sp.ckpt = ckpt ? static_cast<float*>(ckpt) : nullptr;
   sp.top = reinterpret_cast<float*>(keep);
   if (ckpt) prep = reinterpret_cast<float*>(keep + g.top_bytes + g.bc_bytes);   // kept for the backward
-  int rc = launch_prep<T>(sp, d, g, AT, AL, D, prep, link_words, st);
+  sp.AT = AT; sp.AL = AL; sp.D = D;
+  int rc = g.fwd_split && !ckpt && !g.sliced ? zero_page(&sp.zeros) : launch_prep<T>(sp, d, g, prep, link_words, st);   // (split_owns_setup)
   if (rc) return rc;
   if ((!ckpt || sizeof(T) == 2) && !g.packed_bc) {   // the kernel takes the tensors as they are (fp32: only where no backward will want the packed copy)
     sp.bcd[0] = BT; sp.bcd[1] = BL; sp.bcd[2] = C; sp.bcd[3] = BT;
@@ -3776,7 +3797,8 @@ int run_bwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
   sp.ring = w; w += g.ring_bytes;
   char* ck = ckpt ? const_cast<char*>(static_cast<const char*>(ckpt)) : w;
   if (ckpt) prep = reinterpret_cast<float*>(ck + g.ckpt_diag_bytes + g.top_bytes + g.bc_bytes);   // as the forward left it
-  int rc = launch_prep<T>(sp, d, g, AT, AL, D, prep, link_words, st, ckpt != nullptr);
+  sp.AT = AT; sp.AL = AL; sp.D = D;
+  int rc = launch_prep<T>(sp, d, g, prep, link_words, st, ckpt != nullptr);
   if (rc) return rc;
   sp.ckpt = reinterpret_cast<float*>(ck);
   sp.top = reinterpret_cast<float*>(ck + g.ckpt_diag_bytes);

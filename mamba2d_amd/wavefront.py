@@ -53,6 +53,9 @@ layernorm_linear_act_fwd_op = torch.ops.m2dscan.layernorm_linear_act_fwd
 train_block_op = torch.ops.m2dscan.train_block
 infer_stage_op = torch.ops.m2dscan.infer_stage
 widen_op = torch.ops.m2dscan.widen
+entry_op = torch.ops.m2dscan.entry.default
+scan_op = torch.ops.m2dscan.scan.default
+_OWN_OPS = (scan_fwd_op, scan_bwd_op, proj_fwd_op, proj_bwd_op)
 
 # Keep the forward's anti-diagonal checkpoints for the backward (faster backward, more saved
 # memory) or rebuild them inside the backward (nothing saved beyond the inputs, like the
@@ -312,6 +315,13 @@ def _grouped_scan_bwd(x, deltaT, deltaL, AT, AL, BT, BL, C, D, dy, cks, flip, in
     return (*[t.to(x.dtype) for t in sums], *joined, d_D)
 
 
+def _eager(x) -> bool:
+    """Whether a call on x can be issued from C++ in one operator (csrc/m2d_entry.cpp): a plain tensor on the GPU, not
+    traced and not under forward-mode differentiation, and nobody has put something else in place of the operators."""
+    return (type(x) is torch.Tensor and x.is_cuda and not torch.compiler.is_compiling()
+            and (scan_fwd_op, scan_bwd_op, proj_fwd_op, proj_bwd_op) == _OWN_OPS and torch.autograd.forward_ad._current_level < 0)
+
+
 class _ScanOnParams(torch.autograd.Function):
     """The Function behind ``wf_cuda_fn_pr``: 16 states, and told by its caller whether autograd
     records the call (``recording``)."""
@@ -359,6 +369,8 @@ class wf_cuda_fn_pr(torch.autograd.Function):
 
     @classmethod
     def apply(cls, x, deltaT, deltaL, AT, AL, BT, BL, C, D, flip=False):
+        if not torch.is_grad_enabled() and _eager(x) and AT.shape[-1] == STATES_PER_CALL:
+            return scan_op(x, deltaT, deltaL, AT, AL, BT, BL, C, D, bool(flip), _interval())
         return _ScanOnParams.apply(x, deltaT, deltaL, AT, AL, BT, BL, C, D, flip, torch.is_grad_enabled())
 
 
@@ -486,6 +498,9 @@ def wavefront_scan_cuda(x, AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_
         raise ValueError(f"Unknown recomputation mode, got {recomp}...")
     if FUSED_PROJECTIONS and _proj_kernels_cover(x, AT_log, dt_projT_w):
         # the casts of the weights to x.dtype happen inside (no copies of the parameters)
+        if _eager(x):
+            return entry_op(x, [AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D],
+                            recomp == "full", bool(flip), SAVE_CHECKPOINTS, _interval())
         return wf_cuda_fn_proj.apply(x, AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D,
                                      recomp == "full", flip, torch.is_grad_enabled())
 
