@@ -12,14 +12,12 @@
 //             dz = [dpreT wT | dpreL wL | dB_T | dB_L | dC] ;  dx += dz Wx
 //             dWx = dz^T x ;  dw = dpre^T r ;  db = sum dpre      (sums over all positions)
 //
-// Arithmetic is fp32 on the vector ALUs: a thread owns one position of the tile and multiplies
-// it with weights that are uniform over the wave, so the weights arrive through scalar loads and
-// cost no vector registers or LDS traffic.  The host packs the weights once per call into padded,
-// transposed copies so that those loads are aligned runs of 16 floats with no edge cases.
+// The products run on the matrix cores: bf16 tensors whose rows are whole 16-byte chunks through bf16 operands, all
+// others through fp32 ones; sums are fp32 in both.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <atomic>
+#include <type_traits>
 
 #include "m2dscan.h"
 
@@ -30,10 +28,7 @@ constexpr int kTP = 64;       // positions per tile (one per lane)
 constexpr int kKC = 64;       // channels per chunk of the inner dimension
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-constexpr int kXS = kKC + 1;  // row stride (floats) of a 64 x 64 tile in LDS, odd: lanes reading one column hit 64 banks
-constexpr int kXS4 = kKC + 4; // the same for tiles read as float4
 constexpr int kMaxR = 32;     // largest dt_rank
-constexpr int kMaxRounds = 4; // 16-wide output chunks per wave
 
 struct bf16_t { uint16_t v; };
 
@@ -90,62 +85,42 @@ struct ProjArgs {
   int sum_parts;                         // > 0: dBT points to that many fp32 records [P][dC | dBT | dBL][16] to add up (the scan's per-workgroup sums)
   void *r_out, *dT_out, *dL_out, *BT_out, *BL_out, *C_out, *dx;
   float* bc_packed;                      // (P,48) fp32 records for the scan kernels instead of BT_out, BL_out, C_out (or null)
-  // packed weights, fp32, zero where padded
-  const float *Wt;                       // [Epad][Opad]   Wx transposed
-  const float *wTt, *wLt;                // [R][Epad]      dt weights transposed
-  const float *bTp, *bLp;                // [Epad]
-  const float *Wp;                       // [O][Epad]      Wx
-  const float *wTp, *wLp;                // [Epad][Rpad]   dt weights
-  // packed weights for the matrix-core kernels, bf16, zero where padded
+  const float *Wx, *wT, *bT, *wL, *bL;   // the weights as the caller holds them (for the fp32 products)
+  int round;                             // ... to be rounded to bf16 by the kernels that read them
+  const float *bTp, *bLp;                // [Epad] packed biases, fp32, zero where padded
+  // packed weights for the bf16 products, zero where padded
   const uint16_t *Wb;                    // [Opad][Epad]   Wx
   const uint16_t *wTb, *wLb;             // [Epad][32]     dt weights
   const uint16_t *wTtb, *wLtb;           // [Rpad][Epad]   dt weights transposed
   const uint16_t *WxTb;                  // [Epad][Opad32] Wx transposed
-  float* dz;                             // (P,O4) fp32, rows padded to a multiple of 4
-  // the same for the matrix-core kernels, bf16
+  float* dz;                             // (P,Opad) fp32, padding behind the low-rank part (o' order)
+  // the same for the bf16 products
   uint16_t* dzt;                         // (P16, Opad)    dz, P16 = positions rounded up to 16
   uint16_t* dpt;                         // [2](P16, E)    dpreT, dpreL
   float* part;                           // per-workgroup sums of the weight gradients
   float *dWx, *dwT, *dbT, *dwL, *dbL;    // outputs of the reduction
   int64_t P;
-  int E, R, O, O4, Epad, Opad, Opad32, Rpad;
+  int E, R, O, Epad, Opad, Opad32, Rpad;
   int ntiles, G, ne;
 };
-
-// Packed weights are read through the constant address space: they were written by an earlier
-// launch, and a wave-uniform load from that space is a scalar load whatever the kernel stores.
-typedef const __attribute__((address_space(4))) float* const_floats;
-__device__ __forceinline__ const_floats as_const(const float* p) { return (const_floats)(uintptr_t)p; }
 
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
 // ------------------------------------------------------------------------------- weights
 struct PackArgs {
   const float *Wx, *wT, *bT, *wL, *bL;
-  float *Wt, *wTt, *wLt, *bTp, *bLp;     // forward set (or null)
-  float *Wp, *wTp, *wLp;                 // backward set (or null)
-  uint16_t *Wb, *wTb, *wLb;              // forward set of the matrix-core kernels (or null)
-  uint16_t *wTtb, *wLtb, *WxTb;          // backward set of the matrix-core kernels (or null)
+  float *bTp, *bLp;                      // forward set (or null)
+  uint16_t *Wb, *wTb, *wLb;
+  uint16_t *wTtb, *wLtb, *WxTb;          // backward set (or null)
   int E, R, O, Epad, Opad, Opad32, Rpad;
-  int round;                             // round every weight to bf16 first (the bf16 copies are rounded anyway)
+  int round;                             // round the biases to bf16 first (the bf16 copies are rounded anyway)
 };
 
-// Padded copies of the weights.  One thread per element of the largest copy.
+// Padded copies of the weights for the bf16 products.  One thread per element of the largest copy.
 __global__ void m2d_proj_pack_kernel(const PackArgs k) {
-  // a weight as the kernels are to see it
+  // a bias as the kernels are to see it
   auto w = [&](const float* p, int i) { return k.round ? as_stored(p[i], static_cast<const bf16_t*>(nullptr)) : p[i]; };
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k.Wt) {
-    if (i < k.Epad * k.Opad) {
-      const int e = i / k.Opad, o = i - e * k.Opad;
-      k.Wt[i] = (e < k.E && o < k.O) ? w(k.Wx, o * k.E + e) : 0.f;
-    }
-    if (i < k.R * k.Epad) {
-      const int q = i / k.Epad, e = i - q * k.Epad;
-      k.wTt[i] = e < k.E ? w(k.wT, e * k.R + q) : 0.f;
-      k.wLt[i] = e < k.E ? w(k.wL, e * k.R + q) : 0.f;
-    }
-  }
   if (k.bTp && i < k.Epad) {
     k.bTp[i] = i < k.E ? w(k.bT, i) : 0.f;
     k.bLp[i] = i < k.E ? w(k.bL, i) : 0.f;
@@ -173,315 +148,6 @@ __global__ void m2d_proj_pack_kernel(const PackArgs k) {
       k.wTtb[i] = ok ? f32_to_bf16_bits(k.wT[e * k.R + q]) : 0;
       k.wLtb[i] = ok ? f32_to_bf16_bits(k.wL[e * k.R + q]) : 0;
     }
-  }
-  if (k.Wp) {
-    if (i < k.O * k.Epad) {
-      const int o = i / k.Epad, e = i - o * k.Epad;
-      k.Wp[i] = e < k.E ? w(k.Wx, o * k.E + e) : 0.f;
-    }
-    if (i < k.Epad * k.Rpad) {
-      const int e = i / k.Rpad, q = i - e * k.Rpad;
-      const bool ok = e < k.E && q < k.R;
-      k.wTp[i] = ok ? w(k.wT, e * k.R + q) : 0.f;
-      k.wLp[i] = ok ? w(k.wL, e * k.R + q) : 0.f;
-    }
-  }
-}
-
-// ------------------------------------------------------------------------------- tiles
-// A tile is 64 positions x 64 channels of a (P,E) array, 16 elements per thread.  The loads of a
-// tile are issued back to back into registers and converted when they are consumed, so that a
-// thread waits for memory once per tile and not once per row.
-// VEC (E a multiple of the 16-byte vector): thread t holds, for l < NL, the EPL elements from
-//   column (ci % CPR) * EPL of row ci / CPR, ci = l * 256 + t.  Otherwise element i = l * 256 + t,
-//   row i / 64, column i % 64.
-template <typename T, bool VEC>
-struct Tile {
-  static constexpr int EPL = VEC ? 16 / (int)sizeof(T) : 1;
-  static constexpr int NL = 16 / EPL;
-  static constexpr int CPR = kKC / EPL;
-  struct Regs { uint4 q[VEC ? NL : 1]; float v[VEC ? 1 : 16]; };
-
-  static __device__ __forceinline__ void pos(int t, int l, int& row, int& col) {
-    const int ci = l * kThreads + t;
-    row = ci / CPR;
-    col = (ci % CPR) * EPL;
-  }
-  static __device__ __forceinline__ void load(Regs& r, const T* base, int64_t p0, int64_t P, int E, int e0, int t) {
-#pragma unroll
-    for (int l = 0; l < NL; ++l) {
-      int row, col;
-      pos(t, l, row, col);
-      const int64_t p = p0 + row;
-      const bool ok = p < P && e0 + col < E;
-      if constexpr (VEC) r.q[l] = ok ? *reinterpret_cast<const uint4*>(base + p * E + e0 + col) : make_uint4(0, 0, 0, 0);
-      else r.v[l] = ok ? ld(base + p * E + e0 + col) : 0.f;
-    }
-  }
-  // element j < EPL of load l
-  static __device__ __forceinline__ float get(const Regs& r, int l, int j) {
-    if constexpr (!VEC) return r.v[l];
-    else {
-      const uint32_t w[4] = {r.q[l].x, r.q[l].y, r.q[l].z, r.q[l].w};
-      if constexpr (sizeof(T) == 4) return __uint_as_float(w[j]);
-      else return __uint_as_float((j & 1) ? (w[j >> 1] & 0xffff0000u) : (w[j >> 1] << 16));
-    }
-  }
-  // v(l, j) for every element -> tile[row * stride + col]
-  template <typename F>
-  static __device__ __forceinline__ void to_lds(float* tile, int stride, int t, F value) {
-#pragma unroll
-    for (int l = 0; l < NL; ++l) {
-      int row, col;
-      pos(t, l, row, col);
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) tile[row * stride + col + j] = value(l, j);
-    }
-  }
-  // tile[row * stride + col] (+ what `plus` holds) -> global, rows and channels inside the array only
-  static __device__ __forceinline__ void store(const float* tile, int stride, T* base, int64_t p0, int64_t P, int E, int e0,
-                                               int t, const Regs* plus) {
-#pragma unroll
-    for (int l = 0; l < NL; ++l) {
-      int row, col;
-      pos(t, l, row, col);
-      const int64_t p = p0 + row;
-      if (!(p < P && e0 + col < E)) continue;
-      float v[EPL];
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) v[j] = tile[row * stride + col + j] + (plus ? get(*plus, l, j) : 0.f);
-      T* dst = base + p * E + e0 + col;
-      if constexpr (!VEC) st(dst, v[0]);
-      else if constexpr (sizeof(T) == 4) *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-      else {
-        uint32_t w[4];
-#pragma unroll
-        for (int h = 0; h < 4; ++h) w[h] = pack_bf16_pair(v[2 * h], v[2 * h + 1]);
-        *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
-      }
-    }
-  }
-};
-
-// acc[j] += sum_e tile[lane][e] * w[e * stride + j], e < 64, j < 16; w is uniform over the wave
-__device__ __forceinline__ void row_times_weights(const float* tile_row, const_floats w, int stride, float (&acc)[16]) {
-#pragma unroll 4
-  for (int e = 0; e < kKC; ++e) {
-    const float v = tile_row[e];
-    const_floats we = w + e * stride;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = __builtin_fmaf(v, we[j], acc[j]);
-  }
-}
-
-// ------------------------------------------------------------------------------- forward
-// One workgroup per tile of 64 positions.  LDS: xs[64][65] (a chunk of x, later the deltaT tile),
-// zs[64][O+1] (z), outL[64][65] (the deltaL tile).
-template <typename T, bool VEC>
-__global__ __launch_bounds__(kThreads) void m2d_proj_fwd_kernel(const ProjArgs a) {
-  using TL = Tile<T, VEC>;
-  extern __shared__ float smem[];
-  float* xs = smem;
-  float* zs = smem + kTP * kXS;
-  float* outL = zs + kTP * (a.O + 1);
-  float* outT = xs;
-  const int zst = a.O + 1;
-  const int wave = wave_id(), lane = threadIdx.x & 63, tid = threadIdx.x;
-  const int64_t p0 = (int64_t)blockIdx.x * kTP;
-  const T* x = static_cast<const T*>(a.x);
-  const int nOC = a.Opad / 16, nkc = a.Epad / kKC;
-
-  float acc[kMaxRounds][16];
-#pragma unroll
-  for (int rd = 0; rd < kMaxRounds; ++rd)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[rd][j] = 0.f;
-
-  typename TL::Regs xr;
-  TL::load(xr, x, p0, a.P, a.E, 0, tid);
-  for (int kc = 0; kc < nkc; ++kc) {
-    TL::to_lds(xs, kXS, tid, [&](int l, int j) { return TL::get(xr, l, j); });
-    __syncthreads();
-    if (kc + 1 < nkc) TL::load(xr, x, p0, a.P, a.E, (kc + 1) * kKC, tid);   // under way during the products
-#pragma unroll
-    for (int rd = 0; rd < kMaxRounds; ++rd) {
-      const int oc = wave + kWaves * rd;
-      if (oc < nOC) row_times_weights(xs + lane * kXS, as_const(a.Wt) + (int64_t)kc * kKC * a.Opad + oc * 16, a.Opad, acc[rd]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int rd = 0; rd < kMaxRounds; ++rd) {
-    const int oc = wave + kWaves * rd;
-    if (oc < nOC) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        if (oc * 16 + j < a.O) zs[lane * zst + oc * 16 + j] = acc[rd][j];
-    }
-  }
-  __syncthreads();
-
-  // ---- low-rank inputs and B_T, B_L, C: a row of the tile per wave at a time
-  const int R = a.R, R2 = 2 * a.R;
-  T* r_out = static_cast<T*>(a.r_out);
-  for (int c = wave; c < kTP; c += kWaves) {
-    const int64_t p = p0 + c;
-    if (p >= a.P) break;   // uniform
-    const float* z = zs + c * zst;
-    for (int q = lane; q < R2; q += 64) st(r_out + p * R2 + q, z[q]);
-    if (lane < 3 * kN) {
-      if (a.bc_packed) {
-        a.bc_packed[p * (3 * kN) + record_slot(lane)] = as_stored(z[R2 + lane], r_out);
-      } else {
-        T* out = static_cast<T*>(lane < kN ? a.BT_out : (lane < 2 * kN ? a.BL_out : a.C_out));
-        st(out + p * kN + (lane & (kN - 1)), z[R2 + lane]);
-      }
-    }
-  }
-
-  // ---- delta = softplus(r w^T + b), 64 channels at a time: a thread works out 16 channels of
-  // its position with wave-uniform weights, the tile goes out row-wise through LDS
-  const float* zrow = zs + lane * zst;
-  for (int eg = 0; eg < nkc; ++eg) {
-    const int e0 = eg * kKC + wave * 16;
-    float sT[16], sL[16];
-    const_floats bt = as_const(a.bTp) + e0;
-    const_floats bl = as_const(a.bLp) + e0;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) { sT[j] = bt[j]; sL[j] = bl[j]; }
-    for (int q = 0; q < R; ++q) {
-      // the dt projections see the low-rank inputs as the tensor holds them
-      const float zT = as_stored(zrow[q], r_out), zL = as_stored(zrow[R + q], r_out);
-      const_floats wt = as_const(a.wTt) + q * a.Epad + e0;
-      const_floats wl = as_const(a.wLt) + q * a.Epad + e0;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        sT[j] = __builtin_fmaf(zT, wt[j], sT[j]);
-        sL[j] = __builtin_fmaf(zL, wl[j], sL[j]);
-      }
-    }
-    if (eg > 0) __syncthreads();   // the tiles of the previous group have gone out
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      outT[lane * kXS + wave * 16 + j] = softplus(sT[j]);
-      outL[lane * kXS + wave * 16 + j] = softplus(sL[j]);
-    }
-    __syncthreads();
-    TL::store(outT, kXS, static_cast<T*>(a.dT_out), p0, a.P, a.E, eg * kKC, tid, nullptr);
-    TL::store(outL, kXS, static_cast<T*>(a.dL_out), p0, a.P, a.E, eg * kKC, tid, nullptr);
-  }
-}
-
-// ------------------------------------------------------------------------------- backward, data
-// One workgroup per tile.  LDS: dps[2][64][65] (chunks of dpreT, dpreL; reused for the dx tile),
-// dzs[64][O+1].  Writes dz for the weight-gradient kernel and adds dz Wx to dx.
-template <typename T, bool VEC>
-__global__ __launch_bounds__(kThreads) void m2d_proj_bwd_data_kernel(const ProjArgs a) {
-  using TL = Tile<T, VEC>;
-  extern __shared__ float smem[];
-  float* dps = smem;
-  float* dzs = smem + 2 * kTP * kXS;
-  const int zst = a.O + 1;
-  const int wave = wave_id(), lane = threadIdx.x & 63, tid = threadIdx.x;
-  const int64_t p0 = (int64_t)blockIdx.x * kTP;
-  const int R = a.R, R2 = 2 * a.R;
-  const int nRC = a.Rpad / 16;   // 16-wide chunks of one dt weight; 2*nRC chunks in all (T then L)
-  const int nkc = a.Epad / kKC;
-  const T* dT = static_cast<const T*>(a.dT);
-  const T* dL = static_cast<const T*>(a.dL);
-  const T* ddT = static_cast<const T*>(a.ddT);
-  const T* ddL = static_cast<const T*>(a.ddL);
-  const bool given = a.dpre_given != 0;   // (uniform) ddT, ddL are dpre already
-  const int64_t Pv = given ? 0 : a.P;     // rows of deltaT, deltaL to read: none then
-
-  // dB_T, dB_L, dC of the tile: 64 x 16 contiguous elements each, 4 per thread
-  float bc[3][4];
-#pragma unroll
-  for (int w = 0; w < 3; ++w) {
-    const T* src = static_cast<const T*>(w == 0 ? a.dBT : (w == 1 ? a.dBL : a.dC));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int i = k * kThreads + tid;
-      bc[w][k] = p0 + (i >> 4) < a.P ? ld(src + p0 * kN + i) : 0.f;
-    }
-  }
-
-  float acc[kMaxRounds][16];
-#pragma unroll
-  for (int rd = 0; rd < kMaxRounds; ++rd)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[rd][j] = 0.f;
-
-  for (int kc = 0; kc < nkc; ++kc) {
-    typename TL::Regs gT, vT, gL, vL;
-    TL::load(gT, ddT, p0, a.P, a.E, kc * kKC, tid);
-    TL::load(vT, dT, p0, Pv, a.E, kc * kKC, tid);
-    TL::load(gL, ddL, p0, a.P, a.E, kc * kKC, tid);
-    TL::load(vL, dL, p0, Pv, a.E, kc * kKC, tid);
-    TL::to_lds(dps, kXS, tid, [&](int l, int j) { return TL::get(gT, l, j) * (given ? 1.f : softplus_slope(TL::get(vT, l, j))); });
-    TL::to_lds(dps + kTP * kXS, kXS, tid, [&](int l, int j) { return TL::get(gL, l, j) * (given ? 1.f : softplus_slope(TL::get(vL, l, j))); });
-    __syncthreads();
-#pragma unroll
-    for (int rd = 0; rd < kMaxRounds; ++rd) {
-      const int ci = wave + kWaves * rd;
-      if (ci < 2 * nRC) {
-        const bool isL = ci >= nRC;
-        const int qc = isL ? ci - nRC : ci;
-        row_times_weights(dps + (isL ? kTP * kXS : 0) + lane * kXS,
-                          as_const(isL ? a.wLp : a.wTp) + (int64_t)kc * kKC * a.Rpad + qc * 16, a.Rpad, acc[rd]);
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int rd = 0; rd < kMaxRounds; ++rd) {
-    const int ci = wave + kWaves * rd;
-    if (ci < 2 * nRC) {
-      const bool isL = ci >= nRC;
-      const int qc = isL ? ci - nRC : ci;
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        if (qc * 16 + j < R) dzs[lane * zst + (isL ? R : 0) + qc * 16 + j] = acc[rd][j];
-    }
-  }
-#pragma unroll
-  for (int w = 0; w < 3; ++w)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int i = k * kThreads + tid;
-      dzs[(i >> 4) * zst + R2 + w * kN + (i & 15)] = bc[w][k];
-    }
-  __syncthreads();
-
-  for (int c = wave; c < kTP; c += kWaves) {
-    const int64_t p = p0 + c;
-    if (p >= a.P) break;   // uniform
-    for (int o = lane; o < a.O4; o += 64) a.dz[p * a.O4 + o] = o < a.O ? dzs[c * zst + o] : 0.f;
-  }
-
-  // ---- dx += dz Wx, 64 channels at a time (16 per wave), through LDS for row-wise stores
-  T* dx = static_cast<T*>(a.dx);
-  float* outs = dps;
-  for (int eg = 0; eg < nkc; ++eg) {
-    typename TL::Regs old;
-    TL::load(old, dx, p0, a.P, a.E, eg * kKC, tid);
-    float s[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) s[j] = 0.f;
-    const_floats w = as_const(a.Wp) + eg * kKC + wave * 16;
-    const float* zrow = dzs + lane * zst;
-#pragma unroll 2
-    for (int o = 0; o < a.O; ++o) {
-      const float v = zrow[o];
-      const_floats wo = w + (int64_t)o * a.Epad;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) s[j] = __builtin_fmaf(v, wo[j], s[j]);
-    }
-    if (eg > 0) __syncthreads();   // the previous tile has gone out
-#pragma unroll
-    for (int j = 0; j < 16; ++j) outs[lane * kXS + wave * 16 + j] = s[j];
-    __syncthreads();
-    TL::store(outs, kXS, dx, p0, a.P, a.E, eg * kKC, tid, &old);
   }
 }
 
@@ -952,149 +618,470 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_bwd_weights_mfma_kernel(con
   }
 }
 
-// ------------------------------------------------------------------------------- backward, weights
-// Grid (G, ne): workgroup (g, ey) adds up, over the tiles g, g+G, ..., the gradients of the weights
-// that touch channels [64 ey, 64 ey + 64) and leaves them in part[g][ey][row][64]:
+// ------------------------------------------------------------------------------- fp32 products
+// fp32 tensors, and bf16 ones whose rows are no whole 16-byte chunks, take the products through
+// v_mfma_f32_16x16x4f32: fp32 operands and sums, half again the rate of the vector ALUs measured here, and a weight is
+// one register of a lane in place of a scalar load the whole wave waits for.  Operands (lane l, n = l & 15, kb = l >> 4):
+//   A[n][kb], B[kb][n], one register each;  D[4 kb + i][n], i < 4.
+// The inner index may run in any order, the same one for A and B: at step j of 16 a lane holds index 4 kb + j, so both
+// operands are float4 loads along a row, and a D tile (4 consecutive rows of a column per lane) is at once the B operand
+// of the next product over its rows.  Positions are columns everywhere: z feeds the step sizes' products, and dz those
+// of dx, without leaving the registers, and a lane stores 4 consecutive channels.
+// A wave owns NT x 16 positions and needs no other wave: no LDS, no barrier, no packed copies of the weights.
+// What bounds them is the traffic of the (P,E) arrays and, on few positions, the chain load - product - product - store.
+// The outputs of Wx come in NL = ceil(2R/16) tiles of low-rank inputs and one tile each of B_T, B_L, C; "o'" below counts
+// them with the padding behind 2R.
+template <typename T, bool V4>
+__device__ __forceinline__ f32x4 row4(const T* row, int c, int n) {   // elements c..c+3 of a row of n; past the end any element of the row
+  f32x4 v;
+  if constexpr (V4) {
+    const int cc = c < n ? c : n - 4;
+    if constexpr (sizeof(T) == 4) v = *reinterpret_cast<const f32x4*>(row + cc);
+    else {
+      const uint2 q = *reinterpret_cast<const uint2*>(row + cc);
+      v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u);
+      v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = ld(row + (c + j < n ? c + j : n - 1));
+  }
+  return v;
+}
+__device__ __forceinline__ f32x4 none_past(f32x4 v, int c, int n) {   // element j zero where c + j >= n
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = c + j < n ? v[j] : 0.f;
+  return v;
+}
+template <typename T, bool V4>
+__device__ __forceinline__ void put4(T* row, int c, int n, f32x4 v) {
+  if constexpr (V4) {
+    if (c >= n) return;
+    if constexpr (sizeof(T) == 4) *reinterpret_cast<f32x4*>(row + c) = v;
+    else *reinterpret_cast<uint2*>(row + c) = make_uint2(pack_bf16_pair(v[0], v[1]), pack_bf16_pair(v[2], v[3]));
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (c + j < n) st(row + c + j, v[j]);
+  }
+}
+// a weight as the kernels are to see it (bf16 tensors: rounded if the caller asks for it)
+template <typename T>
+__device__ __forceinline__ f32x4 weights_of(const ProjArgs& a, f32x4 v) {
+  if constexpr (sizeof(T) == 2) {
+    if (a.round) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = as_stored(v[j], static_cast<const bf16_t*>(nullptr));
+    }
+  }
+  return v;
+}
+__device__ __forceinline__ f32x4 mfma4(float x, float y, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
+// The four ranks o' = c .. c+3 of the stacked dt weights as they are for one of the two (first: its first o'): the
+// element index inside a row of R, and whether the rank is one of its own.
+struct Ranks { int at[4]; bool own[4]; };
+__device__ __forceinline__ Ranks ranks_of(int c, int first, int R) {
+  Ranks r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int q = c + j - first;
+    r.own[j] = q >= 0 && q < R;
+    r.at[j] = r.own[j] ? q : 0;
+  }
+  return r;
+}
+
+template <typename T, bool V4, int NL, int NT>
+__global__ __launch_bounds__(kThreads) void m2d_proj_fwd_f32_kernel(const ProjArgs a) {
+  constexpr int NO = NL + 3;
+  const int lane = threadIdx.x & 63, n = lane & 15, kb = lane >> 4;
+  const int64_t p0 = ((int64_t)blockIdx.x * kWaves + wave_id()) * (16 * NT);
+  if (p0 >= a.P) return;
+  const int E = a.E, R = a.R, R2 = 2 * a.R;
+  const int left = (int)(a.P - p0 < 16 * NT ? a.P - p0 : 16 * NT);
+  const T* x = static_cast<const T*>(a.x) + p0 * E;
+  int pl[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) pl[t] = 16 * t + n < left ? 16 * t + n : left - 1;
+  // the rows of Wx behind row n of every tile: B_T, B_L, C in the order of the scan's records (see record_slot) if packed
+  int wrow[NO];
+#pragma unroll
+  for (int ot = 0; ot < NO; ++ot) {
+    const int i = n & 3, state = 4 * (i == 1 ? 2 : (i == 2 ? 1 : i)) + (n >> 2);
+    const int o = ot < NL ? 16 * ot + n : R2 + 16 * (ot - NL) + (a.bc_packed ? state : n);
+    wrow[ot] = (ot < NL && o >= R2 ? R2 - 1 : o) * E;    // (rows of padding repeat one: their products are dropped)
+  }
+  f32x4 z[NT][NO];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int ot = 0; ot < NO; ++ot) z[t][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 xv[NT], wv[NO];
+  auto fetch = [&](int c) {
+    const int e = c + 4 * kb;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) xv[t] = row4<T, V4>(x + (int64_t)pl[t] * E, e, E);
+#pragma unroll
+    for (int ot = 0; ot < NO; ++ot) wv[ot] = row4<float, V4>(a.Wx + wrow[ot], e, E);
+  };
+  fetch(0);
+  for (int c = 0; c < E; c += 16) {
+    f32x4 xc[NT], wc[NO];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) xc[t] = xv[t];
+#pragma unroll
+    for (int ot = 0; ot < NO; ++ot) wc[ot] = weights_of<T>(a, wv[ot]);
+    if (c + 16 < E) fetch(c + 16);
+    if (c + 16 > E) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) xc[t] = none_past(xc[t], c + 4 * kb, E);
+#pragma unroll
+      for (int ot = 0; ot < NO; ++ot) wc[ot] = none_past(wc[ot], c + 4 * kb, E);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int ot = 0; ot < NO; ++ot)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) z[t][ot] = mfma4(wc[ot][j], xc[t][j], z[t][ot]);
+  }
+
+  // low-rank inputs (the step sizes' products see them as the tensor holds them) and B_T, B_L, C
+  const T* as = nullptr;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const bool live = 16 * t + n < left;
+    const int64_t p = p0 + 16 * t + n;
+#pragma unroll
+    for (int ot = 0; ot < NO; ++ot) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) z[t][ot][j] = as_stored(z[t][ot][j], as);
+      const int o = 16 * ot + 4 * kb;
+      if (!live) continue;
+      if (ot < NL) {
+        T* dst = static_cast<T*>(a.r_out) + p * R2;
+        if (R2 % 4 == 0) put4<T, true>(dst, o, R2, z[t][ot]);
+        else put4<T, false>(dst, o, R2, z[t][ot]);
+      } else if (a.bc_packed) {
+        put4<float, true>(a.bc_packed + p * (3 * kN) + (ot - NL) * kN, 4 * kb, kN, z[t][ot]);
+      } else {
+        put4<T, true>(static_cast<T*>(ot == NL ? a.BT_out : (ot == NL + 1 ? a.BL_out : a.C_out)) + p * kN, 4 * kb, kN, z[t][ot]);
+      }
+    }
+  }
+
+  // delta = softplus(r w^T + b), 16 channels at a time
+  Ranks rk[2][NL];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int lt = 0; lt < NL; ++lt) rk[h][lt] = ranks_of(16 * lt + 4 * kb, h * R, R);
+  f32x4 dw[2][NL], bias[2];
+  auto fetch_dt = [&](int e0) {
+    const int e = e0 + n < E ? e0 + n : E - 1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float* w = (h ? a.wL : a.wT) + e * R;
+#pragma unroll
+      for (int lt = 0; lt < NL; ++lt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dw[h][lt][j] = w[rk[h][lt].at[j]];
+      bias[h] = row4<float, V4>(h ? a.bL : a.bT, e0 + 4 * kb, E);
+    }
+  };
+  fetch_dt(0);
+  for (int e0 = 0; e0 < E; e0 += 16) {
+    f32x4 s[NT][2], w[2][NL];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4 b = weights_of<T>(a, bias[h]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) s[t][h] = b;
+#pragma unroll
+      for (int lt = 0; lt < NL; ++lt) {
+        w[h][lt] = weights_of<T>(a, dw[h][lt]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[h][lt][j] = rk[h][lt].own[j] ? w[h][lt][j] : 0.f;
+      }
+    }
+    if (e0 + 16 < E) fetch_dt(e0 + 16);
+#pragma unroll
+    for (int lt = 0; lt < NL; ++lt)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (h ? 16 * lt + 16 <= R : 16 * lt >= R) continue;   // (uniform) the tile holds no rank of this half
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) s[t][h] = mfma4(w[h][lt][j], z[t][lt][j], s[t][h]);
+      }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (16 * t + n >= left) continue;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[t][h][j] = softplus(s[t][h][j]);
+        put4<T, V4>(static_cast<T*>(h ? a.dL_out : a.dT_out) + (p0 + 16 * t + n) * E, e0 + 4 * kb, E, s[t][h]);
+      }
+    }
+  }
+}
+
+// Writes dz (fp32, rows of 16 (NL + 3), o' order) for the weights' gradients and adds dz Wx to dx.
+template <typename T, bool V4, int NL, int NT>
+__global__ __launch_bounds__(kThreads) void m2d_proj_bwd_data_f32_kernel(const ProjArgs a) {
+  constexpr int NO = NL + 3;
+  const int lane = threadIdx.x & 63, n = lane & 15, kb = lane >> 4;
+  const int64_t p0 = ((int64_t)blockIdx.x * kWaves + wave_id()) * (16 * NT);
+  if (p0 >= a.P) return;
+  const int E = a.E, R = a.R, R2 = 2 * a.R;
+  const int left = (int)(a.P - p0 < 16 * NT ? a.P - p0 : 16 * NT);
+  const bool given = a.dpre_given != 0;   // (uniform) ddT, ddL are dpre already
+  int64_t at[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) at[t] = p0 + (16 * t + n < left ? 16 * t + n : left - 1);
+
+  f32x4 z[NT][NO];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+#pragma unroll
+    for (int ot = 0; ot < NL; ++ot) z[t][ot] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 3; ++w)
+      z[t][NL + w] = row4<T, true>(static_cast<const T*>(w == 0 ? a.dBT : (w == 1 ? a.dBL : a.dC)) + at[t] * kN, 4 * kb, kN);
+  }
+  // dz of the low-rank inputs: row n of tile lt is rank 16 lt + n of the two stacked
+  int q[2][NL];
+  bool own[2][NL];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int lt = 0; lt < NL; ++lt) {
+      const int k = 16 * lt + n - h * R;
+      own[h][lt] = k >= 0 && k < R;
+      q[h][lt] = own[h][lt] ? k : 0;
+    }
+  f32x4 gv[2][NT], dv[2][NT], wv[2][NL];
+  auto fetch = [&](int c) {
+    const int e = c + 4 * kb;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        gv[h][t] = row4<T, V4>(static_cast<const T*>(h ? a.ddL : a.ddT) + at[t] * E, e, E);
+        if (!given) dv[h][t] = row4<T, V4>(static_cast<const T*>(h ? a.dL : a.dT) + at[t] * E, e, E);
+      }
+#pragma unroll
+      for (int lt = 0; lt < NL; ++lt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) wv[h][lt][j] = (h ? a.wL : a.wT)[(e + j < E ? e + j : E - 1) * R + q[h][lt]];
+    }
+  };
+  fetch(0);
+  for (int c = 0; c < E; c += 16) {
+    f32x4 g[2][NT], w[2][NL];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        g[h][t] = gv[h][t];
+        if (!given) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) g[h][t][j] *= softplus_slope(dv[h][t][j]);
+        }
+      }
+#pragma unroll
+      for (int lt = 0; lt < NL; ++lt) {
+        w[h][lt] = weights_of<T>(a, wv[h][lt]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[h][lt][j] = own[h][lt] ? w[h][lt][j] : 0.f;
+      }
+    }
+    if (c + 16 < E) fetch(c + 16);
+    if (c + 16 > E) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) g[h][t] = none_past(g[h][t], c + 4 * kb, E);
+    }
+#pragma unroll
+    for (int lt = 0; lt < NL; ++lt)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (h ? 16 * lt + 16 <= R : 16 * lt >= R) continue;   // (uniform) the tile holds no rank of this half
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) z[t][lt] = mfma4(w[h][lt][j], g[h][t][j], z[t][lt]);
+      }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (16 * t + n >= left) continue;
+#pragma unroll
+    for (int ot = 0; ot < NO; ++ot) *reinterpret_cast<f32x4*>(a.dz + at[t] * (16 * NO) + 16 * ot + 4 * kb) = z[t][ot];
+  }
+
+  // dx += dz Wx, 64 channels at a time: a float4 of a row of Wx is row n of four tiles, channel 4n + c of the 64 in tile c,
+  // so the four tiles of a lane hold the channels 16 kb + 4i + c
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    f32x4 s[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 old = row4<T, V4>(static_cast<const T*>(a.dx) + at[t] * E, e0 + 16 * kb + 4 * i, E);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[t][c][i] = old[c];
+      }
+#pragma unroll
+    for (int ot = 0; ot < NO; ++ot)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int oo = 16 * ot + 4 * kb + j;
+        const int o = ot < NL ? (oo < R2 ? oo : R2 - 1) : oo - 16 * NL + R2;   // (rows of padding: dz is zero)
+        const f32x4 w = weights_of<T>(a, row4<float, V4>(a.Wx + o * E, e0 + 4 * n, E));
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) s[t][c] = mfma4(w[c], z[t][ot][j], s[t][c]);
+      }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (16 * t + n >= left) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        put4<T, V4>(static_cast<T*>(a.dx) + at[t] * E, e0 + 16 * kb + 4 * i, E, f32x4{s[t][0][i], s[t][1][i], s[t][2][i], s[t][3][i]});
+    }
+  }
+}
+
+// Grid (G, ne): workgroup (g, ey) adds up, over the tiles of 64 positions g, g+G, ..., the gradients of the weights that
+// touch channels [64 ey, 64 ey + 64) and leaves them in part[g][ey][row][64]:
 //   rows 0..O-1      dWx[o][.]      = sum_p dz[p][o] x[p][.]
 //   rows O..O+R-1    dwT[.][q]      = sum_p dpreT[p][.] rT[p][q]      rows O+R..O+2R-1 the same for L
 //   rows O+2R, +1    dbT[.], dbL[.] = sum_p dpre[p][.]
-// LDS: xs[64][68], dpT[64][65], dpL[64][65], dzs[64][O4], rs[64][2R].  The loads of the next tile
-// are under way while the sums of the current one are formed.
-template <typename T, bool VEC>
-__global__ __launch_bounds__(kThreads) void m2d_proj_bwd_weights_kernel(const ProjArgs a) {
-  using TL = Tile<T, VEC>;
-  extern __shared__ float smem[];
-  const int O4 = a.O4;
-  const int R = a.R, R2 = 2 * a.R;
-  float* xs = smem;
-  float* dpT = xs + kTP * kXS4;
-  float* dpL = dpT + kTP * kXS;
-  float* dzs = dpL + kTP * kXS;
-  float* rs = dzs + kTP * O4;
-  const int wave = wave_id(), lane = threadIdx.x & 63, tid = threadIdx.x;
-  const int ey = blockIdx.y;
-  const T* x = static_cast<const T*>(a.x);
-  const T* rr = static_cast<const T*>(a.r);
-  const T* dT = static_cast<const T*>(a.dT);
-  const T* dL = static_cast<const T*>(a.dL);
-  const T* ddT = static_cast<const T*>(a.ddT);
-  const T* ddL = static_cast<const T*>(a.ddL);
+// Positions are the inner index here, 4 to a step, one per lane group kb: a lane's float4 along the channels (or along
+// the first 64 outputs) is row or column n of four tiles, so a step is four float4 loads and 24 to 44 products.  A wave
+// takes 16 positions of a tile; the four waves add up in LDS at the end.
+template <typename T, bool V4, int NL>
+__global__ __launch_bounds__(kThreads) void m2d_proj_bwd_weights_f32_kernel(const ProjArgs a) {
+  constexpr int NO = NL + 3, RT = NL > 2 ? 2 : 1;
+  extern __shared__ float sum[];
+  const int lane = threadIdx.x & 63, n = lane & 15, kb = lane >> 4, wave = wave_id();
+  const int E = a.E, R = a.R, R2 = 2 * a.R, e0 = blockIdx.y * kKC;
   const bool given = a.dpre_given != 0;   // (uniform) ddT, ddL are dpre already
-  const int64_t Pv = given ? 0 : a.P;     // rows of deltaT, deltaL to read: none then
-  const int nmt = (O4 / 4) * 16;   // 4 x 4 blocks of dWx: (o4, e4), e4 fastest
-  constexpr int kZQ = (kTP * ((2 * kMaxR + 3 * kN + 3) / 4) + kThreads - 1) / kThreads;   // float4 of dz per thread, at most
-  constexpr int kRQ = (kTP * 2 * kMaxR + kThreads - 1) / kThreads;                        // elements of r per thread, at most
-  const int nzq = kTP * O4 / 4, nrq = kTP * R2;
-
-  float aw[2][16], ar[2][kMaxR / kWaves], ab[2] = {0.f, 0.f};
+  f32x4 aw[4][4], ax[NL > 1 ? NL - 1 : 1][4], ad[2][RT][4], ab[2];
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int c = 0; c < 4; ++c) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) aw[h][j] = 0.f;
+    for (int o = 0; o < 4; ++o) aw[o][c] = zero;
 #pragma unroll
-    for (int i = 0; i < kMaxR / kWaves; ++i) ar[h][i] = 0.f;
+    for (int o = 0; o + 1 < NL; ++o) ax[o][c] = zero;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) ad[h][r][c] = zero;
   }
+  ab[0] = ab[1] = zero;
 
-  typename TL::Regs xr, gT, vT, gL, vL;
-  float4 zq[kZQ];
-  float rq[kRQ];
-  auto fetch = [&](int tile) {
-    const int64_t p0 = (int64_t)tile * kTP;
-    TL::load(xr, x, p0, a.P, a.E, ey * kKC, tid);
-    TL::load(gT, ddT, p0, a.P, a.E, ey * kKC, tid);
-    TL::load(vT, dT, p0, Pv, a.E, ey * kKC, tid);
-    TL::load(gL, ddL, p0, a.P, a.E, ey * kKC, tid);
-    TL::load(vL, dL, p0, Pv, a.E, ey * kKC, tid);
-    const int64_t left = a.P - p0;   // rows of the tile inside the array, if fewer than 64
-    const float4* zsrc = reinterpret_cast<const float4*>(a.dz + p0 * O4);
-#pragma unroll
-    for (int k = 0; k < kZQ; ++k) {
-      const int i = k * kThreads + tid;
-      zq[k] = (i < nzq && (int64_t)(4 * i) < left * O4) ? zsrc[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-#pragma unroll
-    for (int k = 0; k < kRQ; ++k) {
-      const int i = k * kThreads + tid;
-      rq[k] = (i < nrq && (int64_t)i < left * R2) ? ld(rr + p0 * R2 + i) : 0.f;
-    }
-  };
-
-  if ((int)blockIdx.x < a.ntiles) fetch(blockIdx.x);
-  for (int tile = blockIdx.x; tile < a.ntiles; tile += a.G) {
-    TL::to_lds(xs, kXS4, tid, [&](int l, int j) { return TL::get(xr, l, j); });
-    TL::to_lds(dpT, kXS, tid, [&](int l, int j) { return TL::get(gT, l, j) * (given ? 1.f : softplus_slope(TL::get(vT, l, j))); });
-    TL::to_lds(dpL, kXS, tid, [&](int l, int j) { return TL::get(gL, l, j) * (given ? 1.f : softplus_slope(TL::get(vL, l, j))); });
-#pragma unroll
-    for (int k = 0; k < kZQ; ++k) {
-      const int i = k * kThreads + tid;
-      if (i < nzq) reinterpret_cast<float4*>(dzs)[i] = zq[k];
-    }
-#pragma unroll
-    for (int k = 0; k < kRQ; ++k) {
-      const int i = k * kThreads + tid;
-      if (i < nrq) rs[i] = rq[k];
-    }
-    __syncthreads();
-    if (tile + a.G < a.ntiles) fetch(tile + a.G);
+  f32x4 zv, xv, gv[2], dv[2];
+  float zx[NL > 1 ? NL - 1 : 1], rv[2][RT];
+  auto fetch = [&](int64_t p_raw) {
+    const bool ok = p_raw < a.P;
+    const int64_t p = ok ? p_raw : a.P - 1;
+    const float* z = a.dz + p * (16 * NO);
+    zv = *reinterpret_cast<const f32x4*>(z + 4 * n);
+    xv = row4<T, V4>(static_cast<const T*>(a.x) + p * E, e0 + 4 * n, E);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int mt = tid + kThreads * h;
-      if (mt < nmt) {
-        const float4* zp = reinterpret_cast<const float4*>(dzs + 4 * (mt >> 4));
-        const float4* xp = reinterpret_cast<const float4*>(xs + 4 * (mt & 15));
-#pragma unroll 4
-        for (int c = 0; c < kTP; ++c) {
-          const float4 z4 = zp[c * (O4 / 4)], x4 = xp[c * (kXS4 / 4)];
-          const float zz[4] = {z4.x, z4.y, z4.z, z4.w}, xx[4] = {x4.x, x4.y, x4.z, x4.w};
+      gv[h] = row4<T, V4>(static_cast<const T*>(h ? a.ddL : a.ddT) + p * E, e0 + 4 * n, E);
+      if (!given) dv[h] = row4<T, V4>(static_cast<const T*>(h ? a.dL : a.dT) + p * E, e0 + 4 * n, E);
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) aw[h][4 * i + j] = __builtin_fmaf(zz[i], xx[j], aw[h][4 * i + j]);
-        }
-      }
+      for (int r = 0; r < RT; ++r) rv[h][r] = ld(static_cast<const T*>(a.r) + p * R2 + h * R + (16 * r + n < R ? 16 * r + n : R - 1));
     }
-    // dt weights: this thread's channel is `lane`, its ranks are wave, wave + 4, ...
-#pragma unroll 2
-    for (int c = 0; c < kTP; ++c) {
-      const float tT = dpT[c * kXS + lane], tL = dpL[c * kXS + lane];
-      const float* rc = rs + c * R2;
-      if (wave == 0) { ab[0] += tT; ab[1] += tL; }
 #pragma unroll
-      for (int i = 0; i < kMaxR / kWaves; ++i) {
-        const int q = wave + kWaves * i;
-        if (q < R) {
-          ar[0][i] = __builtin_fmaf(tT, rc[q], ar[0][i]);
-          ar[1][i] = __builtin_fmaf(tL, rc[R + q], ar[1][i]);
-        }
+    for (int o = 0; o + 1 < NL; ++o) zx[o] = z[64 + 16 * o + n];
+  };
+  const int steps = ((a.ntiles - (int)blockIdx.x + a.G - 1) / a.G) * 4;    // (G <= ntiles: at least 4)
+  auto position = [&](int s) { return ((int64_t)blockIdx.x + (int64_t)(s >> 2) * a.G) * kTP + wave * 16 + (s & 3) * 4 + kb; };
+  fetch(position(0));
+  for (int s = 0; s < steps; ++s) {
+    const bool ok = position(s) < a.P;
+    f32x4 zc = zv, xc = xv, g[2];
+    float zxc[NL > 1 ? NL - 1 : 1], rc[2][RT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      g[h] = gv[h];
+      if (!given) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) g[h][j] *= softplus_slope(dv[h][j]);
       }
+#pragma unroll
+      for (int r = 0; r < RT; ++r) rc[h][r] = rv[h][r];
+    }
+#pragma unroll
+    for (int o = 0; o + 1 < NL; ++o) zxc[o] = zx[o];
+    if (s + 1 < steps) fetch(position(s + 1));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { zc[j] = ok ? zc[j] : 0.f; g[0][j] = ok ? g[0][j] : 0.f; g[1][j] = ok ? g[1][j] : 0.f; }
+    ab[0] += g[0]; ab[1] += g[1];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int o = 0; o < 4; ++o) aw[o][c] = mfma4(zc[o], xc[c], aw[o][c]);
+#pragma unroll
+      for (int o = 0; o + 1 < NL; ++o) ax[o][c] = mfma4(ok ? zxc[o] : 0.f, xc[c], ax[o][c]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < RT; ++r) ad[h][r][c] = mfma4(g[h][c], rc[h][r], ad[h][r][c]);
+    }
+  }
+
+  // the four waves in turn, in the layout of the parts
+  const int rows = a.O + R2 + 2;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      ab[h][j] += __shfl_xor(ab[h][j], 16, 64);
+      ab[h][j] += __shfl_xor(ab[h][j], 32, 64);
+    }
+  for (int w = 0; w < kWaves; ++w) {
+    if (w == wave) {
+      auto add4 = [&](int row, int col, f32x4 v) {
+        f32x4* d = reinterpret_cast<f32x4*>(sum + row * kKC + col);
+        *d = w ? *d + v : v;
+      };
+      auto row_of = [&](int oo) { return oo < 16 * NL ? (oo < R2 ? oo : -1) : oo - 16 * NL + R2; };   // o' -> row, -1: padding
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+          const int row = row_of(4 * (4 * kb + i) + o);
+          if (row >= 0) add4(row, 4 * n, f32x4{aw[o][0][i], aw[o][1][i], aw[o][2][i], aw[o][3][i]});
+        }
+#pragma unroll
+        for (int o = 0; o + 1 < NL; ++o) {
+          const int row = row_of(64 + 16 * o + 4 * kb + i);
+          if (row >= 0) add4(row, 4 * n, f32x4{ax[o][0][i], ax[o][1][i], ax[o][2][i], ax[o][3][i]});
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            if (16 * r + n < R)
+              add4(a.O + h * R + 16 * r + n, 4 * (4 * kb + i), f32x4{ad[h][r][0][i], ad[h][r][1][i], ad[h][r][2][i], ad[h][r][3][i]});
+      }
+      if (kb < 2) add4(a.O + R2 + kb, 4 * n, kb ? ab[1] : ab[0]);
     }
     __syncthreads();
   }
-
-  float* out = a.part + ((int64_t)blockIdx.x * a.ne + ey) * (int64_t)(a.O + R2 + 2) * kKC;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int mt = tid + kThreads * h;
-    if (mt < nmt) {
-      const int o0 = 4 * (mt >> 4), e0 = 4 * (mt & 15);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (o0 + i < a.O)
-          *reinterpret_cast<float4*>(out + (o0 + i) * kKC + e0) = make_float4(aw[h][4 * i], aw[h][4 * i + 1], aw[h][4 * i + 2], aw[h][4 * i + 3]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < kMaxR / kWaves; ++i) {
-    const int q = wave + kWaves * i;
-    if (q < R) {
-      out[(a.O + q) * kKC + lane] = ar[0][i];
-      out[(a.O + R + q) * kKC + lane] = ar[1][i];
-    }
-  }
-  if (wave == 0) {
-    out[(a.O + R2) * kKC + lane] = ab[0];
-    out[(a.O + R2 + 1) * kKC + lane] = ab[1];
-  }
+  float* out = a.part + ((int64_t)blockIdx.x * a.ne + blockIdx.y) * (int64_t)rows * kKC;
+  for (int i = threadIdx.x; i < rows * (kKC / 4); i += kThreads) reinterpret_cast<f32x4*>(out)[i] = reinterpret_cast<const f32x4*>(sum)[i];
 }
 
 // Sums the per-workgroup parts in a fixed order and scatters them to the five weight gradients.
@@ -1130,13 +1117,12 @@ inline bool misaligned(const void* p, size_t a) { return (reinterpret_cast<uintp
 
 struct ProjGeometry {
   int64_t P;
-  int E, R, O, O4, Epad, Opad, Opad32, Rpad, ntiles, G, ne;
-  bool vec;    // rows of the (P,E) arrays start on 16-byte boundaries
-  bool mfma;   // bf16 and vec: products on the matrix cores
+  int E, R, O, Epad, Opad, Opad32, Rpad, ntiles, G, ne;
+  bool mfma;   // bf16, and rows of the (P,E) arrays start on 16-byte boundaries: products with bf16 operands
   // forward workspace
-  size_t off_Wt, off_wTt, off_wLt, off_bTp, off_bLp, off_Wb, off_wTb, off_wLb, bytes_fwd;
+  size_t off_bTp, off_bLp, off_Wb, off_wTb, off_wLb, bytes_fwd;
   // backward workspace
-  size_t off_Wp, off_wTp, off_wLp, off_wTtb, off_wLtb, off_WxTb, off_dz, off_dpt, off_part, bytes_bwd;
+  size_t off_wTtb, off_wLtb, off_WxTb, off_dz, off_dpt, off_part, bytes_bwd;
 };
 
 int check_proj(const m2d_desc* d, int R) {
@@ -1153,21 +1139,16 @@ ProjGeometry proj_geometry(const m2d_desc* d, int R) {
   ProjGeometry g;
   g.P = (int64_t)d->B * d->H * d->W;
   g.E = d->E; g.R = R; g.O = 2 * R + 3 * kN;
-  g.O4 = (g.O + 3) & ~3;
   g.Epad = (g.E + kKC - 1) / kKC * kKC;
   g.Opad = (g.O + 15) / 16 * 16;
   g.Opad32 = (g.O + 31) / 32 * 32;
   g.Rpad = (R + 15) / 16 * 16;
   g.ntiles = (int)((g.P + kTP - 1) / kTP);
   g.ne = g.Epad / kKC;
-  g.vec = d->E % (d->dtype == M2D_F32 ? 4 : 8) == 0;
-  g.mfma = g.vec && d->dtype == M2D_BF16;
+  g.mfma = d->dtype == M2D_BF16 && d->E % 8 == 0;
   const int want = 512 / g.ne > 0 ? 512 / g.ne : 1;   // about two workgroups per compute unit in all
   g.G = g.ntiles < want ? g.ntiles : want;
   size_t o = 0;
-  g.off_Wt = o; o += align256((size_t)g.Epad * g.Opad * 4);
-  g.off_wTt = o; o += align256((size_t)R * g.Epad * 4);
-  g.off_wLt = o; o += align256((size_t)R * g.Epad * 4);
   g.off_bTp = o; o += align256((size_t)g.Epad * 4);
   g.off_bLp = o; o += align256((size_t)g.Epad * 4);
   g.off_Wb = o; o += align256((size_t)g.Opad * g.Epad * 2);
@@ -1175,9 +1156,6 @@ ProjGeometry proj_geometry(const m2d_desc* d, int R) {
   g.off_wLb = o; o += align256((size_t)g.Epad * 32 * 2);
   g.bytes_fwd = o;
   o = 0;
-  g.off_Wp = o; o += align256((size_t)g.O * g.Epad * 4);
-  g.off_wTp = o; o += align256((size_t)g.Epad * g.Rpad * 4);
-  g.off_wLp = o; o += align256((size_t)g.Epad * g.Rpad * 4);
   g.off_wTtb = o; o += align256((size_t)g.Rpad * g.Epad * 2);
   g.off_wLtb = o; o += align256((size_t)g.Rpad * g.Epad * 2);
   g.off_WxTb = o; o += align256((size_t)g.Epad * g.Opad32 * 2);
@@ -1185,7 +1163,7 @@ ProjGeometry proj_geometry(const m2d_desc* d, int R) {
     g.off_dz = o; o += align256((size_t)g.ntiles * kTP * g.Opad * 2);
     g.off_dpt = o; o += align256((size_t)2 * g.ntiles * kTP * g.E * 2);
   } else {
-    g.off_dz = o; o += align256((size_t)g.P * g.O4 * 4);
+    g.off_dz = o; o += align256((size_t)g.P * g.Opad * 4);
     g.off_dpt = o;
   }
   g.off_part = o; o += align256((size_t)g.G * g.ne * (g.O + 2 * R + 2) * kKC * 4);
@@ -1194,28 +1172,11 @@ ProjGeometry proj_geometry(const m2d_desc* d, int R) {
 }
 
 void fill(ProjArgs& a, const ProjGeometry& g) {
-  a.P = g.P; a.E = g.E; a.R = g.R; a.O = g.O; a.O4 = g.O4; a.Epad = g.Epad; a.Opad = g.Opad; a.Opad32 = g.Opad32; a.Rpad = g.Rpad;
+  a.P = g.P; a.E = g.E; a.R = g.R; a.O = g.O; a.Epad = g.Epad; a.Opad = g.Opad; a.Opad32 = g.Opad32; a.Rpad = g.Rpad;
   a.ntiles = g.ntiles; a.G = g.G; a.ne = g.ne;
 }
 
 inline bool launched() { return hipGetLastError() == hipSuccess; }
-
-constexpr int kMaxLdsWeights = (kTP * kXS4 + 2 * kTP * kXS + kTP * ((2 * kMaxR + 3 * kN + 3) & ~3) + kTP * 2 * kMaxR) * 4;
-
-template <typename T, bool VEC>
-bool allow_lds_weights() {
-  // more than 64 KB of dynamic LDS has to be allowed once per device (one bit per device ordinal)
-  static std::atomic<uint64_t> seen{0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  const uint64_t bit = 1ull << (dev & 63);
-  if (seen.load(std::memory_order_relaxed) & bit) return true;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&m2d_proj_bwd_weights_kernel<T, VEC>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsWeights) != hipSuccess)
-    return false;
-  seen.fetch_or(bit, std::memory_order_relaxed);
-  return true;
-}
 
 int run_proj_fwd_mfma(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
   const size_t lds = (size_t)kWaves * (16 * kStageStride * 4 + 2 * 16 * kLowStride * 2);
@@ -1223,35 +1184,62 @@ int run_proj_fwd_mfma(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) 
   return launched() ? M2D_OK : M2D_ERR_HIP;
 }
 
-template <typename T, bool VEC>
-int run_proj_fwd(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
-  const size_t lds = (size_t)(2 * kTP * kXS + kTP * (g.O + 1)) * 4;
-  hipLaunchKernelGGL((m2d_proj_fwd_kernel<T, VEC>), dim3(g.ntiles), dim3(kThreads), lds, st, a);
+// The fp32 products' kernels: V4 where the rows of the (P,E) arrays and of Wx are whole runs of 4 elements, NL tiles of
+// low-rank inputs, NT tiles of 16 positions per wave.
+template <typename F>
+int with_tiles(int R, F f) {
+  switch ((2 * R + 15) / 16) {
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    default: return f(std::integral_constant<int, 4>{});
+  }
+}
+
+template <typename T, bool V4, int NT>
+int run_proj_fwd_f32(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
+  return with_tiles(g.R, [&](auto nl) -> int {
+    const unsigned grid = (unsigned)((g.P + 16 * NT * kWaves - 1) / (16 * NT * kWaves));
+    hipLaunchKernelGGL((m2d_proj_fwd_f32_kernel<T, V4, nl(), NT>), dim3(grid), dim3(kThreads), 0, st, a);
+    return launched() ? M2D_OK : M2D_ERR_HIP;
+  });
+}
+
+int run_reduce(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(m2d_proj_reduce_kernel, dim3(g.O + 2 * g.R + 2, g.ne), dim3(64 * kRedSlices), 0, st, a);
   return launched() ? M2D_OK : M2D_ERR_HIP;
 }
 
-template <typename T, bool VEC>
-int run_proj_bwd(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
-  if (g.mfma) {
-    const size_t lds_data = (size_t)kWaves * (16 * kStageStride * 4 + 16 * (g.Opad32 + 8) * 2);
-    hipLaunchKernelGGL(m2d_proj_bwd_data_mfma_kernel, dim3(g.ntiles), dim3(kThreads), lds_data, st, a);
-    if (!launched()) return M2D_ERR_HIP;
-    const size_t lds_w = (size_t)(3 * kKC + g.Opad + 2 * 16 * ((g.R + 1 + 15) / 16)) * kPosStride * 2;
-    hipLaunchKernelGGL(m2d_proj_bwd_weights_mfma_kernel, dim3(g.G, g.ne), dim3(kThreads), lds_w, st, a);
-    if (!launched()) return M2D_ERR_HIP;
-    hipLaunchKernelGGL(m2d_proj_reduce_kernel, dim3(g.O + 2 * g.R + 2, g.ne), dim3(64 * kRedSlices), 0, st, a);
-    return launched() ? M2D_OK : M2D_ERR_HIP;
-  } else {
-    const size_t lds_data = (size_t)(2 * kTP * kXS + kTP * (g.O + 1)) * 4;
-    hipLaunchKernelGGL((m2d_proj_bwd_data_kernel<T, VEC>), dim3(g.ntiles), dim3(kThreads), lds_data, st, a);
-  }
+int run_proj_bwd_mfma(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
+  const size_t lds_data = (size_t)kWaves * (16 * kStageStride * 4 + 16 * (g.Opad32 + 8) * 2);
+  hipLaunchKernelGGL(m2d_proj_bwd_data_mfma_kernel, dim3(g.ntiles), dim3(kThreads), lds_data, st, a);
   if (!launched()) return M2D_ERR_HIP;
-  const size_t lds_w = (size_t)(kTP * kXS4 + 2 * kTP * kXS + kTP * g.O4 + kTP * 2 * g.R) * 4;
-  if (!allow_lds_weights<T, VEC>()) return M2D_ERR_HIP;
-  hipLaunchKernelGGL((m2d_proj_bwd_weights_kernel<T, VEC>), dim3(g.G, g.ne), dim3(kThreads), lds_w, st, a);
+  const size_t lds_w = (size_t)(3 * kKC + g.Opad + 2 * 16 * ((g.R + 1 + 15) / 16)) * kPosStride * 2;
+  hipLaunchKernelGGL(m2d_proj_bwd_weights_mfma_kernel, dim3(g.G, g.ne), dim3(kThreads), lds_w, st, a);
   if (!launched()) return M2D_ERR_HIP;
-  hipLaunchKernelGGL(m2d_proj_reduce_kernel, dim3(g.O + 2 * g.R + 2, g.ne), dim3(64 * kRedSlices), 0, st, a);
-  return launched() ? M2D_OK : M2D_ERR_HIP;
+  return run_reduce(g, a, st);
+}
+
+template <typename T, bool V4, int NT>
+int run_proj_bwd_f32(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
+  return with_tiles(g.R, [&](auto nl) -> int {
+    const unsigned grid = (unsigned)((g.P + 16 * NT * kWaves - 1) / (16 * NT * kWaves));
+    hipLaunchKernelGGL((m2d_proj_bwd_data_f32_kernel<T, V4, nl(), NT>), dim3(grid), dim3(kThreads), 0, st, a);
+    if (!launched()) return M2D_ERR_HIP;
+    const size_t lds_w = (size_t)(g.O + 2 * g.R + 2) * kKC * 4;   // (at most 45 KB)
+    hipLaunchKernelGGL((m2d_proj_bwd_weights_f32_kernel<T, V4, nl()>), dim3(g.G, g.ne), dim3(kThreads), lds_w, st, a);
+    if (!launched()) return M2D_ERR_HIP;
+    return run_reduce(g, a, st);
+  });
+}
+
+// Two tiles of positions per wave share the loads of the weights, where that still leaves every SIMD two waves.
+template <typename F>
+int with_layout(bool f32, const ProjGeometry& g, F f) {
+  using std::integral_constant;
+  auto tiles = [&](auto t, auto v4) -> int { return g.P >= 65536 ? f(t, v4, integral_constant<int, 2>{}) : f(t, v4, integral_constant<int, 1>{}); };
+  auto rows = [&](auto t) -> int { return g.E % 4 == 0 ? tiles(t, std::true_type{}) : tiles(t, std::false_type{}); };
+  return f32 ? rows(float{}) : rows(bf16_t{});
 }
 
 }  // namespace
@@ -1282,30 +1270,29 @@ int m2d_proj_fwd(const m2d_desc* desc, int dt_rank, const void* x, const float* 
   char* ws = static_cast<char*>(workspace);
   PackArgs k = {};
   k.Wx = x_proj_w; k.wT = dt_projT_w; k.bT = dt_projT_b; k.wL = dt_projL_w; k.bL = dt_projL_b;
-  k.Wt = reinterpret_cast<float*>(ws + g.off_Wt);
-  k.wTt = reinterpret_cast<float*>(ws + g.off_wTt);
-  k.wLt = reinterpret_cast<float*>(ws + g.off_wLt);
-  k.bTp = reinterpret_cast<float*>(ws + g.off_bTp);
-  k.bLp = reinterpret_cast<float*>(ws + g.off_bLp);
-  if (g.mfma) {   // the matrix-core kernel reads the bf16 set
-    k.Wt = nullptr;
+  if (g.mfma) {
+    k.bTp = reinterpret_cast<float*>(ws + g.off_bTp);
+    k.bLp = reinterpret_cast<float*>(ws + g.off_bLp);
     k.Wb = reinterpret_cast<uint16_t*>(ws + g.off_Wb);
     k.wTb = reinterpret_cast<uint16_t*>(ws + g.off_wTb);
     k.wLb = reinterpret_cast<uint16_t*>(ws + g.off_wLb);
+    k.E = g.E; k.R = g.R; k.O = g.O; k.Epad = g.Epad; k.Opad = g.Opad; k.Opad32 = g.Opad32; k.Rpad = g.Rpad;
+    k.round = (desc->flags & M2D_FLAG_ROUND_WEIGHTS) != 0;
+    const int n = g.Epad * (g.Opad > 32 ? g.Opad : 32);   // the largest forward copy
+    hipLaunchKernelGGL(m2d_proj_pack_kernel, dim3((n + 255) / 256), dim3(256), 0, st, k);
+    if (!launched()) return M2D_ERR_HIP;
   }
-  k.E = g.E; k.R = g.R; k.O = g.O; k.Epad = g.Epad; k.Opad = g.Opad; k.Opad32 = g.Opad32; k.Rpad = g.Rpad;
-  k.round = (desc->flags & M2D_FLAG_ROUND_WEIGHTS) && desc->dtype == M2D_BF16;
-  const int n = g.Epad * (g.Opad > 32 ? g.Opad : 32);   // the largest forward copy
-  hipLaunchKernelGGL(m2d_proj_pack_kernel, dim3((n + 255) / 256), dim3(256), 0, st, k);
-  if (!launched()) return M2D_ERR_HIP;
   ProjArgs a = {};
   fill(a, g);
-  a.x = x; a.Wt = k.Wt; a.wTt = k.wTt; a.wLt = k.wLt; a.bTp = k.bTp; a.bLp = k.bLp;
+  a.x = x; a.bTp = k.bTp; a.bLp = k.bLp;
+  a.Wx = x_proj_w; a.wT = dt_projT_w; a.bT = dt_projT_b; a.wL = dt_projL_w; a.bL = dt_projL_b;
+  a.round = (desc->flags & M2D_FLAG_ROUND_WEIGHTS) && desc->dtype == M2D_BF16;
   a.Wb = k.Wb; a.wTb = k.wTb; a.wLb = k.wLb;
   a.r_out = lowrank; a.dT_out = deltaT; a.dL_out = deltaL; a.BT_out = BT; a.BL_out = BL; a.C_out = C;
   a.bc_packed = packed ? static_cast<float*>(BT) : nullptr;
-  if (desc->dtype == M2D_F32) return g.vec ? run_proj_fwd<float, true>(g, a, st) : run_proj_fwd<float, false>(g, a, st);
-  return g.mfma ? run_proj_fwd_mfma(g, a, st) : run_proj_fwd<bf16_t, false>(g, a, st);
+  return g.mfma ? run_proj_fwd_mfma(g, a, st) : with_layout(desc->dtype == M2D_F32, g, [&](auto t, auto v4, auto nt) -> int {
+    return run_proj_fwd_f32<decltype(t), v4(), nt()>(g, a, st);
+  });
 }
 
 int m2d_proj_bwd(const m2d_desc* desc, int dt_rank, const void* x, const void* lowrank, const void* deltaT,
@@ -1340,34 +1327,31 @@ int m2d_proj_bwd_parts(const m2d_desc* desc, int dt_rank, int sum_parts, const v
   char* ws = static_cast<char*>(workspace);
   PackArgs k = {};
   k.Wx = x_proj_w; k.wT = dt_projT_w; k.wL = dt_projL_w;
-  k.Wp = reinterpret_cast<float*>(ws + g.off_Wp);
-  k.wTp = reinterpret_cast<float*>(ws + g.off_wTp);
-  k.wLp = reinterpret_cast<float*>(ws + g.off_wLp);
-  if (g.mfma) {   // the data kernel reads the bf16 set; the weight-gradient kernel needs no weights
-    k.Wp = nullptr;
+  if (g.mfma) {   // for the data kernel; the weight-gradient kernel needs no weights
     k.wTtb = reinterpret_cast<uint16_t*>(ws + g.off_wTtb);
     k.wLtb = reinterpret_cast<uint16_t*>(ws + g.off_wLtb);
     k.WxTb = reinterpret_cast<uint16_t*>(ws + g.off_WxTb);
+    k.E = g.E; k.R = g.R; k.O = g.O; k.Epad = g.Epad; k.Opad = g.Opad; k.Opad32 = g.Opad32; k.Rpad = g.Rpad;
+    int n = g.Opad32 * g.Epad;
+    if (g.Epad * g.Rpad > n) n = g.Epad * g.Rpad;
+    hipLaunchKernelGGL(m2d_proj_pack_kernel, dim3((n + 255) / 256), dim3(256), 0, st, k);
+    if (!launched()) return M2D_ERR_HIP;
   }
-  k.E = g.E; k.R = g.R; k.O = g.O; k.Epad = g.Epad; k.Opad = g.Opad; k.Opad32 = g.Opad32; k.Rpad = g.Rpad;
-  k.round = (desc->flags & M2D_FLAG_ROUND_WEIGHTS) && desc->dtype == M2D_BF16;
-  int n = g.Opad32 * g.Epad;
-  if (g.Epad * g.Rpad > n) n = g.Epad * g.Rpad;
-  hipLaunchKernelGGL(m2d_proj_pack_kernel, dim3((n + 255) / 256), dim3(256), 0, st, k);
-  if (!launched()) return M2D_ERR_HIP;
   ProjArgs a = {};
   fill(a, g);
   a.x = x; a.r = lowrank; a.dT = deltaT; a.dL = deltaL; a.dpre_given = given ? 1 : 0; a.sum_parts = sum_parts;
   a.ddT = d_deltaT; a.ddL = d_deltaL; a.dBT = d_BT; a.dBL = d_BL; a.dC = d_C; a.dx = dx;
-  a.Wp = k.Wp; a.wTp = k.wTp; a.wLp = k.wLp;
+  a.Wx = x_proj_w; a.wT = dt_projT_w; a.wL = dt_projL_w;
+  a.round = (desc->flags & M2D_FLAG_ROUND_WEIGHTS) && desc->dtype == M2D_BF16;
   a.wTtb = k.wTtb; a.wLtb = k.wLtb; a.WxTb = k.WxTb;
   a.dz = reinterpret_cast<float*>(ws + g.off_dz);
   a.dzt = reinterpret_cast<uint16_t*>(ws + g.off_dz);
   a.dpt = reinterpret_cast<uint16_t*>(ws + g.off_dpt);
   a.part = reinterpret_cast<float*>(ws + g.off_part);
   a.dWx = d_x_proj_w; a.dwT = d_dt_projT_w; a.dbT = d_dt_projT_b; a.dwL = d_dt_projL_w; a.dbL = d_dt_projL_b;
-  if (desc->dtype == M2D_F32) return g.vec ? run_proj_bwd<float, true>(g, a, st) : run_proj_bwd<float, false>(g, a, st);
-  return g.vec ? run_proj_bwd<bf16_t, true>(g, a, st) : run_proj_bwd<bf16_t, false>(g, a, st);
+  return g.mfma ? run_proj_bwd_mfma(g, a, st) : with_layout(desc->dtype == M2D_F32, g, [&](auto t, auto v4, auto nt) -> int {
+    return run_proj_bwd_f32<decltype(t), v4(), nt()>(g, a, st);
+  });
 }
 
 }  // extern "C"

@@ -1365,7 +1365,7 @@ __device__ __forceinline__ float skip_gain(const ScanParams& p, int e) {
 }
 // The set-up launch (m2d_prep_kernel) is for kernels whose lanes hold all states of a channel, for a backward that will
 // read the same values, and for progress counts.  A lane here holds 4 states of one channel, so a forward with neither
-// works them out itself and saves the launch and the gap behind it (4 of 15 us on one 14x14x320 image).
+// works them out itself and saves the launch and the gap behind it.
 template <bool CKPT, int MODE>
 constexpr bool split_owns_setup() { return !CKPT && MODE != kModeSliced; }
 __device__ float m2d_zero_page[kZeroFloats];     // the page of zeros of such a forward: never written
