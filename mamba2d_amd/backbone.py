@@ -23,6 +23,7 @@ import weakref
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook as _global_hooks
 
 from . import wavefront
 from .wavefront import (dwconv3x3_fwd_op, layernorm_fwd_op, layernorm_linear_act_fwd_op, linear_act_fwd_op, mlp_fwd_op,
@@ -399,7 +400,7 @@ class ResBlock(nn.Module):
         mix, mlp = self.token_mixer, self.MLP
         if not (x.is_cuda and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda") and x.dim() == 4 and x.numel() > 0
                 and torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.dtype in (torch.float32, torch.bfloat16)
-                and type(mix) is M2DBlock and not torch.compiler.is_compiling() and wavefront.FUSED_PROJECTIONS):
+                and type(mix) is M2DBlock and wavefront._direct(x) and not _global_hooks() and wavefront.FUSED_PROJECTIONS):
             return None
         C = x.shape[-1]
         if C % 32 or C > 128 or x.shape[1] < 2 or x.shape[2] < 2 or mix.recomp not in ("partial", "full"):
@@ -428,7 +429,7 @@ class ResBlock(nn.Module):
                     path.act2.scale, path.act2.bias, path.pwconv2.weight]
             want += [(C,), (C,), (2 * C, C), (1,), (1,), (2 * C, 1, 3, 3), (1,), (1,), (C, 2 * C)]
         for t, shape in zip(par, want):
-            if t is None or t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() % 16 or (shape is not None and t.shape != shape) \
+            if t is None or type(t) not in wavefront._PLAIN_TYPES or t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() % 16 or (shape is not None and t.shape != shape) \
                     or t.device != x.device:
                 return None
         if mix.x_proj.bias is not None or mix.AT_log.shape[1] != wavefront.STATES_PER_CALL or mix.dt_projT.weight.shape[1] > 32:
@@ -479,7 +480,7 @@ class ResBlock(nn.Module):
             mix = self.token_mixer
             keep1, keep2 = _kept(x, self.drop_path, self.training), _kept(x, self.drop_path, self.training)
             local_eps = mix.local_norm.eps if mix.local_norm is not None else 0.0
-            y = train_block_op(x.float().contiguous(), par, keep1, keep2, self.norm1.eps, self.norm2.eps, local_eps, mix.flip,
+            y = train_block_op(wavefront._c(x.float()), par, keep1, keep2, self.norm1.eps, self.norm2.eps, local_eps, mix.flip,
                                mix.recomp == "full", wavefront.SAVE_CHECKPOINTS, wavefront._interval())
             return y, None
         n1 = self.norm1(x) if normed is None else normed
@@ -572,7 +573,7 @@ def _infer_stage(stage, x):
     else (gradients, training mode, hooks, foreign modules, parameters of mixed types), or where somebody has put
     another operator in the place of one that the call stands for (to count or to time it)."""
     if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 4 and x.numel() > 0 and x.is_contiguous() and len(stage) > 1
-            and x.shape[3] % 16 == 0 and x.shape[3] <= 512 and not torch.compiler.is_compiling()):
+            and x.shape[3] % 16 == 0 and x.shape[3] <= 512 and wavefront._direct(x) and not _global_hooks()):
         return None
     if _module_ops() != _OWN_OPS or not wavefront.FUSED_PROJECTIONS:
         return None

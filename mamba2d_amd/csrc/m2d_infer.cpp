@@ -122,12 +122,14 @@ Tensor infer_stage(const Tensor& x_in, at::TensorList par, at::IntArrayRef kinds
     const bool last = blk + 1 == kinds.size();
     const Tensor &next_w = par[at], &next_b = par[at + 1];      // norm1 of the next block, or the stage's norm
     const double next_eps = last ? eps[3 * kinds.size()] : eps[3 * (blk + 1)];
+    shaped(p[kN1W], {C}); shaped(p[kN1B], {C});
     const Tensor n1 = normed.defined() ? normed : r.norm(x, p[kN1W], p[kN1B], eps[3 * blk]);
     Tensor term, term2;
     const Tensor *rs1, *n2w, *n2b, *f1w, *f1b, *f2w, *f2b, *rs2;
     if (att) {
       const int64_t hd = p[aQnW].size(0), nh = p[aQkv].size(0) / 3 / hd, L = r.H * r.W;
       shaped(p[aQkv], {3 * nh * hd, C}); shaped(p[aProj], {C, nh * hd}); shaped(cos, {L, hd}); shaped(sin, {L, hd});
+      for (int i : {(int)aQnW, (int)aQnB, (int)aKnW, (int)aKnB}) shaped(p[i], {hd});
       TORCH_CHECK(cos.is_contiguous() && sin.is_contiguous() && cos.scalar_type() == at::kBFloat16 && sin.scalar_type() == at::kBFloat16,
                   "m2dscan: cos and sin must be contiguous bfloat16 tensors");
       const Tensor qkv = r.linear(n1, p[aQkv], nullptr, M2D_ACT_NONE, nullptr, nullptr, M2D_ACT_NONE, nullptr, nullptr);
@@ -139,8 +141,11 @@ Tensor infer_stage(const Tensor& x_in, at::TensorList par, at::IntArrayRef kinds
       rs1 = p + aRs1; n2w = p + aN2W; n2b = p + aN2B; f1w = p + aFc1W; f1b = p + aFc1B; f2w = p + aFc2W; f2b = p + aFc2B; rs2 = p + aRs2;
     } else {
       const bool local = kind >= kScanLocal, flip = kind & 1;
+      shaped(p[kInW], {C, C}); shaped(p[kInB], {C}); shaped(p[kOutW], {C, C}); shaped(p[kOutB], {C});
       if (local) {
         const int64_t M = p[kPw1].size(0);
+        shaped(p[kLnW], {C}); shaped(p[kLnB], {C});
+        for (int i : {(int)kS1S, (int)kS1B, (int)kS2S, (int)kS2B}) TORCH_CHECK(p[i].numel() == 1, "m2dscan: a StarReLU's scale or bias is no single value");
         shaped(p[kPw1], {M, C}); shaped(p[kDw], {M, 1, 3, 3}); shaped(p[kPw2], {C, M});
         Tensor a;
         if (C % 32 == 0 && C <= 128 && M % 16 == 0 && M <= 512) {
@@ -155,7 +160,6 @@ Tensor infer_stage(const Tensor& x_in, at::TensorList par, at::IntArrayRef kinds
         check(m2d_dwconv3x3_fwd((int)r.B, (int)r.H, (int)r.W, (int)M, M2D_BF16, r.wd, a.data_ptr(), p[kDw].data_ptr(), d.data_ptr(), r.st));
         term2 = r.linear(d, p[kPw2], nullptr, M2D_ACT_STARRELU, p + kS2S, p + kS2B, M2D_ACT_NONE, nullptr, nullptr);
       }
-      shaped(p[kInW], {C, C}); shaped(p[kOutW], {C, C});
       const Tensor u = r.linear(n1, p[kInW], p + kInB, M2D_ACT_NONE, nullptr, nullptr, M2D_ACT_GELU, nullptr, nullptr);
       const Tensor* w = &wide[wat];
       wat += kD - kATLog + 1;

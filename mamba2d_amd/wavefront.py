@@ -315,11 +315,23 @@ def _grouped_scan_bwd(x, deltaT, deltaL, AT, AL, BT, BL, C, D, dy, cks, flip, in
     return (*[t.to(x.dtype) for t in sums], *joined, d_D)
 
 
-def _eager(x) -> bool:
-    """Whether a call on x can be issued from C++ in one operator (csrc/m2d_entry.cpp): a plain tensor on the GPU, not
-    traced and not under forward-mode differentiation, and nobody has put something else in place of the operators."""
-    return (type(x) is torch.Tensor and x.is_cuda and not torch.compiler.is_compiling()
-            and (scan_fwd_op, scan_bwd_op, proj_fwd_op, proj_bwd_op) == _OWN_OPS and torch.autograd.forward_ad._current_level < 0)
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _direct(*tensors) -> bool:
+    """Whether a call on these tensors may go around the dispatched operators: plain tensors, and nobody watches the
+    operators that run (compilation, tracing, a dispatch mode such as fake tensors or selective checkpointing, a functorch
+    transform, forward-mode differentiation).  The C++ sequences call the library without the dispatcher in between: a trace
+    would hold their allocations only, and vmap would take the batched tensor apart behind their back."""
+    return (not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None
+            and torch.autograd.forward_ad._current_level < 0 and all(type(t) in _PLAIN_TYPES for t in tensors))
+
+
+def _eager(x, *params) -> bool:
+    """Whether a call on x can be issued from C++ in one operator (csrc/m2d_entry.cpp): on the GPU, unobserved, and nobody
+    has put something else in place of the operators."""
+    return x.is_cuda and (scan_fwd_op, scan_bwd_op, proj_fwd_op, proj_bwd_op) == _OWN_OPS and _direct(x, *params)
 
 
 class _ScanOnParams(torch.autograd.Function):
@@ -369,7 +381,7 @@ class wf_cuda_fn_pr(torch.autograd.Function):
 
     @classmethod
     def apply(cls, x, deltaT, deltaL, AT, AL, BT, BL, C, D, flip=False):
-        if not torch.is_grad_enabled() and _eager(x) and AT.shape[-1] == STATES_PER_CALL:
+        if not torch.is_grad_enabled() and AT.shape[-1] == STATES_PER_CALL and _eager(x, deltaT, deltaL, AT, AL, BT, BL, C, D):
             return scan_op(x, deltaT, deltaL, AT, AL, BT, BL, C, D, bool(flip), _interval())
         return _ScanOnParams.apply(x, deltaT, deltaL, AT, AL, BT, BL, C, D, flip, torch.is_grad_enabled())
 
@@ -498,11 +510,10 @@ def wavefront_scan_cuda(x, AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_
         raise ValueError(f"Unknown recomputation mode, got {recomp}...")
     if FUSED_PROJECTIONS and _proj_kernels_cover(x, AT_log, dt_projT_w):
         # the casts of the weights to x.dtype happen inside (no copies of the parameters)
-        if _eager(x):
-            return entry_op(x, [AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D],
-                            recomp == "full", bool(flip), SAVE_CHECKPOINTS, _interval())
-        return wf_cuda_fn_proj.apply(x, AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D,
-                                     recomp == "full", flip, torch.is_grad_enabled())
+        params = [AT_log, AL_log, x_proj_w, dt_projT_w, dt_projT_b, dt_projL_w, dt_projL_b, D]
+        if _eager(x, *params):
+            return entry_op(x, params, recomp == "full", bool(flip), SAVE_CHECKPOINTS, _interval())
+        return wf_cuda_fn_proj.apply(x, *params, recomp == "full", flip, torch.is_grad_enabled())
 
     x_proj_w = x_proj_w.to(x.dtype)
     dt_projT_w = dt_projT_w.to(x.dtype)
