@@ -359,7 +359,8 @@ int m2d_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, con
 
 /* y = post(x weight^T + bias) for wide layers and few positions (P (P,K) and (P,N) bf16, post_act nothing or GELU of the
  * layer's output rounded to bf16): K and N multiples of 32, any size.  Reads its operands straight from memory, made for
- * the latency of a few hundred positions; beyond about a thousand a tiled product is faster. */
+ * the latency of a few hundred positions; beyond about a thousand a tiled product is faster.  With GELU, bf16 weights, K up
+ * to 320, N a multiple of 64 and more than 512 positions it is a tiled product itself. */
 int m2d_wide_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias, int post_act,
                         void* y, void* stream);
 

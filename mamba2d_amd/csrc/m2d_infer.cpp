@@ -22,8 +22,10 @@ enum Attn { aN1W, aN1B, aQkv, aQnW, aQnB, aKnW, aKnB, aProj, aRs1, aN2W, aN2B, a
 enum Kind { kScan = 0, kScanFlipped = 1, kScanLocal = 2, kScanLocalFlipped = 3, kAttention = 4 };
 
 // Up to this many rows a wide layer runs in the library's kernel without staging (host 3 us against 19, device about the
-// same up to 400 rows); beyond it the stock product's tiles win (320 -> 1280 at 784 rows: 9.6 us against 5.4).
+// same up to 400 rows); beyond it the stock product's tiles win (320 -> 1280 at 784 rows: 9.6 us against 5.4), unless a
+// GELU follows: that layer's own kernel writes its outputs once, where the stock product and activation write them twice.
 constexpr int64_t kFewPositions = 512;
+constexpr int64_t kMostPositions = 1 << 20;      // what m2d_wide_linear_fwd takes
 
 struct Run {
   int64_t B, H, W, C, P;
@@ -50,7 +52,9 @@ struct Run {
       return y;
     }
     TORCH_CHECK(pre != M2D_ACT_STARRELU && post != M2D_ACT_STARRELU, "m2dscan: StarReLU next to a wide layer");
-    if (pre == M2D_ACT_NONE && P <= kFewPositions && K % 32 == 0 && N % 32 == 0) {
+    const bool few = P <= kFewPositions;
+    const bool gelu = post == M2D_ACT_GELU && wd == M2D_BF16 && K <= 320 && N % 64 == 0 && P <= kMostPositions;
+    if (pre == M2D_ACT_NONE && (few || gelu) && K % 32 == 0 && N % 32 == 0) {
       Tensor y = make(N);
       check(m2d_wide_linear_fwd(P, (int)K, (int)N, wd, x.data_ptr(), w.data_ptr(), ptr(b), post, y.data_ptr(), st));
       return y;

@@ -729,31 +729,56 @@ __global__ __launch_bounds__(256, 2) void m2d_train_wgrad_kernel(const WgradArgs
 }
 
 // ------------------------------------------------------------- sums of the workgroups' parts
-// out[i] = sum_s part[s * stride + i], in a fixed order; up to kMaxSegs sums in one launch.
+// out[i] = sum_s part[s * stride + i], in a fixed order; up to kMaxSegs sums in one launch.  Bound by memory (58 MB of parts
+// for a block of 64 channels, most of them still in the last-level cache) as long as enough loads are under way: a
+// workgroup takes 16 shares of the parts for 64 results, four to a thread where the parts are whole 16-byte pieces
+// (the weights), else for 16 results (the StarReLU's and the depthwise filters' sums, a few thousand), and a thread has
+// four loads under way (37 -> 17 us for the block of 64x56x56x64).  The shares are added in order through LDS, so the sums
+// do not depend on the form.
 constexpr int kMaxSegs = 24;
-struct Seg { const float* part; float* out; int64_t stride; int n, parts, first; };
+struct Seg { const float* part; float* out; int64_t stride; int n, parts, first, wide; };
 struct ReduceArgs { Seg s[kMaxSegs]; int nsegs; };
 
-__global__ __launch_bounds__(256) void m2d_train_reduce_kernel(const ReduceArgs a) {
-  // 16 results x 16 shares of the parts per workgroup, the shares added in order through LDS
-  __shared__ float red[16][17];
-  int si = 0;
-  while (si + 1 < a.nsegs && (int)blockIdx.x >= a.s[si + 1].first) ++si;
-  const Seg s = a.s[si];
+template <typename V> __device__ __forceinline__ V zero_of();
+template <> __device__ __forceinline__ float zero_of<float>() { return 0.f; }
+template <> __device__ __forceinline__ f32x4_t zero_of<f32x4_t>() { return f32x4_t{0.f, 0.f, 0.f, 0.f}; }
+
+template <typename V>
+__device__ __forceinline__ void reduce_parts(const Seg& s, int block, V (*red)[17]) {
+  constexpr int kV = sizeof(V) / 4;
   const int col = threadIdx.x & 15, share = threadIdx.x >> 4;
-  const int i = ((int)blockIdx.x - s.first) * 16 + col;
-  float v = 0.f;
+  const int i = (block * 16 + col) * kV;
+  V v = zero_of<V>();
   if (i < s.n) {
-    for (int p = share; p < s.parts; p += 16) v += s.part[p * s.stride + i];
+    const float* src = s.part + i;
+    int p = share;
+    for (; p + 48 < s.parts; p += 64) {
+      V o[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) o[u] = *reinterpret_cast<const V*>(src + (p + 16 * u) * s.stride);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v += o[u];
+    }
+    for (; p < s.parts; p += 16) v += *reinterpret_cast<const V*>(src + p * s.stride);
   }
   red[share][col] = v;
   __syncthreads();
   if (share == 0 && i < s.n) {
-    float t = 0.f;
+    V t = zero_of<V>();
 #pragma unroll
     for (int k = 0; k < 16; ++k) t += red[k][col];
-    s.out[i] = t;
+    *reinterpret_cast<V*>(s.out + i) = t;
   }
+}
+
+__global__ __launch_bounds__(256) void m2d_train_reduce_kernel(const ReduceArgs a) {
+  __shared__ f32x4_t red[16][17];
+  int si = 0;
+  while (si + 1 < a.nsegs && (int)blockIdx.x >= a.s[si + 1].first) ++si;
+  const Seg s = a.s[si];
+  const int block = (int)blockIdx.x - s.first;
+  if (s.wide) reduce_parts<f32x4_t>(s, block, red);
+  else reduce_parts<float>(s, block, reinterpret_cast<float (*)[17]>(red));
 }
 
 inline int launched() { return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP; }
@@ -979,8 +1004,9 @@ int m2d_train_reduce(int nsegs, const m2d_reduce_seg* segs, void* stream) {
       const m2d_reduce_seg& s = segs[at];
       if (!s.part || !s.out) return M2D_ERR_NULL_POINTER;
       if (s.n < 1 || s.parts < 1) return M2D_ERR_BAD_SHAPE;
-      a.s[a.nsegs++] = {s.part, s.out, s.stride, s.n, s.parts, (int)blocks};
-      blocks += (s.n + 15) / 16;
+      const int wide = s.n % 4 == 0 && s.stride % 4 == 0 && !misaligned(s.part, 16) && !misaligned(s.out, 16) ? 1 : 0;
+      a.s[a.nsegs++] = {s.part, s.out, s.stride, s.n, s.parts, (int)blocks, wide};
+      blocks += wide ? (s.n + 63) / 64 : (s.n + 15) / 16;
       if (blocks >= ((int64_t)1 << 30)) return M2D_ERR_UNSUPPORTED;
     }
     hipLaunchKernelGGL(m2d_train_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a);
