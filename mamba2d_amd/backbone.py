@@ -16,6 +16,7 @@ Differences in how it runs (not in what it computes):
     acts per cell and commutes with the flip;
   * the rotary tables of the attention stages are built once per grid size.
 """
+import itertools
 import math
 import operator
 import weakref
@@ -41,6 +42,11 @@ def _inference(*tensors):
     return not torch.is_grad_enabled() or not any(t.requires_grad for t in tensors)
 
 
+def _untouched(mod):
+    """A call past the module's own call gives what the call would: nobody has put another ``forward`` on the instance."""
+    return "forward" not in mod.__dict__
+
+
 ACT_NONE, ACT_GELU, ACT_STARRELU = 0, 1, 2
 
 
@@ -52,7 +58,7 @@ def _act(kind, star, t):
 
 def _norm_joins(norm, x, w):
     """The LayerNorm ``norm`` over x's last axis can run inside the kernel of the layer (weights ``w``) that reads it."""
-    return (isinstance(norm, nn.LayerNorm) and norm.weight is not None and norm.bias is not None
+    return (isinstance(norm, nn.LayerNorm) and _untouched(norm) and norm.weight is not None and norm.bias is not None
             and tuple(norm.normalized_shape) == (x.shape[-1],) and norm.weight.dtype == w.dtype and norm.bias.dtype == w.dtype
             and _inference(norm.weight, norm.bias))
 
@@ -67,8 +73,8 @@ def linear_act(lin, x, pre=ACT_NONE, post=ACT_NONE, star=None, norm=None):
     N, K = w.shape
     extra = [t for t in (b, *((star.scale, star.bias) if star is not None else ())) if t is not None]
     if (x.is_cuda and x.dtype == torch.bfloat16 and _inference(x, w, *extra) and w.dtype in (torch.float32, torch.bfloat16)
-            and K % 32 == 0 and K <= 256 and N % 16 == 0 and N <= 512 and x.numel() > 0
-            and (star is None or star.scale.dtype == w.dtype)):
+            and K % 32 == 0 and K <= 256 and N % 16 == 0 and N <= 512 and x.numel() > 0 and _untouched(lin)
+            and (star is None or (star.scale.dtype == w.dtype and _untouched(star)))):
         ps = (star.scale, star.bias) if pre == ACT_STARRELU else (None, None)
         qs = (star.scale, star.bias) if post == ACT_STARRELU else (None, None)
         if norm is not None and pre == ACT_NONE and K <= 128 and _norm_joins(norm, x, w):
@@ -144,7 +150,7 @@ class MLP(nn.Module):
         w1, w2 = self.fc1.weight, self.fc2.weight
         if (x.is_cuda and x.dtype == torch.bfloat16 and x.numel() > 0 and x.shape[-1] in (32, 64) and w1.shape[0] == 4 * w1.shape[1]
                 and _inference(x, w1, w2, self.fc1.bias, self.fc2.bias) and w1.dtype in (torch.float32, torch.bfloat16)
-                and w2.dtype == w1.dtype):
+                and w2.dtype == w1.dtype and _untouched(self.fc1) and _untouched(self.fc2)):
             # both layers in one kernel: the hidden activations, four times x, never reach memory
             if norm is not None and _norm_joins(norm, x, w1):
                 return mlp_fwd_op(x.contiguous(), w1, self.fc1.bias, w2, self.fc2.bias, norm.weight, norm.bias, norm.eps)
@@ -154,7 +160,7 @@ class MLP(nn.Module):
     def takes_norm(self, x, norm):
         """norm(x) would not be written: the kernel of the first layer computes it."""
         w1 = self.fc1.weight
-        return (x.is_cuda and x.dtype == torch.bfloat16 and x.numel() > 0
+        return (x.is_cuda and x.dtype == torch.bfloat16 and x.numel() > 0 and _untouched(self) and _untouched(self.fc1)
                 and _inference(x, w1, self.fc2.weight, self.fc1.bias, self.fc2.bias)
                 and w1.dtype in (torch.float32, torch.bfloat16) and self.fc2.weight.dtype == w1.dtype and _norm_joins(norm, x, w1)
                 and w1.shape[1] % 32 == 0 and w1.shape[1] <= 128 and w1.shape[0] % 16 == 0 and w1.shape[0] <= 512)
@@ -185,7 +191,7 @@ class SepConv(nn.Module):
         w = self.dwconv.weight
         if (x.is_cuda and _inference(x, w) and self.dwconv.kernel_size == (3, 3) and self.dwconv.padding == (1, 1)
                 and x.dtype in (torch.float32, torch.bfloat16) and w.dtype in (torch.float32, torch.bfloat16)
-                and x.shape[-1] % (8 if x.dtype == torch.bfloat16 else 4) == 0 and x.numel() > 0):
+                and x.shape[-1] % (8 if x.dtype == torch.bfloat16 else 4) == 0 and x.numel() > 0 and _untouched(self.dwconv)):
             # the library's depthwise kernel (the stock library falls back to a generic direct
             # convolution for channel-last bf16 here, ten times slower than the memory traffic allows)
             x = dwconv3x3_fwd_op(x.contiguous(), w)
@@ -245,7 +251,9 @@ class M2DBlock(nn.Module):
     def forward(self, x, split=False):           # (B, H, W, C)
         """The mixed tokens; with ``split`` and a local path, the two terms of the sum, for a caller that
         adds them in a pass of its own."""
-        local = self.local_path(x, norm=self.local_norm) if self.local_path is not None else None
+        local = None
+        if self.local_path is not None:
+            local = self.local_path(x, norm=self.local_norm) if _untouched(self.local_path) else self.local_path(self.local_norm(x))
         u = linear_act(self.in_proj, x, post=ACT_GELU)
         y = wavefront_scan_cuda(u, self.AT_log, self.AL_log, self.x_proj.weight,
                                 self.dt_projT.weight, self.dt_projT.bias,
@@ -307,7 +315,7 @@ class RoPEAttention2D(nn.Module):
         qn, kn, hd = self.q_norm, self.k_norm, self.head_dim
         if (qkv.is_cuda and _inference(qkv, qn.weight, qn.bias, kn.weight, kn.bias) and qkv.dtype in (torch.float32, torch.bfloat16)
                 and qn.weight.dtype in (torch.float32, torch.bfloat16) and qn.eps == kn.eps and hd & (hd - 1) == 0
-                and 8 <= hd <= 128 and qkv.numel() > 0):
+                and 8 <= hd <= 128 and qkv.numel() > 0 and _untouched(qn) and _untouched(kn)):
             if hd == 32 and H * W <= 256 and qkv.dtype == torch.bfloat16:
                 # the whole attention in one kernel, a head per workgroup, answering in the projection's layout
                 o = rope_attention_fwd_op(qkv, cos, sin, qn.weight, qn.bias, kn.weight, kn.bias, qn.eps, hd ** -0.5)
@@ -340,8 +348,9 @@ def _kept(x, p, training):
 
 
 def _plain(mod, kind):
-    """The module is what its class says: exactly ``kind``, without hooks that a call past its forward would skip."""
-    return type(mod) is kind and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks)
+    """The module is what its class says: exactly ``kind``, without anything that a call past its own call would skip."""
+    return (type(mod) is kind and _untouched(mod)
+            and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks))
 
 
 class ResBlock(nn.Module):
@@ -369,7 +378,7 @@ class ResBlock(nn.Module):
     def _residual(x, scale, branch, branch2=None):
         """scale(x) + branch (+ branch2); with a learned scale, at inference on the GPU, in one pass."""
         terms = (branch,) if branch2 is None else (branch, branch2)
-        if (isinstance(scale, Scale) and x.is_cuda and _inference(x, scale.scale, *terms) and x.is_contiguous()
+        if (isinstance(scale, Scale) and _untouched(scale) and x.is_cuda and _inference(x, scale.scale, *terms) and x.is_contiguous()
                 and all(t.is_contiguous() and t.dtype == x.dtype and t.shape == x.shape for t in terms)
                 and x.dtype in (torch.float32, torch.bfloat16) and scale.scale.dtype in (torch.float32, torch.bfloat16)
                 and x.shape[-1] % 8 == 0 and x.numel() > 0):
@@ -381,6 +390,7 @@ class ResBlock(nn.Module):
         """(y, norm(y)) for y = scale(x) + sum(terms); (y, None) without a norm.  At inference on the GPU the update
         and the LayerNorm behind it are one pass over the rows."""
         if (norm is not None and isinstance(scale, Scale) and x.is_cuda and x.is_contiguous() and x.numel() > 0
+                and _untouched(scale) and _untouched(norm)
                 and _inference(x, scale.scale, norm.weight, norm.bias, *terms)
                 and all(t.is_contiguous() and t.dtype == x.dtype and t.shape == x.shape for t in terms)
                 and x.dtype in (torch.float32, torch.bfloat16) and scale.scale.dtype in (torch.float32, torch.bfloat16)
@@ -484,7 +494,7 @@ class ResBlock(nn.Module):
                                mix.recomp == "full", wavefront.SAVE_CHECKPOINTS, wavefront._interval())
             return y, None
         n1 = self.norm1(x) if normed is None else normed
-        if isinstance(self.token_mixer, M2DBlock) and not self.training:
+        if isinstance(self.token_mixer, M2DBlock) and not self.training and _untouched(self.token_mixer):
             mixed = self.token_mixer(n1, split=True)       # scan path and local path, summed in the update
             terms = mixed if isinstance(mixed, tuple) else (mixed,)
         else:
@@ -519,9 +529,10 @@ class _StagePlan:
 
     def __init__(self, stage, kinds, par, eps, att):
         self.kinds, self.par, self.eps, self.att = kinds, par, eps, att
-        self.own, self.keys, self.was, self.hooks = [], [], [], []
+        self.own, self.keys, self.was, self.hooks, self.dicts = [], [], [], [], []
         for m in stage.modules():
             d = m.__dict__
+            self.dicts.append(d)
             for own in (m._modules, m._parameters, {k: d[k] for k in self.OPTIONS if k in d}):
                 for k, v in own.items():
                     self.own.append(own if own is m._modules or own is m._parameters else d)
@@ -535,7 +546,7 @@ class _StagePlan:
     def holds(self, stage):
         try:
             return (all(map(operator.is_, map(operator.getitem, self.own, self.keys), self.was)) and not any(self.hooks)
-                    and len(stage) == len(self.kinds) + 1)
+                    and not any(map(operator.contains, self.dicts, itertools.repeat("forward"))) and len(stage) == len(self.kinds) + 1)
         except KeyError:
             return False
 
@@ -546,7 +557,7 @@ _STAGE_PLANS = weakref.WeakKeyDictionary()
 def _stage_plan(stage, x):
     mods = list(stage)
     end = mods[-1]
-    if type(end) is not LayerNorm or end.weight is None or end.bias is None or end.training:
+    if type(end) is not LayerNorm or end.weight is None or end.bias is None or end.training or not all(map(_untouched, stage.modules())):
         return None
     kinds, par, eps, att = [], [], [], None
     for m in mods[:-1]:
@@ -635,10 +646,11 @@ class Mamba2DBackbone(nn.Module):
             return fast
         mods = list(stage)
         normed = None
+        own = lambda m: isinstance(m, ResBlock) and type(m).forward is ResBlock.forward and _untouched(m)
         for i, m in enumerate(mods):
-            if isinstance(m, ResBlock):
+            if own(m):
                 nxt = mods[i + 1] if i + 1 < len(mods) else None
-                follows = nxt.norm1 if isinstance(nxt, ResBlock) else nxt if isinstance(nxt, nn.LayerNorm) else None
+                follows = nxt.norm1 if own(nxt) else nxt if isinstance(nxt, nn.LayerNorm) else None
                 x, normed = m.forward_fused(x, normed, follows)
             elif isinstance(m, nn.LayerNorm) and normed is not None:
                 x, normed = normed, None
