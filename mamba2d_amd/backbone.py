@@ -43,8 +43,9 @@ def _inference(*tensors):
 
 
 def _untouched(mod):
-    """A call past the module's own call gives what the call would: nobody has put another ``forward`` on the instance."""
-    return "forward" not in mod.__dict__
+    """A call past the module's own call gives what the call would: nobody has put another ``forward`` on the instance,
+    and it has no hooks."""
+    return not ("forward" in mod.__dict__ or mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks)
 
 
 ACT_NONE, ACT_GELU, ACT_STARRELU = 0, 1, 2
@@ -349,8 +350,7 @@ def _kept(x, p, training):
 
 def _plain(mod, kind):
     """The module is what its class says: exactly ``kind``, without anything that a call past its own call would skip."""
-    return (type(mod) is kind and _untouched(mod)
-            and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks))
+    return type(mod) is kind and _untouched(mod)
 
 
 class ResBlock(nn.Module):

@@ -1,5 +1,5 @@
 """Calls that go past a module's own ``forward`` (a stage as one call, a block as one function, a norm inside its reader's
-kernel) are for modules that nobody watches: a ``forward`` put on an instance has to run, also when it comes
+kernel) are for modules that nobody watches: a hook or a ``forward`` put on an instance has to run, also when it comes
 after a plan was made, and must be gone when it is taken away."""
 import pytest
 import torch
@@ -24,29 +24,40 @@ EVERY = [(kind, name) for kind in CALLED for name in CALLED[kind]]
 
 
 @pytest.mark.parametrize("kind,name", EVERY, ids=lambda v: str(v))
-def test_stage_plan_is_for_plain_modules(kind, name):
+@pytest.mark.parametrize("way", ["forward", "hook", "pre_hook"])
+def test_stage_plan_is_for_plain_modules(kind, name, way):
     stage = stage_of(kind)
     x = torch.zeros(1, 4, 4, 32)
     with torch.no_grad():
         plan = backbone._stage_plan(stage, x)
         assert plan is not None and plan.holds(stage)
         mod = stage[0].get_submodule(name)
-        mod.forward = lambda *a, **k: None
+        if way == "forward":
+            mod.forward = lambda *a, **k: None
+            undo = lambda: delattr(mod, "forward")
+        else:
+            undo = (mod.register_forward_hook if way == "hook" else mod.register_forward_pre_hook)(lambda *a: None).remove
         assert not plan.holds(stage) and backbone._stage_plan(stage, x) is None
-        del mod.forward
+        undo()
         assert plan.holds(stage) and backbone._stage_plan(stage, x) is not None
 
 
 @pytest.mark.parametrize("target", ["block", "end"])
-def test_replaced_blocks_and_norms_of_a_stage_run(target):
+def test_watched_blocks_and_norms_of_a_stage_run(target):
+    """The modules of a stage: a hook on a block, or on the norm behind the last block, sees its call and may change it."""
     stage = stage_of("attention")
     x = torch.randn(1, 4, 4, 32)
     seen = []
     with torch.no_grad():
+        y = backbone.Mamba2DBackbone._run_stage(stage, x)
         mod = stage[0] if target == "block" else stage[-1]
+        handle = mod.register_forward_hook(lambda m, a, out: (seen.append(1), out + 1.0)[1])
+        z = backbone.Mamba2DBackbone._run_stage(stage, x)
+        assert seen == [1] and not torch.allclose(y, z)
+        handle.remove()
         mod.forward = lambda t: (seen.append(2), t)[1]
         backbone.Mamba2DBackbone._run_stage(stage, x)
-        assert seen == [2]
+        assert seen == [1, 2]
 
 
 @pytest.mark.gpu
@@ -70,16 +81,20 @@ def test_training_block_is_for_plain_modules(name):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", CALLED["scan"])
-def test_replaced_forward_runs_at_inference(name):
-    """Through the kernels that join a norm or an activation to their neighbour."""
-    print(f"\ncase watched stage {name}", flush=True)
-    stage = stage_of("scan").cuda().bfloat16()
-    x = torch.randn(1, 4, 4, 32, device="cuda").bfloat16()
+@pytest.mark.parametrize("train", [False, True])
+def test_hooks_of_a_stage_run(name, train):
+    """bf16 inference and mixed training past the kernels that join a norm or an activation to their neighbour."""
+    print(f"\ncase watched stage {name} {train}", flush=True)
+    with torch.device("cuda"):
+        stage = stage_of("scan")
+        x = torch.randn(1, 4, 4, 32)
+    if not train:
+        stage, x = stage.bfloat16(), x.bfloat16()
     seen = []
-    mod = stage[0].get_submodule(name)
-    plain = mod.forward
-    with torch.no_grad():
-        assert backbone._infer_stage(stage, x) is not None
-        mod.forward = lambda t: (seen.append(1), plain(t))[1]
+    with torch.set_grad_enabled(train):
+        assert train or backbone._infer_stage(stage, x) is not None      # (the plan is there before the hooks)
+    for block in stage[:2]:
+        block.get_submodule(name).register_forward_hook(lambda *a: seen.append(1))
+    with torch.set_grad_enabled(train), torch.autocast("cuda", dtype=torch.bfloat16, enabled=train):
         backbone.Mamba2DBackbone._run_stage(stage, x)
-    assert seen == [1]
+    assert seen == [1, 1]
