@@ -223,7 +223,7 @@ __global__ __launch_bounds__(kDwThreads) void m2d_dwconv3x3_kernel(const DwArgs 
           float v[V];
           Chunk<T>::unpack(win[i][slot], v);
 #pragma unroll
-          for (int j = 0; j < V; ++j) { const float t = fmaxf(v[j], 0.f); v[j] = __builtin_fmaf(star_s * t, t, star_b); }
+          for (int j = 0; j < V; ++j) v[j] = star_relu(v[j], star_s, star_b);
           Chunk<T>::store(reinterpret_cast<T*>(&win[i][slot]), v);
         }
       }
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(kEwThreads) void m2d_starrelu_kernel(const EwArgs a
     float v[V];
     Chunk<T>::load(X + i * V, v);
 #pragma unroll
-    for (int j = 0; j < V; ++j) { const float t = fmaxf(v[j], 0.f); v[j] = __builtin_fmaf(sc * t, t, bi); }
+    for (int j = 0; j < V; ++j) v[j] = star_relu(v[j], sc, bi);
     Chunk<T>::store(Y + i * V, v);
   }
 }
@@ -435,7 +435,7 @@ enum { kActNone = 0, kActGelu = 1, kActStarRelu = 2, kActLayerNorm = 3 };   // t
 
 __device__ __forceinline__ float act(int kind, float v, float s, float b) {
   if (kind == kActGelu) return gelu_exact(v);
-  if (kind == kActStarRelu) { const float t = fmaxf(v, 0.f); return __builtin_fmaf(s * t, t, b); }
+  if (kind == kActStarRelu) return star_relu(v, s, b);
   return v;
 }
 

@@ -88,6 +88,16 @@ __device__ __forceinline__ f32x4_t mfma_bf16(uint4 a, uint4 b, f32x4_t c) {
 }
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 
+// max(v, 0) that hands a NaN on, as the stock operator does (fmaxf returns the other operand): one v_maximum3_f32
+__device__ __forceinline__ float relu(float v) { return __builtin_elementwise_maximum(v, 0.f); }
+// StarReLU, s relu(v)^2 + b
+__device__ __forceinline__ float star_relu(float v, float s, float b) {
+  const float t = relu(v);
+  return __builtin_fmaf(s * t, t, b);
+}
+// d times the slope of StarReLU at t = relu(v): nothing where the activation is flat, whatever d is (0 x infinity would
+// be a NaN there; the stock operator selects)
+__device__ __forceinline__ float star_relu_back(float d, float t, float s) { return t <= 0.f ? 0.f : d * (2.f * s * t); }
 
 // erf by Abramowitz & Stegun 7.1.26 (absolute error below 1.5e-7), one v_exp_f32 and one v_rcp_f32
 __device__ __forceinline__ float gelu_exact(float v) {

@@ -45,13 +45,8 @@ __device__ __forceinline__ float gelu_slope(float v) {
 enum { kActNone = 0, kActGelu = 1, kActStarRelu = 2 };
 __device__ __forceinline__ float act(int kind, float v, float s, float b) {
   if (kind == kActGelu) return gelu_exact(v);
-  if (kind == kActStarRelu) { const float t = fmaxf(v, 0.f); return __builtin_fmaf(s * t, t, b); }
+  if (kind == kActStarRelu) return star_relu(v, s, b);
   return v;
-}
-__device__ __forceinline__ float act_slope(int kind, float v, float s) {
-  if (kind == kActGelu) return gelu_slope(v);
-  if (kind == kActStarRelu) return 2.f * s * fmaxf(v, 0.f);
-  return 1.f;
 }
 
 template <int G>
@@ -419,8 +414,8 @@ __global__ __launch_bounds__(256) void m2d_train_dwconv_bwd_kernel(const DwBwdAr
         float o[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float t = fmaxf(p[j], 0.f);
-          // what the forward's convolution read: StarReLU rounded to bf16
+          const float t = relu(p[j]);
+          // (the forward's convolution read this rounded to bf16)
           const float st = __builtin_fmaf(sc * t, t, bi);
           float d = 0.f;
 #pragma unroll
@@ -434,7 +429,7 @@ __global__ __launch_bounds__(256) void m2d_train_dwconv_bwd_kernel(const DwBwdAr
           }
           acc[9][j] = __builtin_fmaf(d, t * t, acc[9][j]);
           acc[10][j] += d;
-          o[j] = d * (2.f * sc * t);
+          o[j] = star_relu_back(d, t, sc);
         }
         st4bf(a.dp + img + ((int64_t)h * a.W + w) * a.C, o);
       }
@@ -528,7 +523,7 @@ __global__ __launch_bounds__(kLinThreads) void m2d_train_linear_bwd_kernel(const
           uint32_t w4[4] = {A[kc].x, A[kc].y, A[kc].z, A[kc].w};
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            w4[j] = pack_bf16(bf_lo(w4[j]) * act_slope(a.post, bf_lo(z4[j]), 1.f), bf_hi(w4[j]) * act_slope(a.post, bf_hi(z4[j]), 1.f));
+            w4[j] = pack_bf16(bf_lo(w4[j]) * gelu_slope(bf_lo(z4[j])), bf_hi(w4[j]) * gelu_slope(bf_hi(z4[j])));
           A[kc] = make_uint4(w4[0], w4[1], w4[2], w4[3]);
         }
     }
@@ -562,10 +557,10 @@ __global__ __launch_bounds__(kLinThreads) void m2d_train_linear_bwd_kernel(const
             if (a.pre == kActStarRelu) {
 #pragma unroll
               for (int j = 0; j < 8; ++j) {
-                const float t = fmaxf(xv[j], 0.f);
+                const float t = relu(xv[j]);
                 sum_s = __builtin_fmaf(v[j], t * t, sum_s);
                 sum_b += v[j];
-                v[j] *= 2.f * pre_s * t;
+                v[j] = star_relu_back(v[j], t, pre_s);
               }
             } else {
 #pragma unroll
@@ -664,7 +659,7 @@ __global__ __launch_bounds__(256, 2) void m2d_train_wgrad_kernel(const WgradArgs
         const uint32_t z4[4] = {zq[k].x, zq[k].y, zq[k].z, zq[k].w};
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          g4[j] = pack_bf16(bf_lo(g4[j]) * act_slope(a.post, bf_lo(z4[j]), 1.f), bf_hi(g4[j]) * act_slope(a.post, bf_hi(z4[j]), 1.f));
+          g4[j] = pack_bf16(bf_lo(g4[j]) * gelu_slope(bf_lo(z4[j])), bf_hi(g4[j]) * gelu_slope(bf_hi(z4[j])));
       }
       if (a.pre != kActNone) {      // (rows past the end meet zero rows of g)
 #pragma unroll
