@@ -33,3 +33,12 @@ def test_fp32_weights_without_autocast(monkeypatch, dim, mixer, positions):
         monkeypatch.setattr(backbone, "_infer_stage", lambda stage, x: None)
         want = outcome()
     assert got == want == (torch.bfloat16 if (dim, mixer) == (64, "2D_local") else "refused")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_fp16_autocast_keeps_to_the_modules(dtype):
+    """Under fp16 autocast the stock products answer in fp16: no sequence of bf16 kernels."""
+    print(f"\ncase fp16 autocast {dtype}", flush=True)
+    stage, x = stage_of(64, "RopeAttention").to(dtype), torch.randn(2, 6, 7, 64, device="cuda").bfloat16()
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        assert backbone._infer_stage(stage, x) is None
