@@ -588,6 +588,9 @@ def _infer_stage(stage, x):
         return None
     if _module_ops() != _OWN_OPS or not wavefront.FUSED_PROJECTIONS:
         return None
+    autocast = torch.is_autocast_enabled("cuda")
+    if autocast and torch.get_autocast_dtype("cuda") != torch.bfloat16:      # (the stock products would answer in that type)
+        return None
     plan = _STAGE_PLANS.get(stage)
     if plan is None or not plan.holds(stage):
         plan = _stage_plan(stage, x)
@@ -599,7 +602,7 @@ def _infer_stage(stage, x):
         return None
     cos = sin = x
     if att is not None:
-        if x.shape[1] * x.shape[2] > 256 or (dtype == torch.float32 and not torch.is_autocast_enabled("cuda")):
+        if x.shape[1] * x.shape[2] > 256 or (dtype == torch.float32 and not autocast):
             return None      # (larger grids take another attention; fp32 weights meet bf16 activations only under autocast)
         cos, sin = att._rope_tables(x.shape[1], x.shape[2], x.device, x.dtype)
     out = infer_stage_op(x, plan.par, plan.kinds, plan.eps, cos, sin, 32 ** -0.5)

@@ -13,6 +13,7 @@
 namespace {
 
 using at::Tensor;
+using m2dshim::dispatched;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
@@ -66,8 +67,10 @@ struct Entry : public torch::autograd::Function<Entry> {
     const Tensor dy = whole(grads[0].to(x.scalar_type()));
     Tensor low, dT, dL, BC, ck;
     const Tensor none = at::empty({0}, x.options());
+    const bool graph = at::GradMode::is_enabled();
     if (full) {
-      auto pr = m2dshim::proj_fwd(x, w[2], w[3], w[4], w[5], w[6], w[0].size(1), true, true);
+      auto pr = graph ? dispatched<decltype(m2dshim::proj_fwd)>("m2dscan::proj_fwd").call(x, w[2], w[3], w[4], w[5], w[6], w[0].size(1), true, true)
+                      : m2dshim::proj_fwd(x, w[2], w[3], w[4], w[5], w[6], w[0].size(1), true, true);
       low = pr[0]; dT = pr[1]; dL = pr[2]; BC = pr[3];
       ck = at::empty({1}, x.options().dtype(at::kByte));
     } else {
@@ -77,9 +80,14 @@ struct Entry : public torch::autograd::Function<Entry> {
     // channels d_BT, d_BL, d_C have one reader, the projections' backward: where its products run on the matrix cores it
     // takes the scan's per-workgroup sums as they are.
     const bool parts = x.scalar_type() == at::kBFloat16 && x.size(3) % 8 == 0;
-    auto g = m2dshim::scan_bwd(x, dT, dL, w[0], w[1], BC, none, none, w[7], dy, ck, flip, true, true, true, interval, parts);
+    auto g = graph ? dispatched<decltype(m2dshim::scan_bwd)>("m2dscan::scan_bwd").call(x, dT, dL, w[0], w[1], BC, none, none, w[7], dy, ck, flip,
+                                                                                       true, true, true, interval, parts)
+                   : m2dshim::scan_bwd(x, dT, dL, w[0], w[1], BC, none, none, w[7], dy, ck, flip, true, true, true, interval, parts);
     // g[0] holds the scan's own gradient of x; the projections add theirs in place
-    auto q = m2dshim::proj_bwd(x, low, dT, dL, w[2], w[3], w[5], g[1], g[2], g[5], g[6], g[7], g[0], true, true, parts ? g[5].size(0) : 0);
+    const int64_t np = parts ? g[5].size(0) : 0;
+    auto q = graph ? dispatched<decltype(m2dshim::proj_bwd)>("m2dscan::proj_bwd").call(x, low, dT, dL, w[2], w[3], w[5], g[1], g[2], g[5], g[6],
+                                                                                       g[7], g[0], true, true, np)
+                   : m2dshim::proj_bwd(x, low, dT, dL, w[2], w[3], w[5], g[1], g[2], g[5], g[6], g[7], g[0], true, true, np);
     variable_list out = {g[0], g[3], g[4], std::get<0>(q), std::get<1>(q), std::get<2>(q), std::get<3>(q), std::get<4>(q), g[8]};
     for (int i = 0; i < kPar; ++i) out[1 + i] = out[1 + i].to(raw[i].scalar_type());
     out.resize(out.size() + 4);      // the options take none

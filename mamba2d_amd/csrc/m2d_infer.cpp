@@ -5,6 +5,7 @@
 // image take; here the same kernels in the same order cost a few microseconds each.  The matrix products of the wide
 // layers stay with the stock library (at::linear, which also follows autocast), as in the modules.
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/library.h>
 
@@ -52,7 +53,8 @@ struct Run {
       return y;
     }
     TORCH_CHECK(pre != M2D_ACT_STARRELU && post != M2D_ACT_STARRELU, "m2dscan: StarReLU next to a wide layer");
-    const bool few = P <= kFewPositions;
+    // (fp32 weights meet bf16 activations under autocast only: without it the stock product below refuses them)
+    const bool few = P <= kFewPositions && (wd == M2D_BF16 || at::autocast::is_autocast_enabled(at::kCUDA));
     const bool gelu = post == M2D_ACT_GELU && wd == M2D_BF16 && K <= 320 && N % 64 == 0 && P <= kMostPositions;
     if (pre == M2D_ACT_NONE && (few || gelu) && K % 32 == 0 && N % 32 == 0) {
       Tensor y = make(N);

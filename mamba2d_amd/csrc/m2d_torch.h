@@ -2,6 +2,7 @@
 #ifndef M2D_TORCH_H
 #define M2D_TORCH_H
 #include <ATen/ATen.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/hip/HIPStream.h>
 
 #include <tuple>
@@ -34,6 +35,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> proj_bwd(const Tensor& x, con
                                                             Tensor dx, bool round_weights, bool dpre, int64_t sum_parts);
 
 std::vector<Tensor> widen(at::TensorList in);      // m2d_infer.cpp
+
+// Operator m2dscan::<name> through the dispatcher, for an autograd function whose backward is itself recorded
+// (create_graph): the library has no second derivatives, and the dispatched operators are the ones that say so, with a
+// warning, when somebody differentiates through them.
+template <typename F>
+c10::TypedOperatorHandle<F> dispatched(const char* name) {
+  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
+}
 
 }  // namespace m2dshim
 #endif

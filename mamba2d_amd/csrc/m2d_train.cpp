@@ -5,6 +5,8 @@
 // sequence of the library's kernels on one stream (9 + 12 launches beside the scan's own), issued from here: no
 // Python between them, no cast kernels (the fp32 parameters are read as they are), activations rounded to bf16 where
 // autocast rounds them.
+#include <ATen/autocast_mode.h>
+#include <torch/csrc/autograd/autograd.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
@@ -58,6 +60,47 @@ const float* opt(const OptTensor& t) { return t.has_value() && t->defined() ? t-
 
 Tensor bf16_like(const Tensor& x, int64_t C) {
   return at::empty({x.size(0), x.size(1), x.size(2), C}, x.options().dtype(at::kBFloat16));
+}
+
+// bf16 autocast while it lives.
+struct Autocast {
+  const bool was = at::autocast::is_autocast_enabled(at::kCUDA);
+  const at::ScalarType dtype = at::autocast::get_autocast_dtype(at::kCUDA);
+  Autocast() {
+    at::autocast::increment_nesting();
+    at::autocast::set_autocast_enabled(at::kCUDA, true);
+    at::autocast::set_autocast_dtype(at::kCUDA, at::kBFloat16);
+  }
+  ~Autocast() {
+    if (at::autocast::decrement_nesting() == 0) at::autocast::clear_cache();
+    at::autocast::set_autocast_enabled(at::kCUDA, was);
+    at::autocast::set_autocast_dtype(at::kCUDA, dtype);
+  }
+};
+
+// The block in stock operators and the entry point's, as its modules compute it under autocast: what its gradients are
+// taken from where they are to be differentiated themselves.
+Tensor stock_block(const Tensor& x, const std::vector<Tensor>& p, const Tensor& keep1, const Tensor& keep2, const std::vector<double>& eps,
+                   bool flip, bool full, int64_t interval) {
+  const Autocast on;
+  const int64_t C = x.size(3);
+  auto star = [](const Tensor& v, const Tensor& s, const Tensor& b) { return at::addcmul(b, s, at::relu(v).square()); };
+  auto kept = [](const Tensor& v, const Tensor& keep) { return keep.defined() ? v * keep.view({-1, 1, 1, 1}) : v; };
+  const Tensor n1 = at::layer_norm(x, {C}, p[kN1W], p[kN1B], eps[0]);
+  Tensor local;
+  if (p.size() == kAll) {
+    const Tensor a = star(at::linear(at::layer_norm(n1, {C}, p[kLnW], p[kLnB], eps[2]), p[kPw1]), p[kS1S], p[kS1B]);
+    const Tensor c = at::conv2d(a.permute({0, 3, 1, 2}), p[kDw], {}, 1, 1, 1, 2 * C).permute({0, 2, 3, 1});
+    local = at::linear(star(c, p[kS2S], p[kS2B]), p[kPw2]);
+  }
+  using Entry = Tensor(const Tensor&, at::TensorList, bool, bool, bool, int64_t);
+  const std::vector<Tensor> scan(p.begin() + kATLog, p.begin() + kD + 1);
+  const Tensor y = m2dshim::dispatched<Entry>("m2dscan::entry").call(at::gelu(at::linear(n1, p[kInW], p[kInB])), scan, full, flip, !full, interval);
+  Tensor mix = at::linear(at::gelu(y), p[kOutW], p[kOutB]);
+  if (local.defined()) mix = mix + local;
+  const Tensor x1 = x * p[kRs1] + kept(mix, keep1);
+  const Tensor h = at::linear(at::layer_norm(x1, {C}, p[kN2W], p[kN2B], eps[1]), p[kFc1W], p[kFc1B]);
+  return x1 * p[kRs2] + kept(at::linear(at::gelu(h), p[kFc2W], p[kFc2B]), keep2);
 }
 
 struct Block : public torch::autograd::Function<Block> {
@@ -130,6 +173,7 @@ struct Block : public torch::autograd::Function<Block> {
     TORCH_CHECK(dy.scalar_type() == at::kFloat, "m2dscan: the gradient of a block's output must be float32, got ", dy.scalar_type());
     dy = dy.contiguous();
     if (reinterpret_cast<uintptr_t>(dy.data_ptr()) % 16) dy = dy.clone();
+    if (at::GradMode::is_enabled()) return recorded(x, p, dy, keep1, keep2, eps, flip, full, interval);
 
     // one workspace for the workgroups' sums of all parameter gradients
     std::vector<m2d_reduce_seg> segs;
@@ -223,10 +267,31 @@ struct Block : public torch::autograd::Function<Block> {
     if (s.local) { seg(kLnW, o_n1 + 2 * C, 5 * C, np); seg(kLnB, o_n1 + 3 * C, 5 * C, np); }
     check(m2d_train_reduce((int)segs.size(), segs.data(), st));
 
+    return of_all(dx, out);
+  }
+
+  static variable_list of_all(const Tensor& dx, const std::vector<Tensor>& par) {
     variable_list all = {dx};
-    all.insert(all.end(), out.begin(), out.end());
+    all.insert(all.end(), par.begin(), par.end());
     all.resize(all.size() + 9);      // keep1, keep2 and the seven options take none
     return all;
+  }
+
+  // The gradients with a graph behind them (create_graph).  Every input goes in as a view of its own, so that a gradient
+  // stops there also where one input was computed from another.
+  static variable_list recorded(const Tensor& x, const std::vector<Tensor>& p, const Tensor& dy, const Tensor& keep1, const Tensor& keep2,
+                                const std::vector<double>& eps, bool flip, bool full, int64_t interval) {
+    std::vector<Tensor> in = {x.view_as(x)};
+    for (const Tensor& t : p) in.push_back(t.view_as(t));
+    const Tensor y = stock_block(in[0], {in.begin() + 1, in.end()}, keep1, keep2, eps, flip, full, interval);
+    variable_list asked;
+    for (const Tensor& t : in)
+      if (t.requires_grad()) asked.push_back(t);
+    const variable_list g = torch::autograd::grad({y}, asked, {dy}, true, true, true);
+    std::vector<Tensor> out;
+    size_t at = 0;
+    for (const Tensor& t : in) out.push_back(t.requires_grad() ? g[at++] : Tensor());
+    return of_all(out[0], {out.begin() + 1, out.end()});
   }
 };
 

@@ -718,6 +718,11 @@ __device__ __forceinline__ Ranks ranks_of(int c, int first, int R) {
   return r;
 }
 
+// Of the NL = ceil(2R / 16) tiles of ranks, those before this one hold ranks of T only, those behind it ranks of L and
+// padding; this one may hold both.  Its products are made for each half on its own, with zeros (forward) or rows that are
+// dropped (backward) in the place of the other's: an infinite value must not meet a zero weight.
+template <int NL> constexpr int kMixed = (NL - 1) / 2;
+
 template <typename T, bool V4, int NL, int NT>
 __global__ __launch_bounds__(kThreads) void m2d_proj_fwd_f32_kernel(const ProjArgs a) {
   constexpr int NO = NL + 3;
@@ -803,6 +808,17 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_fwd_f32_kernel(const ProjAr
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int lt = 0; lt < NL; ++lt) rk[h][lt] = ranks_of(16 * lt + 4 * kb, h * R, R);
+  f32x4 zl[NT];      // the mixed tile as L has it
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int lt = kMixed<NL>; lt < NL; ++lt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float v = z[t][lt][j];
+        if (lt == kMixed<NL>) zl[t][j] = rk[1][lt].own[j] ? v : 0.f;
+        z[t][lt][j] = rk[lt > kMixed<NL>][lt].own[j] ? v : 0.f;
+      }
   f32x4 dw[2][NL], bias[2];
   auto fetch_dt = [&](int e0) {
     const int e = e0 + n < E ? e0 + n : E - 1;
@@ -836,11 +852,11 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_fwd_f32_kernel(const ProjAr
     for (int lt = 0; lt < NL; ++lt)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        if (h ? 16 * lt + 16 <= R : 16 * lt >= R) continue;   // (uniform) the tile holds no rank of this half
+        if ((h ? lt < kMixed<NL> : lt > kMixed<NL>) || (h && 16 * lt + 16 <= R)) continue;   // (uniform) no rank of this half
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int t = 0; t < NT; ++t) s[t][h] = mfma4(w[h][lt][j], z[t][lt][j], s[t][h]);
+          for (int t = 0; t < NT; ++t) s[t][h] = mfma4(w[h][lt][j], h && lt == kMixed<NL> ? zl[t][j] : z[t][lt][j], s[t][h]);
       }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -878,17 +894,19 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_bwd_data_f32_kernel(const P
     for (int w = 0; w < 3; ++w)
       z[t][NL + w] = row4<T, true>(static_cast<const T*>(w == 0 ? a.dBT : (w == 1 ? a.dBL : a.dC)) + at[t] * kN, 4 * kb, kN);
   }
-  // dz of the low-rank inputs: row n of tile lt is rank 16 lt + n of the two stacked
+  // dz of the low-rank inputs: row n of tile lt is rank 16 lt + n of the two stacked (rows of the other half, and of
+  // padding, repeat one: they are dropped)
   int q[2][NL];
-  bool own[2][NL];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int lt = 0; lt < NL; ++lt) {
       const int k = 16 * lt + n - h * R;
-      own[h][lt] = k >= 0 && k < R;
-      q[h][lt] = own[h][lt] ? k : 0;
+      q[h][lt] = k >= 0 && k < R ? k : 0;
     }
+  f32x4 zl[NT];      // L's product with the mixed tile
+#pragma unroll
+  for (int t = 0; t < NT; ++t) zl[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 gv[2][NT], dv[2][NT], wv[2][NL];
   auto fetch = [&](int c) {
     const int e = c + 4 * kb;
@@ -919,11 +937,7 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_bwd_data_f32_kernel(const P
         }
       }
 #pragma unroll
-      for (int lt = 0; lt < NL; ++lt) {
-        w[h][lt] = weights_of<T>(a, wv[h][lt]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w[h][lt][j] = own[h][lt] ? w[h][lt][j] : 0.f;
-      }
+      for (int lt = 0; lt < NL; ++lt) w[h][lt] = weights_of<T>(a, wv[h][lt]);
     }
     if (c + 16 < E) fetch(c + 16);
     if (c + 16 > E) {
@@ -936,13 +950,26 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_bwd_data_f32_kernel(const P
     for (int lt = 0; lt < NL; ++lt)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        if (h ? 16 * lt + 16 <= R : 16 * lt >= R) continue;   // (uniform) the tile holds no rank of this half
+        if ((h ? lt < kMixed<NL> : lt > kMixed<NL>) || (h && 16 * lt + 16 <= R)) continue;   // (uniform) no rank of this half
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int t = 0; t < NT; ++t) z[t][lt] = mfma4(w[h][lt][j], g[h][t][j], z[t][lt]);
+          for (int t = 0; t < NT; ++t) {
+            f32x4& to = h && lt == kMixed<NL> ? zl[t] : z[t][lt];
+            to = mfma4(w[h][lt][j], g[h][t][j], to);
+          }
       }
   }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int lt = kMixed<NL>; lt < NL; ++lt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int o = 16 * lt + 4 * kb + j;
+        if (lt == kMixed<NL>) z[t][lt][j] = o < R ? z[t][lt][j] : zl[t][j];
+        z[t][lt][j] = o < R2 ? z[t][lt][j] : 0.f;
+      }
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     if (16 * t + n >= left) continue;
@@ -968,7 +995,11 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_bwd_data_f32_kernel(const P
       for (int j = 0; j < 4; ++j) {
         const int oo = 16 * ot + 4 * kb + j;
         const int o = ot < NL ? (oo < R2 ? oo : R2 - 1) : oo - 16 * NL + R2;   // (rows of padding: dz is zero)
-        const f32x4 w = weights_of<T>(a, row4<float, V4>(a.Wx + o * E, e0 + 4 * n, E));
+        f32x4 w = weights_of<T>(a, row4<float, V4>(a.Wx + o * E, e0 + 4 * n, E));
+        if (ot == NL - 1) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) w[c] = oo < R2 ? w[c] : 0.f;
+        }
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll

@@ -214,6 +214,11 @@ def _rope_qknorm_fwd_fake(qkv, cos, sin, q_weight, q_bias, k_weight, k_bias, eps
     return qkv.new_empty((B, nh, L, hd)), qkv.new_empty((B, nh, L, hd))
 
 
+@torch.library.register_fake("m2dscan::widen")
+def _widen_fake(tensors):
+    return [torch.empty_like(t, dtype=torch.float32) for t in tensors]
+
+
 def fused_backward_math(dDAT, dDAL, dHS_total, deltaT, deltaL, AT, AL, BT, BL, x):
     """The reference's tensor algebra behind ``wf_bwd`` (``wavefront_cuda.py:97-139``), for callers of the
     operator pair ``wf_fwd_op`` / ``wf_bwd_op``: from ``dDAT``, ``dDAL`` and ``dBX`` (``dHS_total``), all

@@ -101,3 +101,18 @@ def test_fused_backward_math_against_autograd():
     want = [res["d_x"] - (inp["dy"] * inp["D"]).numpy(), res["d_deltaT"], res["d_deltaL"], res["d_AT"], res["d_AL"], res["d_BT"], res["d_BL"]]
     for got, w in zip(out, want):
         assert so.rel_err(got, w) < 1e-12
+
+
+@pytest.mark.parametrize("params", [torch.float32, torch.bfloat16])
+def test_entry_point_under_fake_tensors(wf, params):
+    """The whole entry point on fake tensors, also with bf16 parameters (widened in one operator on the GPU)."""
+    from torch._subclasses import FakeTensorMode
+    B, H, W, E, N, R = 2, 5, 7, 32, 16, 2
+    with FakeTensorMode():
+        f = lambda *s, dt=params: torch.empty(*s, dtype=dt, device="cuda").requires_grad_(True)
+        x = f(B, H, W, E, dt=torch.bfloat16)
+        p = [f(E, N), f(E, N), f(2 * R + 3 * N, E), f(E, R), f(E), f(E, R), f(E), f(E)]
+        y = wf.wavefront_scan_cuda(x, *p)
+        assert y.shape == x.shape and y.dtype == x.dtype
+        wide = wf.wf_cuda_fn_proj._params(x, *p)      # (what the backward starts with; it needs a device to run)
+        assert [(w.shape, w.dtype) for w in wide] == [(t.shape, torch.float32) for t in p]
