@@ -426,7 +426,7 @@ int run_rope(const RopeArgs& a, int G, hipStream_t st) {
 // v_mfma_f32_16x16x32_bf16 as they come from memory (lane l: row l & 15, columns 8 (l >> 4) + j of a step
 // of 32), W's rows are the B operands (lane l: output l & 15, the same columns), results leave through a
 // per-wave LDS block so that memory sees 16-byte pieces of rows.  pre and post are nothing, GELU (exact
-// form, through erf) or StarReLU: the activation that the block applies before or after the layer.
+// form) or StarReLU: the activation that the block applies before or after the layer.
 constexpr int kLinThreads = 256;
 constexpr int kLinWaves = 4;
 constexpr int kLinStage = 72;      // floats per row of a wave's result block: 64 + 8
@@ -727,7 +727,7 @@ __global__ __launch_bounds__(256) void m2d_wide_linear_kernel(const WideArgs a) 
 // ------------------------------------------------------ wide linear layers with a GELU behind them, bf16
 // y = GELU(x W^T + bias) for more positions than the kernel above is made for and up to 320 inputs (the first layer of the
 // MLP in the third stage).  The stock product and the activation after it write the widest tensor of a block twice and
-// read it once; here it is written once, and the kernel is bound by the exact GELU of every output (about 17 vector
+// read it once; here it is written once, and the kernel is bound by the exact GELU of every output (about 16 vector
 // slots a value, half of the time) and the products.  A wave keeps 32 positions' rows in registers as they come from
 // memory and walks over the outputs 32 at a time; the 32 rows of W lie in LDS, read by all waves, while the next 32 are
 // on their way; three workgroups fit a compute unit, which is why 320 inputs are the most (with workgroups of 8 waves, two

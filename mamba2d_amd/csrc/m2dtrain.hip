@@ -29,19 +29,6 @@ __device__ __forceinline__ void ld4(const float* p, float (&v)[4]) {
 }
 __device__ __forceinline__ void st4(float* p, const float (&v)[4]) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
 
-// d GELU(v) / dv = Phi(v) + v phi(v), with the same erf as gelu_exact
-__device__ __forceinline__ float gelu_slope(float v) {
-  const float z = fabsf(v) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.3275911f, z, 1.f));
-  float poly = __builtin_fmaf(t, 1.061405429f, -1.453152027f);
-  poly = __builtin_fmaf(t, poly, 1.421413741f);
-  poly = __builtin_fmaf(t, poly, -0.284496736f);
-  poly = __builtin_fmaf(t, poly, 0.254829592f);
-  const float ex = __builtin_amdgcn_exp2f(-z * z * 1.44269504088896341f);      // exp(-v^2 / 2)
-  const float q = 0.5f * poly * t * ex;                                         // 1 - Phi(|v|)
-  return __builtin_fmaf(v * 0.39894228040143268f, ex, v < 0.f ? q : 1.f - q);
-}
-
 enum { kActNone = 0, kActGelu = 1, kActStarRelu = 2 };
 __device__ __forceinline__ float act(int kind, float v, float s, float b) {
   if (kind == kActGelu) return gelu_exact(v);
