@@ -573,7 +573,9 @@ def _stage_plan(stage, x):
             att = m.token_mixer
     par += [end.weight, end.bias]
     eps.append(end.eps)
-    if any(t is None for t in par):
+    # (a tensor that is no registered parameter is nothing that the plan could find changed on a later call)
+    registered = set(map(id, stage.parameters()))
+    if any(id(t) not in registered for t in par):
         return None
     return _StagePlan(stage, kinds, par, eps, att)
 

@@ -98,3 +98,20 @@ def test_hooks_of_a_stage_run(name, train):
     with torch.set_grad_enabled(train), torch.autocast("cuda", dtype=torch.bfloat16, enabled=train):
         backbone.Mamba2DBackbone._run_stage(stage, x)
     assert seen == [1, 1]
+
+
+def test_stage_plan_is_for_registered_parameters():
+    """A tensor that stands in a parameter's place as a plain attribute (as sharding tools leave one, a new one each time) is
+    nothing that a plan could compare on the next call."""
+    stage = stage_of("scan")
+    x = torch.zeros(1, 4, 4, 32)
+    with torch.no_grad():
+        plan = backbone._stage_plan(stage, x)
+        fc1 = stage[0].MLP.fc1
+        kept = fc1.weight
+        del fc1.weight
+        fc1.weight = kept.detach().clone()
+        assert not plan.holds(stage) and backbone._stage_plan(stage, x) is None
+        del fc1.weight
+        fc1.weight = kept
+        assert backbone._stage_plan(stage, x) is not None
