@@ -575,7 +575,7 @@ def _stage_plan(stage, x):
     eps.append(end.eps)
     # (a tensor that is no registered parameter is nothing that the plan could find changed on a later call)
     registered = set(map(id, stage.parameters()))
-    if any(id(t) not in registered for t in par):
+    if any(id(t) not in registered or type(t) not in wavefront._PLAIN_TYPES for t in par):
         return None
     return _StagePlan(stage, kinds, par, eps, att)
 

@@ -115,3 +115,17 @@ def test_stage_plan_is_for_registered_parameters():
         del fc1.weight
         fc1.weight = kept
         assert backbone._stage_plan(stage, x) is not None
+
+
+class _Watched(torch.Tensor):
+    pass
+
+
+def test_stage_plan_is_for_plain_parameters():
+    """A parameter of another tensor class (quantized or distributed, say) goes through the dispatched operators."""
+    stage = stage_of("scan")
+    x = torch.zeros(1, 4, 4, 32)
+    with torch.no_grad():
+        fc1 = stage[0].MLP.fc1
+        fc1.weight = torch.nn.Parameter(fc1.weight.detach().as_subclass(_Watched))
+        assert type(fc1.weight) is not torch.nn.Parameter and backbone._stage_plan(stage, x) is None
