@@ -43,9 +43,10 @@ def _inference(*tensors):
 
 
 def _untouched(mod):
-    """A call past the module's own call gives what the call would: nobody has put another ``forward`` on the instance,
-    and it has no hooks."""
-    return not ("forward" in mod.__dict__ or mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks)
+    """A call past the module's own call gives what the call would: its ``forward`` is that of a class known here (not of
+    a subclass such as an adapter, nor one that was put on the class or on the instance), and it has no hooks."""
+    return type(mod).forward in _FORWARDS and not ("forward" in mod.__dict__ or mod._forward_hooks or mod._forward_pre_hooks
+                                                   or mod._backward_hooks or mod._backward_pre_hooks)
 
 
 ACT_NONE, ACT_GELU, ACT_STARRELU = 0, 1, 2
@@ -448,20 +449,20 @@ class ResBlock(nn.Module):
 
     def _infer_parameters(self, x):
         """(kind, parameters in the order of ``m2dscan::infer_stage``, eps of norm1, norm2 and the mixer's own norm) for a
-        block whose inference is that operator's sequence of kernels; None otherwise."""
+        block of untouched modules whose inference is that operator's sequence of kernels; None otherwise."""
         mix, mlp = self.token_mixer, self.MLP
         n1, n2, s1, s2, fc1, fc2 = self.norm1, self.norm2, self.res_scale1, self.res_scale2, mlp.fc1, mlp.fc2
-        if not (_plain(mlp, MLP) and type(s1) is Scale and type(s2) is Scale and type(n1) is LayerNorm and type(n2) is LayerNorm
-                and _plain(fc1, nn.Linear) and _plain(fc2, nn.Linear)):
+        if not (type(mlp) is MLP and type(s1) is Scale and type(s2) is Scale and type(n1) is LayerNorm and type(n2) is LayerNorm
+                and type(fc1) is nn.Linear and type(fc2) is nn.Linear):
             return None
         tail = [s1.scale, n2.weight, n2.bias, fc1.weight, fc1.bias, fc2.weight, fc2.bias, s2.scale]
-        if _plain(mix, RoPEAttention2D):
+        if type(mix) is RoPEAttention2D:
             qn, kn = mix.q_norm, mix.k_norm
-            if not (mix.head_dim == 32 and qn.eps == kn.eps and _plain(mix.qkv, nn.Linear)
-                    and _plain(mix.proj, nn.Linear) and mix.qkv.bias is None and mix.proj.bias is None):
+            if not (mix.head_dim == 32 and qn.eps == kn.eps and type(mix.qkv) is nn.Linear
+                    and type(mix.proj) is nn.Linear and mix.qkv.bias is None and mix.proj.bias is None):
                 return None
             return 4, [n1.weight, n1.bias, mix.qkv.weight, qn.weight, qn.bias, kn.weight, kn.bias, mix.proj.weight, *tail], (n1.eps, n2.eps, qn.eps)
-        if not (_plain(mix, M2DBlock) and _plain(mix.in_proj, nn.Linear) and _plain(mix.out_proj, nn.Linear)
+        if not (type(mix) is M2DBlock and type(mix.in_proj) is nn.Linear and type(mix.out_proj) is nn.Linear
                 and mix.recomp in ("partial", "full") and mix.x_proj.bias is None and mix.AT_log.shape[1] == wavefront.STATES_PER_CALL and mix.dt_projT.weight.shape[1] <= 32):
             return None
         par = [n1.weight, n1.bias, mix.in_proj.weight, mix.in_proj.bias, mix.AT_log, mix.AL_log, mix.x_proj.weight, mix.dt_projT.weight,
@@ -470,7 +471,7 @@ class ResBlock(nn.Module):
         if path is None:
             return int(mix.flip), par, (n1.eps, n2.eps, 0.0)
         conv = path.dwconv
-        if not (_plain(path, SepConv) and type(mix.local_norm) is LayerNorm and _plain(path.pwconv1, nn.Linear) and _plain(path.pwconv2, nn.Linear)
+        if not (type(path) is SepConv and type(mix.local_norm) is LayerNorm and type(path.pwconv1) is nn.Linear and type(path.pwconv2) is nn.Linear
                 and type(conv) is nn.Conv2d and conv.kernel_size == (3, 3) and conv.padding == (1, 1) and conv.stride == (1, 1)
                 and conv.dilation == (1, 1) and conv.bias is None and conv.padding_mode == "zeros" and type(path.act1) is StarReLU
                 and type(path.act2) is StarReLU and path.pwconv1.bias is None and path.pwconv2.bias is None
@@ -511,8 +512,13 @@ class ResBlock(nn.Module):
         return self.forward_fused(x)[0]
 
 
+_KINDS = (nn.Linear, nn.Conv2d, nn.LayerNorm, nn.Sequential, nn.Identity, LayerNorm, StarReLU, Scale, MLP, SepConv, M2DBlock, RoPEAttention2D,
+          ResBlock)
+_FORWARDS = frozenset(kind.forward for kind in _KINDS)
+
+
 def _module_ops():
-    return (dwconv3x3_fwd_op, layernorm_fwd_op, layernorm_linear_act_fwd_op, linear_act_fwd_op, mlp_fwd_op, rope_attention_fwd_op,
+    return (*(kind.forward for kind in _KINDS), dwconv3x3_fwd_op, layernorm_fwd_op, layernorm_linear_act_fwd_op, linear_act_fwd_op, mlp_fwd_op, rope_attention_fwd_op,
             scale_residual_fwd_op, scale_residual_layernorm_fwd_op, wavefront_scan_cuda)
 
 
@@ -527,10 +533,12 @@ class _StagePlan:
     OPTIONS = ("training", "eps", "flip", "recomp", "kernel_size", "padding", "stride", "dilation", "padding_mode", "head_dim", "num_heads",
                "rope_base", "axis_dim", "normalized_shape")
 
-    def __init__(self, stage, kinds, par, eps, att):
+    def __init__(self, mods, kinds, par, eps, att):
         self.kinds, self.par, self.eps, self.att = kinds, par, eps, att
         self.own, self.keys, self.was, self.hooks, self.dicts = [], [], [], [], []
-        for m in stage.modules():
+        self.mods = mods[1:]      # (not the stage: the table of plans must not keep its key alive)
+        self.types = list(map(type, self.mods))
+        for m in mods:
             d = m.__dict__
             self.dicts.append(d)
             for own in (m._modules, m._parameters, {k: d[k] for k in self.OPTIONS if k in d}):
@@ -546,6 +554,7 @@ class _StagePlan:
     def holds(self, stage):
         try:
             return (all(map(operator.is_, map(operator.getitem, self.own, self.keys), self.was)) and not any(self.hooks)
+                    and all(map(operator.is_, map(type, self.mods), self.types))
                     and not any(map(operator.contains, self.dicts, itertools.repeat("forward"))) and len(stage) == len(self.kinds) + 1)
         except KeyError:
             return False
@@ -555,9 +564,9 @@ _STAGE_PLANS = weakref.WeakKeyDictionary()
 
 
 def _stage_plan(stage, x):
-    mods = list(stage)
+    mods, within = list(stage), list(stage.modules())
     end = mods[-1]
-    if type(end) is not LayerNorm or end.weight is None or end.bias is None or end.training or not all(map(_untouched, stage.modules())):
+    if type(end) is not LayerNorm or end.weight is None or end.bias is None or end.training or not all(map(_untouched, within)):
         return None
     kinds, par, eps, att = [], [], [], None
     for m in mods[:-1]:
@@ -574,10 +583,10 @@ def _stage_plan(stage, x):
     par += [end.weight, end.bias]
     eps.append(end.eps)
     # (a tensor that is no registered parameter is nothing that the plan could find changed on a later call)
-    registered = set(map(id, stage.parameters()))
-    if any(id(t) not in registered or type(t) not in wavefront._PLAIN_TYPES for t in par):
+    registered = {id(t) for m in within for t in m._parameters.values()}
+    if any(t is None or id(t) not in registered or type(t) not in wavefront._PLAIN_TYPES for t in par):
         return None
-    return _StagePlan(stage, kinds, par, eps, att)
+    return _StagePlan(within, kinds, par, eps, att)
 
 
 def _infer_stage(stage, x):
@@ -651,7 +660,7 @@ class Mamba2DBackbone(nn.Module):
             return fast
         mods = list(stage)
         normed = None
-        own = lambda m: isinstance(m, ResBlock) and type(m).forward is ResBlock.forward and _untouched(m)
+        own = lambda m: isinstance(m, ResBlock) and _untouched(m)
         for i, m in enumerate(mods):
             if own(m):
                 nxt = mods[i + 1] if i + 1 < len(mods) else None

@@ -129,3 +129,34 @@ def test_stage_plan_is_for_plain_parameters():
         fc1 = stage[0].MLP.fc1
         fc1.weight = torch.nn.Parameter(fc1.weight.detach().as_subclass(_Watched))
         assert type(fc1.weight) is not torch.nn.Parameter and backbone._stage_plan(stage, x) is None
+
+
+class _Scaled(torch.nn.Linear):
+    """A layer with something beside its weight, as adapters have it."""
+
+    def forward(self, x):
+        return 3 * super().forward(x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["token_mixer.in_proj", "token_mixer.out_proj", "token_mixer.local_path.pwconv1", "token_mixer.local_path.pwconv2",
+                                  "MLP.fc1", "MLP.fc2"])
+@pytest.mark.parametrize("way", ["subclass", "class"])
+def test_other_layers_run_their_own_forward(monkeypatch, name, way):
+    print(f"\ncase other layer {name} {way}", flush=True)
+    stage = stage_of("scan").cuda().bfloat16()
+    x = torch.randn(1, 4, 4, 32, device="cuda").bfloat16()
+    run = lambda: backbone.Mamba2DBackbone._run_stage(stage, x)
+    seen = []
+    with torch.no_grad():
+        before = run()
+        if way == "subclass":
+            stage[0].get_submodule(name).__class__ = _Scaled
+            assert not torch.equal(run(), before)
+        else:
+            plain = torch.nn.Linear.forward
+            with monkeypatch.context() as m:
+                m.setattr(torch.nn.Linear, "forward", lambda self, t: (seen.append(self), plain(self, t))[1])
+                run()
+            assert stage[0].get_submodule(name) in seen
+            assert torch.equal(run(), before)
