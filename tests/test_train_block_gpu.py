@@ -73,7 +73,7 @@ def test_block_drop_path_and_frozen_parameters():
         y = block(x)
     y.sum().backward()
     same = (y == x * (block.res_scale1.scale * block.res_scale2.scale)).flatten(1).all(1)
-    assert 0 < int(same.sum()) < 16 or torch.isfinite(y).all()
+    assert 0 < int(same.sum()) < 16 and torch.isfinite(y).all()      # (a quarter of the samples drop both branches)
     dropped = (x.grad == 1).flatten(1).all(1)
     assert torch.equal(same, dropped)
     assert block.MLP.fc1.weight.grad is None and block.MLP.fc2.weight.grad is not None
