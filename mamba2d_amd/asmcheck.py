@@ -1,15 +1,18 @@
 """Build-time check of the generated gfx950 assembly for hazards that the compiler cannot see.
 
 The scan kernels fold DPP row shifts into arithmetic instructions with inline assembly
-(v_fmac_f32_dpp, v_mul_f32_dpp, v_add_f32_dpp).  The compiler's hazard recogniser does not look
-inside inline assembly, so two rules of the ISA are the source's own responsibility:
+(v_fmac_f32_dpp, v_mul_f32_dpp, v_add_f32_dpp), and write boundary rows through with stores of their own.
+The compiler's hazard recogniser does not look inside inline assembly, so three rules of the ISA are the
+source's own responsibility:
 
 * a VGPR that a DPP instruction reads through the lane shift (its src0) must not have been
   written by a vector instruction in the two preceding issue slots;
 * a VGPR written by a transcendental instruction (v_exp/v_log/v_rcp/v_rsq/v_sqrt) must not be
-  read by a vector instruction in the next issue slot.
+  read by a vector instruction in the next issue slot;
+* the VGPRs whose contents a store of more than 8 bytes (written in inline assembly) sends must not be written by a vector instruction in the
+  next two issue slots (the store still reads them).
 
-The source arranges its code so that neither can happen; this module verifies it on the assembly
+The source arranges its code so that none of them can happen; this module verifies it on the assembly
 that was actually produced, and the build fails if it finds a violation.
 
 It also reads the compiler's own per-kernel summary for register spills: the scan kernels are
@@ -23,6 +26,7 @@ import re
 _DPP = re.compile(r"(v_\w+_dpp)\s+v(\d+),\s*v(\d+),\s*v(\d+)")
 _WRITE = re.compile(r"(v_\w+|ds_read\w*|global_load\w*|scratch_load\w*|buffer_load\w*)\s+(?:v\[(\d+):(\d+)\]|v(\d+))")
 _TRANS = re.compile(r"v_(exp|log|rcp|rsq|sqrt)_f32")
+_WIDE_STORE = re.compile(r"global_store_dwordx[34]\s+\S+,\s*v\[(\d+):(\d+)\]")
 _NOP = re.compile(r"s_nop (\d+)")
 _KERNEL = re.compile(r"^(_Z\w+):")
 
@@ -38,13 +42,15 @@ def _written(inst: str) -> set:
 
 def check_text(text: str):
     """Returns (number of DPP instructions seen, list of (kernel, producer, consumer) violations)."""
-    kernel, hist, ndpp, bad = None, [], 0, []
+    kernel, hist, ndpp, bad, inline = None, [], 0, [], False
     for line in text.splitlines():
         t = line.strip()
         k = _KERNEL.match(t)
         if k:
             kernel, hist = k.group(1), []
             continue
+        if t.startswith((";;#ASMSTART", ";;#ASMEND")):
+            inline = t.startswith(";;#ASMSTART")
         if not line.startswith("\t") or not t or t[0] in ".;":
             continue
         m = _DPP.match(t)
@@ -53,7 +59,7 @@ def check_text(text: str):
             regs = {int(m.group(2)), int(m.group(3)), int(m.group(4))}
             shifted = int(m.group(3))
             slots = 0
-            for prev, width in reversed(hist):
+            for prev, width, _ in reversed(hist):
                 w = _written(prev)
                 if slots < 1 and _TRANS.match(prev) and w & regs:
                     bad.append((kernel, prev, t))
@@ -64,8 +70,19 @@ def check_text(text: str):
                 slots += width
                 if slots >= 2:
                     break
+        if t.startswith("v_"):
+            w = _written(t)
+            slots = 0
+            for prev, width, own in reversed(hist):
+                if slots >= 2:
+                    break
+                s = _WIDE_STORE.match(prev)
+                if s and own and w & set(range(int(s.group(1)), int(s.group(2)) + 1)):
+                    bad.append((kernel, prev, t))
+                    break
+                slots += width
         n = _NOP.match(t)
-        hist.append((t, int(n.group(1)) + 1 if n else 1))
+        hist.append((t, int(n.group(1)) + 1 if n else 1, inline))
         del hist[:-8]
     return ndpp, bad
 

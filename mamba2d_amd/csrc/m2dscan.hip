@@ -361,10 +361,12 @@ __device__ __forceinline__ uint32_t link_poll(const uint32_t* ptr) {
 __device__ __forceinline__ void link_publish(uint32_t* ptr, uint32_t v) {
   asm volatile("global_store_dword %0, %1, off sc1" ::"v"(ptr), "v"(v) : "memory");
 }
-// 16 bytes of a boundary row, written through at device scope
+// 16 bytes of a boundary row, written through at device scope.  A store of more than 8 bytes reads its data while the next
+// instructions issue: a vector instruction may write those registers again two wait states later at the earliest, which the compiler
+// sees to for its own stores but not for one in inline assembly.
 __device__ __forceinline__ void store_row_device_scope(float4* dst, float4 v) {
   const v4f_t w = {v.x, v.y, v.z, v.w};
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(dst), "v"(w) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(dst), "v"(w) : "memory");
 }
 template <int PUB>   // the thread that publishes: one of a wave that waits, so that it knows of a wait given up
 struct LinkT {

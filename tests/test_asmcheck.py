@@ -47,3 +47,18 @@ def test_kernels_that_ask_for_scratch_memory_are_listed():
     text = ("\t.amdhsa_kernel _ZN1k3fooEv\n\t\t.amdhsa_private_segment_fixed_size 0\n\t.end_amdhsa_kernel\n"
             "\t.amdhsa_kernel _ZN1k3barEv\n\t\t.amdhsa_private_segment_fixed_size 932\n\t.end_amdhsa_kernel\n")
     assert asmcheck.spilling_kernels(text) == [("_ZN1k3barEv", 932)]
+
+
+def test_wide_store_data_overwritten_too_early():
+    plain = "global_store_dwordx4 v[10:11], v[4:7], off sc1"
+    store = f";;#ASMSTART\n\t{plain}\n\t;;#ASMEND"
+    for first in range(4, 8):
+        write = f"v_mul_f32_e32 v{first}, v20, v21"
+        assert len(asmcheck.check_text(listing(store, write))[1]) == 1
+        assert len(asmcheck.check_text(listing(store, "v_mul_f32_e32 v30, v20, v21", write))[1]) == 1
+        assert asmcheck.check_text(listing(store, "s_nop 1", write))[1] == []
+        assert asmcheck.check_text(listing(store, "s_nop 0", "v_mul_f32_e32 v30, v20, v21", write))[1] == []
+    assert asmcheck.check_text(listing(store, "v_mul_f32_e32 v8, v20, v21"))[1] == []      # another register
+    assert asmcheck.check_text(listing(plain, "v_mul_f32_e32 v4, v20, v21"))[1] == []      # the compiler's own: it knows the rule
+    assert asmcheck.check_text(listing(store.replace("x4", "x2").replace("[4:7]", "[4:5]"),
+                                       "v_mul_f32_e32 v4, v20, v21"))[1] == []             # 8 bytes are read at issue
