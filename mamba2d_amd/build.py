@@ -50,7 +50,7 @@ SPILL_ALLOWANCE = [(re.compile(r"m2d_bwd_kernelI\w*Li8ELb1E\w*EEv"), 64)]   # (<
 # A kernel that runs out of scalar registers parks some in lanes of a vector register; the compiler then reserves a
 # few bytes of scratch for that register without ever storing it.  Allowed up to this many bytes per lane, and only
 # where the kernel has no scratch load or store at all.
-UNTOUCHED_SCRATCH = 64
+UNTOUCHED_SCRATCH = 128
 
 
 def build_lib(verbose: bool = True) -> str:

@@ -336,14 +336,16 @@ struct Stage {
 // completion is awaited once per block by staging_landed() (counter vmcnt), not before every LDS
 // read that follows it, which is what the compiler does for the builtin.
 // DEVICE_SCOPE: read past the L1 (data written earlier in the same launch by this workgroup).
+__device__ __forceinline__ uint32_t lds_offset(char* at) { return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) char*)at); }
 template <bool DEVICE_SCOPE>
-__device__ __forceinline__ void lds_fill16(const void* src, char* lds_window) {
-  const uint32_t base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) char*)lds_window);
+__device__ __forceinline__ void lds_fill16_at(const void* src, uint32_t base) {
   if constexpr (DEVICE_SCOPE)
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off sc1" ::"v"(src), "s"(base) : "memory", "m0");
   else
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(base) : "memory", "m0");
 }
+template <bool DEVICE_SCOPE>
+__device__ __forceinline__ void lds_fill16(const void* src, char* lds_window) { lds_fill16_at<DEVICE_SCOPE>(src, lds_offset(lds_window)); }
 
 // ---- linked sweep: hand-off between the workgroups of neighbouring bands inside one launch.
 // Boundary rows and progress counts are written through to memory and read past the caches at
@@ -388,6 +390,8 @@ struct LinkT {
   }
   // this workgroup's results mean nothing: it gave up waiting, or a band it depends on did
   __device__ __forceinline__ bool broken() const { return gave_up || seen == kLinkAbort; }
+  // (uniform) the neighbour is known to have `need` blocks done
+  __device__ __forceinline__ bool ready(uint32_t need) const { return !dep || seen >= need; }
   // (uniform) returns once the neighbour has `need` blocks done
   __device__ __forceinline__ void wait_for(uint32_t need) {
     if (!dep || seen >= need) return;
@@ -1324,308 +1328,7 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW, EC>()) * 64) void m2d
   }
 }
 
-// ------------------------------------------------------- forward, the states of a channel split over lanes
-// Few images leave most of the device idle with the kernel above (a wave per 4 channels of an
-// image), and a sweep then takes as long as one wave needs for its chain of instructions.  Here the
-// 16 states of ONE channel are split over the 4 lane groups of a wave (lane = (state group g, row r),
-// 4 states per lane): four times as many waves, each with about a third of the instructions per
-// step.  A workgroup has 8 waves = 8 channels.  Staging, schedules and memory formats are those of
-// m2d_fwd_kernel; y of a cell is the sum over the 4 lane groups (two lane-swap steps), stored by group 0.
-constexpr int kSplitWaves = 8;
-constexpr int kSplitHalfWaves = 4;   // where workgroups of 8 would leave compute units idle
-// Workgroups of 4 waves: a step of a wave that has a SIMD to itself takes as long as its chain of
-// instructions, and of those under a third are the step's arithmetic; the rest stages the next block (positions,
-// addresses, copies, the wait for the neighbouring band).  So such a workgroup gets 4 more waves that do nothing but
-// stage (and, in the backward, add up the channel sums of every step), one to a SIMD beside a wave that does nothing
-// but sweep: the two chains run side by side.
-// Workgroups of 8 sweeping waves have the same 4 (3 waves to a SIMD, 168 registers a lane: 1024x1024x64 fp32 forward
-// 2.29 -> 2.10 ms, backward 4.97 -> 4.39; 32 images of 56x56x64 bf16, one stream each, 0.146 -> 0.134 and 0.338 ->
-// 0.284), except where rows are not whole 16-byte chunks (SX false: the compiler's
-// register allocator fails on those kernels at 768 threads).  With 8 more the backward no longer fits the registers
-// of a lane at 4 waves to a SIMD and ran a quarter slower.
-constexpr int kSplitHelpers = 4;
-template <int MODE, int NWS, bool SX = true>
-constexpr int split_helpers() { return (NWS == kSplitHalfWaves || SX) ? kSplitHelpers : 0; }
-__device__ __forceinline__ float sum_over_groups(float v) {
-  v = fold16(v, v);
-  return fold32(v, v);
-}
-// the value a tensor of type T would hold
-__device__ __forceinline__ float as_stored(float v, const float*) { return v; }
-__device__ __forceinline__ float as_stored(float v, const bf16_t*) { return bf16_bits_to_f32(f32_to_bf16_bits(v)); }
-
-// A * log2 e and D from the caller's tensors: of type T, or the parameters as the module holds them (fp32 A_log and D:
-// A = -exp(A_log), and both are rounded to T, which is what the reference's casts to x.dtype do, wavefront_cuda.py:72-73,
-// 90-91, 332).
-template <typename T>
-__device__ __forceinline__ float gate_rate(const ScanParams& p, const void* A, int i) {
-  return (p.raw ? as_stored(-expf(static_cast<const float*>(A)[i]), static_cast<const T*>(nullptr)) : IO<T>::ld(static_cast<const T*>(A) + i)) * kLog2e;
-}
-template <typename T>
-__device__ __forceinline__ float skip_gain(const ScanParams& p, int e) {
-  return p.raw ? as_stored(static_cast<const float*>(p.D)[e], static_cast<const T*>(nullptr)) : IO<T>::ld(static_cast<const T*>(p.D) + e);
-}
-// The set-up launch (m2d_prep_kernel) is for kernels whose lanes hold all states of a channel, for a backward that will
-// read the same values, and for progress counts.  A lane here holds 4 states of one channel, so a forward with neither
-// works them out itself and saves the launch and the gap behind it.
-template <bool CKPT, int MODE>
-constexpr bool split_owns_setup() { return !CKPT && MODE != kModeSliced; }
-__device__ float m2d_zero_page[kZeroFloats];     // the page of zeros of such a forward: never written
-
-template <typename T, bool CKPT, bool WRITE_Y, bool STAGE_X, int MODE, int NWS = kSplitWaves>
-__global__ __launch_bounds__((NWS + split_helpers<MODE, NWS, STAGE_X>()) * 64) void m2d_fwd_split_kernel(const ScanParams pin) {
-  static_assert(MODE != kModeStacked, "stacked images are many: they never need the split");
-  constexpr bool SLICED = MODE == kModeSliced;
-  constexpr bool OWN_SETUP = split_owns_setup<CKPT, MODE>();
-  const ScanParams& p = pin;
-  __builtin_assume(p.stacked == 0);
-  __builtin_assume(p.rb == kRB);
-  __builtin_assume(p.S >= kHB + kCK - 1);
-  constexpr int NW = NWS, CW = NW;
-  constexpr int NH = split_helpers<MODE, NWS, STAGE_X>();   // waves that only stage (then the first NW waves only sweep)
-  constexpr int NSTG = NH ? NH : NW;               // waves that share the copies of a block
-  using SG = Stage<T, 3, CW, false>;
-  constexpr bool WIDEN = sizeof(T) == 2;
-  extern __shared__ float4 smem[];
-  char* lds = reinterpret_cast<char*>(smem);       // two staging buffers
-  char* raw = lds + 2 * SG::kBytes;                // [2][kRawBytes] (16-bit B_T, B_L, C on their way)
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int lb = SLICED ? (int)blockIdx.x : logical_block(p.nwg);
-  int m_lo = 0, m_hi = p.nblk;
-  int my_band = 0;
-  LinkT<NH ? NW * 64 : 0> link;
-  if constexpr (SLICED) {
-    const int per = p.B * p.bpb;
-    my_band = lb / per;
-    lb -= my_band * per;
-    m_lo = my_band * p.sl_nbb;
-    m_hi = m_lo + p.sl_nbb;
-    link.mine = p.prog + ((int64_t)my_band * per + lb) * kLinkStride;
-    link.dep = my_band > 0 ? link.mine - per * kLinkStride : nullptr;
-    link.err = p.link_err;
-    link.rig(p, my_band);
-  }
-  const bool helper = NH && wave >= NW;             // (uniform) stages, never sweeps
-  const bool stages = !NH || helper;
-  const int swave = NH ? wave - NW : wave;          // the wave's turn among those that stage
-  const int b = lb / p.bpb;
-  const int e_wg0 = (lb % p.bpb) * CW;
-  const int g = lane >> kHBShift, r = lane & (kHB - 1);   // state group, lane row
-  const int rbands = row_bands(p, r);
-  const int ch_loc = helper ? 0 : wave;             // the wave's channel inside the workgroup
-  const bool ch_ok = !helper && e_wg0 + ch_loc < p.E;   // (uniform) idle waves still take part in staging and barriers
-  const int e0 = ch_ok ? e_wg0 + ch_loc : p.E - 1;
-  for (int i = threadIdx.x; i < 2 * SG::kBytes / 16; i += (NW + NH) * 64) smem[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-
-  // Position 4g + w of a record is met by register w: state sinv(4g + w) in fold order, state 4g + w
-  // where the records come straight from fp32 tensors (natural order).
-  const bool direct = (WIDEN || !CKPT) && p.bc_direct != 0;   // (uniform)
-  float a2t[4], a2l[4];
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const int q = w == 1 ? 2 : (w == 2 ? 1 : w);   // sinv<true>(4g + w) = q * 4 + g
-    const int n = (!WIDEN && direct) ? 4 * g + w : q * 4 + g;
-    a2t[w] = OWN_SETUP ? gate_rate<T>(p, p.AT, e0 * kN + n) : p.A2T[e0 * kN + n];
-    a2l[w] = OWN_SETUP ? gate_rate<T>(p, p.AL, e0 * kN + n) : p.A2L[e0 * kN + n];
-  }
-  static_assert(sinv<true>(1) == 8 && sinv<true>(6) == 5 && sinv<true>(15) == 15, "fold order");
-  const float dsk = OWN_SETUP ? skip_gain<T>(p, e0) : p.Df[e0];
-  settle_loads();
-  __syncthreads();
-
-  const T* X = static_cast<const T*>(p.x);
-  const T* DT = static_cast<const T*>(p.dT);
-  const T* DL = static_cast<const T*>(p.dL);
-  const T* DY = DL;
-  const int64_t img_cell0 = (int64_t)b * p.Hs * p.W;
-  const int64_t img_bytes = img_cell0 * p.E * (int64_t)sizeof(T);
-  char* Yimg = static_cast<char*>(p.y) + img_bytes;
-  const char* Ximg = reinterpret_cast<const char*>(X) + img_bytes;
-  const char* DTimg = reinterpret_cast<const char*>(DT) + img_bytes;
-  const char* DLimg = reinterpret_cast<const char*>(DL) + img_bytes;
-  const uint32_t estep = (uint32_t)(p.flip ? -p.E : p.E) * (uint32_t)sizeof(T);
-  const uint32_t wrap_adj = (uint32_t)(p.rb * p.W - p.S) * estep;
-  const float g1 = r == 0 ? 1.f : 0.f;             // the ghost's T input coefficient
-
-  // the lane's group of B_T (the ghost: of the row above), of B_L and C (the ghost: zeros of its own row)
-  const uint32_t row_off = r * 16 + g * SG::kPlane;
-  const uint32_t rec_off = r == 0 ? SG::top_off(ch_loc) + g * SG::kPlane : row_off;
-  const uint32_t const_off = SG::kConstPlane * SG::kPlane + r * 16;
-  const uint32_t xd_off = SG::kXOff + SG::x_off(r, ch_loc + (CW < SG::kElem ? e_wg0 & (SG::kElem - 1) : 0));   // (4 channels of a 16-bit tensor: their half of the chunk)
-  constexpr uint32_t kXK = SG::kXStepBytes;
-
-  BlockPos bp;
-  uint32_t cell_off0 = 0;
-  float h[4] = {0.f, 0.f, 0.f, 0.f};
-  typename Snap<T>::quad* ckp = nullptr;
-
-  auto step = [&](const char* bufc, int k) {
-    float xv = 0.f, dtv = 0.f, dlv = 0.f;
-    const bool inr = ch_ok && ((bp.in_grid >> k) & 1u);
-    const uint32_t goff = cell_off0 + (uint32_t)k * estep + (k >= bp.kw ? wrap_adj : 0u);
-    if constexpr (STAGE_X) {
-      const T* xr = reinterpret_cast<const T*>(bufc + xd_off + k * kXK);
-      xv = IO<T>::ld(xr); dtv = IO<T>::ld(xr + SG::kXTauBytes / sizeof(T)); dlv = IO<T>::ld(xr + 2 * SG::kXTauBytes / sizeof(T));
-    } else if (inr) {
-      xv = IO<T>::ld(reinterpret_cast<const T*>(Ximg + goff));
-      dtv = IO<T>::ld(reinterpret_cast<const T*>(DTimg + goff));
-      dlv = IO<T>::ld(reinterpret_cast<const T*>(DLimg + goff));
-    }
-    const float4 kk = *reinterpret_cast<const float4*>(bufc + const_off + k * SG::kKStr);
-    const float4 b4 = *reinterpret_cast<const float4*>(bufc + rec_off + k * SG::kKStr);
-    const float4 l4 = *reinterpret_cast<const float4*>(bufc + row_off + SG::kBLOff + k * SG::kKStr);
-    const float4 c4 = WRITE_Y ? *reinterpret_cast<const float4*>(bufc + row_off + SG::kCOff + k * SG::kKStr) : make_float4(0, 0, 0, 0);
-    const float offT = kk.x, offL = kk.y, cT = kk.z, cL = kk.w;
-    const float bq[4] = {b4.x, b4.y, b4.z, b4.w}, lq[4] = {l4.x, l4.y, l4.z, l4.w}, cq[4] = {c4.x, c4.y, c4.z, c4.w};
-    const float sT = __builtin_fmaf(cT * dtv, xv, g1);
-    const float sL = cL * dlv * xv;
-    // gates before chains (see m2d_fwd_kernel: no DPP multiply-add right behind the v_exp that makes its gate)
-    float aT[4], aL[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) aT[w] = fexp2(__builtin_fmaf(dtv, a2t[w], offT));
-    pin4(aT);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) aL[w] = fexp2(__builtin_fmaf(dlv, a2l[w], offL));
-    pin4(aL);
-    __builtin_amdgcn_sched_barrier(0);
-    if (CKPT && k == 0) Snap<T>::store(ckp, h[0], h[1], h[2], h[3]);   // the lane's states as they are before this step
-    float acc = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      float u = sL * lq[w];
-      u = __builtin_fmaf(sT, bq[w], u);
-      u = fma_row_below(aT[w], h[w], u);
-      const float hn = __builtin_fmaf(aL[w], h[w], u);
-      h[w] = hn;
-      if (WRITE_Y) acc = __builtin_fmaf(hn, cq[w], acc);
-    }
-    if (p.nbands > 1) {   // last row of a band: the next band's ghost will replay it
-      const bool wk = k >= bp.kw;
-      const int bk = wk ? bp.bnd0 + 1 : bp.bnd0;
-      if (inr && r == kRB && bk + 1 < p.nbands) {
-        const int ck = wk ? bp.col0 + k - p.S : bp.col0 + k;
-        float4* tw = reinterpret_cast<float4*>(p.top + ((((int64_t)bk * p.B + b) * p.W + ck) * p.E + e0) * kN) + g;
-        const float4 row = make_float4(h[0], h[1], h[2], h[3]);
-        if constexpr (SLICED) store_row_device_scope(tw, row); else *tw = row;
-      }
-    }
-    if constexpr (WRITE_Y) {
-      const float yv = __builtin_fmaf(xv, dsk, sum_over_groups(acc));
-      if (inr && g == 0) IO<T>::st(reinterpret_cast<T*>(Yimg + goff), yv);
-    }
-  };
-
-  Pos A = pos_of(p, m_lo * kCK - (kHB - 1));     // position of the stream index t0 - 15 (wave-uniform)
-  bp = block_pos(p, A, r, rbands);
-  int cell0 = cell_of(p, bp.bnd0, r, bp.col0);
-  if constexpr (SLICED) { if (stages) link.wait_for(link_need_fwd(0, p.sl_nbb)); }
-  BlockPos bpq = bp;     // 16-bit direct records: the block after the next (fetched two blocks ahead)
-  int cellq = cell0;
-  int rp = 0;
-  if (direct) {
-    if constexpr (WIDEN) {
-      if (stages) bc_raw_copy<NSTG>(p, pin.bcd, raw, b, bp, cell0, swave, lane, true);
-      bpq = block_pos(p, pos_after(p, A, kCK), r, rbands);
-      cellq = cell_of(p, bpq.bnd0, r, bpq.col0);
-      if (stages) bc_raw_copy<NSTG>(p, pin.bcd, raw + kRawBytes, b, bpq, cellq, swave, lane, m_lo + 1 < m_hi);
-    } else {
-      if (stages) bc_direct_copy<T, CW, NSTG>(p, pin.bcd, lds, b, bp, cell0, swave, lane);
-    }
-    if (stages) stage_block<T, 3, CW, false, STAGE_X, NSTG, true>(p, lds, b, A, bp, cell0, e_wg0, swave, lane, X, DT, DL, DY);
-    if constexpr (WIDEN) {
-      staging_fence();
-      if (stages) bc_widen<SG, NSTG>(raw, lds, swave, lane);
-    }
-  } else {
-    if (stages) stage_block<T, 3, CW, false, STAGE_X, NSTG>(p, lds, b, A, bp, cell0, e_wg0, swave, lane, X, DT, DL, DY);
-  }
-  staging_fence();
-  int cur = 0;
-  // The sweep over the blocks of the window, as a wave of the given role runs it: kAll stages and sweeps; with waves
-  // that only stage, those run it as kStager and the others as kSweeper, each with its own part of the work and all
-  // with the same barriers.
-  auto sweep = [&](auto role) {
-  constexpr int ROLE = decltype(role)::value;
-  constexpr bool STAGES = ROLE != kSweeper, SWEEPS = ROLE != kStager;
-  for (int m = m_lo; m < m_hi; ++m) {
-    const bool last = m + 1 == m_hi;
-    const Pos An = pos_after(p, A, kCK);
-    BlockPos bpn;
-    int celln;
-    if (WIDEN && direct) {
-      bpn = bpq;
-      celln = cellq;
-      bpq = block_pos(p, pos_after(p, An, kCK), r, rbands);
-      cellq = cell_of(p, bpq.bnd0, r, bpq.col0);
-      if constexpr (STAGES) bc_raw_copy<NSTG>(p, pin.bcd, raw + rp * kRawBytes, b, bpq, cellq, swave, lane, m + 2 < m_hi);
-    } else {
-      bpn = block_pos(p, An, r, rbands);
-      celln = cell_of(p, bpn.bnd0, r, bpn.col0);
-    }
-    if (STAGES && !last) {
-      if constexpr (SLICED) link.wait_for(link_need_fwd(m + 1 - m_lo, p.sl_nbb));
-      if (direct) {
-        if constexpr (!WIDEN) bc_direct_copy<T, CW, NSTG>(p, pin.bcd, lds + (cur ^ 1) * SG::kBytes, b, bpn, celln, swave, lane);
-        stage_block<T, 3, CW, false, STAGE_X, NSTG, true>(p, lds + (cur ^ 1) * SG::kBytes, b, An, bpn, celln, e_wg0, swave, lane, X, DT, DL, DY);
-        if constexpr (WIDEN) bc_widen<SG, NSTG>(raw + (rp ^ 1) * kRawBytes, lds + (cur ^ 1) * SG::kBytes, swave, lane);
-      } else {
-        stage_block<T, 3, CW, false, STAGE_X, NSTG>(p, lds + (cur ^ 1) * SG::kBytes, b, An, bpn, celln, e_wg0, swave, lane, X, DT, DL, DY);
-      }
-    }
-    rp ^= 1;
-    if constexpr (SWEEPS) {
-    cell_off0 = (uint32_t)(cell0 * p.E + e0) * (uint32_t)sizeof(T);
-    if constexpr (CKPT) {   // every lane stores, without a branch inside the step: see m2d_fwd_kernel
-      const bool keep = m > 0 && snapshot_kept(p, m, m_lo);
-      ckp = snapshot_at<T>(p, b, (keep && ch_ok) ? snapshot_index<SLICED>(p, m, m_lo, my_band) : 0, e0, p.ck_nblk) + snap_lane(r) + snap_quad(g);
-    }
-    const char* bufc = lds + cur * SG::kBytes;
-    // (uniform) stores that the wave is sure to issue in the first three steps, after the copies for the
-    // next block: y where some lane is on the grid at all three, the boundary row where the band's last row
-    // is and another band follows.  They need not have completed when the block ends, only the copies.
-    const bool on3 = ch_ok && (bp.in_grid & 7u) == 7u;
-    const bool y_thrice = WRITE_Y && __any(on3);
-    const bool top_thrice = p.nbands > 1 && __any(on3 && r == kRB && bp.kw >= kCK && bp.bnd0 + 1 < p.nbands);
-    // Linked sweep: the band below needs, of the newest block it is told about, the boundary rows of the steps 0 and
-    // 1 only (link_need_fwd).  With just the stores issued after those of step 1 left in flight (y of step 1, row and
-    // y of step 2), this block counts as done at its end.
-    const int younger = SLICED ? (y_thrice ? 2 : 0) + (top_thrice ? 1 : 0)
-                               : (CKPT ? 1 : 0) + (y_thrice ? 3 : 0) + (top_thrice ? 3 : 0);
-#pragma unroll
-    for (int k = 0; k < kCK; ++k) {
-      if (k == kCK - 1) staging_landed_behind_n(younger);
-      if (k == 0 || k == kCK / 2) lead_if_younger<NW>(wave, k == 0);
-      step(bufc, k);
-    }
-    } else {
-      staging_landed();   // the next block's operands are in place
-    }
-    __syncthreads();
-    if constexpr (SLICED && STAGES) link.publish((uint32_t)(m - m_lo + 1));
-    cur ^= 1;
-    A = An;
-    bp = bpn;
-    cell0 = celln;
-  }
-  };
-  if constexpr (NH == 0) sweep(std::integral_constant<int, kAll>{});
-  else if (helper) sweep(std::integral_constant<int, kStager>{});
-  else sweep(std::integral_constant<int, kSweeper>{});
-  if constexpr (SLICED) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    link.publish((uint32_t)p.sl_nbb);
-    bool broken = link.broken();
-    if constexpr (NH > 0) {   // only the waves that wait know: they tell the others (the staging buffers are free now)
-      if ((int)threadIdx.x == link.pub) *reinterpret_cast<volatile uint32_t*>(lds) = broken ? 1u : 0u;
-      __syncthreads();
-      broken = *reinterpret_cast<volatile uint32_t*>(lds) != 0u;
-    }
-    if (WRITE_Y && broken) poison_band<T>(p, my_band, b, e_wg0, CW, p.y, nullptr, nullptr);
-  }
-}
+#include "m2dsplit.h"   // forward and backward for few images: the states of a channel split over lanes
 
 // ----------------------------------------------------------------------------------- backward
 // Channel sums by lane-swap butterflies.  The wave holds 4 channel slots; for a group of 4 states
@@ -2708,373 +2411,6 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
   }
 }
 
-// ------------------------------------------------------ backward, the states of a channel split over lanes
-// The counterpart of m2d_fwd_split_kernel: lane = (state group g, row r), 4 states per lane, a wave
-// per channel, 8 channels per workgroup.  With only 4 states a lane keeps the gates of all four
-// steps of a block from the recomputation to the adjoint, and sweeps a block in one pass.  Sums over
-// the states of a cell (for d_delta and d_x) are taken across the 4 lane groups by lane swaps; sums
-// over channels (d_C, d_BT, d_BL) across the 8 waves through LDS, as in m2d_bwd_kernel, a float4 of
-// four states per lane.  Memory formats are those of m2d_bwd_kernel.
-template <typename T, bool STAGE_X, int MODE, int NWS = kSplitWaves>
-__global__ __launch_bounds__((NWS + split_helpers<MODE, NWS, STAGE_X>()) * 64) void m2d_bwd_split_kernel(const ScanParams pin) {
-  static_assert(MODE != kModeStacked, "stacked images are many: they never need the split");
-  constexpr bool SLICED = MODE == kModeSliced;
-  const ScanParams& p = pin;
-  __builtin_assume(p.stacked == 0);
-  __builtin_assume(p.rb == kRB);
-  __builtin_assume(p.S >= kHB + kCK - 1);
-  constexpr int NW = NWS, CW = NW;
-  constexpr int NH = split_helpers<MODE, NWS, STAGE_X>();   // waves that only stage and add up the channel sums (then the first NW waves only sweep)
-  constexpr int NSTG = NH ? NH : NW;               // waves that share the copies of a block
-  static_assert(NH == 0 || NH >= 3, "three waves add up the channel sums");
-  constexpr int SLOT = 3 * 64;           // float4s per wave in one exchange buffer
-  using SG = Stage<T, 4, CW, true>;
-  constexpr bool WIDEN = sizeof(T) == 2;
-  extern __shared__ float4 smem[];
-  float4* slots = smem;                                            // [2][wave][3][64], used alternately: one barrier per step
-  char* lds = reinterpret_cast<char*>(slots + 2 * NW * SLOT);      // two staging buffers
-  char* raw = lds + 2 * SG::kBytes;                                // [2][kRawBytes]
-  const bool direct = WIDEN && p.bc_direct != 0;   // (uniform)
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int lb = SLICED ? (int)blockIdx.x : logical_block(p.nwg);
-  int m_lo = 0, m_hi = p.nblk;
-  int my_band = 0;
-  LinkT<NH ? NW * 64 : 0> link;
-  if constexpr (SLICED) {   // the window of one band; the bands are launched from the last to the first
-    const int per = p.B * p.bpb;
-    const int kk = lb / per;
-    lb -= kk * per;
-    my_band = p.nbands - 1 - kk;
-    m_lo = my_band * p.sl_nbb;
-    m_hi = m_lo + p.sl_nbb;
-    link.mine = p.prog + ((int64_t)my_band * per + lb) * kLinkStride;
-    link.dep = my_band + 1 < p.nbands ? link.mine + per * kLinkStride : nullptr;
-    link.err = p.link_err;
-    link.rig(p, my_band);
-  }
-  const bool helper = NH && wave >= NW;      // (uniform) stages and adds up, never sweeps
-  const bool stages = !NH || helper;
-  const int swave = NH ? wave - NW : wave;   // the wave's turn among those that stage
-  const int b = lb / p.bpb;
-  const int eg = lb % p.bpb;
-  const int e_wg0 = eg * CW;
-  const int g = lane >> kHBShift, r = lane & (kHB - 1);
-  const int rbands = row_bands(p, r);
-  const int ch_loc = helper ? 0 : wave;
-  const bool ch_ok = !helper && e_wg0 + ch_loc < p.E;   // (uniform)
-  const int e = ch_ok ? e_wg0 + ch_loc : p.E - 1;
-  for (int i = threadIdx.x; i < 2 * SG::kBytes / 16; i += (NW + NH) * 64) reinterpret_cast<float4*>(lds)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  // register w of the lane meets position 4g + w of a record: state perm(w) * 4 + g (fold order)
-  int state_of[4];
-  float a2t[4], a2l[4];
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    state_of[w] = (w == 1 ? 2 : (w == 2 ? 1 : w)) * 4 + g;
-    a2t[w] = p.A2T[e * kN + state_of[w]];
-    a2l[w] = p.A2L[e * kN + state_of[w]];
-  }
-  const float dsk = p.Df[e];
-  settle_loads();
-
-  const T* X = static_cast<const T*>(p.x);
-  const T* DT = static_cast<const T*>(p.dT);
-  const T* DL = static_cast<const T*>(p.dL);
-  const T* DY = static_cast<const T*>(p.dy);
-  const int64_t img_cell0 = (int64_t)b * p.Hs * p.W;
-  const int64_t img_bytes = img_cell0 * p.E * (int64_t)sizeof(T);
-  const char* Ximg = reinterpret_cast<const char*>(X) + img_bytes;
-  const char* DTimg = reinterpret_cast<const char*>(DT) + img_bytes;
-  const char* DLimg = reinterpret_cast<const char*>(DL) + img_bytes;
-  const char* DYimg = reinterpret_cast<const char*>(DY) + img_bytes;
-  // the three per-cell results are stored by three of the four lane groups: group 0 d_deltaT, 2 d_deltaL, 1 d_x
-  char* OUTimg = (g == 0 ? static_cast<char*>(p.ddT) : (g == 2 ? static_cast<char*>(p.ddL) : static_cast<char*>(p.dx))) + img_bytes;
-  char* BOTimg = reinterpret_cast<char*>(p.bot + (int64_t)b * p.W * p.E * kN);   // + band * bot_stride
-  char* PARTimg = reinterpret_cast<char*>(p.part + ((int64_t)eg * p.Ptot + img_cell0) * (3 * kN));
-
-  float accAT[4], accAL[4], accD = 0.f, muT[4], muL[4];
-#pragma unroll
-  for (int w = 0; w < 4; ++w) { accAT[w] = 0.f; accAL[w] = 0.f; muT[w] = 0.f; muL[w] = 0.f; }
-  // the lane's group of (B_T, B_L, C): a grid row reads those of its cell; the upper ghost (lane 0) the row
-  // above as its B_T; the lower ghost (lane 15) the row of mu_T below as its C (see m2d_bwd_kernel)
-  const uint32_t rec_off = (r == 0 ? SG::top_off(ch_loc) : (r == kHB - 1 ? SG::bot_off(ch_loc) - SG::kCOff : r * 16)) + g * SG::kPlane;
-  const uint32_t const_off = SG::kConstPlane * SG::kPlane + r * 16;
-  const uint32_t xd_off = SG::kXOff + SG::x_off(r, ch_loc + (CW < SG::kElem ? e_wg0 & (SG::kElem - 1) : 0));   // (4 channels of a 16-bit tensor: their half of the chunk)
-  constexpr uint32_t kXK = SG::kXStepBytes;
-  // channel sums: the first 6 waves add up; wave 2v + c takes components 2c, 2c+1 of every lane's float4 of
-  // tensor v.  They are kept per cell as [C, B_T, B_L][16] in the natural order of the states.
-  // (workgroups of 4 waves: the first 3 add up, a whole float4 each)
-  // (with waves that only stage: the first 3 of those, a whole float4 each)
-  constexpr bool QUADS = NH > 0 || NW < 6;
-  const bool f_on = NH ? (helper && swave < 3) : wave < (QUADS ? 3 : 6);
-  const int f_v = QUADS ? swave : wave >> 1, f_c = QUADS ? 0 : wave & 1;
-  const uint32_t f_sub0 = (uint32_t)(f_v * kN + (f_c ? 1 : 0) * 4 + g) * (uint32_t)sizeof(float);   // component 2c: state perm(2c) * 4 + g, perm = (0, 2, 1, 3)
-  const uint32_t f_sub1 = (uint32_t)(f_v * kN + (f_c ? 3 : 2) * 4 + g) * (uint32_t)sizeof(float);   // component 2c + 1
-  const float g1 = r == 0 ? 1.f : 0.f;
-  const float gb1 = r == kHB - 1 ? 1.f : 0.f;
-  const uint32_t estep = (uint32_t)(p.flip ? -p.E : p.E) * (uint32_t)sizeof(T);
-  const uint32_t wrap_adj = (uint32_t)(p.rb * p.W - p.S) * estep;
-  const uint32_t pstep = (uint32_t)(p.flip ? -1 : 1) * (uint32_t)(3 * kN * sizeof(float));
-  const uint32_t pwrap_adj = (uint32_t)(p.rb * p.W - p.S) * pstep;
-
-  BlockPos bp;
-  uint32_t cell_off0 = 0, f_off0 = 0;
-  typename Snap<T>::quad cknext = Snap<T>::zero();
-  auto load_ckpt = [&](int mm, bool take) {   // take: the forward kept the lane's state before block mm
-    cknext = Snap<T>::zero();
-    if (mm != 0 && take) {
-      int ln = lane;
-      asm volatile("" : "+v"(ln));   // the lane's place is worked out here, not carried in a register across the block (the kernel has none to spare)
-      cknext = *(snapshot_at<T>(p, b, mm, e, p.nblk) + snap_lane(ln & (kHB - 1)) + snap_quad(ln >> kHBShift));
-    }   // (this kernel: a snapshot for every block)
-  };
-  auto pos_before = [&](Pos Q) {
-    Q.col -= kCK;
-    if (Q.col < 0) { Q.col += p.S; Q.bnd -= 1; }
-    return Q;
-  };
-
-  Pos A = pos_of(p, (m_hi - 1) * kCK - (kHB - 1));
-  __syncthreads();   // the zeros are in place before the first copies land on them
-  bp = block_pos(p, A, r, rbands);
-  int cell0 = cell_of(p, bp.bnd0, r, bp.col0);
-  bool ck_take = snapshot_lane(p, Pos{bp.bnd0, bp.col0}, r, ch_ok);
-  load_ckpt(m_hi - 1, ck_take);
-  if constexpr (SLICED) { if (stages) link.wait_for(link_need_bwd(p.sl_nbb - 1, p.sl_nbb)); }
-  auto raw_copy_for = [&](Pos A2, char* dst, bool live) {
-    if (!stages) return;   // (uniform)
-    const BlockPos q2 = block_pos(p, A2, r, rbands);
-    bc_raw_copy<NSTG>(p, pin.bcd, dst, b, q2, cell_of(p, q2.bnd0, r, q2.col0), swave, lane, live);
-  };
-  int rp = 0;
-  if (direct) {
-    if (stages) bc_raw_copy<NSTG>(p, pin.bcd, raw, b, bp, cell0, swave, lane, true);
-    raw_copy_for(pos_before(A), raw + kRawBytes, m_hi - 2 >= m_lo);
-    if (stages) stage_block<T, 4, CW, true, STAGE_X, NSTG, true>(p, lds, b, A, bp, cell0, e_wg0, swave, lane, X, DT, DL, DY);
-    staging_fence();
-    if (stages) bc_widen<SG, NSTG>(raw, lds, swave, lane);
-  } else {
-    if (stages) stage_block<T, 4, CW, true, STAGE_X, NSTG>(p, lds, b, A, bp, cell0, e_wg0, swave, lane, X, DT, DL, DY);
-  }
-  staging_fence();
-  int cur = 0;
-  int xpar = 0;
-
-  // The sweep over the blocks of the window, as a wave of the given role runs it (see m2d_fwd_split_kernel); the
-  // waves that stage also add up the channel sums of every step.
-  auto sweep = [&](auto role) {
-  constexpr int ROLE = decltype(role)::value;
-  constexpr bool STAGES = ROLE != kSweeper, SWEEPS = ROLE != kStager;
-  for (int m = m_hi - 1; m >= m_lo; --m) {
-    const int t0 = m * kCK;
-    const char* bufc = lds + cur * SG::kBytes;
-    float hb[kCK + 1][4], gT[kCK][4], gL[kCK][4];
-    if constexpr (SWEEPS) { const float4 v = Snap<T>::widen(cknext); hb[0][0] = v.x; hb[0][1] = v.y; hb[0][2] = v.z; hb[0][3] = v.w; }
-    const Pos Aprev = pos_before(A);
-    const BlockPos bpn = block_pos(p, Aprev, r, rbands);
-    const int celln = cell_of(p, bpn.bnd0, r, bpn.col0);
-    if constexpr (SWEEPS) ck_take = snapshot_lane(p, Pos{bpn.bnd0, bpn.col0}, r, ch_ok);
-    if constexpr (STAGES) { if (direct) raw_copy_for(pos_before(Aprev), raw + rp * kRawBytes, m - 2 >= m_lo); }
-    if (STAGES && m > m_lo) {
-      if constexpr (SLICED) link.wait_for(link_need_bwd(m - 1 - m_lo, p.sl_nbb));
-      if (direct) {
-        stage_block<T, 4, CW, true, STAGE_X, NSTG, true>(p, lds + (cur ^ 1) * SG::kBytes, b, Aprev, bpn, celln, e_wg0, swave, lane, X, DT, DL, DY);
-        bc_widen<SG, NSTG>(raw + (rp ^ 1) * kRawBytes, lds + (cur ^ 1) * SG::kBytes, swave, lane);
-      } else {
-        stage_block<T, 4, CW, true, STAGE_X, NSTG>(p, lds + (cur ^ 1) * SG::kBytes, b, Aprev, bpn, celln, e_wg0, swave, lane, X, DT, DL, DY);
-      }
-    }
-    rp ^= 1;
-    if constexpr (SWEEPS) cell_off0 = (uint32_t)(cell0 * p.E + e) * (uint32_t)sizeof(T);
-    if constexpr (STAGES) f_off0 = (uint32_t)cell0 * (uint32_t)(3 * kN * sizeof(float));
-
-    // ---- recompute the states of the block, keeping the gates
-    if constexpr (SWEEPS)
-#pragma unroll
-    for (int k = 0; k < kCK; ++k) {
-      if (t0 + k < p.T_total) {
-        const float4 kk = *reinterpret_cast<const float4*>(bufc + const_off + k * SG::kKStr);
-        const float offT = kk.x, offL = kk.y, cT = kk.z, cL = kk.w;
-        float xv = 0.f, dtv = 0.f, dlv = 0.f;
-        if constexpr (STAGE_X) {
-          const T* xr = reinterpret_cast<const T*>(bufc + xd_off + k * kXK);
-          xv = IO<T>::ld(xr); dtv = IO<T>::ld(xr + SG::kXTauBytes / sizeof(T)); dlv = IO<T>::ld(xr + 2 * SG::kXTauBytes / sizeof(T));
-        } else if (ch_ok && ((bp.in_grid >> k) & 1u)) {
-          const uint32_t off = cell_off0 + (uint32_t)k * estep + (k >= bp.kw ? wrap_adj : 0u);
-          xv = IO<T>::ld(reinterpret_cast<const T*>(Ximg + off));
-          dtv = IO<T>::ld(reinterpret_cast<const T*>(DTimg + off));
-          dlv = IO<T>::ld(reinterpret_cast<const T*>(DLimg + off));
-        }
-        const char* rec = bufc + (rec_off + k * SG::kKStr);
-        const float4 b4 = *reinterpret_cast<const float4*>(rec);
-        const float4 l4 = *reinterpret_cast<const float4*>(rec + SG::kBLOff);
-        const float bq[4] = {b4.x, b4.y, b4.z, b4.w}, lq[4] = {l4.x, l4.y, l4.z, l4.w};
-        const float sT = __builtin_fmaf(cT * dtv, xv, g1);
-        const float sL = cL * dlv * xv;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) gT[k][w] = fexp2(__builtin_fmaf(dtv, a2t[w], offT));
-        pin4(gT[k]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) gL[k][w] = fexp2(__builtin_fmaf(dlv, a2l[w], offL));
-        pin4(gL[k]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          float u = sL * lq[w];
-          u = __builtin_fmaf(sT, bq[w], u);
-          u = fma_row_below(gT[k][w], hb[k][w], u);
-          hb[k + 1][w] = __builtin_fmaf(gL[k][w], hb[k][w], u);
-        }
-      } else {
-#pragma unroll
-        for (int w = 0; w < 4; ++w) { gT[k][w] = 0.f; gL[k][w] = 0.f; hb[k + 1][w] = 0.f; }
-      }
-    }
-    // ---- adjoint over the block, last step first
-#pragma unroll
-    for (int k = kCK - 1; k >= 0; --k) {
-      if (k == 0) staging_landed();   // before the last stores of the block
-      if constexpr (SWEEPS) { if (k == (kCK > 1 ? 1 : 0) && m > m_lo) load_ckpt(m - 1, ck_take); }
-      if (t0 + k < p.T_total) {
-       if constexpr (SWEEPS) {
-        const float4 kk = *reinterpret_cast<const float4*>(bufc + const_off + k * SG::kKStr);
-        const float cT = kk.z, cL = kk.w;
-        const bool inr = ch_ok && ((bp.in_grid >> k) & 1u);
-        const uint32_t goff = cell_off0 + (uint32_t)k * estep + (k >= bp.kw ? wrap_adj : 0u);
-        float xv = 0.f, dtv = 0.f, dlv = 0.f, dyv = 0.f;
-        if constexpr (STAGE_X) {
-          const T* xr = reinterpret_cast<const T*>(bufc + xd_off + k * kXK);
-          xv = IO<T>::ld(xr); dtv = IO<T>::ld(xr + SG::kXTauBytes / sizeof(T)); dlv = IO<T>::ld(xr + 2 * SG::kXTauBytes / sizeof(T));
-          dyv = IO<T>::ld(xr + 3 * SG::kXTauBytes / sizeof(T));
-        } else if (inr) {
-          xv = IO<T>::ld(reinterpret_cast<const T*>(Ximg + goff));
-          dtv = IO<T>::ld(reinterpret_cast<const T*>(DTimg + goff));
-          dlv = IO<T>::ld(reinterpret_cast<const T*>(DLimg + goff));
-          dyv = IO<T>::ld(reinterpret_cast<const T*>(DYimg + goff));
-        }
-        const char* rec = bufc + (rec_off + k * SG::kKStr);
-        const float4 b4 = *reinterpret_cast<const float4*>(rec);
-        const float4 l4 = *reinterpret_cast<const float4*>(rec + SG::kBLOff);
-        const float4 c4 = *reinterpret_cast<const float4*>(rec + SG::kCOff);
-        const float bq[4] = {b4.x, b4.y, b4.z, b4.w}, lq[4] = {l4.x, l4.y, l4.z, l4.w}, cq[4] = {c4.x, c4.y, c4.z, c4.w};
-        const float qT = cT * dtv * xv, qL = cL * dlv * xv;   // zero on lanes that are not grid cells
-        const float dyl = dyv + gb1;
-        float sT = 0.f, sL = 0.f, zT = 0.f, zL = 0.f;
-        float vC[4], vBT[4], vBL[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const float lam = __builtin_fmaf(dyl, cq[w], add_row_above(muL[w], muT[w]));
-          const float mT = gT[k][w] * lam, mL = gL[k][w] * lam;
-          muT[w] = mT;
-          muL[w] = mL;
-          const float ZT = mul_row_below(mT, hb[k][w]), ZL = mL * hb[k][w];
-          accAT[w] = __builtin_fmaf(ZT, dtv, accAT[w]);
-          accAL[w] = __builtin_fmaf(ZL, dlv, accAL[w]);
-          zT = __builtin_fmaf(ZT, a2t[w], zT);
-          zL = __builtin_fmaf(ZL, a2l[w], zL);
-          sT = __builtin_fmaf(lam, bq[w], sT);
-          sL = __builtin_fmaf(lam, lq[w], sL);
-          vBT[w] = qT * lam;
-          vBL[w] = qL * lam;
-          vC[w] = dyv * hb[k + 1][w];
-        }
-        float4* sw = slots + (xpar * NW + wave) * SLOT + lane;
-        sw[0] = make_float4(vC[0], vC[1], vC[2], vC[3]);
-        sw[64] = make_float4(vBT[0], vBT[1], vBT[2], vBT[3]);
-        sw[128] = make_float4(vBL[0], vBL[1], vBL[2], vBL[3]);
-        if (p.nbands > 1) {   // first row of a band: the lower ghost of the band above will replay its muT
-          const bool wk = k >= bp.kw;
-          if (inr && r == 1 && (wk ? bp.bnd0 + 1 : bp.bnd0) >= 1) {
-            const int ck = wk ? bp.col0 + k - p.S : bp.col0 + k;
-            float4* bb = reinterpret_cast<float4*>(BOTimg + (wk ? bp.bnd0 + 1 : bp.bnd0) * p.bot_stride * (int64_t)sizeof(float) +
-                                                   (uint32_t)(ck * p.E + e) * (uint32_t)(kN * sizeof(float))) + g;
-            const float4 row = make_float4(muT[0], muT[1], muT[2], muT[3]);
-            if constexpr (SLICED) store_row_device_scope(bb, row); else *bb = row;
-          }
-        }
-        // the lane's share (its 4 states) of d_deltaT, d_deltaL and d_x of the cell; summed over the 4
-        // groups, the totals arrive in the lanes of group 0, 2 and 1
-        const float pT = __builtin_fmaf(cT * xv, sT, kLn2 * zT);
-        const float pL = __builtin_fmaf(cL * xv, sL, kLn2 * zL);
-        const float pX = __builtin_fmaf(cT * dtv, sT, cL * dlv * sL);
-        float tot = fold16(fold32(pT, pL), fold32(pX, 0.f));
-        accD = __builtin_fmaf(dyv, xv, accD);
-        if (p.dpre && (g & 1) == 0) tot *= softplus_slope<T>(g == 0 ? dtv : dlv);   // gradients with respect to what the softplus was applied to
-        if (g == 1) tot = __builtin_fmaf(dyv, dsk, tot);
-        if (inr && g != 3) IO<T>::st(reinterpret_cast<T*>(OUTimg + goff), tot);
-       }
-        // ---- across the waves of the workgroup
-        __syncthreads();
-        if (STAGES && f_on && ((bp.in_grid >> k) & 1u)) {
-          const uint32_t off = f_off0 + (uint32_t)k * pstep + (k >= bp.kw ? pwrap_adj : 0u);
-          if constexpr (QUADS) {
-            const float4* sl = slots + xpar * NW * SLOT + f_v * 64 + lane;
-            float4 sum = sl[0];
-#pragma unroll
-            for (int w = 1; w < NW; ++w) { const float4 o = sl[w * SLOT]; sum.x += o.x; sum.y += o.y; sum.z += o.z; sum.w += o.w; }
-            // component j holds state perm(j) * 4 + g, perm = (0, 2, 1, 3)
-            float* dst = reinterpret_cast<float*>(PARTimg + off + (uint32_t)(f_v * kN + g) * (uint32_t)sizeof(float));
-            dst[0] = sum.x; dst[8] = sum.y; dst[4] = sum.z; dst[12] = sum.w;
-          } else {
-            const float2* sl = reinterpret_cast<const float2*>(slots + xpar * NW * SLOT + f_v * 64 + lane) + f_c;
-            float2 sum = sl[0];
-#pragma unroll
-            for (int w = 1; w < NW; ++w) { sum.x += sl[2 * w * SLOT].x; sum.y += sl[2 * w * SLOT].y; }
-            *reinterpret_cast<float*>(PARTimg + off + f_sub0) = sum.x;
-            *reinterpret_cast<float*>(PARTimg + off + f_sub1) = sum.y;
-          }
-        }
-        xpar ^= 1;
-      }
-    }
-    __syncthreads();
-    if constexpr (SLICED && STAGES) link.publish((uint32_t)(m_hi - m));   // (this block counts: see m2d_bwd_kernel)
-    A = Aprev;
-    bp = bpn;
-    cell0 = celln;
-    cur ^= 1;
-  }
-  };
-  if constexpr (NH == 0) sweep(std::integral_constant<int, kAll>{});
-  else if (helper) sweep(std::integral_constant<int, kStager>{});
-  else sweep(std::integral_constant<int, kSweeper>{});
-  bool broken = false;
-  if constexpr (SLICED) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    link.publish((uint32_t)p.sl_nbb);
-    broken = link.broken() || link_poll(p.link_err) != 0u;   // (also a workgroup of the forward sweep that rebuilt the snapshots for this launch)
-    if constexpr (NH > 0) {   // only the waves that wait know of a wait given up: they tell the others (the staging buffers are free now)
-      if ((int)threadIdx.x == link.pub) *reinterpret_cast<volatile uint32_t*>(lds) = link.broken() ? 1u : 0u;
-      __syncthreads();
-      broken = broken || *reinterpret_cast<volatile uint32_t*>(lds) != 0u;
-    }
-    if (broken) poison_band<T>(p, my_band, b, e_wg0, CW, p.dx, p.ddT, p.ddL);
-  }
-
-  // ---- sums over positions: reduce over the rows of the band (the 16 lanes of a group)
-  float red[9];
-#pragma unroll
-  for (int w = 0; w < 4; ++w) { red[w] = accAT[w]; red[4 + w] = accAL[w]; }
-  red[8] = broken ? __builtin_nanf("") : accD;
-  if (broken) { red[0] = __builtin_nanf(""); red[4] = __builtin_nanf(""); }   // (d_AT, d_AL, d_D of the channel say so too)
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    float v = red[k];
-#pragma unroll
-    for (int off = kHB >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    red[k] = v;
-  }
-  if (ch_ok && r == 0) {
-    const int64_t slot_e = ((int64_t)b * p.pa_slots + (SLICED ? my_band : 0)) * p.E + e;
-    float* pa = p.pA + slot_e * (2 * kN);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) { pa[state_of[w]] = red[w]; pa[kN + state_of[w]] = red[4 + w]; }
-    if (g == 0) p.pD[slot_e] = red[8];
-  }
-}
-
 // -------------------------------------------------------------------------- small helper kernels
 template <typename T>
 __global__ void m2d_prep_kernel(const ScanParams p, float* zeros, float* A2T, float* A2L, float* Df, uint32_t* link_words, int n_link_words) {
@@ -3416,7 +2752,7 @@ Geometry make_geometry(const m2d_desc* d) {
   // Workgroups of 8 waves (8 channels) under way on at most half of the compute units: workgroups of 4 then run on
   // twice as many, each wave with a SIMD to itself (a sweep of few images is as fast as one wave gets through its
   // blocks).
-  // Both sizes of workgroup have 4 more waves that stage for them (split_helpers).  In the linked sweep workgroups of
+  // Both sizes of workgroup have 4 more waves that stage for them (kSplitStagers).  In the linked sweep workgroups of
   // 4 stay ahead up to 7 of them under way for every 5 units (measured, E=64 fp32, forward+backward kernels with
   // workgroups of 4 against 8: 384x384 1.65 against 1.86 ms, 512x512 2.56 against 2.61, 640x640 3.63 against 3.29,
   // 768x768 5.08 against 4.10).
@@ -3571,12 +2907,12 @@ int stage_bc(ScanParams& sp, const m2d_desc* d, const void* BT, const void* BL, 
 }
 
 // Development aid: -DM2D_QUICK=1 builds only the kernels of many 16-bit images in one stream each, in workgroups of
-// 8 waves (a twentieth of the compile time), -DM2D_QUICK=2 (3) only the linked sweep of fp32 (16-bit) images in workgroups of 4 waves;
+// 8 waves (a twentieth of the compile time), -DM2D_QUICK=2 (3) only the linked sweep of fp32 (16-bit) images in workgroups of 4 waves, =4 (5) one stream per 16-bit (fp32) image in those;
 // every other problem then answers M2D_ERR_UNSUPPORTED.
 #if defined(M2D_QUICK) && M2D_QUICK >= 2 && M2D_QUICK <= 3
 #define M2D_BUILT(T, SX, MODE, NW, OTHER) (sizeof(T) == (M2D_QUICK == 3 ? 2 : 4) && (MODE) == kModeSliced && (NW) == 4)
 #elif defined(M2D_QUICK)
-#define M2D_BUILT(T, SX, MODE, NW, OTHER) (sizeof(T) == 2 && (SX) && (MODE) == kModeSweep && (NW) == (M2D_QUICK == 1 ? 8 : 4) && (OTHER))
+#define M2D_BUILT(T, SX, MODE, NW, OTHER) (sizeof(T) == (M2D_QUICK == 5 ? 4 : 2) && (SX) && (MODE) == kModeSweep && (NW) == (M2D_QUICK == 1 ? 8 : 4) && ((OTHER) || M2D_QUICK > 3))
 #else
 #define M2D_BUILT(T, SX, MODE, NW, OTHER) true
 #endif
@@ -3593,16 +2929,14 @@ int launch_fwd_as(const ScanParams& sp, hipStream_t st) {
   }
 }
 
-template <typename T, int NWS = kSplitWaves>
-constexpr size_t fwd_split_lds_bytes() { return 2 * (size_t)Stage<T, 3, NWS, false>::kBytes + (sizeof(T) == 2 ? 2 * kRawBytes : 0); }
 template <typename T, bool CK, bool WY, bool SX, int MODE, int NWS = kSplitWaves>
 int launch_fwd_split_as(const ScanParams& sp, hipStream_t st) {
   if constexpr (!M2D_BUILT(T, SX, MODE, NWS, false)) return M2D_ERR_UNSUPPORTED; else {
-  constexpr size_t lds = fwd_split_lds_bytes<T, NWS>();
+  constexpr size_t lds = SplitFwdLds<T, NWS, SX>::kBytes;
   static_assert(lds <= kLdsPerWorkgroup, "staging must fit the LDS");
   static std::atomic<uint64_t> seen{0};
   if (!allow_dynamic_lds(reinterpret_cast<const void*>(&m2d_fwd_split_kernel<T, CK, WY, SX, MODE, NWS>), lds, seen)) return M2D_ERR_HIP;
-  hipLaunchKernelGGL((m2d_fwd_split_kernel<T, CK, WY, SX, MODE, NWS>), dim3((unsigned)sp.nwg), dim3((NWS + split_helpers<MODE, NWS, SX>()) * 64), lds, st, sp);
+  hipLaunchKernelGGL((m2d_fwd_split_kernel<T, CK, WY, SX, MODE, NWS>), dim3((unsigned)sp.nwg), dim3((NWS + kSplitStagers) * 64), lds, st, sp);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
   }
 }
@@ -3743,18 +3077,14 @@ int launch_bwd2_as(const ScanParams& sp, hipStream_t st) {
   }
 }
 
-template <typename T, int NWS = kSplitWaves>
-constexpr size_t bwd_split_lds_bytes() {
-  return sizeof(float4) * 2 * NWS * 3 * 64 + 2 * (size_t)Stage<T, 4, NWS, true>::kBytes + (sizeof(T) == 2 ? 2 * kRawBytes : 0);
-}
 template <typename T, bool SX, int MODE, int NWS = kSplitWaves>
 int launch_bwd_split_as(const ScanParams& sp, hipStream_t st) {
   if constexpr (!M2D_BUILT(T, SX, MODE, NWS, false)) return M2D_ERR_UNSUPPORTED; else {
-  constexpr size_t lds = bwd_split_lds_bytes<T, NWS>();
+  constexpr size_t lds = SplitBwdLds<T, NWS, SX>::kBytes;
   static_assert(lds <= kLdsPerWorkgroup, "exchange buffers and staging must fit the LDS");
   static std::atomic<uint64_t> seen{0};
   if (!allow_dynamic_lds(reinterpret_cast<const void*>(&m2d_bwd_split_kernel<T, SX, MODE, NWS>), lds, seen)) return M2D_ERR_HIP;
-  hipLaunchKernelGGL((m2d_bwd_split_kernel<T, SX, MODE, NWS>), dim3((unsigned)sp.nwg), dim3((NWS + split_helpers<MODE, NWS, SX>()) * 64), lds, st, sp);
+  hipLaunchKernelGGL((m2d_bwd_split_kernel<T, SX, MODE, NWS>), dim3((unsigned)sp.nwg), dim3((NWS + kSplitStagers) * 64), lds, st, sp);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
   }
 }
@@ -3967,11 +3297,9 @@ int m2d_scan_plan(const m2d_desc* desc, int pass, char* text, size_t cap) {
   else if (g.stacked) snprintf(sched, sizeof sched, "stacked images, %d per stream, %d bands", g.ips, g.nbands);
   else snprintf(sched, sizeof sched, "one stream per image, %d band%s back to back", g.nbands, g.nbands == 1 ? "" : "s");
   if (split) {
-    const int helpers = (nw == kSplitHalfWaves ? split_helpers<kModeSliced, kSplitHalfWaves>() : g.stage_x ? split_helpers<kModeSliced, kSplitWaves, true>() : split_helpers<kModeSliced, kSplitWaves, false>());
-    char extra[48] = "";
-    if (helpers) snprintf(extra, sizeof extra, " and %d that stage", helpers);
-    snprintf(text, cap, "%s: %s, %lld workgroups of %d waves%s, %d channels each, 4 states per lane",
-             fwd ? "m2d_fwd_split_kernel" : "m2d_bwd_split_kernel", sched, wgs, nw, extra, nw);
+    const bool values = nw == kSplitWaves && !g.stage_x;   // rows that are no whole chunks: x and the step sizes go through registers, value by value
+    snprintf(text, cap, "%s: %s, %lld workgroups of %d waves%s, %d channels each, 4 states per lane%s",
+             fwd ? "m2d_fwd_split_kernel" : "m2d_bwd_split_kernel", sched, wgs, nw, values ? "" : " and 4 that stage", nw, values ? ", and 4 more waves that stage value by value" : "");
   }
   else {
     // (workgroups of 4 waves have waves that only stage, except in the backward that replays the forward between snapshots)
