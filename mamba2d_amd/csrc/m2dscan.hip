@@ -2696,89 +2696,118 @@ Geometry make_geometry(const m2d_desc* d) {
   // Few images with many bands leave most of the device idle when each image is one sequential
   // stream.  Then every band gets workgroups of its own (a padded stream, one window of S steps
   // per band), all in one launch, and band k trails band k-1 by kLinkLag blocks of steps.
+  const int nblk_stream = g.nblk;
+  const int s_link = (d->W + kHB - 1 + kCK - 1) / kCK * kCK;
+  const int nbb_link = (s_link < 28 ? 28 : s_link) / kCK;
+  const int64_t lagged = (nbb_link + kLinkLag) / (kLinkLag + 1);   // bands whose windows overlap in time (the lag and a block more for the polling)
+  auto set_schedule = [&](bool sliced) {
+    g.sliced = sliced;
+    if (!sliced) return;
+    g.nbb = nbb_link;
+    g.S = nbb_link * kCK;
+    g.T_total = g.nbands * g.S;
+    g.nblk = g.nbands * g.nbb;
+  };
+  g.nbb = 0;
+  // For kernels whose lanes hold all 16 states of a channel:
   // (two or three bands: only where a band is much longer than the 28 steps by which a band trails its neighbour)
-  g.sliced = !g.stacked && (g.nbands >= 4 || (g.nbands >= 2 && d->W >= 64)) && (int64_t)B * groups <= ncu / 4;
-  if (g.sliced && g.nbands == 4) {
+  bool link_whole = !g.stacked && (g.nbands >= 4 || (g.nbands >= 2 && d->W >= 64)) && (int64_t)B * groups <= ncu / 4;
+  if (link_whole && g.nbands == 4) {
     // Four bands (more bands favour the linked sweep again: 84x84 measured) and a batch that fills half the device with workgroups of 4 waves, but not with
     // every band under way on workgroups of its own: one stream per image on workgroups of 4 waves
     // is then the faster schedule (56x56, 64 images of 32 channels: 0.99 -> 0.93 ms forward+backward).
-    int s_sl = (d->W + kHB - 1 + kCK - 1) / kCK * kCK;
-    if (s_sl < 28) s_sl = 28;
-    const int64_t lagged = (s_sl / kCK + kLinkLag) / (kLinkLag + 1);   // bands whose windows overlap in time (a block more for the polling)
     const int64_t under_way = lagged < g.nbands ? lagged : g.nbands;
     const int64_t half = (int64_t)B * ((d->E + kFwdHalfWaves * g.CS - 1) / (kFwdHalfWaves * g.CS));
-    if (half > (int64_t)B * groups && half <= ncu && half >= ncu / 2 && half * under_way > ncu) g.sliced = false;
+    if (half > (int64_t)B * groups && half <= ncu && half >= ncu / 2 && half * under_way > ncu) link_whole = false;
   }
-  g.nbb = 0;
-  if (g.sliced) {
-    g.S = (d->W + kHB - 1 + kCK - 1) / kCK * kCK;
-    if (g.S < 28) g.S = 28;
-    g.nbb = g.S / kCK;
-    g.T_total = g.nbands * g.S;
-    g.nblk = g.nbands * g.nbb;
-  }
-  // forward: two channels per lane where that saves rounds of workgroups (one workgroup per compute
-  // unit at a time, 256 units) and the two staging buffers of such a workgroup fit the LDS (bf16
-  // operands only).  A sweep with two channels per lane takes about 1.8 times
-  // as long as one with a single channel (measured: 1.6 at 28x28, 2.0 at 56x56), so it pays only
-  // when it at least halves the rounds: 128 channels x 128 images, not 32 channels x 256 images
-  // (where half of every workgroup would idle).
-  // (fp32 operands: such a kernel would need more registers than a lane has, and is not built)
-  const size_t lds_ec2 = d->dtype == M2D_BF16 ? fwd_lds_bytes<bf16_t, 2>() : kLdsPerWorkgroup + 1;
-  const int64_t wg1 = (int64_t)B * ((d->E + kFwdWaves * g.CS - 1) / (kFwdWaves * g.CS));
-  const int64_t wg2 = (int64_t)B * ((d->E + kFwdWaves * g.CS * 2 - 1) / (kFwdWaves * g.CS * 2));
-  const bool ec2 = (d->E % 2 == 0) && lds_ec2 <= kLdsPerWorkgroup && 18 * ((wg2 + ncu - 1) / ncu) < 10 * ((wg1 + ncu - 1) / ncu);
-  g.fwd_ec = ec2 ? 2 : 1;
-  // forward of a small batch in one stream per image: workgroups of 4 waves (16 channels) where those
-  // are more than the workgroups of 8 and still no more than the compute units
   const int64_t wg_half = (int64_t)B * ((d->E + kFwdHalfWaves * g.CS - 1) / (kFwdHalfWaves * g.CS));
-  // (in the linked sweep the windows of about nbb / (kLinkLag + 1) bands overlap in time: the lag and a block for the polling)
-  const int64_t together = g.sliced ? ((g.nbb + kLinkLag) / (kLinkLag + 1) < g.nbands ? (g.nbb + kLinkLag) / (kLinkLag + 1) : g.nbands) : 1;
-  // (a linked sweep may exceed the units by a few workgroups while most bands are under way: its start
-  // and its end, with fewer bands, still gain)
-  const int64_t room = g.sliced ? ncu + ncu / 16 : ncu;
-  g.fwd_nw = (!g.stacked && !ec2 && wg_half > wg1 && wg_half * together <= room) ? kFwdHalfWaves : kFwdWaves;
-  g.fwd_bpb = (d->E + g.fwd_nw * g.CS * g.fwd_ec - 1) / (g.fwd_nw * g.CS * g.fwd_ec);
-  g.fwd_wpb = g.fwd_bpb * g.fwd_nw;
-  // Few waves under way (a wave per 4 channels, the bands of a linked sweep that overlap in time): fewer
-  // than three for every four SIMDs.  Then a wave per channel, each with a quarter of the states.
-  const int64_t waves_whole = (int64_t)B * ((d->E + g.CS - 1) / g.CS) * together;
-  const bool may_split = !g.stacked && !(d->flags & M2D_FLAG_WHOLE_STATES) && g.ck_shift == 0;
-  // One stream per image: only while the workgroups of 8 channels all run at once.  The backward has a compute unit to
-  // itself, so one workgroup more than units is a second round of them, and the whole-state kernels in workgroups of 4
-  // waves are then ahead (B=33..48 at 56x56x64 bf16: forward+backward kernels 0.85 -> 0.76 ms; B=32: 0.48 against 0.76).
-  const bool few_enough = waves_whole <= 3 * ncu && (g.sliced || (int64_t)B * ((d->E + kSplitWaves - 1) / kSplitWaves) <= ncu);
-  g.fwd_split = may_split && ((d->flags & M2D_FLAG_SPLIT_STATES) || few_enough);
-  // Workgroups of 8 waves (8 channels) under way on at most half of the compute units: workgroups of 4 then run on
-  // twice as many, each wave with a SIMD to itself (a sweep of few images is as fast as one wave gets through its
-  // blocks).
-  // Both sizes of workgroup have 4 more waves that stage for them (kSplitStagers).  In the linked sweep workgroups of
-  // 4 stay ahead up to 7 of them under way for every 5 units (measured, E=64 fp32, forward+backward kernels with
-  // workgroups of 4 against 8: 384x384 1.65 against 1.86 ms, 512x512 2.56 against 2.61, 640x640 3.63 against 3.29,
-  // 768x768 5.08 against 4.10).
-  const int64_t wg4 = (int64_t)B * ((d->E + kSplitHalfWaves - 1) / kSplitHalfWaves) * together;
-  // (one stream per image: workgroups of 4 only while each has a compute unit)
-  const int split_nw = (g.sliced ? 5 * wg4 <= 7 * ncu : wg4 <= ncu) ? kSplitHalfWaves : kSplitWaves;
-  if (g.fwd_split) {
+  auto set_whole = [&] {
+    // forward: two channels per lane where that saves rounds of workgroups (one workgroup per compute
+    // unit at a time, 256 units) and the two staging buffers of such a workgroup fit the LDS (bf16
+    // operands only).  A sweep with two channels per lane takes about 1.8 times
+    // as long as one with a single channel (measured: 1.6 at 28x28, 2.0 at 56x56), so it pays only
+    // when it at least halves the rounds: 128 channels x 128 images, not 32 channels x 256 images
+    // (where half of every workgroup would idle).
+    // (fp32 operands: such a kernel would need more registers than a lane has, and is not built)
+    const size_t lds_ec2 = d->dtype == M2D_BF16 ? fwd_lds_bytes<bf16_t, 2>() : kLdsPerWorkgroup + 1;
+    const int64_t wg1 = (int64_t)B * ((d->E + kFwdWaves * g.CS - 1) / (kFwdWaves * g.CS));
+    const int64_t wg2 = (int64_t)B * ((d->E + kFwdWaves * g.CS * 2 - 1) / (kFwdWaves * g.CS * 2));
+    const bool ec2 = (d->E % 2 == 0) && lds_ec2 <= kLdsPerWorkgroup && 18 * ((wg2 + ncu - 1) / ncu) < 10 * ((wg1 + ncu - 1) / ncu);
+    g.fwd_ec = ec2 ? 2 : 1;
+    // forward of a small batch in one stream per image: workgroups of 4 waves (16 channels) where those
+    // are more than the workgroups of 8 and still no more than the compute units
+    const int64_t together = g.sliced ? (lagged < g.nbands ? lagged : g.nbands) : 1;
+    // (a linked sweep may exceed the units by a few workgroups while most bands are under way: its start
+    // and its end, with fewer bands, still gain)
+    const int64_t room = g.sliced ? ncu + ncu / 16 : ncu;
+    g.fwd_nw = (!g.stacked && !ec2 && wg_half > wg1 && wg_half * together <= room) ? kFwdHalfWaves : kFwdWaves;
+    g.fwd_bpb = (d->E + g.fwd_nw * g.CS * g.fwd_ec - 1) / (g.fwd_nw * g.CS * g.fwd_ec);
+    g.fwd_wpb = g.fwd_bpb * g.fwd_nw;
+    g.bwd_nw = (!g.stacked && wg_half > (int64_t)B * groups && wg_half * together <= room) ? kFwdHalfWaves : kBwdWaves;
+    g.bwd_bpb = (d->E + g.bwd_nw * g.CS - 1) / (g.bwd_nw * g.CS);
+    g.bwd_wpb = g.bwd_bpb * g.bwd_nw;
+  };
+  set_schedule(link_whole);
+  set_whole();
+  // A wave per channel, each lane with a quarter of the states, gets through a block of steps in a third of the time, but takes four times as many
+  // waves.  Which is faster, and in which schedule, is a matter of how many workgroups follow each other on a compute unit (a backward
+  // kernel has the unit to itself) and of the chain of bands: blocks that one unit sweeps, times what a block takes.  Measured, forward keeping snapshots
+  // and backward, relative to a workgroup of 4 waves with a quarter of the states each (56x56x64 bf16, all units busy): 8 such waves
+  // 1.47, whole states 3.0 in workgroups of 4 waves (16 channels), 4.2 in workgroups of 8 (32 channels).
+  // In the linked sweep a band trails its neighbour by 6 blocks, and the shorter of the two, the chain of bands and the work per unit, hides
+  // behind the longer but for about a fifth (where units have more than one workgroup to sweep).
+  // What this rule takes from the whole states, forward + backward in ms: 30x60x50x40 fp32 0.517 -> 0.312, 8x100x120x96 bf16 0.891 -> 0.615,
+  // 8x256x256x64 bf16 3.13 -> 2.09, 20x28x28x200 fp32 0.296 -> 0.192, 40x56x56x64 bf16 0.620 -> 0.513, 2048x2048x64 fp32 forward 6.39 -> 4.82;
+  // and leaves with them: 32x128x128x64 bf16 2.00 (split 2.17), 8x512x512x64 bf16 7.6 (8.0), 64x28x28x128 bf16 0.280 (0.389).
+  // Near the line the whole states stay: fewer channel sums, and snapshots every 2 steps.
+  constexpr int64_t kSplit4 = 100, kSplit8 = 147, kWhole4 = 300, kWhole8 = 417;
+  auto stream_cost = [&](int64_t wgs, int64_t block) { return (wgs + ncu - 1) / ncu * nblk_stream * block; };
+  auto link_cost = [&](int64_t wgs, int64_t block) {
+    const int64_t work = (wgs * g.nbands + ncu - 1) / ncu * nbb_link, chain = nbb_link + (int64_t)(g.nbands - 1) * (kLinkLag - 1);
+    return (work > chain ? work + chain / 5 : chain + (work > nbb_link ? work / 5 : 0)) * block;
+  };
+  const int64_t whole_block = g.bwd_nw == kFwdHalfWaves ? kWhole4 : kWhole8;
+  const int64_t whole_cost = g.sliced ? link_cost((int64_t)B * g.bwd_bpb, whole_block) : stream_cost((int64_t)B * g.bwd_bpb, whole_block);
+  const int64_t wg4 = (int64_t)B * ((d->E + kSplitHalfWaves - 1) / kSplitHalfWaves), wg8 = (int64_t)B * ((d->E + kSplitWaves - 1) / kSplitWaves);
+  int split_nw = kSplitHalfWaves;
+  bool split_link = false;
+  int64_t split_cost = stream_cost(wg4, kSplit4);
+  if (stream_cost(wg8, kSplit8) < split_cost) { split_cost = stream_cost(wg8, kSplit8); split_nw = kSplitWaves; }
+  if (g.nbands >= 2) {
+    // Workgroups of 4 stay ahead up to 7 of them under way for every 5 units (E=64 fp32, forward+backward kernels with workgroups of 4
+    // against 8: 384x384 1.23 against 1.44 ms, 512x512 1.95 against 2.05, 640x640 2.77 against 2.67, 768x768 3.93 against 3.35): each
+    // reads B_T, B_L, C again and leaves channel sums of its own.
+    if (5 * wg4 * (lagged < g.nbands ? lagged : g.nbands) <= 7 * ncu && link_cost(wg4, kSplit4) < split_cost) { split_cost = link_cost(wg4, kSplit4); split_nw = kSplitHalfWaves; split_link = true; }
+    if (link_cost(wg8, kSplit8) < split_cost) { split_cost = link_cost(wg8, kSplit8); split_nw = kSplitWaves; split_link = true; }
+  }
+  const bool may_split = !g.stacked && !(d->flags & M2D_FLAG_WHOLE_STATES) && g.ck_shift == 0 && !g.snap32;
+  const bool split = may_split && ((d->flags & M2D_FLAG_SPLIT_STATES) || 100 * split_cost < 93 * whole_cost);
+  g.fwd_split = g.bwd_split = false;
+  if (split) {
+    if (split_link != g.sliced) {
+      g.S = (g.nbands > 1 && d->W >= 26) ? d->W : (d->W + kHB - 1 > 26 ? d->W + kHB - 1 : 26);
+      g.T_total = (g.nbands - 1) * g.S + d->W + g.rows_last;
+      g.nblk = nblk_stream;
+      g.nbb = 0;
+      set_schedule(split_link);
+      set_whole();
+    }
+    g.fwd_split = true;
     g.fwd_ec = 1;
     g.fwd_nw = split_nw;
     g.fwd_bpb = (d->E + split_nw - 1) / split_nw;
     g.fwd_wpb = g.fwd_bpb * g.fwd_nw;
-  }
-  g.bwd_nw = (!g.stacked && wg_half > (int64_t)B * groups && wg_half * together <= room) ? kFwdHalfWaves : kBwdWaves;
-  g.bwd_bpb = (d->E + g.bwd_nw * g.CS - 1) / (g.bwd_nw * g.CS);
-  g.bwd_wpb = g.bwd_bpb * g.bwd_nw;
-  // (the backward keeps one set of channel sums per workgroup of an image: with 8 channels per workgroup
-  // that memory is bounded here unless the caller insists)
-  const size_t split_part = sizeof(float) * (size_t)((d->E + split_nw - 1) / split_nw) * 3 * kN * (size_t)d->B * d->H * d->W;
-  g.bwd_split = may_split && ((d->flags & M2D_FLAG_SPLIT_STATES) || (few_enough && split_part <= ((size_t)2 << 30)));
-  if (g.bwd_split) {
-    g.bwd_nw = split_nw;
-    g.bwd_bpb = (d->E + split_nw - 1) / split_nw;
-    g.bwd_wpb = g.bwd_bpb * g.bwd_nw;
+    // (the backward keeps one set of channel sums per workgroup of an image: with 8 channels per workgroup
+    // that memory is bounded here unless the caller insists)
+    const size_t split_part = sizeof(float) * (size_t)((d->E + split_nw - 1) / split_nw) * 3 * kN * (size_t)d->B * d->H * d->W;
+    g.bwd_split = (d->flags & M2D_FLAG_SPLIT_STATES) || split_part <= ((size_t)2 << 30);
+    if (g.bwd_split) {
+      g.bwd_nw = split_nw;
+      g.bwd_bpb = (d->E + split_nw - 1) / split_nw;
+      g.bwd_wpb = g.bwd_bpb * g.bwd_nw;
+    }
   }
   if (g.snap32) {
-    g.fwd_split = g.bwd_split = false;
     g.fwd_ec = 1;
     g.fwd_nw = g.bwd_nw = kFwdHalfWaves;
     g.fwd_bpb = g.bwd_bpb = (d->E + kFwdHalfWaves * g.CS - 1) / (kFwdHalfWaves * g.CS);

@@ -21,18 +21,19 @@ CASES = [
     (2, 2, 2, 4, "one stream per image", 4),      # a single block
     (2, 3, 4, 5, "one stream per image", 4),      # two blocks
     (3, 9, 5, 9, "one stream per image", 4),      # one band, three workgroups, the last with one channel
-    (2, 28, 26, 8, "one stream per image", 4),    # two bands, the shortest stride
-    (2, 28, 27, 6, "one stream per image", 4),
-    (2, 30, 30, 8, "one stream per image", 4),    # ... the longest that is sent and read back by one wave
-    (2, 30, 31, 6, "one stream per image", 4),    # ... the shortest that is not
-    (2, 42, 32, 16, "one stream per image", 4),
+    (64, 28, 26, 16, "one stream per image", 4),  # two bands, the shortest stride
+    (40, 28, 27, 22, "one stream per image", 4),
+    (60, 30, 30, 14, "one stream per image", 4),  # ... the longest that is sent and read back by one wave
+    (60, 30, 31, 14, "one stream per image", 4),  # ... the shortest that is not
+    (50, 42, 32, 20, "one stream per image", 4),
     (40, 16, 27, 40, "one stream per image", 8),
     (40, 30, 31, 41, "one stream per image", 8),
-    (1, 57, 13, 3, "linked sweep", 4),            # windows of 28 steps
+    (1, 28, 28, 12, "linked sweep", 4),           # two bands
+    (1, 30, 70, 3, "linked sweep", 4),
     (1, 70, 50, 8, "linked sweep", 4),
-    (3, 61, 17, 30, "linked sweep", 4),
-    (8, 70, 50, 64, "linked sweep", 8),
-    (8, 60, 50, 61, "linked sweep", 8),
+    (3, 61, 17, 30, "linked sweep", 4),           # windows of 32 steps
+    (18, 70, 50, 64, "linked sweep", 8),
+    (36, 45, 40, 61, "linked sweep", 8),
 ]
 
 
