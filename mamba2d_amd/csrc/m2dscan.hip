@@ -1973,11 +1973,21 @@ __global__ __launch_bounds__((NW + (REPLAY ? 0 : whole_helpers<MODE, NW>())) * 6
 // where the snapshots weigh most).
 template <typename T, int NW>
 constexpr int bwd2_exchange_sets() {   // sets of [wave][3][64] float2: 2 halves x 2 steps where they fit, else 2 used alternately per step
+  if (NW == kFwdHalfWaves) return 8;   // (both halves at once: [sub-block][half][step])
   return sizeof(float2) * 4 * NW * 3 * 64 + sizeof(float) * NW * 4 * 2 * kN + 256 +
          2 * (size_t)Stage<T, 4, NW * 4, true>::kBytes + (sizeof(T) == 2 ? 2 * kRawBytes : 0) <= 160 * 1024 ? 4 : 2;
 }
+// Workgroups of 16 channels: two waves share the 4 channels that a wave has otherwise, a half of the states each, both halves of a sub-block
+// at once, and 4 more waves stage, add up the channel sums, and add and store the two halves' shares of d_deltaT, d_deltaL, d_x.
+// (A workgroup has the compute unit to itself: with a wave per 4 channels every SIMD had a single sweeping wave, which issues a vector
+// instruction every 4 to 5 clocks where two take 2.5.  64 images of 56x56x64 bf16, 256 workgroups: 0.469 -> 0.371 ms.)
+template <int NW>
+constexpr bool bwd2_halves() { return NW == kFwdHalfWaves; }
+template <int MODE, int NW>
+constexpr int bwd2_threads() { return (NW * (bwd2_halves<NW>() ? 2 : 1) + whole_helpers<MODE, NW>()) * 64; }
 template <typename T, bool STAGE_X, int MODE, int NW = kBwdWaves>
-__global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd2_kernel(const ScanParams pin) {
+__global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(const ScanParams pin) {
+  constexpr bool HALVES = bwd2_halves<NW>();
   static_assert(MODE != kModeSliced, "the linked sweep keeps a snapshot every 4 steps");
   constexpr bool STACKED = MODE == kModeStacked;
   ScanParams p = pin;   // (stacked images: the height is shortened below for a last, shorter stack)
@@ -1991,16 +2001,20 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
   constexpr int SLOT = 3 * 64;           // float2s per wave in one exchange set
   constexpr int CW = NW * CS;
   constexpr bool PERM = true;
+  constexpr int NSW = HALVES ? 2 * NW : NW;       // waves that sweep
   constexpr int NH = whole_helpers<MODE, NW>();   // waves that only stage and add up the channel sums (then the first NW waves only sweep)
   constexpr int NSTG = NH ? NH : NW;              // waves that share the copies of a block and the sums of a half-pass
   using SG = Stage<T, 4, CW, true>;
   extern __shared__ float4 smem[];
   constexpr int XSETS = bwd2_exchange_sets<T, NW>();
-  constexpr bool BATCH = XSETS == 4;
+  constexpr bool BATCH = XSETS >= 4;
+  static_assert(!HALVES || NH == 4, "the staging waves add up the two halves' shares");
   static_assert(NH == 0 || BATCH, "the waves that stage add up the sums of a half-pass in one go");
   float2* slots = reinterpret_cast<float2*>(smem);                       // BATCH: [half][step of the sub-block][wave][3][64], else [2][wave][3][64]
   float* a_lds = reinterpret_cast<float*>(slots + XSETS * NW * SLOT);    // [wave][CS][2][16], fold order
-  char* lds = reinterpret_cast<char*>(a_lds + NW * CS * 2 * kN);         // 2 staging buffers
+  float2* share_d = reinterpret_cast<float2*>(a_lds + NW * CS * 2 * kN); // HALVES: [sub-block][half][step][wave][64] shares of d_deltaT and d_deltaL
+  float* share_x = reinterpret_cast<float*>(share_d + (HALVES ? 8 * NW * 64 : 0));   // ... of d_x
+  char* lds = reinterpret_cast<char*>(share_x + (HALVES ? 8 * NW * 64 : 0));         // 2 staging buffers
   constexpr bool WIDEN = sizeof(T) == 2;
   char* raw = lds + 2 * SG::kBytes;         // [2][kRawBytes]: 16-bit B_T, B_L, C on their way
   const bool direct = WIDEN && p.bc_direct != 0;   // (uniform)
@@ -2017,13 +2031,15 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
     p.rows_last = p.H - (p.nbands - 1) * p.rb;
   }
   const int e_wg0 = eg * CW;
-  const bool helper = NH && wave >= NW;      // (uniform) stages and adds up, never sweeps
+  const bool helper = NH && wave >= NSW;     // (uniform) stages and adds up, never sweeps
   const bool stages = !NH || helper;
-  const int swave = NH ? wave - NW : wave;   // the wave's turn among those that stage
+  const int cwave = HALVES ? wave % NW : wave;   // the wave's turn among those of the workgroup's channels
+  const int my_half = HALVES ? wave / NW : 0;    // HALVES: the half of the states that the wave sweeps
+  const int swave = NH ? wave - NSW : wave;   // the wave's turn among those that stage
   const int slot = lane >> kHBShift, r = lane & (kHB - 1);
   const int rbands = row_bands(p, r);
   const int rk = STACKED ? skew_row(p, r) : r;
-  const int ch_loc = (helper ? swave : wave) * CS + slot;
+  const int ch_loc = (helper ? swave : cwave) * CS + slot;
   const int e_raw = e_wg0 + ch_loc;
   const bool ch_ok = !helper && e_raw < p.E;
   const int e = e_raw < p.E ? e_raw : p.E - 1;
@@ -2032,7 +2048,7 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
     mine[spos<true>(r)] = p.A2T[e * kN + r];
     mine[kN + spos<true>(r)] = p.A2L[e * kN + r];
   }
-  for (int i = threadIdx.x; i < 2 * SG::kBytes / 16; i += (NW + NH) * 64) reinterpret_cast<float4*>(lds)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int i = threadIdx.x; i < 2 * SG::kBytes / 16; i += (NSW + NH) * 64) reinterpret_cast<float4*>(lds)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   const uint32_t a_base_off = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) float*)(a_lds + ch_loc * (2 * kN)));
   const float dsk = p.Df[e];
   settle_loads();
@@ -2053,10 +2069,11 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
   char* BOTimg = reinterpret_cast<char*>(p.bot + (int64_t)b * p.W * p.E * kN);
   char* PARTimg = reinterpret_cast<char*>(p.part + ((int64_t)eg * p.Ptot + img_cell0) * (3 * kN));
 
-  float accAT[kN], accAL[kN], accD = 0.f;
-  float muT[kN], muL[kN];
+  constexpr int kNS = HALVES ? kN / 2 : kN;   // states of a lane (HALVES: by their place in the half)
+  float accAT[kNS], accAL[kNS], accD = 0.f;
+  float muT[kNS], muL[kNS];
 #pragma unroll
-  for (int n = 0; n < kN; ++n) { accAT[n] = 0.f; accAL[n] = 0.f; muT[n] = 0.f; muL[n] = 0.f; }
+  for (int n = 0; n < kNS; ++n) { accAT[n] = 0.f; accAL[n] = 0.f; muT[n] = 0.f; muL[n] = 0.f; }
   const uint32_t rec_off = STACKED ? r * 16 : (r == 0 ? SG::top_off(ch_loc) : (r == kHB - 1 ? SG::bot_off(ch_loc) - SG::kCOff : r * 16));
   const uint32_t xd_off = SG::kXOff + SG::x_off(r, ch_loc);
   constexpr uint32_t kXK = SG::kXStepBytes;
@@ -2119,11 +2136,13 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
   // Snapshot quads on their way, per half of the states: qa[half] the state before the sub-block that the half's next
   // half-pass sweeps (fetched two half-passes ahead: when the half's pass before starts), qn[half] the state behind
   // that sub-block, which is the state before the sub-block that the half swept last (its qa, kept as it came).
-  quad_t qa[2][2], qn[2][2];
+  constexpr int PASSES = HALVES ? 1 : 2;   // half-passes of a wave per sub-block
+  quad_t qa[PASSES][2], qn[PASSES][2];
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    load_snap(qa[hf], 2 * (m_hi - 1) + 1, hf, take1);
-    load_snap(qn[hf], 2 * (m_hi - 1) + 2, hf, take2);
+  for (int ps = 0; ps < PASSES; ++ps) {
+    const int hf = HALVES ? my_half : ps;
+    load_snap(qa[ps], 2 * (m_hi - 1) + 1, hf, take1);
+    load_snap(qn[ps], 2 * (m_hi - 1) + 2, hf, take2);
   }
   auto raw_copy_for = [&](Pos A2, char* dst, bool live) {
     const BlockPos q2 = block_pos(p, A2, rk, rbands);
@@ -2172,20 +2191,41 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
     for (int sub = 1; sub >= 0; --sub) {
       const int k0 = 2 * sub;
       float part2[2][4];   // the state sums of the first half wait here for the second
+      float2 slope[2];     // (HALVES, a wave that stages)
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
+      for (int pass = 0; pass < PASSES; ++pass) {
+       const int half = HALVES ? my_half : pass;   // (HALVES: uniform)
+       constexpr int kLast = PASSES - 1;
        if constexpr (!SWEEPS) {   // a wave that only stages: its copies have landed before the barrier that ends the block
-        if (sub == 0 && half == 1) staging_landed();
+        if constexpr (HALVES) {   // the slopes of the softplus at the cells whose results come next (behind the barrier the step sizes may be copied over)
+          if (p.dpre) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+              const int k = k0 + ks;
+              float dtv = 0.f, dlv = 0.f;
+              if constexpr (STAGE_X) {
+                const T* xr = reinterpret_cast<const T*>(bufc + xd_off + k * kXK);
+                dtv = IO<T>::ld(xr + SG::kXTauBytes / sizeof(T)); dlv = IO<T>::ld(xr + 2 * SG::kXTauBytes / sizeof(T));
+              } else if (e_raw < p.E && ((bp.in_grid >> k) & 1u)) {
+                const uint32_t off = (uint32_t)(cell0 * p.E + e) * (uint32_t)sizeof(T) + (uint32_t)k * estep + (k >= bp.kw ? wrap_adj : 0u);
+                dtv = IO<T>::ld(reinterpret_cast<const T*>(DTimg + off));
+                dlv = IO<T>::ld(reinterpret_cast<const T*>(DLimg + off));
+              }
+              slope[ks] = make_float2(softplus_slope<T>(dtv), softplus_slope<T>(dlv));
+            }
+          }
+        }
+        if (sub == 0 && pass == kLast) staging_landed();
        } else {
         float ha[8], hb1[8], hn[8], gT[8], gL[8];
         lead_if_younger<NW>(wave, true);    // (until the second step of the adjoint below)
-        widen8(qa[half], ha);
-        widen8(qn[half], hn);
-        qn[half][0] = qa[half][0]; qn[half][1] = qa[half][1];
+        widen8(qa[pass], ha);
+        widen8(qn[pass], hn);
+        qn[pass][0] = qa[pass][0]; qn[pass][1] = qa[pass][1];
         // the quads of this half's next pass (the first sub-block's passes fetch behind this block's copies for the
         // second sub-block, the second's for the block to come, in time for that block's wait for everything in flight)
-        if (sub == 1) load_snap(qa[half], 2 * m, half, take0);
-        else if (m > 0) load_snap(qa[half], 2 * (m - 1) + 1, half, take1n);
+        if (sub == 1) load_snap(qa[pass], 2 * m, half, take0);
+        else if (m > 0) load_snap(qa[pass], 2 * (m - 1) + 1, half, take1n);
         // ---- recompute the state between the two steps
         if (t0 + k0 < p.T_total) {
           const int k = k0;
@@ -2241,7 +2281,7 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
           const int k = k0 + ks;
           const int t = t0 + k;
           if (ks == 0) lead_if_younger<NW>(wave, false);
-          if (sub == 0 && half == 1 && ks == 0) staging_landed();   // before the last stores of the block, see the forward kernel
+          if (sub == 0 && pass == kLast && ks == 0) staging_landed();   // before the last stores of the block, see the forward kernel
           if (t < p.T_total) {
             const float (&hbk)[8] = ks == 1 ? hb1 : ha;    // the state before this step
             const float (&hnk)[8] = ks == 1 ? hn : hb1;    // ... and behind it
@@ -2267,8 +2307,8 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
             const float qT = cT * dtv * xv, qL = cL * dlv * xv;   // zero on lanes that are not grid cells
             const float dyl = dyv + gb1;
             float sT = 0.f, sL = 0.f, zT = 0.f, zL = 0.f;
-            if (half == 1) { sT = part2[ks][0]; sL = part2[ks][1]; zT = part2[ks][2]; zL = part2[ks][3]; }
-            float* sw = reinterpret_cast<float*>(slots + ((BATCH ? 2 * half + ks : xpar) * NW + wave) * SLOT + lane);
+            if (pass == 1) { sT = part2[ks][0]; sL = part2[ks][1]; zT = part2[ks][2]; zL = part2[ks][3]; }
+            float* sw = reinterpret_cast<float*>(slots + ((HALVES ? 4 * sub + 2 * half + ks : (BATCH ? 2 * half + ks : xpar)) * NW + cwave) * SLOT + lane);
 #pragma unroll
             for (int mgl = 0; mgl < 2; ++mgl) {
               const int mg = 2 * half + mgl;
@@ -2281,7 +2321,7 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
               float vC[4], vBT[4], vBL[4];
 #pragma unroll
               for (int qi = 0; qi < 4; ++qi) {
-                const int n = fold_state(mg, qi), s8 = 4 * mgl + qi;
+                const int s8 = 4 * mgl + qi, n = HALVES ? s8 : fold_state(2 * pass + mgl, qi);
                 const float a2t = atq[qi], a2l = alq[qi];
                 const float aT = ks == 0 ? gT[s8] : fexp2(__builtin_fmaf(dtv, a2t, offT));
                 const float aL = ks == 0 ? gL[s8] : fexp2(__builtin_fmaf(dlv, a2l, offL));
@@ -2311,11 +2351,19 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
                 char* bb = BOTimg + (wk ? bp.bnd0 + 1 : bp.bnd0) * p.bot_stride * (int64_t)sizeof(float) +
                            (uint32_t)(ck * p.E + e) * (uint32_t)(kN * sizeof(float));
 #pragma unroll
-                for (int q = 2 * half; q < 2 * half + 2; ++q)
-                  reinterpret_cast<float4*>(bb)[q] = make_float4(muT[sinv<PERM>(4 * q)], muT[sinv<PERM>(4 * q + 1)], muT[sinv<PERM>(4 * q + 2)], muT[sinv<PERM>(4 * q + 3)]);
+                for (int ql = 0; ql < 2; ++ql) {
+                  const int q0 = HALVES ? 0 : 4 * (2 * pass + ql);   // (a quad is a state group: HALVES has them in place)
+                  if constexpr (HALVES) reinterpret_cast<float4*>(bb)[2 * half + ql] = make_float4(muT[4 * ql], muT[4 * ql + 1], muT[4 * ql + 2], muT[4 * ql + 3]);
+                  else reinterpret_cast<float4*>(bb)[2 * pass + ql] = make_float4(muT[sinv<PERM>(q0)], muT[sinv<PERM>(q0 + 1)], muT[sinv<PERM>(q0 + 2)], muT[sinv<PERM>(q0 + 3)]);
+                }
               }
             }
-            if (half == 0) {
+            if constexpr (HALVES) {   // the half's shares of the results
+              accD = __builtin_fmaf(dyv, xv, accD);
+              const int at = ((2 * sub + half) * 2 + ks) * (NW * 64) + cwave * 64 + lane;
+              share_d[at] = make_float2(__builtin_fmaf(cT * xv, sT, kLn2 * zT), __builtin_fmaf(cL * xv, sL, kLn2 * zL));
+              share_x[at] = __builtin_fmaf(cT * dtv, sT, __builtin_fmaf(cL * dlv, sL, half == 0 ? dyv * dsk : 0.f));
+            } else if (pass == 0) {
               part2[ks][0] = sT; part2[ks][1] = sL; part2[ks][2] = zT; part2[ks][3] = zL;
             } else {
               accD = __builtin_fmaf(dyv, xv, accD);
@@ -2360,18 +2408,36 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
           __syncthreads();
           if constexpr (STAGES)
 #pragma unroll
-          for (int rd = 0; rd < (2 * 3 + NSTG - 1) / NSTG; ++rd) {
+          for (int rd = 0; rd < ((HALVES ? 4 : 2) * 3 + NSTG - 1) / NSTG; ++rd) {
             const int jj = rd * NSTG + swave;                 // (uniform)
-            if (jj < 2 * 3) {
-              const int ks = jj / 3, v = jj - 3 * ks;
+            if (jj < (HALVES ? 4 : 2) * 3) {
+              const int sets = jj / 3, v = jj - 3 * sets;
+              const int ks = HALVES ? sets & 1 : sets, half = HALVES ? sets >> 1 : pass;
               const int k = k0 + ks;
               if (t0 + k < p.T_total && ((bp.in_grid >> k) & 1u)) {
                 const uint32_t off = f_off0 + (uint32_t)k * pstep + (k >= bp.kw ? pwrap_adj : 0u) + (uint32_t)((v * kN + 2 * half) * sizeof(float));
-                const float2* sl = slots + (2 * half + ks) * NW * SLOT + v * 64 + lane;
+                const float2* sl = slots + ((HALVES ? 4 * sub : 0) + 2 * half + ks) * NW * SLOT + v * 64 + lane;
                 float2 sum = sl[0];
 #pragma unroll
                 for (int w = 1; w < NW; ++w) { sum.x += sl[w * SLOT].x; sum.y += sl[w * SLOT].y; }
                 *reinterpret_cast<float2*>(PARTimg + off) = sum;
+              }
+            }
+          }
+          if constexpr (HALVES && STAGES) {   // the results of the staging wave's four channels: both halves' shares
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+              const int k = k0 + ks;
+              if (t0 + k < p.T_total && e_raw < p.E && ((bp.in_grid >> k) & 1u)) {
+                const int at = (4 * sub + ks) * (NW * 64) + swave * 64 + lane;
+                const float2 a = share_d[at], c = share_d[at + 2 * NW * 64];
+                float gdT = a.x + c.x, gdL = a.y + c.y;
+                const float gx = share_x[at] + share_x[at + 2 * NW * 64];
+                const uint32_t goff = (uint32_t)(cell0 * p.E + e) * (uint32_t)sizeof(T) + (uint32_t)k * estep + (k >= bp.kw ? wrap_adj : 0u);
+                if (p.dpre) { gdT *= slope[ks].x; gdL *= slope[ks].y; }   // (uniform) gradients with respect to what the softplus was applied to
+                IO<T>::st(reinterpret_cast<T*>(DDTimg + goff), gdT);
+                IO<T>::st(reinterpret_cast<T*>(DDLimg + goff), gdL);
+                IO<T>::st(reinterpret_cast<T*>(DXimg + goff), gx);
               }
             }
           }
@@ -2391,12 +2457,12 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
   else sweep(std::integral_constant<int, kSweeper>{});
 
   // ---- sums over positions: reduce over the rows of the band (lanes of one channel slot)
-  float red[2 * kN + 1];
+  float red[2 * kNS + 1];
 #pragma unroll
-  for (int n = 0; n < kN; ++n) { red[n] = accAT[n]; red[kN + n] = accAL[n]; }
-  red[2 * kN] = accD;
+  for (int n = 0; n < kNS; ++n) { red[n] = accAT[n]; red[kNS + n] = accAL[n]; }
+  red[2 * kNS] = accD;
 #pragma unroll
-  for (int k = 0; k < 2 * kN + 1; ++k) {
+  for (int k = 0; k < 2 * kNS + 1; ++k) {
     float v = red[k];
 #pragma unroll
     for (int off = kHB >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -2406,8 +2472,12 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW>()) * 64) void m2d_bwd
     const int64_t slot_e = (int64_t)b * p.pa_slots * p.E + e;
     float* pa = p.pA + slot_e * (2 * kN);
 #pragma unroll
-    for (int n = 0; n < 2 * kN; ++n) pa[n] = red[n];
-    p.pD[slot_e] = red[2 * kN];
+    for (int n = 0; n < kNS; ++n) {
+      const int state = HALVES ? fold_state(n / 4, n % 4) + my_half * (fold_state(2, 0) - fold_state(0, 0)) : n;
+      pa[state] = red[n];
+      pa[kN + state] = red[kNS + n];
+    }
+    if (!HALVES || my_half == 0) p.pD[slot_e] = red[2 * kNS];
   }
 }
 
@@ -2590,7 +2660,7 @@ struct Geometry {
   int HB, hb_shift, CS, nbands, nblk;
   int S, T_total, rows_last;         // stream stride, total steps, rows of the last band
   int rb;                            // grid rows per band
-  int fwd_ec, fwd_nw, fwd_wpb, fwd_bpb;   // forward: channels per lane, waves per workgroup, waves and workgroups per image
+  int fwd_ec, fwd_nw, fwd_wpb, fwd_bpb;   // forward: channels per lane (split states: per wave), waves per workgroup, waves and workgroups per image
   int bwd_nw, bwd_wpb, bwd_bpb;      // backward: waves per workgroup, waves and workgroups (channel groups) per image
   bool fwd_split, bwd_split;         // the states of a channel split over the lanes (a wave per channel: m2d_fwd_split_kernel, m2d_bwd_split_kernel)
   bool stage_x;                      // x, delta, dy rows are whole 16-byte chunks: stage them through LDS
@@ -2642,6 +2712,7 @@ Geometry make_geometry(const m2d_desc* d) {
   const int64_t ncu = device_cus();
   g.HB = kHB;
   g.hb_shift = kHBShift;
+  g.stage_x = (d->E % (d->dtype == M2D_BF16 ? 8 : 4)) == 0;
   g.CS = 64 / g.HB;
   const int groups = (d->E + kBwdWaves * g.CS - 1) / (kBwdWaves * g.CS);   // workgroups per image
   // Grids of a single band (14x14, 7x7, 10x10 ...): a sweep spends as many steps filling and
@@ -2753,20 +2824,21 @@ Geometry make_geometry(const m2d_desc* d) {
   // waves.  Which is faster, and in which schedule, is a matter of how many workgroups follow each other on a compute unit (a backward
   // kernel has the unit to itself) and of the chain of bands: blocks that one unit sweeps, times what a block takes.  Measured, forward keeping snapshots
   // and backward, relative to a workgroup of 4 waves with a quarter of the states each (56x56x64 bf16, all units busy): 8 such waves
-  // 1.47, whole states 3.0 in workgroups of 4 waves (16 channels), 4.2 in workgroups of 8 (32 channels).
+  // 1.47, whole states 4.2 in workgroups of 8 waves (32 channels), and in workgroups of 16 channels 3.0 in the linked sweep and 2.35
+  // in one stream per image (where 8 waves share the work of 4: m2d_bwd2_kernel, and the forward below).
   // In the linked sweep a band trails its neighbour by 6 blocks, and the shorter of the two, the chain of bands and the work per unit, hides
   // behind the longer but for about a fifth (where units have more than one workgroup to sweep).
   // What this rule takes from the whole states, forward + backward in ms: 30x60x50x40 fp32 0.517 -> 0.312, 8x100x120x96 bf16 0.891 -> 0.615,
-  // 8x256x256x64 bf16 3.13 -> 2.09, 20x28x28x200 fp32 0.296 -> 0.192, 40x56x56x64 bf16 0.620 -> 0.513, 2048x2048x64 fp32 forward 6.39 -> 4.82;
+  // 8x256x256x64 bf16 3.13 -> 2.09, 20x28x28x200 fp32 0.296 -> 0.192, 2048x2048x64 fp32 forward 6.39 -> 4.82;
   // and leaves with them: 32x128x128x64 bf16 2.00 (split 2.17), 8x512x512x64 bf16 7.6 (8.0), 64x28x28x128 bf16 0.280 (0.389).
   // Near the line the whole states stay: fewer channel sums, and snapshots every 2 steps.
-  constexpr int64_t kSplit4 = 100, kSplit8 = 147, kWhole4 = 300, kWhole8 = 417;
+  constexpr int64_t kSplit4 = 100, kSplit8 = 147, kWhole4 = 235, kWhole4Linked = 300, kWhole8 = 417;
   auto stream_cost = [&](int64_t wgs, int64_t block) { return (wgs + ncu - 1) / ncu * nblk_stream * block; };
   auto link_cost = [&](int64_t wgs, int64_t block) {
     const int64_t work = (wgs * g.nbands + ncu - 1) / ncu * nbb_link, chain = nbb_link + (int64_t)(g.nbands - 1) * (kLinkLag - 1);
     return (work > chain ? work + chain / 5 : chain + (work > nbb_link ? work / 5 : 0)) * block;
   };
-  const int64_t whole_block = g.bwd_nw == kFwdHalfWaves ? kWhole4 : kWhole8;
+  const int64_t whole_block = g.bwd_nw != kFwdHalfWaves ? kWhole8 : (g.sliced ? kWhole4Linked : kWhole4);
   const int64_t whole_cost = g.sliced ? link_cost((int64_t)B * g.bwd_bpb, whole_block) : stream_cost((int64_t)B * g.bwd_bpb, whole_block);
   const int64_t wg4 = (int64_t)B * ((d->E + kSplitHalfWaves - 1) / kSplitHalfWaves), wg8 = (int64_t)B * ((d->E + kSplitWaves - 1) / kSplitWaves);
   int split_nw = kSplitHalfWaves;
@@ -2807,13 +2879,22 @@ Geometry make_geometry(const m2d_desc* d) {
       g.bwd_wpb = g.bwd_bpb * g.bwd_nw;
     }
   }
+  // The forward beside a backward in workgroups of 16 channels, one stream per image: 8 waves with two channels each and a quarter of
+  // the states per lane, which keep a SIMD busy where 4 waves that hold all states leave it to one (64 images of 56x56x64 bf16: forward
+  // 0.160 -> 0.133 ms, keeping snapshots 0.167 -> 0.140; with twice as many images, two rounds of either, they are level: 0.262 against 0.264).
+  if (!split && !g.stacked && !g.sliced && g.stage_x && g.fwd_nw == kFwdHalfWaves && g.ck_shift == 0 && !g.snap32 && !(d->flags & M2D_FLAG_WHOLE_STATES)) {
+    g.fwd_split = true;
+    g.fwd_ec = 2;
+    g.fwd_nw = kSplitWaves;
+    g.fwd_bpb = (d->E + kSplitWaves * g.fwd_ec - 1) / (kSplitWaves * g.fwd_ec);
+    g.fwd_wpb = g.fwd_bpb * g.fwd_nw;
+  }
   if (g.snap32) {
     g.fwd_ec = 1;
     g.fwd_nw = g.bwd_nw = kFwdHalfWaves;
     g.fwd_bpb = g.bwd_bpb = (d->E + kFwdHalfWaves * g.CS - 1) / (kFwdHalfWaves * g.CS);
     g.fwd_wpb = g.bwd_wpb = g.fwd_bpb * kFwdHalfWaves;
   }
-  g.stage_x = (d->E % (d->dtype == M2D_BF16 ? 8 : 4)) == 0;
   const size_t P = (size_t)d->B * d->H * d->W;
   g.prep_bytes = align_up(sizeof(float) * (kZeroFloats + (size_t)2 * d->E * kN + d->E));
   g.packed_bc = (d->flags & M2D_FLAG_PACKED_BC) != 0;   // the caller brings the records: nothing to reserve
@@ -2824,7 +2905,7 @@ Geometry make_geometry(const m2d_desc* d) {
   g.ck_nblk = g.sliced ? g.nbands * g.ck_pb : (g.nblk + every - 1) / every;
   // A snapshot every 2 steps, for the backward kernel that recomputes one step in two: where every image (or stack)
   // is one stream and a lane holds all states of its channel.  Other schedules keep one every 4 steps.
-  g.ck_half = (d->ckpt_interval == 2 || d->ckpt_interval == 0) && !g.sliced && !g.fwd_split && !g.bwd_split && !g.snap32;
+  g.ck_half = (d->ckpt_interval == 2 || d->ckpt_interval == 0) && !g.sliced && !(g.fwd_split && g.fwd_ec == 1) && !g.bwd_split && !g.snap32;
   if (g.ck_half) g.ck_nblk = 2 * g.nblk + 1;   // before the steps 0 and 2 of every block, and behind the last block
   g.ckpt_diag_bytes = align_up((d->dtype == M2D_BF16 && !g.snap32 ? 2 : sizeof(float)) * (size_t)B * g.ck_nblk * d->E * kN * g.HB);   // (16-bit tensors: bf16 snapshots unless fp32 ones are asked for)
   const size_t bwd_wgs = (size_t)(g.sliced ? g.nbands : 1) * B * g.bwd_bpb;
@@ -2958,16 +3039,24 @@ int launch_fwd_as(const ScanParams& sp, hipStream_t st) {
   }
 }
 
-template <typename T, bool CK, bool WY, bool SX, int MODE, int NWS = kSplitWaves>
+template <typename T, bool CK, bool WY, bool SX, int MODE, int NWS = kSplitWaves, int EC = 1, bool HALF = false>
 int launch_fwd_split_as(const ScanParams& sp, hipStream_t st) {
-  if constexpr (!M2D_BUILT(T, SX, MODE, NWS, false)) return M2D_ERR_UNSUPPORTED; else {
-  constexpr size_t lds = SplitFwdLds<T, NWS, SX>::kBytes;
+  if constexpr (!M2D_BUILT(T, SX, MODE, NWS, EC == 2)) return M2D_ERR_UNSUPPORTED; else {
+  constexpr size_t lds = SplitFwdLds<T, NWS, SX, EC>::kBytes;
   static_assert(lds <= kLdsPerWorkgroup, "staging must fit the LDS");
   static std::atomic<uint64_t> seen{0};
-  if (!allow_dynamic_lds(reinterpret_cast<const void*>(&m2d_fwd_split_kernel<T, CK, WY, SX, MODE, NWS>), lds, seen)) return M2D_ERR_HIP;
-  hipLaunchKernelGGL((m2d_fwd_split_kernel<T, CK, WY, SX, MODE, NWS>), dim3((unsigned)sp.nwg), dim3((NWS + kSplitStagers) * 64), lds, st, sp);
+  if (!allow_dynamic_lds(reinterpret_cast<const void*>(&m2d_fwd_split_kernel<T, CK, WY, SX, MODE, NWS, EC, HALF>), lds, seen)) return M2D_ERR_HIP;
+  hipLaunchKernelGGL((m2d_fwd_split_kernel<T, CK, WY, SX, MODE, NWS, EC, HALF>), dim3((unsigned)sp.nwg), dim3((NWS + kSplitStagers) * 64), lds, st, sp);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
   }
+}
+// two channels a wave: one stream per image, rows of whole chunks
+template <typename T>
+int launch_fwd_split_pairs(const ScanParams& sp, bool ckpt, bool write_y, hipStream_t st) {
+  if (!ckpt) return launch_fwd_split_as<T, false, true, true, kModeSweep, kSplitWaves, 2>(sp, st);
+  if (sp.ck_half)
+    return write_y ? launch_fwd_split_as<T, true, true, true, kModeSweep, kSplitWaves, 2, true>(sp, st) : launch_fwd_split_as<T, true, false, true, kModeSweep, kSplitWaves, 2, true>(sp, st);
+  return write_y ? launch_fwd_split_as<T, true, true, true, kModeSweep, kSplitWaves, 2>(sp, st) : launch_fwd_split_as<T, true, false, true, kModeSweep, kSplitWaves, 2>(sp, st);
 }
 // (x and deltas of a workgroup's channels are one or two 16-byte chunks per cell, or 4 channels of a 16-bit tensor half of one)
 template <typename T, int MODE>
@@ -3018,6 +3107,7 @@ int launch_fwd(const ScanParams& sp0, const m2d_desc* d, const Geometry& g, bool
         return write_y ? launch_fwd_as<T, 1, true, true, false, kModeSweep, kFwdHalfWaves, false, float>(sp, st) : launch_fwd_as<T, 1, true, false, false, kModeSweep, kFwdHalfWaves, false, float>(sp, st);
       }
     }
+    if (g.fwd_split && g.fwd_ec == 2) return launch_fwd_split_pairs<T>(sp, ckpt, write_y, st);
     if (g.fwd_split)
       return g.sliced ? launch_fwd_split<T, kModeSliced>(sp, g.stage_x, ckpt, write_y, st, g.fwd_nw)
                       : launch_fwd_split<T, kModeSweep>(sp, g.stage_x, ckpt, write_y, st, g.fwd_nw);
@@ -3091,17 +3181,17 @@ int launch_bwd_as(const ScanParams& sp, hipStream_t st) {
 
 template <typename T, int NW>
 constexpr size_t bwd2_lds_bytes() {
-  return sizeof(float2) * bwd2_exchange_sets<T, NW>() * NW * 3 * 64 + sizeof(float) * NW * 4 * 2 * kN + 256 +
+  return sizeof(float2) * bwd2_exchange_sets<T, NW>() * NW * 3 * 64 + sizeof(float) * NW * 4 * 2 * kN + (bwd2_halves<NW>() ? sizeof(float) * 3 * 8 * NW * 64 : 256) +
          2 * (size_t)Stage<T, 4, NW * 4, true>::kBytes + (sizeof(T) == 2 ? 2 * kRawBytes : 0);
 }
-template <typename T, bool SX, int MODE, int NW>
+template <typename T, bool SX, int MODE, int NW = kBwdWaves>
 int launch_bwd2_as(const ScanParams& sp, hipStream_t st) {
   if constexpr (!M2D_BUILT(T, SX, MODE, NW, true)) return M2D_ERR_UNSUPPORTED; else {
   constexpr size_t lds = bwd2_lds_bytes<T, NW>();
   static_assert(lds <= kLdsPerWorkgroup, "exchange sets and staging must fit the LDS");
   static std::atomic<uint64_t> seen{0};
   if (!allow_dynamic_lds(reinterpret_cast<const void*>(&m2d_bwd2_kernel<T, SX, MODE, NW>), lds, seen)) return M2D_ERR_HIP;
-  hipLaunchKernelGGL((m2d_bwd2_kernel<T, SX, MODE, NW>), dim3((unsigned)sp.nwg), dim3((NW + whole_helpers<MODE, NW>()) * 64), lds, st, sp);
+  hipLaunchKernelGGL((m2d_bwd2_kernel<T, SX, MODE, NW>), dim3((unsigned)sp.nwg), dim3(bwd2_threads<MODE, NW>()), lds, st, sp);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
   }
 }
@@ -3328,13 +3418,15 @@ int m2d_scan_plan(const m2d_desc* desc, int pass, char* text, size_t cap) {
   if (split) {
     const bool values = nw == kSplitWaves && !g.stage_x;   // rows that are no whole chunks: x and the step sizes go through registers, value by value
     snprintf(text, cap, "%s: %s, %lld workgroups of %d waves%s, %d channels each, 4 states per lane%s",
-             fwd ? "m2d_fwd_split_kernel" : "m2d_bwd_split_kernel", sched, wgs, nw, values ? "" : " and 4 that stage", nw, values ? ", and 4 more waves that stage value by value" : "");
+             fwd ? "m2d_fwd_split_kernel" : "m2d_bwd_split_kernel", sched, wgs, nw, values ? "" : " and 4 that stage", nw * per_lane, values ? ", and 4 more waves that stage value by value" : "");
+    if (g.ck_half) strncat(text, ", a snapshot every 2 steps", cap - strlen(text) - 1);
   }
   else {
     // (workgroups of 4 waves have waves that only stage, except in the backward that replays the forward between snapshots)
     const bool helped = !g.stacked && nw == kFwdHalfWaves && per_lane == 1 && (fwd || g.ck_shift == 0);
     char extra[48] = "";
     if (helped) snprintf(extra, sizeof extra, " and %d that stage", kWholeHelpers);
+    if (helped && !fwd && g.ck_half) snprintf(extra, sizeof extra, " in two halves and %d that stage", kWholeHelpers);
     snprintf(text, cap, "%s: %s, %lld workgroups of %d waves%s, %d channels each, 16 states per lane%s",
              fwd ? "m2d_fwd_kernel" : (g.ck_half ? "m2d_bwd2_kernel" : "m2d_bwd_kernel"), sched, wgs, nw, extra, nw * g.CS * per_lane,
              g.ck_half ? (fwd ? ", a snapshot every 2 steps" : ", a snapshot every 2 steps and one step in two recomputed") : "");

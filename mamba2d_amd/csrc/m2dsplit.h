@@ -98,6 +98,14 @@ __device__ __forceinline__ float split_x(const char* at) {   // one value of x, 
 template <bool DEVICE_SCOPE>
 __device__ __forceinline__ void split_fill16(const void* src, uint32_t at) { lds_fill16_at<DEVICE_SCOPE>(src, __builtin_amdgcn_readfirstlane(at)); }
 
+// EC values of neighbouring channels (two: they are in one chunk)
+template <typename T, bool SX, int EC>
+__device__ __forceinline__ void split_xs(const char* at, float (&v)[EC]) {
+  if constexpr (EC == 1) v[0] = split_x<T, SX>(at);
+  else if constexpr (sizeof(T) == 4) { const float2 q = *reinterpret_cast<const float2*>(at); v[0] = q.x; v[1] = q.y; }
+  else { const uint32_t q = *reinterpret_cast<const uint32_t*>(at); v[0] = __uint_as_float(q << 16); v[1] = __uint_as_float(q & 0xffff0000u); }
+}
+
 // Where a lane's (step, row) of a block is.  The linked sweep stays inside one band, and its columns count from the start of the
 // band's window (below 0 and from W on: off the grid); otherwise the stream wraps from band to band.
 template <bool SLICED>
@@ -162,6 +170,17 @@ __device__ __forceinline__ void split_store(bf16_t* dst, float v, bool live) {
   uint64_t saved;
   const uint32_t bits = f32_to_bf16_bits(v);
   asm volatile("s_and_saveexec_b64 %0, %3\n\tglobal_store_short %1, %2, off\n\ts_mov_b64 exec, %0" : "=&s"(saved) : "v"(dst), "v"(bits), "s"(__ballot(live)) : "memory", "scc");
+}
+// four neighbouring values
+__device__ __forceinline__ void split_store_quad(float* dst, float4 v, bool live) {
+  uint64_t saved;
+  const v4f_t w = {v.x, v.y, v.z, v.w};
+  asm volatile("s_and_saveexec_b64 %0, %3\n\tglobal_store_dwordx4 %1, %2, off\n\ts_mov_b64 exec, %0\n\ts_nop 0" : "=&s"(saved) : "v"(dst), "v"(w), "s"(__ballot(live)) : "memory", "scc");
+}
+__device__ __forceinline__ void split_store_quad(bf16_t* dst, float4 v, bool live) {
+  uint64_t saved;
+  const uint64_t w = (uint64_t)f32_to_bf16_bits(v.x) | (uint64_t)f32_to_bf16_bits(v.y) << 16 | (uint64_t)f32_to_bf16_bits(v.z) << 32 | (uint64_t)f32_to_bf16_bits(v.w) << 48;
+  asm volatile("s_and_saveexec_b64 %0, %3\n\tglobal_store_dwordx2 %1, %2, off\n\ts_mov_b64 exec, %0" : "=&s"(saved) : "v"(dst), "v"(w), "s"(__ballot(live)) : "memory", "scc");
 }
 // the four values at 0, 32, 16 and 48 bytes (a lane's states of a channel sum: the components j hold states perm(j) * 4 + g, perm = 0, 2, 1, 3)
 __device__ __forceinline__ void split_store_sum(void* dst, float4 v, bool live) {
@@ -287,29 +306,33 @@ __device__ __forceinline__ void split_vals_put(const SplitVals<T, NT, CW>& o, ch
 // whose results make a window: window q holds those of the steps 4q - 1 .. 4q + 2.  While window q is filled, the staging
 // waves send window q - 1 to memory and fetch the operands of block q + 3 (boundary rows: of block q + 1): a block takes
 // less time than a fetch from memory.
-template <typename T, int NW, bool SX>
+template <typename T, int NW, bool SX, int EC = 1>
 struct SplitFwdLds {
-  using SG = SplitStage<T, 3, NW, false, SX>;
+  static constexpr int CW = NW * EC;
+  using SG = SplitStage<T, 3, CW, false, SX>;
   static constexpr int kBufs = 4;
-  static constexpr int kYCh = kHB * 16 + 32;               // the shares of y of one channel at one step: [row][state group] floats (32 bytes more: four channels are read at once)
-  static constexpr int kYStep = NW * kYCh;
+  // the shares of y of one channel at one step: [row][state group] floats (a few bytes more: lanes that read together meet different banks)
+  static constexpr int kYCh = kHB * 16 + (EC == 1 ? 32 : 16);
+  static constexpr int kYStep = CW * kYCh;
   static constexpr int kYBytes = kCK * kYStep;             // one window
-  static constexpr int kRStep = NW * 64;                   // the band's last row at one step: [channel][state group] float4s
+  static constexpr int kRStep = CW * 64;                   // the band's last row at one step: [channel][state group] float4s
   static constexpr int kRBytes = kCK * kRStep;
   static constexpr int kY = kBufs * SG::kBytes, kR = kY + 2 * kYBytes, kFlag = kR + 2 * kRBytes, kBytes = kFlag + 16;   // flag: the wave that waits has given up
 };
-template <typename T, bool CKPT, bool WRITE_Y, bool SX, int MODE, int NW = kSplitWaves>
+template <typename T, bool CKPT, bool WRITE_Y, bool SX, int MODE, int NW = kSplitWaves, int EC = 1, bool HALF = false>
 __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kernel(const ScanParams pin) {
   static_assert(MODE != kModeStacked, "stacked images are many: they never need the split");
   constexpr bool SLICED = MODE == kModeSliced;
   constexpr bool OWN_SETUP = split_owns_setup<CKPT, MODE>();
   constexpr bool WIDEN = sizeof(T) == 2;
-  constexpr int CW = NW;
+  constexpr int CW = NW * EC;
+  static_assert(EC == 1 || (EC == 2 && SX && NW == kSplitWaves && !SLICED), "two channels a wave: rows of whole chunks, one stream per image");
+  static_assert(!HALF || (CKPT && !SLICED), "snapshots every 2 steps: kept by a forward of one stream per image");
   const ScanParams& p = pin;
   __builtin_assume(p.stacked == 0);
   __builtin_assume(p.rb == kRB);
   __builtin_assume(p.S >= kHB + kCK - 1);
-  using L = SplitFwdLds<T, NW, SX>;
+  using L = SplitFwdLds<T, NW, SX, EC>;
   using SG = typename L::SG;
   extern __shared__ float4 smem[];
   char* lds = reinterpret_cast<char*>(smem);
@@ -338,21 +361,25 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kerne
   if (wave < NW) {
     // ------------------------------------------------------------------------------ sweeps
     const int g = lane >> kHBShift, r = lane & (kHB - 1);   // state group, lane row
-    const int ch = wave;
-    const bool ch_ok = e_wg0 + ch < p.E;                    // (uniform) idle waves still take part in the barriers
-    const int e0 = ch_ok ? e_wg0 + ch : p.E - 1;
-    float a2t[4], a2l[4];
+    const int ch = wave * EC;                               // the wave's (first) channel
+    const bool ch_ok = e_wg0 + ch < p.E;                    // (uniform) idle waves still take part in the barriers (EC = 2: E is even)
+    const int e0 = ch_ok ? e_wg0 + ch : p.E - EC;
+    float a2t[EC][4], a2l[EC][4], dskg[EC];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int n = (!WIDEN && direct) ? 4 * g + w : (w == 1 ? 2 : (w == 2 ? 1 : w)) * 4 + g;   // the state that register w meets: 4g + w, or sinv(4g + w)
-      a2t[w] = OWN_SETUP ? gate_rate<T>(p, p.AT, e0 * kN + n) : p.A2T[e0 * kN + n];
-      a2l[w] = OWN_SETUP ? gate_rate<T>(p, p.AL, e0 * kN + n) : p.A2L[e0 * kN + n];
+    for (int c = 0; c < EC; ++c) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int n = (!WIDEN && direct) ? 4 * g + w : (w == 1 ? 2 : (w == 2 ? 1 : w)) * 4 + g;   // the state that register w meets: 4g + w, or sinv(4g + w)
+        a2t[c][w] = OWN_SETUP ? gate_rate<T>(p, p.AT, (e0 + c) * kN + n) : p.A2T[(e0 + c) * kN + n];
+        a2l[c][w] = OWN_SETUP ? gate_rate<T>(p, p.AL, (e0 + c) * kN + n) : p.A2L[(e0 + c) * kN + n];
+      }
+      dskg[c] = g == 0 ? (OWN_SETUP ? skip_gain<T>(p, e0 + c) : p.Df[e0 + c]) : 0.f;   // (x * D is in the share of group 0)
     }
     static_assert(sinv<true>(1) == 8 && sinv<true>(6) == 5 && sinv<true>(15) == 15, "fold order");
-    const float dskg = g == 0 ? (OWN_SETUP ? skip_gain<T>(p, e0) : p.Df[e0]) : 0.f;   // (x * D is in the share of group 0)
     const float g1 = r == 0 ? 1.f : 0.f;                    // the ghost's T input coefficient
     // a grid row reads its own B_T; the ghost (lane 0) the row above as its B_T, and zeros as its B_L and C
     const uint32_t bt_off = r == 0 ? SG::row_off(SG::kTop, ch, g) : SG::bc_off(0, g, r);
+    const uint32_t bt_ch = r == 0 ? 64 : 0;                 // (EC = 2) ... of the second channel
     const uint32_t bt_step = r == 0 ? SG::kStep : SG::kBCStep;
     const uint32_t bl_off = SG::bc_off(1, g, r);
     const uint32_t k_off = SG::kConst + r * 16;
@@ -361,48 +388,58 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kerne
     char* rw = lds + L::kR + ch * 64 + g * 16;
     const bool last_row = r == kRB && p.nbands > 1;         // the band's last row: the next band's ghost will replay it
     typename Snap<T>::quad* ckp = nullptr;
-    if constexpr (CKPT) ckp = snapshot_at<T>(p, b, m_lo, e0, p.ck_nblk) + snap_lane(r) + snap_quad(g);
-    const int64_t ck_step = (int64_t)p.E * (kN / 4 * kHB);
+    if constexpr (CKPT) ckp = snapshot_at<T>(p, b, HALF ? 2 * m_lo : m_lo, e0, p.ck_nblk) + snap_lane(r) + snap_quad(g);
+    const int64_t ck_step = (int64_t)p.E * (kN / 4 * kHB);  // (from one snapshot to the next)
     settle_loads();
 
-    struct Ops { float4 kk, bt, bl, cc; float x, dt, dl; };
+    struct Ops { float4 kk, bt[EC], bl, cc; float x[EC], dt[EC], dl[EC]; };
     auto fetch = [&](uint32_t buf, int k, Ops& o) {
       const char* at = lds + buf;
       o.kk = *reinterpret_cast<const float4*>(at + k_off + k * SG::kStep);
-      o.dt = split_x<T, SX>(at + x_off + SG::kXTensor + k * SG::kXStep);
-      o.dl = split_x<T, SX>(at + x_off + 2 * SG::kXTensor + k * SG::kXStep);
-      o.x = split_x<T, SX>(at + x_off + k * SG::kXStep);
+      split_xs<T, SX, EC>(at + x_off + SG::kXTensor + k * SG::kXStep, o.dt);
+      split_xs<T, SX, EC>(at + x_off + 2 * SG::kXTensor + k * SG::kXStep, o.dl);
+      split_xs<T, SX, EC>(at + x_off + k * SG::kXStep, o.x);
       o.bl = *reinterpret_cast<const float4*>(at + bl_off + k * SG::kBCStep);
-      o.bt = *reinterpret_cast<const float4*>(at + bt_off + k * bt_step);
+#pragma unroll
+      for (int c = 0; c < EC; ++c) o.bt[c] = *reinterpret_cast<const float4*>(at + bt_off + c * bt_ch + k * bt_step);
       if constexpr (WRITE_Y) o.cc = *reinterpret_cast<const float4*>(at + bl_off + SG::kBCTensor + k * SG::kBCStep);
     };
-    float h[4] = {0.f, 0.f, 0.f, 0.f};
+    float h[EC][4];
+#pragma unroll
+    for (int c = 0; c < EC; ++c)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) h[c][w] = 0.f;
     auto step = [&](const Ops& o, int k, int par) {   // par: the window that takes the results
-      const float sT = __builtin_fmaf(o.kk.z * o.dt, o.x, g1);
-      const float sL = o.kk.w * o.dl * o.x;
-      // gates before chains (see m2d_fwd_kernel: no DPP multiply-add right behind the v_exp that makes its gate)
-      float aT[4], aL[4];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) aT[w] = fexp2(__builtin_fmaf(o.dt, a2t[w], o.kk.x));
+      for (int c = 0; c < EC; ++c) {
+        const float sT = __builtin_fmaf(o.kk.z * o.dt[c], o.x[c], g1);
+        const float sL = o.kk.w * o.dl[c] * o.x[c];
+        // gates before chains (see m2d_fwd_kernel: no DPP multiply-add right behind the v_exp that makes its gate)
+        float aT[4], aL[4];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) aL[w] = fexp2(__builtin_fmaf(o.dl, a2l[w], o.kk.y));
-      pin4(aT); pin4(aL);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (CKPT) { if (k == 0 && ch_ok) Snap<T>::store(ckp, h[0], h[1], h[2], h[3]); }   // the lane's states as they are before this block
-      const float bq[4] = {o.bt.x, o.bt.y, o.bt.z, o.bt.w}, lq[4] = {o.bl.x, o.bl.y, o.bl.z, o.bl.w};
+        for (int w = 0; w < 4; ++w) aT[w] = fexp2(__builtin_fmaf(o.dt[c], a2t[c][w], o.kk.x));
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        float u = sL * lq[w];
-        u = __builtin_fmaf(sT, bq[w], u);
-        u = fma_row_below(aT[w], h[w], u);
-        h[w] = __builtin_fmaf(aL[w], h[w], u);
-      }
-      const int slot = (k + 1) & (kCK - 1);
-      if (last_row) *reinterpret_cast<float4*>(rw + par * L::kRBytes + slot * L::kRStep) = make_float4(h[0], h[1], h[2], h[3]);
-      if constexpr (WRITE_Y) {
-        const float y0 = __builtin_fmaf(h[2], o.cc.z, __builtin_fmaf(h[0], o.cc.x, o.x * dskg));
-        const float y1 = __builtin_fmaf(h[3], o.cc.w, h[1] * o.cc.y);
-        *reinterpret_cast<float*>(yw + par * L::kYBytes + slot * L::kYStep) = y0 + y1;
+        for (int w = 0; w < 4; ++w) aL[w] = fexp2(__builtin_fmaf(o.dl[c], a2l[c][w], o.kk.y));
+        pin4(aT); pin4(aL);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (CKPT) {   // the lane's states as they are before this step
+          if ((k == 0 || (HALF && k == 2)) && ch_ok) Snap<T>::store(ckp + (HALF && k == 2 ? ck_step : 0) + c * (kN / 4 * kHB), h[c][0], h[c][1], h[c][2], h[c][3]);
+        }
+        const float bq[4] = {o.bt[c].x, o.bt[c].y, o.bt[c].z, o.bt[c].w}, lq[4] = {o.bl.x, o.bl.y, o.bl.z, o.bl.w};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          float u = sL * lq[w];
+          u = __builtin_fmaf(sT, bq[w], u);
+          u = fma_row_below(aT[w], h[c][w], u);
+          h[c][w] = __builtin_fmaf(aL[w], h[c][w], u);
+        }
+        const int slot = (k + 1) & (kCK - 1);
+        if (last_row) *reinterpret_cast<float4*>(rw + c * 64 + par * L::kRBytes + slot * L::kRStep) = make_float4(h[c][0], h[c][1], h[c][2], h[c][3]);
+        if constexpr (WRITE_Y) {
+          const float y0 = __builtin_fmaf(h[c][2], o.cc.z, __builtin_fmaf(h[c][0], o.cc.x, o.x[c] * dskg[c]));
+          const float y1 = __builtin_fmaf(h[c][3], o.cc.w, h[c][1] * o.cc.y);
+          *reinterpret_cast<float*>(yw + c * L::kYCh + par * L::kYBytes + slot * L::kYStep) = y0 + y1;
+        }
       }
     };
     __syncthreads();   // the first block is in place
@@ -421,9 +458,14 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kerne
       __syncthreads();
       fetch(next, 0, opsA);          // (behind the last block: what an earlier one left there, never used)
       step(opsB, 3, par ^ 1);
-      if constexpr (CKPT) { ckp += ck_step; }
+      if constexpr (CKPT) ckp += HALF ? 2 * ck_step : ck_step;
       par ^= 1;
       buf = next;
+    }
+    if constexpr (CKPT && HALF) {   // the state behind the last block: what the sweep's last step left is among it
+#pragma unroll
+      for (int c = 0; c < EC; ++c)
+        if (ch_ok) Snap<T>::store(ckp + c * (kN / 4 * kHB), h[c][0], h[c][1], h[c][2], h[c][3]);
     }
     __syncthreads();   // the last window
   } else {
@@ -502,10 +544,11 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kerne
       }
       rq = rq.moved(p, kCK);
     };
-    // y: wave 1 the steps 0 and 1 of a window, wave 2 the steps 2 and 3; lane (row, channel of four)
-    const int y_row = lane >> 2, y_ch = lane & 3;
+    // y: wave 1 the steps 0 and 1 of a window, wave 2 the steps 2 and 3; lane (row, channel of four), or (16 channels) (row, four channels)
+    const int y_row = lane >> 2, y_ch = (lane & 3) * (EC == 2 ? 4 : 1);
     Tr yq;                                                   // the lane's row at the first of the wave's steps in the window to be sent next
     yq.start(p, my_band, 2 * (sw - 1) - 1, y_row);
+    constexpr int kYStores = !WRITE_Y ? 0 : (EC == 2 ? 2 : 2 * (CW / 4));
     auto send_y = [&](int par, int steps) {                  // kYStores
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -513,15 +556,19 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kerne
         const int kw = 2 * (sw - 1) + i;                     // (uniform) step of the window
         const bool ok = t.on(p) && kw < steps;
         const uint32_t off = cell_bytes_off(t.cell, (uint32_t)p.E * (uint32_t)sizeof(T)) + (uint32_t)(e_wg0 + y_ch) * (uint32_t)sizeof(T);
+        auto share = [&](int c) {
+          const float4 s = *reinterpret_cast<const float4*>(lds + L::kY + par * L::kYBytes + kw * L::kYStep + c * L::kYCh + y_row * 16);
+          return (s.x + s.y) + (s.z + s.w);
+        };
+        if constexpr (EC == 2) {
+          split_store_quad(reinterpret_cast<T*>(Yimg + off), make_float4(share(y_ch), share(y_ch + 1), share(y_ch + 2), share(y_ch + 3)), ok && e_wg0 + y_ch < p.E);
+        } else {
 #pragma unroll
-        for (int j = 0; j < CW / 4; ++j) {
-          const float4 s = *reinterpret_cast<const float4*>(lds + L::kY + par * L::kYBytes + kw * L::kYStep + (4 * j + y_ch) * L::kYCh + y_row * 16);
-          split_store(reinterpret_cast<T*>(Yimg + off) + 4 * j, (s.x + s.y) + (s.z + s.w), ok && e_wg0 + 4 * j + y_ch < p.E);
+          for (int j = 0; j < CW / 4; ++j) split_store(reinterpret_cast<T*>(Yimg + off) + 4 * j, share(4 * j + y_ch), ok && e_wg0 + 4 * j + y_ch < p.E);
         }
       }
       yq = yq.moved(p, kCK);
     };
-    constexpr int kYStores = WRITE_Y ? 2 * (CW / 4) : 0;
 
     const int n = m_hi - m_lo;                               // blocks of the window
     // Rows of this workgroup's own previous band are sent and acknowledged two blocks before they are read back, if the stream's
