@@ -1980,7 +1980,7 @@ constexpr int bwd2_exchange_sets() {   // sets of [wave][3][64] float2: 2 halves
 // Workgroups of 16 channels: two waves share the 4 channels that a wave has otherwise, a half of the states each, both halves of a sub-block
 // at once, and 4 more waves stage, add up the channel sums, and add and store the two halves' shares of d_deltaT, d_deltaL, d_x.
 // (A workgroup has the compute unit to itself: with a wave per 4 channels every SIMD had a single sweeping wave, which issues a vector
-// instruction every 4 to 5 clocks where two take 2.5.  64 images of 56x56x64 bf16, 256 workgroups: 0.469 -> 0.371 ms.)
+// instruction every 4 to 5 clocks where two take 2.5.  64 images of 56x56x64 bf16, 256 workgroups: 0.469 -> 0.345 ms.)
 template <int NW>
 constexpr bool bwd2_halves() { return NW == kFwdHalfWaves; }
 template <int MODE, int NW>
@@ -2166,6 +2166,9 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
   auto sweep = [&](auto role) {
   constexpr int ROLE = decltype(role)::value;
   constexpr bool STAGES = ROLE != kSweeper, SWEEPS = ROLE != kStager;
+  // (HALVES: what the others wait for at the barriers goes first, and of the two that sweep on a SIMD the younger for the first part of a
+  // sub-block, see lead_if_younger: 64 images of 56x56x64 bf16 0.367 -> 0.345 ms; either without the other 1 to 2 %)
+  if constexpr (HALVES && ROLE == kStager) __builtin_amdgcn_s_setprio(3);
   for (int m = m_hi - 1; m >= 0; --m) {
     const int t0 = m * kCK;
     const char* bufc = lds + cur * SG::kBytes;
@@ -2218,7 +2221,7 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
         if (sub == 0 && pass == kLast) staging_landed();
        } else {
         float ha[8], hb1[8], hn[8], gT[8], gL[8];
-        lead_if_younger<NW>(wave, true);    // (until the second step of the adjoint below)
+        lead_if_younger<NSW>(wave, true);   // (until the second step of the adjoint below)
         widen8(qa[pass], ha);
         widen8(qn[pass], hn);
         qn[pass][0] = qa[pass][0]; qn[pass][1] = qa[pass][1];
@@ -2280,7 +2283,7 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
         for (int ks = 1; ks >= 0; --ks) {
           const int k = k0 + ks;
           const int t = t0 + k;
-          if (ks == 0) lead_if_younger<NW>(wave, false);
+          if (ks == 0) lead_if_younger<NSW>(wave, false);
           if (sub == 0 && pass == kLast && ks == 0) staging_landed();   // before the last stores of the block, see the forward kernel
           if (t < p.T_total) {
             const float (&hbk)[8] = ks == 1 ? hb1 : ha;    // the state before this step
@@ -2879,10 +2882,15 @@ Geometry make_geometry(const m2d_desc* d) {
       g.bwd_wpb = g.bwd_bpb * g.bwd_nw;
     }
   }
-  // The forward beside a backward in workgroups of 16 channels, one stream per image: 8 waves with two channels each and a quarter of
-  // the states per lane, which keep a SIMD busy where 4 waves that hold all states leave it to one (64 images of 56x56x64 bf16: forward
-  // 0.160 -> 0.133 ms, keeping snapshots 0.167 -> 0.140; with twice as many images, two rounds of either, they are level: 0.262 against 0.264).
-  if (!split && !g.stacked && !g.sliced && g.stage_x && g.fwd_nw == kFwdHalfWaves && g.ck_shift == 0 && !g.snap32 && !(d->flags & M2D_FLAG_WHOLE_STATES)) {
+  // The forward of one stream per image where rows are whole chunks: 8 waves with two channels each and a quarter of the states per
+  // lane.  Beside 4 waves that hold all states of 16 channels, which leave a SIMD to one wave each, they are ahead throughout (64 images of
+  // 56x56x64 bf16: 0.160 -> 0.127 ms, keeping snapshots 0.167 -> 0.131).  Beside 8 waves that hold all states of 32 channels they
+  // need two rounds for one, each with a start that takes as long as 3 blocks, and are ahead where a sweep is long (128 images of 56x56x64
+  // bf16, 60 blocks: 0.264 -> 0.255 ms, keeping snapshots 0.283 -> 0.263; 64 of 28x28x128, 18 blocks: 0.079 against 0.086).
+  const int64_t wg_pairs = (int64_t)B * ((d->E + 2 * kSplitWaves - 1) / (2 * kSplitWaves));
+  const bool pairs = g.fwd_nw == kFwdHalfWaves ||
+                     (g.fwd_ec == 1 && 208 * ((wg_pairs + ncu - 1) / ncu) * (nblk_stream + 3) < 440 * (((int64_t)B * g.fwd_bpb + ncu - 1) / ncu) * nblk_stream);
+  if (!split && !g.stacked && !g.sliced && g.stage_x && pairs && g.ck_shift == 0 && !g.snap32 && !(d->flags & M2D_FLAG_WHOLE_STATES)) {
     g.fwd_split = true;
     g.fwd_ec = 2;
     g.fwd_nw = kSplitWaves;
