@@ -2987,7 +2987,7 @@ int launch_prep(ScanParams& sp, const m2d_desc* d, const Geometry& g, float* bas
   float* A2L = A2T + (size_t)d->E * kN;
   float* Df = A2L + (size_t)d->E * kN;
   sp.zeros = zeros; sp.A2T = A2T; sp.A2L = A2L; sp.Df = Df;
-  if (ready && n_link == 0) return M2D_OK;   // the forward of this problem filled the area, and there is nothing to clear
+  if (ready && n_link == 0) return M2D_OK;   // the forward of this problem fills or has filled the area, and there is nothing to clear
   const int n = d->E * kN > kZeroFloats ? d->E * kN : kZeroFloats;
   hipLaunchKernelGGL(m2d_prep_kernel<T>, dim3((n + 255) / 256), dim3(256), 0, st, sp, zeros, A2T, A2L, Df, link_words, n_link);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
@@ -3158,7 +3158,9 @@ int run_fwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
   sp.top = reinterpret_cast<float*>(keep);
   if (ckpt) prep = reinterpret_cast<float*>(keep + g.top_bytes + g.bc_bytes);   // kept for the backward
   sp.AT = AT; sp.AL = AL; sp.D = D;
-  int rc = g.fwd_split && !ckpt && !g.sliced ? zero_page(&sp.zeros) : launch_prep<T>(sp, d, g, prep, link_words, st);   // (split_owns_setup)
+  const bool own = g.fwd_split && !g.sliced;   // (split_owns_setup)
+  int rc = launch_prep<T>(sp, d, g, prep, link_words, st, own);
+  if (!rc && own) rc = zero_page(&sp.zeros);   // (the area's own zeros are being written by this launch)
   if (rc) return rc;
   if ((!ckpt || sizeof(T) == 2) && !g.packed_bc) {   // the kernel takes the tensors as they are (fp32: only where no backward will want the packed copy)
     sp.bcd[0] = BT; sp.bcd[1] = BL; sp.bcd[2] = C; sp.bcd[3] = BT;

@@ -42,11 +42,11 @@ template <typename T>
 __device__ __forceinline__ float skip_gain(const ScanParams& p, int e) {
   return p.raw ? as_stored(static_cast<const float*>(p.D)[e], static_cast<const T*>(nullptr)) : IO<T>::ld(static_cast<const T*>(p.D) + e);
 }
-// The set-up launch (m2d_prep_kernel) is for kernels whose lanes hold all states of a channel, for a backward that will
-// read the same values, and for progress counts.  A lane here holds 4 states of one channel, so a forward with neither
-// works them out itself and saves the launch and the gap behind it.
-template <bool CKPT, int MODE>
-constexpr bool split_owns_setup() { return !CKPT && MODE != kModeSliced; }
+// The set-up launch (m2d_prep_kernel) is for kernels whose lanes hold all states of a channel, and for progress counts.  A lane
+// here holds 4 states of a channel or two, so a forward of one stream per image works its own out and saves the launch and the gap
+// behind it (4.7 us); where it keeps snapshots, the workgroups of the first image leave the area as a backward will want it.
+template <int MODE>
+constexpr bool split_owns_setup() { return MODE != kModeSliced; }
 __device__ float m2d_zero_page[kZeroFloats];     // the page of zeros of such a forward: never written
 
 // ------------------------------------------------------------------------------ operands in LDS
@@ -323,7 +323,7 @@ template <typename T, bool CKPT, bool WRITE_Y, bool SX, int MODE, int NW = kSpli
 __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kernel(const ScanParams pin) {
   static_assert(MODE != kModeStacked, "stacked images are many: they never need the split");
   constexpr bool SLICED = MODE == kModeSliced;
-  constexpr bool OWN_SETUP = split_owns_setup<CKPT, MODE>();
+  constexpr bool OWN_SETUP = split_owns_setup<MODE>();
   constexpr bool WIDEN = sizeof(T) == 2;
   constexpr int CW = NW * EC;
   static_assert(EC == 1 || (EC == 2 && SX && NW == kSplitWaves && !SLICED), "two channels a wave: rows of whole chunks, one stream per image");
@@ -376,6 +376,24 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kerne
       dskg[c] = g == 0 ? (OWN_SETUP ? skip_gain<T>(p, e0 + c) : p.Df[e0 + c]) : 0.f;   // (x * D is in the share of group 0)
     }
     static_assert(sinv<true>(1) == 8 && sinv<true>(6) == 5 && sinv<true>(15) == 15, "fold order");
+    if constexpr (OWN_SETUP && CKPT) {   // the area that m2d_prep_kernel fills for others: [zeros][A2T][A2L][D]
+      if (b == 0 && ch_ok && r == 0) {
+        float* A2T = const_cast<float*>(p.A2T);
+        float* A2L = const_cast<float*>(p.A2L);
+#pragma unroll
+        for (int c = 0; c < EC; ++c) {
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {   // (a forward that keeps snapshots has the states in fold order)
+            const int n = (e0 + c) * kN + (w == 1 ? 2 : (w == 2 ? 1 : w)) * 4 + g;
+            A2T[n] = a2t[c][w];
+            A2L[n] = a2l[c][w];
+          }
+          if (g == 0) const_cast<float*>(p.Df)[e0 + c] = dskg[c];
+        }
+      }
+      static_assert(kZeroFloats == 64, "a lane each");
+      if (b == 0 && e_wg0 == 0 && wave == 0) const_cast<float*>(p.A2T)[lane - kZeroFloats] = 0.f;
+    }
     const float g1 = r == 0 ? 1.f : 0.f;                    // the ghost's T input coefficient
     // a grid row reads its own B_T; the ghost (lane 0) the row above as its B_T, and zeros as its B_L and C
     const uint32_t bt_off = r == 0 ? SG::row_off(SG::kTop, ch, g) : SG::bc_off(0, g, r);
