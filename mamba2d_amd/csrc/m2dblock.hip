@@ -418,14 +418,17 @@ int run_rope(const RopeArgs& a, int G, hipStream_t st) {
 // the pointwise convolutions of the local path and the MLP at 64 or 128 channels
 // (models/mamba2d.py:166-176, models/utils.py:58-81, 87-118).  These products are bandwidth-bound: a row
 // of x is 128 to 512 bytes and is used once.  The weight matrix lives in LDS as bf16 for the whole
-// (persistent) workgroup; a wave owns 16 rows, whose 16-byte pieces are the A operands of
+// (persistent) workgroup; a wave owns 16 rows, whose 16-byte pieces are the second operands of
 // v_mfma_f32_16x16x32_bf16 as they come from memory (lane l: row l & 15, columns 8 (l >> 4) + j of a step
-// of 32), W's rows are the B operands (lane l: output l & 15, the same columns), results leave through a
-// per-wave LDS block so that memory sees 16-byte pieces of rows.  pre and post are nothing, GELU (exact
-// form) or StarReLU: the activation that the block applies before or after the layer.
+// of 32), W's rows are the first operands (lane l: output l & 15, the same columns), so that a lane ends with
+// four neighbouring outputs of a row and, after an exchange with a neighbour, stores 16 bytes.  pre and post are
+// nothing, GELU (exact form) or StarReLU: the activation that the block applies before or after the layer.
+// A workgroup sees few tiles, so the waits count: per launch (batch of 128, 64 to 256 inputs), with a load in a branch
+// for every step of 32, a read of the bias per tile and the results through a block in LDS, 43, 38 and 44 us for up to
+// 64, 128 and 256 inputs; with loads and bias ahead of the tiles 33, 36 and 40; with the results stored from registers, and as
+// many workgroups as registers allow, 32, 35 and 34 (x and y at the rate of a copy: 10 to 20).
 constexpr int kLinThreads = 256;
-constexpr int kLinWaves = 4;
-constexpr int kLinStage = 72;      // floats per row of a wave's result block: 64 + 8
+constexpr int kLinMargin = 18 * 1024;   // bytes of LDS that the choice of slices leaves free
 constexpr int kLinMaxKC = 16;      // steps of 32 along K: K <= 512
 enum { kActNone = 0, kActGelu = 1, kActStarRelu = 2, kActLayerNorm = 3 };   // the last one only before the layer, and only inside this file
 
@@ -529,45 +532,66 @@ struct LinArgs {
   void* z;              // (P, N) bf16 or null: the layer's output before post, for a caller whose backward wants its slope
 };
 
+// a and b hold 4 values each of two tiles of 16 in lane row kb (the lane's number / 16).  Rows 0 and 2 end with a's values of
+// rows kb and kb + 1, rows 1 and 3 with b's of rows kb - 1 and kb.
+__device__ __forceinline__ uint4 halves_exchanged(const uint2 a, const uint2 b) {
+  const auto x = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false), y = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
+  return make_uint4(x[0], y[0], x[1], y[1]);
+}
+
+constexpr int lin_per_cu(int kcmax) { return kcmax <= 2 ? 6 : kcmax <= 8 ? 4 : 2; }   // workgroups whose registers fit a compute unit
+
 template <int KCMAX>   // steps of 32 along K that the kernel is built for: 2, 4, 8 or 16
-__global__ __launch_bounds__(kLinThreads) void m2d_linear_kernel(const LinArgs a) {
+__global__ __launch_bounds__(kLinThreads, lin_per_cu(KCMAX)) void m2d_linear_kernel(const LinArgs a) {
   extern __shared__ float smem[];
   const int tid = threadIdx.x, l = tid & 63, mn = l & 15, kb = l >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ws = a.K + 8;                                // bf16 per row of W in LDS: rows stay 16-byte aligned and spread over the banks
   uint16_t* wl = reinterpret_cast<uint16_t*>(smem);
-  float* stage = smem + (a.Ns * ws / 2 + 3) / 4 * 4 + wave * 16 * kLinStage;
-  const int slice = blockIdx.x % a.nsplit, nbase = slice * a.Ns;   // this workgroup's outputs: nbase .. nbase + Ns
-  const int first_tile = blockIdx.x / a.nsplit, tile_step = gridDim.x / a.nsplit;
+  float* bias = smem + (a.Ns * ws / 2 + 3) / 4 * 4;
+  float* lnp = bias + a.Ns;
+  // Workgroups go to the 8 XCDs in turn: the slices of a tile follow each other on one XCD, so that its L2 fetches the rows
+  // of x once for all of them.
+  const int j = blockIdx.x / 8;
+  const int slice = j % a.nsplit, nbase = slice * a.Ns;   // this workgroup's outputs: nbase .. nbase + Ns
+  const int first_tile = j / a.nsplit * 8 + blockIdx.x % 8, tile_step = gridDim.x / a.nsplit;
+  if (first_tile >= a.ntiles) return;      // (the whole workgroup: the grid is rounded up to whole eights)
   const int kp = a.K / 8, pieces = a.Ns * kp;
-  stage_rows(a.w, a.wbf16, (int64_t)nbase * a.K, pieces, tid, [&](int i, const uint4& q) {
-    const int n = i / kp;
-    *reinterpret_cast<uint4*>(wl + n * ws + 8 * (i - n * kp)) = q;
-  });
-  float* lnp = smem + (a.Ns * ws / 2 + 3) / 4 * 4 + kLinWaves * 16 * kLinStage;      // behind the waves' result blocks
-  if (a.pre == kActLayerNorm)
-    for (int i = tid; i < a.K; i += kLinThreads) { lnp[i] = ldw(a.ln_w, a.wbf16, i); lnp[a.K + i] = ldw(a.ln_b, a.wbf16, i); }
-  __syncthreads();
-  const float pre_s = a.pre == kActStarRelu ? ldw(a.pre_s, a.wbf16, 0) : 0.f, pre_b = a.pre == kActStarRelu ? ldw(a.pre_b, a.wbf16, 0) : 0.f;
-  const float post_s = a.post == kActStarRelu ? ldw(a.post_s, a.wbf16, 0) : 0.f, post_b = a.post == kActStarRelu ? ldw(a.post_b, a.wbf16, 0) : 0.f;
   const int KC = a.K / 32;
   const uint16_t* X = static_cast<const uint16_t*>(a.x);
   uint16_t* Y = static_cast<uint16_t*>(a.y);
   // The rows of the next tile are fetched while the current one is worked on: with the weights in LDS
-  // few waves fit a compute unit, too few to cover the latency of memory by themselves.
+  // few waves fit a compute unit, too few to cover the latency of memory by themselves.  Rows past the end repeat the last
+  // one and are not stored, steps past K repeat the last one and are not used: a load in a branch is waited for at the
+  // branch's end, which made one wait per step of a tile's rows instead of none.
   uint4 Anext[KCMAX];
   auto fetch = [&](int tile) {
-    const int64_t q0 = (int64_t)tile * 64 + wave * 16;
+    const int64_t q = (int64_t)tile * 64 + wave * 16 + mn;
+    const uint16_t* row = X + (q < a.P ? q : a.P - 1) * a.K + 8 * kb;
 #pragma unroll
-    for (int kc = 0; kc < KCMAX; ++kc) {
-      Anext[kc] = make_uint4(0u, 0u, 0u, 0u);
-      if (kc < KC && tile < a.ntiles && q0 + mn < a.P) Anext[kc] = ld16(X + (q0 + mn) * a.K + 32 * kc + 8 * kb);
-    }
+    for (int kc = 0; kc < KCMAX; ++kc) Anext[kc] = ld16(row + 32 * (kc < KC ? kc : KC - 1));
   };
+  // Everything a workgroup reads once is on its way before the first of it is waited for.
   fetch(first_tile);
-  for (int tile = first_tile; tile < a.ntiles; tile += tile_step) {
-    const int64_t p0 = (int64_t)tile * 64 + wave * 16;
-    const int rows = (int)(a.P - p0 < 16 ? a.P - p0 : 16);     // rows of the wave inside the array (may be <= 0)
+  const int tn = tid < a.Ns ? tid : a.Ns - 1, tk = tid < a.K ? tid : a.K - 1;
+  const float bias0 = a.bias ? ldw(a.bias, a.wbf16, nbase + tn) : 0.f;
+  const float lnw0 = a.pre == kActLayerNorm ? ldw(a.ln_w, a.wbf16, tk) : 0.f, lnb0 = a.pre == kActLayerNorm ? ldw(a.ln_b, a.wbf16, tk) : 0.f;
+  const float pre_s = a.pre == kActStarRelu ? ldw(a.pre_s, a.wbf16, 0) : 0.f, pre_b = a.pre == kActStarRelu ? ldw(a.pre_b, a.wbf16, 0) : 0.f;
+  const float post_s = a.post == kActStarRelu ? ldw(a.post_s, a.wbf16, 0) : 0.f, post_b = a.post == kActStarRelu ? ldw(a.post_b, a.wbf16, 0) : 0.f;
+  stage_rows(a.w, a.wbf16, (int64_t)nbase * a.K, pieces, tid, [&](int i, const uint4& q) {
+    const int n = i / kp;
+    *reinterpret_cast<uint4*>(wl + n * ws + 8 * (i - n * kp)) = q;
+  });
+  // (read from memory at every tile, the bias's wait was one for the next tile's rows too: they are counted in order)
+  if (tid < a.Ns) bias[tid] = bias0;
+  for (int i = tid + kLinThreads; i < a.Ns; i += kLinThreads) bias[i] = a.bias ? ldw(a.bias, a.wbf16, nbase + i) : 0.f;
+  if (a.pre == kActLayerNorm && tid < a.K) { lnp[tid] = lnw0; lnp[a.K + tid] = lnb0; }      // (K <= 128)
+  __syncthreads();
+  // A wave's tiles end at the last row.  Its lanes past that row hold and store the row's own values once more, so no store
+  // sits in a branch and the wait for the next tile's rows leaves the stores behind them under way.
+  for (int tile = first_tile; (int64_t)tile * 64 + wave * 16 < a.P; tile += tile_step) {
+    const int64_t p = (int64_t)tile * 64 + wave * 16 + mn;
+    const int64_t out = (p < a.P ? p : a.P - 1) * a.N + nbase;
     uint4 A[KCMAX];
 #pragma unroll
     for (int kc = 0; kc < KCMAX; ++kc) A[kc] = Anext[kc];
@@ -585,45 +609,32 @@ __global__ __launch_bounds__(kLinThreads) void m2d_linear_kernel(const LinArgs a
           A[kc] = make_uint4(w4[0], w4[1], w4[2], w4[3]);
         }
     }
-    for (int n0 = 0; n0 < a.Ns; n0 += 64) {
+    // W's rows are the first operand: lane (mn, kb) ends with outputs 4 kb + i of position mn.  Two tiles of 16 outputs at a time;
+    // lanes of neighbouring kb exchange halves and store 8 neighbouring outputs each.  An odd last tile is taken twice.
+    for (int n0 = 0; n0 < a.Ns; n0 += 32) {
+      const int second = n0 + 16 < a.Ns ? 16 : 0;
+      uint2 zq[2], yq[2];
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int n = n0 + 16 * nt + mn;
+      for (int t = 0; t < 2; ++t) {
+        const int nt = n0 + (t ? second : 0);
+        const uint16_t* wrow = wl + (nt + mn) * ws + 8 * kb;
         f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-        if (n0 + 16 * nt < a.Ns) {   // (uniform)
-          const uint16_t* wrow = wl + n * ws + 8 * kb;
 #pragma unroll
-          for (int kc = 0; kc < KCMAX; ++kc)
-            if (kc < KC) acc = mfma_bf16(A[kc], ld16(wrow + 32 * kc), acc);
-          const float bn = a.bias ? ldw(a.bias, a.wbf16, nbase + n) : 0.f;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] = a.z ? acc[i] + bn : act(a.post, acc[i] + bn, post_s, post_b);
+        for (int kc = 0; kc < KCMAX; ++kc)
+          if (kc < KC) acc = mfma_bf16(ld16(wrow + 32 * kc), A[kc], acc);
+        const float4 bn = *reinterpret_cast<const float4*>(bias + nt + 4 * kb);
+        acc[0] += bn.x; acc[1] += bn.y; acc[2] += bn.z; acc[3] += bn.w;
+        if (a.z) {   // (uniform) both values leave; the activation reads what is stored, as the backward will
+          zq[t] = make_uint2(pack_bf16(acc[0], acc[1]), pack_bf16(acc[2], acc[3]));
+          acc[0] = bf_lo(zq[t].x); acc[1] = bf_hi(zq[t].x); acc[2] = bf_lo(zq[t].y); acc[3] = bf_hi(zq[t].y);
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) stage[(4 * kb + i) * kLinStage + 16 * nt + mn] = acc[i];   // position 4 kb + i, output 16 nt + mn
+        for (int i = 0; i < 4; ++i) acc[i] = act(a.post, acc[i], post_s, post_b);
+        yq[t] = make_uint2(pack_bf16(acc[0], acc[1]), pack_bf16(acc[2], acc[3]));
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {   // the block's 16 x 8 pieces of 8 outputs, two per lane
-        const int piece = l + 64 * k, c = piece >> 3, c8 = 8 * (piece & 7);
-        if (c < rows && n0 + c8 < a.Ns) {
-          float4 lo = *reinterpret_cast<const float4*>(stage + c * kLinStage + c8);
-          float4 hi = *reinterpret_cast<const float4*>(stage + c * kLinStage + c8 + 4);
-          if (a.z) {   // (uniform) both values leave; the activation reads what is stored, as the backward will
-            const uint4 q = make_uint4(pack_bf16(lo.x, lo.y), pack_bf16(lo.z, lo.w), pack_bf16(hi.x, hi.y), pack_bf16(hi.z, hi.w));
-            *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.z) + (p0 + c) * a.N + nbase + n0 + c8) = q;
-            lo = make_float4(act(a.post, bf_lo(q.x), post_s, post_b), act(a.post, bf_hi(q.x), post_s, post_b),
-                             act(a.post, bf_lo(q.y), post_s, post_b), act(a.post, bf_hi(q.y), post_s, post_b));
-            hi = make_float4(act(a.post, bf_lo(q.z), post_s, post_b), act(a.post, bf_hi(q.z), post_s, post_b),
-                             act(a.post, bf_lo(q.w), post_s, post_b), act(a.post, bf_hi(q.w), post_s, post_b));
-          }
-          *reinterpret_cast<uint4*>(Y + (p0 + c) * a.N + nbase + n0 + c8) =
-              make_uint4(pack_bf16(lo.x, lo.y), pack_bf16(lo.z, lo.w), pack_bf16(hi.x, hi.y), pack_bf16(hi.z, hi.w));
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const int64_t at = out + n0 + (kb & 1 ? second : 0) + 4 * (kb & 2);
+      if (a.z) *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.z) + at) = halves_exchanged(zq[0], zq[1]);
+      *reinterpret_cast<uint4*>(Y + at) = halves_exchanged(yq[0], yq[1]);
     }
   }
 }
@@ -869,31 +880,32 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
       d[1] = make_uint2(q.z, q.w);
     });
   };
-  stage_weights(a.w1, HD, C, w1l, W1S);
-  stage_weights(a.w2, C, HD, w2l, W2S);
-  for (int i = tid; i < HD; i += kLinThreads) b1l[i] = a.b1 ? ldw(a.b1, a.wbf16, i) : 0.f;
-  float* lnp = b1l + HD;
-  if (a.ln_w)
-    for (int i = tid; i < C; i += kLinThreads) { lnp[i] = ldw(a.ln_w, a.wbf16, i); lnp[C + i] = ldw(a.ln_b, a.wbf16, i); }
+  const uint16_t* X = static_cast<const uint16_t*>(a.x);
+  uint16_t* Y = static_cast<uint16_t*>(a.y);
+  uint4 Xnext[KC];
+  auto fetch = [&](int tile) {      // (rows past the end repeat the last one, see m2d_linear_kernel)
+    const int64_t q = (int64_t)tile * 64 + wave * 16 + mn;
+    const uint16_t* row = X + (q < a.P ? q : a.P - 1) * C + 8 * kb;
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) Xnext[kc] = ld16(row + 32 * kc);
+  };
+  static_assert(HD <= kLinThreads, "one hidden unit's bias a thread");
+  fetch(blockIdx.x);
+  const int th = tid < HD ? tid : HD - 1, tc = tid < C ? tid : C - 1;
+  const float b10 = a.b1 ? ldw(a.b1, a.wbf16, th) : 0.f;
+  const float lnw0 = a.ln_w ? ldw(a.ln_w, a.wbf16, tc) : 0.f, lnb0 = a.ln_w ? ldw(a.ln_b, a.wbf16, tc) : 0.f;
   float b2v[NO][4];
 #pragma unroll
   for (int no = 0; no < NO; ++no)
 #pragma unroll
     for (int i = 0; i < 4; ++i) b2v[no][i] = a.b2 ? ldw(a.b2, a.wbf16, 16 * no + 4 * kb + i) : 0.f;
+  stage_weights(a.w1, HD, C, w1l, W1S);
+  stage_weights(a.w2, C, HD, w2l, W2S);
+  if (tid < HD) b1l[tid] = b10;
+  float* lnp = b1l + HD;
+  if (a.ln_w && tid < C) { lnp[tid] = lnw0; lnp[C + tid] = lnb0; }
   __syncthreads();
-  const uint16_t* X = static_cast<const uint16_t*>(a.x);
-  uint16_t* Y = static_cast<uint16_t*>(a.y);
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  uint4 Xnext[KC];
-  auto fetch = [&](int tile) {
-    const int64_t q0 = (int64_t)tile * 64 + wave * 16;
-#pragma unroll
-    for (int kc = 0; kc < KC; ++kc) {
-      Xnext[kc] = make_uint4(0u, 0u, 0u, 0u);
-      if (tile < a.ntiles && q0 + mn < a.P) Xnext[kc] = ld16(X + (q0 + mn) * C + 32 * kc + 8 * kb);
-    }
-  };
-  fetch(blockIdx.x);
   for (int tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
     const int64_t p0 = (int64_t)tile * 64 + wave * 16;
     uint4 Xf[KC];
@@ -955,8 +967,13 @@ inline bool allow_big_lds() {
   return true;
 }
 
-inline size_t linear_lds_bytes(int K, int N, bool ln = false) {
-  return ((size_t)N * (K + 8) / 2 + 3) / 4 * 4 * 4 + (size_t)kLinWaves * 16 * kLinStage * 4 + (ln ? (size_t)2 * K * 4 : 0);
+// LDS of the kernel: the slice of W, its bias, the normalisation's weight and bias.
+inline size_t linear_lds_bytes(int K, int N, bool ln) {
+  return ((size_t)N * (K + 8) / 2 + 3) / 4 * 4 * 4 + (size_t)N * 4 + (ln ? (size_t)2 * K * 4 : 0);
+}
+// What the choice of slices and the limit of what is taken count with.
+inline size_t linear_slice_bytes(int K, int N, bool ln) {
+  return ((size_t)N * (K + 8) / 2 + 3) / 4 * 4 * 4 + kLinMargin + (ln ? (size_t)2 * K * 4 : 0);
 }
 
 // ------------------------------------------ attention of the rotary stages, one head per workgroup
@@ -1386,9 +1403,9 @@ static int run_linear(int64_t P, int K, int N, int weight_dtype, const void* x, 
   // Slices of the outputs, so that a workgroup's share of the weights leaves room for four workgroups on a
   // compute unit (each slice reads the rows of x again; they are the smaller side where N is large).
   int nsplit = 1;
-  while (linear_lds_bytes(K, N / nsplit, ln) > 40 * 1024 && (N / nsplit) % 32 == 0 && N / nsplit > 64) nsplit *= 2;
+  while (linear_slice_bytes(K, N / nsplit, ln) > 40 * 1024 && (N / nsplit) % 32 == 0 && N / nsplit > 64) nsplit *= 2;
   const int Ns = N / nsplit;
-  if (linear_lds_bytes(K, Ns, ln) > kLinMaxLds) return M2D_ERR_UNSUPPORTED;
+  if (linear_slice_bytes(K, Ns, ln) > kLinMaxLds) return M2D_ERR_UNSUPPORTED;
   if ((P + 63) / 64 >= ((int64_t)1 << 31)) return M2D_ERR_UNSUPPORTED;
   if (misaligned(x, 16) || misaligned(y, 16) || misaligned(weight, 16) || (bias && misaligned(bias, 4))) return M2D_ERR_MISALIGNED;
   if (ln && (misaligned(ln_w, 4) || misaligned(ln_b, 4))) return M2D_ERR_MISALIGNED;
@@ -1402,10 +1419,12 @@ static int run_linear(int64_t P, int K, int N, int weight_dtype, const void* x, 
   if (lds > 64 * 1024 && !allow_big_lds()) return M2D_ERR_HIP;
   // persistent: the weights are loaded into LDS once per workgroup; as many workgroups as fit the device at once
   int per_cu = (int)(160 * 1024 / lds);
-  if (per_cu > 8) per_cu = 8;
+  const int most = lin_per_cu(K <= 64 ? 2 : K <= 128 ? 4 : K <= 256 ? 8 : 16);
+  if (per_cu > most) per_cu = most;
   int grid = 256 * per_cu / nsplit;     // workgroups per slice
-  if (grid > a.ntiles) grid = a.ntiles;
-  if (grid < 1) grid = 1;
+  grid = grid / 8 * 8;
+  if (grid > a.ntiles) grid = (a.ntiles + 7) / 8 * 8;
+  if (grid < 8) grid = 8;
   grid *= nsplit;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 g((unsigned)grid), t(kLinThreads);
