@@ -189,7 +189,8 @@ int m2d_scan_plan(const m2d_desc* desc, int pass, char* text, size_t cap);
  * torch.empty.  The scratch that m2d_scan_fwd takes as `workspace` lives in a static device array
  * of M2D_NOALLOC_SCRATCH_BYTES inside the library (each GPU the library runs on holds one copy until
  * the process ends); the call allocates and frees nothing.  A problem whose
- * m2d_scan_workspace_bytes(desc, M2D_PASS_FWD, 0) exceeds that size is rejected with
+ * m2d_scan_workspace_bytes(desc, M2D_PASS_FWD, 0) exceeds that size runs as with M2D_FLAG_WHOLE_STATES, which needs the
+ * least scratch; one that is too large that way as well is rejected with
  * M2D_ERR_TOO_LARGE before anything is launched (this check comes first: a call with NULL tensors on
  * a problem that is too large reports M2D_ERR_TOO_LARGE).  All calls on one GPU share the array: two calls
  * that overlap on one GPU (different streams or threads) race; calls on one stream are ordered.  Besides

@@ -3502,7 +3502,13 @@ int m2d_scan_fwd_noalloc(const m2d_desc* desc, const void* x, const void* deltaT
                          void* stream) {
   int rc = check_desc(desc);
   if (rc) return rc;
-  if (workspace_bytes_of(make_geometry(desc), M2D_PASS_FWD, 0) > (size_t)M2D_NOALLOC_SCRATCH_BYTES) return M2D_ERR_TOO_LARGE;
+  // A linked sweep keeps a progress count of 256 bytes per band and workgroup, and split states have four to eight times the
+  // workgroups: where those counts are what does not fit, the problem runs with whole states.
+  m2d_desc fits = *desc;
+  if (workspace_bytes_of(make_geometry(&fits), M2D_PASS_FWD, 0) > (size_t)M2D_NOALLOC_SCRATCH_BYTES) {
+    fits.flags = (fits.flags & ~M2D_FLAG_SPLIT_STATES) | M2D_FLAG_WHOLE_STATES;
+    if (workspace_bytes_of(make_geometry(&fits), M2D_PASS_FWD, 0) > (size_t)M2D_NOALLOC_SCRATCH_BYTES) return M2D_ERR_TOO_LARGE;
+  }
   // address of the current device's copy of the array, looked up once per device
   static std::atomic<void*> addr[64];
   int dev = 0;
@@ -3514,7 +3520,7 @@ int m2d_scan_fwd_noalloc(const m2d_desc* desc, const void* x, const void* deltaT
   }
   // nothing in the workspace has to be zero on entry: the set-up kernel rewrites the page of zeros,
   // boundary rows and carried state are written before they are read
-  return m2d_scan_fwd(desc, x, deltaT, deltaL, AT, AL, BT, BL, C, D, y, nullptr, 0, ws, (size_t)M2D_NOALLOC_SCRATCH_BYTES, stream);
+  return m2d_scan_fwd(&fits, x, deltaT, deltaL, AT, AL, BT, BL, C, D, y, nullptr, 0, ws, (size_t)M2D_NOALLOC_SCRATCH_BYTES, stream);
 }
 
 }  // extern "C"

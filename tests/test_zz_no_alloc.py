@@ -60,3 +60,36 @@ def test_too_large_is_rejected_before_any_launch():
     rc = cabi.lib.m2d_scan_fwd_noalloc(ctypes.byref(d), *([vp(4096)] * 10), vp(0))
     assert rc == cabi.M2D_ERR_TOO_LARGE
     assert "M2D_NOALLOC_SCRATCH_BYTES" in cabi.status_str(rc)
+
+
+# Problems whose own plan (linked sweeps of split states) needs more than the array and whose plan of whole states does not.
+FIT_AS_WHOLE = [(24, 69, 123, 44, torch.bfloat16), (52, 42, 24, 144, torch.float32), (35, 627, 2, 123, torch.bfloat16), (74, 986, 20, 5, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("B,H,W,E,dtype", FIT_AS_WHOLE)
+def test_a_problem_that_fits_with_whole_states_is_taken(B, H, W, E, dtype):
+    """Host only: the output is misaligned, so that nothing is launched where there is a GPU; the check of the size comes first."""
+    from mamba2d_amd import cabi
+    kind = cabi.M2D_F32 if dtype == torch.float32 else cabi.M2D_BF16
+    whole = cabi.Desc(B, H, W, E, 16, kind, cabi.M2D_FLAG_WHOLE_STATES, 0)
+    assert cabi.lib.m2d_scan_workspace_bytes(ctypes.byref(whole), cabi.M2D_PASS_FWD, 0) <= cabi.NOALLOC_SCRATCH_BYTES
+    for flags in (0, cabi.M2D_FLAG_SPLIT_STATES, cabi.M2D_FLAG_WHOLE_STATES):
+        d = cabi.Desc(B, H, W, E, 16, kind, flags, 0)
+        rc = cabi.lib.m2d_scan_fwd_noalloc(ctypes.byref(d), *([ctypes.c_void_p(4096)] * 9), ctypes.c_void_p(4100), ctypes.c_void_p(0))
+        assert rc != cabi.M2D_ERR_TOO_LARGE, (flags, cabi.status_str(rc))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,W,E,dtype", [FIT_AS_WHOLE[0], FIT_AS_WHOLE[1], FIT_AS_WHOLE[3]])
+def test_values_of_a_problem_that_fits_with_whole_states(B, H, W, E, dtype):
+    """The same sums in another order: fp32 to rounding; bf16 outputs differ by at most one rounding of the result (2^-8 of a value)
+    and of the largest for sums that cancel."""
+    from mamba2d_amd import cabi
+    say(f"\ncase no_alloc as whole B={B} H={H} W={W} E={E} dtype={dtype}")
+    inp = so.make_inputs(B, H, W, E, 16, seed=21, dtype=dtype)
+    a = [inp[k].cuda() for k in so.INPUT_NAMES]
+    want = cabi.scan_fwd(*a).float()
+    y = torch.full_like(a[0], float("nan"))
+    cabi.scan_fwd_noalloc(*a, y)
+    torch.cuda.synchronize()
+    assert so.rel_err(y.float().cpu(), want.cpu()) < (1e-5 if dtype == torch.float32 else 2 ** -8)
