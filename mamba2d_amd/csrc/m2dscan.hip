@@ -2671,7 +2671,7 @@ struct Geometry {
   bool stacked;                      // images of one band stacked into tall images of independent bands
   int ips, vB, vH;                   // images per stack; number and height of what the kernels sweep
   int nbb;                           // linked sweep: blocks per band
-  size_t link_bytes;                 // linked sweep: error word and the two arrays of progress counts (forward, backward)
+  size_t link_fwd_bytes, link_bytes; // linked sweep: error word and the forward's progress counts; these and the backward's
   int ck_shift, ck_pb, ck_nblk;      // checkpoint interval: log2 of the blocks per kept snapshot; kept snapshots per band (linked sweep) and per image
   bool ck_half;                      // a snapshot every 2 steps: m2d_fwd_kernel<..., HALF> and m2d_bwd2_kernel
   bool snap32;                       // bf16 tensors with fp32 snapshots (M2D_FLAG_FP32_SNAPSHOTS)
@@ -2922,6 +2922,7 @@ Geometry make_geometry(const m2d_desc* d) {
   g.top_bytes = rows ? align_up(sizeof(float) * (size_t)(g.nbands - 1) * B * d->W * d->E * kN) : 0;
   g.bot_bytes = rows ? align_up(sizeof(float) * (size_t)(g.sliced ? g.nbands : 1) * B * d->W * d->E * kN) : 0;
   const size_t chains = (size_t)B * (g.fwd_bpb > g.bwd_bpb ? g.fwd_bpb : g.bwd_bpb);
+  g.link_fwd_bytes = g.sliced ? align_up(sizeof(uint32_t) * (64 + (size_t)g.nbands * B * g.fwd_bpb * kLinkStride)) : 0;
   g.link_bytes = g.sliced ? align_up(sizeof(uint32_t) * (64 + 2 * g.nbands * chains * kLinkStride)) : 0;
   g.part_bytes = align_up(sizeof(float) * (size_t)g.bwd_bpb * 3 * P * kN);
   const size_t slots = g.sliced ? g.nbands : 1;
@@ -2936,7 +2937,7 @@ Geometry make_geometry(const m2d_desc* d) {
 size_t ckpt_bytes_of(const Geometry& g) { return g.ckpt_diag_bytes + g.top_bytes + g.bc_bytes + g.prep_bytes; }
 
 size_t workspace_bytes_of(const Geometry& g, int pass, int have_ckpt) {
-  size_t n = g.prep_bytes + g.link_bytes;
+  size_t n = g.prep_bytes + (pass == M2D_PASS_FWD ? g.link_fwd_bytes : g.link_bytes);
   if (pass == M2D_PASS_FWD) {
     if (!have_ckpt) n += g.top_bytes + g.bc_bytes;
   } else {
@@ -2979,8 +2980,8 @@ inline bool allow_dynamic_lds(const void* kernel, size_t bytes, std::atomic<uint
 
 // Set-up area: [page of zeros][A_T*log2e][A_L*log2e][D], all fp32.
 template <typename T>
-int launch_prep(ScanParams& sp, const m2d_desc* d, const Geometry& g, float* base, uint32_t* link_words, hipStream_t st, bool ready = false) {
-  const int n_link = (int)(g.link_bytes / sizeof(uint32_t));
+int launch_prep(ScanParams& sp, const m2d_desc* d, const Geometry& g, float* base, uint32_t* link_words, size_t link_bytes, hipStream_t st, bool ready = false) {
+  const int n_link = (int)(link_bytes / sizeof(uint32_t));
   sp.link_err = link_words;   // (the first 64 words: the error word; then forward counts, then backward counts)
   float* zeros = base;
   float* A2T = base + kZeroFloats;
@@ -3152,14 +3153,14 @@ int run_fwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
   char* w = static_cast<char*>(ws);
   float* prep = reinterpret_cast<float*>(w);
   w += g.prep_bytes;
-  uint32_t* link_words = reinterpret_cast<uint32_t*>(w); w += g.link_bytes;
+  uint32_t* link_words = reinterpret_cast<uint32_t*>(w); w += g.link_fwd_bytes;
   char* keep = ckpt ? static_cast<char*>(ckpt) + g.ckpt_diag_bytes : w;   // [top][packed B,C]
   sp.ckpt = ckpt ? static_cast<float*>(ckpt) : nullptr;
   sp.top = reinterpret_cast<float*>(keep);
   if (ckpt) prep = reinterpret_cast<float*>(keep + g.top_bytes + g.bc_bytes);   // kept for the backward
   sp.AT = AT; sp.AL = AL; sp.D = D;
   const bool own = g.fwd_split && !g.sliced;   // (split_owns_setup)
-  int rc = launch_prep<T>(sp, d, g, prep, link_words, st, own);
+  int rc = launch_prep<T>(sp, d, g, prep, link_words, g.link_fwd_bytes, st, own);
   if (!rc && own) rc = zero_page(&sp.zeros);   // (the area's own zeros are being written by this launch)
   if (rc) return rc;
   if ((!ckpt || sizeof(T) == 2) && !g.packed_bc) {   // the kernel takes the tensors as they are (fp32: only where no backward will want the packed copy)
@@ -3259,7 +3260,7 @@ int run_bwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
   char* ck = ckpt ? const_cast<char*>(static_cast<const char*>(ckpt)) : w;
   if (ckpt) prep = reinterpret_cast<float*>(ck + g.ckpt_diag_bytes + g.top_bytes + g.bc_bytes);   // as the forward left it
   sp.AT = AT; sp.AL = AL; sp.D = D;
-  int rc = launch_prep<T>(sp, d, g, prep, link_words, st, ckpt != nullptr);
+  int rc = launch_prep<T>(sp, d, g, prep, link_words, g.link_bytes, st, ckpt != nullptr);
   if (rc) return rc;
   sp.ckpt = reinterpret_cast<float*>(ck);
   sp.top = reinterpret_cast<float*>(ck + g.ckpt_diag_bytes);

@@ -115,6 +115,18 @@ def test_buffer_sizes_scale_linearly_in_area(cabi):
     assert cabi.lib.m2d_scan_ckpt_bytes(ctypes.byref(D(cabi, N=3))) == 0
 
 
+def test_forward_scratch_holds_its_own_progress_counts_only(cabi):
+    """A linked sweep keeps 256 bytes per workgroup (and as much for the error word); a forward that is given a checkpoint
+    buffer needs these and the set-up area, each rounded up to 256 bytes, and nothing for the backward."""
+    import re
+    for dtype, (B, H, W, E) in ((0, (1, 256, 256, 64)), (1, (4, 128, 128, 64)), (1, (24, 69, 123, 44))):
+        d = D(cabi, B=B, H=H, W=W, E=E, dtype=dtype)
+        plan = cabi.scan_plan(B, H, W, E, "f32" if dtype == 0 else "bf16", cabi.M2D_PASS_FWD)
+        workgroups = int(re.search(r"linked sweep, \d+ bands, (\d+) workgroups", plan).group(1))
+        setup = 4 * (64 + 2 * E * 16 + E)
+        assert 0 <= cabi.lib.m2d_scan_workspace_bytes(ctypes.byref(d), 0, 1) - (setup + 256 * (workgroups + 1)) < 512
+
+
 def test_checkpoint_interval_shrinks_the_snapshots(cabi):
     """m2d_desc.ckpt_interval = 8 / 16: a half / a quarter of the snapshots (band boundary rows and, for fp32, the
     packed B|C stay), a small ring of replayed snapshots per workgroup in the backward's scratch, and the one
