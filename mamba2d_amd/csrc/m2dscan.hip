@@ -2823,6 +2823,16 @@ Geometry make_geometry(const m2d_desc* d) {
   };
   set_schedule(link_whole);
   set_whole();
+  // The forward of one stream per image where rows are whole chunks: 8 waves with two channels each and a quarter of the states per
+  // lane.  Beside 4 waves that hold all states of 16 channels, which leave a SIMD to one wave each, they are ahead throughout (64 images of
+  // 56x56x64 bf16: 0.160 -> 0.127 ms, keeping snapshots 0.167 -> 0.131).  Beside 8 waves that hold all states of 32 channels they
+  // need two rounds for one, each with a start that takes as long as 3 blocks, and are ahead where a sweep is long (128 images of 56x56x64
+  // bf16, 60 blocks: 0.264 -> 0.255 ms, keeping snapshots 0.283 -> 0.263; 64 of 28x28x128, 18 blocks: 0.079 against 0.086).
+  const int64_t wg_pairs = (int64_t)B * ((d->E + 2 * kSplitWaves - 1) / (2 * kSplitWaves));
+  auto pairs = [&] {   // (of the schedule that set_whole was last called for)
+    return !g.sliced && g.stage_x && (g.fwd_nw == kFwdHalfWaves ||
+           (g.fwd_ec == 1 && 208 * ((wg_pairs + ncu - 1) / ncu) * (nblk_stream + 3) < 440 * (((int64_t)B * g.fwd_bpb + ncu - 1) / ncu) * nblk_stream));
+  };
   // A wave per channel, each lane with a quarter of the states, gets through a block of steps in a third of the time, but takes four times as many
   // waves.  Which is faster, and in which schedule, is a matter of how many workgroups follow each other on a compute unit (a backward
   // kernel has the unit to itself) and of the chain of bands: blocks that one unit sweeps, times what a block takes.  Measured, forward keeping snapshots
@@ -2841,6 +2851,7 @@ Geometry make_geometry(const m2d_desc* d) {
     const int64_t work = (wgs * g.nbands + ncu - 1) / ncu * nbb_link, chain = nbb_link + (int64_t)(g.nbands - 1) * (kLinkLag - 1);
     return (work > chain ? work + chain / 5 : chain + (work > nbb_link ? work / 5 : 0)) * block;
   };
+  auto cost = [&](bool linked, int64_t wgs, int64_t block) { return linked ? link_cost(wgs, block) : stream_cost(wgs, block); };
   const int64_t whole_block = g.bwd_nw != kFwdHalfWaves ? kWhole8 : (g.sliced ? kWhole4Linked : kWhole4);
   const int64_t whole_cost = g.sliced ? link_cost((int64_t)B * g.bwd_bpb, whole_block) : stream_cost((int64_t)B * g.bwd_bpb, whole_block);
   const int64_t wg4 = (int64_t)B * ((d->E + kSplitHalfWaves - 1) / kSplitHalfWaves), wg8 = (int64_t)B * ((d->E + kSplitWaves - 1) / kSplitWaves);
@@ -2848,49 +2859,79 @@ Geometry make_geometry(const m2d_desc* d) {
   bool split_link = false;
   int64_t split_cost = stream_cost(wg4, kSplit4);
   if (stream_cost(wg8, kSplit8) < split_cost) { split_cost = stream_cost(wg8, kSplit8); split_nw = kSplitWaves; }
+  // (one set of channel sums per workgroup of an image: with 4 or 8 channels per workgroup that memory is bounded here unless the caller insists)
+  auto sums_fit = [&](int nw) { return sizeof(float) * (size_t)((d->E + nw - 1) / nw) * 3 * kN * (size_t)d->B * d->H * d->W <= ((size_t)2 << 30); };
+  const bool link4 = g.nbands >= 2 && 5 * wg4 * (lagged < g.nbands ? lagged : g.nbands) <= 7 * ncu;
   if (g.nbands >= 2) {
     // Workgroups of 4 stay ahead up to 7 of them under way for every 5 units (E=64 fp32, forward+backward kernels with workgroups of 4
     // against 8: 384x384 1.23 against 1.44 ms, 512x512 1.95 against 2.05, 640x640 2.77 against 2.67, 768x768 3.93 against 3.35): each
     // reads B_T, B_L, C again and leaves channel sums of its own.
-    if (5 * wg4 * (lagged < g.nbands ? lagged : g.nbands) <= 7 * ncu && link_cost(wg4, kSplit4) < split_cost) { split_cost = link_cost(wg4, kSplit4); split_nw = kSplitHalfWaves; split_link = true; }
+    if (link4 && link_cost(wg4, kSplit4) < split_cost) { split_cost = link_cost(wg4, kSplit4); split_nw = kSplitHalfWaves; split_link = true; }
     if (link_cost(wg8, kSplit8) < split_cost) { split_cost = link_cost(wg8, kSplit8); split_nw = kSplitWaves; split_link = true; }
   }
   const bool may_split = !g.stacked && !(d->flags & M2D_FLAG_WHOLE_STATES) && g.ck_shift == 0 && !g.snap32;
-  const bool split = may_split && ((d->flags & M2D_FLAG_SPLIT_STATES) || 100 * split_cost < 93 * whole_cost);
+  bool split = may_split && ((d->flags & M2D_FLAG_SPLIT_STATES) || 100 * split_cost < 93 * whole_cost);
+  auto schedule_for = [&](bool linked) {
+    g.S = (g.nbands > 1 && d->W >= 26) ? d->W : (d->W + kHB - 1 > 26 ? d->W + kHB - 1 : 26);
+    g.T_total = (g.nbands - 1) * g.S + d->W + g.rows_last;
+    g.nblk = nblk_stream;
+    g.nbb = 0;
+    set_schedule(linked);
+    set_whole();
+  };
+  // Where the channel sums of the split backward would pass their bound, the backward is the one of whole states in the forward's schedule, and what
+  // suits a pair of split kernels may not suit this pair: 5x1362x43x319 fp32, forward + backward kernels, took 11.6 ms linked with whole states
+  // and 16.6 with a split forward in one stream per image.  So there the two passes that will run are priced, each by what its own block takes, in
+  // units of 10 ns: medians over 1000 problems drawn over all sizes and both types, each in every plan it can have; rows of whole 16-byte chunks, and others.
+  // Of 1000 problems 93 get another plan by it (nearly all of more than 2^26 values): forward + backward kernels 0.82 of the time, the worst 1.12.
+  struct Block { int64_t fwd[2], bwd[2]; };
+  constexpr Block kBlock4 = {{89, 114}, {237, 260}}, kBlock4Linked = {{90, 110}, {245, 280}}, kBlock8 = {{128, 162}, {362, 420}}, kBlock8Linked = {{138, 164}, {386, 447}};
+  constexpr Block kBlockWhole4 = {{250, 407}, {516, 756}}, kBlockWhole4Linked = {{257, 387}, {759, 1177}}, kBlockWhole8 = {{417, 423}, {1006, 1165}}, kBlockWhole8Linked = {{436, 491}, {1178, 1366}};
+  constexpr int64_t kBlockPairs = 189, kBlockTwoChannels[2] = {720, 754}, kBlockBwd4[2] = {810, 1340}, kBlockBwd8[2] = {1205, 1423};   // (m2d_bwd_kernel in one stream: behind a forward of split states)
+  const int ragged = g.stage_x ? 0 : 1;
+  auto whole_block_of = [&](int nw) -> const Block& { return nw == kFwdHalfWaves ? (g.sliced ? kBlockWhole4Linked : kBlockWhole4) : (g.sliced ? kBlockWhole8Linked : kBlockWhole8); };
+  auto whole_fwd_cost = [&] {   // (these two: of the schedule that set_whole was last called for)
+    if (pairs()) return kBlockPairs * ((wg_pairs + ncu - 1) / ncu) * (nblk_stream + 3);
+    return cost(g.sliced, (int64_t)B * g.fwd_bpb, g.fwd_ec == 2 ? kBlockTwoChannels[ragged] : whole_block_of(g.fwd_nw).fwd[ragged]);
+  };
+  auto whole_bwd_cost = [&](bool behind_split) {
+    const int64_t block = behind_split && !g.sliced ? (g.bwd_nw == kFwdHalfWaves ? kBlockBwd4 : kBlockBwd8)[ragged] : whole_block_of(g.bwd_nw).bwd[ragged];
+    return cost(g.sliced, (int64_t)B * g.bwd_bpb, block);
+  };
+  auto split_fwd_cost = [&](int nw, bool linked) { return cost(linked, nw == kSplitWaves ? wg8 : wg4, (nw == kSplitWaves ? (linked ? kBlock8Linked : kBlock8) : (linked ? kBlock4Linked : kBlock4)).fwd[ragged]); };
+  auto split_bwd_cost = [&](int nw, bool linked) { return cost(linked, nw == kSplitWaves ? wg8 : wg4, (nw == kSplitWaves ? (linked ? kBlock8Linked : kBlock8) : (linked ? kBlock4Linked : kBlock4)).bwd[ragged]); };
+  const bool sums_bound = may_split && !(d->flags & M2D_FLAG_SPLIT_STATES) && !sums_fit(split_nw);
+  if (sums_bound) {
+    const bool whole_link = g.sliced;
+    int64_t least = whole_fwd_cost() + whole_bwd_cost(false);
+    split = false;
+    auto offer = [&](int nw, bool linked) {
+      if (linked != g.sliced) schedule_for(linked);
+      const int64_t pair = split_fwd_cost(nw, linked) + (sums_fit(nw) ? split_bwd_cost(nw, linked) : whole_bwd_cost(true));
+      if (pair < least) { least = pair; split = true; split_nw = nw; split_link = linked; }
+    };
+    offer(kSplitHalfWaves, false);
+    offer(kSplitWaves, false);
+    if (link4) offer(kSplitHalfWaves, true);
+    if (g.nbands >= 2) offer(kSplitWaves, true);
+    if (!split && g.sliced != whole_link) schedule_for(whole_link);
+  }
   g.fwd_split = g.bwd_split = false;
   if (split) {
-    if (split_link != g.sliced) {
-      g.S = (g.nbands > 1 && d->W >= 26) ? d->W : (d->W + kHB - 1 > 26 ? d->W + kHB - 1 : 26);
-      g.T_total = (g.nbands - 1) * g.S + d->W + g.rows_last;
-      g.nblk = nblk_stream;
-      g.nbb = 0;
-      set_schedule(split_link);
-      set_whole();
-    }
+    if (split_link != g.sliced) schedule_for(split_link);
     g.fwd_split = true;
     g.fwd_ec = 1;
     g.fwd_nw = split_nw;
     g.fwd_bpb = (d->E + split_nw - 1) / split_nw;
     g.fwd_wpb = g.fwd_bpb * g.fwd_nw;
-    // (the backward keeps one set of channel sums per workgroup of an image: with 8 channels per workgroup
-    // that memory is bounded here unless the caller insists)
-    const size_t split_part = sizeof(float) * (size_t)((d->E + split_nw - 1) / split_nw) * 3 * kN * (size_t)d->B * d->H * d->W;
-    g.bwd_split = (d->flags & M2D_FLAG_SPLIT_STATES) || split_part <= ((size_t)2 << 30);
+    g.bwd_split = (d->flags & M2D_FLAG_SPLIT_STATES) || sums_fit(split_nw);
     if (g.bwd_split) {
       g.bwd_nw = split_nw;
       g.bwd_bpb = (d->E + split_nw - 1) / split_nw;
       g.bwd_wpb = g.bwd_bpb * g.bwd_nw;
     }
   }
-  // The forward of one stream per image where rows are whole chunks: 8 waves with two channels each and a quarter of the states per
-  // lane.  Beside 4 waves that hold all states of 16 channels, which leave a SIMD to one wave each, they are ahead throughout (64 images of
-  // 56x56x64 bf16: 0.160 -> 0.127 ms, keeping snapshots 0.167 -> 0.131).  Beside 8 waves that hold all states of 32 channels they
-  // need two rounds for one, each with a start that takes as long as 3 blocks, and are ahead where a sweep is long (128 images of 56x56x64
-  // bf16, 60 blocks: 0.264 -> 0.255 ms, keeping snapshots 0.283 -> 0.263; 64 of 28x28x128, 18 blocks: 0.079 against 0.086).
-  const int64_t wg_pairs = (int64_t)B * ((d->E + 2 * kSplitWaves - 1) / (2 * kSplitWaves));
-  const bool pairs = g.fwd_nw == kFwdHalfWaves ||
-                     (g.fwd_ec == 1 && 208 * ((wg_pairs + ncu - 1) / ncu) * (nblk_stream + 3) < 440 * (((int64_t)B * g.fwd_bpb + ncu - 1) / ncu) * nblk_stream);
-  if (!split && !g.stacked && !g.sliced && g.stage_x && pairs && g.ck_shift == 0 && !g.snap32 && !(d->flags & M2D_FLAG_WHOLE_STATES)) {
+  if (!split && !g.stacked && pairs() && g.ck_shift == 0 && !g.snap32 && !(d->flags & M2D_FLAG_WHOLE_STATES)) {
     g.fwd_split = true;
     g.fwd_ec = 2;
     g.fwd_nw = kSplitWaves;

@@ -184,6 +184,23 @@ def test_plan_names_kernel_and_schedule(cabi):
     assert cabi.lib.m2d_scan_plan(ctypes.byref(D(cabi, H=1)), 0, buf, 8) == 2 and buf.value == b""
 
 
+def test_plan_beyond_the_bound_on_channel_sums(cabi):
+    """Where the split backward's channel sums pass their bound, the pair of passes that runs is what is compared: a forward of split
+    states is no reason for a schedule in which the whole-state backward is slow."""
+    import torch
+    f32, bf16 = torch.float32, torch.bfloat16
+    # whole states throughout: measured 1.1 to 1.6 times as fast as split forwards in one stream with m2d_bwd_kernel behind them
+    for B, H, W, E, dtype, start in ((5, 1362, 43, 319, f32, "m2d_bwd_kernel: linked sweep"), (7, 80, 679, 256, bf16, "m2d_bwd_kernel: linked sweep"),
+                                     (245, 355, 104, 16, bf16, "m2d_bwd2_kernel: one stream")):
+        plan = cabi.scan_plan(B, H, W, E, dtype, cabi.M2D_PASS_BWD)
+        assert plan.startswith(start), plan
+        assert plan == cabi.scan_plan(B, H, W, E, dtype, cabi.M2D_PASS_BWD, flags=cabi.M2D_FLAG_WHOLE_STATES)
+    # a forward of split states in a schedule that suits the backward
+    for B, H, W, E, dtype in ((11, 283, 206, 176, bf16), (109, 179, 96, 84, bf16), (1, 1280, 1280, 64, f32), (1, 2048, 2048, 64, f32), (1, 2048, 2048, 64, bf16)):
+        assert cabi.scan_plan(B, H, W, E, dtype, cabi.M2D_PASS_FWD).startswith("m2d_fwd_split_kernel: linked sweep")
+        assert cabi.scan_plan(B, H, W, E, dtype, cabi.M2D_PASS_BWD).startswith("m2d_bwd_kernel: linked sweep")
+
+
 def test_python_surface_matches_reference_names():
     """models/kernels/wavefront_cuda.py exposes these names; models/mamba2d.py:10 imports one."""
     from mamba2d_amd.kernels import wavefront_cuda as w
