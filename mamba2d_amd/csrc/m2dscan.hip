@@ -2659,6 +2659,7 @@ constexpr size_t bwd_lds_bytes() {
 static_assert(fwd_lds_bytes<float, 1>() <= kLdsPerWorkgroup && fwd_lds_bytes<bf16_t, 1>() <= kLdsPerWorkgroup, "forward staging must fit the LDS");
 static_assert(bwd_lds_bytes<float>() <= kLdsPerWorkgroup && bwd_lds_bytes<bf16_t>() <= kLdsPerWorkgroup, "backward staging must fit the LDS");
 
+struct ForwardKernel { bool split; int ec, nw, bpb; };
 struct Geometry {
   int HB, hb_shift, CS, nbands, nblk;
   int S, T_total, rows_last;         // stream stride, total steps, rows of the last band
@@ -2666,6 +2667,7 @@ struct Geometry {
   int fwd_ec, fwd_nw, fwd_wpb, fwd_bpb;   // forward: channels per lane (split states: per wave), waves per workgroup, waves and workgroups per image
   int bwd_nw, bwd_wpb, bwd_bpb;      // backward: waves per workgroup, waves and workgroups (channel groups) per image
   bool fwd_split, bwd_split;         // the states of a channel split over the lanes (a wave per channel: m2d_fwd_split_kernel, m2d_bwd_split_kernel)
+  ForwardKernel alone;               // the forward that keeps no snapshots (the same schedule and scratch; often the same kernel)
   bool stage_x;                      // x, delta, dy rows are whole 16-byte chunks: stage them through LDS
   bool sliced;                       // linked sweep: bands on workgroups of their own, handing boundary rows to each other inside one launch
   bool stacked;                      // images of one band stacked into tall images of independent bands
@@ -2931,11 +2933,12 @@ Geometry make_geometry(const m2d_desc* d) {
       g.bwd_wpb = g.bwd_bpb * g.bwd_nw;
     }
   }
+  const int pairs_bpb = (d->E + 2 * kSplitWaves - 1) / (2 * kSplitWaves);
   if (!split && !g.stacked && pairs() && g.ck_shift == 0 && !g.snap32 && !(d->flags & M2D_FLAG_WHOLE_STATES)) {
     g.fwd_split = true;
     g.fwd_ec = 2;
     g.fwd_nw = kSplitWaves;
-    g.fwd_bpb = (d->E + kSplitWaves * g.fwd_ec - 1) / (kSplitWaves * g.fwd_ec);
+    g.fwd_bpb = pairs_bpb;
     g.fwd_wpb = g.fwd_bpb * g.fwd_nw;
   }
   if (g.snap32) {
@@ -2943,6 +2946,22 @@ Geometry make_geometry(const m2d_desc* d) {
     g.fwd_nw = g.bwd_nw = kFwdHalfWaves;
     g.fwd_bpb = g.bwd_bpb = (d->E + kFwdHalfWaves * g.CS - 1) / (kFwdHalfWaves * g.CS);
     g.fwd_wpb = g.bwd_wpb = g.fwd_bpb * kFwdHalfWaves;
+  }
+  // The plan is for a forward that keeps snapshots and its backward, and split states gain most in the backward.  A forward that keeps none may have
+  // a faster kernel in one stream per image: beside split states the one with two channels per lane (20x39x29x436 bf16: 0.268 -> 0.207 ms, 66x18x15x122
+  // 0.120 -> 0.100) or the pairs (196x84x49x16 0.199 -> 0.155); beside whole states that only the bound on channel sums asks for, split states
+  // (12x42x874x310 fp32: 2.98 -> 2.27).  Of 75 drawn problems that this takes the forward is 0.86 of what it was, none slower.
+  g.alone = {g.fwd_split, g.fwd_ec, g.fwd_nw, g.fwd_bpb};
+  if (may_split && !g.sliced && (split || sums_bound) && !(d->flags & M2D_FLAG_SPLIT_STATES)) {
+    const Geometry kept = g;
+    set_whole();
+    const int64_t whole_cost_alone = whole_fwd_cost();
+    const ForwardKernel whole = pairs() ? ForwardKernel{true, 2, kSplitWaves, pairs_bpb} : ForwardKernel{false, g.fwd_ec, g.fwd_nw, g.fwd_bpb};
+    g = kept;
+    const int nw = !sums_bound ? split_nw : (split_fwd_cost(kSplitHalfWaves, false) < split_fwd_cost(kSplitWaves, false) ? kSplitHalfWaves : kSplitWaves);
+    const int64_t split_cost_alone = split_fwd_cost(nw, false);
+    if (split && 100 * whole_cost_alone < 97 * split_cost_alone) g.alone = whole;
+    else if (sums_bound && (split || 100 * split_cost_alone < 90 * whole_cost_alone)) g.alone = {true, 1, nw, (d->E + nw - 1) / nw};
   }
   const size_t P = (size_t)d->B * d->H * d->W;
   g.prep_bytes = align_up(sizeof(float) * (kZeroFloats + (size_t)2 * d->E * kN + d->E));
@@ -3409,7 +3428,8 @@ int m2d_scan_fwd(const m2d_desc* desc, const void* x, const void* deltaT, const 
   for (const void* q : req) if (!q) return M2D_ERR_NULL_POINTER;
   for (const void* q : req) if (misaligned(q, 16)) return M2D_ERR_MISALIGNED;
   if (misaligned(workspace, 256) || (ckpt && misaligned(ckpt, 256))) return M2D_ERR_MISALIGNED;
-  const Geometry g = make_geometry(desc);
+  Geometry g = make_geometry(desc);
+  if (!ckpt) { g.fwd_split = g.alone.split; g.fwd_ec = g.alone.ec; g.fwd_nw = g.alone.nw; g.fwd_bpb = g.alone.bpb; }
   if (workspace_bytes < workspace_bytes_of(g, M2D_PASS_FWD, ckpt != nullptr)) return M2D_ERR_WORKSPACE;
   if (ckpt && ckpt_bytes < ckpt_bytes_of(g)) return M2D_ERR_WORKSPACE;
   ScanParams sp = {};
@@ -3486,6 +3506,11 @@ int m2d_scan_plan(const m2d_desc* desc, int pass, char* text, size_t cap) {
   if (g.ck_shift) {
     const size_t n = strlen(text);
     if (n + 1 < cap) snprintf(text + n, cap - n, fwd ? ", a snapshot every %d steps" : ", a snapshot every %d steps and the forward replayed in between", kCK << g.ck_shift);
+  }
+  if (fwd && (g.alone.split != g.fwd_split || g.alone.ec != g.fwd_ec || g.alone.nw != g.fwd_nw)) {
+    const size_t n = strlen(text);
+    if (n + 1 < cap) snprintf(text + n, cap - n, "; without snapshots %s, %lld workgroups of %d channels", g.alone.split ? "m2d_fwd_split_kernel" : "m2d_fwd_kernel",
+                              (long long)g.vB * g.alone.bpb, (g.alone.split ? 1 : g.CS) * g.alone.nw * g.alone.ec);
   }
   return M2D_OK;
 }
