@@ -2828,12 +2828,17 @@ Geometry make_geometry(const m2d_desc* d) {
   // The forward of one stream per image where rows are whole chunks: 8 waves with two channels each and a quarter of the states per
   // lane.  Beside 4 waves that hold all states of 16 channels, which leave a SIMD to one wave each, they are ahead throughout (64 images of
   // 56x56x64 bf16: 0.160 -> 0.127 ms, keeping snapshots 0.167 -> 0.131).  Beside 8 waves that hold all states of 32 channels they
-  // need two rounds for one, each with a start that takes as long as 3 blocks, and are ahead where a sweep is long (128 images of 56x56x64
-  // bf16, 60 blocks: 0.264 -> 0.255 ms, keeping snapshots 0.283 -> 0.263; 64 of 28x28x128, 18 blocks: 0.079 against 0.086).
+  // often need two rounds for one, each with a start that takes as long as 3 blocks, and are ahead where a sweep is long (128 images of 56x56x64
+  // bf16, 60 blocks: 0.264 -> 0.255 ms, keeping snapshots 0.283 -> 0.263; 64 of 28x28x128, 18 blocks: 0.079 against 0.086).  Their share of the time of
+  // whole states at twice the rounds, keeping snapshots, bands back to back, 57 drawn problems: 0.99 to 1.11 up to 26 blocks, 0.91 to 1.05 up to 52
+  // where the line is, 0.92 to 1.00 beyond; on grids of one band, and on narrow ones whose bands are padded, 1.00 to 1.05 at any length in bf16 and 0.85 to 1.07 in fp32
+  // (whole states are faster where lanes have no cell), and 1.00 to 1.08 without snapshots.  At fewer than twice the rounds 0.73 to 0.97.
   const int64_t wg_pairs = (int64_t)B * ((d->E + 2 * kSplitWaves - 1) / (2 * kSplitWaves));
-  auto pairs = [&] {   // (of the schedule that set_whole was last called for)
-    return !g.sliced && g.stage_x && (g.fwd_nw == kFwdHalfWaves ||
-           (g.fwd_ec == 1 && 208 * ((wg_pairs + ncu - 1) / ncu) * (nblk_stream + 3) < 440 * (((int64_t)B * g.fwd_bpb + ncu - 1) / ncu) * nblk_stream));
+  auto pairs = [&](bool keeping) {   // (of the schedule that set_whole was last called for)
+    if (g.sliced || !g.stage_x || g.fwd_ec != 1) return false;
+    if (g.fwd_nw == kFwdHalfWaves) return true;
+    const int64_t rounds = (wg_pairs + ncu - 1) / ncu, rounds_whole = ((int64_t)B * g.fwd_bpb + ncu - 1) / ncu;
+    return 208 * rounds * (nblk_stream + 3) < 440 * rounds_whole * nblk_stream && (rounds < 2 * rounds_whole || (g.nbands > 1 && d->W >= 26) || (keeping && d->dtype == M2D_F32));
   };
   // A wave per channel, each lane with a quarter of the states, gets through a block of steps in a third of the time, but takes four times as many
   // waves.  Which is faster, and in which schedule, is a matter of how many workgroups follow each other on a compute unit (a backward
@@ -2892,8 +2897,8 @@ Geometry make_geometry(const m2d_desc* d) {
   constexpr int64_t kBlockPairs = 189, kBlockTwoChannels[2] = {720, 754}, kBlockBwd4[2] = {810, 1340}, kBlockBwd8[2] = {1205, 1423};   // (m2d_bwd_kernel in one stream: behind a forward of split states)
   const int ragged = g.stage_x ? 0 : 1;
   auto whole_block_of = [&](int nw) -> const Block& { return nw == kFwdHalfWaves ? (g.sliced ? kBlockWhole4Linked : kBlockWhole4) : (g.sliced ? kBlockWhole8Linked : kBlockWhole8); };
-  auto whole_fwd_cost = [&] {   // (these two: of the schedule that set_whole was last called for)
-    if (pairs()) return kBlockPairs * ((wg_pairs + ncu - 1) / ncu) * (nblk_stream + 3);
+  auto whole_fwd_cost = [&](bool keeping) {   // (these two: of the schedule that set_whole was last called for)
+    if (pairs(keeping)) return kBlockPairs * ((wg_pairs + ncu - 1) / ncu) * (nblk_stream + 3);
     return cost(g.sliced, (int64_t)B * g.fwd_bpb, g.fwd_ec == 2 ? kBlockTwoChannels[ragged] : whole_block_of(g.fwd_nw).fwd[ragged]);
   };
   auto whole_bwd_cost = [&](bool behind_split) {
@@ -2905,7 +2910,7 @@ Geometry make_geometry(const m2d_desc* d) {
   const bool sums_bound = may_split && !(d->flags & M2D_FLAG_SPLIT_STATES) && !sums_fit(split_nw);
   if (sums_bound) {
     const bool whole_link = g.sliced;
-    int64_t least = whole_fwd_cost() + whole_bwd_cost(false);
+    int64_t least = whole_fwd_cost(true) + whole_bwd_cost(false);
     split = false;
     auto offer = [&](int nw, bool linked) {
       if (linked != g.sliced) schedule_for(linked);
@@ -2934,7 +2939,7 @@ Geometry make_geometry(const m2d_desc* d) {
     }
   }
   const int pairs_bpb = (d->E + 2 * kSplitWaves - 1) / (2 * kSplitWaves);
-  if (!split && !g.stacked && pairs() && g.ck_shift == 0 && !g.snap32 && !(d->flags & M2D_FLAG_WHOLE_STATES)) {
+  if (!split && !g.stacked && pairs(true) && g.ck_shift == 0 && !g.snap32 && !(d->flags & M2D_FLAG_WHOLE_STATES)) {
     g.fwd_split = true;
     g.fwd_ec = 2;
     g.fwd_nw = kSplitWaves;
@@ -2952,16 +2957,16 @@ Geometry make_geometry(const m2d_desc* d) {
   // 0.120 -> 0.100) or the pairs (196x84x49x16 0.199 -> 0.155); beside whole states that only the bound on channel sums asks for, split states
   // (12x42x874x310 fp32: 2.98 -> 2.27).  Of 75 drawn problems that this takes the forward is 0.86 of what it was, none slower.
   g.alone = {g.fwd_split, g.fwd_ec, g.fwd_nw, g.fwd_bpb};
-  if (may_split && !g.sliced && (split || sums_bound) && !(d->flags & M2D_FLAG_SPLIT_STATES)) {
+  if (may_split && !g.sliced && (split || sums_bound || g.fwd_ec == 2) && !(d->flags & M2D_FLAG_SPLIT_STATES)) {
     const Geometry kept = g;
     set_whole();
-    const int64_t whole_cost_alone = whole_fwd_cost();
-    const ForwardKernel whole = pairs() ? ForwardKernel{true, 2, kSplitWaves, pairs_bpb} : ForwardKernel{false, g.fwd_ec, g.fwd_nw, g.fwd_bpb};
+    const int64_t whole_cost_alone = whole_fwd_cost(false);
+    const ForwardKernel whole = pairs(false) ? ForwardKernel{true, 2, kSplitWaves, pairs_bpb} : ForwardKernel{false, g.fwd_ec, g.fwd_nw, g.fwd_bpb};
     g = kept;
     const int nw = !sums_bound ? split_nw : (split_fwd_cost(kSplitHalfWaves, false) < split_fwd_cost(kSplitWaves, false) ? kSplitHalfWaves : kSplitWaves);
     const int64_t split_cost_alone = split_fwd_cost(nw, false);
-    if (split && 100 * whole_cost_alone < 97 * split_cost_alone) g.alone = whole;
-    else if (sums_bound && (split || 100 * split_cost_alone < 90 * whole_cost_alone)) g.alone = {true, 1, nw, (d->E + nw - 1) / nw};
+    if (!split || 100 * whole_cost_alone < 97 * split_cost_alone) g.alone = whole;
+    if (sums_bound && 100 * split_cost_alone < (split ? 100 : 90) * whole_cost_alone) g.alone = {true, 1, nw, (d->E + nw - 1) / nw};
   }
   const size_t P = (size_t)d->B * d->H * d->W;
   g.prep_bytes = align_up(sizeof(float) * (kZeroFloats + (size_t)2 * d->E * kN + d->E));

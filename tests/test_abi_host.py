@@ -184,6 +184,21 @@ def test_plan_names_kernel_and_schedule(cabi):
     assert cabi.lib.m2d_scan_plan(ctypes.byref(D(cabi, H=1)), 0, buf, 8) == 2 and buf.value == b""
 
 
+def test_plan_of_a_full_batch_forward(cabi):
+    """Two channels a wave at twice the rounds of workgroups: long sweeps whose bands follow each other without a gap."""
+    import torch
+    f32, bf16 = torch.float32, torch.bfloat16
+    pairs = "8 waves and 4 that stage, 16 channels each"
+    for B, H, W, E, dtype, taken in ((128, 56, 56, 64, bf16, True), (28, 47, 70, 192, bf16, True), (120, 28, 28, 64, bf16, False),    # 60, 72 and 18 blocks
+                                     (178, 9, 768, 24, bf16, False), (38, 5, 1337, 168, bf16, False),                               # one band
+                                     (150, 1483, 4, 152, bf16, False), (68, 714, 4, 88, bf16, False),                               # padded bands
+                                     (95, 269, 3, 152, f32, True), (129, 13, 1512, 32, f32, True),                                  # ... keeping fp32 snapshots
+                                     (67, 143, 6, 280, bf16, True), (193, 34, 8, 80, bf16, True)):                                  # ... at 5 rounds for 3, 4 for 3
+        plan = cabi.scan_plan(B, H, W, E, dtype, cabi.M2D_PASS_FWD)
+        assert (pairs in plan) == taken and plan.startswith("m2d_fwd_split_kernel: one stream" if taken else "m2d_fwd_kernel: one stream"), plan
+        assert ("; without snapshots m2d_fwd_kernel" in plan) == (taken and dtype == f32)
+
+
 def test_plan_beyond_the_bound_on_channel_sums(cabi):
     """Where the split backward's channel sums pass their bound, the pair of passes that runs is what is compared: a forward of split
     states is no reason for a schedule in which the whole-state backward is slow."""

@@ -1,5 +1,5 @@
 """Forwards that keep no snapshots and run another kernel for it than the forward of a training step: two channels per lane or the pairs
-beside split states, split states beside whole ones.  Values against the oracle at the tolerances of the scan's other tests; the largest
+beside split states, split states beside whole ones, whole states beside the pairs.  Values against the oracle at the tolerances of the scan's other tests; the largest
 (split states beside whole ones exist beyond 2 GiB of channel sums only) against the forward that keeps snapshots, the same
 fp32 sums in another order."""
 import numpy as np
@@ -15,6 +15,7 @@ SMALL = [
     (33, 26, 6, 276, torch.bfloat16, "m2d_fwd_kernel, 165 workgroups of 64 channels"),         # a last workgroup of 20
     (249, 33, 28, 16, torch.bfloat16, "m2d_fwd_split_kernel, 249 workgroups of 16 channels"),
     (181, 12, 35, 12, torch.float32, "m2d_fwd_split_kernel, 181 workgroups of 16 channels"),   # 4 of the 16 past the end
+    (228, 121, 2, 20, torch.float32, "m2d_fwd_kernel, 228 workgroups of 32 channels"),         # the pairs where snapshots are kept
 ]
 LARGE = (12, 42, 874, 310, torch.float32, "m2d_fwd_split_kernel, 468 workgroups of 8 channels")
 
