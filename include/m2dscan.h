@@ -64,8 +64,9 @@ typedef struct m2d_desc {
                                  2: two snapshots per block of 4 steps; the backward then recomputes one step in two
                                     and computes every gate once (its kernel is bound by instruction issue, not by
                                     memory: it trades bytes for instructions).  Only where every image (or stack of
-                                    small images) is swept as one stream with all 16 states of a channel in one lane;
-                                    the other schedules (few large images) keep 4, also when 2 is asked for.
+                                    small images) is swept as one stream and the backward is m2d_bwd2_kernel, whose lanes
+                                    hold 16 or 8 states of a channel (the forward before it may hold 4); the other
+                                    schedules and the split-state backward keep 4, also when 2 is asked for.
                                  4: one snapshot per block; the backward recomputes the block.
                                  8, 16: a half / a quarter of the snapshots of 4; the backward replays the forward
                                     over the blocks in between (4 or 12 steps of every 8 or 16) before it sweeps them.

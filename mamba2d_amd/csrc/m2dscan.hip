@@ -3502,10 +3502,10 @@ int m2d_scan_plan(const m2d_desc* desc, int pass, char* text, size_t cap) {
     // (workgroups of 4 waves have waves that only stage, except in the backward that replays the forward between snapshots)
     const bool helped = !g.stacked && nw == kFwdHalfWaves && per_lane == 1 && (fwd || g.ck_shift == 0);
     char extra[48] = "";
-    if (helped) snprintf(extra, sizeof extra, " and %d that stage", kWholeHelpers);
-    if (helped && !fwd && g.ck_half) snprintf(extra, sizeof extra, " in two halves and %d that stage", kWholeHelpers);
-    snprintf(text, cap, "%s: %s, %lld workgroups of %d waves%s, %d channels each, 16 states per lane%s",
-             fwd ? "m2d_fwd_kernel" : (g.ck_half ? "m2d_bwd2_kernel" : "m2d_bwd_kernel"), sched, wgs, nw, extra, nw * g.CS * per_lane,
+    const bool halves = helped && !fwd && g.ck_half;   // (two waves to 4 channels, 8 of the 16 states each)
+    if (helped) snprintf(extra, sizeof extra, "%s and %d that stage", halves ? " in two halves" : "", kWholeHelpers);
+    snprintf(text, cap, "%s: %s, %lld workgroups of %d waves%s, %d channels each, %d states per lane%s",
+             fwd ? "m2d_fwd_kernel" : (g.ck_half ? "m2d_bwd2_kernel" : "m2d_bwd_kernel"), sched, wgs, halves ? 2 * nw : nw, extra, nw * g.CS * per_lane, halves ? kN / 2 : kN,
              g.ck_half ? (fwd ? ", a snapshot every 2 steps" : ", a snapshot every 2 steps and one step in two recomputed") : "");
   }
   if (g.ck_shift) {
