@@ -49,8 +49,18 @@ SPILL_ALLOWANCE = [(re.compile(r"m2d_bwd_kernelI\w*Li8ELb1E\w*EEv"), 64)]   # (<
 
 # A kernel that runs out of scalar registers parks some in lanes of a vector register; the compiler then reserves a
 # few bytes of scratch for that register without ever storing it.  Allowed up to this many bytes per lane, and only
-# where the kernel has no scratch load or store at all.
-UNTOUCHED_SCRATCH = 128
+# where the kernel has no scratch load or store at all; a little more for the backward of split states with 8 sweeping
+# waves in the linked sweep, which keeps the link's state in scalar registers as well (68 bytes, 17 registers' worth).
+UNTOUCHED_SCRATCH = 64
+UNTOUCHED_ALLOWANCE = [(re.compile(r"m2d_bwd_split_kernelI\w*Lb[01]ELi1ELi8EEE"), 68)]   # (<..., linked sweep, 8 waves>)
+
+
+def spill_allowed(kernel: str, nbytes: int, accesses: int) -> bool:
+    """Whether a kernel may have `nbytes` of scratch per lane, touched by `accesses` instructions."""
+    if any(pat.search(kernel) and nbytes <= cap for pat, cap in SPILL_ALLOWANCE):
+        return True
+    cap = max([UNTOUCHED_SCRATCH] + [c for pat, c in UNTOUCHED_ALLOWANCE if pat.search(kernel)])
+    return accesses == 0 and nbytes <= cap
 
 
 def build_lib(verbose: bool = True) -> str:
@@ -86,9 +96,7 @@ def build_lib(verbose: bool = True) -> str:
                                    "\n".join(f"  {k}: {p}  ->  {c}" for k, p, c in bad[:8]))
             with open(path) as f:
                 accesses = asmcheck.scratch_accesses(f.read())
-            spills = [(k, n) for k, n in asmcheck.spills_in_file(path)
-                      if not any(pat.search(k) and n <= cap for pat, cap in SPILL_ALLOWANCE)
-                      and not (n <= UNTOUCHED_SCRATCH and accesses.get(k, 1) == 0)]
+            spills = [(k, n) for k, n in asmcheck.spills_in_file(path) if not spill_allowed(k, n, accesses.get(k, 1))]
             if spills:
                 raise RuntimeError("kernels that spill registers to scratch memory:\n" +
                                    "\n".join(f"  {k}: {n} bytes per lane" for k, n in spills[:8]))

@@ -62,3 +62,14 @@ def test_wide_store_data_overwritten_too_early():
     assert asmcheck.check_text(listing(plain, "v_mul_f32_e32 v4, v20, v21"))[1] == []      # the compiler's own: it knows the rule
     assert asmcheck.check_text(listing(store.replace("x4", "x2").replace("[4:7]", "[4:5]"),
                                        "v_mul_f32_e32 v4, v20, v21"))[1] == []             # 8 bytes are read at issue
+
+
+def test_scratch_that_a_kernel_may_have():
+    """Only the kernels that are named may have more than 64 bytes a lane, and none but the replaying backward may touch it."""
+    from mamba2d_amd.build import spill_allowed
+    linked8 = "_ZN12_GLOBAL__N_120m2d_bwd_split_kernelIfLb1ELi1ELi8EEEvNS_10ScanParamsE"
+    linked4, stream8 = linked8.replace("Li8E", "Li4E"), linked8.replace("Li1E", "Li0E")
+    assert spill_allowed(linked8, 68, 0) and not spill_allowed(linked8, 72, 0) and not spill_allowed(linked8, 4, 1)
+    for kernel in (linked4, stream8, "_ZN12_GLOBAL__N_115m2d_bwd2_kernelIfLb0ELi0ELi4EEEvNS_10ScanParamsE"):
+        assert spill_allowed(kernel, 64, 0) and not spill_allowed(kernel, 68, 0) and not spill_allowed(kernel, 36, 2)
+    assert spill_allowed("_ZN12_GLOBAL__N_114m2d_bwd_kernelIfLb1ELi1ELi8ELb1EfEEvNS_10ScanParamsE", 28, 21)
