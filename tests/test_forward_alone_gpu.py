@@ -54,6 +54,26 @@ def test_values_without_snapshots(cscan, case, flip):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("case", SMALL, ids=lambda c: "x".join(map(str, c[:4])))
+def test_entry_point_without_snapshots(case):
+    """The entry point's operands (packed records, raw parameters): the same fp32 sums in another order, in bf16 at most one rounding
+    of the result apart (2^-8 of a value)."""
+    from mamba2d_amd.wavefront import wavefront_scan_cuda
+    B, H, W, E, dtype, _ = case
+    print(f"\ncase entry {case}", flush=True)
+    R, g = max(1, E // 16), torch.Generator(device="cuda").manual_seed(7)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    p = [0.3 * r(E, 16), 0.3 * r(E, 16), r(2 * R + 48, E) / E ** 0.5, r(E, R), r(E) - 2, r(E, R), r(E) - 2, 1 + 0.1 * r(E)]
+    x = r(B, H, W, E).to(dtype)
+    kept = wavefront_scan_cuda(x.clone().requires_grad_(True), *p).detach().float()
+    with torch.no_grad():
+        alone = wavefront_scan_cuda(x, *p).float()
+    recomputed = wavefront_scan_cuda(x.clone().requires_grad_(True), *p, "full").detach().float()
+    assert torch.equal(alone, recomputed)
+    assert float((alone - kept).abs().max() / kept.abs().max()) < (1e-5 if dtype == torch.float32 else 2 ** -8)
+
+
+@pytest.mark.gpu
 def test_largest_without_snapshots():
     from mamba2d_amd import cabi
     B, H, W, E, dtype, _ = LARGE
