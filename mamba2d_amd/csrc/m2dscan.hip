@@ -2842,16 +2842,16 @@ Geometry make_geometry(const m2d_desc* d) {
   };
   // A wave per channel, each lane with a quarter of the states, gets through a block of steps in a third of the time, but takes four times as many
   // waves.  Which is faster, and in which schedule, is a matter of how many workgroups follow each other on a compute unit (a backward
-  // kernel has the unit to itself) and of the chain of bands: blocks that one unit sweeps, times what a block takes.  Measured, forward keeping snapshots
-  // and backward, relative to a workgroup of 4 waves with a quarter of the states each (56x56x64 bf16, all units busy): 8 such waves
-  // 1.47, whole states 4.2 in workgroups of 8 waves (32 channels), and in workgroups of 16 channels 3.0 in the linked sweep and 2.35
-  // in one stream per image (where 8 waves share the work of 4: m2d_bwd2_kernel, and the forward below).
-  // In the linked sweep a band trails its neighbour by 6 blocks, and the shorter of the two, the chain of bands and the work per unit, hides
-  // behind the longer but for about a fifth (where units have more than one workgroup to sweep).
-  // What this rule takes from the whole states, forward + backward in ms: 30x60x50x40 fp32 0.517 -> 0.312, 8x100x120x96 bf16 0.891 -> 0.615,
-  // 8x256x256x64 bf16 3.13 -> 2.09, 20x28x28x200 fp32 0.296 -> 0.192, 2048x2048x64 fp32 forward 6.39 -> 4.82;
-  // and leaves with them: 32x128x128x64 bf16 2.00 (split 2.17), 8x512x512x64 bf16 7.6 (8.0), 64x28x28x128 bf16 0.280 (0.389).
-  // Near the line the whole states stay: fewer channel sums, and snapshots every 2 steps.
+  // kernel has the unit to itself) and of the chain of bands: blocks that one unit sweeps, times what a block takes.  In the linked sweep a band
+  // trails its neighbour by 6 blocks, and the shorter of the two, the chain of bands and the work per unit, hides behind the longer but for about a
+  // fifth (where units have more than one workgroup to sweep).
+  // The constants are ratios: a block of forward keeping snapshots and backward, a workgroup of 4 waves with a quarter of the states each as 100
+  // (1000 problems of both types: 8 such waves 150; whole states in workgroups of 8 waves 437, of 16 channels 303 linked and 216 in one stream; where
+  // rows are no whole chunks all of them take longer, the last 310).  Near the line the whole states stay: fewer channel sums, snapshots every 2
+  // steps.  Both sides, kernels of both passes in ms, whole states against split: 30x60x50x40 fp32 0.522 and 0.324, 8x256x256x64 bf16 3.16 and 2.10,
+  // 20x28x28x200 fp32 0.289 and 0.202, 32x128x128x64 bf16 2.02 and 1.64; on the other side of the line 64x28x28x128 bf16 0.280 and 0.391.
+  // Of 708 problems drawn over all sizes the chosen plans take 1.023 of the time of each one's best; farthest off, 1.3 to 1.5, are widths of no whole
+  // chunks and one to three channels, and grids two to four columns wide, where whole states would be up to 1.09 ahead of the linked sweep.
   constexpr int64_t kSplit4 = 100, kSplit8 = 147, kWhole4 = 235, kWhole4Linked = 300, kWhole8 = 417;
   auto stream_cost = [&](int64_t wgs, int64_t block) { return (wgs + ncu - 1) / ncu * nblk_stream * block; };
   auto link_cost = [&](int64_t wgs, int64_t block) {
@@ -2866,7 +2866,9 @@ Geometry make_geometry(const m2d_desc* d) {
   bool split_link = false;
   int64_t split_cost = stream_cost(wg4, kSplit4);
   if (stream_cost(wg8, kSplit8) < split_cost) { split_cost = stream_cost(wg8, kSplit8); split_nw = kSplitWaves; }
-  // (one set of channel sums per workgroup of an image: with 4 or 8 channels per workgroup that memory is bounded here unless the caller insists)
+  // (one set of channel sums per workgroup of an image: with 4 or 8 channels per workgroup that memory is bounded here unless the caller insists.  A bound
+  // on memory, not on time: at E=64 fp32 the split backward would take 5.42 of 7.35 ms at 1280x1280 for 1.2 GB of scratch more, 12.95 of 14.2 at
+  // 2048x2048 for 3.1 GB; at 8x512x512x64 bf16 6.1 for 5.5 ms and 2.3 GB)
   auto sums_fit = [&](int nw) { return sizeof(float) * (size_t)((d->E + nw - 1) / nw) * 3 * kN * (size_t)d->B * d->H * d->W <= ((size_t)2 << 30); };
   const bool link4 = g.nbands >= 2 && 5 * wg4 * (lagged < g.nbands ? lagged : g.nbands) <= 7 * ncu;
   if (g.nbands >= 2) {

@@ -16,12 +16,8 @@
 // places as it can.  A store takes several times as long to be acknowledged as a block takes, and the counter that a wave waits on
 // retires in order: every block issues the same operations whatever lanes they are for, so that a wave knows how many of them may still be under way
 // (split_landed), and rows of a neighbour, which are fetched at the last moment, come in through a wave that stores nothing before them.
-// Before, every sweeping wave also staged, stored and waited; kernels, forward keeping snapshots / backward:
-//   1x256x256x64 fp32 (304 workgroups of 4 + 4)   0.298 / 0.683 -> 0.196 / 0.480 ms
-//   1x256x256x62 fp32 (rows of no whole chunks)   0.476 / 1.157 -> 0.226 / 0.572
-//   1x512x512x64 fp32                             0.786 / 1.753 -> 0.573 / 1.371
-//   4x128x128x64 bf16                             0.183 / 0.442 -> 0.111 / 0.315
-//   2x14x14x32 fp32 (7 blocks)                    13.5 / 25.4 -> 11.8 / 21.7 us
+// Against sweeping waves that also stage, forward keeping snapshots / backward: 1x256x256x64 fp32 0.298 / 0.683 -> 0.196 / 0.480 ms,
+// 1x256x256x62 (rows of no whole chunks) 0.476 / 1.157 -> 0.226 / 0.572, 4x128x128x64 bf16 0.183 / 0.442 -> 0.111 / 0.315.
 // Memory formats and schedules are those of the whole-state kernels, so either pass may use either layout.
 constexpr int kSplitWaves = 8;       // sweeping waves (channels) per workgroup
 constexpr int kSplitHalfWaves = 4;   // ... where workgroups of 8 would leave compute units idle
