@@ -181,6 +181,13 @@ __device__ __forceinline__ float fold16(float a, float b) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Component q of lane group (slot) i goes to component i of group q: four 4 x 4 transpositions of the lane groups at once, per lane row
+__device__ __forceinline__ float4 slots_turned(float4 v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.x), __float_as_uint(v.z), false, false), b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.y), __float_as_uint(v.w), false, false);
+  const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false), hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return make_float4(__uint_as_float(lo[0]), __uint_as_float(lo[1]), __uint_as_float(hi[0]), __uint_as_float(hi[1]));
+}
+
 struct ScanParams {
   const void *x, *dT, *dL, *dy;
   const float *bt, *bl, *cc;        // B_T, B_L, C in fp32, state n of a cell at [cell*bc_stride + spos(n)]
