@@ -187,6 +187,11 @@ __device__ __forceinline__ float4 slots_turned(float4 v) {
   const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false), hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
   return make_float4(__uint_as_float(lo[0]), __uint_as_float(lo[1]), __uint_as_float(hi[0]), __uint_as_float(hi[1]));
 }
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {   // one v_cvt_pk_bf16_f32
+  typedef float f2v __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2v __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2v){lo, hi}, b2v));
+}
 
 struct ScanParams {
   const void *x, *dT, *dL, *dy;
@@ -822,10 +827,7 @@ template <> struct Snap<bf16_t> {
   typedef u2v quad;
   static __device__ __forceinline__ quad pack(float a, float b, float c, float d) {
     // (a vector conversion is one v_cvt_pk_bf16_f32 per pair; two scalar casts and an OR are four instructions)
-    typedef float f2v __attribute__((ext_vector_type(2)));
-    typedef __bf16 b2v __attribute__((ext_vector_type(2)));
-    return u2v{__builtin_bit_cast(uint32_t, __builtin_convertvector((f2v){a, b}, b2v)),
-               __builtin_bit_cast(uint32_t, __builtin_convertvector((f2v){c, d}, b2v))};
+    return u2v{pack_bf16(a, b), pack_bf16(c, d)};
   }
   static __device__ __forceinline__ void store(quad* dst, float a, float b, float c, float d) { __builtin_nontemporal_store(pack(a, b, c, d), dst); }
   static __device__ __forceinline__ float4 load(const quad* src) { return widen(*src); }
@@ -1978,10 +1980,15 @@ __global__ __launch_bounds__((NW + (REPLAY ? 0 : whole_helpers<MODE, NW>())) * 6
 // up while the other half is computed.
 // Schedules: one stream per image, or stacked images (not the linked sweep, whose problems are few large images
 // where the snapshots weigh most).
+// The results d_deltaT, d_deltaL, d_x of 16-bit tensors leave workgroups of 32 channels through LDS, 64 bytes of a row at a time
+// (bytes of two steps' tile, 0: every lane stores its own values, 8 bytes of a row at a time).  128 images of 56x56x64 bf16:
+// 0.662 -> 0.645 ms.
+template <typename T, int NW>
+constexpr int bwd2_result_tile() { return sizeof(T) == 2 && NW == kBwdWaves ? 2 * 3 * kHB * 64 : 0; }
 template <typename T, int NW>
 constexpr int bwd2_exchange_sets() {   // sets of [wave][3][64] float2: 2 halves x 2 steps where they fit, else 2 used alternately per step
   if (NW == kFwdHalfWaves) return 8;   // (both halves at once: [sub-block][half][step])
-  return sizeof(float2) * 4 * NW * 3 * 64 + sizeof(float) * NW * 4 * 2 * kN + 256 +
+  return sizeof(float2) * 4 * NW * 3 * 64 + sizeof(float) * NW * 4 * 2 * kN + bwd2_result_tile<T, NW>() +
          2 * (size_t)Stage<T, 4, NW * 4, true>::kBytes + (sizeof(T) == 2 ? 2 * kRawBytes : 0) <= 160 * 1024 ? 4 : 2;
 }
 // Workgroups of 16 channels: two waves share the 4 channels that a wave has otherwise, a half of the states each, both halves of a sub-block
@@ -2025,6 +2032,9 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
   constexpr bool WIDEN = sizeof(T) == 2;
   char* raw = lds + 2 * SG::kBytes;         // [2][kRawBytes]: 16-bit B_T, B_L, C on their way
   const bool direct = WIDEN && p.bc_direct != 0;   // (uniform)
+  constexpr bool TILE = bwd2_result_tile<T, NW>() > 0 && STAGE_X;
+  constexpr bool WIDE = !HALVES && 2 * 3 <= NSTG;   // a wave adds up the same sums in both half-passes of a sub-block and stores them together
+  char* tile = raw + (WIDEN ? 2 * kRawBytes : 0);   // TILE: [step of the sub-block][d_deltaT, d_deltaL, d_x][16 rows][CW] results
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lb = logical_block(p.nwg);
@@ -2098,7 +2108,14 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
   const uint32_t wrap_adj = (uint32_t)(p.rb * p.W - p.S) * estep;
   const uint32_t pstep = (uint32_t)(p.flip ? -1 : 1) * (uint32_t)(3 * kN * sizeof(float));
   const uint32_t pwrap_adj = (uint32_t)(p.rb * p.W - p.S) * pstep;
+  // TILE: pieces of 16 bytes (8 channels) of lane row r are at place piece ^ (r >> 2), so that rows which are written together are in different banks
+  constexpr int kTileBytes = kHB * CW * (int)sizeof(T);
+  const uint32_t tile_put = (uint32_t)((slot < 2 ? slot : 2) * kTileBytes + r * 64 + (((wave >> 1) ^ (r >> 2)) * 16 + (wave & 1) * 8));
+  const uint32_t tile_get = (uint32_t)(r * 64 + (slot ^ (r >> 2)) * 16);
+  const bool tile_ok = e_wg0 + 8 * slot < p.E;
+  static_assert(!TILE || (CW * sizeof(T) == 64 && CS == 4), "a row of the tile is four pieces");
   const uint32_t row_const_off = SG::kConstPlane * SG::kPlane + r * 16;
+  const uint32_t bot_step = (uint32_t)p.E * (uint32_t)(kN * sizeof(float)), bot_wrap = (uint32_t)p.S * bot_step;   // boundary rows: bytes from column to column; back to column 0
 
   BlockPos bp;
   uint32_t cell_off0 = 0, f_off0 = 0;
@@ -2195,6 +2212,14 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
     }
     rp ^= 1;
     if constexpr (SWEEPS) cell_off0 = (uint32_t)(cell0 * p.E + e) * (uint32_t)sizeof(T);
+    // The steps at which the lane holds the first row of a band that has one above (bit k), and where its muT goes in the image's one row
+    // buffer (bands follow each other), modulo 2^32.  (With the band's buffer and two
+    // 64-bit products worked out in every step, 128 images of 56x56x64 bf16: 0.645 -> 0.622 ms; 64 images: 0.358 -> 0.350.)
+    uint32_t bot_off0 = 0, bot_steps = 0;
+    if constexpr (SWEEPS && !STACKED) {
+      bot_off0 = (uint32_t)(bp.col0 * p.E + e) * (uint32_t)(kN * sizeof(float));
+      if (ch_ok && r == 1) bot_steps = bp.bnd0 >= 1 ? bp.in_grid : (bp.bnd0 == 0 && bp.kw < kCK ? bp.in_grid & (15u << bp.kw) : 0u);
+    }
     if constexpr (STAGES) f_off0 = (uint32_t)cell0 * (uint32_t)(3 * kN * sizeof(float)) + (BATCH ? (uint32_t)(slot * 4 * sizeof(float)) : f_sub);
 
 #pragma unroll
@@ -2202,6 +2227,7 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
       const int k0 = 2 * sub;
       float part2[2][4];   // the state sums of the first half wait here for the second
       float2 slope[2];     // (HALVES, a wave that stages)
+      float2 first_sum = make_float2(0.f, 0.f);   // WIDE: the first half's sum waits for the second's (a row's 64 bytes in one store: 0.629 -> 0.621 ms)
 #pragma unroll
       for (int pass = 0; pass < PASSES; ++pass) {
        const int half = HALVES ? my_half : pass;   // (HALVES: uniform)
@@ -2354,12 +2380,9 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
               sw[64 * 2 + mgl] = fold16(fold32(vBT[0], vBT[1]), fold32(vBT[2], vBT[3]));
               sw[128 * 2 + mgl] = fold16(fold32(vBL[0], vBL[1]), fold32(vBL[2], vBL[3]));
             }
-            if (p.nbands > 1 && !p.stacked) {   // first row of a band: the lower ghost of the band above will replay its muT
-              const bool wk = k >= bp.kw;
-              if (inr && r == 1 && (wk ? bp.bnd0 + 1 : bp.bnd0) >= 1) {
-                const int ck = wk ? bp.col0 + k - p.S : bp.col0 + k;
-                char* bb = BOTimg + (wk ? bp.bnd0 + 1 : bp.bnd0) * p.bot_stride * (int64_t)sizeof(float) +
-                           (uint32_t)(ck * p.E + e) * (uint32_t)(kN * sizeof(float));
+            if constexpr (!STACKED) {   // first row of a band: the lower ghost of the band above will replay its muT
+              if ((bot_steps >> k) & 1u) {
+                char* bb = BOTimg + (bot_off0 + (uint32_t)k * bot_step - (k >= bp.kw ? bot_wrap : 0u));
 #pragma unroll
                 for (int ql = 0; ql < 2; ++ql) {
                   const int q0 = HALVES ? 0 : 4 * (2 * pass + ql);   // (a quad is a state group: HALVES has them in place)
@@ -2377,15 +2400,21 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
               part2[ks][0] = sT; part2[ks][1] = sL; part2[ks][2] = zT; part2[ks][3] = zL;
             } else {
               accD = __builtin_fmaf(dyv, xv, accD);
-              if (inr) {
+              if (TILE || inr) {
                 float gdT = __builtin_fmaf(cT * xv, sT, kLn2 * zT), gdL = __builtin_fmaf(cL * xv, sL, kLn2 * zL);
                 if (p.dpre) {   // (uniform) gradients with respect to what the softplus was applied to
                   gdT *= softplus_slope<T>(dtv);
                   gdL *= softplus_slope<T>(dlv);
                 }
-                IO<T>::st(reinterpret_cast<T*>(DDTimg + goff), gdT);
-                IO<T>::st(reinterpret_cast<T*>(DDLimg + goff), gdL);
-                IO<T>::st(reinterpret_cast<T*>(DXimg + goff), __builtin_fmaf(cT * dtv, sT, __builtin_fmaf(cL * dlv, sL, dyv * dsk)));
+                const float gdX = __builtin_fmaf(cT * dtv, sT, __builtin_fmaf(cL * dlv, sL, dyv * dsk));
+                if constexpr (TILE) {   // slots 0, 1, 2 end with d_deltaT, d_deltaL, d_x of the wave's four channels (slot 3 stores what slot 2 does)
+                  const float4 q = slots_turned(make_float4(gdT, gdL, gdX, gdX));
+                  *reinterpret_cast<uint2*>(tile + ks * 3 * kTileBytes + tile_put) = make_uint2(pack_bf16(q.x, q.y), pack_bf16(q.z, q.w));
+                } else {
+                  IO<T>::st(reinterpret_cast<T*>(DDTimg + goff), gdT);
+                  IO<T>::st(reinterpret_cast<T*>(DDLimg + goff), gdL);
+                  IO<T>::st(reinterpret_cast<T*>(DXimg + goff), gdX);
+                }
               }
             }
             if constexpr (!BATCH) {   // ---- across the waves, this step: as in m2d_bwd_kernel
@@ -2416,6 +2445,10 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
           // waves; a thread adds up the float2 of the lane (its slot, its row).  The other half's sets are being
           // filled or added up by then; this half's are filled again two barriers from here.
           __syncthreads();
+          if constexpr (TILE && SWEEPS) {   // the next half-pass's quads, asked for two half-passes ago, are here before stores are sent that nobody waits for
+            quad_t (&q)[2] = qa[pass ^ 1];
+            asm volatile("" : "+v"(q[0]), "+v"(q[1]));
+          }
           if constexpr (STAGES)
 #pragma unroll
           for (int rd = 0; rd < ((HALVES ? 4 : 2) * 3 + NSTG - 1) / NSTG; ++rd) {
@@ -2430,7 +2463,19 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
                 float2 sum = sl[0];
 #pragma unroll
                 for (int w = 1; w < NW; ++w) { sum.x += sl[w * SLOT].x; sum.y += sl[w * SLOT].y; }
-                *reinterpret_cast<float2*>(PARTimg + off) = sum;
+                if constexpr (WIDE) {
+                  if (pass == 0) first_sum = sum;
+                  else *reinterpret_cast<float4*>(PARTimg + (off - (uint32_t)(2 * sizeof(float)))) = make_float4(first_sum.x, first_sum.y, sum.x, sum.y);
+                } else {
+                  *reinterpret_cast<float2*>(PARTimg + off) = sum;
+                }
+                if constexpr (TILE) {
+                  if (pass == 1 && tile_ok) {
+                    char* img = v == 0 ? DDTimg : (v == 1 ? DDLimg : DXimg);
+                    const uint32_t to = (uint32_t)(cell0 * p.E + e_wg0 + 8 * slot) * (uint32_t)sizeof(T) + (uint32_t)k * estep + (k >= bp.kw ? wrap_adj : 0u);   // (modulo 2^32: the row's first cell may be off the grid)
+                    *reinterpret_cast<uint4*>(img + to) = *reinterpret_cast<const uint4*>(tile + jj * kTileBytes + tile_get);
+                  }
+                }
               }
             }
           }
@@ -3100,12 +3145,12 @@ int stage_bc(ScanParams& sp, const m2d_desc* d, const void* BT, const void* BL, 
 }
 
 // Development aid: -DM2D_QUICK=1 builds only the kernels of many 16-bit images in one stream each, in workgroups of
-// 8 waves (a twentieth of the compile time), -DM2D_QUICK=2 (3) only the linked sweep of fp32 (16-bit) images in workgroups of 4 waves, =4 (5) one stream per 16-bit (fp32) image in those;
+// 8 waves (a twentieth of the compile time), -DM2D_QUICK=2 (3) only the linked sweep of fp32 (16-bit) images in workgroups of 4 waves, =4 (5) one stream per 16-bit (fp32) image in those, =6 one stream per 16-bit image in either;
 // every other problem then answers M2D_ERR_UNSUPPORTED.
 #if defined(M2D_QUICK) && M2D_QUICK >= 2 && M2D_QUICK <= 3
 #define M2D_BUILT(T, SX, MODE, NW, OTHER) (sizeof(T) == (M2D_QUICK == 3 ? 2 : 4) && (MODE) == kModeSliced && (NW) == 4)
 #elif defined(M2D_QUICK)
-#define M2D_BUILT(T, SX, MODE, NW, OTHER) (sizeof(T) == (M2D_QUICK == 5 ? 4 : 2) && (SX) && (MODE) == kModeSweep && (NW) == (M2D_QUICK == 1 ? 8 : 4) && ((OTHER) || M2D_QUICK > 3))
+#define M2D_BUILT(T, SX, MODE, NW, OTHER) (sizeof(T) == (M2D_QUICK == 5 ? 4 : 2) && (SX) && (MODE) == kModeSweep && (M2D_QUICK == 6 || (NW) == (M2D_QUICK == 1 ? 8 : 4)) && ((OTHER) || M2D_QUICK > 3))
 #else
 #define M2D_BUILT(T, SX, MODE, NW, OTHER) true
 #endif
@@ -3266,7 +3311,7 @@ int launch_bwd_as(const ScanParams& sp, hipStream_t st) {
 
 template <typename T, int NW>
 constexpr size_t bwd2_lds_bytes() {
-  return sizeof(float2) * bwd2_exchange_sets<T, NW>() * NW * 3 * 64 + sizeof(float) * NW * 4 * 2 * kN + (bwd2_halves<NW>() ? sizeof(float) * 3 * 8 * NW * 64 : 256) +
+  return sizeof(float2) * bwd2_exchange_sets<T, NW>() * NW * 3 * 64 + sizeof(float) * NW * 4 * 2 * kN + (bwd2_halves<NW>() ? sizeof(float) * 3 * 8 * NW * 64 : bwd2_result_tile<T, NW>()) +
          2 * (size_t)Stage<T, 4, NW * 4, true>::kBytes + (sizeof(T) == 2 ? 2 * kRawBytes : 0);
 }
 template <typename T, bool SX, int MODE, int NW = kBwdWaves>
