@@ -167,6 +167,14 @@ __device__ __forceinline__ void split_store(bf16_t* dst, float v, bool live) {
   const uint32_t bits = f32_to_bf16_bits(v);
   asm volatile("s_and_saveexec_b64 %0, %3\n\tglobal_store_short %1, %2, off\n\ts_mov_b64 exec, %0" : "=&s"(saved) : "v"(dst), "v"(bits), "s"(__ballot(live)) : "memory", "scc");
 }
+// two neighbouring values
+__device__ __forceinline__ void split_store_pair(float* dst, float a, float b, bool live) {
+  uint64_t saved;
+  typedef float v2f_t __attribute__((ext_vector_type(2)));
+  const v2f_t w = {a, b};
+  asm volatile("s_and_saveexec_b64 %0, %3\n\tglobal_store_dwordx2 %1, %2, off\n\ts_mov_b64 exec, %0" : "=&s"(saved) : "v"(dst), "v"(w), "s"(__ballot(live)) : "memory", "scc");
+}
+__device__ __forceinline__ void split_store_pair(bf16_t* dst, float a, float b, bool live) { split_store4(dst, __uint_as_float(pack_bf16(a, b)), live); }
 // four neighbouring values
 __device__ __forceinline__ void split_store_quad(float* dst, float4 v, bool live) {
   uint64_t saved;
@@ -762,6 +770,10 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_bwd_split_kerne
     const uint32_t k_off = SG::kConst + r * 16;
     const uint32_t x_off = SG::x_off(ch, r, e_wg0);
     char* xw = lds + L::kX + ch * 1024 + lane * 16;
+    // the shares of a row are at place row ^ 4 (pair of channels) ^ 8 (step of the phase): 16 lanes of the wave that adds them up read four
+    // rows of four (pair, step), which are in different banks then
+    char* xw_share = lds + L::kX + 3 * L::kKind + ch * 1024 + (SX ? (lane ^ ((ch >> 1) * 4)) : lane) * 16;
+    char* xw_share_odd = lds + L::kX + 3 * L::kKind + ch * 1024 + (lane ^ ((ch >> 1) * 4) ^ 8) * 16;
     char* rw = lds + L::kR + ch * 64 + g * 16;
     const bool first_row = r == 1 && p.nbands > 1;         // the band's first row: the lower ghost of the band above will replay its muT
     Pos at = pos_of(p, (m_hi - 1) * kCK - r);              // the row at the first step of the block
@@ -871,7 +883,9 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_bwd_split_kerne
         const float pT = __builtin_fmaf(cT * xv, sT, kLn2 * zT);
         const float pL = __builtin_fmaf(cL * xv, sL, kLn2 * zL);
         const float pX = __builtin_fmaf(cT * dtv, sT, cL * dlv * sL);
-        *reinterpret_cast<float4*>(xs + 3 * L::kKind) = make_float4(pT, pL, pX, g == 0 ? dtv : (g == 1 ? dlv : dyv * dsk));
+        char* xsh = xw_share + par * L::kXBytes + (XS == 1 ? 0 : k % XS) * L::kXStep;
+        if (SX && XS > 1 && k % XS == 1) xsh = xw_share_odd + par * L::kXBytes + L::kXStep;
+        *reinterpret_cast<float4*>(xsh) = make_float4(pT, pL, pX, g == 0 ? dtv : (g == 1 ? dlv : dyv * dsk));
         if (first_row) *reinterpret_cast<float4*>(rw + par * L::kRBytes + (XS == 1 ? 0 : k % XS) * L::kRStep) = make_float4(muT[0], muT[1], muT[2], muT[3]);
         if (k == 0) fetch(next, 0, ops[0]);   // (the operands of the block before are in place since the phase before; behind the last block: never used)
         if (k % XS == 0) { __syncthreads(); par ^= 1; }
@@ -929,7 +943,8 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_bwd_split_kerne
     auto buf_of = [&](int j) { return (uint32_t)(j % L::kBufs) * (uint32_t)SG::kBytes; };   // j: block of the window, from its end
     // Every block issues the same operations, also those behind the window (which fetch zeros): the waits below count on it.
     constexpr int kCopies = 4, kRawCopies = 2, kXCopies = (SX ? 4 * SG::kChunks : 0) + SG::kG4;   // per block: of a wave of 0..2; of wave 3
-    constexpr int kStores = XS + XS * (CW / 4);         // a wave's sums and results per phase
+    // a wave's stores per phase: sums and results (SX: wave 2 all results)
+    constexpr int kStores = SX ? XS : XS + XS * (CW / 4), kStores2 = SX ? XS + 3 : kStores;
     auto stage_bc = [&](uint32_t buf) {                        // (waves 0..2)
       if (raw) {
         split_raw_copy<SG>(bq.on(p) ? bc.mine + cell_bytes_off(bq.cell, bc_cell) : zeros, buf + sw * SG::kBCTensor);
@@ -988,9 +1003,36 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_bwd_split_kerne
         split_store_quad(reinterpret_cast<float*>(PARTimg + cell_bytes_off(t.cell, 3 * kN * sizeof(float)) + sum_off), slots_turned(sum[ks]), t.on(p));
       }
     };
-    // d_deltaT, d_deltaL, d_x by the waves 0, 1, 2; lane (row, channel of four)
-    char* const out_img = static_cast<char*>(sw == 0 ? p.ddT : (sw == 1 ? p.ddL : p.dx)) + img_bytes;
+    // d_deltaT, d_deltaL, d_x.  SX: by wave 2, which has all four shares of a channel's results from four reads: lane (row, two neighbouring channels[, step of the phase]).
+    // Otherwise a tensor each by the waves 0, 1, 2; lane (row, channel of four).
     auto send_results = [&](const Tr& t0, int k0, int par) {
+      if constexpr (SX) {
+        if (sw != 2) return;
+        constexpr int kPairs = CW / 2;
+        static_assert(kPairs * XS == 4, "a wave has the results of a phase");
+        const int row = lane >> 2, pair = lane % kPairs, ks = XS == 1 ? 0 : (lane / kPairs) & 1;
+        const Tr t = t0.moved(p, k0 + ks);
+        const bool ok = t.on(p) && e_wg0 + 2 * pair < p.E;
+        const float4* sh = reinterpret_cast<const float4*>(lds + L::kX + par * L::kXBytes + ks * L::kXStep + 3 * L::kKind + pair * 2048) + (row ^ (pair * 4) ^ (ks * 8));
+        float vT[2], vL[2], vX[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const float4 q0 = sh[c * 64], q1 = sh[c * 64 + 16], q2 = sh[c * 64 + 32], q3 = sh[c * 64 + 48];
+          vT[c] = (q0.x + q1.x) + (q2.x + q3.x);
+          vL[c] = (q0.y + q1.y) + (q2.y + q3.y);
+          vX[c] = (q0.z + q1.z) + (q2.z + q3.z) + q2.w;
+          if (p.dpre) {   // (uniform) gradients with respect to what the softplus was applied to
+            vT[c] *= softplus_slope<T>(q0.w);
+            vL[c] *= softplus_slope<T>(q1.w);
+          }
+        }
+        const uint32_t off = cell_bytes_off(t.cell, (uint32_t)p.E * (uint32_t)sizeof(T)) + (uint32_t)(e_wg0 + 2 * pair) * (uint32_t)sizeof(T);
+        split_store_pair(reinterpret_cast<T*>(static_cast<char*>(p.ddT) + img_bytes + off), vT[0], vT[1], ok);
+        split_store_pair(reinterpret_cast<T*>(static_cast<char*>(p.ddL) + img_bytes + off), vL[0], vL[1], ok);
+        split_store_pair(reinterpret_cast<T*>(static_cast<char*>(p.dx) + img_bytes + off), vX[0], vX[1], ok);
+        return;
+      }
+      char* const out_img = static_cast<char*>(sw == 0 ? p.ddT : (sw == 1 ? p.ddL : p.dx)) + img_bytes;
       const int row = lane >> 2, c4 = lane & 3;
 #pragma unroll
       for (int ks = 0; ks < XS; ++ks) {
@@ -1049,8 +1091,8 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_bwd_split_kerne
           }
           if (ph == 0) {                                    // block j + 1 has landed; the block fetched behind it, and what was stored since, may be under way
             stage_bc(buf_of(j + 2));
-            if (raw) { if (j == 0) split_landed<kRawCopies>(); else split_landed<PH * kStores + kRawCopies>(); }
-            else { if (j == 0) split_landed<kCopies>(); else split_landed<PH * kStores + kCopies>(); }
+            if (raw) { if (j == 0) split_landed<kRawCopies>(); else { if (sw == 2) split_landed<PH * kStores2 + kRawCopies>(); else split_landed<PH * kStores + kRawCopies>(); } }
+            else { if (j == 0) split_landed<kCopies>(); else { if (sw == 2) split_landed<PH * kStores2 + kCopies>(); else split_landed<PH * kStores + kCopies>(); } }
             widen(buf_of(j + 1));
           }
         } else {
