@@ -220,6 +220,7 @@ struct ScanParams {
   // that reads its boundary rows polls that count before it stages them.
   int sliced;                       // on/off
   int sl_nbb;                       // blocks per band (S / kCK)
+  int sl_unit, sl_units;            // workgroups of a band and image that go to one XCD together, at most, and how many such units those are (linked_place)
   uint32_t* prog;                   // [nbands][B][workgroups per image] blocks of the band's window whose boundary rows are in memory
   uint32_t* link_err;               // set to 1 by a workgroup that gave up waiting (results are then invalid)
   int link_test;                    // test aid (M2D_FLAG_TEST_DEAD_LINK): 1 + the band whose neighbour never reports, and a wait gives up after a few polls
@@ -253,6 +254,23 @@ __device__ __forceinline__ int logical_block(int nwg) {
   const int per = nwg >> 3;
   if (per == 0 || id >= (per << 3)) return id;
   return (id & 7) * per + (id >> 3);
+}
+
+// Which band (by its turn) and which workgroup of it the workgroup sweeps in a linked launch; false: none, the grid is rounded up.
+// Workgroups are dealt round-robin to the 8 XCDs.  Neighbouring channel groups of a band read the same B_T, B_L, C and the same cache lines of
+// x, deltaT, deltaL: `sl_unit` of them at a time are on one XCD, whose L2 then fetches those once and not up to 8 times.  Units follow each
+// other band by band, so a band's neighbour of the turn before has a lower index still: unit u - n, n >= 1, is either on a lower XCD in the same
+// eight, or in an earlier eight.  Forward keeping snapshots / backward against
+// workgroups in the order of bands and channels: 1x256x256x64 fp32 0.246 / 0.397 -> 0.221 / 0.368 ms, 512x512 0.577 / 1.090 -> 0.487 / 0.925,
+// 1024x1024 1.44 / 3.33 -> 1.33 / 3.01, 4x128x128x64 bf16 0.132 / 0.255 -> 0.115 / 0.245.
+__device__ __forceinline__ bool linked_place(const ScanParams& p, int& turn, int& lb) {
+  const int id = blockIdx.x, q = id >> 3, unit = q / p.sl_unit * 8 + (id & 7);
+  const int per_band = p.B * p.sl_units;
+  turn = unit / per_band;
+  const int rest = unit - turn * per_band, img = rest / p.sl_units, part = rest - img * p.sl_units;
+  const int eg = part * p.bpb / p.sl_units + q % p.sl_unit;      // (units of an image differ by one workgroup at most)
+  lb = img * p.bpb + eg;
+  return turn < p.nbands && eg < (part + 1) * p.bpb / p.sl_units;
 }
 
 // Stream position -> (band, column).  s >= -21 (S >= 7, so 3 strides below zero are in range).
@@ -900,14 +918,14 @@ __global__ __launch_bounds__((NW + whole_helpers<MODE, NW, EC>()) * 64) void m2d
   char* lds = reinterpret_cast<char*>(smem);       // two staging buffers
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int lb = SLICED ? (int)blockIdx.x : logical_block(p.nwg);   // (linked bands keep the launch order: a band waits for a lower index)
+  int lb = 0, turn = 0;
+  if constexpr (SLICED) { if (!linked_place(p, turn, lb)) return; } else lb = logical_block(p.nwg);
   int m_lo = 0, m_hi = p.nblk;                     // blocks of steps this workgroup sweeps
   int my_band = 0;
   LinkT<NH ? NW * 64 : 0> link;
   if constexpr (SLICED) {   // the window of one band
     const int per = p.B * p.bpb;
-    my_band = lb / per;
-    lb -= my_band * per;
+    my_band = turn;
     m_lo = my_band * p.sl_nbb;
     m_hi = m_lo + p.sl_nbb;
     link.mine = p.prog + ((int64_t)my_band * per + lb) * kLinkStride;
@@ -1404,15 +1422,14 @@ __global__ __launch_bounds__((NW + (REPLAY ? 0 : whole_helpers<MODE, NW>())) * 6
   const bool direct = WIDEN && p.bc_direct != 0;   // (uniform)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int lb = SLICED ? (int)blockIdx.x : logical_block(p.nwg);   // (linked bands keep the launch order: a band waits for a lower index)
+  int lb = 0, turn = 0;
+  if constexpr (SLICED) { if (!linked_place(p, turn, lb)) return; } else lb = logical_block(p.nwg);
   int m_lo = 0, m_hi = p.nblk;              // blocks of steps this workgroup sweeps (from m_hi - 1 down to m_lo)
   int my_band = 0;
   LinkT<NH ? NW * 64 : 0> link;
   if constexpr (SLICED) {   // the window of one band; the bands are launched from the last to the first
     const int per = p.B * p.bpb;
-    const int kk = lb / per;
-    lb -= kk * per;
-    my_band = p.nbands - 1 - kk;
+    my_band = p.nbands - 1 - turn;
     m_lo = my_band * p.sl_nbb;
     m_hi = m_lo + p.sl_nbb;
     link.mine = p.prog + ((int64_t)my_band * per + lb) * kLinkStride;
@@ -1527,7 +1544,7 @@ __global__ __launch_bounds__((NW + (REPLAY ? 0 : whole_helpers<MODE, NW>())) * 6
     } else {
       const int mem = member(mm);
       typename Snap<ST>::quad* base =
-          mem != 0 ? static_cast<typename Snap<ST>::quad*>(p.ring) + ((int64_t)blockIdx.x * ((1 << p.ck_shift) - 1) + (mem - 1)) * kRingSlot - e_wg0 * (kN / 4 * kHB)
+          mem != 0 ? static_cast<typename Snap<ST>::quad*>(p.ring) + ((int64_t)(SLICED ? turn * p.B * p.bpb + lb : (int)blockIdx.x) * ((1 << p.ck_shift) - 1) + (mem - 1)) * kRingSlot - e_wg0 * (kN / 4 * kHB)
                    : snapshot_at<ST>(p, b, snapshot_index<SLICED>(p, mm, m_lo, my_band), 0, p.ck_nblk);
       return base + (e * (kN / 4 * kHB) + snap_lane(r));
     }
@@ -3085,6 +3102,22 @@ void fill_common(ScanParams& sp, const m2d_desc* d, const Geometry& g) {
   sp.ring = nullptr;
 }
 
+// Workgroups of a linked launch (see linked_place), whole eights of units.  Units of 4, 8 and 16 are within 2 % of each other where not all units of the
+// device are taken; larger ones put a band of many channels on one or two XCDs (64: 1x84x123x216 bf16 0.070 / 0.165 -> 0.099 / 0.228 ms).  Where bands
+// have to wait for a compute unit, an XCD whose units are the larger ones holds everyone up: there units are of one size, which fits the 32 compute
+// units of an XCD, or bands of so many workgroups that it matters little, or workgroups go out in order (fp32, backward, in units of up to 8 against in order:
+// 5x37x45x100 82.7 and 71.7 us, 1x601x768x136 2.91 and 2.60 ms; 1x335x418x456 2.51 and 2.62, 1024x1024x64 3.01 and 3.33).  The forward of one image
+// is faster in units of 8 throughout (keeping snapshots, 1x601x768x136 1.10 and 1.13 ms, 1x892x601x88 1.04 and 1.10, 1x686x690x140 1.12 and 1.22), of several not (3x298x359x208 1.56 and 1.51).
+inline int linked_grid(ScanParams& sp, bool forward) {
+  const int lagged = (sp.sl_nbb + kLinkLag) / (kLinkLag + 1), under_way = lagged < sp.nbands ? lagged : sp.nbands;
+  const bool wait = 8 * (int64_t)sp.B * sp.bpb * under_way > 7 * (int64_t)device_cus();
+  const int want = !wait || (forward && sp.B == 1) || sp.bpb >= 48 || sp.bpb % 8 == 0 ? 8 : sp.bpb % 4 == 0 ? 4 : sp.bpb % 2 == 0 ? 2 : 1;
+  sp.sl_units = (sp.bpb + want - 1) / want;
+  sp.sl_unit = (sp.bpb + sp.sl_units - 1) / sp.sl_units;
+  const int64_t units = (int64_t)sp.nbands * sp.B * sp.sl_units;
+  return (int)((units + 7) / 8 * 8 * sp.sl_unit);
+}
+
 // A kernel that needs more than 64 KB of dynamic LDS has to be told so once per device (each
 // device loads its own copy of the code object).  `seen` holds one bit per device ordinal.
 inline bool allow_dynamic_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& seen) {
@@ -3260,7 +3293,7 @@ int launch_fwd(const ScanParams& sp0, const m2d_desc* d, const Geometry& g, bool
     return g.stage_x ? launch_fwd_mode<T, 1, true, kModeSweep>(sp, ckpt, write_y, st) : launch_fwd_mode<T, 1, false, kModeSweep>(sp, ckpt, write_y, st);
   };
   if (g.sliced) {   // every band on workgroups of its own, band 0 first: a band waits for the one before it
-    sp.nwg = g.nbands * g.vB * g.fwd_bpb;
+    sp.nwg = linked_grid(sp, true);
     sp.prog = sp.link_err + 64;
   }
   return once();
@@ -3406,7 +3439,7 @@ int run_bwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
     else rc = g.stage_x ? launch_bwd<T, true, kModeSweep>(sp, st, g.bwd_nw, g.snap32) : launch_bwd<T, false, kModeSweep>(sp, st, g.bwd_nw, g.snap32);
   } else {
     // every band on workgroups of its own, the last band first: a band waits for the one below it
-    sp.nwg = g.nbands * g.vB * g.bwd_bpb;
+    sp.nwg = linked_grid(sp, false);
     sp.prog = sp.link_err + 64 + (size_t)g.nbands * g.vB * (g.fwd_bpb > g.bwd_bpb ? g.fwd_bpb : g.bwd_bpb) * kLinkStride;
     if (g.bwd_split) rc = launch_bwd_split<T, kModeSliced>(sp, g.stage_x, st, g.bwd_nw);
     else rc = g.stage_x ? launch_bwd<T, true, kModeSliced>(sp, st, g.bwd_nw, g.snap32) : launch_bwd<T, false, kModeSliced>(sp, st, g.bwd_nw, g.snap32);

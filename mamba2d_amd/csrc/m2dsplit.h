@@ -335,14 +335,14 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_fwd_split_kerne
   char* lds = reinterpret_cast<char*>(smem);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int lb = SLICED ? (int)blockIdx.x : logical_block(p.nwg);
+  int lb = 0, turn = 0;
+  if constexpr (SLICED) { if (!linked_place(p, turn, lb)) return; } else lb = logical_block(p.nwg);
   int m_lo = 0, m_hi = p.nblk;
   int my_band = 0;
   LinkT<(NW + 3) * 64> link;
   if constexpr (SLICED) {
     const int per = p.B * p.bpb;
-    my_band = lb / per;
-    lb -= my_band * per;
+    my_band = turn;
     m_lo = my_band * p.sl_nbb;
     m_hi = m_lo + p.sl_nbb;
     link.mine = p.prog + ((int64_t)my_band * per + lb) * kLinkStride;
@@ -717,15 +717,14 @@ __global__ __launch_bounds__((NW + kSplitStagers) * 64) void m2d_bwd_split_kerne
   char* lds = reinterpret_cast<char*>(smem);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int lb = SLICED ? (int)blockIdx.x : logical_block(p.nwg);
+  int lb = 0, turn = 0;
+  if constexpr (SLICED) { if (!linked_place(p, turn, lb)) return; } else lb = logical_block(p.nwg);
   int m_lo = 0, m_hi = p.nblk;
   int my_band = 0;
   LinkT<(NW + 3) * 64> link;
   if constexpr (SLICED) {   // the window of one band; the bands are launched from the last to the first
     const int per = p.B * p.bpb;
-    const int kk = lb / per;
-    lb -= kk * per;
-    my_band = p.nbands - 1 - kk;
+    my_band = p.nbands - 1 - turn;
     m_lo = my_band * p.sl_nbb;
     m_hi = m_lo + p.sl_nbb;
     link.mine = p.prog + ((int64_t)my_band * per + lb) * kLinkStride;
