@@ -422,7 +422,9 @@ int m2d_widen(int nsegs, const m2d_widen_seg* segs, void* stream);
  * m2d_train_linear_bwd: for y = post(pre(x) weight^T + b) with z the value before post: dx from dy.  post_act nothing or
  *   GELU, pre_act any; pre StarReLU leaves part: (slices, 2) sums for its scale and bias.  K a multiple of 16, N of 32,
  *   both up to 512.
- * m2d_train_wgrad: part: (slices, N K + N) sums for the weight and, with `bias`, the bias of that layer. */
+ * m2d_train_wgrad: part: (slices, N K + N) sums for the weight and, with `bias`, the bias of that layer.
+ * m2d_train_linear_grads: both of the above in one pass, for the shapes (and slices) for which its _parts query is not 0: dx, part as
+ *   m2d_train_wgrad, star_part: (slices, 2) sums for the StarReLU's scale and bias where pre_act is one. */
 int m2d_train_norm_fwd(int64_t rows, int C, int rows_per_sample, const float* x, const float* scale, const void* r, const void* r2,
                        const float* keep, float* x_out, const float* w1, const float* b1, float eps1, void* y1,
                        const float* w2, const float* b2, float eps2, void* y2, void* stream);
@@ -437,6 +439,9 @@ int m2d_train_dwconv_bwd(int B, int H, int W, int C, const void* p, const void* 
 int m2d_train_linear_parts(int64_t P, int K, int N);
 int m2d_train_linear_bwd(int64_t P, int K, int N, const void* dy, const void* z, int post_act, const float* weight, const void* x,
                          int pre_act, const float* pre_scale, void* dx, float* part, void* stream);
+int m2d_train_linear_grads_parts(int64_t P, int N, int K);
+int m2d_train_linear_grads(int64_t P, int N, int K, const void* dy, const void* z, int post_act, const float* weight, const void* x, int pre_act,
+                           const float* pre_scale, const float* pre_bias, int bias, void* dx, float* part, float* star_part, void* stream);
 int m2d_train_wgrad_parts(int64_t P, int N, int K);
 int m2d_train_wgrad(int64_t P, int N, int K, const void* dy, const void* z, int post_act, const void* x, int pre_act,
                     const float* pre_scale, const float* pre_bias, int bias, float* part, void* stream);

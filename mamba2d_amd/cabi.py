@@ -32,7 +32,7 @@ EXPORTS = ("m2d_version", "m2d_status_str", "m2d_desc_check", "m2d_scan_workspac
            "m2d_scale_residual_fwd", "m2d_scale_residual_layernorm_fwd", "m2d_rope_qknorm_fwd", "m2d_rope_attention_fwd", "m2d_mlp_fwd", "m2d_layernorm_linear_fwd", "m2d_linear_fwd", "m2d_profile_enable", "m2d_profile_last_ms", "m2d_valu_rate_probe", "m2d_wf_fwd", "m2d_wf_bwd",
            "m2d_widen", "m2d_wide_linear_fwd", "m2d_linear_keep_fwd", "m2d_starrelu_dwconv3x3_fwd", "m2d_train_norm_fwd", "m2d_train_norm_parts", "m2d_train_norm_bwd",
            "m2d_train_branch", "m2d_train_dwconv_parts", "m2d_train_dwconv_bwd", "m2d_train_linear_parts", "m2d_train_linear_bwd",
-           "m2d_train_wgrad_parts", "m2d_train_wgrad", "m2d_train_reduce")
+           "m2d_train_wgrad_parts", "m2d_train_wgrad", "m2d_train_linear_grads_parts", "m2d_train_linear_grads", "m2d_train_reduce")
 
 
 class Desc(ctypes.Structure):

@@ -182,14 +182,15 @@ struct Block : public torch::autograd::Function<Block> {
     auto take = [&](int64_t n) { const int64_t o = at; at += (n + 63) / 64 * 64; return o; };
     const int np = m2d_train_norm_parts(s.P, C);
     const int64_t o_n2 = take((int64_t)np * 5 * C), o_n1 = take((int64_t)np * 5 * C);
-    struct W { int w, b, N, K, parts; int64_t off; };
-    std::vector<W> ws = {{kFc2W, kFc2B, C, HD, 0, 0}, {kFc1W, kFc1B, HD, C, 0, 0}, {kOutW, kOutB, C, C, 0, 0}, {kInW, kInB, C, C, 0, 0}};
-    if (s.local) { ws.push_back({kPw2, -1, C, M, 0, 0}); ws.push_back({kPw1, -1, M, C, 0, 0}); }
+    struct W { int w, b, N, K, parts; int64_t off; bool both; };      // both: input's and weight's gradient from one kernel
+    std::vector<W> ws = {{kFc2W, kFc2B, C, HD, 0, 0, false}, {kFc1W, kFc1B, HD, C, 0, 0, false}, {kOutW, kOutB, C, C, 0, 0, false}, {kInW, kInB, C, C, 0, 0, false}};
+    if (s.local) { ws.push_back({kPw2, -1, C, M, 0, 0, false}); ws.push_back({kPw1, -1, M, C, 0, 0, false}); }
     for (auto& w : ws) {
-      w.parts = m2d_train_wgrad_parts(s.P, w.N, w.K);
+      w.both = m2d_train_linear_grads_parts(s.P, w.N, w.K) > 0;
+      w.parts = w.both ? m2d_train_linear_grads_parts(s.P, w.N, w.K) : m2d_train_wgrad_parts(s.P, w.N, w.K);
       w.off = take((int64_t)w.parts * ((int64_t)w.N * w.K + w.N));
     }
-    const int lp = s.local ? m2d_train_linear_parts(s.P, M, C) : 0, dp = s.local ? m2d_train_dwconv_parts((int)s.B, (int)s.H, (int)s.W, M) : 0;
+    const int lp = !s.local ? 0 : ws[4].both ? ws[4].parts : m2d_train_linear_parts(s.P, M, C), dp = s.local ? m2d_train_dwconv_parts((int)s.B, (int)s.H, (int)s.W, M) : 0;
     TORCH_CHECK(!s.local || (lp > 0 && dp > 0), "m2dscan: block shapes outside what the training kernels are built for");
     const int64_t o_s2 = take((int64_t)lp * 2), o_dw = take((int64_t)dp * (9 * M + 2));
     Tensor part_t = at::empty({at}, x.options());
@@ -198,27 +199,29 @@ struct Block : public torch::autograd::Function<Block> {
       out[i] = at::empty_like(p[i]);
       segs.push_back({part + off, out[i].data_ptr<float>(), stride, (int32_t)p[i].numel(), parts});
     };
-    auto wgrad = [&](int i, const Tensor& g, const Tensor* z, const Tensor& in, int act, const float* as, const float* ab) {
+    // layer i: the gradient dx of its input `in` and the sums for its weight and bias, from the gradient g of its output (before a GELU behind it, with z)
+    auto layer = [&](int i, const Tensor& g, const Tensor* z, const Tensor& in, int act, const float* as, const float* ab, Tensor& dx, float* sums) {
       const W& w = ws[i];
-      check(m2d_train_wgrad(s.P, w.N, w.K, g.data_ptr(), z ? z->data_ptr() : nullptr, z ? M2D_ACT_GELU : M2D_ACT_NONE, in.data_ptr(), act, as,
-                            ab, w.b >= 0, part + w.off, st));
+      const int post = z ? M2D_ACT_GELU : M2D_ACT_NONE;
+      const void* zp = z ? z->data_ptr() : nullptr;
+      if (w.both) {
+        check(m2d_train_linear_grads(s.P, w.N, w.K, g.data_ptr(), zp, post, f32(p[w.w]), in.data_ptr(), act, as, ab, w.b >= 0, dx.data_ptr(),
+                                     part + w.off, sums, st));
+      } else {
+        check(m2d_train_linear_bwd(s.P, w.K, w.N, g.data_ptr(), zp, post, f32(p[w.w]), act != M2D_ACT_NONE ? in.data_ptr() : nullptr, act, as,
+                                   dx.data_ptr(), sums, st));
+        check(m2d_train_wgrad(s.P, w.N, w.K, g.data_ptr(), zp, post, in.data_ptr(), act, as, ab, w.b >= 0, part + w.off, st));
+      }
       const int64_t stride = (int64_t)w.N * w.K + w.N;
       seg(w.w, w.off, stride, w.parts);
       if (w.b >= 0) seg(w.b, w.off + (int64_t)w.N * w.K, stride, w.parts);
-    };
-    auto dgrad = [&](int K, int N, const Tensor& g, const Tensor* z, const Tensor& w, const Tensor* in, int act, const float* as, Tensor& dx,
-                     float* sums) {
-      check(m2d_train_linear_bwd(s.P, K, N, g.data_ptr(), z ? z->data_ptr() : nullptr, z ? M2D_ACT_GELU : M2D_ACT_NONE, f32(w),
-                                 in ? in->data_ptr() : nullptr, act, as, dx.data_ptr(), sums, st));
     };
 
     // MLP
     Tensor dm = bf16_like(x, C), dh = bf16_like(x, HD), dn = bf16_like(x, C);
     check(m2d_train_branch(s.P * C, (int64_t)rps * C, f32(dy), keep2.defined() ? f32(keep2) : nullptr, dm.data_ptr(), st));
-    dgrad(HD, C, dm, nullptr, p[kFc2W], &h0, M2D_ACT_GELU, nullptr, dh, nullptr);
-    wgrad(0, dm, nullptr, h0, M2D_ACT_GELU, nullptr, nullptr);
-    dgrad(C, HD, dh, nullptr, p[kFc1W], nullptr, M2D_ACT_NONE, nullptr, dn, nullptr);
-    wgrad(1, dh, nullptr, n2, M2D_ACT_NONE, nullptr, nullptr);
+    layer(0, dm, nullptr, h0, M2D_ACT_GELU, nullptr, nullptr, dh, nullptr);
+    layer(1, dh, nullptr, n2, M2D_ACT_NONE, nullptr, nullptr, dn, nullptr);
     // second update and norm2; dm takes the gradient of the mixer's answer
     Tensor dx1 = at::empty_like(x);
     check(m2d_train_norm_bwd(s.P, C, rps, f32(x1), dn.data_ptr(), nullptr, f32(dy), f32(p[kRs2]), keep1.defined() ? f32(keep1) : nullptr,
@@ -229,19 +232,16 @@ struct Block : public torch::autograd::Function<Block> {
     if (s.local) {
       Tensor dc = bf16_like(x, M), dpre = bf16_like(x, M);
       dl = bf16_like(x, C);
-      dgrad(M, C, dm, nullptr, p[kPw2], &conv, M2D_ACT_STARRELU, f32(p[kS2S]), dc, part + o_s2);
-      wgrad(4, dm, nullptr, conv, M2D_ACT_STARRELU, f32(p[kS2S]), f32(p[kS2B]));
+      layer(4, dm, nullptr, conv, M2D_ACT_STARRELU, f32(p[kS2S]), f32(p[kS2B]), dc, part + o_s2);
       seg(kS2S, o_s2, 2, lp); seg(kS2B, o_s2 + 1, 2, lp);
       check(m2d_train_dwconv_bwd((int)s.B, (int)s.H, (int)s.W, M, pre.data_ptr(), dc.data_ptr(), f32(p[kDw]), f32(p[kS1S]), f32(p[kS1B]),
                                  dpre.data_ptr(), part + o_dw, st));
       seg(kDw, o_dw, 9 * M + 2, dp); seg(kS1S, o_dw + 9 * M, 9 * M + 2, dp); seg(kS1B, o_dw + 9 * M + 1, 9 * M + 2, dp);
-      dgrad(C, M, dpre, nullptr, p[kPw1], nullptr, M2D_ACT_NONE, nullptr, dl, nullptr);
-      wgrad(5, dpre, nullptr, nl, M2D_ACT_NONE, nullptr, nullptr);
+      layer(5, dpre, nullptr, nl, M2D_ACT_NONE, nullptr, nullptr, dl, nullptr);
     }
     // scan path
     Tensor dyy = dn;
-    dgrad(C, C, dm, nullptr, p[kOutW], &y, M2D_ACT_GELU, nullptr, dyy, nullptr);
-    wgrad(2, dm, nullptr, y, M2D_ACT_GELU, nullptr, nullptr);
+    layer(2, dm, nullptr, y, M2D_ACT_GELU, nullptr, nullptr, dyy, nullptr);
     Tensor low, dT, dL, BC, ck;
     const Tensor no_bc = at::empty({0}, u.options());
     if (full) {
@@ -256,8 +256,7 @@ struct Block : public torch::autograd::Function<Block> {
     out[kATLog] = g[3]; out[kALLog] = g[4]; out[kD] = g[8];
     std::tie(out[kXProj], out[kDtTW], out[kDtTB], out[kDtLW], out[kDtLB]) =
         m2dshim::proj_bwd(u, low, dT, dL, p[kXProj], p[kDtTW], p[kDtLW], g[1], g[2], g[5], g[6], g[7], du, true, true, g[5].size(0));
-    dgrad(C, C, du, &u0, p[kInW], nullptr, M2D_ACT_NONE, nullptr, dn, nullptr);
-    wgrad(3, du, &u0, n1, M2D_ACT_NONE, nullptr, nullptr);
+    layer(3, du, &u0, n1, M2D_ACT_NONE, nullptr, nullptr, dn, nullptr);
     // first update, norm1 and the local path's norm
     Tensor dx = at::empty_like(x);
     check(m2d_train_norm_bwd(s.P, C, rps, f32(x), dn.data_ptr(), s.local ? dl.data_ptr() : nullptr, f32(dx1), f32(p[kRs1]), nullptr, f32(p[kN1W]),

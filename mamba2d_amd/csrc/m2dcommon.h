@@ -132,6 +132,15 @@ __device__ __forceinline__ float gelu_slope(float v) {
   return t + (v < 0.f ? 0.f : 1.f);
 }
 
+// both, each as above
+__device__ __forceinline__ void gelu_and_slope(float v, float& value, float& slope) {
+  const float ex = __builtin_amdgcn_exp2f(v * v * -0.72134752044448170f);
+  const float q = normal_tail(v);
+  const bool neg = v < 0.f;
+  value = v * (neg ? q : 1.f - q);
+  slope = __builtin_fmaf(v * 0.39894228040143268f, ex, neg ? q : -q) + (neg ? 0.f : 1.f);
+}
+
 inline bool misaligned(const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) != 0; }
 
 }  // namespace

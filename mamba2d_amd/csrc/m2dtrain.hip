@@ -725,6 +725,198 @@ __global__ __launch_bounds__(256, 2) void m2d_train_wgrad_kernel(const WgradArgs
   if (tid < 64 && n0 + tid < a.N) out[(int64_t)a.N * a.K + n0 + tid] = ((dump[tid] + dump[64 + tid]) + dump[128 + tid]) + dump[192 + tid];
 }
 
+// ------------------------------------- both gradients of a linear layer in one pass over its activations, bf16
+// dx = (g W) * slope_pre(x) and dW = g^T pre(x), db = sum g, with g = dy * slope_post(z), for layers of up to 256 inputs and outputs
+// whose tiles eight waves share evenly.  The two kernels above read dy (and x, z) once each and are bound by that; here a
+// tile of T positions is read once: g and pre(x) go to LDS as bf16, where the input's gradient takes g by rows and the weight's gradient takes both by
+// columns (ds_read_b64_tr_b16).  A wave owns 32 inputs (K / 32 waves) and a share of the rest: of the positions for the input's gradient, of the outputs
+// for the weight's, whose sums stay in its registers over all tiles of the workgroup, so that nothing is added up across
+// waves.  W's rows are listed so that a lane ends with the 8 neighbouring inputs of a position that it fetched itself: the slope is
+// taken from registers and 16 bytes are stored, 64 of a row.  One barrier a tile (two buffers); the next tile's loads are under way meanwhile.
+// One workgroup to a unit: each leaves N K sums.  200704 positions, both kernels above -> this one: 64 -> 64 with the GELU
+// before it 42 -> 28 us, 256 -> 64 with it 124 -> 87 (the GELU and its slope at 51 million values: 42 at the rate of the vector ALUs), 64 -> 256 59 -> 36, 128 -> 64 with a StarReLU 52 -> 41.
+constexpr int kGrThreads = 512, kGrMost = 256;      // workgroups at most
+template <int N, int K, int PT>
+struct GradsPlan {
+  static constexpr int WK = K / 32, WN = 8 / WK, T = 16 * WN * PT;      // waves along the inputs, and beside each other; positions of a tile
+  static constexpr int NTW = N / 16 / WN;                               // tiles of 16 outputs of a wave
+  static constexpr int GS = N + 8, XS = K + 8;                          // bf16 per row in LDS
+  static constexpr int kBuf = T * (GS + XS);                            // bf16 of a buffer
+  static constexpr size_t kLds = 2 * (size_t)kBuf * 2;
+  static constexpr int GP = T * N / 8 / kGrThreads;                     // 16-byte pieces of g of a thread
+  static_assert(WK * WN == 8 && NTW * WN * 16 == N && GP >= 1 && T % 32 == 0, "eight waves share the tiles evenly");
+};
+struct GradsArgs {
+  const uint16_t *dy, *z, *x;      // (P, N), (P, N) where post is an activation, (P, K)
+  const float* w;                  // (N, K)
+  const float *pre_s, *pre_b;
+  uint16_t* dx;                    // (P, K)
+  float *part, *star;              // (gridDim.x, N K + N), (gridDim.x, 2) where pre is a StarReLU
+  int64_t P;
+  int post, bias;
+};
+
+// 8 positions of a column, as column_operand, of rows RS apart
+template <int RS>
+__device__ __forceinline__ uint4 column_of(const uint16_t* tile, int c0, int l) {
+  const uint16_t* p = tile + (8 * (l >> 4) + ((l & 15) >> 2)) * RS + c0 + 4 * (l & 3);
+  const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(p));
+  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(p + 4 * RS));
+  const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
+  return make_uint4(a.x, a.y, b.x, b.y);
+}
+
+template <int N, int K, int PT, int PRE>
+__global__ __launch_bounds__(kGrThreads) void m2d_train_linear_grads_kernel(const GradsArgs a) {
+  using L = GradsPlan<N, K, PT>;
+  constexpr int T = L::T, NS = N / 32;
+  extern __shared__ float smem[];
+  uint16_t* lds = reinterpret_cast<uint16_t*>(smem);
+  const int tid = threadIdx.x, l = tid & 63, mn = l & 15, kb = l >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave % L::WK, wn = wave / L::WK;
+  const float pre_s = PRE == kActStarRelu ? a.pre_s[0] : 0.f, pre_b = PRE == kActStarRelu ? a.pre_b[0] : 0.f;
+  const int64_t tiles = (a.P + T - 1) / T;
+  const uint4 z4 = make_uint4(0u, 0u, 0u, 0u);
+  const int xcol = 32 * wk + 8 * kb;                    // the lane's 8 inputs
+  uint4 gq[L::GP], zq[L::GP], xq[PT];
+  auto fetch = [&](int64_t t) {
+#pragma unroll
+    for (int u = 0; u < L::GP; ++u) {
+      const int i = tid + u * kGrThreads, c = 8 * (i % (N / 8));
+      const int64_t pos = t * T + i / (N / 8);
+      gq[u] = zq[u] = z4;
+      if (pos < a.P) {
+        gq[u] = ld16(a.dy + pos * N + c);
+        if (a.post != kActNone) zq[u] = ld16(a.z + pos * N + c);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      const int64_t pos = t * T + 16 * (wn * PT + j) + mn;
+      xq[j] = pos < a.P ? ld16(a.x + pos * K + xcol) : z4;
+    }
+  };
+  fetch(blockIdx.x);
+  // W as the first operand of the input's gradient: lane (m, kb) of step s and tile t holds the outputs 32 s + 8 kb + j of input 32 wk + 8 (m >> 2) + 4 t + (m & 3)
+  uint4 W[2][NS];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const float* src = a.w + (int64_t)(32 * s + 8 * kb) * K + 32 * wk + 8 * (mn >> 2) + 4 * t + (mn & 3);
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = src[j * K];
+      W[t][s] = make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
+    }
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+  const bool with_bias = a.bias && wk == 0;             // (uniform)
+  f32x4_t acc[L::NTW][2], accb[L::NTW];
+#pragma unroll
+  for (int i = 0; i < L::NTW; ++i) acc[i][0] = acc[i][1] = accb[i] = zero;
+  float sum_s = 0.f, sum_b = 0.f;
+  int buf = 0;
+  for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+    uint16_t* Gt = lds + buf * L::kBuf;
+    uint16_t* Xt = Gt + T * L::GS;
+    buf ^= 1;
+#pragma unroll
+    for (int u = 0; u < L::GP; ++u) {
+      const int i = tid + u * kGrThreads, c = 8 * (i % (N / 8));
+      uint32_t g4[4] = {gq[u].x, gq[u].y, gq[u].z, gq[u].w};
+      if (a.post != kActNone) {      // (uniform)
+        const uint32_t q4[4] = {zq[u].x, zq[u].y, zq[u].z, zq[u].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) g4[j] = pack_bf16(bf_lo(g4[j]) * gelu_slope(bf_lo(q4[j])), bf_hi(g4[j]) * gelu_slope(bf_hi(q4[j])));
+      }
+      *reinterpret_cast<uint4*>(Gt + i / (N / 8) * L::GS + c) = make_uint4(g4[0], g4[1], g4[2], g4[3]);
+    }
+    float slope[PT][8];      // of GELU; relu(x) for StarReLU
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      uint4 q = xq[j];
+      if constexpr (PRE != kActNone) {
+        float v[8], o[8];
+        Chunk<bf16_t>::unpack(q, v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if constexpr (PRE == kActGelu) gelu_and_slope(v[i], o[i], slope[j][i]);
+          else { slope[j][i] = relu(v[i]); o[i] = act(kActStarRelu, v[i], pre_s, pre_b); }
+        }
+        q = make_uint4(pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]), pack_bf16(o[4], o[5]), pack_bf16(o[6], o[7]));
+      }
+      *reinterpret_cast<uint4*>(Xt + (16 * (wn * PT + j) + mn) * L::XS + xcol) = q;
+    }
+    if (t + gridDim.x < tiles) fetch(t + gridDim.x);
+    __syncthreads();
+    // the weight's gradient: contraction over the tile's positions
+#pragma unroll
+    for (int s = 0; s < T / 32; ++s) {
+      uint4 bx[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) bx[j] = column_of<L::XS>(Xt + 32 * s * L::XS, 32 * wk + 16 * j, l);
+#pragma unroll
+      for (int i = 0; i < L::NTW; ++i) {
+        const uint4 ag = column_of<L::GS>(Gt + 32 * s * L::GS, 16 * (wn * L::NTW + i), l);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma_bf16(ag, bx[j], acc[i][j]);
+        if (with_bias) accb[i] = mfma_bf16(ag, ones, accb[i]);
+      }
+    }
+    // the input's gradient at the lane's positions
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      const int row = 16 * (wn * PT + j) + mn;
+      f32x4_t d[2] = {zero, zero};
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const uint4 g = ld16(Gt + row * L::GS + 32 * s + 8 * kb);
+        d[0] = mfma_bf16(W[0][s], g, d[0]);
+        d[1] = mfma_bf16(W[1][s], g, d[1]);
+      }
+      float v[8] = {d[0][0], d[0][1], d[0][2], d[0][3], d[1][0], d[1][1], d[1][2], d[1][3]};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if constexpr (PRE == kActGelu) v[i] *= slope[j][i];
+        if constexpr (PRE == kActStarRelu) {      // (rows past the end: g and so v are 0)
+          const float r = slope[j][i];
+          sum_s = __builtin_fmaf(v[i], r * r, sum_s);
+          sum_b += v[i];
+          v[i] = star_relu_back(v[i], r, pre_s);
+        }
+      }
+      const int64_t pos = t * T + row;
+      if (pos < a.P) *reinterpret_cast<uint4*>(a.dx + pos * K + xcol) = make_uint4(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7]));
+    }
+  }
+  // a lane holds, of tile (i, j), the outputs 4 kb + r and the input mn
+  float* out = a.part + (int64_t)blockIdx.x * (N * K + N);
+#pragma unroll
+  for (int i = 0; i < L::NTW; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = 16 * (wn * L::NTW + i) + 4 * kb + r;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) out[n * K + 32 * wk + 16 * j + mn] = acc[i][j][r];
+      if (with_bias && mn == 0) out[N * K + n] = accb[i][r];
+    }
+  if constexpr (PRE == kActStarRelu) {
+    __syncthreads();      // (the buffers are free)
+    sum_s = row_sum<64>(sum_s);
+    sum_b = row_sum<64>(sum_b);
+    if (l == 0) { smem[2 * wave] = sum_s; smem[2 * wave + 1] = sum_b; }
+    __syncthreads();
+    if (tid < 2) {
+      float v = smem[tid];
+#pragma unroll
+      for (int w = 1; w < 8; ++w) v += smem[2 * w + tid];
+      a.star[(int64_t)blockIdx.x * 2 + tid] = v;
+    }
+  }
+}
+
 // ------------------------------------------------------------- sums of the workgroups' parts
 // out[i] = sum_s part[s * stride + i], in a fixed order; up to kMaxSegs sums in one launch.  Bound by memory (58 MB of parts
 // for a block of 64 channels, most of them still in the last-level cache) as long as enough loads are under way: a
@@ -853,9 +1045,64 @@ inline int wgrad_shares(int64_t P, int N, int K) {
   return (int)(shares < 1 ? 1 : shares);
 }
 
+// The layers whose two gradients come from one kernel: those of a block of 64 channels, and of 128 but for its MLP.  (Outputs, inputs, tiles of 16 positions of
+// a wave: as many as two buffers of them fit the LDS, up to 128 positions in all.)
+#define M2D_GRADS_SHAPES(X) X(64, 64, 2) X(64, 256, 4) X(256, 64, 1) X(64, 128, 4) X(128, 64, 2) X(128, 128, 2) X(128, 256, 2) X(256, 128, 1)
+template <int N, int K, int PT>
+int grads_parts(int64_t P) {
+  const int64_t tiles = (P + GradsPlan<N, K, PT>::T - 1) / GradsPlan<N, K, PT>::T;
+  return (int)(tiles < kGrMost ? tiles : kGrMost);
+}
+template <int N, int K, int PT, int PRE>
+int launch_grads(const GradsArgs& a, hipStream_t st) {
+  using L = GradsPlan<N, K, PT>;
+  static_assert(L::kLds <= kLinMaxLds, "two buffers fit the LDS");
+  static std::atomic<uint64_t> seen{0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return M2D_ERR_HIP;
+  const uint64_t bit = 1ull << (dev & 63);
+  const auto kernel = &m2d_train_linear_grads_kernel<N, K, PT, PRE>;
+  if (L::kLds > 64 * 1024 && !(seen.load(std::memory_order_acquire) & bit)) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::kLds) != hipSuccess) return M2D_ERR_HIP;
+    seen.fetch_or(bit, std::memory_order_release);
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grads_parts<N, K, PT>(a.P)), dim3(kGrThreads), L::kLds, st, a);
+  return launched();
+}
+template <int N, int K, int PT>
+int launch_grads_act(const GradsArgs& a, int pre, hipStream_t st) {
+  if (pre == kActGelu) return launch_grads<N, K, PT, kActGelu>(a, st);
+  if (pre == kActStarRelu) return launch_grads<N, K, PT, kActStarRelu>(a, st);
+  return launch_grads<N, K, PT, kActNone>(a, st);
+}
+
 }  // namespace
 
 extern "C" {
+
+int m2d_train_linear_grads_parts(int64_t P, int N, int K) {
+  if (P < 1) return 0;
+#define X(n, k, pt) if (N == n && K == k) return grads_parts<n, k, pt>(P);
+  M2D_GRADS_SHAPES(X)
+#undef X
+  return 0;
+}
+
+int m2d_train_linear_grads(int64_t P, int N, int K, const void* dy, const void* z, int post_act, const float* weight, const void* x, int pre_act,
+                           const float* pre_scale, const float* pre_bias, int bias, void* dx, float* part, float* star_part, void* stream) {
+  if (!dy || !weight || !x || !dx || !part || (post_act != kActNone && !z)) return M2D_ERR_NULL_POINTER;
+  if (pre_act == kActStarRelu && (!pre_scale || !pre_bias || !star_part)) return M2D_ERR_NULL_POINTER;
+  if (P < 1 || K < 1 || N < 1) return M2D_ERR_BAD_SHAPE;
+  if ((post_act != kActNone && post_act != kActGelu) || pre_act < kActNone || pre_act > kActStarRelu) return M2D_ERR_UNSUPPORTED;
+  if (misaligned(dy, 16) || misaligned(z, 16) || misaligned(x, 16) || misaligned(dx, 16) || misaligned(weight, 4)) return M2D_ERR_MISALIGNED;
+  GradsArgs a = {static_cast<const uint16_t*>(dy), static_cast<const uint16_t*>(z), static_cast<const uint16_t*>(x), weight, pre_scale, pre_bias,
+                 static_cast<uint16_t*>(dx), part, star_part, P, post_act, bias};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+#define X(n, k, pt) if (N == n && K == k) return launch_grads_act<n, k, pt>(a, pre_act, st);
+  M2D_GRADS_SHAPES(X)
+#undef X
+  return M2D_ERR_UNSUPPORTED;
+}
 
 int m2d_train_norm_fwd(int64_t rows, int C, int rows_per_sample, const float* x, const float* scale, const void* r, const void* r2,
                        const float* keep, float* x_out, const float* w1, const float* b1, float eps1, void* y1, const float* w2,
