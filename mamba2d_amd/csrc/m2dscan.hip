@@ -2951,19 +2951,20 @@ Geometry make_geometry(const m2d_desc* d) {
   // fifth (where units have more than one workgroup to sweep).
   // The constants are ratios: a block of forward keeping snapshots and backward, a workgroup of 4 waves with a quarter of the states each as 100
   // (1000 problems of both types: 8 such waves 150; whole states in workgroups of 8 waves 437, of 16 channels 303 linked and 216 in one stream; where
-  // rows are no whole chunks all of them take longer, the last 310).  Near the line the whole states stay: fewer channel sums, snapshots every 2
+  // rows are no whole chunks all of them take longer, the last 310).  In the linked sweep whole states in workgroups of 8 waves have fallen behind by more: as
+  // 417 the split states, where they ran, took 0.80 of what the ratios said (median of 14 problems, 0.74 to 0.88; 16x138x162x104 bf16 1.91 of 2.41 ms, 3x132x170x488 1.79 of 2.11).  Near the line the whole states stay: fewer channel sums, snapshots every 2
   // steps.  Both sides, kernels of both passes in ms, whole states against split: 30x60x50x40 fp32 0.522 and 0.324, 8x256x256x64 bf16 3.16 and 2.10,
   // 20x28x28x200 fp32 0.289 and 0.202, 32x128x128x64 bf16 2.02 and 1.64; on the other side of the line 64x28x28x128 bf16 0.280 and 0.391.
   // Of 708 problems drawn over all sizes the chosen plans take 1.023 of the time of each one's best; farthest off, 1.3 to 1.5, are widths of no whole
   // chunks and one to three channels, and grids two to four columns wide, where whole states would be up to 1.09 ahead of the linked sweep.
-  constexpr int64_t kSplit4 = 100, kSplit8 = 147, kWhole4 = 235, kWhole4Linked = 300, kWhole8 = 417;
+  constexpr int64_t kSplit4 = 100, kSplit8 = 147, kWhole4 = 235, kWhole4Linked = 300, kWhole8 = 417, kWhole8Linked = 480;
   auto stream_cost = [&](int64_t wgs, int64_t block) { return (wgs + ncu - 1) / ncu * nblk_stream * block; };
   auto link_cost = [&](int64_t wgs, int64_t block) {
     const int64_t work = (wgs * g.nbands + ncu - 1) / ncu * nbb_link, chain = nbb_link + (int64_t)(g.nbands - 1) * (kLinkLag - 1);
     return (work > chain ? work + chain / 5 : chain + (work > nbb_link ? work / 5 : 0)) * block;
   };
   auto cost = [&](bool linked, int64_t wgs, int64_t block) { return linked ? link_cost(wgs, block) : stream_cost(wgs, block); };
-  const int64_t whole_block = g.bwd_nw != kFwdHalfWaves ? kWhole8 : (g.sliced ? kWhole4Linked : kWhole4);
+  const int64_t whole_block = g.bwd_nw != kFwdHalfWaves ? (g.sliced ? kWhole8Linked : kWhole8) : (g.sliced ? kWhole4Linked : kWhole4);
   const int64_t whole_cost = g.sliced ? link_cost((int64_t)B * g.bwd_bpb, whole_block) : stream_cost((int64_t)B * g.bwd_bpb, whole_block);
   const int64_t wg4 = (int64_t)B * ((d->E + kSplitHalfWaves - 1) / kSplitHalfWaves), wg8 = (int64_t)B * ((d->E + kSplitWaves - 1) / kSplitWaves);
   int split_nw = kSplitHalfWaves;
