@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <type_traits>
 
 #include "m2dscan.h"
@@ -290,6 +291,145 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_fwd_mfma_kern
         if (c < rows && e0 + c8 < a.E) *reinterpret_cast<uint4*>(out + (uint32_t)(c * a.E + e0 + c8)) = pack8(v);
       });
       wave_sync_lds();
+    }
+  }
+}
+
+// Forward for up to 256 channels and a rank of up to 16.  The kernel above, left with the wider ones (whose weights fill the LDS, and whose low-rank
+// inputs don't fit one step of 32), is bound by its weight tiles: every wave of 16 positions fetches all of them, 14 KB for 2 KB of x at 64 channels,
+// from the caches.  Here a workgroup stays for many tiles and holds the weights in LDS, rounded to bf16 as it
+// reads them from the caller's tensors (no packing launch), and the weights' rows are the first operands, so that a lane (position mn, group kb) ends with
+// neighbouring outputs of its position and stores them from registers: 4 of a record of B_T, B_L, C, whose rows are listed in the records' order, and 8
+// step sizes, for which a pair of tiles lists its rows as 8 (m >> 2) + 4 t + (m & 3).  The low-rank inputs of the step sizes stay in the registers
+// that they were made in: the second product lists its contraction in their order, and those of the other step size are masked out, so that
+// an infinite value of one does not meet the other's zero weights.  Against the kernel above
+// and its packing launch, ten calls in a row: 64x56x56x64 43.1 -> 28.8 us (104 MB, 3.6 TB/s), 4x128x128x64 19.6 -> 13.4, 64x28x28x128 28.2 -> 22.7,
+// 64x14x14x256 27.0 -> 24.4, 200000 positions of 32 channels 39.2 -> 18.3, 4096 of 64 11.1 -> 7.2; no size measured was slower.  What is left at 64 channels
+// is the copying in of the weights and the softplus.
+constexpr int kFlD = 40;      // bf16 per row of the step sizes' weights in LDS: 32 + 8
+constexpr int kFlMaxE = 256, kFlMaxR = 16;
+constexpr size_t fl_lds_bytes(int Epad, int NL) { return ((size_t)(16 * NL + 3 * kN) * (Epad + 8) + 2 * (size_t)Epad * kFlD) * 2 + 2 * (size_t)Epad * 4; }
+__device__ __forceinline__ f32x4 lds_f4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+template <int KS, int NL, bool PACKED>   // steps of 32 channels at most; tiles of 16 low-rank inputs
+__global__ __launch_bounds__(kThreads) void m2d_proj_fwd_lds_kernel(const ProjArgs a) {
+  extern __shared__ float smem[];
+  const int tid = threadIdx.x, wave = wave_id(), l = tid & 63, mn = l & 15, kb = l >> 4;
+  constexpr int NZ = 16 * NL + 3 * kN;
+  const int E = a.E, Epad = (E + 31) / 32 * 32, ks = Epad / 32, R = a.R, R2 = 2 * a.R, LW = Epad + 8;
+  uint16_t* wz = reinterpret_cast<uint16_t*>(smem);
+  uint16_t* wT = wz + NZ * LW;
+  uint16_t* wL = wT + Epad * kFlD;
+  float* bT = reinterpret_cast<float*>(wL + Epad * kFlD);
+  float* bL = bT + Epad;
+  const bf16_t* x = static_cast<const bf16_t*>(a.x);
+  const int ntiles = (int)((a.P + kTP - 1) / kTP);
+  uint4 next[KS];
+  auto fetch = [&](int tile) {
+    const int64_t pm = (int64_t)tile * kTP + wave * 16 + mn;
+    const bf16_t* row = x + (pm < a.P ? pm : a.P - 1) * E;      // rows past the end repeat the last one and are not stored
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int e = 32 * s + 8 * kb;
+      next[s] = load16(row + (e < E ? e : 0));                  // (channels past E meet zero weights, but must be finite: masked below)
+    }
+  };
+  fetch(blockIdx.x);
+  for (int i = tid; i < NZ * (Epad / 4); i += kThreads) {
+    const int row = i / (Epad / 4), c = 4 * (i - row * (Epad / 4)), t = row >> 4, m = row & 15;
+    const int q = m & 3, state = PACKED ? 4 * (q == 1 ? 2 : (q == 2 ? 1 : q)) + (m >> 2) : m;
+    const int o = t < NL ? row : R2 + 16 * (t - NL) + state;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (c < E && (t >= NL || o < R2)) v = *reinterpret_cast<const float4*>(a.Wx + (int64_t)o * E + c);
+    *reinterpret_cast<uint2*>(wz + row * LW + c) = make_uint2(pack2(v.x, v.y), pack2(v.z, v.w));
+  }
+  for (int i = tid; i < Epad * 16; i += kThreads) {             // slots 2 (i % 16) and the next of channel e: low-rank inputs o, o + 1
+    const int e = i >> 4, s = 2 * (i & 15), j = s & 7, o = (j < 4 ? j : 12 + j) + 4 * (s >> 3);
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (e < E) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        if (o + k < R) v[k] = a.wT[(int64_t)e * R + o + k];
+        else if (o + k < R2) v[2 + k] = a.wL[(int64_t)e * R + o + k - R];
+      }
+    }
+    *reinterpret_cast<uint32_t*>(wT + e * kFlD + s) = pack2(v[0], v[1]);
+    *reinterpret_cast<uint32_t*>(wL + e * kFlD + s) = pack2(v[2], v[3]);
+  }
+  for (int e = tid; e < Epad; e += kThreads) {
+    const float t = e < E ? a.bT[e] : 0.f, v = e < E ? a.bL[e] : 0.f;
+    bT[e] = a.round ? as_stored(t, static_cast<const bf16_t*>(nullptr)) : t;
+    bL[e] = a.round ? as_stored(v, static_cast<const bf16_t*>(nullptr)) : v;
+  }
+  // which of the lane's low-rank inputs are the T step size's, which the L one's
+  uint32_t mT[2 * NL], mL[2 * NL];
+#pragma unroll
+  for (int w = 0; w < 2 * NL; ++w) {
+    const int o = 16 * (w >> 1) + 4 * kb + 2 * (w & 1);
+    mT[w] = (o < R ? 0xffffu : 0u) | (o + 1 < R ? 0xffff0000u : 0u);
+    mL[w] = (o >= R && o < R2 ? 0xffffu : 0u) | (o + 1 >= R && o + 1 < R2 ? 0xffff0000u : 0u);
+  }
+  __syncthreads();
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int64_t pm = (int64_t)tile * kTP + wave * 16 + mn;
+    const bool in = pm < a.P;
+    uint4 X[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) X[s] = 32 * s + 8 * kb < E ? next[s] : zero16();
+    if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
+    uint2 z[NL + 3];
+#pragma unroll
+    for (int t = 0; t < NL + 3; ++t) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        if (s < ks) acc = mfma16(load16(wz + (16 * t + mn) * LW + 32 * s + 8 * kb), X[s], acc);
+      z[t] = make_uint2(pack2(acc[0], acc[1]), pack2(acc[2], acc[3]));
+    }
+    if (in) {
+      bf16_t* r = static_cast<bf16_t*>(a.r_out) + pm * R2;
+#pragma unroll
+      for (int t = 0; t < NL; ++t) {
+        const int o = 16 * t + 4 * kb;
+        if ((R2 & 3) == 0) {      // (uniform)
+          if (o < R2) *reinterpret_cast<uint2*>(r + o) = z[t];
+        } else {
+          const uint32_t w[2] = {z[t].x, z[t].y};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (o + i < R2) r[o + i].v = (uint16_t)(w[i >> 1] >> (16 * (i & 1)));
+        }
+      }
+#pragma unroll
+      for (int w = 0; w < 3; ++w) {
+        const uint2 q = z[NL + w];
+        if constexpr (PACKED) {
+          *reinterpret_cast<float4*>(a.bc_packed + pm * (3 * kN) + w * kN + 4 * kb) = make_float4(bf16_lo(q.x), bf16_hi(q.x), bf16_lo(q.y), bf16_hi(q.y));
+        } else {
+          *reinterpret_cast<uint2*>(static_cast<bf16_t*>(w == 0 ? a.BT_out : (w == 1 ? a.BL_out : a.C_out)) + pm * kN + 4 * kb) = q;
+        }
+      }
+    }
+    const uint4 lowT = make_uint4(z[0].x & mT[0], z[0].y & mT[1], NL > 1 ? z[NL - 1].x & mT[2 * NL - 2] : 0u, NL > 1 ? z[NL - 1].y & mT[2 * NL - 1] : 0u);
+    const uint4 lowL = make_uint4(z[0].x & mL[0], z[0].y & mL[1], NL > 1 ? z[NL - 1].x & mL[2 * NL - 2] : 0u, NL > 1 ? z[NL - 1].y & mL[2 * NL - 1] : 0u);
+    for (int e0 = 0; e0 < E; e0 += 32) {
+      const int e = e0 + 8 * kb, row = e0 + 8 * (mn >> 2) + (mn & 3);
+      uint4 out[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float v[8];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const f32x4 d = mfma16(load16((h ? wL : wT) + (row + 4 * t) * kFlD + 8 * kb), h ? lowL : lowT, lds_f4((h ? bL : bT) + e + 4 * t));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[4 * t + i] = softplus(d[i]);
+        }
+        out[h] = pack8(v);
+      }
+      if (in && e < E) {
+        *reinterpret_cast<uint4*>(static_cast<bf16_t*>(a.dT_out) + pm * E + e) = out[0];
+        *reinterpret_cast<uint4*>(static_cast<bf16_t*>(a.dL_out) + pm * E + e) = out[1];
+      }
     }
   }
 }
@@ -1242,6 +1382,37 @@ int run_proj_fwd_mfma(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) 
   return launched() ? M2D_OK : M2D_ERR_HIP;
 }
 
+// The weights in LDS, straight from the caller's tensors: see the kernel.
+bool proj_fwd_in_lds(const ProjGeometry& g) { return g.mfma && g.E <= kFlMaxE && g.R <= kFlMaxR; }
+template <int KS, int NL>
+int launch_proj_fwd_lds(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
+  const int Epad = (g.E + 31) / 32 * 32;
+  const size_t lds = fl_lds_bytes(Epad, NL);
+  auto go = [&](auto kernel) -> int {
+    if (lds > 64 * 1024) {   // (more dynamic LDS than that has to be allowed, once per kernel and device)
+      static std::atomic<uint64_t> seen{0};
+      int dev = 0;
+      if (hipGetDevice(&dev) != hipSuccess) return M2D_ERR_HIP;
+      const uint64_t bit = 1ull << (dev & 63);
+      if (!(seen.load(std::memory_order_acquire) & bit)) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)fl_lds_bytes(kFlMaxE, NL)) != hipSuccess) return M2D_ERR_HIP;
+        seen.fetch_or(bit, std::memory_order_release);
+      }
+    }
+    const int64_t tiles = (g.P + kTP - 1) / kTP;
+    int64_t grid = 256 * (int64_t)((160 * 1024) / lds < 6 ? (160 * 1024) / lds : 6);   // as many workgroups as the device holds
+    if (grid > tiles) grid = tiles;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kThreads), lds, st, a);
+    return launched() ? M2D_OK : M2D_ERR_HIP;
+  };
+  return a.bc_packed ? go(&m2d_proj_fwd_lds_kernel<KS, NL, true>) : go(&m2d_proj_fwd_lds_kernel<KS, NL, false>);
+}
+int run_proj_fwd_lds(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
+  auto ranks = [&](auto ks) -> int { return g.R <= 8 ? launch_proj_fwd_lds<decltype(ks)::value, 1>(g, a, st) : launch_proj_fwd_lds<decltype(ks)::value, 2>(g, a, st); };
+  if (g.E <= 64) return ranks(std::integral_constant<int, 2>{});
+  return g.E <= 128 ? ranks(std::integral_constant<int, 4>{}) : ranks(std::integral_constant<int, 8>{});
+}
+
 // The fp32 products' kernels: V4 where the rows of the (P,E) arrays and of Wx are whole runs of 4 elements, NL tiles of
 // low-rank inputs, NT tiles of 16 positions per wave.
 template <typename F>
@@ -1328,7 +1499,7 @@ int m2d_proj_fwd(const m2d_desc* desc, int dt_rank, const void* x, const float* 
   char* ws = static_cast<char*>(workspace);
   PackArgs k = {};
   k.Wx = x_proj_w; k.wT = dt_projT_w; k.bT = dt_projT_b; k.wL = dt_projL_w; k.bL = dt_projL_b;
-  if (g.mfma) {
+  if (g.mfma && !proj_fwd_in_lds(g)) {
     k.bTp = reinterpret_cast<float*>(ws + g.off_bTp);
     k.bLp = reinterpret_cast<float*>(ws + g.off_bLp);
     k.Wb = reinterpret_cast<uint16_t*>(ws + g.off_Wb);
@@ -1348,6 +1519,7 @@ int m2d_proj_fwd(const m2d_desc* desc, int dt_rank, const void* x, const float* 
   a.Wb = k.Wb; a.wTb = k.wTb; a.wLb = k.wLb;
   a.r_out = lowrank; a.dT_out = deltaT; a.dL_out = deltaL; a.BT_out = BT; a.BL_out = BL; a.C_out = C;
   a.bc_packed = packed ? static_cast<float*>(BT) : nullptr;
+  if (proj_fwd_in_lds(g)) return run_proj_fwd_lds(g, a, st);
   return g.mfma ? run_proj_fwd_mfma(g, a, st) : with_layout(desc->dtype == M2D_F32, g, [&](auto t, auto v4, auto nt) -> int {
     return run_proj_fwd_f32<decltype(t), v4(), nt()>(g, a, st);
   });
