@@ -309,7 +309,7 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_fwd_mfma_kern
 constexpr int kFlD = 40;      // bf16 per row of the step sizes' weights in LDS: 32 + 8
 constexpr int kFlMaxE = 256, kFlMaxR = 16;
 constexpr size_t fl_lds_bytes(int Epad, int NL) { return ((size_t)(16 * NL + 3 * kN) * (Epad + 8) + 2 * (size_t)Epad * kFlD) * 2 + 2 * (size_t)Epad * 4; }
-__device__ __forceinline__ f32x4 lds_f4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ f32x4 load_f4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
 template <int KS, int NL, bool PACKED>   // steps of 32 channels at most; tiles of 16 low-rank inputs
 __global__ __launch_bounds__(kThreads) void m2d_proj_fwd_lds_kernel(const ProjArgs a) {
@@ -420,7 +420,7 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_fwd_lds_kernel(const ProjAr
         float v[8];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          const f32x4 d = mfma16(load16((h ? wL : wT) + (row + 4 * t) * kFlD + 8 * kb), h ? lowL : lowT, lds_f4((h ? bL : bT) + e + 4 * t));
+          const f32x4 d = mfma16(load16((h ? wL : wT) + (row + 4 * t) * kFlD + 8 * kb), h ? lowL : lowT, load_f4((h ? bL : bT) + e + 4 * t));
 #pragma unroll
           for (int i = 0; i < 4; ++i) v[4 * t + i] = softplus(d[i]);
         }
@@ -434,38 +434,10 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_fwd_lds_kernel(const ProjAr
   }
 }
 
-// Backward, data.  LDS: per wave one [16][Opad32 + 8] bf16 block (the rows of dz) and the [16][68]
-// fp32 block the dx tiles leave through.  dz and dpre are also written out as bf16 arrays for the
-// weight-gradient kernel.
-__global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_bwd_data_mfma_kernel(const ProjArgs a) {
-  extern __shared__ float smem[];
-  const int wave = wave_id(), l = threadIdx.x & 63, mn = l & 15, kb = l >> 4;
-  const int zst = a.Opad32 + 8;
-  float* stage = smem + wave * (16 * kStageStride + 16 * zst / 2);   // [16][68] floats, then [16][zst] bf16
-  uint16_t* zs = reinterpret_cast<uint16_t*>(stage + 16 * kStageStride);
-  for (int i = l; i < 16 * zst / 2; i += 64) reinterpret_cast<uint32_t*>(zs)[i] = 0u;   // padding columns: zero
-  const int64_t p0 = (int64_t)blockIdx.x * kTP + wave * 16;
-  const int rows = (int)(a.P - p0 < 16 ? a.P - p0 : 16);   // positions of the wave inside the array (may be <= 0)
-  const int R = a.R, R2 = 2 * a.R, NQ = a.Rpad / 16;
-  // wave-uniform bases (the wave's first position); lanes add 32-bit element offsets
-  const bf16_t* dT = static_cast<const bf16_t*>(a.dT) + p0 * a.E;
-  const bf16_t* dL = static_cast<const bf16_t*>(a.dL) + p0 * a.E;
-  const bf16_t* ddT = static_cast<const bf16_t*>(a.ddT) + p0 * a.E;
-  const bf16_t* ddL = static_cast<const bf16_t*>(a.ddL) + p0 * a.E;
-  bf16_t* dx = static_cast<bf16_t*>(a.dx) + p0 * a.E;
-  // rows past the end of the arrays (up to the next multiple of 16) are written too, as zeros
-  uint16_t* dzt = a.dzt + p0 * a.Opad;
-  uint16_t* dptT = a.dpt + p0 * a.E;
-  uint16_t* dptL = dptT + (int64_t)a.ntiles * kTP * a.E;
-  const uint4 z4 = make_uint4(0, 0, 0, 0);
-  const bool given = a.dpre_given != 0;   // (uniform) ddT, ddL are dpre already: nothing to derive or to write out
-
-  // Memory latency is covered by the other waves of the compute unit (registers are kept low
-  // for that), not by fetching ahead.
-  // dB_T, dB_L, dC: lane l holds 4 values of position l >> 2
-  const int cb = l >> 2, n0 = 4 * (l & 3);
-  uint2 bc[3];
-  if (a.sum_parts > 0) {   // (uniform) the scan's per-workgroup channel sums, added up here in their order and rounded once
+// The gradients of B_T, B_L, C of a wave's positions, four values of position p0 + cb from n0 on: the caller's arrays, or
+// (sum_parts > 0) the scan's per-workgroup channel sums, added up here in their order and rounded once.
+__device__ __forceinline__ void sum_channels(const ProjArgs& a, int64_t p0, int rows, int cb, int n0, uint2 (&bc)[3]) {
+  if (a.sum_parts > 0) {   // (uniform)
     // Twelve loads are under way at a time: with one (a loop over the parts for each of the three sums) a wave of 16
     // positions waited for memory 3 x parts times in a row: 70 -> 43 us for 4x128x128x64 (8 parts), 79 -> 60 for
     // 64x56x56x64 (4 parts; 283 MB, 4.7 TB/s).
@@ -514,6 +486,40 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_bwd_data_mfma
       bc[w] = cb < rows ? *reinterpret_cast<const uint2*>(src + (uint32_t)(cb * kN + n0)) : make_uint2(0, 0);
     }
   }
+}
+
+// Backward, data.  LDS: per wave one [16][Opad32 + 8] bf16 block (the rows of dz) and the [16][68]
+// fp32 block the dx tiles leave through.  dz and dpre are also written out as bf16 arrays for the
+// weight-gradient kernel.
+__global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_bwd_data_mfma_kernel(const ProjArgs a) {
+  extern __shared__ float smem[];
+  const int wave = wave_id(), l = threadIdx.x & 63, mn = l & 15, kb = l >> 4;
+  const int zst = a.Opad32 + 8;
+  float* stage = smem + wave * (16 * kStageStride + 16 * zst / 2);   // [16][68] floats, then [16][zst] bf16
+  uint16_t* zs = reinterpret_cast<uint16_t*>(stage + 16 * kStageStride);
+  for (int i = l; i < 16 * zst / 2; i += 64) reinterpret_cast<uint32_t*>(zs)[i] = 0u;   // padding columns: zero
+  const int64_t p0 = (int64_t)blockIdx.x * kTP + wave * 16;
+  const int rows = (int)(a.P - p0 < 16 ? a.P - p0 : 16);   // positions of the wave inside the array (may be <= 0)
+  const int R = a.R, R2 = 2 * a.R, NQ = a.Rpad / 16;
+  // wave-uniform bases (the wave's first position); lanes add 32-bit element offsets
+  const bf16_t* dT = static_cast<const bf16_t*>(a.dT) + p0 * a.E;
+  const bf16_t* dL = static_cast<const bf16_t*>(a.dL) + p0 * a.E;
+  const bf16_t* ddT = static_cast<const bf16_t*>(a.ddT) + p0 * a.E;
+  const bf16_t* ddL = static_cast<const bf16_t*>(a.ddL) + p0 * a.E;
+  bf16_t* dx = static_cast<bf16_t*>(a.dx) + p0 * a.E;
+  // rows past the end of the arrays (up to the next multiple of 16) are written too, as zeros
+  uint16_t* dzt = a.dzt + p0 * a.Opad;
+  uint16_t* dptT = a.dpt + p0 * a.E;
+  uint16_t* dptL = dptT + (int64_t)a.ntiles * kTP * a.E;
+  const uint4 z4 = make_uint4(0, 0, 0, 0);
+  const bool given = a.dpre_given != 0;   // (uniform) ddT, ddL are dpre already: nothing to derive or to write out
+
+  // Memory latency is covered by the other waves of the compute unit (registers are kept low
+  // for that), not by fetching ahead.
+  // dB_T, dB_L, dC: lane l holds 4 values of position l >> 2
+  const int cb = l >> 2, n0 = 4 * (l & 3);
+  uint2 bc[3];
+  sum_channels(a, p0, rows, cb, n0, bc);
 
   // dz[., rank] = dpre w, channels as the inner dimension
   f32x4 accT[2], accL[2];
@@ -618,6 +624,157 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_bwd_data_mfma
       }
     });
     wave_sync_lds();
+  }
+}
+
+// Backward, data, for up to 256 channels and a rank of up to 16; the kernel above has the wider ones, whose weights fill the LDS.  It moves what it must (64x56x56x64 with
+// 4 parts of channel sums: 283 MB), and what it lost were waits: for the packing launch before it, for weight tiles that each wave fetched from the caches,
+// and for dx, asked for at the end.  Here a workgroup rounds the weights into LDS from the caller's tensors, and everything is asked for before the first
+// wait, dx too where registers allow four workgroups a compute unit (up to 64 channels; with 128 three fitted, and 784 tiles of 64x28x28x128 took a second
+// generation for the last 16: whole backward 56.5 us against 50.3 without).  The weights' rows are the first operands, so dx leaves from registers, 16 bytes a lane.
+// Backward of the projections in all, ten calls in a row: 64x56x56x64, 4 parts 91.5 -> 81.9 us, 64x28x28x128, 8 parts 57.7 -> 50.3, 4x128x128x64, 8 parts 47.2 ->
+// 42.3, 64x14x14x256, 16 parts 46.7 -> 43.1, 200000 positions of 32 channels 68.8 -> 53.7, 1568 of 64 17.4 -> 14.9; bit for bit the same results.
+template <int KS>   // steps of 32 channels at most
+__global__ __launch_bounds__(kThreads, KS <= 4 ? 4 : 2) void m2d_proj_bwd_data_lds_kernel(const ProjArgs a) {
+  extern __shared__ float smem[];
+  const int tid = threadIdx.x, wave = wave_id(), l = tid & 63, mn = l & 15, kb = l >> 4;
+  const int E = a.E, Epad = (E + 31) / 32 * 32, R = a.R, R2 = 2 * a.R, O = a.O, LQ = Epad + 8, zst = a.Opad32 + 8;
+  uint16_t* wq = reinterpret_cast<uint16_t*>(smem);   // [2][16 ranks][LQ]: weights of the step sizes
+  uint16_t* wx = wq + 32 * LQ;                         // [Epad][zst]: x_proj transposed
+  uint16_t* zs = wx + Epad * zst + wave * 16 * zst;    // the wave's rows of dz
+  const int64_t p0 = (int64_t)blockIdx.x * kTP + wave * 16;
+  const int rows = (int)(a.P - p0 < 16 ? a.P - p0 : 16);   // positions of the wave inside the array (may be <= 0)
+  const bool given = a.dpre_given != 0;   // (uniform) ddT, ddL are dpre already: nothing to derive or to write out
+  const bool in = mn < rows;
+  const int64_t off = (p0 + mn < a.P ? p0 + mn : a.P - 1) * E;   // rows past the end repeat the last one: masked, not stored
+  const uint4 z4 = make_uint4(0, 0, 0, 0);
+
+  // the weights first, then everything else that memory is asked for: all of it is under way before the first wait
+  constexpr int kHold = 3;   // pairs of outputs x 4 channels of a thread
+  f32x4 hw0[kHold], hw1[kHold];
+  const int nwx = (a.Opad32 / 2) * (Epad / 4);
+  auto wx_at = [&](int i, int& o, int& c) {
+    o = 2 * (i / (Epad / 4));
+    c = 4 * (i - (o / 2) * (Epad / 4));
+    return i < nwx;
+  };
+  auto get_wx = [&](int i, int k) -> f32x4 {      // output 2 pair + k, padding: zeros
+    int o, c;
+    const bool ok = wx_at(i, o, c) && o < O && c < E;   // (O is even)
+    const f32x4 v = load_f4(a.Wx + (ok ? (o + k) * E + c : 0));
+    return ok ? v : (f32x4){0.f, 0.f, 0.f, 0.f};
+  };
+  auto put_wx = [&](int i, f32x4 u, f32x4 v) {
+    int o, c;
+    if (!wx_at(i, o, c)) return;
+    uint32_t* dst = reinterpret_cast<uint32_t*>(wx + c * zst + o);
+    dst[0] = pack2(u[0], v[0]);
+    dst[zst / 2] = pack2(u[1], v[1]);
+    dst[zst] = pack2(u[2], v[2]);
+    dst[3 * (zst / 2)] = pack2(u[3], v[3]);
+  };
+#pragma unroll
+  for (int u = 0; u < kHold; ++u) { hw0[u] = get_wx(tid + u * kThreads, 0); hw1[u] = get_wx(tid + u * kThreads, 1); }
+  uint4 X[2][KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int e = 32 * s + 8 * kb, at = e < E ? e : 0;
+    X[0][s] = load16(static_cast<const bf16_t*>(a.ddT) + off + at);
+    X[1][s] = load16(static_cast<const bf16_t*>(a.ddL) + off + at);
+  }
+  constexpr bool kAhead = KS <= 2;   // (registers) dx is asked for ahead too
+  uint4 was[kAhead ? KS : 1];
+  if constexpr (kAhead) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) was[s] = load16(static_cast<const bf16_t*>(a.dx) + off + (32 * s + 8 * kb < E ? 32 * s + 8 * kb : 0));
+  }
+  for (int i = tid; i < 16 * Epad; i += kThreads) {   // (the step sizes' weights, all ranks of a channel side by side: a few loads)
+    const int q = i & 15, e = i >> 4;
+    const bool ok = q < R && e < E;
+    wq[q * LQ + e] = ok ? f32_to_bf16_bits(a.wT[e * R + q]) : 0;
+    wq[(16 + q) * LQ + e] = ok ? f32_to_bf16_bits(a.wL[e * R + q]) : 0;
+  }
+#pragma unroll
+  for (int u = 0; u < kHold; ++u) put_wx(tid + u * kThreads, hw0[u], hw1[u]);
+  for (int i = tid + kHold * kThreads; i < nwx; i += kThreads) put_wx(i, get_wx(i, 0), get_wx(i, 1));
+  for (int i = l; i < 16 * zst / 2; i += 64) reinterpret_cast<uint32_t*>(zs)[i] = 0u;   // padding columns: zero
+
+  const int cb = l >> 2, n0 = 4 * (l & 3);   // dB_T, dB_L, dC: lane l holds 4 values of position l >> 2
+  uint2 bc[3];
+  sum_channels(a, p0, rows, cb, n0, bc);
+  __syncthreads();
+
+  // dz[., rank] = dpre w, channels as the inner dimension
+  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int e = 32 * s + 8 * kb;
+    if (32 * s >= E) break;      // (uniform)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      uint4 v = in && e < E ? X[h][s] : z4;
+      if (!given) {
+        const uint4 d = in && e < E ? load16(static_cast<const bf16_t*>(h ? a.dL : a.dT) + off + e) : z4;
+        const uint32_t gw[4] = {v.x, v.y, v.z, v.w}, dw[4] = {d.x, d.y, d.z, d.w};
+        uint32_t r[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) r[k] = pack2(bf16_lo(gw[k]) * softplus_slope(bf16_lo(dw[k])), bf16_hi(gw[k]) * softplus_slope(bf16_hi(dw[k])));
+        v = make_uint4(r[0], r[1], r[2], r[3]);
+        // for the weight-gradient kernel; rows past the end too, as zeros
+        if (e < E) *reinterpret_cast<uint4*>(a.dpt + (h ? (int64_t)a.ntiles * kTP * E : 0) + (p0 + mn) * E + e) = v;
+      }
+      acc[h] = mfma16(load16(wq + (16 * h + mn) * LQ + e), v, acc[h]);
+    }
+  }
+  // rows of dz to LDS as bf16: operand of the next product, and source of the copy in memory
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int q = 4 * kb + i;
+    if (q < R) {
+      zs[mn * zst + q] = f32_to_bf16_bits(acc[0][i]);
+      zs[mn * zst + R + q] = f32_to_bf16_bits(acc[1][i]);
+    }
+  }
+#pragma unroll
+  for (int w = 0; w < 3; ++w) {
+    uint32_t* dst = reinterpret_cast<uint32_t*>(zs + cb * zst + R2 + w * kN + n0);   // even offsets: 4-byte aligned
+    dst[0] = bc[w].x;
+    dst[1] = bc[w].y;
+  }
+  wave_sync_lds();
+  {
+    uint16_t* dzt = a.dzt + p0 * a.Opad;   // rows past the end of the arrays (up to the next tile) are written too, as zeros
+    const int per_row = a.Opad / 8;        // 16-byte pieces of a row
+    for (int i = l; i < 16 * per_row; i += 64) {
+      const int c = i / per_row, o8 = i - c * per_row;
+      *reinterpret_cast<uint4*>(dzt + (uint32_t)(c * a.Opad + 8 * o8)) = load16(zs + c * zst + 8 * o8);
+    }
+  }
+  // dx += dz Wx, outputs as the inner dimension; a pair of tiles lists its rows so that a lane ends with 8 neighbouring channels
+  uint4 A2[3];
+#pragma unroll
+  for (int ks = 0; ks < 3; ++ks) A2[ks] = 32 * ks < a.Opad32 ? load16(zs + mn * zst + 32 * ks + 8 * kb) : z4;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int e = 32 * s + 8 * kb, row = 32 * s + 8 * (mn >> 2) + (mn & 3);
+    if (32 * s >= E) break;      // (uniform)
+    bf16_t* at = static_cast<bf16_t*>(a.dx) + off + (e < E ? e : 0);
+    const uint4 old = kAhead ? was[kAhead ? s : 0] : load16(at);
+    float v[8];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 3; ++ks)
+        if (32 * ks < a.Opad32) d = mfma16(load16(wx + (row + 4 * t) * zst + 32 * ks + 8 * kb), A2[ks], d);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[4 * t + i] = d[i];
+    }
+    const uint32_t w[4] = {old.x, old.y, old.z, old.w};
+    float sum[8];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { sum[2 * k] = bf16_lo(w[k]) + v[2 * k]; sum[2 * k + 1] = bf16_hi(w[k]) + v[2 * k + 1]; }
+    if (in && e < E) *reinterpret_cast<uint4*>(at) = pack8(sum);
   }
 }
 
@@ -1383,32 +1540,35 @@ int run_proj_fwd_mfma(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) 
 }
 
 // The weights in LDS, straight from the caller's tensors: see the kernel.
-bool proj_fwd_in_lds(const ProjGeometry& g) { return g.mfma && g.E <= kFlMaxE && g.R <= kFlMaxR; }
-template <int KS, int NL>
+bool proj_in_lds(const ProjGeometry& g) { return g.mfma && g.E <= kFlMaxE && g.R <= kFlMaxR; }
+// More dynamic LDS than 64 KB has to be allowed, once per kernel and device.
+template <auto Kernel>
+bool allow_lds(size_t bytes) {
+  static std::atomic<uint64_t> seen{0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (seen.load(std::memory_order_acquire) & bit) return true;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
+  seen.fetch_or(bit, std::memory_order_release);
+  return true;
+}
+template <int KS, int NL, bool PACKED>
 int launch_proj_fwd_lds(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
-  const int Epad = (g.E + 31) / 32 * 32;
-  const size_t lds = fl_lds_bytes(Epad, NL);
-  auto go = [&](auto kernel) -> int {
-    if (lds > 64 * 1024) {   // (more dynamic LDS than that has to be allowed, once per kernel and device)
-      static std::atomic<uint64_t> seen{0};
-      int dev = 0;
-      if (hipGetDevice(&dev) != hipSuccess) return M2D_ERR_HIP;
-      const uint64_t bit = 1ull << (dev & 63);
-      if (!(seen.load(std::memory_order_acquire) & bit)) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)fl_lds_bytes(kFlMaxE, NL)) != hipSuccess) return M2D_ERR_HIP;
-        seen.fetch_or(bit, std::memory_order_release);
-      }
-    }
-    const int64_t tiles = (g.P + kTP - 1) / kTP;
-    int64_t grid = 256 * (int64_t)((160 * 1024) / lds < 6 ? (160 * 1024) / lds : 6);   // as many workgroups as the device holds
-    if (grid > tiles) grid = tiles;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kThreads), lds, st, a);
-    return launched() ? M2D_OK : M2D_ERR_HIP;
-  };
-  return a.bc_packed ? go(&m2d_proj_fwd_lds_kernel<KS, NL, true>) : go(&m2d_proj_fwd_lds_kernel<KS, NL, false>);
+  const size_t lds = fl_lds_bytes((g.E + 31) / 32 * 32, NL);
+  if (lds > 64 * 1024 && !allow_lds<&m2d_proj_fwd_lds_kernel<KS, NL, PACKED>>(fl_lds_bytes(kFlMaxE, NL))) return M2D_ERR_HIP;
+  const int64_t tiles = (g.P + kTP - 1) / kTP;
+  int64_t grid = 256 * (int64_t)((160 * 1024) / lds < 6 ? (160 * 1024) / lds : 6);   // as many workgroups as the device holds
+  if (grid > tiles) grid = tiles;
+  hipLaunchKernelGGL((m2d_proj_fwd_lds_kernel<KS, NL, PACKED>), dim3((unsigned)grid), dim3(kThreads), lds, st, a);
+  return launched() ? M2D_OK : M2D_ERR_HIP;
 }
 int run_proj_fwd_lds(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
-  auto ranks = [&](auto ks) -> int { return g.R <= 8 ? launch_proj_fwd_lds<decltype(ks)::value, 1>(g, a, st) : launch_proj_fwd_lds<decltype(ks)::value, 2>(g, a, st); };
+  auto ranks = [&](auto ks) -> int {
+    constexpr int KS = decltype(ks)::value;
+    if (g.R <= 8) return a.bc_packed ? launch_proj_fwd_lds<KS, 1, true>(g, a, st) : launch_proj_fwd_lds<KS, 1, false>(g, a, st);
+    return a.bc_packed ? launch_proj_fwd_lds<KS, 2, true>(g, a, st) : launch_proj_fwd_lds<KS, 2, false>(g, a, st);
+  };
   if (g.E <= 64) return ranks(std::integral_constant<int, 2>{});
   return g.E <= 128 ? ranks(std::integral_constant<int, 4>{}) : ranks(std::integral_constant<int, 8>{});
 }
@@ -1439,10 +1599,24 @@ int run_reduce(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
   return launched() ? M2D_OK : M2D_ERR_HIP;
 }
 
+template <int KS>
+int launch_proj_bwd_lds(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
+  auto bytes = [](int Epad, int Opad32) { return ((size_t)32 * (Epad + 8) + (size_t)(Epad + 16 * kWaves) * (Opad32 + 8)) * 2; };
+  const size_t lds = bytes((g.E + 31) / 32 * 32, g.Opad32), most = bytes(32 * KS, 96);
+  if (most > 64 * 1024 && !allow_lds<&m2d_proj_bwd_data_lds_kernel<KS>>(most)) return M2D_ERR_HIP;
+  hipLaunchKernelGGL(m2d_proj_bwd_data_lds_kernel<KS>, dim3(g.ntiles), dim3(kThreads), lds, st, a);
+  return launched() ? M2D_OK : M2D_ERR_HIP;
+}
 int run_proj_bwd_mfma(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
-  const size_t lds_data = (size_t)kWaves * (16 * kStageStride * 4 + 16 * (g.Opad32 + 8) * 2);
-  hipLaunchKernelGGL(m2d_proj_bwd_data_mfma_kernel, dim3(g.ntiles), dim3(kThreads), lds_data, st, a);
-  if (!launched()) return M2D_ERR_HIP;
+  int rc;
+  if (proj_in_lds(g)) {
+    rc = g.E <= 64 ? launch_proj_bwd_lds<2>(g, a, st) : (g.E <= 128 ? launch_proj_bwd_lds<4>(g, a, st) : launch_proj_bwd_lds<8>(g, a, st));
+  } else {
+    const size_t lds_data = (size_t)kWaves * (16 * kStageStride * 4 + 16 * (g.Opad32 + 8) * 2);
+    hipLaunchKernelGGL(m2d_proj_bwd_data_mfma_kernel, dim3(g.ntiles), dim3(kThreads), lds_data, st, a);
+    rc = launched() ? M2D_OK : M2D_ERR_HIP;
+  }
+  if (rc) return rc;
   const size_t lds_w = (size_t)(3 * kKC + g.Opad + 2 * 16 * ((g.R + 1 + 15) / 16)) * kPosStride * 2;
   hipLaunchKernelGGL(m2d_proj_bwd_weights_mfma_kernel, dim3(g.G, g.ne), dim3(kThreads), lds_w, st, a);
   if (!launched()) return M2D_ERR_HIP;
@@ -1499,7 +1673,7 @@ int m2d_proj_fwd(const m2d_desc* desc, int dt_rank, const void* x, const float* 
   char* ws = static_cast<char*>(workspace);
   PackArgs k = {};
   k.Wx = x_proj_w; k.wT = dt_projT_w; k.bT = dt_projT_b; k.wL = dt_projL_w; k.bL = dt_projL_b;
-  if (g.mfma && !proj_fwd_in_lds(g)) {
+  if (g.mfma && !proj_in_lds(g)) {
     k.bTp = reinterpret_cast<float*>(ws + g.off_bTp);
     k.bLp = reinterpret_cast<float*>(ws + g.off_bLp);
     k.Wb = reinterpret_cast<uint16_t*>(ws + g.off_Wb);
@@ -1519,7 +1693,7 @@ int m2d_proj_fwd(const m2d_desc* desc, int dt_rank, const void* x, const float* 
   a.Wb = k.Wb; a.wTb = k.wTb; a.wLb = k.wLb;
   a.r_out = lowrank; a.dT_out = deltaT; a.dL_out = deltaL; a.BT_out = BT; a.BL_out = BL; a.C_out = C;
   a.bc_packed = packed ? static_cast<float*>(BT) : nullptr;
-  if (proj_fwd_in_lds(g)) return run_proj_fwd_lds(g, a, st);
+  if (proj_in_lds(g)) return run_proj_fwd_lds(g, a, st);
   return g.mfma ? run_proj_fwd_mfma(g, a, st) : with_layout(desc->dtype == M2D_F32, g, [&](auto t, auto v4, auto nt) -> int {
     return run_proj_fwd_f32<decltype(t), v4(), nt()>(g, a, st);
   });
@@ -1557,7 +1731,7 @@ int m2d_proj_bwd_parts(const m2d_desc* desc, int dt_rank, int sum_parts, const v
   char* ws = static_cast<char*>(workspace);
   PackArgs k = {};
   k.Wx = x_proj_w; k.wT = dt_projT_w; k.wL = dt_projL_w;
-  if (g.mfma) {   // for the data kernel; the weight-gradient kernel needs no weights
+  if (g.mfma && !proj_in_lds(g)) {   // for the data kernel; the weight-gradient kernel needs no weights
     k.wTtb = reinterpret_cast<uint16_t*>(ws + g.off_wTtb);
     k.wLtb = reinterpret_cast<uint16_t*>(ws + g.off_wLtb);
     k.WxTb = reinterpret_cast<uint16_t*>(ws + g.off_WxTb);

@@ -1,4 +1,4 @@
-"""GPU tests of the forward projections with their weights in LDS (m2d_proj_fwd, bf16, up to 256 channels and a rank of 16).
+"""GPU tests of the projections with their weights in LDS (m2d_proj_fwd, m2d_proj_bwd_parts; bf16, up to 256 channels and a rank of 16).
 
 The products are repeated in fp64 from the operands that the kernel has: weights rounded to bf16, the low-rank inputs as bf16.
 What is left is the fp32 accumulation and one rounding to bf16 of a result: half a unit in the last place, 2^-9 relative, which an
@@ -58,7 +58,7 @@ CASES = [(1, 8, 1), (15, 16, 1), (16, 24, 2), (17, 32, 2), (63, 40, 3), (64, 64,
 
 @pytest.mark.parametrize("P,E,R", CASES, ids=lambda v: str(v))
 def test_products_of_the_operands(cabi, P, E, R):
-    print(f"\ncase proj_fwd_small {P} {E} {R}", flush=True)
+    print(f"\ncase proj_small {P} {E} {R}", flush=True)
     x, w = make(P, E, R)
     xd, wd = x.cuda(), [t.cuda() for t in w]
     out = cabi.proj_fwd(xd, *wd, N)
@@ -84,7 +84,7 @@ def test_products_of_the_operands(cabi, P, E, R):
 @pytest.mark.parametrize("E,R", [(64, 4), (72, 9)])
 def test_values_that_are_not_finite_stay_in_their_position(cabi, E, R):
     """An infinite low-rank input of one step size must not reach the other, a NaN none of the other positions."""
-    print(f"\ncase proj_fwd_small nonfinite {E} {R}", flush=True)
+    print(f"\ncase proj_small nonfinite {E} {R}", flush=True)
     x, w = make(70, E, R)
     w = [t.clone() for t in w]
     w[0][R - 1] = 0
@@ -99,3 +99,47 @@ def test_values_that_are_not_finite_stay_in_their_position(cabi, E, R):
         assert torch.equal(u[:, keep], v[:, keep])
     assert b[0][0, 3, 0, R - 1].isinf() and all(t[0, 20].isnan().all() for t in b)
     assert b[2][0, 3].isfinite().all()
+
+
+# the same edges; channel sums of the scan in parts (0: whole arrays in bf16), whose loads go out in fours and a remainder
+BWD = [(1, 8, 1, 0), (15, 16, 1, 1), (17, 32, 2, 2), (63, 40, 3, 4), (64, 64, 4, 5), (65, 72, 5, 8), (130, 96, 6, 0), (127, 128, 8, 16),
+       (129, 136, 9, 3), (64, 160, 10, 0), (77, 200, 13, 7), (192, 248, 16, 4), (333, 256, 16, 9), (50, 64, 16, 0), (9000, 24, 2, 6)]
+
+
+@pytest.mark.parametrize("dpre", [False, True], ids=["d_delta", "dpre"])
+@pytest.mark.parametrize("P,E,R,parts", BWD, ids=lambda v: str(v))
+def test_input_gradient_of_the_operands(cabi, P, E, R, parts, dpre):
+    """dx, against fp64 products of the operands that the kernel has.  A gradient before the second product is rounded to bf16 and may
+    fall on the next value: 2^-8 of it, with the product's weights; dx itself is rounded once: 2^-8 of it."""
+    print(f"\ncase proj_bwd_small {P} {E} {R} {parts} {dpre}", flush=True)
+    x, w = make(P, E, R, 1)
+    g = torch.Generator().manual_seed(P + E)
+    bf = lambda n: torch.randn(1, P, 1, n, generator=g).bfloat16()
+    low, dT, dL, ddT, ddL, dx0 = bf(2 * R), bf(E).abs(), bf(E).abs(), bf(E), bf(E), bf(E)
+    if parts:
+        sums = torch.randn(parts, 1, P, 1, 3 * N, generator=g)
+        d3 = [sums.sum(0)[0, :, 0, k * N:(k + 1) * N].bfloat16() for k in (1, 2, 0)]      # records hold d_C, d_BT, d_BL
+        given = (sums.cuda(), None, None)
+    else:
+        d3 = [bf(N) for _ in range(3)]
+        given = tuple(t.cuda() for t in d3)
+        d3 = [t[0, :, 0] for t in d3]
+    dx = dx0.cuda()
+    c = lambda t: t.cuda()
+    gw = cabi.proj_bwd(c(x), c(low), None if dpre else c(dT), None if dpre else c(dL), c(w[0]), c(w[1]), c(w[3]), c(ddT), c(ddL), *given, dx,
+                       dpre=dpre, sum_parts=parts)
+    torch.cuda.synchronize()
+    wx, wT, wL = [t.bfloat16().double() for t in (w[0], w[1], w[3])]
+    flat = lambda t: t.double()[0, :, 0]
+    pre = [flat(a) if dpre else (flat(a) * -torch.expm1(-flat(b))) for a, b in ((ddT, dT), (ddL, dL))]
+    dz = torch.cat([pre[0].bfloat16().double() @ wT, pre[1].bfloat16().double() @ wL] + [t.double() for t in d3], 1)
+    # d_delta times the slope is rounded to bf16 before the first product, and may fall on the next value as well
+    moved = 2.0 ** -8 * torch.cat([pre[0].abs() @ wT.abs() + dz[:, :R].abs(), pre[1].abs() @ wL.abs() + dz[:, R:2 * R].abs(), dz[:, 2 * R:].abs()], 1)
+    want = flat(dx0) + dz @ wx
+    lim = moved @ wx.abs() + 2.0 ** -8 * want.abs() + 1e-5 * want.abs().max()
+    bad = (flat(dx.cpu()) - want).abs() > lim
+    assert not bad.any(), (int(bad.sum()), float((flat(dx.cpu()) - want).abs().max()))
+    # the weight gradients read the dz and dpre that this kernel wrote
+    for got, ref in ((gw[0], dz.T @ flat(x)), (gw[1], pre[0].T @ flat(low)[:, :R]), (gw[2], pre[0].sum(0)), (gw[3], pre[1].T @ flat(low)[:, R:]),
+                     (gw[4], pre[1].sum(0))):
+        assert got.shape == ref.shape and float((got.double().cpu() - ref).abs().max()) < 2e-2 * float(ref.abs().max())
