@@ -39,3 +39,10 @@ def test_infinite_and_undefined_values_pass_through():
     w = torch.ones(64, 64, dtype=torch.bfloat16, device="cuda")
     y = cabi.wide_linear_fwd(x, w, None, gelu=True).float()
     assert torch.isinf(y[3]).all() and torch.isnan(y[599]).all() and (y[:3] == 0).all() and (y[4:599] == 0).all()
+
+
+@pytest.mark.parametrize("case", [(150001, 64, 64, True), (98304, 32, 128, False), (98305, 288, 64, True), (49152, 320, 128, True)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_ranges_of_several_tiles(case):
+    """Few outputs and many positions: a workgroup's range of units takes it through several tiles, also where the units go out evenly."""
+    test_against_float64(case)
