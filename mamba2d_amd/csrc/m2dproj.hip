@@ -303,9 +303,10 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_fwd_mfma_kern
 // step sizes, for which a pair of tiles lists its rows as 8 (m >> 2) + 4 t + (m & 3).  The low-rank inputs of the step sizes stay in the registers
 // that they were made in: the second product lists its contraction in their order, and those of the other step size are masked out, so that
 // an infinite value of one does not meet the other's zero weights.  Against the kernel above
-// and its packing launch, ten calls in a row: 64x56x56x64 43.1 -> 28.8 us (104 MB, 3.6 TB/s), 4x128x128x64 19.6 -> 13.4, 64x28x28x128 28.2 -> 22.7,
-// 64x14x14x256 27.0 -> 24.4, 200000 positions of 32 channels 39.2 -> 18.3, 4096 of 64 11.1 -> 7.2; no size measured was slower.  What is left at 64 channels
-// is the copying in of the weights and the softplus.
+// and its packing launch, ten calls in a row: 64x56x56x64 43.1 -> 24.7 us (104 MB, 4.2 TB/s), 4x128x128x64 19.6 -> 11.8, 64x28x28x128 28.2 -> 18.4,
+// 64x14x14x256 27.0 -> 18.6, 200000 positions of 32 channels 39.2 -> 16.6, 4096 of 64 11.1 -> 5.2; no size measured was slower.  A thread's share of the
+// weights is asked for at once: with loops that waited for each load they were 28.8, 13.4, 22.7, 24.4, 18.3 and 7.2.  What is left at 64 channels is
+// the copying in of the weights and the softplus.
 constexpr int kFlD = 40;      // bf16 per row of the step sizes' weights in LDS: 32 + 8
 constexpr int kFlMaxE = 256, kFlMaxR = 16;
 constexpr size_t fl_lds_bytes(int Epad, int NL) { return ((size_t)(16 * NL + 3 * kN) * (Epad + 8) + 2 * (size_t)Epad * kFlD) * 2 + 2 * (size_t)Epad * 4; }
@@ -334,32 +335,47 @@ __global__ __launch_bounds__(kThreads) void m2d_proj_fwd_lds_kernel(const ProjAr
       next[s] = load16(row + (e < E ? e : 0));                  // (channels past E meet zero weights, but must be finite: masked below)
     }
   };
-  fetch(blockIdx.x);
-  for (int i = tid; i < NZ * (Epad / 4); i += kThreads) {
-    const int row = i / (Epad / 4), c = 4 * (i - row * (Epad / 4)), t = row >> 4, m = row & 15;
+  // All of the workgroup's loads go out before the first wait: the weights, a thread's share unrolled, then its first rows of x.
+  constexpr int kPieces = (NZ * 8 * KS + kThreads - 1) / kThreads, kDt = 2 * KS;
+  const int nz = NZ * (Epad / 4), ndt = E * R;
+  f32x4 hz[kPieces];
+  float hT[kDt], hL[kDt];
+#pragma unroll
+  for (int u = 0; u < kPieces; ++u) {
+    const int i = tid + u * kThreads, row = i / (Epad / 4), c = 4 * (i - row * (Epad / 4)), t = row >> 4, m = row & 15;
     const int q = m & 3, state = PACKED ? 4 * (q == 1 ? 2 : (q == 2 ? 1 : q)) + (m >> 2) : m;
     const int o = t < NL ? row : R2 + 16 * (t - NL) + state;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (c < E && (t >= NL || o < R2)) v = *reinterpret_cast<const float4*>(a.Wx + (int64_t)o * E + c);
-    *reinterpret_cast<uint2*>(wz + row * LW + c) = make_uint2(pack2(v.x, v.y), pack2(v.z, v.w));
+    const bool ok = i < nz && c < E && (t >= NL || o < R2);
+    hz[u] = load_f4(a.Wx + (ok ? o * E + c : 0));
+    if (!ok) hz[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
-  for (int i = tid; i < Epad * 16; i += kThreads) {             // slots 2 (i % 16) and the next of channel e: low-rank inputs o, o + 1
-    const int e = i >> 4, s = 2 * (i & 15), j = s & 7, o = (j < 4 ? j : 12 + j) + 4 * (s >> 3);
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
-    if (e < E) {
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        if (o + k < R) v[k] = a.wT[(int64_t)e * R + o + k];
-        else if (o + k < R2) v[2 + k] = a.wL[(int64_t)e * R + o + k - R];
-      }
-    }
-    *reinterpret_cast<uint32_t*>(wT + e * kFlD + s) = pack2(v[0], v[1]);
-    *reinterpret_cast<uint32_t*>(wL + e * kFlD + s) = pack2(v[2], v[3]);
+  for (int u = 0; u < kDt; ++u) {
+    const int i = tid + u * kThreads;
+    hT[u] = a.wT[i < ndt ? i : 0];
+    hL[u] = a.wL[i < ndt ? i : 0];
   }
-  for (int e = tid; e < Epad; e += kThreads) {
-    const float t = e < E ? a.bT[e] : 0.f, v = e < E ? a.bL[e] : 0.f;
-    bT[e] = a.round ? as_stored(t, static_cast<const bf16_t*>(nullptr)) : t;
-    bL[e] = a.round ? as_stored(v, static_cast<const bf16_t*>(nullptr)) : v;
+  const float hbT = a.bT[tid < E ? tid : 0], hbL = a.bL[tid < E ? tid : 0];   // (E <= the threads of a workgroup)
+  fetch(blockIdx.x);
+  for (int i = tid; i < 2 * Epad * kFlD / 8; i += kThreads) reinterpret_cast<uint4*>(wT)[i] = zero16();   // (wL follows)
+  if (tid < Epad) {
+    bT[tid] = tid >= E ? 0.f : (a.round ? as_stored(hbT, static_cast<const bf16_t*>(nullptr)) : hbT);
+    bL[tid] = tid >= E ? 0.f : (a.round ? as_stored(hbL, static_cast<const bf16_t*>(nullptr)) : hbL);
+  }
+#pragma unroll
+  for (int u = 0; u < kPieces; ++u) {
+    const int i = tid + u * kThreads, row = i / (Epad / 4), c = 4 * (i - row * (Epad / 4));
+    if (i < nz) *reinterpret_cast<uint2*>(wz + row * LW + c) = make_uint2(pack2(hz[u][0], hz[u][1]), pack2(hz[u][2], hz[u][3]));
+  }
+  __syncthreads();
+  auto slot_of = [](int o) { return 8 * ((o & 15) >> 2) + (o & 3) + (o < 16 ? 0 : 4); };   // of low-rank input o in the second product
+#pragma unroll
+  for (int u = 0; u < kDt; ++u) {
+    const int i = tid + u * kThreads, e = i / R, q = i - e * R;
+    if (i < ndt) {
+      wT[e * kFlD + slot_of(q)] = f32_to_bf16_bits(hT[u]);
+      wL[e * kFlD + slot_of(q + R)] = f32_to_bf16_bits(hL[u]);
+    }
   }
   // which of the lane's low-rank inputs are the T step size's, which the L one's
   uint32_t mT[2 * NL], mL[2 * NL];
@@ -632,8 +648,9 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_bwd_data_mfma
 // and for dx, asked for at the end.  Here a workgroup rounds the weights into LDS from the caller's tensors, and everything is asked for before the first
 // wait, dx too where registers allow four workgroups a compute unit (up to 64 channels; with 128 three fitted, and 784 tiles of 64x28x28x128 took a second
 // generation for the last 16: whole backward 56.5 us against 50.3 without).  The weights' rows are the first operands, so dx leaves from registers, 16 bytes a lane.
-// Backward of the projections in all, ten calls in a row: 64x56x56x64, 4 parts 91.5 -> 81.9 us, 64x28x28x128, 8 parts 57.7 -> 50.3, 4x128x128x64, 8 parts 47.2 ->
-// 42.3, 64x14x14x256, 16 parts 46.7 -> 43.1, 200000 positions of 32 channels 68.8 -> 53.7, 1568 of 64 17.4 -> 14.9; bit for bit the same results.
+// Backward of the projections in all, ten calls in a row: 64x56x56x64, 4 parts 91.5 -> 77.6 us, 64x28x28x128, 8 parts 57.7 -> 48.0, 4x128x128x64, 8 parts 47.2 ->
+// 40.8, 64x14x14x256, 16 parts 46.7 -> 39.8, 200000 positions of 32 channels 68.8 -> 51.9, 1568 of 64 17.4 -> 13.9 (with the step sizes' weights in a loop that
+// waited for each load 81.9, 50.3, 42.3, 43.1, 53.7 and 14.9); bit for bit the same results.
 template <int KS>   // steps of 32 channels at most
 __global__ __launch_bounds__(kThreads, KS <= 4 ? 4 : 2) void m2d_proj_bwd_data_lds_kernel(const ProjArgs a) {
   extern __shared__ float smem[];
@@ -675,6 +692,15 @@ __global__ __launch_bounds__(kThreads, KS <= 4 ? 4 : 2) void m2d_proj_bwd_data_l
   };
 #pragma unroll
   for (int u = 0; u < kHold; ++u) { hw0[u] = get_wx(tid + u * kThreads, 0); hw1[u] = get_wx(tid + u * kThreads, 1); }
+  constexpr int kDt = 2 * KS;
+  const int ndt = E * R;
+  float hT[kDt], hL[kDt];
+#pragma unroll
+  for (int u = 0; u < kDt; ++u) {
+    const int i = tid + u * kThreads;
+    hT[u] = a.wT[i < ndt ? i : 0];
+    hL[u] = a.wL[i < ndt ? i : 0];
+  }
   uint4 X[2][KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
@@ -688,16 +714,20 @@ __global__ __launch_bounds__(kThreads, KS <= 4 ? 4 : 2) void m2d_proj_bwd_data_l
 #pragma unroll
     for (int s = 0; s < KS; ++s) was[s] = load16(static_cast<const bf16_t*>(a.dx) + off + (32 * s + 8 * kb < E ? 32 * s + 8 * kb : 0));
   }
-  for (int i = tid; i < 16 * Epad; i += kThreads) {   // (the step sizes' weights, all ranks of a channel side by side: a few loads)
-    const int q = i & 15, e = i >> 4;
-    const bool ok = q < R && e < E;
-    wq[q * LQ + e] = ok ? f32_to_bf16_bits(a.wT[e * R + q]) : 0;
-    wq[(16 + q) * LQ + e] = ok ? f32_to_bf16_bits(a.wL[e * R + q]) : 0;
+  for (int i = tid; i < 32 * LQ / 8; i += kThreads) reinterpret_cast<uint4*>(wq)[i] = z4;
+  for (int i = l; i < 16 * zst / 2; i += 64) reinterpret_cast<uint32_t*>(zs)[i] = 0u;   // padding columns: zero
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kDt; ++u) {
+    const int i = tid + u * kThreads, e = i / R, q = i - e * R;
+    if (i < ndt) {
+      wq[q * LQ + e] = f32_to_bf16_bits(hT[u]);
+      wq[(16 + q) * LQ + e] = f32_to_bf16_bits(hL[u]);
+    }
   }
 #pragma unroll
   for (int u = 0; u < kHold; ++u) put_wx(tid + u * kThreads, hw0[u], hw1[u]);
   for (int i = tid + kHold * kThreads; i < nwx; i += kThreads) put_wx(i, get_wx(i, 0), get_wx(i, 1));
-  for (int i = l; i < 16 * zst / 2; i += 64) reinterpret_cast<uint32_t*>(zs)[i] = 0u;   // padding columns: zero
 
   const int cb = l >> 2, n0 = 4 * (l & 3);   // dB_T, dB_L, dC: lane l holds 4 values of position l >> 2
   uint2 bc[3];
@@ -1558,7 +1588,8 @@ int launch_proj_fwd_lds(const ProjGeometry& g, const ProjArgs& a, hipStream_t st
   const size_t lds = fl_lds_bytes((g.E + 31) / 32 * 32, NL);
   if (lds > 64 * 1024 && !allow_lds<&m2d_proj_fwd_lds_kernel<KS, NL, PACKED>>(fl_lds_bytes(kFlMaxE, NL))) return M2D_ERR_HIP;
   const int64_t tiles = (g.P + kTP - 1) / kTP;
-  int64_t grid = 256 * (int64_t)((160 * 1024) / lds < 6 ? (160 * 1024) / lds : 6);   // as many workgroups as the device holds
+  constexpr size_t most = KS == 2 ? 6 : (KS == 4 ? 4 : 2);   // workgroups whose registers fit a compute unit
+  int64_t grid = 256 * (int64_t)((160 * 1024) / lds < most ? (160 * 1024) / lds : most);   // as many as the device holds
   if (grid > tiles) grid = tiles;
   hipLaunchKernelGGL((m2d_proj_fwd_lds_kernel<KS, NL, PACKED>), dim3((unsigned)grid), dim3(kThreads), lds, st, a);
   return launched() ? M2D_OK : M2D_ERR_HIP;
