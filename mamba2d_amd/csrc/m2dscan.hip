@@ -2972,8 +2972,8 @@ Geometry make_geometry(const m2d_desc* d) {
   int64_t split_cost = stream_cost(wg4, kSplit4);
   if (stream_cost(wg8, kSplit8) < split_cost) { split_cost = stream_cost(wg8, kSplit8); split_nw = kSplitWaves; }
   // (one set of channel sums per workgroup of an image: with 4 or 8 channels per workgroup that memory is bounded here unless the caller insists.  A bound
-  // on memory, not on time: at E=64 fp32 the split backward would take 5.42 of 7.35 ms at 1280x1280 for 1.2 GB of scratch more, 12.95 of 14.2 at
-  // 2048x2048 for 3.1 GB; at 8x512x512x64 bf16 6.1 for 5.5 ms and 2.3 GB)
+  // on memory, not on time: at E=64 fp32 the split backward would take 4.34 of 7.3 ms at 1280x1280 for 1.2 GB of scratch more, 10.2 of 13.2 at
+  // 2048x2048 for 3.1 GB)
   auto sums_fit = [&](int nw) { return sizeof(float) * (size_t)((d->E + nw - 1) / nw) * 3 * kN * (size_t)d->B * d->H * d->W <= ((size_t)2 << 30); };
   const bool link4 = g.nbands >= 2 && 5 * wg4 * (lagged < g.nbands ? lagged : g.nbands) <= 7 * ncu;
   if (g.nbands >= 2) {

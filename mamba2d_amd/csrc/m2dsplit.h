@@ -16,7 +16,7 @@
 // places as it can.  A store takes several times as long to be acknowledged as a block takes, and the counter that a wave waits on
 // retires in order: every block issues the same operations whatever lanes they are for, so that a wave knows how many of them may still be under way
 // (split_landed), and rows of a neighbour, which are fetched at the last moment, come in through a wave that stores nothing before them.
-// Against sweeping waves that also stage, forward keeping snapshots / backward: 1x256x256x64 fp32 0.298 / 0.683 -> 0.196 / 0.480 ms,
+// Against sweeping waves that also stage, forward keeping snapshots / backward: 1x256x256x64 fp32 0.298 / 0.683 -> 0.196 / 0.480 ms (0.183 / 0.382 with the wider stores),
 // 1x256x256x62 (rows of no whole chunks) 0.476 / 1.157 -> 0.226 / 0.572, 4x128x128x64 bf16 0.183 / 0.442 -> 0.111 / 0.315.
 // Memory formats and schedules are those of the whole-state kernels, so either pass may use either layout.
 constexpr int kSplitWaves = 8;       // sweeping waves (channels) per workgroup
