@@ -2166,6 +2166,7 @@ __global__ __launch_bounds__((bwd2_threads<MODE, NW>())) void m2d_bwd2_kernel(co
   const uint32_t tile_get = (uint32_t)(r * 64 + (slot ^ (r >> 2)) * 16);
   const bool tile_ok = e_wg0 + 8 * slot < p.E;
   static_assert(!TILE || (CW * sizeof(T) == 64 && CS == 4), "a row of the tile is four pieces");
+  static_assert(!TILE || (BATCH && WIDE), "the tile is stored where a half-pass's channel sums are added up");
   const uint32_t row_const_off = SG::kConstPlane * SG::kPlane + r * 16;
   const uint32_t bot_step = (uint32_t)p.E * (uint32_t)(kN * sizeof(float)), bot_wrap = (uint32_t)p.S * bot_step;   // boundary rows: bytes from column to column; back to column 0
 
