@@ -738,17 +738,18 @@ __global__ __launch_bounds__(256) void m2d_wide_linear_kernel(const WideArgs a) 
 // slots a value, half of the time) and the products.  A wave keeps 32 positions' rows in registers as they come from
 // memory and walks over the outputs 32 at a time; the 32 rows of W lie in LDS, read by all waves, while the next 32 are
 // on their way; three workgroups fit a compute unit, which is why 320 inputs are the most (with workgroups of 8 waves, two
-// waves to a SIMD, 320 -> 1280 took 68 us at 25088 positions).  The work is dealt out in units of 32 outputs, in equal ranges
-// to as many workgroups as the chip holds, a range going on into the next tile of positions; slices of a tile, 784 workgroups at
-// 25088 positions, left 16 of them for a second round.  W's rows are the first operand of the product, so a lane
+// waves to a SIMD, 320 -> 1280 took 68 us at 25088 positions).  W's rows are the first operand of the product, so a lane
 // ends with four neighbouring outputs of a position at a time, which leave through LDS as 64-byte pieces.
-// 320 -> 1280, in slices and in ranges: 50176 positions 100 and 80 us, 25088 55 and 47, 19600 46 and 38, 12544 32 and 30, 6272
-// 22 and 21; the stock pair: 25088 positions 61 us, 6272 28, 1568 25 (bound by the host; 12 here).
+// 320 -> 1280, the fewest equal slices of a tile's outputs that make 768 workgroups, and the slices chosen below: 50176 positions 93 and 77 us,
+// 25088 52 and 46, 19600 43 and 40, 12544 31 and 27, 6272 22 and 18, 1568 11.5 both; the stock pair 61 us at 25088, 28 at 6272.
+// Equal ranges of the whole work for 768 workgroups, a range going on into the next tile, took 77, 46, 38, 29, 21 and 11.5, but lost 2 to 20 %
+// to slices where outputs are few or inputs many (40000 positions, 320 -> 256: 28.4 us against 23.2), as a tile's rows of x are then
+// waited for in the middle of a workgroup.
 // 512 -> 2048 at 6272 positions, with 16 positions to a wave so that it fits: 44 us against 34, so those stay stock.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 constexpr int64_t kGlFewest = 512;      // positions up to which the kernel above is the faster one
 constexpr int kGlInputs = 320;          // most inputs with which three workgroups fit a compute unit's LDS
-constexpr int kGlWant = 768;            // workgroups that the chip holds
+constexpr int64_t kGlMost = 8192;       // workgroups beyond which more slices are not looked at
 constexpr int kGlWaves = 4, kGlThreads = 64 * kGlWaves, kGlRows = 32 * kGlWaves;
 constexpr int kGlStage = 32 + 8;        // bf16 per staged position
 struct GeluLinArgs {
@@ -756,7 +757,8 @@ struct GeluLinArgs {
   uint16_t* y;
   int64_t P;
   int K, N;
-  int units, share, over;      // units: 32 outputs of a tile of positions, a tile's follow each other; of a workgroup: share, `over` of them one more
+  int nsplit, steps, over;       // slices of the outputs; steps of 64 of them in a slice, `over` slices have one more
+  uint32_t per_slice;            // 2^32 / nsplit, rounded up: exact as a quotient while (workgroups) x nsplit < 2^32
 };
 
 // KS: steps of 16 inputs the kernel is built for (the operands past K are zero)
@@ -770,24 +772,29 @@ __global__ __launch_bounds__(kGlThreads, 3) void m2d_gelu_linear_kernel(const Ge
   __shared__ __attribute__((aligned(16))) float bl[2][32];      // bias of the 32 outputs
   const int tid = threadIdx.x, l = tid & 63, r = l & 31, h = l >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // the workgroup's units; neighbouring ranges, which share the rows of x of a tile, go to the same XCD (workgroups are
-  // dealt out round-robin over 8)
-  const int mine = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const uint32_t wgs = gridDim.x, ones = (uint32_t)(mine * a.over) / wgs;      // (the larger shares are spread evenly: a compute unit gets some of both)
-  const int begin = mine * a.share + (int)ones, count = a.share + (int)((uint32_t)((mine + 1) * a.over) / wgs - ones), chunks = a.N / 32;
-  if (begin >= a.units) return;      // (the whole workgroup: two units each, and fewer pairs than workgroups)
-  int64_t tile = begin / chunks;
-  int chunk = begin - (int)tile * chunks;
+  // the slices of the same positions go to the same XCD (workgroups are dealt out round-robin over 8), whose L2 then holds their
+  // rows of x for all of them: an eighth of all slices each, which may part those of one tile, so that no XCD has a tile more than another.
+  // (Every division here was 0.1 us of each workgroup's start: 4000 positions, 256 -> 1024 10.7 us, 11.2 with four of them.)
+  const uint32_t mine = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const uint32_t tile = a.nsplit == 1 ? mine : __umulhi(mine, a.per_slice);
+  const int slice = (int)(mine - tile * (uint32_t)a.nsplit);
+  const int n0 = 64 * (slice * a.steps + (slice < a.over ? slice : a.over)), chunks = 2 * (a.steps + (slice < a.over ? 1 : 0));
+  const int64_t p0 = (int64_t)tile * kGlRows + wave * 32;
+  if ((int64_t)tile * kGlRows >= a.P) return;      // (the whole workgroup)
+  const int64_t first = p0 < a.P ? p0 : a.P - 1;      // rows past the end repeat the last one and are not stored
+  const int left = a.P - first < 32 ? (int)(a.P - first) : 32, stored = p0 < a.P ? left : 0;
+  const int row = r < left ? r : left - 1;
+  uint16_t* y = a.y + first * a.N + n0;
   const int wr = tid / kPer, wc = 8 * (tid % kPer);
   uint4 next[kPieces];
   float nb = 0.f;
   const uint4 z4 = make_uint4(0u, 0u, 0u, 0u);
   auto fetch = [&](int chunk) {
-    const uint16_t* src = a.w + (int64_t)(32 * chunk) * a.K;
+    const uint16_t* src = a.w + (int64_t)(n0 + 32 * chunk) * a.K;
 #pragma unroll
     for (int u = 0; u < kPieces; ++u)
       if (wc + 8 * kPer * u < a.K) next[u] = ld16(src + (uint32_t)(wr * a.K + wc + 8 * kPer * u));
-    if (tid < 32) nb = a.bias ? __uint_as_float((uint32_t)a.bias[32 * chunk + tid] << 16) : 0.f;
+    if (tid < 32) nb = a.bias ? __uint_as_float((uint32_t)a.bias[n0 + 32 * chunk + tid] << 16) : 0.f;
   };
   auto put = [&](int b) {
 #pragma unroll
@@ -802,53 +809,43 @@ __global__ __launch_bounds__(kGlThreads, 3) void m2d_gelu_linear_kernel(const Ge
       if (at >= a.K && at < 16 * KS) *reinterpret_cast<uint4*>(&wl[0][wr * kRow + at]) = *reinterpret_cast<uint4*>(&wl[1][wr * kRow + at]) = z4;
     }
   }
+  fetch(0);
+  uint4 X[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) X[s] = 16 * s < a.K ? ld16(a.x + first * a.K + (uint32_t)(row * a.K + 16 * s + 8 * h)) : z4;
+  put(0);
+  __syncthreads();
   uint16_t* st = staged[wave];
-  fetch(chunk);
-  int b = 0;
-  for (int rest = count; rest > 0; ++tile) {
-    const int64_t p0 = tile * kGlRows + wave * 32;
-    const int64_t first = p0 < a.P ? p0 : a.P - 1;      // rows past the end repeat the last one and are not stored
-    const int left = a.P - first < 32 ? (int)(a.P - first) : 32, stored = p0 < a.P ? left : 0;
-    const int row = r < left ? r : left - 1;
-    uint4 X[KS];
+  for (int c = 0; c < chunks; ++c) {
+    const bool more = c + 1 < chunks;
+    if (more) fetch(c + 1);
+    f32x16_t acc;
+    const uint16_t* wrow = &wl[c & 1][r * kRow + 8 * h];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) X[s] = 16 * s < a.K ? ld16(a.x + first * a.K + (uint32_t)(row * a.K + 16 * s + 8 * h)) : z4;
-    if (rest == count) { put(0); __syncthreads(); }
-    const int here = chunks - chunk < rest ? chunks - chunk : rest;
-    rest -= here;
-    for (int c = chunk; c < chunk + here; ++c, b ^= 1) {
-      const bool more = c + 1 < chunk + here || rest > 0;
-      uint16_t* y = a.y + first * a.N + 32 * c;
-      if (more) fetch(c + 1 < chunks ? c + 1 : 0);
-      f32x16_t acc;
-      const uint16_t* wrow = &wl[b][r * kRow + 8 * h];
+    for (int g = 0; g < 4; ++g) {
+      const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(&bl[c & 1][8 * g + 4 * h]);
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(&bl[b][8 * g + 4 * h]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[4 * g + i] = b4[i];
-      }
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, ld16(wrow + 16 * s)), __builtin_bit_cast(bf16x8_t, X[s]), acc, 0, 0, 0);
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {      // the lane's outputs 8 g + 4 h .. + 3
-        // the stock layer stores its output before the activation reads it: the same rounding here
-        const uint32_t q0 = pack_bf16(acc[4 * g], acc[4 * g + 1]), q1 = pack_bf16(acc[4 * g + 2], acc[4 * g + 3]);
-        *reinterpret_cast<uint2*>(st + r * kGlStage + 8 * g + 4 * h) =
-            make_uint2(pack_bf16(gelu_exact(bf_lo(q0)), gelu_exact(bf_hi(q0))), pack_bf16(gelu_exact(bf_lo(q1)), gelu_exact(bf_hi(q1))));
-      }
-      if (more) put(b ^ 1);      // (its readers passed the barrier at the end of the last chunk)
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int m = (l >> 2) + 16 * k, c8 = 8 * (l & 3);
-        if (m < stored) *reinterpret_cast<uint4*>(y + (int64_t)16 * k * a.N + (uint32_t)((l >> 2) * a.N + c8)) = ld16(st + m * kGlStage + c8);
-      }
-      __syncthreads();
+      for (int i = 0; i < 4; ++i) acc[4 * g + i] = b4[i];
     }
-    chunk = 0;
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, ld16(wrow + 16 * s)), __builtin_bit_cast(bf16x8_t, X[s]), acc, 0, 0, 0);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {      // the lane's outputs 8 g + 4 h .. + 3
+      // the stock layer stores its output before the activation reads it: the same rounding here
+      const uint32_t q0 = pack_bf16(acc[4 * g], acc[4 * g + 1]), q1 = pack_bf16(acc[4 * g + 2], acc[4 * g + 3]);
+      *reinterpret_cast<uint2*>(st + r * kGlStage + 8 * g + 4 * h) =
+          make_uint2(pack_bf16(gelu_exact(bf_lo(q0)), gelu_exact(bf_hi(q0))), pack_bf16(gelu_exact(bf_lo(q1)), gelu_exact(bf_hi(q1))));
+    }
+    if (more) put((c + 1) & 1);      // (its readers passed the barrier at the end of the last chunk)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int m = (l >> 2) + 16 * k, c8 = 8 * (l & 3);
+      if (m < stored) *reinterpret_cast<uint4*>(y + (int64_t)16 * k * a.N + 32 * c + (uint32_t)((l >> 2) * a.N + c8)) = ld16(st + m * kGlStage + c8);
+    }
+    __syncthreads();
   }
 }
 
@@ -1461,17 +1458,24 @@ int m2d_wide_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x
   if (weight_dtype != M2D_F32 && weight_dtype != M2D_BF16) return M2D_ERR_UNSUPPORTED;
   if (K % 32 != 0 || N % 32 != 0 || P > ((int64_t)1 << 20) || (post_act != kActNone && post_act != kActGelu)) return M2D_ERR_UNSUPPORTED;
   if (misaligned(x, 16) || misaligned(weight, 16) || misaligned(y, 16) || misaligned(bias, 16)) return M2D_ERR_MISALIGNED;
-  if (post_act == kActGelu && weight_dtype == M2D_BF16 && P > kGlFewest && K <= kGlInputs && N % 64 == 0 && (P + kGlRows - 1) / kGlRows * (N / 32) < ((int64_t)1 << 31)) {
+  if (post_act == kActGelu && weight_dtype == M2D_BF16 && P > kGlFewest && K <= kGlInputs && N % 64 == 0) {
     GeluLinArgs a = {static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(weight), static_cast<const uint16_t*>(bias),
-                     static_cast<uint16_t*>(y), P, K, N, 0, 0, 0};
+                     static_cast<uint16_t*>(y), P, K, N, 1, 0, 0, 0};
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int64_t tiles = (P + kGlRows - 1) / kGlRows;
-    // as many workgroups as the chip holds, with equal shares of the units, of two at least (a tile has an even number)
-    a.units = (int)(tiles * (N / 32));
-    const int pairs = (a.units / 2 + 7) / 8 * 8, wgs = pairs < kGlWant ? pairs : kGlWant;
-    a.share = pairs <= kGlWant ? 2 : a.units / wgs;
-    a.over = pairs <= kGlWant ? 0 : a.units % wgs;
-    const dim3 g((unsigned)wgs), t(kGlThreads);
+    // Slices of whole 64-output steps.  A compute unit is done when the one with the most workgroups is: an eighth of them goes to
+    // each XCD, to its 32 units evenly, and one workgroup on a unit takes as long as two (chains of loads and products).  A workgroup's
+    // start is worth half a unit of 32 outputs.  Of all numbers of slices, measured for 116 sizes (513 to 150000 positions, 128 to 1280
+    // outputs, 64 to 320 inputs), the one chosen takes 1.002 of the fastest's time, 1.07 at most; the fewest with 768 workgroups up to 1.34.
+    int64_t least = 0;
+    for (int d = 1; d <= N / 64 && (d == 1 || tiles * d <= kGlMost); ++d) {
+      const int64_t on_unit = ((tiles * d + 7) / 8 + 31) / 32, cost = (on_unit < 2 ? 2 : on_unit) * (4 * ((N / 64 + d - 1) / d) + 1);
+      if (d == 1 || cost < least) { least = cost; a.nsplit = d; }
+    }
+    a.steps = N / 64 / a.nsplit;
+    a.over = N / 64 % a.nsplit;
+    a.per_slice = a.nsplit == 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + a.nsplit - 1) / a.nsplit);
+    const dim3 g((unsigned)((tiles * a.nsplit + 7) / 8 * 8)), t(kGlThreads);
     if (K <= 256) hipLaunchKernelGGL(m2d_gelu_linear_kernel<16>, g, t, 0, st, a);
     else hipLaunchKernelGGL(m2d_gelu_linear_kernel<20>, g, t, 0, st, a);
     return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;

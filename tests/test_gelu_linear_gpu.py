@@ -43,6 +43,12 @@ def test_infinite_and_undefined_values_pass_through():
 
 @pytest.mark.parametrize("case", [(150001, 64, 64, True), (98304, 32, 128, False), (98305, 288, 64, True), (49152, 320, 128, True)],
                          ids=lambda c: "x".join(map(str, c)))
-def test_ranges_of_several_tiles(case):
-    """Few outputs and many positions: a workgroup's range of units takes it through several tiles, also where the units go out evenly."""
+def test_more_tiles_than_fit(case):
+    """Few outputs and many positions: more tiles than the device holds workgroups, in one slice and in two."""
+    test_against_float64(case)
+
+
+@pytest.mark.parametrize("case", [(19700, 96, 320, True), (31999, 320, 448, True), (12700, 288, 576, False)], ids=lambda c: "x".join(map(str, c)))
+def test_slices_of_unequal_length(case):
+    """5, 7 and 9 steps of 64 outputs in 3, 2 and 5 slices, with tiles whose slices are on two XCDs."""
     test_against_float64(case)
