@@ -69,3 +69,40 @@ def test_both_gradients(shape, acts):
             want = torch.stack([(back * t * t).sum(), back.sum()])
             terms = torch.stack([(mag * t * t).sum(), mag.sum()])
             assert ((star[:slices].double().sum(0) - want).abs() <= (N + 64) * 2.0 ** -24 * terms + 1e-5).all()
+
+
+@pytest.mark.parametrize("acts", [(NONE, NONE), (NONE, GELU), (GELU, NONE), (NONE, STAR)], ids=["plain", "gelu_before", "gelu_behind", "star_before"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"{s[0]}x{s[1]}")
+def test_every_tile_counts(shape, acts):
+    """Workgroups that take two and three tiles, the last of them of 7 rows, so that both buffers are filled again.  Operands are -1, 0 and 1,
+    and an activation or slope of those is a bf16 value that is a multiple of 2^-11 and no larger than 1.1: every product is a multiple of
+    2^-11, every sum stays below 2^13, and so fp32 holds them exactly in any order.  A lost, doubled or overwritten row would show."""
+    from mamba2d_amd import cabi
+    N, K, T = shape
+    post, pre = acts
+    P = 513 * T + 7
+    print(f"\ncase every tile {shape} {acts} P={P}", flush=True)
+    g = torch.Generator().manual_seed(K + N)
+    r = lambda *s: torch.randint(-1, 2, s, generator=g).bfloat16()
+    dy, z, x, w = r(P, N), r(P, N), r(P, K), r(N, K).float()
+    scale, shift = torch.tensor([0.5]), torch.tensor([-0.25])
+    dev = [t.cuda() for t in (dy, z, x, w, scale, shift)]
+    slices = cabi.lib.m2d_train_linear_grads_parts(ctypes.c_int64(P), N, K)
+    dx = torch.empty(P, K, dtype=torch.bfloat16, device="cuda")
+    part, star = torch.empty(slices, N * K + N, device="cuda"), torch.empty(slices, 2, device="cuda")
+    ptr, null = cabi._ptr, cabi._ptr(None)
+    cabi.check(cabi.lib.m2d_train_linear_grads(ctypes.c_int64(P), N, K, ptr(dev[0]), ptr(dev[1]) if post else null, post, ptr(dev[3]), ptr(dev[2]), pre,
+                                               ptr(dev[4]), ptr(dev[5]), 1, ptr(dx), ptr(part), ptr(star), cabi._stream(dx.device)))
+    part, star, dx = part.double().sum(0).cpu(), star.double().sum(0).cpu(), dx.cpu()
+    go, xd = dy.double(), x.double()
+    if post:
+        go = (go * gelu_slope(z.double())).bfloat16().double()
+    t = xd.clamp(min=0)
+    xa = gelu(xd).bfloat16().double() if pre == GELU else 0.5 * t * t - 0.25 if pre == STAR else xd
+    back = go @ w.double()
+    assert torch.equal(part[:N * K].view(N, K), go.T @ xa)
+    assert torch.equal(part[N * K:], go.sum(0))
+    if pre == STAR:
+        assert torch.equal(star, torch.stack([(back * t * t).sum(), back.sum()]))
+    if pre != GELU:      # (its slope is no bf16 value)
+        assert torch.equal(dx, (back * t if pre == STAR else back).bfloat16())
