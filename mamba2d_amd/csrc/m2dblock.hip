@@ -1465,12 +1465,14 @@ int m2d_wide_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x
     const int64_t tiles = (P + kGlRows - 1) / kGlRows;
     // Slices of whole 64-output steps.  A compute unit is done when the one with the most workgroups is: an eighth of them goes to
     // each XCD, to its 32 units evenly, and one workgroup on a unit takes as long as two (chains of loads and products).  A workgroup's
-    // start is worth half a unit of 32 outputs.  Of all numbers of slices, measured for 116 sizes (513 to 150000 positions, 128 to 1280
-    // outputs, 64 to 320 inputs), the one chosen takes 1.002 of the fastest's time, 1.07 at most; the fewest with 768 workgroups up to 1.34.
+    // start is worth half a unit of 32 outputs.  More slices have to save a twenty-fifth: where they come out about even, fewer are faster, as outputs
+    // beyond the last-level cache then leave in longer rows (150000 positions, 320 -> 1024: 1 slice 181 us, 4 slices 212, which cost 1 in 160
+    // less by this rule).  Of all numbers of slices, measured for 392 sizes (600 to 250000 positions, 64 to 1280 outputs, 64 to 320 inputs),
+    // the one chosen takes 1.005 of the fastest's time, 1.16 at most (100000 positions, 320 -> 448); the fewest with 768 workgroups 1.04 of the chosen one's.
     int64_t least = 0;
     for (int d = 1; d <= N / 64 && (d == 1 || tiles * d <= kGlMost); ++d) {
       const int64_t on_unit = ((tiles * d + 7) / 8 + 31) / 32, cost = (on_unit < 2 ? 2 : on_unit) * (4 * ((N / 64 + d - 1) / d) + 1);
-      if (d == 1 || cost < least) { least = cost; a.nsplit = d; }
+      if (d == 1 || 25 * cost < 24 * least) { least = cost; a.nsplit = d; }
     }
     a.steps = N / 64 / a.nsplit;
     a.over = N / 64 % a.nsplit;
