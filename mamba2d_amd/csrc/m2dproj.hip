@@ -309,6 +309,7 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_fwd_mfma_kern
 // the copying in of the weights and the softplus.
 constexpr int kFlD = 40;      // bf16 per row of the step sizes' weights in LDS: 32 + 8
 constexpr int kFlMaxE = 256, kFlMaxR = 16;
+constexpr int kUnits = 256;   // compute units of an MI355X
 constexpr size_t fl_lds_bytes(int Epad, int NL) { return ((size_t)(16 * NL + 3 * kN) * (Epad + 8) + 2 * (size_t)Epad * kFlD) * 2 + 2 * (size_t)Epad * 4; }
 __device__ __forceinline__ f32x4 load_f4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
@@ -643,7 +644,8 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_bwd_data_mfma
   }
 }
 
-// Backward, data, for up to 256 channels and a rank of up to 16; the kernel above has the wider ones, whose weights fill the LDS.  It moves what it must (64x56x56x64 with
+// Backward, data, for up to 256 channels and a rank of up to 16; the kernel above has the wider ones, whose weights fill the LDS, and many positions of the
+// widest of these (proj_bwd_in_lds).  It moves what it must (64x56x56x64 with
 // 4 parts of channel sums: 283 MB), and what it lost were waits: for the packing launch before it, for weight tiles that each wave fetched from the caches,
 // and for dx, asked for at the end.  Here a workgroup rounds the weights into LDS from the caller's tensors, and everything is asked for before the first
 // wait, dx too where registers allow four workgroups a compute unit (up to 64 channels; with 128 three fitted, and 784 tiles of 64x28x28x128 took a second
@@ -1569,8 +1571,16 @@ int run_proj_fwd_mfma(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) 
   return launched() ? M2D_OK : M2D_ERR_HIP;
 }
 
-// The weights in LDS, straight from the caller's tensors: see the kernel.
+// The weights in LDS, straight from the caller's tensors: see the kernels.
 bool proj_in_lds(const ProjGeometry& g) { return g.mfma && g.E <= kFlMaxE && g.R <= kFlMaxR; }
+// In the backward a workgroup of 64 positions fills the LDS for itself, so two have to share a compute unit, one filling while the other
+// multiplies, unless one round of workgroups does it.  More than 224 channels with a rank above 8 (84 KB) are alone: projections' backward at
+// 16384 positions of 256 channels, packed weights against LDS, 47.6 and 41.9 us, but at 16500 53.6 and 59.4, at 50176 101 and 117; 240 channels,
+// rank 13, 400000 positions 753 and 810.  With a rank of 8 (63 KB) the LDS stays ahead: 400000 of 256 channels 679 and 623 us.
+size_t bwd_lds_bytes(int Epad, int Opad32) { return ((size_t)32 * (Epad + 8) + (size_t)(Epad + 16 * kWaves) * (Opad32 + 8)) * 2; }
+bool proj_bwd_in_lds(const ProjGeometry& g) {
+  return proj_in_lds(g) && (2 * bwd_lds_bytes((g.E + 31) / 32 * 32, g.Opad32) <= 160 * 1024 || g.ntiles <= kUnits);
+}
 // More dynamic LDS than 64 KB has to be allowed, once per kernel and device.
 template <auto Kernel>
 bool allow_lds(size_t bytes) {
@@ -1589,7 +1599,7 @@ int launch_proj_fwd_lds(const ProjGeometry& g, const ProjArgs& a, hipStream_t st
   if (lds > 64 * 1024 && !allow_lds<&m2d_proj_fwd_lds_kernel<KS, NL, PACKED>>(fl_lds_bytes(kFlMaxE, NL))) return M2D_ERR_HIP;
   const int64_t tiles = (g.P + kTP - 1) / kTP;
   constexpr size_t most = KS == 2 ? 6 : (KS == 4 ? 4 : 2);   // workgroups whose registers fit a compute unit
-  int64_t grid = 256 * (int64_t)((160 * 1024) / lds < most ? (160 * 1024) / lds : most);   // as many as the device holds
+  int64_t grid = kUnits * (int64_t)((160 * 1024) / lds < most ? (160 * 1024) / lds : most);   // as many as the device holds
   if (grid > tiles) grid = tiles;
   hipLaunchKernelGGL((m2d_proj_fwd_lds_kernel<KS, NL, PACKED>), dim3((unsigned)grid), dim3(kThreads), lds, st, a);
   return launched() ? M2D_OK : M2D_ERR_HIP;
@@ -1632,15 +1642,14 @@ int run_reduce(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
 
 template <int KS>
 int launch_proj_bwd_lds(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
-  auto bytes = [](int Epad, int Opad32) { return ((size_t)32 * (Epad + 8) + (size_t)(Epad + 16 * kWaves) * (Opad32 + 8)) * 2; };
-  const size_t lds = bytes((g.E + 31) / 32 * 32, g.Opad32), most = bytes(32 * KS, 96);
+  const size_t lds = bwd_lds_bytes((g.E + 31) / 32 * 32, g.Opad32), most = bwd_lds_bytes(32 * KS, 96);
   if (most > 64 * 1024 && !allow_lds<&m2d_proj_bwd_data_lds_kernel<KS>>(most)) return M2D_ERR_HIP;
   hipLaunchKernelGGL(m2d_proj_bwd_data_lds_kernel<KS>, dim3(g.ntiles), dim3(kThreads), lds, st, a);
   return launched() ? M2D_OK : M2D_ERR_HIP;
 }
 int run_proj_bwd_mfma(const ProjGeometry& g, const ProjArgs& a, hipStream_t st) {
   int rc;
-  if (proj_in_lds(g)) {
+  if (proj_bwd_in_lds(g)) {
     rc = g.E <= 64 ? launch_proj_bwd_lds<2>(g, a, st) : (g.E <= 128 ? launch_proj_bwd_lds<4>(g, a, st) : launch_proj_bwd_lds<8>(g, a, st));
   } else {
     const size_t lds_data = (size_t)kWaves * (16 * kStageStride * 4 + 16 * (g.Opad32 + 8) * 2);
@@ -1762,7 +1771,7 @@ int m2d_proj_bwd_parts(const m2d_desc* desc, int dt_rank, int sum_parts, const v
   char* ws = static_cast<char*>(workspace);
   PackArgs k = {};
   k.Wx = x_proj_w; k.wT = dt_projT_w; k.wL = dt_projL_w;
-  if (g.mfma && !proj_in_lds(g)) {   // for the data kernel; the weight-gradient kernel needs no weights
+  if (g.mfma && !proj_bwd_in_lds(g)) {   // for the data kernel; the weight-gradient kernel needs no weights
     k.wTtb = reinterpret_cast<uint16_t*>(ws + g.off_wTtb);
     k.wLtb = reinterpret_cast<uint16_t*>(ws + g.off_wLtb);
     k.WxTb = reinterpret_cast<uint16_t*>(ws + g.off_WxTb);

@@ -103,7 +103,9 @@ def test_values_that_are_not_finite_stay_in_their_position(cabi, E, R):
 
 # the same edges; channel sums of the scan in parts (0: whole arrays in bf16), whose loads go out in fours and a remainder
 BWD = [(1, 8, 1, 0), (15, 16, 1, 1), (17, 32, 2, 2), (63, 40, 3, 4), (64, 64, 4, 5), (65, 72, 5, 8), (130, 96, 6, 0), (127, 128, 8, 16),
-       (129, 136, 9, 3), (64, 160, 10, 0), (77, 200, 13, 7), (192, 248, 16, 4), (333, 256, 16, 9), (50, 64, 16, 0), (9000, 24, 2, 6)]
+       (129, 136, 9, 3), (64, 160, 10, 0), (77, 200, 13, 7), (192, 248, 16, 4), (333, 256, 16, 9), (50, 64, 16, 0), (9000, 24, 2, 6),
+       # either side of the line beyond which the widest layers go back to packed weights (256 tiles of 64 positions, where one workgroup fits a unit)
+       (16384, 232, 9, 2), (16385, 232, 9, 0), (16390, 256, 16, 3), (16390, 256, 8, 3)]
 
 
 @pytest.mark.parametrize("dpre", [False, True], ids=["d_delta", "dpre"])
