@@ -3145,10 +3145,15 @@ void fill_common(ScanParams& sp, const m2d_desc* d, const Geometry& g) {
 // units of an XCD, or bands of so many workgroups that it matters little, or workgroups go out in order (fp32, backward, in units of up to 8 against in order:
 // 5x37x45x100 82.7 and 71.7 us, 1x601x768x136 2.91 and 2.60 ms; 1x335x418x456 2.51 and 2.62, 1024x1024x64 3.01 and 3.33).  The forward of one image
 // is faster in units of 8 throughout (keeping snapshots, 1x601x768x136 1.10 and 1.13 ms, 1x892x601x88 1.04 and 1.10, 1x686x690x140 1.12 and 1.22), of several not (3x298x359x208 1.56 and 1.51).
-inline int linked_grid(ScanParams& sp, bool forward) {
+// A split forward on whole chunks whose band, of all images, is 4 or 8 workgroups has few lines to share, and in order its bands meet on the same XCDs, or on
+// every other one: in order it takes 0.98 of the time (39 problems, 0.94 to 1.03; keeping snapshots 1x148x228x32 bf16 132 and 122 us, 2x90x153x16 82.3 and 79.6,
+// 1x419x223x16 257 and 247).  1 or 2 workgroups: the same within 1 %; 3, 5, 6, 7: units by 2 %; rows of no whole chunks, fetched value by value: units, by up
+// to 14 % (1x520x600x14 bf16 482 and 541); the backward: no difference.
+inline int linked_grid(ScanParams& sp, bool forward, bool chunks) {
   const int lagged = (sp.sl_nbb + kLinkLag) / (kLinkLag + 1), under_way = lagged < sp.nbands ? lagged : sp.nbands;
   const bool wait = 8 * (int64_t)sp.B * sp.bpb * under_way > 7 * (int64_t)device_cus();
-  const int want = !wait || (forward && sp.B == 1) || sp.bpb >= 48 || sp.bpb % 8 == 0 ? 8 : sp.bpb % 4 == 0 ? 4 : sp.bpb % 2 == 0 ? 2 : 1;
+  const bool meet = forward && chunks && !wait && ((int64_t)sp.B * sp.bpb == 4 || (int64_t)sp.B * sp.bpb == 8);
+  const int want = meet ? 1 : !wait || (forward && sp.B == 1) || sp.bpb >= 48 || sp.bpb % 8 == 0 ? 8 : sp.bpb % 4 == 0 ? 4 : sp.bpb % 2 == 0 ? 2 : 1;
   sp.sl_units = (sp.bpb + want - 1) / want;
   sp.sl_unit = (sp.bpb + sp.sl_units - 1) / sp.sl_units;
   const int64_t units = (int64_t)sp.nbands * sp.B * sp.sl_units;
@@ -3330,7 +3335,7 @@ int launch_fwd(const ScanParams& sp0, const m2d_desc* d, const Geometry& g, bool
     return g.stage_x ? launch_fwd_mode<T, 1, true, kModeSweep>(sp, ckpt, write_y, st) : launch_fwd_mode<T, 1, false, kModeSweep>(sp, ckpt, write_y, st);
   };
   if (g.sliced) {   // every band on workgroups of its own, band 0 first: a band waits for the one before it
-    sp.nwg = linked_grid(sp, true);
+    sp.nwg = linked_grid(sp, true, g.fwd_split && g.stage_x);
     sp.prog = sp.link_err + 64;
   }
   return once();
@@ -3476,7 +3481,7 @@ int run_bwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
     else rc = g.stage_x ? launch_bwd<T, true, kModeSweep>(sp, st, g.bwd_nw, g.snap32) : launch_bwd<T, false, kModeSweep>(sp, st, g.bwd_nw, g.snap32);
   } else {
     // every band on workgroups of its own, the last band first: a band waits for the one below it
-    sp.nwg = linked_grid(sp, false);
+    sp.nwg = linked_grid(sp, false, g.stage_x);
     sp.prog = sp.link_err + 64 + (size_t)g.nbands * g.vB * (g.fwd_bpb > g.bwd_bpb ? g.fwd_bpb : g.bwd_bpb) * kLinkStride;
     if (g.bwd_split) rc = launch_bwd_split<T, kModeSliced>(sp, g.stage_x, st, g.bwd_nw);
     else rc = g.stage_x ? launch_bwd<T, true, kModeSliced>(sp, st, g.bwd_nw, g.snap32) : launch_bwd<T, false, kModeSliced>(sp, st, g.bwd_nw, g.snap32);
