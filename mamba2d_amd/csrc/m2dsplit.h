@@ -274,9 +274,11 @@ __device__ __forceinline__ void split_x_copy(const ScanParams& p, const char* im
     split_fill16<false>(ok && ch < p.E ? img + off : reinterpret_cast<const char*>(p.zeros), tensor + c * SG::kSet);
   }
 }
-// ... and where they are not: value by value, through registers, by wave sw for its channels sw, sw + 4 of the workgroup
+// ... and where they are not: value by value, through registers, by wave sw for its channels sw, sw + 4 of the workgroup.  The registers take the values as
+// they are in memory, and 16-bit ones are widened when they are put in place, a block later: widened where they are fetched, a wave waited there for its loads
+// and for every store before them (bf16, forward keeping snapshots / backward: 3x64x90x292 156 / 420 -> 125 / 363 us, 2x100x26x100 72 / 167 -> 61 / 144).
 template <typename T, int NT, int CW>
-struct SplitVals { float v[CW / kSplitStagers][NT]; };
+struct SplitVals { T v[CW / kSplitStagers][NT]; };
 template <typename T, int NT, int CW>
 __device__ __forceinline__ void split_vals_fetch(const ScanParams& p, const char* const (&img)[4], uint32_t cell, bool ok, int e_wg0, int sw, SplitVals<T, NT, CW>& o) {
 #pragma unroll
@@ -285,7 +287,7 @@ __device__ __forceinline__ void split_vals_fetch(const ScanParams& p, const char
     const uint32_t off = (cell * (uint32_t)p.E + (uint32_t)e) * (uint32_t)sizeof(T);
     const bool live = ok && e < p.E;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) o.v[j][t] = live ? IO<T>::ld(reinterpret_cast<const T*>(img[t] + off)) : 0.f;
+    for (int t = 0; t < NT; ++t) o.v[j][t] = live ? *reinterpret_cast<const T*>(img[t] + off) : T{};
   }
 }
 template <typename T, int NT, int CW, typename SG>
@@ -294,7 +296,7 @@ __device__ __forceinline__ void split_vals_put(const SplitVals<T, NT, CW>& o, ch
   for (int j = 0; j < CW / kSplitStagers; ++j)
 #pragma unroll
     for (int t = 0; t < NT; ++t)
-      *reinterpret_cast<float*>(buf + SG::kX + t * SG::kXTensor + ((sw + kSplitStagers * j) * kCK * kHB + lane) * 4) = o.v[j][t];
+      *reinterpret_cast<float*>(buf + SG::kX + t * SG::kXTensor + ((sw + kSplitStagers * j) * kCK * kHB + lane) * 4) = IO<T>::ld(&o.v[j][t]);
 }
 
 // ---------------------------------------------------------------------------------------- forward
