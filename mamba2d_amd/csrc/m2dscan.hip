@@ -3149,11 +3149,17 @@ void fill_common(ScanParams& sp, const m2d_desc* d, const Geometry& g) {
 // every other one: in order it takes 0.98 of the time (39 problems, 0.94 to 1.03; keeping snapshots 1x148x228x32 bf16 132 and 122 us, 2x90x153x16 82.3 and 79.6,
 // 1x419x223x16 257 and 247).  1 or 2 workgroups: the same within 1 %; 3, 5, 6, 7: units by 2 %; rows of no whole chunks, fetched value by value: units, by up
 // to 14 % (1x520x600x14 bf16 482 and 541); the backward: no difference.
-inline int linked_grid(ScanParams& sp, bool forward, bool chunks) {
+// 16-bit tensors whose bands have 48 workgroups or more (the forward of one image: 32) and have to wait: units of 2, by
+// measurement (why 16-bit tensors alone is not known; a line holds twice as many of their channels).  Against in order, units of 8 and of 2, both passes: 40 problems
+// of 48 and more, mean 1.00 and 0.99, ten and three of them slower by more than 3 %, most 1.14 and 1.13 (2x97x111x424, forward, 146 us in order, 166 and 145; backward
+// 442, 490 and 436); forward of one image with 32 to 47, 28 problems: 0.99 and 0.98, five and none (1x392x432x288 1.03 and 0.92).  fp32 keeps 8 (25 and 6
+// problems: 0.97 and 0.90, units of 2 0.97 and 0.94).
+inline int linked_grid(ScanParams& sp, bool forward, bool chunks, bool half) {
   const int lagged = (sp.sl_nbb + kLinkLag) / (kLinkLag + 1), under_way = lagged < sp.nbands ? lagged : sp.nbands;
   const bool wait = 8 * (int64_t)sp.B * sp.bpb * under_way > 7 * (int64_t)device_cus();
   const bool meet = forward && chunks && !wait && ((int64_t)sp.B * sp.bpb == 4 || (int64_t)sp.B * sp.bpb == 8);
-  const int want = meet ? 1 : !wait || (forward && sp.B == 1) || sp.bpb >= 48 || sp.bpb % 8 == 0 ? 8 : sp.bpb % 4 == 0 ? 4 : sp.bpb % 2 == 0 ? 2 : 1;
+  const bool wide = half && wait && sp.bpb >= (forward && sp.B == 1 ? 32 : 48);
+  const int want = meet ? 1 : wide ? 2 : !wait || (forward && sp.B == 1) || sp.bpb >= 48 || sp.bpb % 8 == 0 ? 8 : sp.bpb % 4 == 0 ? 4 : sp.bpb % 2 == 0 ? 2 : 1;
   sp.sl_units = (sp.bpb + want - 1) / want;
   sp.sl_unit = (sp.bpb + sp.sl_units - 1) / sp.sl_units;
   const int64_t units = (int64_t)sp.nbands * sp.B * sp.sl_units;
@@ -3335,7 +3341,7 @@ int launch_fwd(const ScanParams& sp0, const m2d_desc* d, const Geometry& g, bool
     return g.stage_x ? launch_fwd_mode<T, 1, true, kModeSweep>(sp, ckpt, write_y, st) : launch_fwd_mode<T, 1, false, kModeSweep>(sp, ckpt, write_y, st);
   };
   if (g.sliced) {   // every band on workgroups of its own, band 0 first: a band waits for the one before it
-    sp.nwg = linked_grid(sp, true, g.fwd_split && g.stage_x);
+    sp.nwg = linked_grid(sp, true, g.fwd_split && g.stage_x, d->dtype == M2D_BF16);
     sp.prog = sp.link_err + 64;
   }
   return once();
@@ -3481,7 +3487,7 @@ int run_bwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
     else rc = g.stage_x ? launch_bwd<T, true, kModeSweep>(sp, st, g.bwd_nw, g.snap32) : launch_bwd<T, false, kModeSweep>(sp, st, g.bwd_nw, g.snap32);
   } else {
     // every band on workgroups of its own, the last band first: a band waits for the one below it
-    sp.nwg = linked_grid(sp, false, g.stage_x);
+    sp.nwg = linked_grid(sp, false, g.stage_x, d->dtype == M2D_BF16);
     sp.prog = sp.link_err + 64 + (size_t)g.nbands * g.vB * (g.fwd_bpb > g.bwd_bpb ? g.fwd_bpb : g.bwd_bpb) * kLinkStride;
     if (g.bwd_split) rc = launch_bwd_split<T, kModeSliced>(sp, g.stage_x, st, g.bwd_nw);
     else rc = g.stage_x ? launch_bwd<T, true, kModeSliced>(sp, st, g.bwd_nw, g.snap32) : launch_bwd<T, false, kModeSliced>(sp, st, g.bwd_nw, g.snap32);
