@@ -302,7 +302,8 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_fwd_mfma_kern
 // neighbouring outputs of its position and stores them from registers: 4 of a record of B_T, B_L, C, whose rows are listed in the records' order, and 8
 // step sizes, for which a pair of tiles lists its rows as 8 (m >> 2) + 4 t + (m & 3).  The low-rank inputs of the step sizes stay in the registers
 // that they were made in: the second product lists its contraction in their order, and those of the other step size are masked out, so that
-// an infinite value of one does not meet the other's zero weights.  Against the kernel above
+// an infinite value of one does not meet the other's zero weights.  With a rank above 4 a step size's fp32 sum is thereby formed in another order than in
+// the kernel above, of the same operands: it may round to the neighbouring bf16 value.  Against the kernel above
 // and its packing launch, ten calls in a row: 64x56x56x64 43.1 -> 24.7 us (104 MB, 4.2 TB/s), 4x128x128x64 19.6 -> 11.8, 64x28x28x128 28.2 -> 18.4,
 // 64x14x14x256 27.0 -> 18.6, 200000 positions of 32 channels 39.2 -> 16.6, 4096 of 64 11.1 -> 5.2; no size measured was slower.  A thread's share of the
 // weights is asked for at once: with loops that waited for each load they were 28.8, 13.4, 22.7, 24.4, 18.3 and 7.2.  What is left at 64 channels is
@@ -647,9 +648,11 @@ __global__ __launch_bounds__(kThreads, M2D_PROJ_OCC) void m2d_proj_bwd_data_mfma
 // Backward, data, for up to 256 channels and a rank of up to 16; the kernel above has the wider ones, whose weights fill the LDS, and many positions of the
 // widest of these (proj_bwd_in_lds).  It moves what it must (64x56x56x64 with
 // 4 parts of channel sums: 283 MB), and what it lost were waits: for the packing launch before it, for weight tiles that each wave fetched from the caches,
-// and for dx, asked for at the end.  Here a workgroup rounds the weights into LDS from the caller's tensors, and everything is asked for before the first
-// wait, dx too where registers allow four workgroups a compute unit (up to 64 channels; with 128 three fitted, and 784 tiles of 64x28x28x128 took a second
-// generation for the last 16: whole backward 56.5 us against 50.3 without).  The weights' rows are the first operands, so dx leaves from registers, 16 bytes a lane.
+// and for dx, asked for at the end.  Here a workgroup rounds the weights into LDS from the caller's tensors, and most of what it reads is asked for before the
+// first wait: the step sizes' weights, their gradients, three pieces of x_proj a thread (two outputs of four channels
+// each: all of it up to 64 channels; of the 4 pieces at 128 channels and the 12 at 256 with a rank of 16 the rest are fetched one by one), and dx where registers allow four workgroups a compute unit (up to 64 channels; with 128
+// three fitted, and 784 tiles of 64x28x28x128 took a second generation for the last 16: whole backward 56.5 us against 50.3 without).  The channel sums
+// follow when the weights are in place, and without dpre the step sizes are fetched where they are used.  The weights' rows are the first operands, so dx leaves from registers, 16 bytes a lane.
 // Backward of the projections in all, ten calls in a row: 64x56x56x64, 4 parts 91.5 -> 77.6 us, 64x28x28x128, 8 parts 57.7 -> 48.0, 4x128x128x64, 8 parts 47.2 ->
 // 40.8, 64x14x14x256, 16 parts 46.7 -> 39.8, 200000 positions of 32 channels 68.8 -> 51.9, 1568 of 64 17.4 -> 13.9 (with the step sizes' weights in a loop that
 // waited for each load 81.9, 50.3, 42.3, 43.1, 53.7 and 14.9); bit for bit the same results.
@@ -668,7 +671,7 @@ __global__ __launch_bounds__(kThreads, KS <= 4 ? 4 : 2) void m2d_proj_bwd_data_l
   const int64_t off = (p0 + mn < a.P ? p0 + mn : a.P - 1) * E;   // rows past the end repeat the last one: masked, not stored
   const uint4 z4 = make_uint4(0, 0, 0, 0);
 
-  // the weights first, then everything else that memory is asked for: all of it is under way before the first wait
+  // the weights first, then the gradients and dx, all under way before the first wait
   constexpr int kHold = 3;   // pairs of outputs x 4 channels of a thread
   f32x4 hw0[kHold], hw1[kHold];
   const int nwx = (a.Opad32 / 2) * (Epad / 4);

@@ -2952,11 +2952,13 @@ Geometry make_geometry(const m2d_desc* d) {
   // fifth (where units have more than one workgroup to sweep).
   // The constants are ratios: a block of forward keeping snapshots and backward, a workgroup of 4 waves with a quarter of the states each as 100
   // (1000 problems of both types: 8 such waves 150; whole states in workgroups of 8 waves 437, of 16 channels 303 linked and 216 in one stream; where
-  // rows are no whole chunks all of them take longer, the last 310).  In the linked sweep whole states in workgroups of 8 waves have fallen behind by more: as
-  // 417 the split states, where they ran, took 0.80 of what the ratios said (median of 14 problems, 0.74 to 0.88; 16x138x162x104 bf16 1.91 of 2.41 ms, 3x132x170x488 1.79 of 2.11).  Near the line the whole states stay: fewer channel sums, snapshots every 2
+  // rows are no whole chunks all of them take longer, the last 310; all taken before the stores of sums and results became wider, since when the split
+  // backward is 10 to 25 % faster and the one of whole states 6 %: split states would win a little more often than this gives them).  In the linked sweep whole states in workgroups of 8 waves have fallen behind by more: as
+  // 417 the split states, where they ran, took 0.80 of what the ratios said (median of 14 problems, 0.74 to 0.88; 16x138x162x104 bf16 1.91 of 2.41 ms, 3x132x170x488 1.79 of 2.11; the 21 of 5998 drawn problems that change
+  // plan by it take 0.71 to 0.90 of the time).  Near the line the whole states stay: fewer channel sums, snapshots every 2
   // steps.  Both sides, kernels of both passes in ms, whole states against split: 30x60x50x40 fp32 0.522 and 0.324, 8x256x256x64 bf16 3.16 and 2.10,
   // 20x28x28x200 fp32 0.289 and 0.202, 32x128x128x64 bf16 2.02 and 1.64; on the other side of the line 64x28x28x128 bf16 0.280 and 0.391.
-  // Of 708 problems drawn over all sizes the chosen plans take 1.023 of the time of each one's best; farthest off, 1.3 to 1.5, are widths of no whole
+  // Of 708 problems drawn over all sizes the chosen plans took, with those kernels, 1.023 of the time of each one's best; farthest off, 1.3 to 1.5, are widths of no whole
   // chunks and one to three channels, and grids two to four columns wide, where whole states would be up to 1.09 ahead of the linked sweep.
   constexpr int64_t kSplit4 = 100, kSplit8 = 147, kWhole4 = 235, kWhole4Linked = 300, kWhole8 = 417, kWhole8Linked = 480;
   auto stream_cost = [&](int64_t wgs, int64_t block) { return (wgs + ncu - 1) / ncu * nblk_stream * block; };
@@ -2997,7 +2999,8 @@ Geometry make_geometry(const m2d_desc* d) {
   // Where the channel sums of the split backward would pass their bound, the backward is the one of whole states in the forward's schedule, and what
   // suits a pair of split kernels may not suit this pair: 5x1362x43x319 fp32, forward + backward kernels, took 11.6 ms linked with whole states
   // and 16.6 with a split forward in one stream per image.  So there the two passes that will run are priced, each by what its own block takes, in
-  // units of 10 ns: medians over 1000 problems drawn over all sizes and both types, each in every plan it can have; rows of whole 16-byte chunks, and others.
+  // units of 10 ns: medians over 1000 problems drawn over all sizes and both types, each in every plan it can have; rows of whole 16-byte chunks, and others; of the kernels
+  // before the wider stores, too.
   // Of 1000 problems 93 get another plan by it (nearly all of more than 2^26 values): forward + backward kernels 0.82 of the time, the worst 1.12.
   struct Block { int64_t fwd[2], bwd[2]; };
   constexpr Block kBlock4 = {{89, 114}, {237, 260}}, kBlock4Linked = {{90, 110}, {245, 280}}, kBlock8 = {{128, 162}, {362, 420}}, kBlock8Linked = {{138, 164}, {386, 447}};

@@ -735,7 +735,7 @@ __global__ __launch_bounds__(256, 2) void m2d_train_wgrad_kernel(const WgradArgs
 // taken from registers and 16 bytes are stored, 64 of a row.  One barrier a tile (two buffers); the next tile's loads are under way meanwhile.
 // One workgroup to a unit: each leaves N K sums.  200704 positions, both kernels above -> this one: 64 -> 64 with the GELU
 // before it 42 -> 28 us, 256 -> 64 with it 124 -> 87 (the GELU and its slope at 51 million values: 42 at the rate of the vector ALUs), 64 -> 256 59 -> 36, 128 -> 64 with a StarReLU 52 -> 41.
-constexpr int kGrThreads = 512, kGrMost = 256;      // workgroups at most
+constexpr int kGrThreads = 512, kGrMost = 256;      // workgroups at most: the compute units of an MI355X
 template <int N, int K, int PT>
 struct GradsPlan {
   static constexpr int WK = K / 32, WN = 8 / WK, T = 16 * WN * PT;      // waves along the inputs, and beside each other; positions of a tile
@@ -1046,7 +1046,9 @@ inline int wgrad_shares(int64_t P, int N, int K) {
 }
 
 // The layers whose two gradients come from one kernel: those of a block of 64 channels, and of 128 but for its MLP.  (Outputs, inputs, tiles of 16 positions of
-// a wave: as many as two buffers of them fit the LDS, up to 128 positions in all.)
+// a wave: as many as two buffers of them fit the LDS, up to 128 positions in all.)  At any number of positions: with the adding up of what each leaves, all eight
+// at 196 to 200704 positions take 0.49 to 0.98 of the two kernels' time, but for 128 -> 256 at 6272, where it is 25.2 us either way (14x14 cells: 8.8 us
+// against 16.9 for 64 -> 64, 11.1 against 17.8 for 256 -> 128).  What grows is the memory of the sums: 256 sets beside 64 at 256 x 128, 34 MB.
 #define M2D_GRADS_SHAPES(X) X(64, 64, 2) X(64, 256, 4) X(256, 64, 1) X(64, 128, 4) X(128, 64, 2) X(128, 128, 2) X(128, 256, 2) X(256, 128, 1)
 template <int N, int K, int PT>
 int grads_parts(int64_t P) {
