@@ -34,6 +34,7 @@ HIPCC_FLAGS = [
 # kernels are memory-bound and do better with the default scheduler.
 SOURCES = {
     "m2dscan.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
+    "m2drows.hip": [],
     "m2dproj.hip": [],
     "m2dblock.hip": [],
     "m2dtrain.hip": [],

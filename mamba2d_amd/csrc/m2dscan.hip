@@ -42,6 +42,7 @@
 #include <type_traits>
 
 #include "../../include/m2dscan.h"
+#include "m2drows.h"
 
 // Scratch of m2d_scan_fwd_noalloc: the workspace of a forward call, for callers that cannot
 // allocate.  Every device that loads the library holds its own copy at its own address; host code
@@ -2773,6 +2774,7 @@ struct Geometry {
   int bwd_nw, bwd_wpb, bwd_bpb;      // backward: waves per workgroup, waves and workgroups (channel groups) per image
   bool fwd_split, bwd_split;         // the states of a channel split over the lanes (a wave per channel: m2d_fwd_split_kernel, m2d_bwd_split_kernel)
   ForwardKernel alone;               // the forward that keeps no snapshots (the same schedule and scratch; often the same kernel)
+  m2drows::Plan rows;                // ... or, where rows.rows > 0, m2d_fwd_rows_kernel (in the same scratch)
   bool stage_x;                      // x, delta, dy rows are whole 16-byte chunks: stage them through LDS
   bool sliced;                       // linked sweep: bands on workgroups of their own, handing boundary rows to each other inside one launch
   bool stacked;                      // images of one band stacked into tall images of independent bands
@@ -3079,6 +3081,20 @@ Geometry make_geometry(const m2d_desc* d) {
     if (!split || 100 * whole_cost_alone < 97 * split_cost_alone) g.alone = whole;
     if (sums_bound && 100 * split_cost_alone < (split ? 100 : 90) * whole_cost_alone) g.alone = {true, 1, nw, (d->E + nw - 1) / nw};
   }
+  // m2d_fwd_rows_kernel where it takes less time than that kernel: a sweeping wave of it needs 0.2 us a cell with bf16 tensors and 0.225 with fp32 ones
+  // (0.17 to 0.22 and 0.16 to 0.25 over 120 drawn problems; less where units are not full), a launch 3 us more; the kernels above are priced by their blocks, in the same
+  // units of 10 ns.  It has to promise 7 %.  Where a forward without snapshots has another kernel than one that keeps them anyhow, it stays with that.
+  g.rows = m2drows::Plan{};
+  const bool same = g.alone.split == g.fwd_split && g.alone.ec == g.fwd_ec && g.alone.nw == g.fwd_nw;
+  const m2drows::Plan by_rows = may_split && same && !(d->flags & (M2D_FLAG_SPLIT_STATES | M2D_FLAG_TEST_DEAD_LINK)) ? m2drows::make_plan(d->B, d->H, d->W, d->E, (int)ncu) : m2drows::Plan{};
+  int64_t rows_cost = 0, above_cost = 0;
+  if (by_rows.rows) {
+    rows_cost = by_rows.cells * (d->dtype == M2D_BF16 ? 40 : 45) / 2 + 300;
+    const int64_t wgs = (int64_t)B * g.alone.bpb;
+    if (g.alone.split && g.alone.ec == 2) above_cost = kBlockPairs * ((wgs + ncu - 1) / ncu) * (nblk_stream + 3);
+    else if (g.alone.split) above_cost = split_fwd_cost(g.alone.nw, g.sliced);
+    else above_cost = cost(g.sliced, wgs, g.alone.ec == 2 ? kBlockTwoChannels[ragged] : whole_block_of(g.alone.nw).fwd[ragged]);
+  }
   const size_t P = (size_t)d->B * d->H * d->W;
   g.prep_bytes = align_up(sizeof(float) * (kZeroFloats + (size_t)2 * d->E * kN + d->E));
   g.packed_bc = (d->flags & M2D_FLAG_PACKED_BC) != 0;   // the caller brings the records: nothing to reserve
@@ -3101,6 +3117,7 @@ Geometry make_geometry(const m2d_desc* d) {
   g.link_fwd_bytes = g.sliced ? align_up(sizeof(uint32_t) * (64 + (size_t)g.nbands * B * g.fwd_bpb * kLinkStride)) : 0;
   g.link_bytes = g.sliced ? align_up(sizeof(uint32_t) * (64 + 2 * g.nbands * chains * kLinkStride)) : 0;
   g.part_bytes = align_up(sizeof(float) * (size_t)g.bwd_bpb * 3 * P * kN);
+  if (by_rows.rows && 100 * rows_cost < 93 * above_cost && by_rows.wrap_bytes <= g.top_bytes + g.bc_bytes) g.rows = by_rows;
   const size_t slots = g.sliced ? g.nbands : 1;
   g.pa_bytes = align_up(sizeof(float) * (size_t)B * slots * d->E * 2 * kN);
   g.pd_bytes = align_up(sizeof(float) * (size_t)B * slots * d->E);
@@ -3382,6 +3399,20 @@ int run_fwd(const m2d_desc* d, const Geometry& g, ScanParams sp, const void* AT,
   return rc;
 }
 
+// The forward without snapshots where m2d_fwd_rows_kernel is the faster one: it sets itself up, and the rows that a workgroup hands to itself are where boundary rows would be
+int run_rows(const m2d_desc* d, const Geometry& g, const ScanParams& sp, const void* AT, const void* AL, const void* BT, const void* BL, const void* C, const void* D, void* ws, hipStream_t st) {
+  m2drows::Args a = {};
+  a.x = sp.x; a.dT = sp.dT; a.dL = sp.dL; a.AT = AT; a.AL = AL; a.D = D; a.y = sp.y;
+  if (g.packed_bc) a.rec = static_cast<const float*>(BT);
+  else { a.BT = BT; a.BL = BL; a.C = C; }
+  a.wrap = reinterpret_cast<float*>(static_cast<char*>(ws) + g.prep_bytes + g.link_fwd_bytes);
+  a.B = d->B; a.H = d->H; a.W = d->W; a.E = d->E; a.flip = sp.flip; a.raw = sp.raw;
+  if (g_profile) (void)hipEventRecord(g_ev[M2D_PASS_FWD][0], st);
+  const int err = m2drows::launch_fwd(g.rows, a, d->dtype == M2D_BF16, st);
+  if (g_profile) (void)hipEventRecord(g_ev[M2D_PASS_FWD][1], st);
+  return err == hipSuccess ? M2D_OK : M2D_ERR_HIP;
+}
+
 template <typename T, bool SX, int MODE, int NW, bool REPLAY = false, typename ST = T>
 int launch_bwd_as(const ScanParams& sp, hipStream_t st) {
   if constexpr (!M2D_BUILT(T, SX, MODE, NW, !REPLAY)) return M2D_ERR_UNSUPPORTED; else {
@@ -3579,6 +3610,7 @@ int m2d_scan_fwd(const m2d_desc* desc, const void* x, const void* deltaT, const 
   fill_common(sp, desc, g);
   sp.x = x; sp.dT = deltaT; sp.dL = deltaL; sp.y = y;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (!ckpt && g.rows.rows) return run_rows(desc, g, sp, AT, AL, BT, BL, C, D, workspace, st);
   return desc->dtype == M2D_F32 ? run_fwd<float>(desc, g, sp, AT, AL, BT, BL, C, D, ckpt, workspace, st)
                                 : run_fwd<bf16_t>(desc, g, sp, AT, AL, BT, BL, C, D, ckpt, workspace, st);
 }
@@ -3650,7 +3682,10 @@ int m2d_scan_plan(const m2d_desc* desc, int pass, char* text, size_t cap) {
     const size_t n = strlen(text);
     if (n + 1 < cap) snprintf(text + n, cap - n, fwd ? ", a snapshot every %d steps" : ", a snapshot every %d steps and the forward replayed in between", kCK << g.ck_shift);
   }
-  if (fwd && (g.alone.split != g.fwd_split || g.alone.ec != g.fwd_ec || g.alone.nw != g.fwd_nw)) {
+  if (fwd && g.rows.rows) {
+    const size_t n = strlen(text);
+    if (n + 1 < cap) snprintf(text + n, cap - n, "; without snapshots m2d_fwd_rows_kernel, %d workgroups of %d bands of %d rows and %d channels", g.rows.workgroups, g.rows.slots, g.rows.rows, 16 * (8 / g.rows.slots));
+  } else if (fwd && (g.alone.split != g.fwd_split || g.alone.ec != g.fwd_ec || g.alone.nw != g.fwd_nw)) {
     const size_t n = strlen(text);
     if (n + 1 < cap) snprintf(text + n, cap - n, "; without snapshots %s, %lld workgroups of %d channels", g.alone.split ? "m2d_fwd_split_kernel" : "m2d_fwd_kernel",
                               (long long)g.vB * g.alone.bpb, (g.alone.split ? 1 : g.CS) * g.alone.nw * g.alone.ec);

@@ -1,0 +1,102 @@
+"""m2d_fwd_rows_kernel (the forward without snapshots of batches that fill the device): every number of bands side by side and of rows a
+band, one round of bands and two (rows handed on through memory), odd widths, heights that end inside a band, channel groups that
+are not full, several images a workgroup, both types and directions.  Values against the oracle at the tolerances of the scan's other tests,
+and against the forward that keeps snapshots: the same fp32 sums in another order, in bf16 at most one rounding of a value apart."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import scan_oracle as so
+
+BF16, F32 = torch.bfloat16, torch.float32
+TOL = {F32: 1e-4, BF16: 2e-2}
+CASES = [
+    # B, H, W, E, dtype, bands side by side, rows a band
+    (79, 7, 2, 52, BF16, 1, 7),       # one block of columns
+    (23, 11, 2, 132, BF16, 2, 6),
+    (129, 17, 9, 52, F32, 2, 6),      # two rounds, the second with one band
+    (90, 14, 3, 52, F32, 2, 7),
+    (154, 25, 9, 64, BF16, 2, 7),     # two rounds
+    (173, 16, 2, 12, F32, 2, 8),
+    (136, 29, 12, 36, BF16, 2, 8),    # two rounds
+    (61, 18, 2, 36, F32, 4, 6),
+    (142, 38, 11, 20, BF16, 4, 6),    # two rounds
+    (259, 28, 2, 4, BF16, 4, 7),      # 4 channels, two images a workgroup, the last alone
+    (131, 56, 13, 20, F32, 4, 7),     # two rounds
+    (144, 32, 2, 12, F32, 4, 8),
+    (142, 58, 12, 20, BF16, 4, 8),    # two rounds
+    (87, 43, 2, 12, BF16, 8, 6),
+    (131, 50, 2, 12, F32, 8, 7),
+    (91, 60, 2, 12, BF16, 8, 8),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:4])))
+def test_plan_names_the_rows_kernel(case):
+    from mamba2d_amd import cabi
+    plan = cabi.scan_plan(*case[:5], cabi.M2D_PASS_FWD)
+    assert "; without snapshots m2d_fwd_rows_kernel" in plan and plan.endswith(f"of {case[5]} bands of {case[6]} rows and {128 // case[5]} channels"), plan
+    for flags in (cabi.M2D_FLAG_SPLIT_STATES, cabi.M2D_FLAG_WHOLE_STATES):      # (a lane layout that the caller asks for)
+        assert "rows_kernel" not in cabi.scan_plan(*case[:5], cabi.M2D_PASS_FWD, flags=flags)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("flip", [False, True], ids=["tl", "br"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:4])))
+def test_values(cscan, case, flip):
+    from mamba2d_amd import cabi
+    B, H, W, E, dtype = case[:5]
+    print(f"\ncase {case} flip={flip}", flush=True)
+    inp = so.make_inputs(B, H, W, E, 16, seed=H * W + E, dtype=dtype)
+    ref = {k: v.double() for k, v in inp.items()}
+    if flip:
+        for k in ("x", "deltaT", "deltaL", "BT", "BL", "C"):
+            ref[k] = torch.flip(ref[k], dims=(1, 2)).contiguous()
+    want = cscan.forward(*[ref[k] for k in so.INPUT_NAMES])
+    want = np.flip(want, axis=(1, 2)).copy() if flip else want
+    dev = [inp[k].cuda() for k in so.INPUT_NAMES]
+    y = cabi.scan_fwd(*dev, flip=flip)
+    y_kept, _ = cabi.scan_fwd(*dev, save_ckpt=True, flip=flip)
+    again = cabi.scan_fwd(*dev, flip=flip)
+    torch.cuda.synchronize()
+    assert so.rel_err(y.float().cpu(), want) < TOL[dtype]
+    assert torch.equal(y, again)
+    y, y_kept = y.float(), y_kept.float()
+    assert float((y - y_kept).abs().max() / y_kept.abs().max()) < (1e-5 if dtype == F32 else 2 ** -8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [c for c in CASES if c[3] >= 20 and c[1] > 10], ids=lambda c: "x".join(map(str, c[:4])))
+def test_entry_point(case):
+    """The entry point's operands: packed records, raw parameters."""
+    from mamba2d_amd.wavefront import wavefront_scan_cuda
+    B, H, W, E, dtype = case[:5]
+    print(f"\ncase entry {case}", flush=True)
+    R, g = max(1, E // 16), torch.Generator(device="cuda").manual_seed(7)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    p = [0.3 * r(E, 16), 0.3 * r(E, 16), r(2 * R + 48, E) / E ** 0.5, r(E, R), r(E) - 2, r(E, R), r(E) - 2, 1 + 0.1 * r(E)]
+    x = r(B, H, W, E).to(dtype)
+    kept = wavefront_scan_cuda(x.clone().requires_grad_(True), *p).detach().float()
+    with torch.no_grad():
+        alone = wavefront_scan_cuda(x, *p).float()
+    assert float((alone - kept).abs().max() / kept.abs().max()) < (1e-5 if dtype == F32 else 2 ** -8)
+
+
+@pytest.mark.gpu
+def test_undefined_values_stay_in_their_image_and_channel():
+    """A NaN and an infinity in two images of a workgroup's three, one channel each: every other image and channel is what it is without them."""
+    from mamba2d_amd import cabi
+    B, H, W, E = 600, 28, 6, 32
+    assert "rows_kernel" in cabi.scan_plan(B, H, W, E, F32, cabi.M2D_PASS_FWD)
+    inp = so.make_inputs(B, H, W, E, 16, seed=3, dtype=F32)
+    dev = [inp[k].cuda() for k in so.INPUT_NAMES]
+    clean = cabi.scan_fwd(*dev)
+    x = dev[0].clone()
+    x[1, H - 1, W - 1, 5] = float("nan")
+    x[2, 0, 0, 7] = float("inf")
+    y = cabi.scan_fwd(x, *dev[1:])
+    same = torch.ones_like(y, dtype=torch.bool)
+    same[1, H - 1, W - 1, 5] = False
+    same[2, :, :, 7] = False
+    assert torch.equal(y[same], clean[same])
+    assert bool(y[1, H - 1, W - 1, 5].isnan()) and not bool(torch.isfinite(y[2, 0, 0, 7]))
