@@ -361,6 +361,14 @@ int m2d_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, con
                    int pre_act, const void* pre_scale, const void* pre_bias,
                    int post_act, const void* post_scale, const void* post_bias, void* y, void* stream);
 
+/* m2d_linear_fwd and the residual update of the block behind it in one pass:
+ * y = residual * scale + (pre(x) weight^T + bias + residual2), in the bits of m2d_linear_fwd followed by m2d_scale_residual_fwd (the layer's
+ * output is rounded to bf16 before it is added).  residual, residual2 (may be NULL) and y are (P,N) bf16, y none of the others;
+ * scale (N) has weight_dtype.  pre_act: M2D_ACT_NONE or M2D_ACT_GELU.  K up to 64 with N up to 64, K up to 128 with N up to 128;
+ * otherwise as m2d_linear_fwd. */
+int m2d_linear_residual_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias, int pre_act,
+                            const void* residual, const void* scale, const void* residual2, void* y, void* stream);
+
 /* y = post(x weight^T + bias) for wide layers and few positions (P (P,K) and (P,N) bf16, post_act nothing or GELU of the
  * layer's output rounded to bf16): K and N multiples of 32, any size.  Reads its operands straight from memory, made for
  * the latency of a few hundred positions; beyond about a thousand a tiled product is faster.  With GELU, bf16 weights, K up
@@ -395,6 +403,13 @@ int m2d_layernorm_linear_fwd(int64_t P, int K, int N, int weight_dtype, const vo
 int m2d_mlp_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x,
                 const void* ln_weight, const void* ln_bias, float eps,
                 const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream);
+
+/* m2d_mlp_fwd with the block's residual update and the norm behind it in the same pass: x_out = x * scale + MLP(x) and
+ * y = LayerNorm(x_out; next_weight, next_bias, next_eps), in the bits of m2d_mlp_fwd followed by m2d_scale_residual_layernorm_fwd.  x_out and y
+ * are (P, C) bf16 and none of the others; scale, next_weight and next_bias (C) have weight_dtype. */
+int m2d_mlp_residual_layernorm_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias,
+                                   float eps, const void* w1, const void* b1, const void* w2, const void* b2, const void* scale,
+                                   const void* next_weight, const void* next_bias, float next_eps, void* x_out, void* y, void* stream);
 
 /* bf16 -> fp32 for up to 64 arrays of n elements per launch: the parameters of a model held in bf16, for the calls that
  * take fp32 parameters. */

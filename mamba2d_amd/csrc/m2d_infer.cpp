@@ -64,6 +64,13 @@ struct Run {
     Tensor y = at::linear(pre == M2D_ACT_GELU ? at::gelu(x) : x, w, b && b->defined() ? c10::optional<Tensor>(*b) : c10::nullopt);
     return post == M2D_ACT_GELU ? at::gelu(y) : y;
   }
+  // x s + (GELU(y) w^T + b + r2)
+  Tensor linear_residual(const Tensor& y, const Tensor& w, const Tensor& b, const Tensor& x, const Tensor& s, const Tensor& r2) const {
+    Tensor o = make(C);
+    check(m2d_linear_residual_fwd(P, (int)C, (int)C, wd, y.data_ptr(), w.data_ptr(), b.data_ptr(), M2D_ACT_GELU, x.data_ptr(), s.data_ptr(),
+                                  r2.defined() ? r2.data_ptr() : nullptr, o.data_ptr(), st));
+    return o;
+  }
   Tensor residual(const Tensor& x, const Tensor& s, const Tensor& r, const Tensor& r2) const {
     Tensor y = make(C);
     check(m2d_scale_residual_fwd(P, (int)C, M2D_BF16, wd, x.data_ptr(), s.data_ptr(), r.data_ptr(), r2.defined() ? r2.data_ptr() : nullptr,
@@ -130,6 +137,8 @@ Tensor infer_stage(const Tensor& x_in, at::TensorList par, at::IntArrayRef kinds
     const double next_eps = last ? eps[3 * kinds.size()] : eps[3 * (blk + 1)];
     shaped(p[kN1W], {C}); shaped(p[kN1B], {C});
     const Tensor n1 = normed.defined() ? normed : r.norm(x, p[kN1W], p[kN1B], eps[3 * blk]);
+    const int64_t HD = p[att ? (int)aFc1W : (int)kFc1W].size(0);
+    const bool narrow = C % 32 == 0 && C <= 128 && HD % 16 == 0 && HD <= 512;
     Tensor term, term2;
     const Tensor *rs1, *n2w, *n2b, *f1w, *f1b, *f2w, *f2b, *rs2;
     if (att) {
@@ -173,19 +182,26 @@ Tensor infer_stage(const Tensor& x_in, at::TensorList par, at::IntArrayRef kinds
       const int64_t N = at_w(kATLog).size(1);
       const auto pr = m2dshim::proj_fwd(u, at_w(kXProj), at_w(kDtTW), at_w(kDtTB), at_w(kDtLW), at_w(kDtLB), N, true, true);
       const Tensor y = std::get<0>(m2dshim::scan_fwd(u, pr[1], pr[2], at_w(kATLog), at_w(kALLog), pr[3], pr[4], pr[5], at_w(kD), false, flip, true, true, 0));
-      term = r.linear(y, p[kOutW], p + kOutB, M2D_ACT_GELU, nullptr, nullptr, M2D_ACT_NONE, nullptr, nullptr);
+      if (narrow) {      // the residual update is part of the output projection (other blocks have it with the norm behind it)
+        shaped(p[kRs1], {C});
+        x = r.linear_residual(y, p[kOutW], p[kOutB], x, p[kRs1], term2);
+      } else {
+        term = r.linear(y, p[kOutW], p + kOutB, M2D_ACT_GELU, nullptr, nullptr, M2D_ACT_NONE, nullptr, nullptr);
+      }
       rs1 = p + kRs1; n2w = p + kN2W; n2b = p + kN2B; f1w = p + kFc1W; f1b = p + kFc1B; f2w = p + kFc2W; f2b = p + kFc2B; rs2 = p + kRs2;
     }
-    const int64_t HD = f1w->size(0);
     shaped(*f1w, {HD, C}); shaped(*f2w, {C, HD}); shaped(*f1b, {HD}); shaped(*f2b, {C});
     for (const Tensor* t : {rs1, n2w, n2b, rs2, &next_w, &next_b}) shaped(*t, {C});
     Tensor branch;
-    if (C % 32 == 0 && C <= 128 && HD % 16 == 0 && HD <= 512) {      // norm2 inside the MLP's first kernel
-      x = r.residual(x, *rs1, term, term2);
-      if ((C == 32 || C == 64) && HD == 4 * C) {
-        branch = r.make(C);
-        check(m2d_mlp_fwd(r.P, (int)C, (int)HD, r.wd, x.data_ptr(), n2w->data_ptr(), n2b->data_ptr(), (float)eps[3 * blk + 1], f1w->data_ptr(),
-                          f1b->data_ptr(), f2w->data_ptr(), f2b->data_ptr(), branch.data_ptr(), r.st));
+    if (narrow) {      // norm2 inside the MLP's first kernel
+      if (term.defined()) x = r.residual(x, *rs1, term, term2);
+      if ((C == 32 || C == 64) && HD == 4 * C) {      // ... and the residual update and the next norm behind it too
+        Tensor xo = r.make(C);
+        normed = r.make(C);
+        check(m2d_mlp_residual_layernorm_fwd(r.P, (int)C, (int)HD, r.wd, x.data_ptr(), n2w->data_ptr(), n2b->data_ptr(), (float)eps[3 * blk + 1],
+                                             f1w->data_ptr(), f1b->data_ptr(), f2w->data_ptr(), f2b->data_ptr(), rs2->data_ptr(),
+                                             next_w.data_ptr(), next_b.data_ptr(), (float)next_eps, xo.data_ptr(), normed.data_ptr(), r.st));
+        x = xo;
       } else {
         Tensor h = r.make(HD);
         check(m2d_layernorm_linear_fwd(r.P, (int)C, (int)HD, r.wd, x.data_ptr(), n2w->data_ptr(), n2b->data_ptr(), (float)eps[3 * blk + 1],
@@ -198,7 +214,7 @@ Tensor infer_stage(const Tensor& x_in, at::TensorList par, at::IntArrayRef kinds
       branch = r.linear(r.linear(n2, *f1w, f1b, M2D_ACT_NONE, nullptr, nullptr, M2D_ACT_GELU, nullptr, nullptr), *f2w, f2b, M2D_ACT_NONE, nullptr,
                         nullptr, M2D_ACT_NONE, nullptr, nullptr);
     }
-    x = r.residual_norm(x, *rs2, branch, none, next_w, next_b, next_eps, normed);
+    if (branch.defined()) x = r.residual_norm(x, *rs2, branch, none, next_w, next_b, next_eps, normed);
   }
   return normed;
 }

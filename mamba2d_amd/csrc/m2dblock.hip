@@ -530,6 +530,7 @@ struct LinArgs {
   const void *ln_w, *ln_b;                       // LayerNorm over the K inputs in front of the layer (pre == kActLayerNorm): weight and bias, (K), type of w
   float ln_eps;
   void* z;              // (P, N) bf16 or null: the layer's output before post, for a caller whose backward wants its slope
+  const void *res_x, *res_r, *res_s;   // RES: the residual stream (P, N) bf16, a second branch (P, N) bf16 or null, and the scale of the stream (N), type of w
 };
 
 // a and b hold 4 values each of two tiles of 16 in lane row kb (the lane's number / 16).  Rows 0 and 2 end with a's values of
@@ -539,10 +540,16 @@ __device__ __forceinline__ uint4 halves_exchanged(const uint2 a, const uint2 b) 
   return make_uint4(x[0], y[0], x[1], y[1]);
 }
 
-constexpr int lin_per_cu(int kcmax) { return kcmax <= 2 ? 6 : kcmax <= 8 ? 4 : 2; }   // workgroups whose registers fit a compute unit
+constexpr int lin_per_cu(int kcmax, bool res = false) { return res ? (kcmax <= 2 ? 4 : 3) : kcmax <= 2 ? 6 : kcmax <= 8 ? 4 : 2; }   // workgroups whose registers fit a compute unit
 
-template <int KCMAX>   // steps of 32 along K that the kernel is built for: 2, 4, 8 or 16
-__global__ __launch_bounds__(kLinThreads, lin_per_cu(KCMAX)) void m2d_linear_kernel(const LinArgs a) {
+// KCMAX: steps of 32 along K that the kernel is built for: 2, 4, 8 or 16.
+// RES: y = res_x * res_s + (layer + res_r), the residual update of the block around the layer, in the bits that the layer's kernel and
+// m2d_scale_residual_kernel gave one after the other (the layer's output is rounded to bf16 before it is added).  Both kernels ran at the rate of
+// memory: without the layer's output going out and back 128x56x56x64 takes 49, 128x28x28x128 37 us where they took 27 + 35 and 25 + 18.
+// The stream's pieces are fetched a tile ahead into the registers that the last tile's pieces have just left: a wait for one leaves the
+// stores behind it under way.
+template <int KCMAX, bool RES = false>
+__global__ __launch_bounds__(kLinThreads, lin_per_cu(KCMAX, RES)) void m2d_linear_kernel(const LinArgs a) {
   extern __shared__ float smem[];
   const int tid = threadIdx.x, l = tid & 63, mn = l & 15, kb = l >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -571,8 +578,21 @@ __global__ __launch_bounds__(kLinThreads, lin_per_cu(KCMAX)) void m2d_linear_ker
 #pragma unroll
     for (int kc = 0; kc < KCMAX; ++kc) Anext[kc] = ld16(row + 32 * (kc < KC ? kc : KC - 1));
   };
+  // a lane's 8 neighbouring outputs of the step of 32 that starts at n0 (see the stores below)
+  auto piece_at = [&](int n0) { return n0 + (kb & 1 && n0 + 16 < a.Ns ? 16 : 0) + 4 * (kb & 2); };
+  constexpr int NR = RES ? KCMAX : 1;                    // (the host sees to Ns <= 32 KCMAX)
+  uint4 RX[NR], RR[NR];
+  auto fetch_res = [&](int tile, int c) {
+    const int64_t q = (int64_t)tile * 64 + wave * 16 + mn, at = (q < a.P ? q : a.P - 1) * a.N + nbase + piece_at(32 * c < a.Ns ? 32 * c : 0);
+    RX[c] = ld16(static_cast<const uint16_t*>(a.res_x) + at);
+    if (a.res_r) RR[c] = ld16(static_cast<const uint16_t*>(a.res_r) + at);      // (uniform)
+  };
   // Everything a workgroup reads once is on its way before the first of it is waited for.
   fetch(first_tile);
+  if constexpr (RES) {
+#pragma unroll
+    for (int c = 0; c < NR; ++c) fetch_res(first_tile, c);
+  }
   const int tn = tid < a.Ns ? tid : a.Ns - 1, tk = tid < a.K ? tid : a.K - 1;
   const float bias0 = a.bias ? ldw(a.bias, a.wbf16, nbase + tn) : 0.f;
   const float lnw0 = a.pre == kActLayerNorm ? ldw(a.ln_w, a.wbf16, tk) : 0.f, lnb0 = a.pre == kActLayerNorm ? ldw(a.ln_b, a.wbf16, tk) : 0.f;
@@ -586,6 +606,8 @@ __global__ __launch_bounds__(kLinThreads, lin_per_cu(KCMAX)) void m2d_linear_ker
   if (tid < a.Ns) bias[tid] = bias0;
   for (int i = tid + kLinThreads; i < a.Ns; i += kLinThreads) bias[i] = a.bias ? ldw(a.bias, a.wbf16, nbase + i) : 0.f;
   if (a.pre == kActLayerNorm && tid < a.K) { lnp[tid] = lnw0; lnp[a.K + tid] = lnb0; }      // (K <= 128)
+  if constexpr (RES)                                     // (no normalisation here: the scale lies in its place)
+    for (int i = tid; i < a.Ns; i += kLinThreads) lnp[i] = ldw(a.res_s, a.wbf16, nbase + i);
   __syncthreads();
   // A wave's tiles end at the last row.  Its lanes past that row hold and store the row's own values once more, so no store
   // sits in a branch and the wait for the next tile's rows leaves the stores behind them under way.
@@ -611,7 +633,7 @@ __global__ __launch_bounds__(kLinThreads, lin_per_cu(KCMAX)) void m2d_linear_ker
     }
     // W's rows are the first operand: lane (mn, kb) ends with outputs 4 kb + i of position mn.  Two tiles of 16 outputs at a time;
     // lanes of neighbouring kb exchange halves and store 8 neighbouring outputs each.  An odd last tile is taken twice.
-    for (int n0 = 0; n0 < a.Ns; n0 += 32) {
+    auto outputs = [&](int n0, auto&& leave) {
       const int second = n0 + 16 < a.Ns ? 16 : 0;
       uint2 zq[2], yq[2];
 #pragma unroll
@@ -632,9 +654,35 @@ __global__ __launch_bounds__(kLinThreads, lin_per_cu(KCMAX)) void m2d_linear_ker
         for (int i = 0; i < 4; ++i) acc[i] = act(a.post, acc[i], post_s, post_b);
         yq[t] = make_uint2(pack_bf16(acc[0], acc[1]), pack_bf16(acc[2], acc[3]));
       }
-      const int64_t at = out + n0 + (kb & 1 ? second : 0) + 4 * (kb & 2);
+      const int64_t at = out + piece_at(n0);
       if (a.z) *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.z) + at) = halves_exchanged(zq[0], zq[1]);
-      *reinterpret_cast<uint4*>(Y + at) = halves_exchanged(yq[0], yq[1]);
+      leave(at, halves_exchanged(yq[0], yq[1]));
+    };
+    if constexpr (RES) {
+#pragma unroll
+      for (int c = 0; c < NR; ++c)
+        if (32 * c < a.Ns)                               // (uniform)
+          outputs(32 * c, [&](int64_t at, const uint4& layer) {
+            const float4* sp = reinterpret_cast<const float4*>(lnp + piece_at(32 * c));
+            const float4 s0 = sp[0], s1 = sp[1];
+            const float sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+            const uint32_t xw[4] = {RX[c].x, RX[c].y, RX[c].z, RX[c].w}, lw[4] = {layer.x, layer.y, layer.z, layer.w};
+            float r[8];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { r[2 * j] = bf_lo(lw[j]); r[2 * j + 1] = bf_hi(lw[j]); }
+            if (a.res_r) {
+              const uint32_t rw[4] = {RR[c].x, RR[c].y, RR[c].z, RR[c].w};
+#pragma unroll
+              for (int j = 0; j < 4; ++j) { r[2 * j] += bf_lo(rw[j]); r[2 * j + 1] += bf_hi(rw[j]); }
+            }
+            uint32_t o[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = pack_bf16(__builtin_fmaf(bf_lo(xw[j]), sc[2 * j], r[2 * j]), __builtin_fmaf(bf_hi(xw[j]), sc[2 * j + 1], r[2 * j + 1]));
+            fetch_res(tile + tile_step, c);
+            *reinterpret_cast<uint4*>(Y + at) = make_uint4(o[0], o[1], o[2], o[3]);
+          });
+    } else {
+      for (int n0 = 0; n0 < a.Ns; n0 += 32) outputs(n0, [&](int64_t at, const uint4& q) { *reinterpret_cast<uint4*>(Y + at) = q; });
     }
   }
 }
@@ -867,9 +915,17 @@ struct MlpArgs {
   int wbf16, ntiles;
   const void *ln_w, *ln_b;   // LayerNorm over C in front of fc1: weight and bias, (C), or null
   float ln_eps;
+  const void *res_s, *nx_w, *nx_b;   // RES: scale of the residual stream, weight and bias of the norm behind the update, (C)
+  float nx_eps;
+  void* xo;               // RES: (P, C) the updated stream; y is its norm
 };
 
-template <int KC>   // C = 32 KC channels, 128 KC hidden units
+// KC: C = 32 KC channels, 128 KC hidden units.
+// RES: xo = x * res_s + MLP(x), y = LayerNorm(xo), the residual update and the next block's norm in the bits that m2d_layernorm_kernel gives behind
+// this one: after an exchange of halves a lane holds whole 8-channel pieces of its row (piece 4 no / 2 + {0, 2, 1, 3}[kb]), and the row's sums are
+// folded in that kernel's order: pieces 4, 2 and 1 apart.  The products and the GELU are what takes this kernel's time, so what
+// it moves beside them costs little: 128x56x56x64 128 us where the two kernels took 110 + 33.
+template <int KC, bool RES = false>
 __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
   constexpr int C = 32 * KC, HD = 4 * C, NH = HD / 16, NO = C / 16, NP = NH / 2;
   constexpr int W1S = C + 8;      // bf16 per row of W1 in LDS (a row per hidden unit)
@@ -912,6 +968,13 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
   if (tid < HD) b1l[tid] = b10;
   float* lnp = b1l + HD;
   if (a.ln_w && tid < C) { lnp[tid] = lnw0; lnp[C + tid] = lnb0; }
+  const float* nxp = lnp + 2 * C;      // RES: scale, weight, bias
+  if constexpr (RES) {
+    if (tid < C) {
+      float* d = lnp + 2 * C + tid;
+      d[0] = ldw(a.res_s, a.wbf16, tid); d[C] = ldw(a.nx_w, a.wbf16, tid); d[2 * C] = ldw(a.nx_b, a.wbf16, tid);
+    }
+  }
   __syncthreads();
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   for (int tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
@@ -919,6 +982,12 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
     uint4 Xf[KC];
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) Xf[kc] = Xnext[kc];
+    uint4 xr[RES ? KC : 1];
+    const int piece = (kb & 1 ? 16 : 0) + 4 * (kb & 2);
+    if constexpr (RES) {               // the stream again, as the results will lie
+#pragma unroll
+      for (int c = 0; c < KC; ++c) xr[c] = ld16(X + (p0 + mn < a.P ? p0 + mn : a.P - 1) * C + 32 * c + piece);
+    }
     fetch(tile + gridDim.x);
     if (a.ln_w) norm_rows<KC>(Xf, KC, C, lnp, a.ln_eps, kb);      // (uniform)
     f32x4_t h[NH];
@@ -938,6 +1007,7 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
     for (int ks = 0; ks < NP; ++ks)
       hf[ks] = make_uint4(pack_bf16(h[2 * ks][0], h[2 * ks][1]), pack_bf16(h[2 * ks][2], h[2 * ks][3]),
                           pack_bf16(h[2 * ks + 1][0], h[2 * ks + 1][1]), pack_bf16(h[2 * ks + 1][2], h[2 * ks + 1][3]));
+    uint2 yq[NO];
 #pragma unroll
     for (int no = 0; no < NO; ++no) {
       f32x4_t acc = zero;
@@ -947,9 +1017,57 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
         const uint2 lo = *reinterpret_cast<const uint2*>(w), hi = *reinterpret_cast<const uint2*>(w + 16);
         acc = mfma_bf16(make_uint4(lo.x, lo.y, hi.x, hi.y), hf[ks], acc);
       }
-      if (p0 + mn < a.P)
-        *reinterpret_cast<uint2*>(Y + (p0 + mn) * C + 16 * no + 4 * kb) =
-            make_uint2(pack_bf16(acc[0] + b2v[no][0], acc[1] + b2v[no][1]), pack_bf16(acc[2] + b2v[no][2], acc[3] + b2v[no][3]));
+      yq[no] = make_uint2(pack_bf16(acc[0] + b2v[no][0], acc[1] + b2v[no][1]), pack_bf16(acc[2] + b2v[no][2], acc[3] + b2v[no][3]));
+      if constexpr (!RES) {
+        if (p0 + mn < a.P) *reinterpret_cast<uint2*>(Y + (p0 + mn) * C + 16 * no + 4 * kb) = yq[no];
+      }
+    }
+    if constexpr (RES) {
+      uint4 xo[KC];
+      float v[KC][8], part[KC];
+      // the sum of a row's pieces: piece ^ 4 is the lane's own other one, ^ 2 and ^ 1 are in the lanes 16 and 32 further
+      auto row_sum = [&](const float (&t)[KC]) {
+        float s = KC == 2 ? t[0] + t[KC - 1] : t[0];
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        return s;
+      };
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const uint4 m = halves_exchanged(yq[2 * c], yq[2 * c + 1]);
+        const uint32_t mw[4] = {m.x, m.y, m.z, m.w}, xw[4] = {xr[c].x, xr[c].y, xr[c].z, xr[c].w};
+        const float* sc = nxp + 32 * c + piece;
+        uint32_t o[4];
+        part[c] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          o[j] = pack_bf16(__builtin_fmaf(bf_lo(xw[j]), sc[2 * j], bf_lo(mw[j])), __builtin_fmaf(bf_hi(xw[j]), sc[2 * j + 1], bf_hi(mw[j])));
+          v[c][2 * j] = bf_lo(o[j]); v[c][2 * j + 1] = bf_hi(o[j]);      // (the norm sees what is stored)
+          part[c] += v[c][2 * j]; part[c] += v[c][2 * j + 1];
+        }
+        xo[c] = make_uint4(o[0], o[1], o[2], o[3]);
+      }
+      const float mean = row_sum(part) * (1.f / C);
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        part[c] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { const float d = v[c][j] - mean; part[c] = __builtin_fmaf(d, d, part[c]); }
+      }
+      const float rstd = rsqrtf(row_sum(part) * (1.f / C) + a.nx_eps);
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const float *w = nxp + C + 32 * c + piece, *b = w + C;
+        uint32_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o[j] = pack_bf16(__builtin_fmaf((v[c][2 * j] - mean) * rstd, w[2 * j], b[2 * j]), __builtin_fmaf((v[c][2 * j + 1] - mean) * rstd, w[2 * j + 1], b[2 * j + 1]));
+        if (p0 + mn < a.P) {
+          const int64_t at = (p0 + mn) * C + 32 * c + piece;
+          *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.xo) + at) = xo[c];
+          *reinterpret_cast<uint4*>(Y + at) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+      }
     }
   }
 }
@@ -968,7 +1086,8 @@ inline bool allow_big_lds() {
   if (seen.load(std::memory_order_acquire) & bit) return true;
   const void* kernels[] = {reinterpret_cast<const void*>(&m2d_linear_kernel<2>), reinterpret_cast<const void*>(&m2d_linear_kernel<4>),
                            reinterpret_cast<const void*>(&m2d_linear_kernel<8>), reinterpret_cast<const void*>(&m2d_linear_kernel<16>),
-                           reinterpret_cast<const void*>(&m2d_mlp_kernel<1>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2>)};
+                           reinterpret_cast<const void*>(&m2d_mlp_kernel<1>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2>),
+                           reinterpret_cast<const void*>(&m2d_mlp_kernel<1, true>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2, true>)};
   for (const void* k : kernels)
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLinMaxLds) != hipSuccess) return false;
   seen.fetch_or(bit, std::memory_order_release);
@@ -1331,8 +1450,8 @@ int m2d_rope_qknorm_fwd(int B, int L, int heads, int head_dim, int dtype, int we
   return dtype == M2D_F32 ? run_rope<float>(a, G, st) : run_rope<bf16_t>(a, G, st);
 }
 
-int m2d_mlp_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias, float eps,
-                const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream) {
+static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias, float eps,
+                   const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream, const MlpArgs* res) {
   if (!x || !w1 || !w2 || !y || (ln_weight != nullptr) != (ln_bias != nullptr)) return M2D_ERR_NULL_POINTER;
   if (P < 1 || C < 1 || hidden < 1) return M2D_ERR_BAD_SHAPE;
   if (weight_dtype != M2D_F32 && weight_dtype != M2D_BF16) return M2D_ERR_UNSUPPORTED;
@@ -1345,16 +1464,34 @@ int m2d_mlp_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, c
   a.ln_w = ln_weight; a.ln_b = ln_bias; a.ln_eps = eps;
   a.x = x; a.w1 = w1; a.b1 = b1; a.w2 = w2; a.b2 = b2; a.y = y; a.P = P; a.wbf16 = weight_dtype == M2D_BF16;
   a.ntiles = (int)((P + 63) / 64);
-  const size_t lds = C == 64 ? mlp_lds_bytes<2>() : mlp_lds_bytes<1>();
+  if (res) { a.res_s = res->res_s; a.nx_w = res->nx_w; a.nx_b = res->nx_b; a.nx_eps = res->nx_eps; a.xo = res->xo; }
+  const size_t lds = (C == 64 ? mlp_lds_bytes<2>() : mlp_lds_bytes<1>()) + (res ? (size_t)3 * C * 4 : 0);
   if (lds > 64 * 1024 && !allow_big_lds()) return M2D_ERR_HIP;
   int per_cu = (int)(160 * 1024 / lds);      // persistent: the weights go to LDS once per workgroup
   if (per_cu > 4) per_cu = 4;
   int grid = 256 * per_cu;
   if (grid > a.ntiles) grid = a.ntiles;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (C == 64) hipLaunchKernelGGL(m2d_mlp_kernel<2>, dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
+  if (res && C == 64) hipLaunchKernelGGL((m2d_mlp_kernel<2, true>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
+  else if (res) hipLaunchKernelGGL((m2d_mlp_kernel<1, true>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
+  else if (C == 64) hipLaunchKernelGGL(m2d_mlp_kernel<2>, dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
   else hipLaunchKernelGGL(m2d_mlp_kernel<1>, dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
+}
+
+int m2d_mlp_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias, float eps,
+                const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream) {
+  return run_mlp(P, C, hidden, weight_dtype, x, ln_weight, ln_bias, eps, w1, b1, w2, b2, y, stream, nullptr);
+}
+
+int m2d_mlp_residual_layernorm_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias,
+                                   float eps, const void* w1, const void* b1, const void* w2, const void* b2, const void* scale,
+                                   const void* next_weight, const void* next_bias, float next_eps, void* x_out, void* y, void* stream) {
+  if (!scale || !next_weight || !next_bias || !x_out) return M2D_ERR_NULL_POINTER;
+  if (misaligned(x_out, 16) || misaligned(scale, 4) || misaligned(next_weight, 4) || misaligned(next_bias, 4)) return M2D_ERR_MISALIGNED;
+  MlpArgs res = {};
+  res.res_s = scale; res.nx_w = next_weight; res.nx_b = next_bias; res.nx_eps = next_eps; res.xo = x_out;
+  return run_mlp(P, C, hidden, weight_dtype, x, ln_weight, ln_bias, eps, w1, b1, w2, b2, y, stream, &res);
 }
 
 int m2d_rope_attention_fwd(int B, int L, int heads, int head_dim, int weight_dtype, const void* qkv, const void* cos,
@@ -1397,7 +1534,7 @@ int m2d_rope_attention_fwd(int B, int L, int heads, int head_dim, int weight_dty
 static int run_linear(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias,
                       int pre_act, const void* pre_scale, const void* pre_bias, int post_act, const void* post_scale,
                       const void* post_bias, void* y, void* stream, const void* ln_w, const void* ln_b, float ln_eps,
-                      void* z = nullptr) {
+                      void* z = nullptr, const LinArgs* res = nullptr) {
   if (!x || !weight || !y) return M2D_ERR_NULL_POINTER;
   const bool ln = pre_act == kActLayerNorm;
   if (ln && (!ln_w || !ln_b)) return M2D_ERR_NULL_POINTER;
@@ -1423,11 +1560,12 @@ static int run_linear(int64_t P, int K, int N, int weight_dtype, const void* x, 
   a.pre = pre_act; a.post = post_act; a.pre_s = pre_scale; a.pre_b = pre_bias; a.post_s = post_scale; a.post_b = post_bias;
   a.ntiles = (int)((P + 63) / 64);
   a.nsplit = nsplit; a.Ns = Ns; a.z = z;
-  const size_t lds = linear_lds_bytes(K, Ns, ln);
+  if (res) { a.res_x = res->res_x; a.res_r = res->res_r; a.res_s = res->res_s; }
+  const size_t lds = linear_lds_bytes(K, Ns, ln) + (res ? (size_t)Ns * 4 : 0);
   if (lds > 64 * 1024 && !allow_big_lds()) return M2D_ERR_HIP;
   // persistent: the weights are loaded into LDS once per workgroup; as many workgroups as fit the device at once
   int per_cu = (int)(160 * 1024 / lds);
-  const int most = lin_per_cu(K <= 64 ? 2 : K <= 128 ? 4 : K <= 256 ? 8 : 16);
+  const int most = lin_per_cu(K <= 64 ? 2 : K <= 128 ? 4 : K <= 256 ? 8 : 16, res != nullptr);
   if (per_cu > most) per_cu = most;
   int grid = 256 * per_cu / nsplit;     // workgroups per slice
   grid = grid / 8 * 8;
@@ -1436,7 +1574,9 @@ static int run_linear(int64_t P, int K, int N, int weight_dtype, const void* x, 
   grid *= nsplit;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 g((unsigned)grid), t(kLinThreads);
-  if (K <= 64) hipLaunchKernelGGL(m2d_linear_kernel<2>, g, t, lds, st, a);
+  if (res && K <= 64) hipLaunchKernelGGL((m2d_linear_kernel<2, true>), g, t, lds, st, a);
+  else if (res) hipLaunchKernelGGL((m2d_linear_kernel<4, true>), g, t, lds, st, a);
+  else if (K <= 64) hipLaunchKernelGGL(m2d_linear_kernel<2>, g, t, lds, st, a);
   else if (K <= 128) hipLaunchKernelGGL(m2d_linear_kernel<4>, g, t, lds, st, a);
   else if (K <= 256) hipLaunchKernelGGL(m2d_linear_kernel<8>, g, t, lds, st, a);
   else hipLaunchKernelGGL(m2d_linear_kernel<16>, g, t, lds, st, a);
@@ -1449,6 +1589,18 @@ int m2d_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, con
   if (pre_act == kActLayerNorm) return M2D_ERR_UNSUPPORTED;      // that one has an entry point of its own
   return run_linear(P, K, N, weight_dtype, x, weight, bias, pre_act, pre_scale, pre_bias, post_act, post_scale, post_bias, y, stream,
                     nullptr, nullptr, 0.f);
+}
+
+int m2d_linear_residual_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias, int pre_act,
+                            const void* residual, const void* scale, const void* residual2, void* y, void* stream) {
+  if (!residual || !scale) return M2D_ERR_NULL_POINTER;
+  if (pre_act != kActNone && pre_act != kActGelu) return M2D_ERR_UNSUPPORTED;
+  if (K > 128 || N > (K <= 64 ? 64 : 128)) return M2D_ERR_UNSUPPORTED;      // the stream's pieces of a row are held in registers
+  if (misaligned(residual, 16) || misaligned(residual2, 16) || misaligned(scale, 4)) return M2D_ERR_MISALIGNED;
+  LinArgs res = {};
+  res.res_x = residual; res.res_r = residual2; res.res_s = scale;
+  return run_linear(P, K, N, weight_dtype, x, weight, bias, pre_act, nullptr, nullptr, kActNone, nullptr, nullptr, y, stream, nullptr, nullptr,
+                    0.f, nullptr, &res);
 }
 
 int m2d_wide_linear_fwd(int64_t P, int K, int N, int weight_dtype, const void* x, const void* weight, const void* bias, int post_act,

@@ -1,0 +1,78 @@
+"""A linear layer and an MLP with the block's residual update in the same kernel, against the kernels one after the other: the same bits,
+at the edges of tiles of rows and outputs; and what they refuse."""
+import ctypes
+
+import pytest
+import torch
+
+gpu = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
+on_gpu = lambda f: gpu[0](gpu[1](f))
+WTYPES = pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16], ids=["w_f32", "w_bf16"])
+
+# rows, inputs, outputs: rows that end inside a wave's 16 and a workgroup's 64, more tiles than workgroups; an odd number of 16 outputs; slices
+LINEAR = [(1, 32, 16), (15, 64, 48), (17, 32, 64), (63, 64, 64), (65, 128, 128), (130, 96, 80), (77, 128, 16), (49, 128, 112), (70001, 64, 64), (70000, 128, 128),
+          (66000, 32, 48)]
+
+
+@on_gpu
+@WTYPES
+@pytest.mark.parametrize("shape", LINEAR, ids=lambda s: "x".join(map(str, s)))
+def test_linear_residual_gives_the_bits_of_two_kernels(shape, wdtype):
+    from mamba2d_amd import cabi
+    P, K, N = shape
+    print(f"\ncase linear residual {shape} {wdtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(P + 3 * K + N)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, res, res2 = (r(P, k).bfloat16() for k in (K, N, N))
+    res[0, 0], res2[P - 1, N - 1] = float("inf"), float("nan")
+    w, b, s = (r(N, K) / K ** 0.5).to(wdtype), r(N).to(wdtype), r(N).to(wdtype)
+    for act, second, bias in ((cabi.ACT_GELU, res2, b), (cabi.ACT_NONE, None, None)):
+        layer = cabi.linear_fwd(x, w, bias, pre=act)
+        want = cabi.scale_residual_fwd(res, s, layer, second)
+        y = torch.full((P + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        cabi.check(cabi.lib.m2d_linear_residual_fwd(P, K, N, cabi._dtype_code(w), cabi._ptr(x), cabi._ptr(w), cabi._ptr(bias), act, cabi._ptr(res), cabi._ptr(s),
+                                                    cabi._ptr(second), cabi._ptr(y), cabi._stream(x.device)))
+        assert (y[P] == 7).all()
+        assert torch.equal(y[:P].isnan(), want.isnan()) and torch.equal(y[:P].nan_to_num(), want.nan_to_num())
+
+
+@on_gpu
+@WTYPES
+@pytest.mark.parametrize("C", [32, 64])
+@pytest.mark.parametrize("P", [1, 15, 16, 63, 65, 1000, 70001])
+def test_mlp_residual_norm_gives_the_bits_of_two_kernels(P, C, wdtype):
+    from mamba2d_amd import cabi
+    print(f"\ncase mlp residual {P}x{C} {wdtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(P + C)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = (3 * r(P, C)).bfloat16()
+    x[P // 2, 3] = float("inf")
+    w1, w2 = (r(4 * C, C) / C ** 0.5).to(wdtype), (r(C, 4 * C) / (2 * C ** 0.5)).to(wdtype)
+    b1, b2, lw, lb, s, nw, nb = (r(n).to(wdtype) for n in (4 * C, C, C, C, C, C, C))
+    for ln, biases in (((lw, lb), (b1, b2)), ((None, None), (None, None))):
+        branch = cabi.mlp_fwd(x, w1, biases[0], w2, biases[1], *ln, 1e-5)
+        want = cabi.scale_residual_layernorm_fwd(x, s, branch, None, nw, nb, 1e-3)
+        xo, y = (torch.full((P + 1, C), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        cabi.check(cabi.lib.m2d_mlp_residual_layernorm_fwd(P, C, 4 * C, cabi._dtype_code(w1), cabi._ptr(x), cabi._ptr(ln[0]), cabi._ptr(ln[1]), 1e-5, cabi._ptr(w1),
+                                                           cabi._ptr(biases[0]), cabi._ptr(w2), cabi._ptr(biases[1]), cabi._ptr(s), cabi._ptr(nw), cabi._ptr(nb), 1e-3,
+                                                           cabi._ptr(xo), cabi._ptr(y), cabi._stream(x.device)))
+        for got, two in zip((xo, y), want):
+            assert (got[P] == 7).all()
+            assert torch.equal(got[:P].isnan(), two.isnan()) and torch.equal(got[:P].nan_to_num(), two.nan_to_num())
+
+
+def test_refusals():
+    """Host checks only: nothing is launched."""
+    from mamba2d_amd import cabi
+    buf = (ctypes.c_char * 4096)()
+    p = (ctypes.addressof(buf) + 255) // 256 * 256
+    linear = lambda P=4, K=64, N=64, wd=1, pre=0, res=p, s=p, res2=None, y=p: cabi.lib.m2d_linear_residual_fwd(P, K, N, wd, p, p, p, pre, res, s, res2, y, None)
+    ok, null, shape, unsupported, misaligned = 0, 1, 2, 3, 5
+    assert [linear(res=None), linear(s=None), linear(y=None)] == [null] * 3
+    assert [linear(K=160), linear(N=80), linear(K=128, N=144), linear(K=48), linear(N=40), linear(pre=cabi.ACT_STARRELU), linear(wd=7)] == [unsupported] * 7
+    assert [linear(res=p + 8), linear(res2=p + 2), linear(s=p + 2), linear(y=p + 4)] == [misaligned] * 4
+    assert linear(P=0) == shape
+    mlp = lambda C=64, s=p, nw=p, xo=p, y=p: cabi.lib.m2d_mlp_residual_layernorm_fwd(4, C, 4 * C, 1, p, None, None, 0.0, p, p, p, p, s, nw, p, 0.0, xo, y, None)
+    assert [mlp(s=None), mlp(nw=None), mlp(xo=None), mlp(y=None)] == [null] * 4
+    assert [mlp(C=128), mlp(C=48)] == [unsupported] * 2
+    assert [mlp(xo=p + 8), mlp(s=p + 2), mlp(y=p + 4)] == [misaligned] * 3
