@@ -484,36 +484,36 @@ __device__ __forceinline__ void norm_rows(uint4 (&A)[KCMAX], int KC, int K, cons
 // Pieces 0 .. pieces-1 of 8 weights from element `first` on, as bf16, to put(piece, value): kStageAhead loads of a thread in
 // flight (one at a time, staging was most of the 8 us that such a layer took on one image's rows).
 constexpr int kStageAhead = 4;
-template <typename PUT>
+template <int TH = kLinThreads, typename PUT>
 __device__ __forceinline__ void stage_rows(const void* w, int wbf16, int64_t first, int pieces, int tid, PUT&& put) {
   if (wbf16) {
     const uint16_t* src = static_cast<const uint16_t*>(w) + first;
-    for (int i0 = tid; i0 < pieces; i0 += kStageAhead * kLinThreads) {
+    for (int i0 = tid; i0 < pieces; i0 += kStageAhead * TH) {
       uint4 q[kStageAhead];
 #pragma unroll
       for (int k = 0; k < kStageAhead; ++k) {
-        const int i = i0 + k * kLinThreads;
+        const int i = i0 + k * TH;
         q[k] = ld16(src + (int64_t)8 * (i < pieces ? i : i0));
       }
 #pragma unroll
       for (int k = 0; k < kStageAhead; ++k)
-        if (i0 + k * kLinThreads < pieces) put(i0 + k * kLinThreads, q[k]);
+        if (i0 + k * TH < pieces) put(i0 + k * TH, q[k]);
     }
   } else {
     const float* src = static_cast<const float*>(w) + first;
-    for (int i0 = tid; i0 < pieces; i0 += kStageAhead * kLinThreads) {
+    for (int i0 = tid; i0 < pieces; i0 += kStageAhead * TH) {
       float4 lo[kStageAhead], hi[kStageAhead];
 #pragma unroll
       for (int k = 0; k < kStageAhead; ++k) {
-        const int i = i0 + k * kLinThreads;
+        const int i = i0 + k * TH;
         const float* p = src + (int64_t)8 * (i < pieces ? i : i0);
         lo[k] = *reinterpret_cast<const float4*>(p);
         hi[k] = *reinterpret_cast<const float4*>(p + 4);
       }
 #pragma unroll
       for (int k = 0; k < kStageAhead; ++k)
-        if (i0 + k * kLinThreads < pieces)
-          put(i0 + k * kLinThreads, make_uint4(pack_bf16(lo[k].x, lo[k].y), pack_bf16(lo[k].z, lo[k].w), pack_bf16(hi[k].x, hi[k].y), pack_bf16(hi[k].z, hi[k].w)));
+        if (i0 + k * TH < pieces)
+          put(i0 + k * TH, make_uint4(pack_bf16(lo[k].x, lo[k].y), pack_bf16(lo[k].z, lo[k].w), pack_bf16(hi[k].x, hi[k].y), pack_bf16(hi[k].z, hi[k].w)));
     }
   }
 }
@@ -924,9 +924,12 @@ struct MlpArgs {
 // RES: xo = x * res_s + MLP(x), y = LayerNorm(xo), the residual update and the next block's norm in the bits that m2d_layernorm_kernel gives behind
 // this one: after an exchange of halves a lane holds whole 8-channel pieces of its row (piece 4 no / 2 + {0, 2, 1, 3}[kb]), and the row's sums are
 // folded in that kernel's order: pieces 4, 2 and 1 apart.  The products and the GELU are what takes this kernel's time, so what
-// it moves beside them costs little: 128x56x56x64 128 us where the two kernels took 110 + 33.
-template <int KC, bool RES = false>
-__global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
+// it moves beside them costs little: 128x56x56x64 83 us where the two kernels took 110 + 33.
+// 32 hidden units at a time go from the first product into the second, one such step a turn of the loop: a wave then needs 113 registers where all 256
+// units of a row at once took 256, and four waves to a SIMD in place of two cover each other's waits for LDS, products and exponentials
+// (401408 rows of 64 channels, RES: 119 -> 83 us; two rows' tiles a wave on the same weights, with three waves a SIMD, 107).
+template <int KC, bool RES, int TH>
+__global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) {
   constexpr int C = 32 * KC, HD = 4 * C, NH = HD / 16, NO = C / 16, NP = NH / 2;
   constexpr int W1S = C + 8;      // bf16 per row of W1 in LDS (a row per hidden unit)
   constexpr int W2S = HD + 4;     // bf16 per row of W2 (a row per output): rows stay 8-byte aligned and spread over the banks
@@ -937,7 +940,7 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
   const int tid = threadIdx.x, l = tid & 63, mn = l & 15, kb = l >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto stage_weights = [&](const void* w, int rows, int cols, uint16_t* dst, int stride) {   // 8 elements at a time
-    stage_rows(w, a.wbf16, 0, rows * (cols / 8), tid, [&](int i, const uint4& q) {
+    stage_rows<TH>(w, a.wbf16, 0, rows * (cols / 8), tid, [&](int i, const uint4& q) {
       const int n = i / (cols / 8), k8 = i - n * (cols / 8);
       uint2* d = reinterpret_cast<uint2*>(dst + n * stride + 8 * k8);      // rows of W2 are 8-byte aligned only
       d[0] = make_uint2(q.x, q.y);
@@ -948,86 +951,81 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
   uint16_t* Y = static_cast<uint16_t*>(a.y);
   uint4 Xnext[KC];
   auto fetch = [&](int tile) {      // (rows past the end repeat the last one, see m2d_linear_kernel)
-    const int64_t q = (int64_t)tile * 64 + wave * 16 + mn;
+    const int64_t q = ((int64_t)tile * (TH / 64) + wave) * 16 + mn;
     const uint16_t* row = X + (q < a.P ? q : a.P - 1) * C + 8 * kb;
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) Xnext[kc] = ld16(row + 32 * kc);
   };
-  static_assert(HD <= kLinThreads, "one hidden unit's bias a thread");
+  static_assert(HD <= TH, "one hidden unit's bias a thread");
   fetch(blockIdx.x);
   const int th = tid < HD ? tid : HD - 1, tc = tid < C ? tid : C - 1;
   const float b10 = a.b1 ? ldw(a.b1, a.wbf16, th) : 0.f;
   const float lnw0 = a.ln_w ? ldw(a.ln_w, a.wbf16, tc) : 0.f, lnb0 = a.ln_w ? ldw(a.ln_b, a.wbf16, tc) : 0.f;
-  float b2v[NO][4];
-#pragma unroll
-  for (int no = 0; no < NO; ++no)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) b2v[no][i] = a.b2 ? ldw(a.b2, a.wbf16, 16 * no + 4 * kb + i) : 0.f;
+  const float b20 = a.b2 ? ldw(a.b2, a.wbf16, tc) : 0.f;
   stage_weights(a.w1, HD, C, w1l, W1S);
   stage_weights(a.w2, C, HD, w2l, W2S);
   if (tid < HD) b1l[tid] = b10;
   float* lnp = b1l + HD;
+  float* b2l = lnp + 2 * C;
+  if (tid < C) b2l[tid] = b20;
   if (a.ln_w && tid < C) { lnp[tid] = lnw0; lnp[C + tid] = lnb0; }
-  const float* nxp = lnp + 2 * C;      // RES: scale, weight, bias
+  const float* nxp = b2l + C;      // RES: scale, weight, bias
   if constexpr (RES) {
     if (tid < C) {
-      float* d = lnp + 2 * C + tid;
+      float* d = b2l + C + tid;
       d[0] = ldw(a.res_s, a.wbf16, tid); d[C] = ldw(a.nx_w, a.wbf16, tid); d[2 * C] = ldw(a.nx_b, a.wbf16, tid);
     }
   }
   __syncthreads();
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  const int piece = (kb & 1 ? 16 : 0) + 4 * (kb & 2);
   for (int tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
-    const int64_t p0 = (int64_t)tile * 64 + wave * 16;
+    const int64_t p = ((int64_t)tile * (TH / 64) + wave) * 16 + mn;      // the lane's row
     uint4 Xf[KC];
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) Xf[kc] = Xnext[kc];
-    uint4 xr[RES ? KC : 1];
-    const int piece = (kb & 1 ? 16 : 0) + 4 * (kb & 2);
-    if constexpr (RES) {               // the stream again, as the results will lie
-#pragma unroll
-      for (int c = 0; c < KC; ++c) xr[c] = ld16(X + (p0 + mn < a.P ? p0 + mn : a.P - 1) * C + 32 * c + piece);
-    }
     fetch(tile + gridDim.x);
     if (a.ln_w) norm_rows<KC>(Xf, KC, C, lnp, a.ln_eps, kb);      // (uniform)
-    f32x4_t h[NH];
+    f32x4_t out[NO];
 #pragma unroll
-    for (int nt = 0; nt < NH; ++nt) {
-      f32x4_t acc = zero;
+    for (int no = 0; no < NO; ++no) out[no] = zero;
+#pragma unroll 1
+    for (int ks = 0; ks < NP; ++ks) {
+      uint2 hq[2];      // the hidden activations as bf16, as fc2 of the stock path would read them
 #pragma unroll
-      for (int kc = 0; kc < KC; ++kc) acc = mfma_bf16(ld16(w1l + (16 * nt + mn) * W1S + 32 * kc + 8 * kb), Xf[kc], acc);
-      const float4 b1 = *reinterpret_cast<const float4*>(b1l + 16 * nt + 4 * kb);
-      h[nt][0] = gelu_exact(acc[0] + b1.x);
-      h[nt][1] = gelu_exact(acc[1] + b1.y);
-      h[nt][2] = gelu_exact(acc[2] + b1.z);
-      h[nt][3] = gelu_exact(acc[3] + b1.w);
+      for (int half = 0; half < 2; ++half) {
+        const uint16_t* w = w1l + (32 * ks + 16 * half + mn) * W1S + 8 * kb;
+        f32x4_t acc = zero;
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) acc = mfma_bf16(ld16(w + 32 * kc), Xf[kc], acc);
+        const float4 b1 = *reinterpret_cast<const float4*>(b1l + 32 * ks + 16 * half + 4 * kb);
+        hq[half] = make_uint2(pack_bf16(gelu_exact(acc[0] + b1.x), gelu_exact(acc[1] + b1.y)), pack_bf16(gelu_exact(acc[2] + b1.z), gelu_exact(acc[3] + b1.w)));
+      }
+#pragma unroll
+      for (int no = 0; no < NO; ++no) {
+        const uint16_t* w = w2l + (16 * no + mn) * W2S + 32 * ks + 4 * kb;      // output 16 no + mn, units 32 ks + 4 kb + {0..3, 16..19}
+        const uint2 lo = *reinterpret_cast<const uint2*>(w), hi = *reinterpret_cast<const uint2*>(w + 16);
+        out[no] = mfma_bf16(make_uint4(lo.x, lo.y, hi.x, hi.y), make_uint4(hq[0].x, hq[0].y, hq[1].x, hq[1].y), out[no]);
+      }
     }
-    uint4 hf[NP];      // the hidden activations as bf16, as fc2 of the stock path would read them
-#pragma unroll
-    for (int ks = 0; ks < NP; ++ks)
-      hf[ks] = make_uint4(pack_bf16(h[2 * ks][0], h[2 * ks][1]), pack_bf16(h[2 * ks][2], h[2 * ks][3]),
-                          pack_bf16(h[2 * ks + 1][0], h[2 * ks + 1][1]), pack_bf16(h[2 * ks + 1][2], h[2 * ks + 1][3]));
     uint2 yq[NO];
 #pragma unroll
     for (int no = 0; no < NO; ++no) {
-      f32x4_t acc = zero;
-#pragma unroll
-      for (int ks = 0; ks < NP; ++ks) {
-        const uint16_t* w = w2l + (16 * no + mn) * W2S + 32 * ks + 4 * kb;      // output 16 no + mn, units 32 ks + 4 kb + {0..3, 16..19}
-        const uint2 lo = *reinterpret_cast<const uint2*>(w), hi = *reinterpret_cast<const uint2*>(w + 16);
-        acc = mfma_bf16(make_uint4(lo.x, lo.y, hi.x, hi.y), hf[ks], acc);
-      }
-      yq[no] = make_uint2(pack_bf16(acc[0] + b2v[no][0], acc[1] + b2v[no][1]), pack_bf16(acc[2] + b2v[no][2], acc[3] + b2v[no][3]));
-      if constexpr (!RES) {
-        if (p0 + mn < a.P) *reinterpret_cast<uint2*>(Y + (p0 + mn) * C + 16 * no + 4 * kb) = yq[no];
-      }
+      const float4 b2 = *reinterpret_cast<const float4*>(b2l + 16 * no + 4 * kb);
+      yq[no] = make_uint2(pack_bf16(out[no][0] + b2.x, out[no][1] + b2.y), pack_bf16(out[no][2] + b2.z, out[no][3] + b2.w));
     }
-    if constexpr (RES) {
-      uint4 xo[KC];
+    if constexpr (!RES) {
+#pragma unroll
+      for (int no = 0; no < NO; ++no)
+        if (p < a.P) *reinterpret_cast<uint2*>(Y + p * C + 16 * no + 4 * kb) = yq[no];
+    } else {
+      uint4 xr[KC], xo[KC];             // the stream again, as the results lie
+#pragma unroll
+      for (int c = 0; c < KC; ++c) xr[c] = ld16(X + (p < a.P ? p : a.P - 1) * C + 32 * c + piece);
       float v[KC][8], part[KC];
       // the sum of a row's pieces: piece ^ 4 is the lane's own other one, ^ 2 and ^ 1 are in the lanes 16 and 32 further
-      auto row_sum = [&](const float (&t)[KC]) {
-        float s = KC == 2 ? t[0] + t[KC - 1] : t[0];
+      auto row_sum = [&](const float (&v)[KC]) {
+        float s = KC == 2 ? v[0] + v[KC - 1] : v[0];
         s += __shfl_xor(s, 16, 64);
         s += __shfl_xor(s, 32, 64);
         return s;
@@ -1062,8 +1060,8 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           o[j] = pack_bf16(__builtin_fmaf((v[c][2 * j] - mean) * rstd, w[2 * j], b[2 * j]), __builtin_fmaf((v[c][2 * j + 1] - mean) * rstd, w[2 * j + 1], b[2 * j + 1]));
-        if (p0 + mn < a.P) {
-          const int64_t at = (p0 + mn) * C + 32 * c + piece;
+        if (p < a.P) {
+          const int64_t at = p * C + 32 * c + piece;
           *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.xo) + at) = xo[c];
           *reinterpret_cast<uint4*>(Y + at) = make_uint4(o[0], o[1], o[2], o[3]);
         }
@@ -1073,9 +1071,15 @@ __global__ __launch_bounds__(kLinThreads) void m2d_mlp_kernel(const MlpArgs a) {
 }
 
 template <int KC>
-constexpr size_t mlp_lds_bytes() { return (size_t)(128 * KC) * (32 * KC + 8) * 2 + (size_t)(32 * KC) * (128 * KC + 4) * 2 + (size_t)(128 * KC) * 4 + (size_t)(64 * KC) * 4; }
+constexpr size_t mlp_lds_bytes() { return (size_t)(128 * KC) * (32 * KC + 8) * 2 + (size_t)(32 * KC) * (128 * KC + 4) * 2 + (size_t)(128 * KC) * 4 + (size_t)(96 * KC) * 4; }
 
 constexpr size_t kLinMaxLds = 160 * 1024;   // LDS of a compute unit
+
+constexpr int kMlpThreads = 512;      // of the kernel for many positions
+template <int KC, bool RES>
+const void* mlp_kernel(bool many) {
+  return many ? reinterpret_cast<const void*>(&m2d_mlp_kernel<KC, RES, kMlpThreads>) : reinterpret_cast<const void*>(&m2d_mlp_kernel<KC, RES, kLinThreads>);
+}
 
 // More than 64 KB of dynamic LDS has to be allowed per kernel and device, once.
 inline bool allow_big_lds() {
@@ -1086,8 +1090,8 @@ inline bool allow_big_lds() {
   if (seen.load(std::memory_order_acquire) & bit) return true;
   const void* kernels[] = {reinterpret_cast<const void*>(&m2d_linear_kernel<2>), reinterpret_cast<const void*>(&m2d_linear_kernel<4>),
                            reinterpret_cast<const void*>(&m2d_linear_kernel<8>), reinterpret_cast<const void*>(&m2d_linear_kernel<16>),
-                           reinterpret_cast<const void*>(&m2d_mlp_kernel<1>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2>),
-                           reinterpret_cast<const void*>(&m2d_mlp_kernel<1, true>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2, true>)};
+                           mlp_kernel<1, false>(false), mlp_kernel<1, false>(true), mlp_kernel<1, true>(false), mlp_kernel<1, true>(true),
+                           mlp_kernel<2, false>(false), mlp_kernel<2, false>(true), mlp_kernel<2, true>(false), mlp_kernel<2, true>(true)};
   for (const void* k : kernels)
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLinMaxLds) != hipSuccess) return false;
   seen.fetch_or(bit, std::memory_order_release);
@@ -1463,19 +1467,28 @@ static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x
   MlpArgs a = {};
   a.ln_w = ln_weight; a.ln_b = ln_bias; a.ln_eps = eps;
   a.x = x; a.w1 = w1; a.b1 = b1; a.w2 = w2; a.b2 = b2; a.y = y; a.P = P; a.wbf16 = weight_dtype == M2D_BF16;
-  a.ntiles = (int)((P + 63) / 64);
   if (res) { a.res_s = res->res_s; a.nx_w = res->nx_w; a.nx_b = res->nx_b; a.nx_eps = res->nx_eps; a.xo = res->xo; }
   const size_t lds = (C == 64 ? mlp_lds_bytes<2>() : mlp_lds_bytes<1>()) + (res ? (size_t)3 * C * 4 : 0);
   if (lds > 64 * 1024 && !allow_big_lds()) return M2D_ERR_HIP;
-  int per_cu = (int)(160 * 1024 / lds);      // persistent: the weights go to LDS once per workgroup
-  if (per_cu > 4) per_cu = 4;
+  // persistent: the weights go to LDS once per workgroup
+  const int fit = (int)(160 * 1024 / lds);
+  // Workgroups of 8 waves where they fill the device: twice the waves that share a copy of the weights (C = 64, RES: 50176 positions 17.0 us, 401408
+  // 82.8; of 6 waves 21.9 and 106); of 4 below, where more of them share out the rows.
+  const bool many = P > 256 * 128;
+  const int rows = many ? kMlpThreads / 4 : 64, per_cu = many ? (fit < 2 ? fit : 2) : (fit < 4 ? fit : 4);
+  a.ntiles = (int)((P + rows - 1) / rows);
   int grid = 256 * per_cu;
   if (grid > a.ntiles) grid = a.ntiles;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (res && C == 64) hipLaunchKernelGGL((m2d_mlp_kernel<2, true>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
-  else if (res) hipLaunchKernelGGL((m2d_mlp_kernel<1, true>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
-  else if (C == 64) hipLaunchKernelGGL(m2d_mlp_kernel<2>, dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
-  else hipLaunchKernelGGL(m2d_mlp_kernel<1>, dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
+  auto go = [&](auto kc, auto with) {
+    constexpr int KC = decltype(kc)::value;
+    constexpr bool RES = decltype(with)::value;
+    if (many) hipLaunchKernelGGL((m2d_mlp_kernel<KC, RES, kMlpThreads>), dim3((unsigned)grid), dim3(kMlpThreads), lds, st, a);
+    else hipLaunchKernelGGL((m2d_mlp_kernel<KC, RES, kLinThreads>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
+  };
+  auto with = [&](auto kc) { if (res) go(kc, std::true_type{}); else go(kc, std::false_type{}); };
+  if (C == 64) with(std::integral_constant<int, 2>{});
+  else with(std::integral_constant<int, 1>{});
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
 }
 
