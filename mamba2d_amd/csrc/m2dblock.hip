@@ -484,8 +484,10 @@ __device__ __forceinline__ void norm_rows(uint4 (&A)[KCMAX], int KC, int K, cons
 // Pieces 0 .. pieces-1 of 8 weights from element `first` on, as bf16, to put(piece, value): kStageAhead loads of a thread in
 // flight (one at a time, staging was most of the 8 us that such a layer took on one image's rows).
 constexpr int kStageAhead = 4;
-template <int TH = kLinThreads, typename PUT>
+// COLS of a row's STRIDE elements are taken (0: the pieces follow each other).
+template <int TH = kLinThreads, int COLS = 0, int STRIDE = 0, typename PUT>
 __device__ __forceinline__ void stage_rows(const void* w, int wbf16, int64_t first, int pieces, int tid, PUT&& put) {
+  auto element = [](int i) { return COLS ? (int64_t)(i / (COLS / 8 + !COLS)) * STRIDE + 8 * (i % (COLS / 8 + !COLS)) : (int64_t)8 * i; };
   if (wbf16) {
     const uint16_t* src = static_cast<const uint16_t*>(w) + first;
     for (int i0 = tid; i0 < pieces; i0 += kStageAhead * TH) {
@@ -493,7 +495,7 @@ __device__ __forceinline__ void stage_rows(const void* w, int wbf16, int64_t fir
 #pragma unroll
       for (int k = 0; k < kStageAhead; ++k) {
         const int i = i0 + k * TH;
-        q[k] = ld16(src + (int64_t)8 * (i < pieces ? i : i0));
+        q[k] = ld16(src + element(i < pieces ? i : i0));
       }
 #pragma unroll
       for (int k = 0; k < kStageAhead; ++k)
@@ -506,7 +508,7 @@ __device__ __forceinline__ void stage_rows(const void* w, int wbf16, int64_t fir
 #pragma unroll
       for (int k = 0; k < kStageAhead; ++k) {
         const int i = i0 + k * TH;
-        const float* p = src + (int64_t)8 * (i < pieces ? i : i0);
+        const float* p = src + element(i < pieces ? i : i0);
         lo[k] = *reinterpret_cast<const float4*>(p);
         hi[k] = *reinterpret_cast<const float4*>(p + 4);
       }
@@ -922,30 +924,37 @@ struct MlpArgs {
 
 // KC: C = 32 KC channels, 128 KC hidden units.
 // RES: xo = x * res_s + MLP(x), y = LayerNorm(xo), the residual update and the next block's norm in the bits that m2d_layernorm_kernel gives behind
-// this one: after an exchange of halves a lane holds whole 8-channel pieces of its row (piece 4 no / 2 + {0, 2, 1, 3}[kb]), and the row's sums are
-// folded in that kernel's order: pieces 4, 2 and 1 apart.  The products and the GELU are what takes this kernel's time, so what
+// this one: after an exchange of halves a lane holds whole 8-channel pieces of its row (piece 4 c + {0, 2, 1, 3}[kb]), and the row's sums are
+// folded in that kernel's order: pieces 8, 4, 2 and 1 apart.  The products and the GELU are what takes this kernel's time, so what
 // it moves beside them costs little: 128x56x56x64 83 us where the two kernels took 110 + 33.
 // 32 hidden units at a time go from the first product into the second, one such step a turn of the loop: a wave then needs 113 registers where all 256
 // units of a row at once took 256, and four waves to a SIMD in place of two cover each other's waits for LDS, products and exponentials
 // (401408 rows of 64 channels, RES: 119 -> 83 us; two rows' tiles a wave on the same weights, with three waves a SIMD, 107).
+// 128 channels: a quarter of the hidden units has its weights in LDS at a time, fetched for every tile of 128 rows; of the two workgroups of a unit
+// one computes while the other fetches.  100352 rows 78 us, where layer, library product and update with norm took 110 (hidden activations of 103 MB out
+// and back); 50176 40 and 62.
+constexpr int mlp_slices(int kc) { return kc <= 2 ? 1 : 4; }
 template <int KC, bool RES, int TH>
 __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) {
-  constexpr int C = 32 * KC, HD = 4 * C, NH = HD / 16, NO = C / 16, NP = NH / 2;
+  constexpr int C = 32 * KC, HD = 4 * C, SL = mlp_slices(KC), HS = HD / SL, NO = C / 16, NP = HS / 32;
   constexpr int W1S = C + 8;      // bf16 per row of W1 in LDS (a row per hidden unit)
-  constexpr int W2S = HD + 4;     // bf16 per row of W2 (a row per output): rows stay 8-byte aligned and spread over the banks
+  constexpr int W2S = HS + 4;     // bf16 per row of W2 (a row per output): rows stay 8-byte aligned and spread over the banks
   extern __shared__ float smem[];
   uint16_t* w1l = reinterpret_cast<uint16_t*>(smem);
-  uint16_t* w2l = w1l + HD * W1S;
+  uint16_t* w2l = w1l + HS * W1S;
   float* b1l = reinterpret_cast<float*>(w2l + C * W2S);
   const int tid = threadIdx.x, l = tid & 63, mn = l & 15, kb = l >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  auto stage_weights = [&](const void* w, int rows, int cols, uint16_t* dst, int stride) {   // 8 elements at a time
-    stage_rows<TH>(w, a.wbf16, 0, rows * (cols / 8), tid, [&](int i, const uint4& q) {
-      const int n = i / (cols / 8), k8 = i - n * (cols / 8);
-      uint2* d = reinterpret_cast<uint2*>(dst + n * stride + 8 * k8);      // rows of W2 are 8-byte aligned only
-      d[0] = make_uint2(q.x, q.y);
-      d[1] = make_uint2(q.z, q.w);
-    });
+  auto put = [&](uint16_t* row, int k8, const uint4& q) {
+    uint2* d = reinterpret_cast<uint2*>(row + 8 * k8);      // rows of W2 are 8-byte aligned only
+    d[0] = make_uint2(q.x, q.y);
+    d[1] = make_uint2(q.z, q.w);
+  };
+  auto stage_weights = [&](int slice) {                       // hidden units slice * HS ..., 8 elements at a time
+    int tid = threadIdx.x;
+    if constexpr (SL > 1) asm volatile("" : "+v"(tid));      // (addresses are worked out here: held across the products they cost 40 registers)
+    stage_rows<TH>(a.w1, a.wbf16, (int64_t)slice * HS * C, HS * (C / 8), tid, [&](int i, const uint4& q) { put(w1l + i / (C / 8) * W1S, i % (C / 8), q); });
+    stage_rows<TH, HS, HD>(a.w2, a.wbf16, slice * HS, C * (HS / 8), tid, [&](int i, const uint4& q) { put(w2l + i / (HS / 8) * W2S, i % (HS / 8), q); });
   };
   const uint16_t* X = static_cast<const uint16_t*>(a.x);
   uint16_t* Y = static_cast<uint16_t*>(a.y);
@@ -956,14 +965,13 @@ __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) 
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) Xnext[kc] = ld16(row + 32 * kc);
   };
-  static_assert(HD <= TH, "one hidden unit's bias a thread");
-  fetch(blockIdx.x);
+  static_assert(HD <= TH && C <= TH, "one hidden unit's bias a thread");
+  if constexpr (SL == 1) fetch(blockIdx.x);
   const int th = tid < HD ? tid : HD - 1, tc = tid < C ? tid : C - 1;
   const float b10 = a.b1 ? ldw(a.b1, a.wbf16, th) : 0.f;
   const float lnw0 = a.ln_w ? ldw(a.ln_w, a.wbf16, tc) : 0.f, lnb0 = a.ln_w ? ldw(a.ln_b, a.wbf16, tc) : 0.f;
   const float b20 = a.b2 ? ldw(a.b2, a.wbf16, tc) : 0.f;
-  stage_weights(a.w1, HD, C, w1l, W1S);
-  stage_weights(a.w2, C, HD, w2l, W2S);
+  if constexpr (SL == 1) stage_weights(0);
   if (tid < HD) b1l[tid] = b10;
   float* lnp = b1l + HD;
   float* b2l = lnp + 2 * C;
@@ -982,30 +990,45 @@ __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) 
   for (int tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
     const int64_t p = ((int64_t)tile * (TH / 64) + wave) * 16 + mn;      // the lane's row
     uint4 Xf[KC];
+    if constexpr (SL > 1) {      // (the weights are waited for at every tile anyhow)
+      fetch(tile);
+      __syncthreads();
+      stage_weights(0);
+    }
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) Xf[kc] = Xnext[kc];
-    fetch(tile + gridDim.x);
+    if constexpr (SL == 1) fetch(tile + gridDim.x);
     if (a.ln_w) norm_rows<KC>(Xf, KC, C, lnp, a.ln_eps, kb);      // (uniform)
     f32x4_t out[NO];
 #pragma unroll
     for (int no = 0; no < NO; ++no) out[no] = zero;
 #pragma unroll 1
-    for (int ks = 0; ks < NP; ++ks) {
-      uint2 hq[2];      // the hidden activations as bf16, as fc2 of the stock path would read them
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const uint16_t* w = w1l + (32 * ks + 16 * half + mn) * W1S + 8 * kb;
-        f32x4_t acc = zero;
-#pragma unroll
-        for (int kc = 0; kc < KC; ++kc) acc = mfma_bf16(ld16(w + 32 * kc), Xf[kc], acc);
-        const float4 b1 = *reinterpret_cast<const float4*>(b1l + 32 * ks + 16 * half + 4 * kb);
-        hq[half] = make_uint2(pack_bf16(gelu_exact(acc[0] + b1.x), gelu_exact(acc[1] + b1.y)), pack_bf16(gelu_exact(acc[2] + b1.z), gelu_exact(acc[3] + b1.w)));
+    for (int slice = 0; slice < SL; ++slice) {
+      if constexpr (SL > 1) {      // (a workgroup's waves have the same tiles)
+        if (slice) {
+          __syncthreads();
+          stage_weights(slice);
+        }
+        __syncthreads();
       }
+#pragma unroll 1
+      for (int ks = 0; ks < NP; ++ks) {
+        uint2 hq[2];      // the hidden activations as bf16, as fc2 of the stock path would read them
 #pragma unroll
-      for (int no = 0; no < NO; ++no) {
-        const uint16_t* w = w2l + (16 * no + mn) * W2S + 32 * ks + 4 * kb;      // output 16 no + mn, units 32 ks + 4 kb + {0..3, 16..19}
-        const uint2 lo = *reinterpret_cast<const uint2*>(w), hi = *reinterpret_cast<const uint2*>(w + 16);
-        out[no] = mfma_bf16(make_uint4(lo.x, lo.y, hi.x, hi.y), make_uint4(hq[0].x, hq[0].y, hq[1].x, hq[1].y), out[no]);
+        for (int half = 0; half < 2; ++half) {
+          const uint16_t* w = w1l + (32 * ks + 16 * half + mn) * W1S + 8 * kb;
+          f32x4_t acc = zero;
+#pragma unroll
+          for (int kc = 0; kc < KC; ++kc) acc = mfma_bf16(ld16(w + 32 * kc), Xf[kc], acc);
+          const float4 b1 = *reinterpret_cast<const float4*>(b1l + slice * HS + 32 * ks + 16 * half + 4 * kb);
+          hq[half] = make_uint2(pack_bf16(gelu_exact(acc[0] + b1.x), gelu_exact(acc[1] + b1.y)), pack_bf16(gelu_exact(acc[2] + b1.z), gelu_exact(acc[3] + b1.w)));
+        }
+#pragma unroll
+        for (int no = 0; no < NO; ++no) {
+          const uint16_t* w = w2l + (16 * no + mn) * W2S + 32 * ks + 4 * kb;      // output 16 no + mn, units 32 ks + 4 kb + {0..3, 16..19}
+          const uint2 lo = *reinterpret_cast<const uint2*>(w), hi = *reinterpret_cast<const uint2*>(w + 16);
+          out[no] = mfma_bf16(make_uint4(lo.x, lo.y, hi.x, hi.y), make_uint4(hq[0].x, hq[0].y, hq[1].x, hq[1].y), out[no]);
+        }
       }
     }
     uint2 yq[NO];
@@ -1022,10 +1045,10 @@ __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) 
       uint4 xr[KC], xo[KC];             // the stream again, as the results lie
 #pragma unroll
       for (int c = 0; c < KC; ++c) xr[c] = ld16(X + (p < a.P ? p : a.P - 1) * C + 32 * c + piece);
-      float v[KC][8], part[KC];
-      // the sum of a row's pieces: piece ^ 4 is the lane's own other one, ^ 2 and ^ 1 are in the lanes 16 and 32 further
+      float part[KC];
+      // the sum of a row's pieces: piece ^ 8 and ^ 4 are the lane's own, ^ 2 and ^ 1 are in the lanes 16 and 32 further
       auto row_sum = [&](const float (&v)[KC]) {
-        float s = KC == 2 ? v[0] + v[KC - 1] : v[0];
+        float s = KC == 4 ? (v[0] + v[KC / 2]) + (v[KC / 4] + v[KC - 1]) : KC == 2 ? v[0] + v[KC - 1] : v[0];
         s += __shfl_xor(s, 16, 64);
         s += __shfl_xor(s, 32, 64);
         return s;
@@ -1040,26 +1063,27 @@ __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) 
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           o[j] = pack_bf16(__builtin_fmaf(bf_lo(xw[j]), sc[2 * j], bf_lo(mw[j])), __builtin_fmaf(bf_hi(xw[j]), sc[2 * j + 1], bf_hi(mw[j])));
-          v[c][2 * j] = bf_lo(o[j]); v[c][2 * j + 1] = bf_hi(o[j]);      // (the norm sees what is stored)
-          part[c] += v[c][2 * j]; part[c] += v[c][2 * j + 1];
+          part[c] += bf_lo(o[j]); part[c] += bf_hi(o[j]);      // (the norm sees what is stored)
         }
         xo[c] = make_uint4(o[0], o[1], o[2], o[3]);
       }
       const float mean = row_sum(part) * (1.f / C);
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
+        const uint32_t xw[4] = {xo[c].x, xo[c].y, xo[c].z, xo[c].w};
         part[c] = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) { const float d = v[c][j] - mean; part[c] = __builtin_fmaf(d, d, part[c]); }
+        for (int j = 0; j < 8; ++j) { const float d = (j & 1 ? bf_hi(xw[j / 2]) : bf_lo(xw[j / 2])) - mean; part[c] = __builtin_fmaf(d, d, part[c]); }
       }
       const float rstd = rsqrtf(row_sum(part) * (1.f / C) + a.nx_eps);
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
         const float *w = nxp + C + 32 * c + piece, *b = w + C;
+        const uint32_t xw[4] = {xo[c].x, xo[c].y, xo[c].z, xo[c].w};
         uint32_t o[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          o[j] = pack_bf16(__builtin_fmaf((v[c][2 * j] - mean) * rstd, w[2 * j], b[2 * j]), __builtin_fmaf((v[c][2 * j + 1] - mean) * rstd, w[2 * j + 1], b[2 * j + 1]));
+          o[j] = pack_bf16(__builtin_fmaf((bf_lo(xw[j]) - mean) * rstd, w[2 * j], b[2 * j]), __builtin_fmaf((bf_hi(xw[j]) - mean) * rstd, w[2 * j + 1], b[2 * j + 1]));
         if (p < a.P) {
           const int64_t at = p * C + 32 * c + piece;
           *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.xo) + at) = xo[c];
@@ -1071,7 +1095,10 @@ __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) 
 }
 
 template <int KC>
-constexpr size_t mlp_lds_bytes() { return (size_t)(128 * KC) * (32 * KC + 8) * 2 + (size_t)(32 * KC) * (128 * KC + 4) * 2 + (size_t)(128 * KC) * 4 + (size_t)(96 * KC) * 4; }
+constexpr size_t mlp_lds_bytes() {
+  constexpr size_t C = 32 * KC, HS = 4 * C / mlp_slices(KC);
+  return HS * (C + 8) * 2 + C * (HS + 4) * 2 + 4 * C * 4 + 3 * C * 4;
+}
 
 constexpr size_t kLinMaxLds = 160 * 1024;   // LDS of a compute unit
 
@@ -1091,7 +1118,8 @@ inline bool allow_big_lds() {
   const void* kernels[] = {reinterpret_cast<const void*>(&m2d_linear_kernel<2>), reinterpret_cast<const void*>(&m2d_linear_kernel<4>),
                            reinterpret_cast<const void*>(&m2d_linear_kernel<8>), reinterpret_cast<const void*>(&m2d_linear_kernel<16>),
                            mlp_kernel<1, false>(false), mlp_kernel<1, false>(true), mlp_kernel<1, true>(false), mlp_kernel<1, true>(true),
-                           mlp_kernel<2, false>(false), mlp_kernel<2, false>(true), mlp_kernel<2, true>(false), mlp_kernel<2, true>(true)};
+                           mlp_kernel<2, false>(false), mlp_kernel<2, false>(true), mlp_kernel<2, true>(false), mlp_kernel<2, true>(true),
+                           reinterpret_cast<const void*>(&m2d_mlp_kernel<4, true, kMlpThreads>)};
   for (const void* k : kernels)
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLinMaxLds) != hipSuccess) return false;
   seen.fetch_or(bit, std::memory_order_release);
@@ -1459,7 +1487,7 @@ static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x
   if (!x || !w1 || !w2 || !y || (ln_weight != nullptr) != (ln_bias != nullptr)) return M2D_ERR_NULL_POINTER;
   if (P < 1 || C < 1 || hidden < 1) return M2D_ERR_BAD_SHAPE;
   if (weight_dtype != M2D_F32 && weight_dtype != M2D_BF16) return M2D_ERR_UNSUPPORTED;
-  if ((C != 32 && C != 64) || hidden != 4 * C) return M2D_ERR_UNSUPPORTED;
+  if ((C != 32 && C != 64 && !(res && C == 128)) || hidden != 4 * C) return M2D_ERR_UNSUPPORTED;
   if ((P + 63) / 64 >= ((int64_t)1 << 31)) return M2D_ERR_UNSUPPORTED;
   if (misaligned(x, 16) || misaligned(y, 16) || misaligned(w1, 16) || misaligned(w2, 16) || (b1 && misaligned(b1, 4)) || (b2 && misaligned(b2, 4)) ||
       (ln_weight && (misaligned(ln_weight, 4) || misaligned(ln_bias, 4))))
@@ -1468,13 +1496,13 @@ static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x
   a.ln_w = ln_weight; a.ln_b = ln_bias; a.ln_eps = eps;
   a.x = x; a.w1 = w1; a.b1 = b1; a.w2 = w2; a.b2 = b2; a.y = y; a.P = P; a.wbf16 = weight_dtype == M2D_BF16;
   if (res) { a.res_s = res->res_s; a.nx_w = res->nx_w; a.nx_b = res->nx_b; a.nx_eps = res->nx_eps; a.xo = res->xo; }
-  const size_t lds = (C == 64 ? mlp_lds_bytes<2>() : mlp_lds_bytes<1>()) + (res ? (size_t)3 * C * 4 : 0);
+  const size_t lds = (C == 128 ? mlp_lds_bytes<4>() : C == 64 ? mlp_lds_bytes<2>() : mlp_lds_bytes<1>()) + (res ? (size_t)3 * C * 4 : 0);
   if (lds > 64 * 1024 && !allow_big_lds()) return M2D_ERR_HIP;
   // persistent: the weights go to LDS once per workgroup
   const int fit = (int)(160 * 1024 / lds);
   // Workgroups of 8 waves where they fill the device: twice the waves that share a copy of the weights (C = 64, RES: 50176 positions 17.0 us, 401408
   // 82.8; of 6 waves 21.9 and 106); of 4 below, where more of them share out the rows.
-  const bool many = P > 256 * 128;
+  const bool many = P > 256 * 128 || C == 128;
   const int rows = many ? kMlpThreads / 4 : 64, per_cu = many ? (fit < 2 ? fit : 2) : (fit < 4 ? fit : 4);
   a.ntiles = (int)((P + rows - 1) / rows);
   int grid = 256 * per_cu;
@@ -1487,7 +1515,8 @@ static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x
     else hipLaunchKernelGGL((m2d_mlp_kernel<KC, RES, kLinThreads>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
   };
   auto with = [&](auto kc) { if (res) go(kc, std::true_type{}); else go(kc, std::false_type{}); };
-  if (C == 64) with(std::integral_constant<int, 2>{});
+  if (C == 128) hipLaunchKernelGGL((m2d_mlp_kernel<4, true, kMlpThreads>), dim3((unsigned)grid), dim3(kMlpThreads), lds, st, a);
+  else if (C == 64) with(std::integral_constant<int, 2>{});
   else with(std::integral_constant<int, 1>{});
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
 }

@@ -61,6 +61,36 @@ def test_mlp_residual_norm_gives_the_bits_of_two_kernels(P, C, wdtype):
             assert torch.equal(got[:P].isnan(), two.isnan()) and torch.equal(got[:P].nan_to_num(), two.nan_to_num())
 
 
+@on_gpu
+@WTYPES
+@pytest.mark.parametrize("P", [1, 16, 127, 129, 1000, 66001])
+def test_mlp_of_128_channels(P, wdtype):
+    """Weights in slices, tiles of 128 rows: the updated stream against fp64 sums of the hidden activations that the layer's own kernel gives, its norm in
+    the bits of the norm's kernel."""
+    from mamba2d_amd import cabi
+    C, H = 128, 512
+    print(f"\ncase mlp residual {P}x{C} {wdtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(P)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = (3 * r(P, C)).bfloat16()
+    w1, w2 = (r(H, C) / C ** 0.5).to(wdtype), (r(C, H) / H ** 0.5).to(wdtype)
+    b1, b2, lw, lb, s, nw, nb = (r(n).to(wdtype) for n in (H, C, C, C, C, C, C))
+    h = cabi.linear_fwd(x, w1, b1, post=cabi.ACT_GELU, ln=(lw, lb, 1e-5)).double()
+    wb = w2.bfloat16().double()
+    branch = h @ wb.t() + b2.double()
+    slack = (H + 2) * 2.0 ** -24 * (h.abs() @ wb.abs().t() + b2.double().abs())      # fp32 sums of H products in any order, and the bias
+    want = x.double() * s.double() + branch
+    xo, y = (torch.full((P + 1, C), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    cabi.check(cabi.lib.m2d_mlp_residual_layernorm_fwd(P, C, H, cabi._dtype_code(w1), cabi._ptr(x), cabi._ptr(lw), cabi._ptr(lb), 1e-5, cabi._ptr(w1),
+                                                       cabi._ptr(b1), cabi._ptr(w2), cabi._ptr(b2), cabi._ptr(s), cabi._ptr(nw), cabi._ptr(nb), 1e-3,
+                                                       cabi._ptr(xo), cabi._ptr(y), cabi._stream(x.device)))
+    assert (xo[P] == 7).all() and (y[P] == 7).all()
+    # two roundings to bf16, each by half a unit in the last of 8 bits (2**-8 of the value): of the MLP's result and of the updated stream
+    assert ((xo[:P].double() - want).abs() <= 1.02 * 2.0 ** -8 * (branch.abs() + want.abs()) + 2 * slack).all()
+    same = cabi.scale_residual_layernorm_fwd(xo[:P].contiguous(), torch.ones_like(s), torch.zeros_like(x), None, nw, nb, 1e-3)
+    assert torch.equal(same[0], xo[:P]) and torch.equal(same[1], y[:P])
+
+
 def test_refusals():
     """Host checks only: nothing is launched."""
     from mamba2d_amd import cabi
@@ -74,5 +104,5 @@ def test_refusals():
     assert linear(P=0) == shape
     mlp = lambda C=64, s=p, nw=p, xo=p, y=p: cabi.lib.m2d_mlp_residual_layernorm_fwd(4, C, 4 * C, 1, p, None, None, 0.0, p, p, p, p, s, nw, p, 0.0, xo, y, None)
     assert [mlp(s=None), mlp(nw=None), mlp(xo=None), mlp(y=None)] == [null] * 4
-    assert [mlp(C=128), mlp(C=48)] == [unsupported] * 2
+    assert [mlp(C=256), mlp(C=48)] == [unsupported] * 2
     assert [mlp(xo=p + 8), mlp(s=p + 2), mlp(y=p + 4)] == [misaligned] * 3
