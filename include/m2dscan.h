@@ -404,6 +404,10 @@ int m2d_mlp_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x,
                 const void* ln_weight, const void* ln_bias, float eps,
                 const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream);
 
+/* m2d_mlp_fwd (no norm) that also keeps the first layer's output: z (P, hidden) bf16, y = fc2(GELU(z)). */
+int m2d_mlp_keep_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* w1, const void* b1, const void* w2, const void* b2,
+                     void* z, void* y, void* stream);
+
 /* m2d_mlp_fwd with the block's residual update and the norm behind it in the same pass: x_out = x * scale + MLP(x) and
  * y = LayerNorm(x_out; next_weight, next_bias, next_eps), in the bits of m2d_mlp_fwd followed by m2d_scale_residual_layernorm_fwd.  x_out and y
  * are (P, C) bf16 and none of the others; scale, next_weight and next_bias (C) have weight_dtype.  C = 128 with hidden = 512 is taken here too: then

@@ -29,7 +29,7 @@ M2D_PASS_FWD, M2D_PASS_BWD = 0, 1
 EXPORTS = ("m2d_version", "m2d_status_str", "m2d_desc_check", "m2d_scan_workspace_bytes",
            "m2d_scan_ckpt_bytes", "m2d_scan_fwd", "m2d_scan_fwd_noalloc", "m2d_scan_link_error", "m2d_scan_plan", "m2d_scan_bwd", "m2d_proj_workspace_bytes", "m2d_proj_fwd",
            "m2d_proj_bwd", "m2d_proj_bwd_parts", "m2d_scan_sum_parts", "m2d_layernorm_fwd", "m2d_dwconv3x3_fwd", "m2d_starrelu_fwd",
-           "m2d_scale_residual_fwd", "m2d_scale_residual_layernorm_fwd", "m2d_rope_qknorm_fwd", "m2d_rope_attention_fwd", "m2d_mlp_fwd", "m2d_layernorm_linear_fwd", "m2d_linear_fwd", "m2d_linear_residual_fwd", "m2d_mlp_residual_layernorm_fwd", "m2d_profile_enable", "m2d_profile_last_ms", "m2d_valu_rate_probe", "m2d_wf_fwd", "m2d_wf_bwd",
+           "m2d_scale_residual_fwd", "m2d_scale_residual_layernorm_fwd", "m2d_rope_qknorm_fwd", "m2d_rope_attention_fwd", "m2d_mlp_fwd", "m2d_layernorm_linear_fwd", "m2d_linear_fwd", "m2d_linear_residual_fwd", "m2d_mlp_residual_layernorm_fwd", "m2d_mlp_keep_fwd", "m2d_profile_enable", "m2d_profile_last_ms", "m2d_valu_rate_probe", "m2d_wf_fwd", "m2d_wf_bwd",
            "m2d_widen", "m2d_wide_linear_fwd", "m2d_linear_keep_fwd", "m2d_starrelu_dwconv3x3_fwd", "m2d_train_norm_fwd", "m2d_train_norm_parts", "m2d_train_norm_bwd",
            "m2d_train_branch", "m2d_train_dwconv_parts", "m2d_train_dwconv_bwd", "m2d_train_linear_parts", "m2d_train_linear_bwd",
            "m2d_train_wgrad_parts", "m2d_train_wgrad", "m2d_train_linear_grads_parts", "m2d_train_linear_grads", "m2d_train_reduce")
@@ -110,6 +110,8 @@ def _load():
     lib.m2d_rope_qknorm_fwd.argtypes = [i32] * 6 + [vp] * 7 + [ctypes.c_float, i32, vp, vp, vp]
     lib.m2d_linear_residual_fwd.restype = i32
     lib.m2d_linear_residual_fwd.argtypes = [ctypes.c_int64, i32, i32, i32, vp, vp, vp, i32, vp, vp, vp, vp, vp]
+    lib.m2d_mlp_keep_fwd.restype = i32
+    lib.m2d_mlp_keep_fwd.argtypes = [ctypes.c_int64, i32, i32, i32] + [vp] * 8
     lib.m2d_mlp_residual_layernorm_fwd.restype = i32
     lib.m2d_mlp_residual_layernorm_fwd.argtypes = [ctypes.c_int64, i32, i32, i32, vp, vp, vp, ctypes.c_float] + [vp] * 7 + [ctypes.c_float, vp, vp, vp]
     lib.m2d_linear_fwd.restype = i32

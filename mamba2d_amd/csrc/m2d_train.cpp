@@ -139,10 +139,15 @@ struct Block : public torch::autograd::Function<Block> {
     check(m2d_train_norm_fwd(s.P, C, rps, f32(x), f32(p[kRs1]), mix.data_ptr(), s.local ? loc.data_ptr() : nullptr, opt(keep1),
                              x1.data_ptr<float>(), f32(p[kN2W]), f32(p[kN2B]), (float)eps2, n2.data_ptr(), nullptr, nullptr, 0.f, nullptr, st));
     Tensor h0 = bf16_like(x, HD), m = mix;      // (the mixer's answer has been added: its buffer takes the MLP's)
-    check(m2d_linear_fwd(s.P, C, HD, M2D_F32, n2.data_ptr(), f32(p[kFc1W]), f32(p[kFc1B]), M2D_ACT_NONE, nullptr, nullptr, M2D_ACT_NONE,
-                         nullptr, nullptr, h0.data_ptr(), st));
-    check(m2d_linear_fwd(s.P, HD, C, M2D_F32, h0.data_ptr(), f32(p[kFc2W]), f32(p[kFc2B]), M2D_ACT_GELU, nullptr, nullptr, M2D_ACT_NONE,
-                         nullptr, nullptr, m.data_ptr(), st));
+    if (C == 32 || C == 64) {      // both layers in one kernel
+      check(m2d_mlp_keep_fwd(s.P, C, HD, M2D_F32, n2.data_ptr(), f32(p[kFc1W]), f32(p[kFc1B]), f32(p[kFc2W]), f32(p[kFc2B]), h0.data_ptr(),
+                             m.data_ptr(), st));
+    } else {
+      check(m2d_linear_fwd(s.P, C, HD, M2D_F32, n2.data_ptr(), f32(p[kFc1W]), f32(p[kFc1B]), M2D_ACT_NONE, nullptr, nullptr, M2D_ACT_NONE,
+                           nullptr, nullptr, h0.data_ptr(), st));
+      check(m2d_linear_fwd(s.P, HD, C, M2D_F32, h0.data_ptr(), f32(p[kFc2W]), f32(p[kFc2B]), M2D_ACT_GELU, nullptr, nullptr, M2D_ACT_NONE,
+                           nullptr, nullptr, m.data_ptr(), st));
+    }
     Tensor x2 = at::empty_like(x);
     check(m2d_train_norm_fwd(s.P, C, rps, f32(x1), f32(p[kRs2]), m.data_ptr(), nullptr, opt(keep2), x2.data_ptr<float>(), nullptr, nullptr, 0.f,
                              nullptr, nullptr, nullptr, 0.f, nullptr, st));

@@ -920,6 +920,7 @@ struct MlpArgs {
   const void *res_s, *nx_w, *nx_b;   // RES: scale of the residual stream, weight and bias of the norm behind the update, (C)
   float nx_eps;
   void* xo;               // RES: (P, C) the updated stream; y is its norm
+  void* z;                // KEEP: (P, 4 C) bf16, the first layer's output before the GELU
 };
 
 // KC: C = 32 KC channels, 128 KC hidden units.
@@ -934,7 +935,9 @@ struct MlpArgs {
 // one computes while the other fetches.  100352 rows 78 us, where layer, library product and update with norm took 110 (hidden activations of 103 MB out
 // and back); 50176 40 and 62.
 constexpr int mlp_slices(int kc) { return kc <= 2 ? 1 : 4; }
-template <int KC, bool RES, int TH>
+// KEEP: fc1's output leaves too, and the GELU reads what is stored, as the backward will: without reading it back the two layers of
+// a training forward take 48 us for 200704 rows of 64 channels where two kernels took 76 (12544: 9.7 and 18).
+template <int KC, bool RES, int TH, bool KEEP = false>
 __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) {
   constexpr int C = 32 * KC, HD = 4 * C, SL = mlp_slices(KC), HS = HD / SL, NO = C / 16, NP = HS / 32;
   constexpr int W1S = C + 8;      // bf16 per row of W1 in LDS (a row per hidden unit)
@@ -1013,7 +1016,7 @@ __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) 
       }
 #pragma unroll 1
       for (int ks = 0; ks < NP; ++ks) {
-        uint2 hq[2];      // the hidden activations as bf16, as fc2 of the stock path would read them
+        uint2 hq[2], zq[2];      // the hidden activations as bf16, as fc2 of the stock path would read them
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
           const uint16_t* w = w1l + (32 * ks + 16 * half + mn) * W1S + 8 * kb;
@@ -1021,7 +1024,16 @@ __global__ __launch_bounds__(TH, TH / 128) void m2d_mlp_kernel(const MlpArgs a) 
 #pragma unroll
           for (int kc = 0; kc < KC; ++kc) acc = mfma_bf16(ld16(w + 32 * kc), Xf[kc], acc);
           const float4 b1 = *reinterpret_cast<const float4*>(b1l + slice * HS + 32 * ks + 16 * half + 4 * kb);
-          hq[half] = make_uint2(pack_bf16(gelu_exact(acc[0] + b1.x), gelu_exact(acc[1] + b1.y)), pack_bf16(gelu_exact(acc[2] + b1.z), gelu_exact(acc[3] + b1.w)));
+          acc[0] += b1.x; acc[1] += b1.y; acc[2] += b1.z; acc[3] += b1.w;
+          if constexpr (KEEP) {
+            zq[half] = make_uint2(pack_bf16(acc[0], acc[1]), pack_bf16(acc[2], acc[3]));
+            acc[0] = bf_lo(zq[half].x); acc[1] = bf_hi(zq[half].x); acc[2] = bf_lo(zq[half].y); acc[3] = bf_hi(zq[half].y);
+          }
+          hq[half] = make_uint2(pack_bf16(gelu_exact(acc[0]), gelu_exact(acc[1])), pack_bf16(gelu_exact(acc[2]), gelu_exact(acc[3])));
+        }
+        if constexpr (KEEP) {
+          const uint4 q = halves_exchanged(zq[0], zq[1]);
+          if (p < a.P) *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.z) + p * HD + slice * HS + 32 * ks + piece) = q;
         }
 #pragma unroll
         for (int no = 0; no < NO; ++no) {
@@ -1119,7 +1131,8 @@ inline bool allow_big_lds() {
                            reinterpret_cast<const void*>(&m2d_linear_kernel<8>), reinterpret_cast<const void*>(&m2d_linear_kernel<16>),
                            mlp_kernel<1, false>(false), mlp_kernel<1, false>(true), mlp_kernel<1, true>(false), mlp_kernel<1, true>(true),
                            mlp_kernel<2, false>(false), mlp_kernel<2, false>(true), mlp_kernel<2, true>(false), mlp_kernel<2, true>(true),
-                           reinterpret_cast<const void*>(&m2d_mlp_kernel<4, true, kMlpThreads>)};
+                           reinterpret_cast<const void*>(&m2d_mlp_kernel<4, true, kMlpThreads>),
+                           reinterpret_cast<const void*>(&m2d_mlp_kernel<2, false, kMlpThreads, true>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2, false, kLinThreads, true>)};
   for (const void* k : kernels)
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLinMaxLds) != hipSuccess) return false;
   seen.fetch_or(bit, std::memory_order_release);
@@ -1483,7 +1496,7 @@ int m2d_rope_qknorm_fwd(int B, int L, int heads, int head_dim, int dtype, int we
 }
 
 static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias, float eps,
-                   const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream, const MlpArgs* res) {
+                   const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream, const MlpArgs* res, void* z = nullptr) {
   if (!x || !w1 || !w2 || !y || (ln_weight != nullptr) != (ln_bias != nullptr)) return M2D_ERR_NULL_POINTER;
   if (P < 1 || C < 1 || hidden < 1) return M2D_ERR_BAD_SHAPE;
   if (weight_dtype != M2D_F32 && weight_dtype != M2D_BF16) return M2D_ERR_UNSUPPORTED;
@@ -1496,6 +1509,7 @@ static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x
   a.ln_w = ln_weight; a.ln_b = ln_bias; a.ln_eps = eps;
   a.x = x; a.w1 = w1; a.b1 = b1; a.w2 = w2; a.b2 = b2; a.y = y; a.P = P; a.wbf16 = weight_dtype == M2D_BF16;
   if (res) { a.res_s = res->res_s; a.nx_w = res->nx_w; a.nx_b = res->nx_b; a.nx_eps = res->nx_eps; a.xo = res->xo; }
+  a.z = z;
   const size_t lds = (C == 128 ? mlp_lds_bytes<4>() : C == 64 ? mlp_lds_bytes<2>() : mlp_lds_bytes<1>()) + (res ? (size_t)3 * C * 4 : 0);
   if (lds > 64 * 1024 && !allow_big_lds()) return M2D_ERR_HIP;
   // persistent: the weights go to LDS once per workgroup
@@ -1510,6 +1524,11 @@ static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto go = [&](auto kc, auto with) {
     constexpr int KC = decltype(kc)::value;
+    if (z) {
+      if (many) hipLaunchKernelGGL((m2d_mlp_kernel<KC, false, kMlpThreads, true>), dim3((unsigned)grid), dim3(kMlpThreads), lds, st, a);
+      else hipLaunchKernelGGL((m2d_mlp_kernel<KC, false, kLinThreads, true>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
+      return;
+    }
     constexpr bool RES = decltype(with)::value;
     if (many) hipLaunchKernelGGL((m2d_mlp_kernel<KC, RES, kMlpThreads>), dim3((unsigned)grid), dim3(kMlpThreads), lds, st, a);
     else hipLaunchKernelGGL((m2d_mlp_kernel<KC, RES, kLinThreads>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
@@ -1524,6 +1543,13 @@ static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x
 int m2d_mlp_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias, float eps,
                 const void* w1, const void* b1, const void* w2, const void* b2, void* y, void* stream) {
   return run_mlp(P, C, hidden, weight_dtype, x, ln_weight, ln_bias, eps, w1, b1, w2, b2, y, stream, nullptr);
+}
+
+int m2d_mlp_keep_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* w1, const void* b1, const void* w2, const void* b2,
+                     void* z, void* y, void* stream) {
+  if (!z) return M2D_ERR_NULL_POINTER;
+  if (misaligned(z, 16)) return M2D_ERR_MISALIGNED;
+  return run_mlp(P, C, hidden, weight_dtype, x, nullptr, nullptr, 0.f, w1, b1, w2, b2, y, stream, nullptr, z);
 }
 
 int m2d_mlp_residual_layernorm_fwd(int64_t P, int C, int hidden, int weight_dtype, const void* x, const void* ln_weight, const void* ln_bias,

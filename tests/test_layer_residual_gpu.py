@@ -63,6 +63,32 @@ def test_mlp_residual_norm_gives_the_bits_of_two_kernels(P, C, wdtype):
 
 @on_gpu
 @WTYPES
+@pytest.mark.parametrize("C", [32, 64])
+@pytest.mark.parametrize("P", [1, 15, 65, 1000, 32769, 70001])
+def test_mlp_that_keeps_its_hidden_values(P, C, wdtype):
+    """The first layer's output in the bits of the layer's own kernel, the second's against fp64 sums of what it reads."""
+    from mamba2d_amd import cabi
+    H = 4 * C
+    print(f"\ncase mlp keep {P}x{C} {wdtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(P + C)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = r(P, C).bfloat16()
+    w1, w2, b1, b2 = ((r(*s) / n ** 0.5).to(wdtype) for s, n in (((H, C), C), ((C, H), H), ((H,), 1), ((C,), 1)))
+    z, y = (torch.full((P + 1, k), 7.0, dtype=torch.bfloat16, device="cuda") for k in (H, C))
+    cabi.check(cabi.lib.m2d_mlp_keep_fwd(P, C, H, cabi._dtype_code(w1), cabi._ptr(x), cabi._ptr(w1), cabi._ptr(b1), cabi._ptr(w2), cabi._ptr(b2), cabi._ptr(z),
+                                         cabi._ptr(y), cabi._stream(x.device)))
+    assert (z[P] == 7).all() and (y[P] == 7).all()
+    assert torch.equal(z[:P], cabi.linear_fwd(x, w1, b1))
+    eye = torch.eye(H, device="cuda").to(wdtype)
+    h = cabi.linear_fwd(z[:P].contiguous(), eye, None, pre=cabi.ACT_GELU).double()      # GELU(z) as a layer's kernel rounds it
+    wb = w2.bfloat16().double()
+    want = h @ wb.t() + b2.double()
+    slack = (H + 2) * 2.0 ** -24 * (h.abs() @ wb.abs().t() + b2.double().abs())      # fp32 sums of H products in any order, and the bias
+    assert ((y[:P].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1.01 * slack).all()      # the result's rounding: half a unit in the last of 8 bits
+
+
+@on_gpu
+@WTYPES
 @pytest.mark.parametrize("P", [1, 16, 127, 129, 1000, 66001])
 def test_mlp_of_128_channels(P, wdtype):
     """Weights in slices, tiles of 128 rows: the updated stream against fp64 sums of the hidden activations that the layer's own kernel gives, its norm in
@@ -105,4 +131,6 @@ def test_refusals():
     mlp = lambda C=64, s=p, nw=p, xo=p, y=p: cabi.lib.m2d_mlp_residual_layernorm_fwd(4, C, 4 * C, 1, p, None, None, 0.0, p, p, p, p, s, nw, p, 0.0, xo, y, None)
     assert [mlp(s=None), mlp(nw=None), mlp(xo=None), mlp(y=None)] == [null] * 4
     assert [mlp(C=256), mlp(C=48)] == [unsupported] * 2
+    keep = lambda C=64, z=p, y=p: cabi.lib.m2d_mlp_keep_fwd(4, C, 4 * C, 1, p, p, p, p, p, z, y, None)
+    assert [keep(z=None), keep(y=None), keep(C=128), keep(C=48), keep(z=p + 8), keep(y=p + 8)] == [null] * 2 + [unsupported] * 2 + [misaligned] * 2
     assert [mlp(xo=p + 8), mlp(s=p + 2), mlp(y=p + 4)] == [misaligned] * 3
