@@ -15,6 +15,7 @@ struct Args {
   const void *BT, *BL, *C;          // ... (B,H,W,16) in the tensors' type
   void* y;
   float* wrap;                      // [rounds - 1][B][groups of 16 channels][W][64] float4: last rows of the last bands of a round
+  uint32_t* link_err;               // error word of a linked sweep's workspace, which this kernel leaves at 0: nothing waits here; null where the plan has none
   int B, H, W, E, flip, raw;
   // the plan (make_plan)
   int nbands, nblk, rounds, stride, groups, images;

@@ -113,6 +113,7 @@ __global__ __launch_bounds__((kSweepers + kStagers) * 64, 3) void m2d_fwd_rows_k
   extern __shared__ float4 smem4[];
   float* smem = reinterpret_cast<float*>(smem4);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (p.link_err && blockIdx.x == 0 && threadIdx.x == 0) *p.link_err = 0;
   // consecutive workgroups are dealt round-robin to 8 XCDs: the channel groups of an image, which read the same records and lines, go to one
   int id = blockIdx.x;
   const int per = gridDim.x >> 3;

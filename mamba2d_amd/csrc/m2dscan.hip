@@ -3406,6 +3406,7 @@ int run_rows(const m2d_desc* d, const Geometry& g, const ScanParams& sp, const v
   if (g.packed_bc) a.rec = static_cast<const float*>(BT);
   else { a.BT = BT; a.BL = BL; a.C = C; }
   a.wrap = reinterpret_cast<float*>(static_cast<char*>(ws) + g.prep_bytes + g.link_fwd_bytes);
+  if (g.sliced) a.link_err = reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + g.prep_bytes);   // (no set-up launch clears it, and m2d_scan_link_error reads it)
   a.B = d->B; a.H = d->H; a.W = d->W; a.E = d->E; a.flip = sp.flip; a.raw = sp.raw;
   if (g_profile) (void)hipEventRecord(g_ev[M2D_PASS_FWD][0], st);
   const int err = m2drows::launch_fwd(g.rows, a, d->dtype == M2D_BF16, st);

@@ -100,3 +100,23 @@ def test_undefined_values_stay_in_their_image_and_channel():
     same[2, :, :, 7] = False
     assert torch.equal(y[same], clean[same])
     assert bool(y[1, H - 1, W - 1, 5].isnan()) and not bool(torch.isfinite(y[2, 0, 0, 7]))
+
+
+@pytest.mark.gpu
+def test_no_link_error_is_reported():
+    """Where the plan of a forward that keeps snapshots is a linked sweep, this kernel leaves the workspace's error word at 0, whatever was there."""
+    import ctypes
+
+    from mamba2d_amd import cabi
+    B, H, W, E, dtype = 131, 56, 13, 20, F32
+    assert cabi.scan_plan(B, H, W, E, dtype, cabi.M2D_PASS_FWD).startswith(("m2d_fwd_split_kernel: linked sweep", "m2d_fwd_kernel: linked sweep"))
+    print("\ncase link error word", flush=True)
+    inp = so.make_inputs(B, H, W, E, 16, seed=1, dtype=dtype)
+    dev = [inp[k].cuda() for k in so.INPUT_NAMES]
+    d = cabi.Desc(B=B, H=H, W=W, E=E, N=16, dtype=0)
+    n = cabi.lib.m2d_scan_workspace_bytes(ctypes.byref(d), cabi.M2D_PASS_FWD, 0)
+    ws, y = torch.full((n,), 255, dtype=torch.uint8, device="cuda"), torch.empty_like(dev[0])
+    cabi.check(cabi.lib.m2d_scan_fwd(ctypes.byref(d), *[cabi._ptr(t) for t in dev], cabi._ptr(y), None, 0, cabi._ptr(ws), n, cabi._stream(y.device)))
+    flag = ctypes.c_int(7)
+    cabi.check(cabi.lib.m2d_scan_link_error(ctypes.byref(d), cabi._ptr(ws), cabi._stream(y.device), ctypes.byref(flag)))
+    assert flag.value == 0
