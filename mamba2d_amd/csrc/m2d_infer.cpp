@@ -199,7 +199,10 @@ Tensor infer_stage(const Tensor& x_in, at::TensorList par, at::IntArrayRef kinds
     Tensor branch;
     if (narrow) {      // norm2 inside the MLP's first kernel
       if (term.defined()) x = r.residual(x, *rs1, term, term2);
-      if ((C == 32 || C == 64 || (C == 128 && r.P >= kWideMlpFrom)) && HD == 4 * C) {      // ... and the residual update and the next norm behind it too
+      // ... and the residual update and the next norm behind it too.  (At 128 channels the second layer is otherwise the stock product, which
+      // refuses fp32 weights without autocast: such a call is refused at every size.)
+      const bool wide = C == 128 && r.P >= kWideMlpFrom && (r.wd == M2D_BF16 || at::autocast::is_autocast_enabled(at::kCUDA));
+      if ((C == 32 || C == 64 || wide) && HD == 4 * C) {
         Tensor xo = r.make(C);
         normed = r.make(C);
         check(m2d_mlp_residual_layernorm_fwd(r.P, (int)C, (int)HD, r.wd, x.data_ptr(), n2w->data_ptr(), n2b->data_ptr(), (float)eps[3 * blk + 1],

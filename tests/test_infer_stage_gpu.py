@@ -86,3 +86,22 @@ def test_widened_parameters_are_exact():
     ts = [torch.randn(n, generator=g).bfloat16().cuda() for n in (1, 255, 256, 257, 5000)] * 14 + [torch.randn(7, generator=g).cuda()]
     out = wf.widen_op(ts)
     assert all(o.dtype == torch.float32 and torch.equal(o, t.float()) for o, t in zip(out, ts))
+
+
+@pytest.mark.parametrize("grid", [(3, 28, 28), (64, 28, 28)], ids=lambda s: "x".join(map(str, s)))
+def test_fp32_weights_need_autocast_beside_a_stock_product(monkeypatch, grid):
+    """At 128 channels the MLP's second layer is a stock product in the modules, which refuses bf16 activations with fp32 weights: so does the one call,
+    also where it has a kernel of its own for that layer."""
+    from mamba2d_amd import backbone
+    say(f"\ncase infer_stage fp32 weights without autocast {grid}")
+    with torch.device("cuda"):
+        stage = backbone.Mamba2DBackbone(n_blocks=(1,), embed_dim=(128,), token_mixer=("2D_local",), res_scale_init_values=(1.0,)).eval().stages["0"]
+        x = torch.randn(*grid, 128, dtype=torch.bfloat16)
+    with torch.no_grad():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert backbone._infer_stage(stage, x) is not None
+        with pytest.raises(RuntimeError, match="dtype"):
+            backbone._infer_stage(stage, x)
+        monkeypatch.setattr(backbone, "_infer_stage", lambda stage, t: None)
+        with pytest.raises(RuntimeError, match="dtype"):
+            backbone.Mamba2DBackbone._run_stage(stage, x)
