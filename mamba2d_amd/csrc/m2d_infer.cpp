@@ -28,9 +28,12 @@ enum Kind { kScan = 0, kScanFlipped = 1, kScanLocal = 2, kScanLocalFlipped = 3, 
 constexpr int64_t kFewPositions = 512;
 constexpr int64_t kMostPositions = 1 << 20;      // what m2d_wide_linear_fwd takes
 
-// From this many rows the MLP of 128 channels is one kernel.  A tile of 128 rows takes it 24 us and up to 512 tiles run at once; three kernels
-// take 21 to 24 us for one image's 784 rows, 62 against 40 for 50176 and 110 against 78 for 100352.
-constexpr int64_t kWideMlpFrom = 2048;
+// From this many rows the MLP of 128 channels is one kernel.  A tile of 128 rows takes it 24 us and up to 512 tiles run at once, so it takes that
+// long for one tile as for 65536 rows, while the three kernels' time grows with the rows from 21 us on.  Two such blocks with everything else, three kernels and
+// one, us, bf16 and fp32 weights: 2352 rows 189.7 and 201.3, 183.1 and 201.3; 6272 211.9 and 217.4, 205.5 and 211.9; 9216 266.3 and 273.2; 12544 252.1 and
+// 252.4, 240.7 and 244.4; 14112 278.2 and 272.1, 269.7 and 269.1; 16384 331.7 and 320.8; 25088 342.4 and 310.2, 335.3 and 306.1; 50176 460.4 and
+// 416.6.  (Of 27 sizes from 14112 rows on none is slower in one kernel, of 34 below 26 are.)
+constexpr int64_t kWideMlpFrom = 14000;
 
 struct Run {
   int64_t B, H, W, C, P;

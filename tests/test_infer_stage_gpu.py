@@ -105,3 +105,22 @@ def test_fp32_weights_need_autocast_beside_a_stock_product(monkeypatch, grid):
         monkeypatch.setattr(backbone, "_infer_stage", lambda stage, t: None)
         with pytest.raises(RuntimeError, match="dtype"):
             backbone.Mamba2DBackbone._run_stage(stage, x)
+
+
+@pytest.mark.parametrize("mode", ["bf16", "mixed"])
+@pytest.mark.parametrize("grid", [(3, 28, 28), (4, 56, 62)], ids=lambda s: "x".join(map(str, s)))
+def test_stage_of_128_channels_below_the_line_of_its_one_kernel_mlp(monkeypatch, grid, mode):
+    """Up to 14000 rows the MLP of 128 channels is a layer, a stock product and an update with norm, which are faster there, and the modules' own: the same
+    bits (the one kernel adds the second product up in another order)."""
+    from mamba2d_amd import backbone
+    say(f"\ncase infer_stage 128 channels {grid} {mode}")
+    torch.manual_seed(5)
+    with torch.device("cuda"):
+        stage = backbone.Mamba2DBackbone(n_blocks=(2,), embed_dim=(128,), token_mixer=("2D_local",), res_scale_init_values=(1.0,)).eval().stages["0"]
+        x = torch.randn(*grid, 128, dtype=torch.bfloat16)
+    stage = stage.bfloat16() if mode == "bf16" else stage
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=mode == "mixed"):
+        got = backbone._infer_stage(stage, x)
+        monkeypatch.setattr(backbone, "_infer_stage", lambda stage, t: None)
+        same = torch.equal(got, backbone.Mamba2DBackbone._run_stage(stage, x))
+    assert same
