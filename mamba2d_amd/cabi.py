@@ -246,7 +246,7 @@ def scan_plan(B, H, W, E, dtype, pass_=M2D_PASS_FWD, N=16, flags=None, ckpt_inte
     """The library's one-line description of how it will run a pass of this problem (m2d_scan_plan)."""
     dt = M2D_F32 if dtype in (torch.float32, "f32") else M2D_BF16
     d = Desc(B, H, W, E, N, dt, SCHEDULE_HINT if flags is None else flags, CKPT_INTERVAL if ckpt_interval is None else ckpt_interval)
-    buf = ctypes.create_string_buffer(320)
+    buf = ctypes.create_string_buffer(512)
     check(lib.m2d_scan_plan(ctypes.byref(d), pass_, buf, len(buf)))
     return buf.value.decode()
 

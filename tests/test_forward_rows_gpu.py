@@ -29,6 +29,25 @@ CASES = [
     (131, 50, 2, 12, F32, 8, 7),
     (91, 60, 2, 12, BF16, 8, 8),
 ]
+# ... with rounds of bands (rows handed on through memory, from three rounds on from more than one place of it) and images that a workgroup sweeps one after the
+# other, the last workgroup not full.  The blocks of a round are as many as columns ask for, or more (padded, so that a row is stored when it is read).
+HANDED = [
+    # B, H, W, E, dtype, bands side by side, rows a band, rounds, images a workgroup
+    (132, 33, 12, 32, BF16, 2, 6, 3, 1),
+    (193, 33, 9, 48, F32, 2, 6, 3, 1),      # padded by a block
+    (299, 69, 2, 48, BF16, 2, 7, 5, 2),     # one block of columns in six
+    (293, 65, 2, 36, F32, 2, 7, 5, 2),
+    (58, 72, 2, 36, BF16, 4, 6, 3, 1),
+    (172, 65, 2, 20, F32, 4, 6, 3, 1),
+    (129, 103, 2, 20, BF16, 4, 7, 4, 1),
+    (261, 65, 15, 12, BF16, 4, 6, 3, 2),    # not padded
+    (521, 71, 2, 12, BF16, 4, 6, 3, 3),     # the last workgroup has two images of three
+    (139, 85, 2, 12, BF16, 8, 6, 2, 1),     # 8 bands: a staging wave for two of them
+    (176, 136, 2, 12, F32, 8, 6, 3, 1),
+    (261, 83, 7, 12, BF16, 8, 6, 2, 2),
+    (293, 94, 23, 4, BF16, 8, 6, 2, 2),     # not padded
+    (281, 168, 2, 12, F32, 8, 7, 3, 2),
+]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:4])))
@@ -40,9 +59,19 @@ def test_plan_names_the_rows_kernel(case):
         assert "rows_kernel" not in cabi.scan_plan(*case[:5], cabi.M2D_PASS_FWD, flags=flags)
 
 
+@pytest.mark.parametrize("case", HANDED, ids=lambda c: "x".join(map(str, c[:4])))
+def test_plan_names_rounds_and_images(case):
+    from mamba2d_amd import cabi
+    plan = cabi.scan_plan(*case[:5], cabi.M2D_PASS_FWD)
+    B, E, slots, rows, rounds, images = case[0], case[3], *case[5:]
+    groups = -(-((E + 15) // 16) // (8 // slots))
+    assert plan.endswith(f"; without snapshots m2d_fwd_rows_kernel, {-(-B // images) * groups} workgroups, {images} images and {rounds} rounds each, "
+                         f"of {slots} bands of {rows} rows and {128 // slots} channels"), plan
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("flip", [False, True], ids=["tl", "br"])
-@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:4])))
+@pytest.mark.parametrize("case", CASES + HANDED, ids=lambda c: "x".join(map(str, c[:4])))
 def test_values(cscan, case, flip):
     from mamba2d_amd import cabi
     B, H, W, E, dtype = case[:5]
