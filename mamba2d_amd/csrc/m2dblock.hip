@@ -1115,11 +1115,6 @@ constexpr size_t mlp_lds_bytes() {
 constexpr size_t kLinMaxLds = 160 * 1024;   // LDS of a compute unit
 
 constexpr int kMlpThreads = 512;      // of the kernel for many positions
-template <int KC, bool RES>
-const void* mlp_kernel(bool many) {
-  return many ? reinterpret_cast<const void*>(&m2d_mlp_kernel<KC, RES, kMlpThreads>) : reinterpret_cast<const void*>(&m2d_mlp_kernel<KC, RES, kLinThreads>);
-}
-
 // More than 64 KB of dynamic LDS has to be allowed per kernel and device, once.
 inline bool allow_big_lds() {
   static std::atomic<uint64_t> seen{0};
@@ -1129,8 +1124,8 @@ inline bool allow_big_lds() {
   if (seen.load(std::memory_order_acquire) & bit) return true;
   const void* kernels[] = {reinterpret_cast<const void*>(&m2d_linear_kernel<2>), reinterpret_cast<const void*>(&m2d_linear_kernel<4>),
                            reinterpret_cast<const void*>(&m2d_linear_kernel<8>), reinterpret_cast<const void*>(&m2d_linear_kernel<16>),
-                           mlp_kernel<1, false>(false), mlp_kernel<1, false>(true), mlp_kernel<1, true>(false), mlp_kernel<1, true>(true),
-                           mlp_kernel<2, false>(false), mlp_kernel<2, false>(true), mlp_kernel<2, true>(false), mlp_kernel<2, true>(true),
+                           reinterpret_cast<const void*>(&m2d_mlp_kernel<2, false, kMlpThreads>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2, false, kLinThreads>),
+                           reinterpret_cast<const void*>(&m2d_mlp_kernel<2, true, kMlpThreads>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2, true, kLinThreads>),
                            reinterpret_cast<const void*>(&m2d_mlp_kernel<4, true, kMlpThreads>),
                            reinterpret_cast<const void*>(&m2d_mlp_kernel<2, false, kMlpThreads, true>), reinterpret_cast<const void*>(&m2d_mlp_kernel<2, false, kLinThreads, true>)};
   for (const void* k : kernels)
@@ -1514,29 +1509,32 @@ static int run_mlp(int64_t P, int C, int hidden, int weight_dtype, const void* x
   if (lds > 64 * 1024 && !allow_big_lds()) return M2D_ERR_HIP;
   // persistent: the weights go to LDS once per workgroup
   const int fit = (int)(160 * 1024 / lds);
-  // Workgroups of 8 waves where they fill the device: twice the waves that share a copy of the weights (C = 64, RES: 50176 positions 17.0 us, 401408
-  // 82.8; of 6 waves 21.9 and 106); of 4 below, where more of them share out the rows.
-  const bool many = P > 256 * 128 || C == 128;
-  const int rows = many ? kMlpThreads / 4 : 64, per_cu = many ? (fit < 2 ? fit : 2) : (fit < 4 ? fit : 4);
+  // 64 channels: workgroups of 8 waves where they fill the device: twice the waves that share a copy of the weights (RES: 50176 positions 17.0 us, 401408
+  // 82.8; of 6 waves 21.9 and 106); of 4 below, where more of them share out the rows.  32 channels: of 4 at any size, up to 8 on a unit, whose tiles of 64 rows leave
+  // less of a round empty (m2d_mlp_fwd, fp32 weights, 2 workgroups of 8 waves on a unit, 4 and 8 of 4 waves: 33000 positions 7.8, 7.1 and 7.1 us, 100352 13.3,
+  // 11.6 and 12.5, 300000 29.7, 28.1 and 27.9, 401408 36.5, 35.7 and 34.6; 65536 8.3, 8.6 and 8.7; RES 100352 16.0, 14.0 and 15.0, 300000 33.5, 31.5 and 31.0).
+  const bool many = C == 128 || (C == 64 && P > 256 * 128);
+  const int rows = many ? kMlpThreads / 4 : 64, most = many ? 2 : C == 32 ? 8 : 4, per_cu = fit < most ? fit : most;
   a.ntiles = (int)((P + rows - 1) / rows);
   int grid = 256 * per_cu;
   if (grid > a.ntiles) grid = a.ntiles;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  auto go = [&](auto kc, auto with) {
-    constexpr int KC = decltype(kc)::value;
-    if (z) {
-      if (many) hipLaunchKernelGGL((m2d_mlp_kernel<KC, false, kMlpThreads, true>), dim3((unsigned)grid), dim3(kMlpThreads), lds, st, a);
-      else hipLaunchKernelGGL((m2d_mlp_kernel<KC, false, kLinThreads, true>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
-      return;
-    }
-    constexpr bool RES = decltype(with)::value;
-    if (many) hipLaunchKernelGGL((m2d_mlp_kernel<KC, RES, kMlpThreads>), dim3((unsigned)grid), dim3(kMlpThreads), lds, st, a);
-    else hipLaunchKernelGGL((m2d_mlp_kernel<KC, RES, kLinThreads>), dim3((unsigned)grid), dim3(kLinThreads), lds, st, a);
+  auto go = [&](auto kc, auto with, auto keep, auto threads) {
+    constexpr int KC = decltype(kc)::value, TH = decltype(threads)::value;
+    constexpr bool RES = decltype(with)::value, KEEP = decltype(keep)::value;
+    hipLaunchKernelGGL((m2d_mlp_kernel<KC, RES, TH, KEEP>), dim3((unsigned)grid), dim3(TH), lds, st, a);
   };
-  auto with = [&](auto kc) { if (res) go(kc, std::true_type{}); else go(kc, std::false_type{}); };
+  auto with = [&](auto kc, auto threads) {
+    if (z) go(kc, std::false_type{}, std::true_type{}, threads);
+    else if (res) go(kc, std::true_type{}, std::false_type{}, threads);
+    else go(kc, std::false_type{}, std::false_type{}, threads);
+  };
+  constexpr std::integral_constant<int, kLinThreads> four{};
+  constexpr std::integral_constant<int, kMlpThreads> eight{};
   if (C == 128) hipLaunchKernelGGL((m2d_mlp_kernel<4, true, kMlpThreads>), dim3((unsigned)grid), dim3(kMlpThreads), lds, st, a);
-  else if (C == 64) with(std::integral_constant<int, 2>{});
-  else with(std::integral_constant<int, 1>{});
+  else if (C == 64 && many) with(std::integral_constant<int, 2>{}, eight);
+  else if (C == 64) with(std::integral_constant<int, 2>{}, four);
+  else with(std::integral_constant<int, 1>{}, four);
   return hipGetLastError() == hipSuccess ? M2D_OK : M2D_ERR_HIP;
 }
 

@@ -134,3 +134,21 @@ def test_refusals():
     keep = lambda C=64, z=p, y=p: cabi.lib.m2d_mlp_keep_fwd(4, C, 4 * C, 1, p, p, p, p, p, z, y, None)
     assert [keep(z=None), keep(y=None), keep(C=128), keep(C=48), keep(z=p + 8), keep(y=p + 8)] == [null] * 2 + [unsupported] * 2 + [misaligned] * 2
     assert [mlp(xo=p + 8), mlp(s=p + 2), mlp(y=p + 4)] == [misaligned] * 3
+
+
+@on_gpu
+@WTYPES
+def test_mlp_of_32_channels_over_several_tiles_a_workgroup(wdtype):
+    """More tiles of 64 rows than workgroups that are launched: the rows are what calls of a few tiles give for them, bit for bit."""
+    from mamba2d_amd import cabi
+    P, C = 64 * 2048 + 64 * 130 + 5, 32
+    print(f"\ncase mlp {P}x{C} {wdtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(C)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = r(P, C).bfloat16()
+    w = [(0.2 * r(*s)).to(wdtype) for s in ((4 * C, C), (4 * C,), (C, 4 * C), (C,), (C,), (C,))]
+    y = cabi.mlp_fwd(x, *w)
+    for at in (0, 64 * 2048 - 300, P - 64 * 131):
+        part = x[at:at + 64 * 131].contiguous()
+        same = torch.equal(cabi.mlp_fwd(part, *w), y[at:at + part.shape[0]])
+        assert same
