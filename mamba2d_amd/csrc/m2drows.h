@@ -2,8 +2,21 @@
 #ifndef M2D_ROWS_H
 #define M2D_ROWS_H
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <stddef.h>
 #include <stdint.h>
+
+// A kernel that needs more than 64 KB of dynamic LDS has to be told so once per device (each
+// device loads its own copy of the code object).  `seen` holds one bit per device ordinal.
+inline bool allow_dynamic_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& seen) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (seen.load(std::memory_order_relaxed) & bit) return true;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
+  seen.fetch_or(bit, std::memory_order_relaxed);
+  return true;
+}
 
 namespace m2drows {
 

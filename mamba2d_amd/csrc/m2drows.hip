@@ -21,7 +21,6 @@
 // 128x14x14x320 0.100 -> 0.068; rows of 4 to 7 channels past a whole chunk, which those fetch value by value, up to 3 times as fast (110x17x12x216 0.163 -> 0.052).
 #include "m2drows.h"
 
-#include <atomic>
 #include <type_traits>
 
 namespace m2drows {
@@ -393,7 +392,7 @@ __global__ __launch_bounds__((kSweepers + kStagers) * 64, 3) void m2d_fwd_rows_k
           if ((c & 3) == 3) yb[(c - 3 + (g & 1) * 2 + (g >> 1)) * 16] = fold16(fold32(pr[0], pr[1]), fold32(pr[2], pr[3]));
           else if (c == NC - 1) { const float f = fold32(pr[0], pr[1]); yb[(c - 1 + (g >> 1)) * 16] = fold16(f, f); }   // (two cells are left)
           // the rows of the step before are in memory when this step ends
-          if (NB > 0 && c == R - 1 && slot == NB - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          if (c == R - 1 && slot == NB - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
           if (i == R - 1) {
             const float4 last = make_float4(hT[0], hT[1], hT[2], hT[3]);
             if (slot == NB - 1) {
@@ -418,21 +417,12 @@ __global__ __launch_bounds__((kSweepers + kStagers) * 64, 3) void m2d_fwd_rows_k
   }
 }
 
-inline bool allow_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& seen) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  const uint64_t bit = 1ull << (dev & 63);
-  if (seen.load(std::memory_order_relaxed) & bit) return true;
-  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
-  seen.fetch_or(bit, std::memory_order_relaxed);
-  return true;
-}
 template <typename T, int R, int NB, bool PACKED>
 int launch_packed(const Plan& plan, const Args& a, hipStream_t st) {
   constexpr size_t lds = Lds<R, NB>::kBytes;
   static_assert(lds <= 160 * 1024, "a compute unit has 160 KB");
   static std::atomic<uint64_t> seen{0};
-  if (!allow_lds(reinterpret_cast<const void*>(&m2d_fwd_rows_kernel<T, R, NB, PACKED>), lds, seen)) return (int)hipErrorInvalidValue;
+  if (!allow_dynamic_lds(reinterpret_cast<const void*>(&m2d_fwd_rows_kernel<T, R, NB, PACKED>), lds, seen)) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL((m2d_fwd_rows_kernel<T, R, NB, PACKED>), dim3((unsigned)plan.workgroups), dim3((kSweepers + kStagers) * 64), lds, st, a);
   return (int)hipGetLastError();
 }

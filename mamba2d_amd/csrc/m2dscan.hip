@@ -3187,18 +3187,6 @@ inline int linked_grid(ScanParams& sp, bool forward, bool chunks, bool half) {
   return (int)((units + 7) / 8 * 8 * sp.sl_unit);
 }
 
-// A kernel that needs more than 64 KB of dynamic LDS has to be told so once per device (each
-// device loads its own copy of the code object).  `seen` holds one bit per device ordinal.
-inline bool allow_dynamic_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& seen) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  const uint64_t bit = 1ull << (dev & 63);
-  if (seen.load(std::memory_order_relaxed) & bit) return true;
-  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
-  seen.fetch_or(bit, std::memory_order_relaxed);
-  return true;
-}
-
 // Set-up area: [page of zeros][A_T*log2e][A_L*log2e][D], all fp32.
 template <typename T>
 int launch_prep(ScanParams& sp, const m2d_desc* d, const Geometry& g, float* base, uint32_t* link_words, size_t link_bytes, hipStream_t st, bool ready = false) {
