@@ -13,12 +13,14 @@
 // sizes into LDS 2 cells ahead of the block that the sweeping waves are at, whose loads thus run on across the barrier; y
 // comes back as sums over a lane's states and quarters (lane swaps), gets x*D and leaves in rows of 16 channels.
 //
-// Bound by the issue of vector instructions: per lane and cell 28 of arithmetic (8 exponentials at half rate) for 4 units, 1.5 for the sums of y and, in the
-// staging wave, about 6; a unit (cell, channel, state) takes 12 issue slots for 11 of arithmetic, against 20 in m2d_fwd_split_kernel.  The two sweeping waves and the
-// staging one of a SIMD keep it issuing 80 % of the time; without the staging waves, each wave bringing its own operands, it was 60 % (128x56x56x64: 0.245 ms).
+// Bound by the issue of vector instructions: a unit (cell, channel, state) is 9 of arithmetic, 2 of them exponentials at half rate; with the sums of y and what the
+// staging waves do it is 11.6 to 11.8 as counted (SQ_INSTS_VALU), against 17.8 in m2d_fwd_split_kernel.  The two sweeping waves and the
+// staging one of a SIMD keep it issuing 86 % of the time where a sweep has 56 blocks (128x56x56x64) and 71 % where it has 14 (64x28x28x128: start and end of the
+// only round); without the staging waves, each wave bringing its own operands, it was 60 % (128x56x56x64: 0.245 ms).
 // Products on the matrix cores do not help: an fp32 16x16x4 takes the vector ALU's time (32 clocks, measured), as much as the 8 multiply-adds it replaces.
-// Forward without snapshots, bf16, against the kernels that it takes over from: 128x56x56x64 0.225 -> 0.178 ms, 128x28x28x128 0.130 -> 0.089, 64x28x28x128 0.076 -> 0.054,
-// 128x14x14x320 0.100 -> 0.068; rows of 4 to 7 channels past a whole chunk, which those fetch value by value, up to 3 times as fast (110x17x12x216 0.163 -> 0.052).
+// Forward without snapshots, bf16, a whole call, against the kernels that it takes over from: 128x56x56x64 0.247 -> 0.187 ms, 128x28x28x128 0.128 -> 0.089,
+// 64x28x28x128 0.075 -> 0.052; rows of 4 channels past a whole chunk of 8, which those fetch value by value: 43x21x39x108 0.109 -> 0.059,
+// 28x51x10x180 0.116 -> 0.046, 34x109x25x52 0.112 -> 0.091.  Images of one band (14x14, 7x7) are stacked in m2d_fwd_kernel: the rule does not price this kernel for them.
 #include "m2drows.h"
 
 #include <type_traits>

@@ -3082,9 +3082,11 @@ Geometry make_geometry(const m2d_desc* d, bool for_alone = false) {
     if (!split || 100 * whole_cost_alone < 97 * split_cost_alone) g.alone = whole;
     if (sums_bound && 100 * split_cost_alone < (split ? 100 : 90) * whole_cost_alone) g.alone = {true, 1, nw, (d->E + nw - 1) / nw};
   }
-  // m2d_fwd_rows_kernel where it takes less time than that kernel: a sweeping wave of it needs 0.2 us a cell with bf16 tensors and 0.225 with fp32 ones
-  // (0.17 to 0.22 and 0.16 to 0.25 over 120 drawn problems; less where units are not full), a launch 3 us more; the kernels above are priced by their blocks, in the same
-  // units of 10 ns.  It has to promise 7 %.  Where a forward without snapshots has another kernel than one that keeps them anyhow, it stays with that.
+  // m2d_fwd_rows_kernel where it takes less time than that kernel: a sweeping wave of it needs 0.2 us a cell with bf16 tensors and 0.225 with fp32 ones, a launch 3 us
+  // more (110 drawn problems that take it, B 4 to 600, H and W 7 to 140, E 8 to 512, 2^19 to 2^26 values: 0.13 to 0.22 and 0.15 to 0.24, least where units are
+  // not full); the kernels above are priced by their blocks, in the same units of 10 ns.  It has to promise 7 %: those 110 take 0.29 to 0.96 of the time they
+  // took, mean 0.64.  Where a forward without snapshots has another kernel than one that keeps them anyhow, it stays with that: caution, not a
+  // measured line (forced on 40 drawn problems that this keeps out, the rows took 0.31 to 1.03 of the time, mean 0.73, five of them 0.98 and more).
   g.rows = m2drows::Plan{};
   const bool same = g.alone.split == g.fwd_split && g.alone.ec == g.fwd_ec && g.alone.nw == g.fwd_nw;
   const m2drows::Plan by_rows = for_alone && may_split && same && !(d->flags & (M2D_FLAG_SPLIT_STATES | M2D_FLAG_TEST_DEAD_LINK)) ? m2drows::make_plan(d->B, d->H, d->W, d->E, (int)ncu) : m2drows::Plan{};
