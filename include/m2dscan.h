@@ -182,7 +182,7 @@ int m2d_scan_link_error(const m2d_desc* desc, const void* workspace, void* strea
  * "m2d_bwd_split_kernel: linked sweep, 19 bands, 304 workgroups of 4 waves and 4 that stage, 4 channels each, 4 states per lane".
  * The forward's line is that of the call that keeps snapshots; where the one that keeps none runs another kernel, it ends in
  * "; without snapshots <kernel>, <n> workgroups of <channels> channels", or, where rows of a band follow each other in a lane, in
- * "; without snapshots m2d_fwd_rows_kernel, <n> workgroups[, <i> images and <k> rounds each,] of <s> bands of <r> rows and <channels> channels".  At
+ * "; without snapshots m2d_fwd_rows_kernel, <n> workgroups[, <i> image(s) and <k> round(s) each,] of <s> bands of <r> rows and <channels> channels".  At
  * most 512 bytes.
  * Writes at most `cap` bytes including the terminating 0; host only, touches no device.  Returns M2D_OK or the
  * status m2d_desc_check gives.  No counterpart in the reference (which has one schedule). */

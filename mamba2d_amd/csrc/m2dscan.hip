@@ -3677,7 +3677,7 @@ int m2d_scan_plan(const m2d_desc* desc, int pass, char* text, size_t cap) {
   if (fwd && g.rows.rows) {
     const size_t n = strlen(text);
     char turns[48] = "";
-    if (g.rows.images > 1 || g.rows.rounds > 1) snprintf(turns, sizeof turns, ", %d images and %d rounds each,", g.rows.images, g.rows.rounds);
+    if (g.rows.images > 1 || g.rows.rounds > 1) snprintf(turns, sizeof turns, ", %d image%s and %d round%s each,", g.rows.images, g.rows.images > 1 ? "s" : "", g.rows.rounds, g.rows.rounds > 1 ? "s" : "");
     if (n + 1 < cap) snprintf(text + n, cap - n, "; without snapshots m2d_fwd_rows_kernel, %d workgroups%s of %d bands of %d rows and %d channels", g.rows.workgroups, turns, g.rows.slots, g.rows.rows, 16 * (8 / g.rows.slots));
   } else if (fwd && (g.alone.split != g.fwd_split || g.alone.ec != g.fwd_ec || g.alone.nw != g.fwd_nw)) {
     const size_t n = strlen(text);

@@ -65,7 +65,7 @@ def test_plan_names_rounds_and_images(case):
     plan = cabi.scan_plan(*case[:5], cabi.M2D_PASS_FWD)
     B, E, slots, rows, rounds, images = case[0], case[3], *case[5:]
     groups = -(-((E + 15) // 16) // (8 // slots))
-    assert plan.endswith(f"; without snapshots m2d_fwd_rows_kernel, {-(-B // images) * groups} workgroups, {images} images and {rounds} rounds each, "
+    assert plan.endswith(f"; without snapshots m2d_fwd_rows_kernel, {-(-B // images) * groups} workgroups, {images} image{'s'[:images > 1]} and {rounds} rounds each, "
                          f"of {slots} bands of {rows} rows and {128 // slots} channels"), plan
 
 
