@@ -2,7 +2,7 @@
 //
 // The block of models/mamba2d.py:191-254 with the token mixer of :157-188 and the local path and MLP of
 // models/utils.py:58-118: x1 = s1 x + mixer(norm1 x), x2 = s2 x1 + MLP(norm2 x1).  Forward and backward are a fixed
-// sequence of the library's kernels on one stream (10 + 17 launches beside the scan's and its projections' 10), issued
+// sequence of the library's kernels on one stream (9 + 11 launches beside the scan's and its projections' 2 + 5), issued
 // from here: no Python between them, no cast kernels (the fp32 parameters are read as they are), activations rounded to
 // bf16 where autocast rounds them.
 #include <ATen/autocast_mode.h>
