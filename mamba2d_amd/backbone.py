@@ -591,7 +591,8 @@ def _stage_plan(stage, x):
 
 def _infer_stage(stage, x):
     """A stage (residual blocks and the LayerNorm behind them) at inference on bf16 activations as one call: the kernels
-    that the modules would run, in their order, without Python in between.  None where a module asks for something
+    that the modules would run, in their order (narrow blocks have the residual updates inside the layers in front of
+    them), without Python in between.  None where a module asks for something
     else (gradients, training mode, hooks, foreign modules, parameters of mixed types), or where somebody has put
     another operator in the place of one that the call stands for (to count or to time it)."""
     if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 4 and x.numel() > 0 and x.is_contiguous() and len(stage) > 1

@@ -1,5 +1,7 @@
 """A backbone stage at inference as one call (m2dscan::infer_stage) against the same stage module by module: the same
-kernels in the same order, so the results must be the same bits; and the cases in which the modules run instead."""
+kernels in the same order, but for the residual updates, which narrow blocks have inside the layers in front of them in the same
+bits, so the results must be the same bits (from 14000 rows on the MLP of 128 channels adds up in another order); and the cases in which the
+modules run instead."""
 import pytest
 import torch
 
